@@ -43,6 +43,8 @@ MN_DEV_API void mn_wide_tune(int llm_min_rows, int rf_min_rows, int sem_min_rows
 MN_DEV_API void mn_lo_drop_mask(unsigned mask);
 /* Tile lists (expert GEMMs): skip the MFMAs and fragment reads of M-fragments without a live row (1, shipped) or run them all (0). */
 MN_DEV_API void mn_gemm256_tune_thin(int on);
+/* The form of every dense gemm256 launch: -1 the rule, 0 the 256 x 256 tiles, 1 .. the small-tile forms of gemm_tile.inl. */
+MN_DEV_API void mn_gemm_tile_tune(int form);
 /* Measurement only: K / V rows are rounded to bf16 when appended to the (fp32) cache — the values a bf16 KV cache would hold. */
 MN_DEV_API void mn_kv_round_bf16(int on);
 

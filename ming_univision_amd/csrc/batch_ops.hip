@@ -243,12 +243,11 @@ extern "C" int mn_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, i
   MN_CHECK_ARG(M >= 1 && N >= 1 && K >= 8 && (K % 8) == 0, "mn_gemm_bf16: bad M=%d N=%d K=%d (K %% 8 == 0)", M, N, K);
   MN_CHECK_ARG((lda % 8) == 0 && (ldw % 8) == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0,
                "mn_gemm_bf16: A/W rows must be 16-byte aligned");
-  // enough 256 x 256 tiles to fill half the chip: the 8-wave 4-phase kernel (gemm256.hip: 1.2 PFLOP/s at 4096^3 against
-  // 0.76 here); smaller problems keep the 128 x 128 tiles (more workgroups, 2-3 per CU)
-  // (gemm256's epilogue stores 4 consecutive columns per lane and loads the bias 8 bytes at a time: C / bias alignment and ldc % 4
-  //  are part of the routing condition, anything else stays on the 128-tile kernel with its scalar epilogue)
+  // whole K-tiles and aligned quadruples of columns: the LDS-DMA kernels of gemm256.hip, which pick their tile by the shape (64 x 64 .. 256 x 256:
+  // 65 x 3072 x 1024 bf16 7.3 us against 23.6 on the 128 x 128 tiles below, 2048 x 2048 x 14336 140 against 220); anything else stays
+  // on the 128-tile kernel with its scalar epilogue (gemm256's stores 4 consecutive columns per lane and loads the bias 8 bytes at a time)
   const bool f32_out = epilogue == MN_GEMM_F32 || epilogue == MN_GEMM_F32_RESID;
-  if (g_gemm_route256 && (K % 64) == 0 && (N % 4) == 0 && mn_cdiv(M, 256) * mn_cdiv(N, 256) >= 128 &&
+  if (g_gemm_route256 && (K % 64) == 0 && (N % 4) == 0 &&
       (int64_t)N * ldw * 2 < ((int64_t)1 << 32) && epilogue >= MN_GEMM_BF16 && epilogue <= MN_GEMM_F32_RESID &&
       (ldc % 4) == 0 && ((uintptr_t)C & (f32_out ? 15 : 7)) == 0 && ((uintptr_t)bias & 7) == 0) {
     static const int map[4] = {MN_G256_BF16, MN_G256_BF16_GELU, MN_G256_F32, MN_G256_F32_RESID};
@@ -282,6 +281,9 @@ extern "C" int mn_gemm_bf16_hilo(const uint16_t* A_hi, int64_t lda, int64_t a_lo
   MN_CHECK_ARG(M >= 1 && N >= 1 && K >= 8 && (K % 8) == 0, "mn_gemm_bf16_hilo: bad M=%d N=%d K=%d (K %% 8 == 0)", M, N, K);
   MN_CHECK_ARG((lda % 8) == 0 && (ldw % 8) == 0 && (a_lo_off % 8) == 0 && (((uintptr_t)A_hi | (uintptr_t)W) & 15) == 0,
                "mn_gemm_bf16_hilo: A/W rows must be 16-byte aligned");
+  // the same rule as mn_gemm_bf16's (operands beyond 4 GiB stay on the 128-tile kernel)
+  if (g_gemm_route256 && mn_gemm256_supported(lda, a_lo_off, ldw, N, M, N, K) && (ldc % 4) == 0 && ((uintptr_t)C & 15) == 0 && ((uintptr_t)bias & 7) == 0)
+    return mn_gemm256(A_hi, lda, a_lo_off, W, ldw, bias, C, ldc, M, N, K, MN_GEMM_F32, stream);
   const int bm = (M <= 32) ? 32 : (M <= 64) ? 64 : 128;
   dim3 grid((unsigned)(mn_cdiv(M, bm) * mn_cdiv(N, BN)), 1);
   const bool glds = g_gemm_glds && (K % BK) == 0;

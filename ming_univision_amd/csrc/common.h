@@ -187,3 +187,4 @@ enum { MN_G256_F32 = 0, MN_G256_BF16 = 1, MN_G256_BF16_GELU = 2, MN_G256_F32_RES
        MN_G256_SWIGLU_BF16_SCALED = 8 };
 extern "C" int mn_gemm256_ex(const mn_g256* a, int epi, int ksplit, void* stream);
 extern "C" int mn_gemm256_slices(int K, int ksplit);
+extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo);

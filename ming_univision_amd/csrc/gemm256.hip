@@ -137,7 +137,8 @@ __device__ __forceinline__ float gelu_erf_bf16out(float x) {
 
 // Epilogue of one output tile.  A lane holds, per (i, j), output row 16 i + fr and the 4 CONSECUTIVE columns 16 j + 4 fq .. +3.
 // One lane's 4 CONSECUTIVE output columns n..n+3 of row m (u: the paired "up" values): bias, epilogue, store.
-template <int EPI>
+// EXACT_GELU: erff itself (the small-tile kernels, whose lanes hold 16 .. 32 values)
+template <int EPI, bool EXACT_GELU = false>
 __device__ __forceinline__ void g256_emit(const G256& p, char* Cz, int m, int n, f32x4 v, f32x4 u, int zslice) {
   constexpr bool paired = epi_paired(EPI);
   if (p.bias && zslice == 0) {
@@ -158,7 +159,8 @@ __device__ __forceinline__ void g256_emit(const G256& p, char* Cz, int m, int n,
     const f32x4 g = *reinterpret_cast<const f32x4*>(p.gate + (int64_t)m * p.ldgate + n);
     *c += g * v;
   } else if (EPI == E_BF16 || EPI == E_BF16_GELU || EPI == E_BF16_RELU2) {
-    if (EPI == E_BF16_GELU) v = f32x4{gelu_erf_bf16out(v.x), gelu_erf_bf16out(v.y), gelu_erf_bf16out(v.z), gelu_erf_bf16out(v.w)};
+    if (EPI == E_BF16_GELU && EXACT_GELU) v = f32x4{gelu_erf_f(v.x), gelu_erf_f(v.y), gelu_erf_f(v.z), gelu_erf_f(v.w)};
+    else if (EPI == E_BF16_GELU) v = f32x4{gelu_erf_bf16out(v.x), gelu_erf_bf16out(v.y), gelu_erf_bf16out(v.z), gelu_erf_bf16out(v.w)};
     if (EPI == E_BF16_RELU2) {                         // the squared relu of a feed-forward's hidden units
       const f32x4 r = f32x4{fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f)};
       v = r * r;
@@ -405,20 +407,91 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const G256 p) {
   g256_epilogue<EPI, HILO, F8>(p, acc, wr, wc, fr, fq, m0, n0, row0, Mg, blockIdx.y, grp);
 }
 
-
+#include "gemm_tile.inl"
 
 }  // namespace
 
 // Tile order: dense problems run in bands of 4 M-tiles inside an XCD's tile range; tile lists keep the N-tiles of a row tile together
 // (bands of 2-8 row tiles measured 0.7 % slower end to end).
-static int g_g256_groupm = 4, g_g256_groupb = 1, g_g256_thin = 1;
+static int g_g256_groupm = 4, g_g256_groupb = 1, g_g256_thin = 1, g_g256_tile = -1;
 #ifdef MN_DEV_HOOKS
+extern "C" MN_DEV_API void mn_gemm_tile_tune(int form) { g_g256_tile = form; }   // A/B hook: the form of every dense launch (0: 256 x 256 tiles; -1: the rule)
 extern "C" MN_DEV_API void mn_gemm256_tune_thin(int on) { g_g256_thin = on; }   // A/B hook: skip the MFMAs of dead M-fragments in tile lists
 extern "C" MN_DEV_API void mn_gemm256_tune_order(int group_m, int group_list) {   // A/B hook (tools/, libmingnative_dev.so only)
   g_g256_groupm = group_m;
   g_g256_groupb = group_list;
 }
 #endif
+
+// ---- which tile ------------------------------------------------------------------------------------------------------------------
+// Forms of a dense launch: 0 = the 256 x 256 kernel above, 1 .. = gemm_tile.inl's.  The choice minimises an estimate of the launch's time,
+//   t = fixed + K-tiles of a workgroup x us per K-tile at w = workgroups / 256 CUs
+// with the constants measured on MI355X (weights cycling through HBM, graph of 48 launches; us): a workgroup alone on its CU needs `alone` per
+// K-tile, rising to `full` when every CU holds one and to `two` when every CU holds two (forms that fit twice); beyond that `per` for each
+// workgroup of a CU, or whole rounds of `full` (forms that fit once: per = 0).  The fixed part is launch, first round trip and epilogue: 4 us
+// for the small tiles, 11 us + 7 per further round for the 256-tile kernel.
+// Where the lines then lie, both sides measured: 65 x 3072 x 1024 bf16: 7.3 us (64 x 64) against 23.7 (256); 256 x 4096 x 1024: 8.2 against
+// 32.1; 1025 hi/lo rows x 1024 x 1024: 12.4 against 25.0; x 3072: 20.5 (128 x 128) against 27.5; 2048 x 2048 x 8192: 79.6 (128 x 128) against 136.6;
+// 16384 x 1024 x 1024: 37.2 (256) against 54.2 (128 x 128); 1025 hi/lo rows x 2752 SwiGLU: 29.9 (256) against 37.8.
+struct TileForm { int form, bm, bn; double fixed, alone, full, two, per; };
+static const TileForm tile_plain[] = {{1, 64, 64, 3.6, 0.23, 0.26, 0.42, 0.30}, {2, 64, 128, 3.9, 0.37, 0.40, 0.75, 0.48}, {3, 128, 128, 4.2, 0.50, 0.61, 0, 0},
+                                      {4, 128, 128, 4.2, 0.55, 0.85, 1.16, 0.85}, {0, 256, 256, 11.0, 0.85, 1.30, 0, 0}};
+static const TileForm tile_hilo[] = {{1, 64, 64, 3.8, 0.41, 0.42, 0.60, 0.41}, {2, 64, 128, 4.0, 0.64, 0.66, 1.00, 0.58}, {3, 128, 128, 4.2, 0.93, 1.04, 0, 0},
+                                     {0, 128, 256, 11.0, 0.87, 1.25, 0, 0}};
+
+static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bool paired) {
+  const double w = (double)(mn_cdiv(M, f.bm) * mn_cdiv(N, paired ? f.bn / 2 : f.bn) * nz) / 256.0;
+  const double rounds = w > 1.0 ? (double)(int64_t)(w + 0.999) : 1.0;
+  double per_tile;
+  if (w <= 1.0) per_tile = f.alone + (f.full - f.alone) * w;
+  else if (f.per == 0) per_tile = f.full * rounds;
+  else if (w <= 2.0) per_tile = f.full + (f.two - f.full) * (w - 1.0);
+  else per_tile = f.per * w > f.two ? f.per * w : f.two;
+  return f.fixed + (f.form == 0 ? 7.0 * (rounds - 1.0) : 0.0) + k_tiles * per_tile;
+}
+
+// the form of a dense M x N x K launch in nz K-slices of Kc, and the estimate of its time
+static int tile_form(int M, int N, int Kc, int nz, bool hilo, bool paired, bool may256, double* us) {
+  const TileForm* t = hilo ? tile_hilo : tile_plain;
+  const int n = hilo ? (int)(sizeof(tile_hilo) / sizeof(TileForm)) : (int)(sizeof(tile_plain) / sizeof(TileForm));
+  int best = 0;
+  double tb = 1e30;
+  for (int i = 0; i < n; ++i) {
+    if (t[i].form == 0 && !may256) continue;
+    const double e = tile_time(t[i], M, N, Kc / BK, nz, paired);
+    if (e < tb) { tb = e; best = t[i].form; }
+  }
+  if (us) *us = tb;
+  return best;
+}
+
+template <int EPI, int BM, int BN, int WM, int WN, int S, bool HILO>
+static void tile_go(const G256& p, int nz, hipStream_t st) {
+  const dim3 grid((unsigned)(mn_cdiv(p.M, BM) * mn_cdiv(p.N, epi_paired(EPI) ? BN / 2 : BN)), nz);
+  hipLaunchKernelGGL((gemm_tile_kernel<EPI, HILO, BM, BN, WM, WN, S>), grid, dim3(WM * WN * 64), 0, st, p);
+}
+
+// stages: as many K-tiles as leave room for two workgroups of the 64-row forms on a CU (64 x 64 hi/lo: 3 x 24 KiB; 64 x 128: 3 x 24, hi/lo
+// 2 x 32 KiB), all of the LDS for the 128 x 128 form (plain 4 x 32, hi/lo 3 x 48 KiB) and two for its two-per-CU variant; deeper pipelines on
+// fewer workgroups measured slower everywhere (64 x 64: 8 stages 8.1 us against 7.3; 64 x 128: 6 stages 66.8 against 53.4 at 1409 x 8192 x 1024)
+template <int EPI>
+static bool tile_launch(const G256& p, int form, int nz, bool hilo, hipStream_t st) {
+  if (hilo) {
+    switch (form) {
+      case 1: tile_go<EPI, 64, 64, 2, 2, 3, true>(p, nz, st); return true;
+      case 2: tile_go<EPI, 64, 128, 2, 2, 2, true>(p, nz, st); return true;
+      case 3: tile_go<EPI, 128, 128, 2, 4, 3, true>(p, nz, st); return true;
+      default: return false;
+    }
+  }
+  switch (form) {
+    case 1: tile_go<EPI, 64, 64, 2, 2, 4, false>(p, nz, st); return true;
+    case 2: tile_go<EPI, 64, 128, 2, 2, 3, false>(p, nz, st); return true;
+    case 3: tile_go<EPI, 128, 128, 2, 4, 4, false>(p, nz, st); return true;
+    case 4: tile_go<EPI, 128, 128, 2, 2, 2, false>(p, nz, st); return true;
+    default: return false;
+  }
+}
 
 // Generic launcher.  Returns the number of split-K slices used (>= 1) or a negative error.
 static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
@@ -442,8 +515,12 @@ static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
     else hipLaunchKernelGGL((gemm256_kernel<E_SWIGLU_BF16, false, true>), grid, dim3(512), 0, st, p);
     return nz;
   }
+  // (the 256-tile kernel's GELU is the 1.5e-7 polynomial: it serves the problems of 128 tiles and more)
+  const bool may256 = epi != E_BF16_GELU || mn_cdiv(p.M, 256) * mn_cdiv(p.N, 256) >= 128;
+  const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : tile_form(p.M, p.N, p.Kc, nz, hilo, paired, may256, nullptr);
 #define G256_GO(E)                                                                          \
   do {                                                                                      \
+    if (form > 0 && tile_launch<E>(p, form, nz, hilo, st)) break;                           \
     if (hilo) hipLaunchKernelGGL((gemm256_kernel<E, true>), grid, dim3(512), 0, st, p);     \
     else hipLaunchKernelGGL((gemm256_kernel<E, false>), grid, dim3(512), 0, st, p);         \
   } while (0)
@@ -472,6 +549,23 @@ extern "C" int mn_gemm256_ex(const mn_g256* a, int epi, int ksplit, void* stream
   if (nz < 0) return nz;
   MN_CHECK_LAUNCH("mn_gemm256_ex");
   return nz;
+}
+
+// Split-K request for a product whose fp32 slabs the consumer sums anyway (it reads nz slabs of M x N where it read one): the slice count with the
+// least estimated time of the launch plus the slabs' traffic (written once, read once, at 4.5 TB/s).  0: one slice is best.
+// 65 x 1024 x 1024 bf16: 1 slice 7.3 us, 8 slices 4.3; 256 x 1024 x 4096: 18.3 against 7.3; 1025 hi/lo rows x 1024 x 2752: 25.1 against 22.9 for 3.
+extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo) {
+  int best = 0;
+  double tb = 1e30;
+  for (int ks = 1; ks <= 16; ++ks) {
+    const int Kc = ks == 1 ? K : (int)(mn_cdiv(mn_cdiv(K, ks), 2 * BK) * 2 * BK), nz = (int)mn_cdiv(K, Kc);
+    if (nz != ks) continue;
+    double t;
+    tile_form(M, N, Kc, nz, hilo != 0, false, true, &t);
+    t += nz * (double)M * N * 8.0 / 4.5e6;
+    if (t < tb - 1e-9) { tb = t; best = ks; }
+  }
+  return best > 1 ? best : 0;
 }
 
 // slices mn_gemm256_ex will use for a ksplit request (whole pairs of K-tiles per slice)

@@ -1,0 +1,135 @@
+// gemm_tile.inl — the small-tile form of gemm256.hip's GEMM, for problems whose 256 x 256 tiles leave most of the chip idle
+// (included inside gemm256.hip's anonymous namespace; same operands, pairing modes, split-K and epilogues).
+//
+// What bounds such a problem is not the matrix cores but latency: a 256-tile kernel on 36 workgroups (1025 hi/lo rows x 1024 columns) or a
+// two-buffer 128-tile kernel on 24 .. 96 spends its time waiting for one K-tile after another (0.6 .. 1 us each from HBM / L2).  So:
+//   * BM x BN tiles from 64 x 64 to 128 x 128, so that a few hundred workgroups exist;
+//   * S stages of LDS (S - 1 K-tiles in flight per workgroup, filled by global_load_lds, retired by counted vmcnt): the first products wait for
+//     one round trip, the rest stream;
+//   * one barrier per K-tile: it says both that every wave's part of K-tile t has landed and that every wave has read K-tile t - 1, whose
+//     buffer the loads of K-tile t + S - 1 may then overwrite.
+// HILO: the LDS image of a K-tile holds BM hi rows, then the same rows' lo parts; both are multiplied into accumulators of their own (the
+// sum is taken once, in the epilogue, as in the 256-tile kernel).
+template <int N>
+__device__ __forceinline__ void wait_vm_n() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory"); }
+
+// all but `rem` K-tiles of L loads each have landed, and this wave's fragment reads are done (rem <= MAX, wave-uniform)
+template <int L, int MAX>
+__device__ __forceinline__ void wait_tiles(int rem) {
+  if constexpr (MAX == 0) {
+    wait_vm_n<0>();
+  } else {
+    if (rem >= MAX) wait_vm_n<L * MAX>();
+    else wait_tiles<L, MAX - 1>(rem);
+  }
+}
+
+template <int EPI, bool HILO, int BM, int BN, int WM, int WN, int S>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
+  constexpr int NW = WM * WN, AR = HILO ? 2 * BM : BM, QA = AR / 8 / NW, QW = BN / 8 / NW, STAGE = (AR + BN) * 128;
+  constexpr int MI = BM / WM / 16, NJ = BN / WN / 16, AI = HILO ? 2 * MI : MI;
+  constexpr bool paired = epi_paired(EPI);
+  static_assert(QA * 8 * NW == AR && QW * 8 * NW == BN && MI >= 1 && NJ >= (paired ? 2 : 1), "whole instructions and fragments per wave");
+  static_assert((QA + QW) * (S - 2) < 64 && S * STAGE <= 160 * 1024, "vmcnt range, LDS");
+  __shared__ __attribute__((aligned(1024))) char lds[S * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN, fr = lane & 15, fq = lane >> 4;
+  constexpr int cols = paired ? BN / 2 : BN;
+  const int tiles_m = (p.M + BM - 1) / BM;
+  // XCD-aware order: an XCD's tiles are consecutive, row tiles fastest, so each XCD reads its own part of the weights and all of the rows
+  int bid = blockIdx.x;
+  {
+    const int nt = gridDim.x, q = nt / 8, r = nt % 8, xcd = bid % 8, idx = bid / 8;
+    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
+  }
+  const int m0 = (bid % tiles_m) * BM, n0 = (bid / tiles_m) * cols;
+  const int kbeg = blockIdx.y * p.Kc, kend = min(p.K, kbeg + p.Kc);
+  const int nk = (kend - kbeg) / BK;
+
+  // per-lane byte offsets (from A / W) of the row behind each 8-row instruction of this wave, k-slot swizzle folded in
+  uint32_t srcA[QA], srcW[QW];
+  const int rin = lane >> 3;
+#pragma unroll
+  for (int q = 0; q < QA; ++q) {
+    const int L = (wave * QA + q) * 8 + rin;
+    const int gm = min(m0 + (HILO && L >= BM ? L - BM : L), p.M - 1);
+    srcA[q] = (uint32_t)(((int64_t)gm * p.lda + (HILO && L >= BM ? p.a_lo_off : 0) + kbeg) * 2 + (((lane & 7) ^ ((L >> 1) & 7)) << 4));
+  }
+#pragma unroll
+  for (int q = 0; q < QW; ++q) {
+    const int L = (wave * QW + q) * 8 + rin;
+    int gn;
+    if (paired) {                                      // a wave's columns: its gate rows, then the up rows of the same units
+      constexpr int WC = BN / WN, half = WC / 2;
+      const int w = L / WC, r = L % WC;
+      gn = min(n0 + w * half + (r % half), p.N - 1) + (r >= half ? (int)p.w_pair_rows : 0);
+    } else {
+      gn = min(n0 + L, p.N - 1);
+    }
+    srcW[q] = (uint32_t)(((int64_t)gn * p.ldw + kbeg) * 2 + (((lane & 7) ^ ((L >> 1) & 7)) << 4));
+  }
+  const char* Ab = reinterpret_cast<const char*>(p.A);
+  const char* Wb = reinterpret_cast<const char*>(p.W);
+  auto stage = [&](int kt, int buf) {
+    const uint32_t koff = (uint32_t)kt * (BK * 2);
+    char* dst = &lds[buf * STAGE];
+#pragma unroll
+    for (int q = 0; q < QW; ++q)
+      __builtin_amdgcn_global_load_lds((glb_void*)(Wb + (srcW[q] + koff)), (lds_void*)(dst + AR * 128 + (wave * QW + q) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int q = 0; q < QA; ++q)
+      __builtin_amdgcn_global_load_lds((glb_void*)(Ab + (srcA[q] + koff)), (lds_void*)(dst + (wave * QA + q) * 1024), 16, 0, 0);
+  };
+  int lane_off[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) lane_off[kk] = fr * 128 + (((4 * kk + fq) ^ ((fr >> 1) & 7)) << 4);
+  f32x4 acc[AI][NJ];
+#pragma unroll
+  for (int i = 0; i < AI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int t = 0; t < S - 1; ++t)
+    if (t < nk) stage(t, t);
+  int buf = 0, nbuf = S - 1;
+  for (int t = 0; t < nk; ++t) {
+    wait_tiles<QA + QW, S - 2>(nk - 1 - t);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + S - 1 < nk) stage(t + S - 1, nbuf);
+    const char* a = &lds[buf * STAGE + wm * (BM / WM) * 128];
+    const char* w = &lds[buf * STAGE + AR * 128 + wn * (BN / WN) * 128];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      bf16x8 af[AI], wf[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) wf[j] = *reinterpret_cast<const bf16x8*>(w + j * 2048 + lane_off[kk]);
+#pragma unroll
+      for (int i = 0; i < AI; ++i) af[i] = *reinterpret_cast<const bf16x8*>(a + (i < MI ? i * 2048 : BM * 128 + (i - MI) * 2048) + lane_off[kk]);
+#pragma unroll
+      for (int i = 0; i < AI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
+    }
+    buf = buf + 1 == S ? 0 : buf + 1;
+    nbuf = nbuf + 1 == S ? 0 : nbuf + 1;
+  }
+
+  char* Cz = reinterpret_cast<char*>(p.C);
+  if (EPI == E_F32) Cz += (int64_t)blockIdx.y * p.c_zstride * 4;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int m = m0 + wm * (BM / WM) + i * 16 + fr;
+#pragma unroll
+    for (int j = 0; j < (paired ? NJ / 2 : NJ); ++j) {
+      const int n = n0 + wn * (cols / WN) + j * 16 + fq * 4;
+      if (m >= p.M || n >= p.N) continue;              // N % 4 == 0 (host check): the 4 columns are all in or all out
+      f32x4 v = acc[i][j], u = {0.f, 0.f, 0.f, 0.f};
+      if (HILO) v += acc[(i + MI) % AI][j];
+      if (paired) { u = acc[i][(j + NJ / 2) % NJ]; if (HILO) u += acc[(i + MI) % AI][(j + NJ / 2) % NJ]; }
+      g256_emit<EPI, true>(p, Cz, m, n, v, u, blockIdx.y);
+    }
+  }
+}

@@ -79,23 +79,12 @@ __global__ __launch_bounds__(256) void rf_swiglu_slabs_kernel(const float* __res
   *reinterpret_cast<u2*>(yr + lo_off) = u2{l0, l1};
 }
 
-// Split-K request of a hi/lo GEMM with `rows` rows: minimise a small cost model of the launch — rounds of workgroups over the
-// 256 CUs x (K-tiles per slice at ~1.9 us each + ~10 us of prologue / epilogue) + the fp32 slab round trip through HBM
-// (written by the GEMM, read by the consumer) — over the slice counts that keep >= 4 K-tiles per slice.  E.g. RF w3
-// (N = 3072, K = 8192): 1024 rows -> 96 tiles -> 2 slices (192 workgroups, one round); 1536 rows -> 144 tiles -> 3 slices
-// (432 workgroups, two rounds of 43 K-tiles instead of one round of 128 on 56 % of the chip).
+// Split-K request of a hi/lo GEMM with `rows` rows whose consumer sums the fp32 slabs (gemm256.hip's estimate of launch + slab traffic).
+// E.g. RF w3 (N = 3072, K = 8192) at 1536 rows: 144 tiles -> 3 slices (432 workgroups, two rounds of 43 K-tiles instead of one round of 128 on
+// 56 % of the chip).
 static int rf_wide_ksplit(int rows, int N, int K) {
-  const double tiles = (double)(mn_cdiv(rows, 128) * mn_cdiv(N, 256));
-  const int kt = K / 64;
-  int best = 1;
-  double best_cost = 1e30;
-  for (int ks = 1; ks <= 16 && kt / ks >= 4; ++ks) {
-    const double rounds = (double)mn_cdiv((int64_t)(tiles * ks), 256);
-    const double slabs = ks > 1 ? (double)ks * rows * N * 8.0 / 4.0e6 : 0.0;      // us at ~4 TB/s, write + read
-    const double cost = rounds * ((double)mn_cdiv(kt, ks) * 1.9 + 10.0) + slabs;
-    if (cost < best_cost) { best_cost = cost; best = ks; }
-  }
-  return best;
+  const int ks = mn_gemm256_plan_ksplit(rows, N, K, 1);
+  return ks > 1 ? ks : 1;
 }
 
 // the fp8-MFMA regime of the wide route (mn_rf_head.arith; mingnative.h section 8): e4m3 weights present, widths in whole 128-k tiles

@@ -118,7 +118,7 @@ class MingTok:
                 li = int(prefix.rsplit(".", 1)[1])
                 w12, b12, w3 = self._sem_pad[0][li], self._sem_pad[1][li], self._sem_pad[2][li]
             hid = w12.shape[0] // 2
-            if x.shape[0] >= 1024 and hid % 4 == 0 and D % 64 == 0:
+            if hid % 4 == 0 and D % 64 == 0:
                 h = ops.gemm256_swiglu(xn, w12, b12)                 # SwiGLU in the GEMM epilogue: no [M, 2*hidden] round trip
             else:
                 h = ops.swiglu_bf16(ops.gemm_bf16(xn, w12, b12))

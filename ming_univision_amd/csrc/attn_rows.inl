@@ -1,0 +1,452 @@
+// attn_rows.inl — attention of runs of rows on the fp32 matrix cores (included inside pmix_ops.hip's anonymous namespace).
+//
+// v_mfma_f32_16x16x4_f32: scores, weights and sums stay 32-bit.  What bounds it is the fp32 MFMA rate (157 TFLOP/s); everything else is laid out so
+// that the products can follow each other.  A workgroup of 4 waves owns up to 64 query vectors of one key/value head — `hv` heads of 64 / hv
+// rows, gathered from consecutive runs of the table — so a staged key tile serves 64 vectors.  (One run of 4 rows x 4 heads per
+// workgroup, the form before, re-read every key for 16 vectors and put four barriers around every 16 keys: 27 TFLOP/s.)
+// Both kernels multiply transposed, S^T[key, q] = K Q^T and O^T[d, q] += V^T P^T: a lane's four scores of a 16-key fragment are exactly the B
+// operand of the value products of those keys (k slot g of step i = key 4 g + i), so the softmax of a query is four registers x two lane
+// swaps and the weights never leave the registers.  Keys and values go HBM -> registers -> one of two LDS tiles while the other is multiplied.
+// Runs of several sequences in one workgroup are walked one sequence after the other; a tile that none of the queries sees is skipped, one that
+// all of them see whole takes no mask arithmetic.  Key splits write the partial layout of the merge kernel, run by run.
+
+// The order of the workgroups: long walks (late rows) first, the next 256 the other way round, so that the two workgroups a CU holds are a long
+// and a short one.
+__device__ __forceinline__ int rows_group() {
+  const int first = (int)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x);        // of this (head, split): one direction for all of its groups
+  return ((first >> 8) & 1) ? (int)blockIdx.x : (int)(gridDim.x - 1 - blockIdx.x);
+}
+
+// the workgroup's runs: first row, rows, cache sequence, first position
+__device__ __forceinline__ void rows_table(const AttnTArgs& a, int b0, int nb, int nbw, int tid, int (*tab)[4]) {
+  if (tid < nbw) {
+    const bool in = tid < nb;
+    const int r = in ? a.blk_tab[2 * (b0 + tid)] : 0;
+    tab[tid][0] = r;
+    tab[tid][1] = in ? min(a.blk_tab[2 * (b0 + tid) + 1], a.rows_per_blk) : 0;
+    tab[tid][2] = in ? a.row_seq[r] : -1;
+    tab[tid][3] = in ? a.row_slot[r] : 0;
+  }
+  __syncthreads();
+}
+
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));      // rows start at any float: a 16-byte load needs 4-byte alignment here
+
+// four consecutive values src[d .. d + 3], zero from n on (VEC: n is a multiple of 4)
+template <bool VEC>
+__device__ __forceinline__ f32x4 load4(const float* src, int d, int n, bool on) {
+  f32x4 t;
+  if (VEC) {
+    t = *reinterpret_cast<const f32x4u*>(src + (d < n ? d : 0));
+    return on && d < n ? t : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float x = src[d + e < n ? d + e : 0];
+    t[e] = on && d + e < n ? x : 0.f;
+  }
+  return t;
+}
+
+// 16 rows x 64 NBW floats HBM -> registers (raw: a select on a loaded value would wait for it here) and registers -> LDS (zero from n on and in
+// rows that do not count): 16 threads per row, 16 bytes per thread and pass
+template <int NBW, bool VEC>
+__device__ __forceinline__ void rows_fetch(f32x4 (&v)[NBW], const float* src, int n, int cg) {
+#pragma unroll
+  for (int ps = 0; ps < NBW; ++ps) {
+    const int d = 4 * (cg + 16 * ps);
+    if (VEC) {
+      v[ps] = *reinterpret_cast<const f32x4u*>(src + (d < n ? d : 0));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[ps][e] = src[d + e < n ? d + e : 0];
+    }
+  }
+}
+template <int NBW, int LDC, bool VEC>
+__device__ __forceinline__ void rows_put(float* __restrict__ dst, const f32x4 (&v)[NBW], int n, int j, int cg, bool ok) {
+#pragma unroll
+  for (int ps = 0; ps < NBW; ++ps) {
+    const int d = 4 * (cg + 16 * ps);
+    f32x4 t = v[ps];
+    if (VEC) {
+      if (!(ok && d < n)) t = f32x4{0.f, 0.f, 0.f, 0.f};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!(ok && d + e < n)) t[e] = 0.f;
+    }
+    *reinterpret_cast<f32x4*>(dst + j * LDC + d) = t;
+  }
+}
+
+// values d .. d + 3 of one query vector's result
+__device__ __forceinline__ void emit4(const AttnTArgs& a, f32x4 v, int row, int64_t col0, int d, bool vec) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (d + e < a.vdim) v[e] = gated(a, v[e], row, col0 + d + e);
+  if (vec) {
+    if (a.out) *reinterpret_cast<f32x4*>(a.out + (int64_t)row * a.ldo + col0 + d) = v;
+    if (a.out16) *reinterpret_cast<uint2*>(a.out16 + (int64_t)row * a.ldo16 + col0 + d) = uint2{cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3])};
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (d + e >= a.vdim) continue;
+    if (a.out) a.out[(int64_t)row * a.ldo + col0 + d + e] = v[e];
+    if (a.out16) a.out16[(int64_t)row * a.ldo16 + col0 + d + e] = f32_to_bf16(v[e]);
+  }
+}
+__device__ __forceinline__ bool emit_vec(const AttnTArgs& a) {
+  return (a.vdim & 3) == 0 && (!a.out || ((a.ldo & 3) == 0 && ((uintptr_t)a.out & 15) == 0)) &&
+         (!a.out16 || ((a.ldo16 & 3) == 0 && ((uintptr_t)a.out16 & 7) == 0));
+}
+
+// Keys and values in arenas of their own, heads of up to 256 values: each wave owns 16 of the 64 vectors with all their dims, queries in registers.
+// K is read 16 bytes at a time (a lane's k slot = dims 16 it + 4 g .. + 3 over four steps, one accumulator per step: four short chains sum more
+// exactly than one long one), V likewise (row c of value fragment 4 vb + e = column 64 vb + 4 c + e); with row strides of 4 mod 64 floats
+// both reads touch every bank once.  One LDS-only barrier per tile.
+// 2048 tokens, 16 heads of 128 over 4 key/value heads (17.2 GF): 632 us in the form before, 211 us here (82 TFLOP/s).
+// VEC: dim and vdim are multiples of 4.
+template <int NBD, int NBV, bool VEC>
+__global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_blk, int hv) {
+  constexpr int KT = NBD + NBV > 4 ? 16 : 32, KF = KT / 16, AQ = 16, LDK = 64 * NBD + 4, LDV = 64 * NBV + 4, TILE = KT * (LDK + LDV);
+  __shared__ __attribute__((aligned(16))) float lds[2 * TILE];        // [2][K tile | V tile]
+  __shared__ int tab[16][4];
+  const int tid = threadIdx.x, gy = blockIdx.y, sp = blockIdx.z;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, g4 = lane >> 4;
+  const int rep = a.H / a.G, chunks = (rep + a.hpc - 1) / a.hpc;
+  const int g = gy / chunks, h0 = g * rep + (gy % chunks) * a.hpc;
+  const int Rc = min(a.hpc, g * rep + rep - h0);
+  const int rw = 16 / hv, nbw = rw * 4 / a.rows_per_blk;                // rows per wave; runs per workgroup
+  const int b0 = rows_group() * nbw, nb = min(nbw, n_blk - b0);
+  rows_table(a, b0, nb, nbw, tid, tab);
+  // this lane's query: column c of the wave's 16
+  const int slot = wave * rw + c / hv, hc = c % hv, run = slot / a.rows_per_blk, rin = slot % a.rows_per_blk;
+  const bool valid = rin < tab[run][1] && hc < Rc;
+  const int row = valid ? tab[run][0] + rin : 0, pos = tab[run][3] + rin;
+  f32x4 q[4 * NBD];
+  {
+    const float* src = a.q + (int64_t)row * a.ldq + (int64_t)(h0 + (valid ? hc : 0)) * a.dim;
+#pragma unroll
+    for (int it = 0; it < 4 * NBD; ++it) q[it] = load4<VEC>(src, 16 * it + 4 * g4, a.dim, valid);
+  }
+  const int Gd = a.G * a.dim, Gv = a.G * a.vdim;
+  for (int s0 = 0; s0 < nb;) {
+    // ---- the runs [s0, s1) of one cache sequence, the keys they see between them ----
+    const int seq = tab[s0][2];
+    int s1 = s0, tF = 0x7fffffff, posL = -1;
+    for (; s1 < nb && tab[s1][2] == seq; ++s1) {
+      tF = min(tF, first_key(a, tab[s1][3]));
+      posL = max(posL, tab[s1][3] + tab[s1][1] - 1);
+    }
+    const int nbL = win_nb(posL, a.window, a.pool), nk = nbL + (posL - tF + 1);
+    const int ntile = (nk + KT - 1) / KT, tps = (ntile + a.nsplit - 1) / a.nsplit;
+    const int t0 = sp * tps, t1 = min(ntile, t0 + tps);
+    const bool mine = valid && run >= s0 && run < s1;
+    // what this lane's query sees: token keys [lo, hi] (as key indices of the walk) and the first my_nb block means
+    const int my_nb = mine ? win_nb(pos, a.window, a.pool) : 0;
+    const int lo = mine ? nbL + first_key(a, pos) - tF : 0x7fffffff, hi = mine ? nbL + pos - tF : -1;
+    int w_lo = lo, w_hi = hi, w_nb = my_nb, w_lo_all = mine ? lo : -1, w_hi_all = mine ? hi : 0x7fffffff;      // over the wave's queries
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) {
+      w_lo = min(w_lo, __shfl_xor(w_lo, o)); w_hi = max(w_hi, __shfl_xor(w_hi, o)); w_nb = max(w_nb, __shfl_xor(w_nb, o));
+      w_lo_all = max(w_lo_all, __shfl_xor(w_lo_all, o)); w_hi_all = min(w_hi_all, __shfl_xor(w_hi_all, o));
+    }
+    w_lo = __builtin_amdgcn_readfirstlane(w_lo); w_hi = __builtin_amdgcn_readfirstlane(w_hi); w_nb = __builtin_amdgcn_readfirstlane(w_nb);
+    w_lo_all = __builtin_amdgcn_readfirstlane(w_lo_all); w_hi_all = __builtin_amdgcn_readfirstlane(w_hi_all);
+    const float* kb = a.k + ((int64_t)seq * a.t_max + tF) * a.ldk + (int64_t)g * a.dim;
+    const float* vb_ = a.v + ((int64_t)seq * a.t_max + tF) * a.ldv + (int64_t)g * a.vdim;
+    const float* pkb = a.pk ? a.pk + (int64_t)seq * a.n_pool_max * Gd + (int64_t)g * a.dim : nullptr;
+    const float* pvb = a.pv ? a.pv + (int64_t)seq * a.n_pool_max * Gv + (int64_t)g * a.vdim : nullptr;
+    f32x4 vk[KF][NBD], vv[KF][NBV];
+    const int fj = tid >> 4, fc = tid & 15;
+    auto fetch = [&](int tile) {
+#pragma unroll
+      for (int f = 0; f < KF; ++f) {
+        const int jj = min(tile * KT + 16 * f + fj, nk - 1);
+        rows_fetch<NBD, VEC>(vk[f], jj < nbL ? pkb + (int64_t)jj * Gd : kb + (int64_t)(jj - nbL) * a.ldk, a.dim, fc);
+        rows_fetch<NBV, VEC>(vv[f], jj < nbL ? pvb + (int64_t)jj * Gv : vb_ + (int64_t)(jj - nbL) * a.ldv, a.vdim, fc);
+      }
+    };
+    auto put = [&](int tile, int buf) {
+      float* K = lds + buf * TILE;
+#pragma unroll
+      for (int f = 0; f < KF; ++f) {
+        const bool ok = tile * KT + 16 * f + fj < nk;
+        rows_put<NBD, LDK, VEC>(K + 16 * f * LDK, vk[f], a.dim, fj, fc, ok);
+        rows_put<NBV, LDV, VEC>(K + KT * LDK + 16 * f * LDV, vv[f], a.vdim, fj, fc, ok);
+      }
+    };
+    float mrun = -INFINITY, lrun = 0.f;                // lrun: this lane's keys only
+    f32x4 acc[4 * NBV];
+#pragma unroll
+    for (int x = 0; x < 4 * NBV; ++x) acc[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (t0 < t1) { fetch(t0); put(t0, 0); }
+    if (t0 + 1 < t1) fetch(t0 + 1);
+    lds_barrier();
+    for (int tile = t0; tile < t1; ++tile) {
+      const int key0 = tile * KT, cur = (tile - t0) & 1;
+      const float* K = lds + cur * TILE;
+      const float* V = K + KT * LDK;
+      if ((key0 <= w_hi && key0 + KT - 1 >= w_lo) || key0 < w_nb) {      // wave-uniform
+        f32x4 s[KF], se[KF][4];
+#pragma unroll
+        for (int f = 0; f < KF; ++f)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) se[f][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int it = 0; it < 4 * NBD; ++it) {
+          f32x4 kf[KF];
+#pragma unroll
+          for (int f = 0; f < KF; ++f) kf[f] = *reinterpret_cast<const f32x4*>(K + (16 * f + c) * LDK + 16 * it + 4 * g4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int f = 0; f < KF; ++f) se[f][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[f][e], q[it][e], se[f][e], 0, 0, 0);
+        }
+#pragma unroll
+        for (int f = 0; f < KF; ++f) s[f] = (se[f][0] + se[f][1]) + (se[f][2] + se[f][3]);
+        if (a.cap > 0.f) {
+#pragma unroll
+          for (int f = 0; f < KF; ++f)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[f][i] = soft_cap(s[f][i], a.cap);
+        }
+        if (!(key0 >= nbL && key0 >= w_lo_all && key0 + KT - 1 <= w_hi_all)) {
+#pragma unroll
+          for (int f = 0; f < KF; ++f)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int j = key0 + 16 * f + 4 * g4 + i;
+              const bool see = ((j < nbL) & (j < my_nb)) | ((j >= lo) & (j <= hi));      // (lo >= nbL)
+              s[f][i] = see ? s[f][i] : -INFINITY;
+            }
+        }
+        float mx = fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3]));
+#pragma unroll
+        for (int f = 1; f < KF; ++f) mx = fmaxf(mx, fmaxf(fmaxf(s[f][0], s[f][1]), fmaxf(s[f][2], s[f][3])));
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float mnew = fmaxf(mrun, mx);
+        const float corr = mrun == -INFINITY ? 0.f : fast_exp(mrun - mnew);
+        float sum = 0.f;
+#pragma unroll
+        for (int f = 0; f < KF; ++f)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            s[f][i] = s[f][i] == -INFINITY ? 0.f : fast_exp(s[f][i] - mnew);
+            sum += s[f][i];
+          }
+        lrun = lrun * corr + sum;
+        if (__ballot(mnew != mrun)) {                  // some query's maximum moved
+#pragma unroll
+          for (int x = 0; x < 4 * NBV; ++x) acc[x] *= corr;
+        }
+        mrun = mnew;
+#pragma unroll
+        for (int f = 0; f < KF; ++f)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int vb = 0; vb < NBV; ++vb) {
+              const f32x4 v4 = *reinterpret_cast<const f32x4*>(V + (16 * f + 4 * g4 + i) * LDV + 64 * vb + 4 * c);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[4 * vb + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[e], s[f][i], acc[4 * vb + e], 0, 0, 0);
+            }
+      }
+      if (tile + 1 < t1) put(tile + 1, cur ^ 1);       // the other tile was last read before the previous barrier
+      if (tile + 2 < t1) fetch(tile + 2);
+      lds_barrier();
+    }
+    lrun += __shfl_xor(lrun, 16);
+    lrun += __shfl_xor(lrun, 32);
+    if (mine) {
+      const int qv = rin * Rc + hc;                    // the vector's place in its run's partial slab
+      float* part = a.nsplit > 1 ? a.part + (((int64_t)(b0 + run) * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)AQ * (2 + a.vdim)) : nullptr;
+      const int64_t col0 = (int64_t)(h0 + hc) * a.vdim;
+      const float inv = part ? 1.f : a.out_scale * softmax_inv(mrun, lrun, a.sink, h0 + hc);
+      const bool vec = emit_vec(a);
+#pragma unroll
+      for (int vb = 0; vb < NBV; ++vb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int d = 64 * vb + 4 * (4 * g4 + i);
+          if (d >= a.vdim) continue;
+          const f32x4 r = f32x4{acc[4 * vb][i], acc[4 * vb + 1][i], acc[4 * vb + 2][i], acc[4 * vb + 3][i]} * inv;
+          if (!part) { emit4(a, r, row, col0, d, vec); continue; }
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (d + e < a.vdim) part[2 * AQ + (int64_t)qv * a.vdim + d + e] = r[e];
+        }
+      if (part && g4 == 0) { part[qv] = mrun; part[AQ + qv] = lrun; }
+    }
+    s0 = s1;
+  }
+}
+
+// Latent attention (one key/value head whose values are the first columns of the keys, up to 640 of them): vectors with all their dims do not
+// fit a wave's registers, so every wave takes all of a workgroup's 32 vectors with a quarter of the dims (queries in registers) and, for the
+// values, a quarter of the columns.  The four partial score tiles meet in LDS, each wave sums them and takes the same softmax: 144 MFMAs of
+// 32 cycles per wave and 16-key tile at 576 + 512 values stand against three barriers, and two or three workgroups share a CU.  (64 vectors
+// at 512 registers and one wave per SIMD: 1450 us on the case below, nothing covers the barriers and 129 registers spill.)
+// 2048 tokens, 16 heads, keys of 576 and values of 512, window 1024 (54.8 GF): 1674 us in the form before, 746 us here.
+template <int NB, bool VEC>
+__global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, int n_blk, int hv) {
+  constexpr int KT = 16, AQ = 16, QF = 2, LDK = 64 * NB + 4, LDS_S = 20;
+  __shared__ __attribute__((aligned(16))) float K[KT * LDK];
+  __shared__ __attribute__((aligned(16))) float Sp[4][16 * QF * LDS_S];     // [wave][query][16 keys]: partial scores
+  __shared__ int tab[16][4];
+  const int tid = threadIdx.x, gy = blockIdx.y, sp = blockIdx.z;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, g4 = lane >> 4;
+  const int rep = a.H / a.G, h0 = gy * a.hpc;
+  const int Rc = min(a.hpc, rep - h0);
+  const int rf = 16 / hv, nbw = rf * QF / a.rows_per_blk;               // rows per 16-vector fragment; runs per workgroup
+  const int b0 = rows_group() * nbw, nb = min(nbw, n_blk - b0);
+  rows_table(a, b0, nb, nbw, tid, tab);
+  const int hc = c % hv, dw = wave * 16 * NB;                           // this wave's dims: dw .. dw + 16 NB - 1
+  int row[QF], pos[QF], run[QF];
+  f32x4 q[QF][NB];
+#pragma unroll
+  for (int f = 0; f < QF; ++f) {
+    const int slot = f * rf + c / hv, rin = slot % a.rows_per_blk;
+    run[f] = slot / a.rows_per_blk;
+    const bool valid = rin < tab[run[f]][1] && hc < Rc;
+    row[f] = valid ? tab[run[f]][0] + rin : -1;
+    pos[f] = tab[run[f]][3] + rin;
+    const float* src = a.q + (int64_t)max(row[f], 0) * a.ldq + (int64_t)(h0 + (valid ? hc : 0)) * a.dim;
+#pragma unroll
+    for (int it = 0; it < NB; ++it) q[f][it] = load4<VEC>(src, dw + 16 * it + 4 * g4, a.dim, valid);
+  }
+  for (int s0 = 0; s0 < nb;) {
+    const int seq = tab[s0][2];
+    int s1 = s0, tF = 0x7fffffff, posL = -1;
+    for (; s1 < nb && tab[s1][2] == seq; ++s1) {
+      tF = min(tF, first_key(a, tab[s1][3]));
+      posL = max(posL, tab[s1][3] + tab[s1][1] - 1);
+    }
+    const int nk = posL - tF + 1;
+    const int ntile = (nk + KT - 1) / KT, tps = (ntile + a.nsplit - 1) / a.nsplit;
+    const int t0 = sp * tps, t1 = min(ntile, t0 + tps);
+    int lo[QF], hi[QF], lo_all = -1, hi_all = 0x7fffffff;
+#pragma unroll
+    for (int f = 0; f < QF; ++f) {
+      const bool mine = row[f] >= 0 && run[f] >= s0 && run[f] < s1;
+      lo[f] = mine ? first_key(a, pos[f]) - tF : 0x7fffffff;
+      hi[f] = mine ? pos[f] - tF : -1;
+      if (mine) { lo_all = max(lo_all, lo[f]); hi_all = min(hi_all, hi[f]); }
+    }
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) { lo_all = max(lo_all, __shfl_xor(lo_all, o)); hi_all = min(hi_all, __shfl_xor(hi_all, o)); }
+    lo_all = __builtin_amdgcn_readfirstlane(lo_all); hi_all = __builtin_amdgcn_readfirstlane(hi_all);
+    const float* kb = a.k + ((int64_t)seq * a.t_max + tF) * a.ldk;
+    f32x4 vk[NB];
+    const int fj = tid >> 4, fc = tid & 15;
+    auto fetch = [&](int tile) { rows_fetch<NB, VEC>(vk, kb + (int64_t)min(tile * KT + fj, nk - 1) * a.ldk, a.dim, fc); };
+    auto put = [&](int tile) { rows_put<NB, LDK, VEC>(K, vk, a.dim, fj, fc, tile * KT + fj < nk); };
+    float mrun[QF], lrun[QF];
+    f32x4 acc[QF][NB];
+#pragma unroll
+    for (int f = 0; f < QF; ++f) {
+      mrun[f] = -INFINITY;
+      lrun[f] = 0.f;
+#pragma unroll
+      for (int x = 0; x < NB; ++x) acc[f][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (t0 < t1) fetch(t0);
+    for (int tile = t0; tile < t1; ++tile) {
+      const int key0 = tile * KT;
+      lds_barrier();                                   // the previous tile's values and partial scores are read
+      put(tile);
+      if (tile + 1 < t1) fetch(tile + 1);              // in flight while this tile is multiplied
+      lds_barrier();
+      {                                                // partial scores over this wave's dims, two chains each
+        f32x4 s[QF][2];
+#pragma unroll
+        for (int f = 0; f < QF; ++f) s[f][0] = s[f][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int it = 0; it < NB; ++it) {
+          const f32x4 kf = *reinterpret_cast<const f32x4*>(K + c * LDK + dw + 16 * it + 4 * g4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int f = 0; f < QF; ++f) s[f][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], q[f][it][e], s[f][e & 1], 0, 0, 0);
+        }
+#pragma unroll
+        for (int f = 0; f < QF; ++f) *reinterpret_cast<f32x4*>(&Sp[wave][(16 * f + c) * LDS_S + 4 * g4]) = s[f][0] + s[f][1];
+      }
+      lds_barrier();
+      const bool whole = key0 >= lo_all && key0 + KT - 1 <= hi_all;
+      f32x4 p[QF];
+#pragma unroll
+      for (int f = 0; f < QF; ++f) {
+        const int o = (16 * f + c) * LDS_S + 4 * g4;
+        f32x4 s = (*reinterpret_cast<const f32x4*>(&Sp[0][o]) + *reinterpret_cast<const f32x4*>(&Sp[1][o])) +
+                  (*reinterpret_cast<const f32x4*>(&Sp[2][o]) + *reinterpret_cast<const f32x4*>(&Sp[3][o]));
+        if (a.cap > 0.f) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[i] = soft_cap(s[i], a.cap);
+        }
+        if (!whole) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int j = key0 + 4 * g4 + i;
+            s[i] = ((j < lo[f]) | (j > hi[f])) ? -INFINITY : s[i];
+          }
+        }
+        float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float mnew = fmaxf(mrun[f], mx);
+        const float corr = mrun[f] == -INFINITY ? 0.f : fast_exp(mrun[f] - mnew);
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          p[f][i] = s[i] == -INFINITY ? 0.f : fast_exp(s[i] - mnew);
+          sum += p[f][i];
+        }
+        lrun[f] = lrun[f] * corr + sum;
+        if (__ballot(mnew != mrun[f])) {
+#pragma unroll
+          for (int x = 0; x < NB; ++x) acc[f][x] *= corr;
+        }
+        mrun[f] = mnew;
+      }
+      // value fragment x of this wave: columns 16 (wave + 4 x) + c
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float v[NB];
+#pragma unroll
+        for (int x = 0; x < NB; ++x) v[x] = K[(4 * g4 + i) * LDK + 16 * (wave + 4 * x) + c];
+#pragma unroll
+        for (int x = 0; x < NB; ++x)
+#pragma unroll
+          for (int f = 0; f < QF; ++f) acc[f][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[x], p[f][i], acc[f][x], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);             // (all four steps' reads at once would not fit the registers)
+      }
+    }
+    const bool vec = emit_vec(a);
+#pragma unroll
+    for (int f = 0; f < QF; ++f) {
+      lrun[f] += __shfl_xor(lrun[f], 16);
+      lrun[f] += __shfl_xor(lrun[f], 32);
+      if (hi[f] < 0) continue;                         // not of this sequence
+      const int qv = (row[f] - tab[run[f]][0]) * Rc + hc;
+      float* part = a.nsplit > 1 ? a.part + (((int64_t)(b0 + run[f]) * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)AQ * (2 + a.vdim)) : nullptr;
+      const int64_t col0 = (int64_t)(h0 + hc) * a.vdim;
+      const float inv = part ? 1.f : a.out_scale * softmax_inv(mrun[f], lrun[f], a.sink, h0 + hc);
+#pragma unroll
+      for (int x = 0; x < NB; ++x) {
+        const int d = 16 * (wave + 4 * x) + 4 * g4;
+        if (d >= a.vdim) continue;
+        const f32x4 r = acc[f][x] * inv;
+        if (!part) { emit4(a, r, row[f], col0, d, vec); continue; }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (d + e < a.vdim) part[2 * AQ + (int64_t)qv * a.vdim + d + e] = r[e];
+      }
+      if (part && wave == 0 && g4 == 0) { part[qv] = mrun[f]; part[AQ + qv] = lrun[f]; }
+    }
+    s0 = s1;
+  }
+}

@@ -96,7 +96,7 @@ HPlan make_plan(const mn_hyb_model* m, int M) {
     if (d.n_gate > p.gate) p.gate = d.n_gate;
     if (d.n_beta > p.beta) p.beta = d.n_beta;
     if (l.kind == MN_HYB_ATTENTION) {
-      const size_t aw = (size_t)4 * mn_num_cus() * 16 * (2 + (size_t)l.vdim) * sizeof(float);
+      const size_t aw = (size_t)4 * mn_num_cus() * 64 * (2 + (size_t)l.vdim) * sizeof(float);
       if (aw > p.attn_ws) p.attn_ws = aw;
     } else if (l.kind == MN_HYB_TALK_ATTENTION) {                // (runs x splits) of a launch stay near two workgroups per compute unit
       const size_t aw = mn_talk_attn_workspace_bytes(mn_num_cus(), l.heads, l.kv_heads, l.dim, M > 1 && m->block_rows > 0 ? m->block_rows : 1, 2);

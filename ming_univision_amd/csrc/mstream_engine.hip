@@ -64,8 +64,8 @@ MPlan make_plan(const mn_ms_model* m, int M) {
     const MDims d = mdims(l);
     up(p.n_in, d.n_in); up(p.cq, d.cq); up(p.cv, d.cv); up(p.hv, d.hv); up(p.n_router, d.n_router);
     if (l.experts > 0) { up(p.top, l.top); up(p.ff, l.expert_ff); up(p.experts, l.experts); }
-    // key splits are chosen so that a launch has about two workgroups per compute unit: (runs x heads x splits) stays below four
-    const size_t aw = (size_t)4 * mn_num_cus() * 16 * (2 + (size_t)l.vdim) * sizeof(float);
+    // key splits are chosen so that a launch has about two workgroups per compute unit: (workgroups of 64 query vectors x splits) stays below four
+    const size_t aw = (size_t)4 * mn_num_cus() * 64 * (2 + (size_t)l.vdim) * sizeof(float);
     if (aw > p.attn_ws) p.attn_ws = aw;
     if (m->arith == MN_SEQ_ARITH_BF16 && M > 8 && M <= 64) {       // scratch of the weight-streaming MFMA route: the largest product of the stack
       const int W = m->width;

@@ -59,8 +59,8 @@ PPlan make_plan(const mn_pmix_model* m, int M) {
     if (l.top > p.top) p.top = l.top;
     if (l.ff > p.ff) p.ff = l.ff;
     if (l.experts > p.experts) p.experts = l.experts;
-    // key splits are chosen so that a launch has about two workgroups per compute unit: (runs x heads x splits) stays below four
-    const size_t aw = (size_t)4 * mn_num_cus() * 16 * (2 + (size_t)l.vdim) * sizeof(float);
+    // key splits are chosen so that a launch has about two workgroups per compute unit: (workgroups of 64 query vectors x splits) stays below four
+    const size_t aw = (size_t)4 * mn_num_cus() * 64 * (2 + (size_t)l.vdim) * sizeof(float);
     if (aw > p.attn_ws) p.attn_ws = aw;
     const size_t gw = mn_mingru_scan_workspace_bytes(M, l.gru);
     if (gw > p.gru_ws) p.gru_ws = gw;

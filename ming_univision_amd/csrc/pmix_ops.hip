@@ -709,43 +709,36 @@ __global__ __launch_bounds__(256) void window_attn_tiled_kernel(AttnTArgs a) {
   }
 }
 
-// Attention on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: scores and weights stay 32-bit), for runs of rows.  A workgroup of
-// 4 waves owns the same 16 query vectors as the tiled form (<= 4 rows x <= 4 heads of one key/value head) and walks its keys —
-// block means, then tokens — in tiles of 16, keys AND values staged through registers into LDS while the previous tile is multiplied:
+// Latent attention of decode rows on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: scores and weights stay 32-bit): the values are the first
+// columns of the keys (one key/value head whose value arena is a view of the key arena).  Workgroup b of 4 waves takes row b and up to
+// 16 of its query heads and walks the row's keys in tiles of 16, staged through registers into LDS while the previous tile is multiplied:
 //   scores   S[16 q, 16 keys] = Q K^T: every wave multiplies its quarter of the head's values (its slice of Q stays in registers),
 //            the partial tiles are summed through LDS, so all four waves hold the same scores, apply the same per-(row, key)
 //            visibility and keep the same running maximum / sum
-//   values   O[16 q, vdim] += P V: the weights go through LDS into the A-operand layout, wave w owns the 16-column blocks w, w + 4, ..
-// NBD / NBV: 64-value blocks of a key / a value (zero padded).  Key splits write the same partial layout as the tiled form.
-// VK: the values are the first columns of the keys (one key/value head whose value arena is a view of the key arena — latent
-// attention): the staged key tile serves both products and no value tile is loaded; NBV <= NBD.  Without a table of runs (decode
-// rows) workgroup b takes row b and its up to 16 query heads.
-template <int NBD, int NBV, bool VK = false>
+//   values   O[16 q, vdim] += P V from the same staged tile: the weights go through LDS into the A-operand layout, wave w owns the 16-column
+//            blocks w, w + 4, ..
+// NBD: 64-value blocks of a key (zero padded).  Key splits write the same partial layout as the tiled form.  (Runs of rows: attn_rows.inl.)
+template <int NBD>
 __global__ __launch_bounds__(256) void window_attn_mfma_kernel(AttnTArgs a) {
-  constexpr int KT = 16, LDP = 20, LDS_S = 17, DP = 64 * NBD, VP = 64 * NBV, LDK = DP + 4, LDV = VK ? LDK : VP + 4, DQ = DP / 4, AQ = 16;
+  constexpr int NBV = NBD, KT = 16, LDP = 20, LDS_S = 17, DP = 64 * NBD, LDK = DP + 4, LDV = LDK, DQ = DP / 4, AQ = 16;
   extern __shared__ float lds[];
   const int tid = threadIdx.x, b = blockIdx.x, gy = blockIdx.y, sp = blockIdx.z;
   const int rep = a.H / a.G, chunks = (rep + a.hpc - 1) / a.hpc;
   const int g = gy / chunks, h0 = g * rep + (gy % chunks) * a.hpc;
   const int Rc = min(a.hpc, g * rep + rep - h0);
-  const int r0 = a.blk_tab ? a.blk_tab[2 * b] : b;
-  const int nr = a.blk_tab ? min(a.blk_tab[2 * b + 1], a.rows_per_blk) : 1;
-  const int nqv = nr * Rc;
-  const int seq = a.row_seq[r0], pos0 = a.row_slot[r0], posL = pos0 + nr - 1;
-  const int nbL = win_nb(posL, a.window, a.pool), tF = first_key(a, pos0);
-  const int nk = nbL + (posL - tF + 1);
+  const int nqv = Rc, seq = a.row_seq[b], pos = a.row_slot[b], tF = first_key(a, pos);
+  const int nk = pos - tF + 1;
   const int ntile = (nk + KT - 1) / KT, tps = (ntile + a.nsplit - 1) / a.nsplit;
   const int t0 = sp * tps, t1 = min(ntile, t0 + tps);
   float* Kl = lds;                       // [16 keys][LDK]
-  float* Vl = VK ? Kl : Kl + KT * LDK;   // [16 keys][LDV]
-  float* Sp = VK ? Kl + KT * LDK : Vl + KT * LDV;   // [4 waves][16 q][LDS_S] partial scores
+  float* Sp = Kl + KT * LDK;             // [4 waves][16 q][LDS_S] partial scores
   float* Pl = Sp + 4 * 16 * LDS_S;       // [16 q][LDP] weights
   const int wave = tid >> 6, lane = tid & 63, c16 = lane & 15, g4 = lane >> 4;
   // the A operands of this wave's score products stay in registers for the whole key walk: query c16, values wave DQ + 4 it + g4
   float qreg[DQ / 4];
   {
     const int qv = min(c16, nqv - 1);
-    const float* src = a.q + (int64_t)(r0 + qv / Rc) * a.ldq + (int64_t)(h0 + qv % Rc) * a.dim;
+    const float* src = a.q + (int64_t)b * a.ldq + (int64_t)(h0 + qv) * a.dim;
 #pragma unroll
     for (int it = 0; it < DQ / 4; ++it) {
       const int d = wave * DQ + 4 * it + g4;
@@ -753,39 +746,23 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(AttnTArgs a) {
       qreg[it] = (c16 < nqv && d < a.dim) ? t : 0.f;
     }
   }
-  int mypos[4], my_nb[4], my_t0[4];
   float mrun[4], lrun[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int qv = 4 * g4 + i;
-    mypos[i] = qv < nqv ? pos0 + qv / Rc : -1;              // -1: no such vector, it sees nothing
-    my_nb[i] = qv < nqv ? win_nb(mypos[i], a.window, a.pool) : 0;
-    my_t0[i] = qv < nqv ? first_key(a, mypos[i]) : 0;
-    mrun[i] = -INFINITY;
-    lrun[i] = 0.f;
-  }
+  for (int i = 0; i < 4; ++i) { mrun[i] = -INFINITY; lrun[i] = 0.f; }
   f32x4 acc[NBV];
 #pragma unroll
   for (int c = 0; c < NBV; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int Gd = a.G * a.dim, Gv = a.G * a.vdim;
   const float* kb = a.k + ((int64_t)seq * a.t_max + tF) * a.ldk + (int64_t)g * a.dim;
-  const float* vb = a.v + ((int64_t)seq * a.t_max + tF) * a.ldv + (int64_t)g * a.vdim;
-  const float* pkb = a.pk ? a.pk + (int64_t)seq * a.n_pool_max * Gd + (int64_t)g * a.dim : nullptr;
-  const float* pvb = a.pv ? a.pv + (int64_t)seq * a.n_pool_max * Gv + (int64_t)g * a.vdim : nullptr;
-  f32x4 vk[NBD], vv[NBV];
+  f32x4 vk[NBD];
   auto fetch = [&](int tile) {
     const int k0 = tile * KT;
-    load16<NBD>(vk, a.dim, tid, [&](int j) { const int jj = min(k0 + j, nk - 1); return jj < nbL ? pkb + (int64_t)jj * Gd : kb + (int64_t)(jj - nbL) * a.ldk; },
-                [&](int j) { return k0 + j < nk; });
-    if (!VK) load16<NBV>(vv, a.vdim, tid, [&](int j) { const int jj = min(k0 + j, nk - 1); return jj < nbL ? pvb + (int64_t)jj * Gv : vb + (int64_t)(jj - nbL) * a.ldv; },
-                [&](int j) { return k0 + j < nk; });
+    load16<NBD>(vk, a.dim, tid, [&](int j) { return kb + (int64_t)min(k0 + j, nk - 1) * a.ldk; }, [&](int j) { return k0 + j < nk; });
   };
   if (t0 < t1) fetch(t0);
   for (int tile = t0; tile < t1; ++tile) {
     const int key0 = tile * KT;
     lds_barrier();                                             // the previous tile's keys, values and weights are consumed
     store16<NBD, LDK>(Kl, vk, tid);
-    if (!VK) store16<NBV, LDV>(Vl, vv, tid);
     if (tile + 1 < t1) fetch(tile + 1);                          // in flight while this tile is multiplied
     lds_barrier();
     {                                                            // partial scores over this wave's quarter of the head's values
@@ -802,13 +779,12 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(AttnTArgs a) {
     }
     lds_barrier();
     float corr[4];
-    const int j = key0 + c16, tok = tF + (j - nbL);
+    const int j = key0 + c16;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int o = (4 * g4 + i) * LDS_S + c16;
       float sc = soft_cap((Sp[o] + Sp[16 * LDS_S + o]) + (Sp[32 * LDS_S + o] + Sp[48 * LDS_S + o]), a.cap);
-      const bool see = j < nk && (j < nbL ? j < my_nb[i] : (tok >= my_t0[i] && tok <= mypos[i]));
-      if (!see) sc = -INFINITY;
+      if (j >= nk || 4 * g4 + i >= nqv) sc = -INFINITY;
       const float mnew = fmaxf(mrun[i], row16_max(sc));
       const float p = (sc == -INFINITY) ? 0.f : fast_exp(sc - mnew);
       corr[i] = (mrun[i] == -INFINITY) ? 0.f : fast_exp(mrun[i] - mnew);
@@ -826,7 +802,7 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(AttnTArgs a) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const float pa = Pl[c16 * LDP + t + 4 * g4];
-      const float* cb = Vl + (t + 4 * g4) * LDV + 16 * wave + c16;
+      const float* cb = Kl + (t + 4 * g4) * LDV + 16 * wave + c16;
 #pragma unroll
       for (int c = 0; c < NBV; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, cb[64 * c], acc[c], 0, 0, 0);
     }
@@ -836,9 +812,9 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(AttnTArgs a) {
   for (int i = 0; i < 4; ++i) {
     const int qv = 4 * g4 + i;
     if (qv >= nqv) continue;
-    const int row = r0 + qv / Rc;
-    const int64_t col0 = (int64_t)(h0 + qv % Rc) * a.vdim;
-    const float inv = a.out_scale * softmax_inv(mrun[i], lrun[i], a.sink, h0 + qv % Rc);
+    const int row = b;
+    const int64_t col0 = (int64_t)(h0 + qv) * a.vdim;
+    const float inv = a.out_scale * softmax_inv(mrun[i], lrun[i], a.sink, h0 + qv);
 #pragma unroll
     for (int c = 0; c < NBV; ++c) {
       const int d = 16 * (wave + 4 * c) + c16;
@@ -854,6 +830,8 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(AttnTArgs a) {
     if (part_out && wave == 0 && c16 == 0) { part_out[qv] = mrun[i]; part_out[AQ + qv] = lrun[i]; }
   }
 }
+
+#include "attn_rows.inl"
 
 // grid (n_blk, G * chunks, ceil(vdim / MERGE_COLS)): the splits' statistics and sums of every vector become its result; a workgroup
 // takes a slice of the value columns (one workgroup a run left the merge of a single decode row on one CU)
@@ -1193,6 +1171,9 @@ AttnShape attn_shape(int H, int G, int one_row) {
   s.chunks = (rep + s.hpc - 1) / s.hpc;
   return s;
 }
+// attn_rows.inl: heads side by side in a wave's 16 query vectors, and the runs of a workgroup
+int attn_rows_heads(int rep) { return rep >= 3 ? 4 : rep; }
+int attn_rows_runs(int rep) { return 4 * (16 / attn_rows_heads(rep)) / 4; }
 }  // namespace
 
 extern "C" int mn_window_attn_splits(int n_blk, int H, int G, int one_row, int max_keys) {
@@ -1202,8 +1183,11 @@ extern "C" int mn_window_attn_splits(int n_blk, int H, int G, int one_row, int m
 extern "C" int mn_window_attn_splits_tile(int n_blk, int H, int G, int one_row, int max_keys, int key_tile) {
   if (n_blk < 1 || H < 1 || G < 1 || (H % G) != 0 || max_keys < 1 || key_tile < 1) return 1;
   const AttnShape sh = attn_shape(H, G, one_row);
-  const int64_t wgs = (int64_t)n_blk * G * sh.chunks, tiles = mn_cdiv(max_keys, key_tile);
+  const int64_t wgs = mn_cdiv(n_blk, one_row ? 1 : attn_rows_runs(H / G)) * G * sh.chunks, tiles = mn_cdiv(max_keys, key_tile);
   int64_t ns = mn_cdiv(2 * (int64_t)mn_num_cus(), wgs);
+  // (a workgroup of 64 vectors has some 10 us of its own: a split of its walk below 128 keys costs more than it saves)
+  const int64_t most = one_row ? tiles : mn_cdiv(max_keys, 128);
+  if (ns > most) ns = most;
   if (ns > tiles) ns = tiles;
   if (ns > 64) ns = 64;
   return ns < 1 ? 1 : (int)ns;
@@ -1291,12 +1275,51 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
   MN_CHECK_ARG(variant == MN_WINDOW_ATTN_VALU || (variant == MN_WINDOW_ATTN_MFMA && mfma_fits),
                "mn_window_pool_attn_blocks: the matrix-core kernel takes runs of rows with dim, vdim <= 256, or values inside keys of dim <= 640");
   if (variant == MN_WINDOW_ATTN_MFMA) {
-    const dim3 gridm((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)nsplit);
     hipStream_t stm = mn_stream(stream);
-    if (vk) {
-      const int nb = dim <= 256 ? (dim + 63) / 64 : (dim <= 320 ? 5 : (dim <= 384 ? 6 : (dim <= 512 ? 8 : 10)));
+    const int nb = dim <= 256 ? (dim + 63) / 64 : (dim <= 320 ? 5 : (dim <= 384 ? 6 : (dim <= 512 ? 8 : 10)));
+    if (!one_row) {                                    // runs of rows: 64 query vectors per workgroup
+      const int hv = attn_rows_heads(H / G);
+      dim3 gridr((unsigned)mn_cdiv(n_blk, attn_rows_runs(H / G)), (unsigned)(G * sh.chunks), (unsigned)nsplit);
+#define MN_WR(D_, V_, E_) hipLaunchKernelGGL((attn_rows_kernel<D_, V_, E_>), gridr, dim3(256), 0, stm, a, n_blk, hv)
+#define MN_WL(D_, E_) hipLaunchKernelGGL((attn_latent_rows_kernel<D_, E_>), gridr, dim3(256), 0, stm, a, n_blk, hv)
+      const bool vec4 = ((dim | vdim) & 3) == 0;       // (rows of any other size go value by value)
+      if (vk) {
+        gridr.x = (unsigned)mn_cdiv(n_blk, attn_rows_runs(H / G) / 2);      // 32 vectors per workgroup
+        const int nbl = (dim + 63) / 64;
+        if (!vec4) {
+          if (nbl <= 2) MN_WL(2, false);
+          else if (nbl <= 5) MN_WL(5, false);
+          else MN_WL(10, false);
+        } else {
+          switch (nbl) {
+            case 1: MN_WL(1, true); break;
+            case 2: MN_WL(2, true); break;
+            case 3: MN_WL(3, true); break;
+            case 4: MN_WL(4, true); break;
+            case 5: MN_WL(5, true); break;
+            case 6: MN_WL(6, true); break;
+            case 7: MN_WL(7, true); break;
+            case 8: MN_WL(8, true); break;
+            case 9: MN_WL(9, true); break;
+            default: MN_WL(10, true); break;
+          }
+        }
+      } else if (!vec4) {
+        if (dim <= 64 && vdim <= 64) MN_WR(1, 1, false);
+        else if (dim <= 128 && vdim <= 128) MN_WR(2, 2, false);
+        else MN_WR(4, 4, false);
+      } else {
+        const int nbd = dim <= 64 ? 1 : (dim <= 128 ? 2 : 4), nbv = vdim <= 64 ? 1 : (vdim <= 128 ? 2 : 4);
+        if (nbd == 1) { if (nbv == 1) MN_WR(1, 1, true); else if (nbv == 2) MN_WR(1, 2, true); else MN_WR(1, 4, true); }
+        else if (nbd == 2) { if (nbv == 1) MN_WR(2, 1, true); else if (nbv == 2) MN_WR(2, 2, true); else MN_WR(2, 4, true); }
+        else { if (nbv == 1) MN_WR(4, 1, true); else if (nbv == 2) MN_WR(4, 2, true); else MN_WR(4, 4, true); }
+      }
+#undef MN_WL
+#undef MN_WR
+    } else {                                           // decode rows whose values lie inside the keys
+      const dim3 gridm((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)nsplit);
       const size_t ldsm = ((size_t)16 * (64 * nb + 4) + 4 * 16 * 17 + 16 * 20) * sizeof(float);
-#define MN_WK(D_) hipLaunchKernelGGL((window_attn_mfma_kernel<D_, D_, true>), gridm, dim3(256), ldsm, stm, a)
+#define MN_WK(D_) hipLaunchKernelGGL((window_attn_mfma_kernel<D_>), gridm, dim3(256), ldsm, stm, a)
       switch (nb) {
         case 1: MN_WK(1); break;
         case 2: MN_WK(2); break;
@@ -1308,14 +1331,6 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
         default: MN_WK(10); break;
       }
 #undef MN_WK
-    } else {
-      const int nbd = dim <= 64 ? 1 : (dim <= 128 ? 2 : 4), nbv = vdim <= 64 ? 1 : (vdim <= 128 ? 2 : 4);
-      const size_t ldsm = ((size_t)16 * (64 * nbd + 4) + (size_t)16 * (64 * nbv + 4) + 4 * 16 * 17 + 16 * 20) * sizeof(float);
-#define MN_WM(D_, V_) hipLaunchKernelGGL((window_attn_mfma_kernel<D_, V_>), gridm, dim3(256), ldsm, stm, a)
-      if (nbd == 1) { if (nbv == 1) MN_WM(1, 1); else if (nbv == 2) MN_WM(1, 2); else MN_WM(1, 4); }
-      else if (nbd == 2) { if (nbv == 1) MN_WM(2, 1); else if (nbv == 2) MN_WM(2, 2); else MN_WM(2, 4); }
-      else { if (nbv == 1) MN_WM(4, 1); else if (nbv == 2) MN_WM(4, 2); else MN_WM(4, 4); }
-#undef MN_WM
     }
     MN_CHECK_LAUNCH("mn_window_pool_attn_blocks(mfma)");
     if (nsplit > 1) {

@@ -68,7 +68,7 @@ PPlan make_plan(const mn_pn_model* m, int M) {
     const PDims d = pdims(l);
     up(p.n_in, d.n_in); up(p.nq, d.nq); up(p.nmid, d.nmid); up(p.hv, d.hv); up(p.ff, l.ff); up(p.side, pad8(l.side)); up(p.heads, l.heads);
     if (l.kind != MN_PN_DELTA) {
-      const size_t aw = (size_t)4 * mn_num_cus() * 16 * (2 + (size_t)d.avd) * sizeof(float);
+      const size_t aw = (size_t)4 * mn_num_cus() * 64 * (2 + (size_t)d.avd) * sizeof(float);
       if (aw > p.attn_ws) p.attn_ws = aw;
     }
     if (m->arith == MN_SEQ_ARITH_BF16 && M > 8 && M <= 64) {       // scratch of the weight-streaming MFMA route: the largest product of the stack

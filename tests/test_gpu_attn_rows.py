@@ -1,0 +1,67 @@
+"""Attention of runs of rows (attn_rows.inl) at the sizes where its grouping can go wrong: row counts around 16 / 32 / 64 vectors, several sequences
+and cached tokens in one workgroup, head groups of every width, windows, chunks, pooled blocks' tiles, key splits, values inside keys.  The
+reference is a plain float64 softmax; fp32 products of up to 600 terms and exponentials at 1e-6: 1e-5 of the largest value."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def run(spans, H, G, d, e, window, cap, chunk, vk, nsplit, t_max):
+    from ming_univision_amd._lib import check, current_stream, lib, ptr
+    from ming_univision_amd.sequences import rows_of_spans
+    L = lib()
+    g = torch.Generator().manual_seed(H * 1000 + d + len(spans))
+    tabs = rows_of_spans(spans, L.mn_window_attn_block_rows())
+    dev = {k: torch.from_numpy(np.ascontiguousarray(v)).cuda() for k, v in tabs.items() if k != "max_len"}
+    M, n_seq = sum(n for _, n, _ in spans), 1 + max(s for s, _, _ in spans)
+    q = torch.randn(M, H * d, generator=g) * d ** -0.5
+    k = torch.randn(n_seq, t_max, G * d, generator=g)
+    v = k if vk else torch.randn(n_seq, t_max, G * e, generator=g)
+    ref, r = torch.empty(M, H, e, dtype=torch.float64), 0
+    for s, n, past in spans:
+        i, j = torch.arange(past, past + n)[:, None], torch.arange(past + n)[None]
+        see = (j <= i) & ((i - j < window) if window else True) & ((i // chunk == j // chunk) if chunk else True)
+        for h in range(H):
+            c = h // (H // G)
+            sc = q[r:r + n].reshape(n, H, d)[:, h].double() @ k[s, :past + n].reshape(-1, G, d)[:, c].double().T
+            sc = cap * torch.tanh(sc / cap) if cap else sc
+            vv = k[s, :past + n].reshape(-1, G, d)[:, c, :e] if vk else v[s, :past + n].reshape(-1, G, e)[:, c]
+            ref[r:r + n, h] = torch.softmax(sc.masked_fill(~see, -float("inf")), -1) @ vv.double()
+        r += n
+    kd, qd = k.cuda(), q.cuda()
+    vd = kd if vk else v.cuda()
+    n_blk, ldv = dev["blk_tab"].shape[0], G * d if vk else G * e
+    ns = nsplit or L.mn_window_attn_splits(n_blk, H, G, 0, tabs["max_len"])
+    ws = torch.empty(max(16, L.mn_window_attn_workspace_bytes(n_blk, H, G, e, 0, ns)), dtype=torch.uint8, device="cuda")
+    out = torch.full((M + 1, H * e), 7.0, device="cuda")
+    check(L.mn_window_pool_attn_blocks_gate(ptr(qd), H * d, ptr(kd), G * d, ptr(vd), ldv, None, None, None, cap, chunk, None, 0, ptr(dev["row_seq"]),
+                                            ptr(dev["row_slot"]), ptr(dev["blk_tab"]), n_blk, 0, H, G, d, e, t_max, 1, window, 0, 1.0, ptr(out), H * e,
+                                            None, 0, ns, ptr(ws), ws.numel(), -1, current_stream()), "attn")
+    assert bool((out[M] == 7.0).all())
+    err = float((out[:M].double().cpu() - ref.reshape(M, -1)).abs().max() / ref.abs().max())
+    assert err < 1e-5, err
+
+
+SPANS = [[(0, 1, 0)], [(0, 63, 0)], [(0, 65, 7)], [(0, 3, 0), (1, 70, 0), (2, 1, 40), (3, 17, 5)], [(1, 130, 0), (0, 5, 200)]]
+
+
+@pytest.mark.parametrize("spans", SPANS)
+@pytest.mark.parametrize("H,G,d,e", [(4, 1, 64, 64), (8, 2, 128, 128), (6, 6, 16, 40), (6, 3, 72, 136), (5, 1, 34, 50), (3, 1, 200, 256)])
+def test_runs(spans, H, G, d, e):
+    for window, cap, chunk, ns in ((0, 0.0, 0, 0), (33, 20.0, 0, 3), (0, 0.0, 48, 2), (200, 0.0, 0, 1)):
+        run(spans, H, G, d, e, window, cap, chunk, False, ns, 256)
+
+
+@pytest.mark.parametrize("spans", SPANS)
+@pytest.mark.parametrize("H,d,e", [(4, 64, 48), (16, 576, 512), (9, 320, 256), (2, 35, 19), (1, 200, 200), (5, 450, 442)])
+def test_values_inside_keys(spans, H, d, e):
+    for window, cap, chunk, ns in ((0, 0.0, 0, 0), (33, 20.0, 0, 3), (0, 0.0, 48, 2)):
+        run(spans, H, 1, d, e, window, cap, chunk, True, ns, 256)
+
+
+def test_three_splits_of_many_groups():
+    """More than 256 workgroups in a head and split: every group exactly once whatever the launch order."""
+    run([(0, 700, 0), (1, 700, 0), (2, 700, 0)], 5, 1, 16, 16, 0, 0.0, 0, False, 3, 704)
+    run([(0, 700, 0), (1, 701, 0)], 4, 1, 32, 32, 0, 0.0, 0, True, 3, 704)

@@ -598,9 +598,10 @@ class BailingMoeDecoder:
 
     def logits(self, hidden):
         """lm_head -> fp32 logits (compute_logit, :1604-1620, norm_head=False)."""
-        if hidden.shape[0] > MAX_ROWS and lib().mn_gemm256_supported(hidden.shape[1], 8, self.lm_head.stride(0), self.lm_head.shape[0],
-                                                                     hidden.shape[0], self.lm_head.shape[0], hidden.shape[1]):
-            return ops.gemm256(ops.split_hilo(hidden.contiguous()), self.lm_head, None, "f32")    # many rows: one MFMA GEMM
+        if hidden.shape[0] > 8 and self.lm_head.data_ptr() % 16 == 0 and lib().mn_gemm256_supported(
+                hidden.shape[1], 8, self.lm_head.stride(0), self.lm_head.shape[0], hidden.shape[0], self.lm_head.shape[0], hidden.shape[1]):
+            # one pass over the vocabulary matrix (the 8-row chunks below read it once each) on the same hi/lo operands
+            return ops.gemm256(ops.split_hilo(hidden.contiguous()), self.lm_head, None, "f32")
         outs = [ops.skinny_gemm(hidden[i:i + 8].contiguous(), self.lm_head) for i in range(0, hidden.shape[0], 8)]
         return torch.cat(outs, 0)
 

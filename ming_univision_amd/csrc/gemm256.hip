@@ -83,8 +83,11 @@ typedef mn_g256 G256;
 
 enum { E_F32 = MN_G256_F32, E_BF16 = MN_G256_BF16, E_BF16_GELU = MN_G256_BF16_GELU, E_F32_RESID = MN_G256_F32_RESID,
        E_SWIGLU_SPLIT = MN_G256_SWIGLU_SPLIT, E_F32_RESID_GATE = MN_G256_F32_RESID_GATE, E_SWIGLU_BF16 = MN_G256_SWIGLU_BF16,
-       E_BF16_RELU2 = MN_G256_BF16_RELU2, E_SWIGLU_BF16_SCALED = MN_G256_SWIGLU_BF16_SCALED };
-__host__ __device__ constexpr bool epi_paired(int epi) { return epi == E_SWIGLU_SPLIT || epi == E_SWIGLU_BF16 || epi == E_SWIGLU_BF16_SCALED; }
+       E_BF16_RELU2 = MN_G256_BF16_RELU2, E_SWIGLU_BF16_SCALED = MN_G256_SWIGLU_BF16_SCALED,
+       E_F32_TAIL_RELU2 = MN_G256_F32_TAIL_RELU2, E_GEGLU_BF16 = MN_G256_GEGLU_BF16 };
+__host__ __device__ constexpr bool epi_paired(int epi) {
+  return epi == E_SWIGLU_SPLIT || epi == E_SWIGLU_BF16 || epi == E_SWIGLU_BF16_SCALED || epi == E_GEGLU_BF16;
+}
 
 __device__ __forceinline__ int lds_off(int buf, int op, int half) { return ((buf * 2 + op) * 2 + half) * HALF_BYTES; }
 
@@ -151,6 +154,17 @@ __device__ __forceinline__ void g256_emit(const G256& p, char* Cz, int m, int n,
   }
   if (EPI == E_F32) {
     *reinterpret_cast<f32x4*>(Cz + ((int64_t)m * p.ldc + n) * 4) = v;
+  } else if (EPI == E_F32_TAIL_RELU2) {                // a feed-forward's hidden units beside other projections of the same rows
+    if (n >= p.tail0 && n < p.tail1) {
+      const f32x4 r = f32x4{fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f)};
+      v = r * r;
+      *reinterpret_cast<u32x2*>(p.C2 + (int64_t)m * p.ldc2 + (n - p.tail0)) = u32x2{cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w)};
+    } else {
+      *reinterpret_cast<f32x4*>(Cz + ((int64_t)m * p.ldc + n) * 4) = v;
+    }
+  } else if (EPI == E_GEGLU_BF16) {
+    *reinterpret_cast<u32x2*>(Cz + ((int64_t)m * p.ldc + n) * 2) =
+        u32x2{cvt_pk_bf16(gelu_tanh_f(v.x) * u.x, gelu_tanh_f(v.y) * u.y), cvt_pk_bf16(gelu_tanh_f(v.z) * u.z, gelu_tanh_f(v.w) * u.w)};
   } else if (EPI == E_F32_RESID) {
     f32x4* c = reinterpret_cast<f32x4*>(Cz + ((int64_t)m * p.ldc + n) * 4);
     *c += v;
@@ -475,20 +489,22 @@ static void tile_go(const G256& p, int nz, hipStream_t st) {
 // 2 x 32 KiB), all of the LDS for the 128 x 128 form (plain 4 x 32, hi/lo 3 x 48 KiB) and two for its two-per-CU variant; deeper pipelines on
 // fewer workgroups measured slower everywhere (64 x 64: 8 stages 8.1 us against 7.3; 64 x 128: 6 stages 66.8 against 53.4 at 1409 x 8192 x 1024)
 template <int EPI>
-static bool tile_launch(const G256& p, int form, int nz, bool hilo, hipStream_t st) {
-  if (hilo) {
-    switch (form) {
-      case 1: tile_go<EPI, 64, 64, 2, 2, 3, true>(p, nz, st); return true;
-      case 2: tile_go<EPI, 64, 128, 2, 2, 2, true>(p, nz, st); return true;
-      case 3: tile_go<EPI, 128, 128, 2, 4, 3, true>(p, nz, st); return true;
-      default: return false;
-    }
-  }
+static bool tile_launch_plain(const G256& p, int form, int nz, hipStream_t st) {
   switch (form) {
     case 1: tile_go<EPI, 64, 64, 2, 2, 4, false>(p, nz, st); return true;
     case 2: tile_go<EPI, 64, 128, 2, 2, 3, false>(p, nz, st); return true;
     case 3: tile_go<EPI, 128, 128, 2, 4, 4, false>(p, nz, st); return true;
     case 4: tile_go<EPI, 128, 128, 2, 2, 2, false>(p, nz, st); return true;
+    default: return false;
+  }
+}
+template <int EPI>
+static bool tile_launch(const G256& p, int form, int nz, bool hilo, hipStream_t st) {
+  if (!hilo) return tile_launch_plain<EPI>(p, form, nz, st);
+  switch (form) {
+    case 1: tile_go<EPI, 64, 64, 2, 2, 3, true>(p, nz, st); return true;
+    case 2: tile_go<EPI, 64, 128, 2, 2, 2, true>(p, nz, st); return true;
+    case 3: tile_go<EPI, 128, 128, 2, 4, 3, true>(p, nz, st); return true;
     default: return false;
   }
 }
@@ -533,6 +549,15 @@ static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
     case E_F32_RESID_GATE: G256_GO(E_F32_RESID_GATE); break;
     case E_SWIGLU_BF16: G256_GO(E_SWIGLU_BF16); break;
     case E_BF16_RELU2: G256_GO(E_BF16_RELU2); break;
+    case E_F32_TAIL_RELU2:
+    case E_GEGLU_BF16:                                   // plain rows only
+      if (hilo || a.g_off || nz > 1) { mn_set_error("gemm256: epilogue %d takes one dense product of plain rows", epi); return MN_EINVAL; }
+      if (epi == E_GEGLU_BF16) {
+        if (!(form > 0 && tile_launch_plain<E_GEGLU_BF16>(p, form, nz, st))) hipLaunchKernelGGL((gemm256_kernel<E_GEGLU_BF16, false>), grid, dim3(512), 0, st, p);
+      } else {
+        if (!(form > 0 && tile_launch_plain<E_F32_TAIL_RELU2>(p, form, nz, st))) hipLaunchKernelGGL((gemm256_kernel<E_F32_TAIL_RELU2, false>), grid, dim3(512), 0, st, p);
+      }
+      break;
     case E_SWIGLU_BF16_SCALED:
       if (hilo || !a.row_scale) { mn_set_error("gemm256: the scaled SwiGLU epilogue takes plain rows and their factors"); return MN_EINVAL; }
       hipLaunchKernelGGL((gemm256_kernel<E_SWIGLU_BF16_SCALED, false>), grid, dim3(512), 0, st, p);

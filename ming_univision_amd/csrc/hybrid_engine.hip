@@ -258,7 +258,11 @@ extern "C" int mn_hyb_step(const mn_hyb_model* m, const mn_hyb_state* st, const 
     const bool h16_only = layer_norm && hh && mfma_ok(l.w_in, W) && route != EXPERTS_INDEXED && (!moe || l.pass == 0);
     const bool cat16_only = cath && mfma_ok(l.w_out, d.n_cat);
     MN_TRY(norm_stage(l.norm1, h16_only ? nullptr : hf, hh));
-    MN_TRY(linear(arith, M, hf, W, hh, W, l.w_in, d.n_in, W, nullptr, pin, d.n_in, gws, gwb, stream));
+    // prompt rows: the feed-forward's hidden units leave the product as the bf16 rows the output product reads
+    bool up_done = false;
+    if (d.n_up > 0 && l.ff_act == MN_HYB_ACT_RELU2 && cat16_only)
+      MN_TRY(linear_relu2_tail(arith, M, hh, W, l.w_in, d.n_in, W, pin, d.n_in, d.off_up, d.off_up + d.n_up, cath + d.hv, d.n_cat, stream, &up_done));
+    if (!up_done) MN_TRY(linear(arith, M, hf, W, hh, W, l.w_in, d.n_in, W, nullptr, pin, d.n_in, gws, gwb, stream));
     // ---- decode rows of the channel-decay mixers: what depends on the stacked product alone, in one launch ----
     const int E = l.experts, top = l.top, eff = l.expert_ff, Z = M * top;
     const bool prepped = one_row && M <= 64 && !cath && (delta || gla) && (d.n_up == 0 || l.ff_act == MN_HYB_ACT_XIELU) && (!moe || (l.table && layer_norm));
@@ -343,7 +347,7 @@ extern "C" int mn_hyb_step(const mn_hyb_model* m, const mn_hyb_state* st, const 
     if (moe && !l.table)
       MN_TRY(mn_router_softmax_topk_rows(pin + d.off_router, d.n_in, M, d.n_router, E, top, l.correction, tidx, tw, ride ? pin + d.off_up : nullptr,
                                          d.n_in, ride ? cat + d.hv : nullptr, d.n_cat, ride ? d.n_up : 0, stream));
-    if (d.n_up > 0 && !ride && !prepped) {
+    if (d.n_up > 0 && !ride && !prepped && !up_done) {
       float* ay = cat16_only ? nullptr : cat + d.hv;
       uint16_t* ah = cath ? cath + d.hv : nullptr;
       if (l.ff_act == MN_HYB_ACT_XIELU)

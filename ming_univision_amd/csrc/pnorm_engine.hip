@@ -212,7 +212,8 @@ extern "C" int mn_pn_step(const mn_pn_model* m, const mn_pn_state* st, const flo
     MN_TRY(mn_rms_scale_add_rows(xr, W, yf, W, l.norm1, m->eps, xh, W, M, W, stream));
     // ---- feed-forward ----
     if (l.ff > 0) {
-      bool fused = false;                                // few rows: the gelu product rides the weight-streaming product's epilogue
+      bool fused = false;                                // the gelu product rides the product's epilogue (prompt rows: as bf16)
+      if (acth && mfma_ok(l.w_down, l.ff)) MN_TRY(linear_geglu_rows(arith, M, xh, W, l.w_gate_up, l.ff, W, acth, l.ff, stream, &fused));
       if (!acth) MN_TRY(linear_geglu(arith, M, xr, W, l.w_gate_up, l.ff, W, act, l.ff, gws, gwb, stream, &fused));
       if (!fused) {
         MN_TRY(linear(arith, M, xr, W, xh, W, l.w_gate_up, 2 * l.ff, W, nullptr, gu, 2 * l.ff, gws, gwb, stream));

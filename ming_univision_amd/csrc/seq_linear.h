@@ -51,6 +51,40 @@ inline int linear_geglu(int arith, int M, const float* A, int64_t lda, const uin
   return mn_skinny_gemm(&a, stream);
 }
 
+// Prompt rows (M > 64, bf16 arithmetic) whose whole-K-tile products take the LDS-DMA GEMM: is this one of them?  (C2 / C rows: quadruples of columns)
+inline bool gemm_epilogue_ok(int arith, int M, const uint16_t* A16, int64_t lda16, const uint16_t* W, int64_t w_rows, int N, int K, const void* C, int64_t ldc) {
+  return arith == MN_SEQ_ARITH_BF16 && M > 64 && A16 && (((uintptr_t)A16 | (uintptr_t)W) & 15) == 0 && mn_gemm256_supported(lda16, 0, K, w_rows, M, N, K) &&
+         (ldc % 4) == 0 && ((uintptr_t)C & 15) == 0;
+}
+
+// C fp32 [M, N] = A W^T except its columns [t0, t1), which go squared-relu'd to C2 as bf16 [M, t1 - t0]: the hidden units' fp32 round trip (2048 x 12288:
+// 200 MB, 56 us of its own launch) is not taken.  *done says whether the step took it.
+inline int linear_relu2_tail(int arith, int M, const uint16_t* A16, int64_t lda16, const uint16_t* W, int N, int K, float* C, int64_t ldc, int t0, int t1,
+                             uint16_t* C2, int64_t ldc2, void* stream, bool* done) {
+  *done = false;
+  if (!gemm_epilogue_ok(arith, M, A16, lda16, W, N, N, K, C, ldc) || (t0 % 4) != 0 || (t1 % 4) != 0 || (ldc2 % 4) != 0 || ((uintptr_t)C2 & 7) != 0) return MN_OK;
+  mn_g256 a;
+  memset(&a, 0, sizeof(a));
+  a.A = A16; a.lda = lda16; a.W = W; a.ldw = K; a.C = C; a.ldc = ldc; a.C2 = C2; a.ldc2 = ldc2; a.tail0 = t0; a.tail1 = t1; a.M = M; a.N = N; a.K = K;
+  const int rc = mn_gemm256_ex(&a, MN_G256_F32_TAIL_RELU2, 1, stream);
+  *done = rc >= 0;
+  return rc < 0 ? rc : MN_OK;
+}
+
+// act bf16 [M, N] = gelu_tanh(A Wg^T) * (A Wu^T), W = [Wg ; Wu], in the epilogue of the product (1409 x 2 x 4096: 16 us of a launch of its own and the
+// fp32 round trip).  The caller's next product must read the bf16 rows.
+inline int linear_geglu_rows(int arith, int M, const uint16_t* A16, int64_t lda16, const uint16_t* W, int N, int K, uint16_t* act, int64_t ldact,
+                             void* stream, bool* done) {
+  *done = false;
+  if (!gemm_epilogue_ok(arith, M, A16, lda16, W, 2 * (int64_t)N, N, K, act, ldact)) return MN_OK;
+  mn_g256 a;
+  memset(&a, 0, sizeof(a));
+  a.A = A16; a.lda = lda16; a.W = W; a.ldw = K; a.w_pair_rows = N; a.C = act; a.ldc = ldact; a.M = M; a.N = N; a.K = K;
+  const int rc = mn_gemm256_ex(&a, MN_G256_GEGLU_BF16, 1, stream);
+  *done = rc >= 0;
+  return rc < 0 ? rc : MN_OK;
+}
+
 // the step's own copy of its input rows (a kernel, not a memcpy node: the step may be captured into a graph)
 __global__ void copy_rows_kernel(const float* __restrict__ x, int64_t ldx, float* __restrict__ y, int n) {
   const int c = blockIdx.x * 256 + threadIdx.x;

@@ -49,3 +49,38 @@ def test_forms(M, N, K):
         else:
             assert rel(ops.gemm256_swiglu(a1, w, b), act) < 2 ** -8
 
+
+
+@pytest.mark.parametrize("M,width,ff", [(65, 64, 96), (130, 128, 516), (300, 64, 1028), (70, 128, 102)])
+def test_activations_in_the_products_epilogue(M, width, ff):
+    """Prompt rows whose hidden units leave the product activated (squared relu beside the mixers' projections; gelu(gate) x up), against the same
+    layers in fp32 arithmetic, where every activation is a launch of its own; a hidden width that is no multiple of 4 keeps the launch."""
+    from ming_univision_amd.configuration import DaberaxConfig, ZuzenexConfig
+    from ming_univision_amd.daberax import DaberaxDecoder
+    from ming_univision_amd.zuzenex import ZuzenexDecoder
+    mlp = dict(kind="dense", ff=ff)
+    zu = ZuzenexConfig(width=width, vocab=40, norm=dict(eps=1e-6), layers=[
+        dict(type="attention", mixer=dict(heads=2, kv_heads=1, dim=20, vdim=32, scale=0.2), mlp=mlp),
+        dict(type="lightning", mixer=dict(heads=2, dim=16, vdim=16, decay=[0.9, 0.99]), mlp=mlp)])
+    da = DaberaxConfig(width=width, vocab=40, norm=dict(eps=1e-6), token_side=dict(dim=8), layers=[
+        dict(type="attention", mixer=dict(heads=2, kv_heads=1, dim=16, vdim=32, scale=0.2), mlp=mlp)])
+    ids = torch.arange(M, device="cuda") % 40
+    for cls, cfg in ((ZuzenexDecoder, zu), (DaberaxDecoder, da)):
+        out = [cls.synthetic(cfg, "cuda", t_max=M + 1, n_seq=1, arith=a).prefill(ids) for a in ("bf16", "f32")]
+        assert rel(out[0], out[1]) < 3e-2                # two layers of products on bf16 operands (2^-9 each, some ten of them, of values up to 4 rms)
+
+
+@pytest.mark.parametrize("M,n", [(1, 4), (3, 1020), (5, 1024), (2, 1028), (70, 2048), (4, 4100), (3, 8192), (2, 8196), (3, 33)])
+def test_residual_and_rms_rows(M, n):
+    """x += m y, RMS norm: rows in registers and the walking form (odd or very wide rows)."""
+    from ming_univision_amd._lib import check, current_stream, lib, ptr
+    g = torch.Generator(device="cuda").manual_seed(M + n)
+    x, y = torch.randn(M, n + 4, generator=g, device="cuda"), torch.randn(M, n + 8, generator=g, device="cuda")
+    w = (1 + 0.1 * torch.randn(n, generator=g, device="cuda")).to(torch.bfloat16)
+    o, o16 = torch.full((M, n + 4), 5.0, device="cuda"), torch.full((M, n + 4), 5.0, device="cuda").to(torch.bfloat16)
+    for yy in (y, None):
+        ref = x[:, :n].double() + (0.5 * y[:, :n].double() if yy is not None else 0)
+        nrm = ref / torch.sqrt((ref * ref).mean(-1, keepdim=True) + 1e-5) * w.double()
+        check(lib().mn_axpy_rms_rows(ptr(x), n + 4, ptr(yy), n + 8, 0.5, ptr(w), 1e-5, ptr(o), n + 4, ptr(o16), n + 4, M, n, current_stream()), "axpy")
+        assert rel(x[:, :n], ref) < 1e-6 and rel(o[:, :n], nrm) < 2e-6 and rel(o16[:, :n], nrm) < 2 ** -8
+        assert bool((o[:, n:] == 5).all()) and bool((o16[:, n:] == 5).all())

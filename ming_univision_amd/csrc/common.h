@@ -190,4 +190,6 @@ enum { MN_G256_F32 = 0, MN_G256_BF16 = 1, MN_G256_BF16_GELU = 2, MN_G256_F32_RES
        MN_G256_GEGLU_BF16 = 10 };                       // gelu(gate) * up, tanh form, as bf16 (paired like SWIGLU_BF16)
 extern "C" int mn_gemm256_ex(const mn_g256* a, int epi, int ksplit, void* stream);
 extern "C" int mn_gemm256_slices(int K, int ksplit);
+extern "C" int mn_axpy_rms_rows_slabs(float* x, int64_t ldx, const float* y, int64_t ldy, int nz, int64_t zs, float mult, const uint16_t* w, float eps,
+                                      float* n_out, int64_t ldn, uint16_t* n16, int64_t ldn16, int M, int n, void* stream);
 extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo);

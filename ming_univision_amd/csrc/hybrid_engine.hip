@@ -57,9 +57,14 @@ HDims hdims(const mn_hyb_layer& l) {
   return d;
 }
 
+// rows of the joined output product's buffer where it may come in slabs: as many for every row count, so that a workspace for more rows serves fewer
+constexpr int SLAB_ROWS = 8192;
+inline size_t out_rows(bool slabs, int M) { return slabs && M < SLAB_ROWS ? (size_t)SLAB_ROWS : (size_t)M; }
+
 struct HPlan {
   int n_in = 1, cq = 1, hv = 1, n_cat = 1, top = 1, eff = 1, eup = 1, experts = 1, dec = 1, gate = 1, beta = 1;
   size_t gemm_ws = 0, attn_ws = 0;
+  bool slabs = false;                        // the joined output product may come as split-K slabs (summed by the next norm)
   int64_t lin = 0;                                               // largest heads x dim x vdim of a lightning recurrence
   size_t gla = 0;                                                // largest bytes of a gla layer's chunk state
 };
@@ -92,6 +97,7 @@ HPlan make_plan(const mn_hyb_model* m, int M) {
       if (up > p.eup) p.eup = up;
       if (l.experts > p.experts) p.experts = l.experts;
     }
+    if (m->norm != MN_HYB_NORM_LAYER && l.ff_kind != MN_HYB_FF_MOE && m->arith == MN_SEQ_ARITH_BF16 && M > 64) p.slabs = true;
     if (d.n_dec > p.dec) p.dec = d.n_dec;
     if (d.n_gate > p.gate) p.gate = d.n_gate;
     if (d.n_beta > p.beta) p.beta = d.n_beta;
@@ -143,7 +149,7 @@ extern "C" size_t mn_hyb_workspace_bytes(const mn_hyb_model* m, int M) {
   n += al(R * p.cq * 4);                               // queries
   n += al(R * p.hv * 4);                               // the recurrence's heads before their norm
   n += al(R * p.n_cat * 4) + al(R * p.n_cat * 2);      // [mixer | activation] + bf16
-  n += al(R * W * 4);                                  // their joined output product
+  n += al(out_rows(p.slabs, M) * W * 4);               // their joined output product
   n += 2 * al(Z * 4);                                  // chosen experts, weights
   n += al(Z * p.eup * 4);                              // [gate ; up] or up of the pairs
   n += al(Z * p.eff * 4) + al(Z * p.eff * 2);          // their activation + bf16
@@ -184,7 +190,7 @@ extern "C" int mn_hyb_step(const mn_hyb_model* m, const mn_hyb_state* st, const 
   float* lo = (float*)take(R * p.hv * 4);
   float* cat = (float*)take(R * p.n_cat * 4);
   uint16_t* cath = (uint16_t*)take(R * p.n_cat * 2);
-  float* yf = (float*)take(R * W * 4);
+  float* yf = (float*)take(out_rows(p.slabs, M) * W * 4);
   int32_t* tidx = (int32_t*)take(Zmax * 4);
   float* tw = (float*)take(Zmax * 4);
   float* gu = (float*)take(Zmax * p.eup * 4);
@@ -215,7 +221,7 @@ extern "C" int mn_hyb_step(const mn_hyb_model* m, const mn_hyb_state* st, const 
   hipLaunchKernelGGL(copy_rows_kernel, dim3((unsigned)mn_cdiv(W, 256), (unsigned)M), dim3(256), 0, hs, x, ldx, xr, W);
   MN_CHECK_LAUNCH("mn_hyb_step(copy)");
   // what has not been added to x yet: a sublayer result, and the results of the experts with their weights
-  struct { const float* y; const float* ye; const int32_t* so; const float* w; float w_all; int top; } pend = {nullptr, nullptr, nullptr, nullptr, 0.f, 0};
+  struct { const float* y; const float* ye; const int32_t* so; const float* w; float w_all; int top, nz; } pend = {nullptr, nullptr, nullptr, nullptr, 0.f, 0, 1};
   const bool layer_norm = m->norm == MN_HYB_NORM_LAYER;
   // decode rows without bf16 copies: residual add + norm as one workgroup per row with the row in registers (the launch the
   // parallel-mixer step uses for its decode rows, here without a filter)
@@ -228,8 +234,8 @@ extern "C" int mn_hyb_step(const mn_hyb_model* m, const mn_hyb_state* st, const 
     else if (fuse && w && h && !h16)
       rc2 = mn_axpy_rms_filter_rows(xr, W, pend.y, W, 1.0f, w, m->eps, nullptr, 0, nullptr, row_seq, row_slot, h, W, M, W, stream);
     else
-      rc2 = mn_axpy_rms_rows(xr, W, pend.y, W, 1.0f, w, m->eps, h, W, h16, W, M, W, stream);
-    pend = {nullptr, nullptr, nullptr, nullptr, 0.f, 0};
+      rc2 = mn_axpy_rms_rows_slabs(xr, W, pend.y, W, pend.y ? pend.nz : 1, (int64_t)M * W, 1.0f, w, m->eps, h, W, h16, W, M, W, stream);
+    pend = {nullptr, nullptr, nullptr, nullptr, 0.f, 0, 1};
     return rc2;
   };
   for (int ri = 0; ri < m->n_runs; ++ri) {
@@ -355,8 +361,12 @@ extern "C" int mn_hyb_step(const mn_hyb_model* m, const mn_hyb_state* st, const 
       else
         MN_TRY(mn_relu2_rows(pin + d.off_up, d.n_in, ay, d.n_cat, ah, d.n_cat, M, d.n_up, stream));
     }
-    MN_TRY(linear(arith, M, cat, d.n_cat, cath, d.n_cat, l.w_out, W, d.n_cat, nullptr, yf, W, gws, gwb, stream));
+    int nz = 0;
+    if (!layer_norm && !moe && p.slabs)
+      MN_TRY(linear_slabs(arith, M, cath, d.n_cat, l.w_out, W, d.n_cat, linear_slices(arith, M, W, d.n_cat, SLAB_ROWS / M), yf, stream, &nz));
+    if (nz == 0) MN_TRY(linear(arith, M, cat, d.n_cat, cath, d.n_cat, l.w_out, W, d.n_cat, nullptr, yf, W, gws, gwb, stream));
     pend.y = yf;
+    pend.nz = nz > 0 ? nz : 1;
     if (moe) {
       const uint16_t* h16 = hh;
       const int32_t* so = nullptr;

@@ -256,23 +256,122 @@ __global__ __launch_bounds__(256) void light_scan_kv_kernel(LightScanArgs s) {
   }
 }
 
-// grid (ceil(dim vdim / 256), H, n_chunks): the workgroup of a sequence's first chunk in the step walks that sequence's chunks
-__global__ __launch_bounds__(256) void light_scan_carry_kernel(LightScanArgs s) {
-  const LightArgs& a = s.b;
-  const int x = blockIdx.x * 256 + threadIdx.x, h = blockIdx.y, c0 = blockIdx.z, de = a.dim * a.vdim;
-  const int r0 = s.chunk_tab[2 * c0];
-  if (a.row_back[r0] != 0 || x >= de) return;
-  const float lam = a.decay[h], ll = lam > 0.f ? logf(lam) : 0.f;
-  float* sp = a.state + ((int64_t)a.row_seq[r0] * a.H + h) * de + x;
-  float S = a.row_slot[r0] == 0 ? 0.f : *sp;
-  for (int ch = c0; ch < s.n_chunks; ++ch) {
-    if (ch > c0 && a.row_back[s.chunk_tab[2 * ch]] == 0) break;      // the next sequence starts here
-    float* w = s.ws + ((int64_t)ch * a.H + h) * de + x;
-    const float kv = *w;
-    *w = S;
-    S = fmaf(powi32(lam, ll, s.chunk_tab[2 * ch + 1]), S, kv);
+// silu of columns [col, col + d) of a chunk's n rows -> LDS rows of ld floats, zero from d and from row n on; f(j) scales row j.  V4 (quadruples, 16-byte
+// aligned rows): four 16-byte loads of a thread in flight at a time — one 4-byte load after another made staging the larger part of both passes
+template <bool V4, typename F>
+__device__ __forceinline__ void stage_silu(float* __restrict__ dst, int ld, const float* __restrict__ src, int64_t lds_, int n, int d, int tid, F f) {
+  if (V4) {
+    const int lq = ld / 4, cnt = LCH * lq;
+    for (int x0 = tid; x0 < cnt; x0 += 1024) {
+      f32x4 t[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int x = x0 + 256 * u, j = x / lq, i = 4 * (x - j * lq);
+        t[u] = *reinterpret_cast<const f32x4*>(src + (int64_t)min(j, n - 1) * lds_ + (i < d ? i : 0));
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int x = x0 + 256 * u, j = x / lq, i = 4 * (x - j * lq);
+        if (x >= cnt) break;
+        const float w = j < n ? f(j) : 0.f;
+        f32x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = j < n && i < d ? silu32(t[u][e]) * w : 0.f;
+        *reinterpret_cast<f32x4*>(dst + j * ld + i) = r;
+      }
+    }
+    return;
   }
-  *sp = S;
+  for (int x = tid; x < LCH * ld; x += 256) {
+    const int j = x / ld, i = x - j * ld;
+    dst[x] = (j < n && i < d) ? silu32(src[(int64_t)j * lds_ + i]) * f(j) : 0.f;
+  }
+}
+
+// Pass 1 on the fp32 matrix cores: wave w owns the 16-row tiles w, w + 4, .. of the own sum, their k columns (all 32 rows) in registers, and walks
+// the 16-column tiles of v.  Bound by the staging and the 64 KB a (chunk, head) writes: 2048 rows x 16 heads of 128 + 128: 44 us with FMAs on
+// four-byte staged rows, 34 us here.
+template <bool V4>
+__global__ __launch_bounds__(256) void light_scan_kv_mfma_kernel(LightScanArgs s, int ldk, int ldv) {
+  extern __shared__ float lds[];             // k [32][ldk] (decayed), v [32][ldv]
+  const LightArgs& a = s.b;
+  const int ch = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, d = a.dim, e = a.vdim;
+  const int r0 = s.chunk_tab[2 * ch], n = s.chunk_tab[2 * ch + 1];
+  const int wave = tid >> 6, lane = tid & 63, c16 = lane & 15, g4 = lane >> 4;
+  float* kl = lds;
+  float* vl = lds + LCH * ldk;
+  const float lam = a.decay[h], ll = lam > 0.f ? logf(lam) : 0.f;
+  const float* row = a.qkv + (int64_t)r0 * a.ldqkv;
+  stage_silu<V4>(kl, ldk, row + (int64_t)a.H * d + (int64_t)h * d, a.ldqkv, n, d, tid, [&](int j) { return powi32(lam, ll, n - 1 - j); });
+  stage_silu<V4>(vl, ldv, row + (int64_t)2 * a.H * d + (int64_t)h * e, a.ldqkv, n, e, tid, [](int) { return 1.0f; });
+  __syncthreads();
+  float* dst = s.ws + ((int64_t)ch * a.H + h) * d * e;
+  for (int ti = wave; 16 * ti < d; ti += 4) {
+    float kf[LCH / 4];
+#pragma unroll
+    for (int it = 0; it < LCH / 4; ++it) kf[it] = kl[(4 * it + g4) * ldk + 16 * ti + c16];
+    for (int tc = 0; 16 * tc < e; tc += 2) {
+      f32x4 a0 = f32x4{0.f, 0.f, 0.f, 0.f}, a1 = a0;
+      const bool two = 16 * (tc + 1) < e;
+      const float* vb = vl + g4 * ldv + 16 * tc + c16;
+#pragma unroll
+      for (int it = 0; it < LCH / 4; ++it) {
+        a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[it], vb[4 * it * ldv], a0, 0, 0, 0);
+        if (two) a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[it], vb[4 * it * ldv + 16], a1, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 16 * ti + 4 * g4 + i, c = 16 * tc + c16;
+        if (r >= d) continue;
+        if (c < e) dst[(int64_t)r * e + c] = a0[i];
+        if (two && c + 16 < e) dst[(int64_t)r * e + c + 16] = a1[i];
+      }
+    }
+  }
+}
+
+// grid (ceil(dim vdim / 256), H): a thread walks its state value through all chunks of the pass, one sequence after the other.  The chunks' table entries
+// come through LDS, 256 at a time, and 16 chunks' sums are requested before the first is used: with a chain of dependent reads per
+// chunk the walk took 45 us for 64 chunks of 16 heads of 128 x 128 (134 MB), 38 us here.
+__global__ __launch_bounds__(256) void light_scan_carry_kernel(LightScanArgs s) {
+  constexpr int PRE = 16, TAB = 256;
+  __shared__ int2 tab[TAB];                            // per chunk: rows; the cache sequence that starts here (-1: none; -2 - seq: it starts from zero)
+  const LightArgs& a = s.b;
+  const int x = blockIdx.x * 256 + threadIdx.x, h = blockIdx.y, de = a.dim * a.vdim;
+  const bool on = x < de;
+  const float lam = a.decay[h], ll = lam > 0.f ? logf(lam) : 0.f;
+  const int64_t step = (int64_t)a.H * de;
+  float* sp = nullptr;
+  float S = 0.f;
+  for (int c0 = 0; c0 < s.n_chunks; c0 += TAB) {
+    const int nc = min(TAB, s.n_chunks - c0);
+    __syncthreads();
+    if ((int)threadIdx.x < nc) {
+      const int row = s.chunk_tab[2 * (c0 + threadIdx.x)], seq = a.row_seq[row];
+      tab[threadIdx.x] = int2{s.chunk_tab[2 * (c0 + threadIdx.x) + 1], a.row_back[row] != 0 ? -1 : (a.row_slot[row] != 0 ? seq : -2 - seq)};
+    }
+    __syncthreads();
+    if (!on) continue;
+    for (int ch = 0; ch < nc; ch += PRE) {
+      float* w = s.ws + ((int64_t)(c0 + ch) * a.H + h) * de + x;
+      float kv[PRE];
+#pragma unroll
+      for (int u = 0; u < PRE; ++u) kv[u] = w[(int64_t)(min(ch + u, nc - 1) - ch) * step];
+#pragma unroll
+      for (int u = 0; u < PRE; ++u) {
+        if (ch + u >= nc) break;
+        const int2 t = tab[ch + u];
+        if (t.y != -1) {                               // uniform: a sequence starts here
+          if (sp) *sp = S;
+          sp = a.state + ((int64_t)(t.y >= 0 ? t.y : -2 - t.y) * a.H + h) * de + x;
+          S = t.y >= 0 ? *sp : 0.f;
+        }
+        w[(int64_t)u * step] = S;
+        S = fmaf(powi32(lam, ll, t.x), S, kv[u]);
+      }
+    }
+  }
+  if (sp) *sp = S;
 }
 
 template <int CV>
@@ -371,7 +470,9 @@ __global__ __launch_bounds__(256) void light_scan_out_kernel(LightScanArgs s) {
 // workgroup of 4 waves owns one (chunk, head): q, k (rows of ldq floats) and v (rows of ldv floats) of the chunk's <= 32 rows are staged
 // activated and zero padded; waves 0 .. 2 multiply the three 16 x 16 score tiles on or below the diagonal and park them, decayed and
 // masked, in LDS; then wave w owns the 16-column tiles w, w + 4, .. of the result, both row tiles at once: Q S0 with the carried state
-// read straight from the workspace (8 loads in flight), times lam^(i + 1) by rows, plus P V.
+// read straight from the workspace (8 loads in flight), times lam^(i + 1) by rows, plus P V.  2048 rows, 16 heads of 128 + 128: 98 us
+// with four-byte staging and state reads, 52 us here (64 MB of states, 50 MB of rows).
+template <bool V4>
 __global__ __launch_bounds__(256) void light_scan_out_mfma_kernel(LightScanArgs s, int ldq, int ldv) {
   extern __shared__ float lds[];             // q [32][ldq], k [32][ldq], v [32][ldv], P [32][36]
   constexpr int LDP = 36;
@@ -384,21 +485,11 @@ __global__ __launch_bounds__(256) void light_scan_out_mfma_kernel(LightScanArgs 
   float* vl = kl + LCH * ldq;
   float* P = vl + LCH * ldv;
   const float lam = a.decay[h], ll = lam > 0.f ? logf(lam) : 0.f;
-  for (int x = tid; x < LCH * ldq; x += 256) {
-    const int j = x / ldq, i = x - j * ldq;
-    float qv = 0.f, kv = 0.f;
-    if (j < n && i < d) {
-      const float* row = a.qkv + (int64_t)(r0 + j) * a.ldqkv + (int64_t)h * d + i;
-      qv = silu32(row[0]);
-      kv = silu32(row[(int64_t)a.H * d]);
-    }
-    ql[x] = qv;
-    kl[x] = kv;
-  }
-  for (int x = tid; x < LCH * ldv; x += 256) {
-    const int j = x / ldv, c = x - j * ldv;
-    vl[x] = (j < n && c < e) ? silu32(a.qkv[(int64_t)(r0 + j) * a.ldqkv + (int64_t)2 * a.H * d + (int64_t)h * e + c]) : 0.f;
-  }
+  const float* row0 = a.qkv + (int64_t)r0 * a.ldqkv;
+  const auto one = [](int) { return 1.0f; };
+  stage_silu<V4>(ql, ldq, row0 + (int64_t)h * d, a.ldqkv, n, d, tid, one);
+  stage_silu<V4>(kl, ldq, row0 + (int64_t)a.H * d + (int64_t)h * d, a.ldqkv, n, d, tid, one);
+  stage_silu<V4>(vl, ldv, row0 + (int64_t)2 * a.H * d + (int64_t)h * e, a.ldqkv, n, e, tid, one);
   __syncthreads();
   const int ksteps = (d + 3) / 4;            // ldq >= 4 ksteps, the padding is zero
   if (wave < 3) {                            // score tiles (0, 0), (1, 0), (1, 1)
@@ -428,6 +519,57 @@ __global__ __launch_bounds__(256) void light_scan_out_mfma_kernel(LightScanArgs 
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) rowf[t][i] = powi32(lam, ll, 16 * t + 4 * g4 + i + 1);
+  if (V4) {
+    // wave tasks: (row tile, 64 columns).  Column fragment u of a task is columns 64 cb + 4 c16 + u, so the carried state, v and the result go 16 bytes
+    // at a time
+    const int tasks = 2 * ((e + 63) / 64);
+    for (int t = wave; t < tasks; t += 4) {
+      const int ti = t & 1, col = 64 * (t >> 1) + 4 * c16;
+      const bool col_ok = col < e;
+      const float* sp = S0 + (col_ok ? col : 0);
+      f32x4 acc[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const float* aq = ql + (16 * ti + c16) * ldq + g4;
+      for (int it0 = 0; it0 < ksteps; it0 += 8) {
+        f32x4 b[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int k = 4 * (it0 + u) + g4;
+          b[u] = *reinterpret_cast<const f32x4*>(sp + (int64_t)(k < d ? k : 0) * e);      // (rows from d on meet zero columns of q)
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          if (it0 + u < ksteps) {
+            const float q = aq[4 * (it0 + u)];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(q, b[u][x], acc[x], 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[x][i] *= ti ? rowf[1][i] : rowf[0][i];
+      const float* pp = P + (16 * ti + c16) * LDP + g4;
+      const float* vb = vl + g4 * ldv + (col_ok ? col : 0);
+#pragma unroll
+      for (int it = 0; it < LCH / 4; ++it) {
+        if (ti == 0 && it >= 4) break;                 // row tile 0 sees keys 0 .. 15 only
+        const f32x4 bv = *reinterpret_cast<const f32x4*>(vb + 4 * it * ldv);
+        const float p = pp[4 * it];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) acc[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, bv[x], acc[x], 0, 0, 0);
+      }
+      if (!col_ok) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 16 * ti + 4 * g4 + i;
+        if (r < n) *reinterpret_cast<f32x4*>(a.out + (int64_t)(r0 + r) * a.ldo + (int64_t)h * e + col) = f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
+      }
+    }
+    return;
+  }
   const int ntile = (e + 15) / 16;
   for (int ct = wave; ct < ntile; ct += 4) {
     const int col = 16 * ct + c16;
@@ -682,15 +824,24 @@ extern "C" int mn_lightning_rows_scan_ex(const float* qkv, int64_t ldqkv, int M,
   hipStream_t st = mn_stream(stream);
   // four value columns per thread where rows of values and of the state are 16-byte aligned
   const bool v4 = (vdim % 4) == 0 && (((uintptr_t)workspace) & 15) == 0;
-  if (v4) hipLaunchKernelGGL((light_scan_kv_kernel<4>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), (size_t)LCH * (dim + vdim) * sizeof(float), st, s);
+  // quadruples of 16-byte aligned values throughout the rows: vector staging
+  const bool r4 = ((dim | vdim) % 4) == 0 && ((ldqkv | ldo) % 4) == 0 && (((uintptr_t)qkv | (uintptr_t)out | (uintptr_t)workspace) & 15) == 0;
+  const int ldk1 = ((dim + 15) / 16 * 16 + 47) / 64 * 64 + 16, ldv1 = ((vdim + 15) / 16 * 16 + 47) / 64 * 64 + 16;      // 16 mod 64: the four rows of an operand read fall in banks of their own
+  const size_t lds1 = (size_t)LCH * (ldk1 + ldv1) * sizeof(float);
+  if (variant == MN_LIGHTNING_SCAN_MFMA && lds1 <= 64 * 1024) {
+    if (r4) hipLaunchKernelGGL((light_scan_kv_mfma_kernel<true>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), lds1, st, s, ldk1, ldv1);
+    else hipLaunchKernelGGL((light_scan_kv_mfma_kernel<false>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), lds1, st, s, ldk1, ldv1);
+  } else if (v4) hipLaunchKernelGGL((light_scan_kv_kernel<4>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), (size_t)LCH * (dim + vdim) * sizeof(float), st, s);
   else hipLaunchKernelGGL((light_scan_kv_kernel<1>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), (size_t)LCH * (dim + vdim) * sizeof(float), st, s);
   MN_CHECK_LAUNCH("mn_lightning_rows_scan(sums)");
-  hipLaunchKernelGGL(light_scan_carry_kernel, dim3((unsigned)mn_cdiv((int64_t)dim * vdim, 256), (unsigned)H, (unsigned)n_chunks), dim3(256), 0, st, s);
+  hipLaunchKernelGGL(light_scan_carry_kernel, dim3((unsigned)mn_cdiv((int64_t)dim * vdim, 256), (unsigned)H), dim3(256), 0, st, s);
   MN_CHECK_LAUNCH("mn_lightning_rows_scan(carry)");
   if (variant == MN_LIGHTNING_SCAN_MFMA) {
     MN_CHECK_ARG(scan_mfma_lds(dim, vdim) <= 64 * 1024, "mn_lightning_rows_scan: heads of %d + %d values do not fit the matrix-core pass", dim, vdim);
-    hipLaunchKernelGGL(light_scan_out_mfma_kernel, dim3((unsigned)n_chunks, (unsigned)H), dim3(256), scan_mfma_lds(dim, vdim), st, s, scan_ldq(dim),
-                       scan_ldv(vdim));
+    if (r4) hipLaunchKernelGGL((light_scan_out_mfma_kernel<true>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), scan_mfma_lds(dim, vdim), st, s,
+                               scan_ldq(dim), scan_ldv(vdim));
+    else hipLaunchKernelGGL((light_scan_out_mfma_kernel<false>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), scan_mfma_lds(dim, vdim), st, s,
+                            scan_ldq(dim), scan_ldv(vdim));
   } else if (v4) hipLaunchKernelGGL((light_scan_out_kernel<4>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), lds3, st, s);
   else hipLaunchKernelGGL((light_scan_out_kernel<1>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), lds3, st, s);
   MN_CHECK_LAUNCH("mn_lightning_rows_scan(outputs)");

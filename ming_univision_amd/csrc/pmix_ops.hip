@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256) void axpy_rms_kernel(float* __restrict__ x, in
 // the same with one workgroup per row and the row in registers (rows of at most 1024 NV values, quadruples of them 16 / 8 bytes aligned): every load is
 // issued before the reduction.  Bound by its bytes: 2048 x 2048 with the add and the bf16 copy (56 MB) 12.3 us, 35 us in the form above
 template <int NV>
-__global__ __launch_bounds__(256) void axpy_rms_reg_kernel(float* __restrict__ x, int64_t ldx, const float* __restrict__ y, int64_t ldy, float mult,
+__global__ __launch_bounds__(256) void axpy_rms_reg_kernel(float* __restrict__ x, int64_t ldx, const float* __restrict__ y, int64_t ldy, int nz, int64_t zs, float mult,
                                                            const bf16_t* __restrict__ w, float eps, float* __restrict__ nout, int64_t ldn,
                                                            bf16_t* __restrict__ n16, int64_t ldn16, int n) {
   __shared__ float red[4];
@@ -96,7 +96,12 @@ __global__ __launch_bounds__(256) void axpy_rms_reg_kernel(float* __restrict__ x
     for (int t = 0; t < NV; ++t) {
       const int c = 4 * (tid + 256 * t);
       if (c >= n) continue;
-      const float4 a = *reinterpret_cast<const float4*>(y + (int64_t)m * ldy + c);
+      const float* yp = y + (int64_t)m * ldy + c;
+      float4 a = *reinterpret_cast<const float4*>(yp);
+      for (int z = 1; z < nz; ++z) {                   // the slabs of a split-K product
+        const float4 b = *reinterpret_cast<const float4*>(yp + z * zs);
+        a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+      }
       v[t].x = fmaf(mult, a.x, v[t].x); v[t].y = fmaf(mult, a.y, v[t].y); v[t].z = fmaf(mult, a.z, v[t].z); v[t].w = fmaf(mult, a.w, v[t].w);
       *reinterpret_cast<float4*>(x + (int64_t)m * ldx + c) = v[t];
     }
@@ -1091,11 +1096,18 @@ __global__ __launch_bounds__(256) void moe_combine_residual_kernel(float* __rest
 
 extern "C" int mn_axpy_rms_rows(float* x, int64_t ldx, const float* y, int64_t ldy, float mult, const uint16_t* w, float eps, float* n_out,
                                 int64_t ldn, uint16_t* n16, int64_t ldn16, int M, int n, void* stream) {
+  return mn_axpy_rms_rows_slabs(x, ldx, y, ldy, 1, 0, mult, w, eps, n_out, ldn, n16, ldn16, M, n, stream);
+}
+
+// the same with y = the sum of nz slabs zs values apart (nz > 1: rows the register form takes)
+extern "C" int mn_axpy_rms_rows_slabs(float* x, int64_t ldx, const float* y, int64_t ldy, int nz, int64_t zs, float mult, const uint16_t* w, float eps,
+                                      float* n_out, int64_t ldn, uint16_t* n16, int64_t ldn16, int M, int n, void* stream) {
   MN_CHECK_ARG(x && M >= 1 && n >= 1 && (w || (!n_out && !n16)), "mn_axpy_rms_rows: bad args");
   hipStream_t st = mn_stream(stream);
   const bool vec = (n % 4) == 0 && n <= 8192 && (ldx % 4) == 0 && (!y || (ldy % 4) == 0) && (!n_out || (ldn % 4) == 0) && (!n16 || (ldn16 % 4) == 0) &&
                    (((uintptr_t)x | (uintptr_t)y | (uintptr_t)n_out) & 15) == 0 && (((uintptr_t)n16 | (uintptr_t)w) & 7) == 0;
-#define MN_AR(V_) hipLaunchKernelGGL((axpy_rms_reg_kernel<V_>), dim3((unsigned)M), dim3(256), 0, st, x, ldx, y, ldy, mult, w, eps, n_out, ldn, n16, ldn16, n)
+  MN_CHECK_ARG(nz == 1 || (nz > 1 && y && vec && (zs % 4) == 0), "mn_axpy_rms_rows: slabs need rows of at most 8192 values, a multiple of 4, 16-byte aligned");
+#define MN_AR(V_) hipLaunchKernelGGL((axpy_rms_reg_kernel<V_>), dim3((unsigned)M), dim3(256), 0, st, x, ldx, y, ldy, nz, zs, mult, w, eps, n_out, ldn, n16, ldn16, n)
   if (vec && n <= 1024) MN_AR(1);
   else if (vec && n <= 2048) MN_AR(2);
   else if (vec && n <= 4096) MN_AR(4);

@@ -85,6 +85,23 @@ inline int linear_geglu_rows(int arith, int M, const uint16_t* A16, int64_t lda1
   return rc < 0 ? rc : MN_OK;
 }
 
+// Split-K slices of C fp32 [M, N] = A W^T for prompt rows whose consumer sums the slabs: 1 = one product (2048 x 2048 x 14336: 142 us in one, 93 us in four
+// plus 10 us of the norm reading them)
+inline int linear_slices(int arith, int M, int N, int K, int most) {
+  if (arith != MN_SEQ_ARITH_BF16 || M <= 64 || (K % 64) != 0 || (N % 4) != 0 || N > 8192) return 1;
+  const int ks = mn_gemm256_plan_ksplit(M, N, K, 0);
+  return ks > most ? (most > 1 ? most : 1) : (ks > 1 ? ks : 1);
+}
+// C = that many slabs M * N apart (room for linear_slices of them); *nz says how many were written, 0: the caller's plain product serves this shape
+inline int linear_slabs(int arith, int M, const uint16_t* A16, int64_t lda16, const uint16_t* W, int N, int K, int ks, float* C, void* stream, int* nz) {
+  *nz = 0;
+  if (ks <= 1 || !gemm_epilogue_ok(arith, M, A16, lda16, W, N, N, K, C, N)) return MN_OK;
+  const int rc = mn_gemm256_splitk(A16, lda16, 0, W, K, nullptr, C, M, N, K, ks, stream);
+  if (rc < 0) return rc;
+  *nz = rc;
+  return MN_OK;
+}
+
 // the step's own copy of its input rows (a kernel, not a memcpy node: the step may be captured into a graph)
 __global__ void copy_rows_kernel(const float* __restrict__ x, int64_t ldx, float* __restrict__ y, int n) {
   const int c = blockIdx.x * 256 + threadIdx.x;

@@ -84,3 +84,37 @@ def test_residual_and_rms_rows(M, n):
         check(lib().mn_axpy_rms_rows(ptr(x), n + 4, ptr(yy), n + 8, 0.5, ptr(w), 1e-5, ptr(o), n + 4, ptr(o16), n + 4, M, n, current_stream()), "axpy")
         assert rel(x[:, :n], ref) < 1e-6 and rel(o[:, :n], nrm) < 2e-6 and rel(o16[:, :n], nrm) < 2 ** -8
         assert bool((o[:, n:] == 5).all()) and bool((o16[:, n:] == 5).all())
+
+
+@pytest.mark.parametrize("T,H,d,e", [(65, 2, 16, 16), (100, 3, 20, 36), (1000, 2, 128, 128), (2100, 1, 64, 100), (70, 2, 6, 10)])
+def test_lightning_scan(T, H, d, e):
+    """The chunked recurrence around its batches of eight chunks, two sequences in one pass (one continuing), vector and scalar staging, against the
+    recurrence in float64."""
+    import numpy as np
+    from ming_univision_amd._lib import check, current_stream, lib, ptr
+    from ming_univision_amd.sequences import rows_of_spans
+    L, g = lib(), torch.Generator().manual_seed(T + d)
+    spans = [(1, T // 3, 0), (0, T - T // 3, 5)]
+    tabs = rows_of_spans(spans, 4, L.mn_lightning_chunk_rows())
+    dev = {k: torch.from_numpy(np.ascontiguousarray(v)).cuda() for k, v in tabs.items() if k != "max_len"}
+    qkv, S0 = torch.randn(T, H * (2 * d + e), generator=g), torch.randn(2, H, d, e, generator=g)
+    decay = torch.tensor([0.5, 0.97, 0.999][:H])
+    state, out = S0.cuda(), torch.empty(T, H * e, device="cuda")
+    n_ch = dev["chunk_tab"].shape[0]
+    ws = torch.empty(L.mn_lightning_scan_workspace_bytes(n_ch, H, d, e), dtype=torch.uint8, device="cuda")
+    qd, dd = qkv.cuda(), decay.cuda()
+    check(L.mn_lightning_rows_scan(ptr(qd), qkv.shape[1], T, H, d, e, ptr(dd), ptr(state), ptr(dev["row_seq"]), ptr(dev["row_slot"]), ptr(dev["row_back"]),
+                                   ptr(dev["chunk_tab"]), n_ch, ptr(out), H * e, ptr(ws), ws.numel(), current_stream()), "scan")
+    act = F.silu(qkv.double())
+    r = 0
+    for seq, n, past in spans:
+        S = S0[seq].double() * (0 if past == 0 else 1)
+        for t in range(r, r + n):
+            q, k, v = act[t, :H * d].reshape(H, d), act[t, H * d:2 * H * d].reshape(H, d), act[t, 2 * H * d:].reshape(H, e)
+            S = decay.double()[:, None, None] * S + k[:, :, None] * v[:, None, :]
+            if t in (r, r + n // 2, r + n - 1):
+                ref = torch.einsum("hde,hd->he", S, q).reshape(-1)
+                # fp32 sums of up to 1 / (1 - decay) = 1000 terms: 1e-5 of the row's largest value
+                assert float((out[t].double().cpu() - ref).abs().max() / ref.abs().max()) < 1e-5, t
+        assert rel(state[seq], S) < 1e-5
+        r += n

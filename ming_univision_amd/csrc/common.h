@@ -92,7 +92,8 @@ __device__ __forceinline__ mn_u4_t fp8x8_to_bf16(uint32_t q0, uint32_t q1) {
 // ---- activations ----------------------------------------------------------------------------
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + __expf(-x)); }
 __device__ __forceinline__ float gelu_erf_f(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f)); }
-__device__ __forceinline__ float gelu_tanh_f(float z) { return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))); }
+// z (1 + tanh u) / 2 = z / (1 + exp(-2 u)): no cancellation on the negative side, where a norm behind it would magnify the error
+__device__ __forceinline__ float gelu_tanh_f(float z) { return z / (1.0f + expf(-1.5957691216057308f * (z + 0.044715f * z * z * z))); }
 // epilogues whose weights hold two row sets per output (the second set at row n + N)
 static inline bool mn_epi_pairs(int epilogue) { return epilogue == MN_EPI_SWIGLU || epilogue == MN_EPI_GEGLU_TANH; }
 

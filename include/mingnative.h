@@ -796,7 +796,7 @@ MN_API int mn_gated_norm_filter_rows(float* x, int64_t ldx, const float* g, int6
                                      float* h, int64_t ldh, int M, int n, void* stream);
 MN_API int mn_softcap_rows(float* z, int64_t ld, int M, int n, float cap, void* stream);
 /* C[z] = alpha * A[z] W[z]^T (+ bias) (* sigmoid(G[z])) for z < batch, operands of batch entry z at base + z * (their _bs stride):
- * fp32 FMA, any M / N / K.  C (fp32) and C16 (bf16 copy) are both optional outputs. */
+ * fp32 products and sums (FMA; more than 8 rows: the fp32 matrix cores), any M / N / K.  C (fp32) and C16 (bf16 copy) are both optional outputs. */
 MN_API int mn_gemm_f32_batched(const float* A, int64_t lda, int64_t a_bs, const uint16_t* W, int64_t ldw, int64_t w_bs,
                                const uint16_t* bias, float* C, int64_t ldc, int64_t c_bs, uint16_t* C16, int64_t ldc16, int64_t c16_bs,
                                const float* G, int64_t ldg, int64_t g_bs, int M, int N, int K, int batch, float alpha, void* stream);
@@ -812,7 +812,7 @@ MN_API int mn_latent_attn(const float* qabs, const float* arena, const int32_t* 
                           int n_blk, int M, int H, int r, int t_max, int max_len, int ks, float* lat, void* workspace,
                           size_t workspace_bytes, void* stream);
 /* The same with the kernel named: MN_LATENT_ATTN_MFMA (what mn_latent_attn runs) = scores and weighted sums on the fp32 matrix
- * cores (v_mfma_f32_16x16x4_f32: fp32 operands and accumulation), 16 query vectors per workgroup, 16-key tiles;
+ * cores (v_mfma_f32_16x16x4_f32: fp32 operands and accumulation), 16 query vectors per workgroup, tiles of 32 keys (r > 512: 16);
  * MN_LATENT_ATTN_VALU = one wave per query vector on fp32 FMA (the plain kernel the other is checked against). */
 enum { MN_LATENT_ATTN_MFMA = 0, MN_LATENT_ATTN_VALU = 1 };
 MN_API int mn_latent_attn_ex(const float* qabs, const float* arena, const int32_t* row_seq, const int32_t* row_len, const int32_t* blk_tab,

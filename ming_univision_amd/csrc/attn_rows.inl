@@ -30,56 +30,6 @@ __device__ __forceinline__ void rows_table(const AttnTArgs& a, int b0, int nb, i
   __syncthreads();
 }
 
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));      // rows start at any float: a 16-byte load needs 4-byte alignment here
-
-// four consecutive values src[d .. d + 3], zero from n on (VEC: n is a multiple of 4)
-template <bool VEC>
-__device__ __forceinline__ f32x4 load4(const float* src, int d, int n, bool on) {
-  f32x4 t;
-  if (VEC) {
-    t = *reinterpret_cast<const f32x4u*>(src + (d < n ? d : 0));
-    return on && d < n ? t : f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float x = src[d + e < n ? d + e : 0];
-    t[e] = on && d + e < n ? x : 0.f;
-  }
-  return t;
-}
-
-// 16 rows x 64 NBW floats HBM -> registers (raw: a select on a loaded value would wait for it here) and registers -> LDS (zero from n on and in
-// rows that do not count): 16 threads per row, 16 bytes per thread and pass
-template <int NBW, bool VEC>
-__device__ __forceinline__ void rows_fetch(f32x4 (&v)[NBW], const float* src, int n, int cg) {
-#pragma unroll
-  for (int ps = 0; ps < NBW; ++ps) {
-    const int d = 4 * (cg + 16 * ps);
-    if (VEC) {
-      v[ps] = *reinterpret_cast<const f32x4u*>(src + (d < n ? d : 0));
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[ps][e] = src[d + e < n ? d + e : 0];
-    }
-  }
-}
-template <int NBW, int LDC, bool VEC>
-__device__ __forceinline__ void rows_put(float* __restrict__ dst, const f32x4 (&v)[NBW], int n, int j, int cg, bool ok) {
-#pragma unroll
-  for (int ps = 0; ps < NBW; ++ps) {
-    const int d = 4 * (cg + 16 * ps);
-    f32x4 t = v[ps];
-    if (VEC) {
-      if (!(ok && d < n)) t = f32x4{0.f, 0.f, 0.f, 0.f};
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (!(ok && d + e < n)) t[e] = 0.f;
-    }
-    *reinterpret_cast<f32x4*>(dst + j * LDC + d) = t;
-  }
-}
-
 // values d .. d + 3 of one query vector's result
 __device__ __forceinline__ void emit4(const AttnTArgs& a, f32x4 v, int row, int64_t col0, int d, bool vec) {
 #pragma unroll
@@ -449,4 +399,44 @@ __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, i
     }
     s0 = s1;
   }
+}
+
+// Decode rows whose values lie inside the keys: workgroup b takes row b and up to 16 of its query heads (the walk: mfma_f32_tiles.h).
+struct SoftCap { float cap; __device__ __forceinline__ float operator()(float s) const { return soft_cap(s, cap); } };
+template <int NB, int KF, bool VEC>
+__global__ __launch_bounds__(256) void attn_latent_decode_kernel(AttnTArgs a) {
+  using Walk = LatentWalk<NB, KF, VEC, SoftCap>;
+  constexpr int KT = Walk::KT, AQ = 16;
+  __shared__ __attribute__((aligned(16))) float lds[Walk::LDS_FLOATS];
+  const int tid = threadIdx.x, b = blockIdx.x, gy = blockIdx.y, sp = blockIdx.z;
+  const int rep = a.H / a.G, chunks = (rep + a.hpc - 1) / a.hpc;
+  const int g = gy / chunks, h0 = g * rep + (gy % chunks) * a.hpc;
+  const int Rc = min(a.hpc, g * rep + rep - h0);
+  const int seq = a.row_seq[b], pos = a.row_slot[b], tF = first_key(a, pos);
+  const int nk = pos - tF + 1;
+  const int ntile = (nk + KT - 1) / KT, tps = (ntile + a.nsplit - 1) / a.nsplit;
+  const int t0 = sp * tps, t1 = min(ntile, t0 + tps);
+  const int wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
+  const float* src = a.q + (int64_t)b * a.ldq + (int64_t)(h0 + min(c, Rc - 1)) * a.dim;
+  f32x4 q[NB], acc[NB];
+#pragma unroll
+  for (int it = 0; it < NB; ++it) q[it] = load4<VEC>(src, wave * 16 * NB + 16 * it + 4 * g4, a.dim, c < Rc);
+  float mrun, lrun;
+  Walk::run(lds, a.k + ((int64_t)seq * a.t_max + tF) * a.ldk + (int64_t)g * a.dim, a.ldk, a.dim, nk, nk, t0, t1, q, SoftCap{a.cap}, mrun, lrun, acc);
+  if (c >= Rc) return;
+  float* part = a.nsplit > 1 ? a.part + (((int64_t)b * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)AQ * (2 + a.vdim)) : nullptr;
+  const bool vec = emit_vec(a);
+  const int64_t col0 = (int64_t)(h0 + c) * a.vdim;
+  const float inv = part ? 1.f : a.out_scale * softmax_inv(mrun, lrun, a.sink, h0 + c);
+#pragma unroll
+  for (int x = 0; x < NB; ++x) {
+    const int d = 16 * (wave + 4 * x) + 4 * g4;
+    if (d >= a.vdim) continue;
+    const f32x4 r = acc[x] * inv;
+    if (!part) { emit4(a, r, b, col0, d, vec); continue; }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (d + e < a.vdim) part[2 * AQ + (int64_t)c * a.vdim + d + e] = r[e];
+  }
+  if (part && wave == 0 && g4 == 0) { part[c] = mrun; part[AQ + c] = lrun; }
 }

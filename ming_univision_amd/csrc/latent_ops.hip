@@ -242,8 +242,6 @@ struct GemmF32 {
   float alpha;
 };
 
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ void f32_store(const GemmF32& a, int z, int m, int n, float v) {
   if (m >= a.M || n >= a.N) return;
   v *= a.alpha;
@@ -279,7 +277,7 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(GemmF32 a) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) ap[i] = a.A + (int64_t)z * a.a_bs + (int64_t)min(m0 + 16 * i + r, a.M - 1) * a.lda;
   const bf16_t* wp = a.W + (int64_t)z * a.w_bs + (int64_t)min(n0 + r, a.N - 1) * a.ldw;
-  f32x4_t fa[2][2];
+  f32x4 fa[2][2];
   ushort4 fw[2];
   float sum[8], low[8];
 #pragma unroll
@@ -291,8 +289,8 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(GemmF32 a) {
       fw[u] = ushort4{0, 0, 0, 0};
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        fa[u][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        if (V4) { if (k < ke) fa[u][i] = *reinterpret_cast<const f32x4_t*>(ap[i] + k); }
+        fa[u][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (V4) { if (k < ke) fa[u][i] = *reinterpret_cast<const f32x4*>(ap[i] + k); }
         else
 #pragma unroll
           for (int t = 0; t < 4; ++t) if (k + t < ke) fa[u][i][t] = ap[i][k + t];
@@ -308,11 +306,11 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(GemmF32 a) {
   };
   if (kb < ke) fetch(kb);
   for (int k0 = kb; k0 < ke; k0 += 32) {
-    f32x4_t ca[2][2], cw[2], p[2][4][2];
+    f32x4 ca[2][2], cw[2], p[2][4][2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       ca[u][0] = fa[u][0]; ca[u][1] = fa[u][1];
-      cw[u] = f32x4_t{bf16_to_f32(fw[u].x), bf16_to_f32(fw[u].y), bf16_to_f32(fw[u].z), bf16_to_f32(fw[u].w)};
+      cw[u] = f32x4{bf16_to_f32(fw[u].x), bf16_to_f32(fw[u].y), bf16_to_f32(fw[u].z), bf16_to_f32(fw[u].w)};
     }
     if (k0 + 32 < ke) fetch(k0 + 32);
 #pragma unroll
@@ -320,7 +318,7 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(GemmF32 a) {
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) p[u][t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ca[u][i][t], cw[u][t], f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        for (int i = 0; i < 2; ++i) p[u][t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ca[u][i][t], cw[u][t], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int i = e >> 2, c = e & 3;
@@ -355,24 +353,24 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(GemmF32 a) {
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64, wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
   const float* A = a.A + (int64_t)z * a.a_bs;
   const bf16_t* W = a.W + (int64_t)z * a.w_bs;
-  f32x4_t acc[2][2][2], fa[2];
+  f32x4 acc[2][2][2], fa[2];
   ushort4 fw[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[u][i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < 2; ++j) acc[u][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {                             // rows past the matrix repeat its last one; nothing of them is stored
       const int e = tid + 256 * t, row = e >> 3, k = k0 + 4 * (e & 7);
       const float* ap = A + (int64_t)min(m0 + row, a.M - 1) * a.lda;
       const bf16_t* wp = W + (int64_t)min(n0 + row, a.N - 1) * a.ldw;
-      fa[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      fa[t] = f32x4{0.f, 0.f, 0.f, 0.f};
       fw[t] = ushort4{0, 0, 0, 0};
       if (V4) {
-        if (k < a.K) { fa[t] = *reinterpret_cast<const f32x4_t*>(ap + k); fw[t] = *reinterpret_cast<const ushort4*>(wp + k); }
+        if (k < a.K) { fa[t] = *reinterpret_cast<const f32x4*>(ap + k); fw[t] = *reinterpret_cast<const ushort4*>(wp + k); }
       } else {
 #pragma unroll
         for (int c = 0; c < 4; ++c) if (k + c < a.K) fa[t][c] = ap[k + c];
@@ -387,8 +385,8 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(GemmF32 a) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int e = tid + 256 * t, at = (e >> 3) * LD + 4 * (e & 7);
-      *reinterpret_cast<f32x4_t*>(&As[b][at]) = fa[t];
-      *reinterpret_cast<f32x4_t*>(&Ws[b][at]) = f32x4_t{bf16_to_f32(fw[t].x), bf16_to_f32(fw[t].y), bf16_to_f32(fw[t].z), bf16_to_f32(fw[t].w)};
+      *reinterpret_cast<f32x4*>(&As[b][at]) = fa[t];
+      *reinterpret_cast<f32x4*>(&Ws[b][at]) = f32x4{bf16_to_f32(fw[t].x), bf16_to_f32(fw[t].y), bf16_to_f32(fw[t].z), bf16_to_f32(fw[t].w)};
     }
   };
   fetch(0);
@@ -400,11 +398,11 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(GemmF32 a) {
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      f32x4_t ra[2], rw[2];
+      f32x4 ra[2], rw[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        ra[i] = *reinterpret_cast<const f32x4_t*>(&As[b][(wm + 16 * i + r) * LD + 16 * u + 4 * q]);
-        rw[i] = *reinterpret_cast<const f32x4_t*>(&Ws[b][(wn + 16 * i + r) * LD + 16 * u + 4 * q]);
+        ra[i] = *reinterpret_cast<const f32x4*>(&As[b][(wm + 16 * i + r) * LD + 16 * u + 4 * q]);
+        rw[i] = *reinterpret_cast<const f32x4*>(&Ws[b][(wn + 16 * i + r) * LD + 16 * u + 4 * q]);
       }
 #pragma unroll
       for (int t = 0; t < 4; ++t)
@@ -516,17 +514,11 @@ __global__ __launch_bounds__(256) void row_fused_kernel(FusedRowArgs a) {
   }
 }
 
-// C[z][m, n] = alpha * A[z][m, :] . W[z][n, :] (+ bias) (* sigmoid(G)) for few rows: one wave per output column and MM rows, lanes over K
+// C[z][m, n] = alpha * A[z][m, :] . W[z][n, :] (+ bias) (* sigmoid(G)) for at most MM rows: one wave per output column, lanes over K
 template <int MM>
 __global__ __launch_bounds__(256) void gemv_f32_kernel(GemmF32 a) {
   const int z = blockIdx.z, n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (n >= a.N) return;
-  const int m0 = blockIdx.y * MM;                       // this workgroup's rows: m0 .. m0 + MM - 1
-  a.M -= m0;
-  a.A += (int64_t)m0 * a.lda;
-  if (a.C) a.C += (int64_t)m0 * a.ldc;
-  if (a.C16) a.C16 += (int64_t)m0 * a.ldc16;
-  if (a.G) a.G += (int64_t)m0 * a.ldg;
   const float* A = a.A + (int64_t)z * a.a_bs;
   const bf16_t* Wr = a.W + (int64_t)z * a.w_bs + (int64_t)n * a.ldw;
   float acc[MM];
@@ -642,131 +634,54 @@ __global__ __launch_bounds__(1024) void latent_attn_kernel(const float* __restri
 
 // ---------------------------------------------------------------------------------------------------------------------------
 // Latent attention on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands, fp32 accumulate — scores and weights stay
-// 32-bit).  A workgroup of 4 waves owns 16 query vectors (row, head) of one run of rows and walks the sequence's latents in tiles
-// of 16 keys staged in LDS:
-//   scores   S[16 q, 16 keys] = Q C^T: every wave multiplies its quarter of the latent components (its slice of Q stays in
-//            registers), the partial tiles are summed through LDS, so all four waves hold the same scores and keep the same
-//            running maximum / sum without talking
-//   values   O[16 q, r] += P C: the weights go through LDS into the A-operand layout, wave w owns the 16-column blocks w, w + 4, ..
-// Operand layouts (lane l, c = l % 16, g = l / 16): A[row c][k g], B[k g][col c], D[row 4 g + i][col c] in VGPR i.
-// (f32x4, load16 / store16, lds_barrier, fast_exp: mfma_f32_tiles.h)
-
-template <int NBW>
+// 32-bit).  A workgroup of 4 waves owns 16 query vectors (row, head) of one run of rows and walks its share of the sequence's latents
+// (LatentWalk, mfma_f32_tiles.h).
+// 32 rows of 16 heads over 2049 latents of 512 (134 MB, 28 us at the card's copy rate): 46 us (2.9 TB/s; a plain sum over
+// as much reaches 3.2); with the loads of the next tile waited for where they were issued, 16 keys a tile and four times the workgroups 60 us (8 rows: 60 us,
+// 18 here).
+struct PlainScore { __device__ __forceinline__ float operator()(float s) const { return s; } };
+template <int NB, int KF, bool VEC>
 __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __restrict__ qabs, const float* __restrict__ arena,
                                                                const int32_t* __restrict__ row_seq, const int32_t* __restrict__ row_len,
                                                                const int32_t* __restrict__ blk_tab, int H, int r, int t_max,
                                                                int tiles_per_split, float* __restrict__ lat, float* __restrict__ part_acc,
                                                                float* __restrict__ part_ml, int KS, int M) {
-  // the latent is padded with zeros to RP = 64 NBW components: every loop below has a compile-time trip count
-  constexpr int KT = 16, LDP = 20, LDS_S = 17, RP = 64 * NBW, LDC = RP + 4, DQ = RP / 4;
-  extern __shared__ float lds[];
+  using Walk = LatentWalk<NB, KF, VEC, PlainScore>;
+  __shared__ __attribute__((aligned(16))) float lds[Walk::LDS_FLOATS];
   const int row0 = blk_tab[2 * blockIdx.x], nrows = blk_tab[2 * blockIdx.x + 1];
   const int nqv = nrows * H, qv0 = blockIdx.y * 16;
   if (qv0 >= nqv) return;
-  float* Cl = lds;                       // [16 keys][LDC]
-  float* Sp = Cl + KT * LDC;             // [4 waves][16 q][LDS_S] partial scores
-  float* Pl = Sp + 4 * 16 * LDS_S;       // [16 q][LDP] weights
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c16 = lane & 15, g4 = lane >> 4;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
   const int64_t seq = row_seq[row0];
-  const int len_max = row_len[row0 + nrows - 1];
-  f32x4 v[NBW];
-  // the A operands of this wave's score products stay in registers for the whole key walk: query c16, components wave DQ + 4 it + g4
-  float qreg[DQ / 4];
-  {
-    const int qv = min(qv0 + c16, nqv - 1);
-    const float* src = qabs + ((int64_t)(row0 + qv / H) * H + qv % H) * r;
+  const int len = row_len[row0 + nrows - 1];
+  const bool on = qv0 + c < nqv;
+  const int qv = on ? qv0 + c : nqv - 1;
+  const int64_t o = (int64_t)(row0 + qv / H) * H + qv % H;
+  f32x4 q[NB], acc[NB];
 #pragma unroll
-    for (int it = 0; it < DQ / 4; ++it) {
-      const int d = wave * DQ + 4 * it + g4;
-      const float t = src[d < r ? d : 0];
-      qreg[it] = (qv0 + c16 < nqv && d < r) ? t : 0.f;
-    }
-  }
-  int mylen[4];
-  float mrun[4], lrun[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int qv = qv0 + 4 * g4 + i;
-    mylen[i] = qv < nqv ? row_len[row0 + qv / H] : 0;
-    mrun[i] = -INFINITY;
-    lrun[i] = 0.f;
-  }
-  f32x4 acc[NBW];
-#pragma unroll
-  for (int b = 0; b < NBW; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int n_tiles = (len_max + KT - 1) / KT;
+  for (int it = 0; it < NB; ++it) q[it] = load4<VEC>(qabs + o * r, wave * 16 * NB + 16 * it + 4 * g4, r, on);
+  const int n_tiles = (len + Walk::KT - 1) / Walk::KT;
   const int t0 = blockIdx.z * tiles_per_split, t1 = min(t0 + tiles_per_split, n_tiles);
-  const float* abase = arena + seq * t_max * r;
-  auto fetch = [&](int tile) {
-    const int k0 = tile * KT;
-    load16<NBW>(v, r, tid, [&](int j) { return abase + (int64_t)min(k0 + j, len_max - 1) * r; }, [&](int j) { return k0 + j < len_max; });
-  };
-  if (t0 < t1) fetch(t0);
-  for (int tile = t0; tile < t1; ++tile) {
-    const int key0 = tile * KT;
-    lds_barrier();                                             // the previous tile's latents and weights are consumed
-    store16<NBW, LDC>(Cl, v, tid);
-    if (tile + 1 < t1) fetch(tile + 1);                          // in flight while this tile is multiplied
-    lds_barrier();
-    {                                                            // partial scores over this wave's quarter of the components
-      f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f}, s2 = f32x4{0.f, 0.f, 0.f, 0.f};      // two chains: a product does not wait for the one before it
-      const float* cb = Cl + c16 * LDC + wave * DQ + g4;
+  float mrun, lrun;
+  Walk::run(lds, arena + seq * t_max * r, r, r, len, on ? row_len[row0 + qv / H] : len, t0, t1, q, PlainScore{}, mrun, lrun, acc);
+  if (!on) return;
+  const float inv = KS == 1 ? 1.0f / lrun : 1.0f;
+  float* dst = KS == 1 ? lat + o * r : part_acc + ((int64_t)blockIdx.z * M * H + o) * r;
 #pragma unroll
-      for (int it = 0; it < DQ / 4; it += 2) {
-        s = __builtin_amdgcn_mfma_f32_16x16x4f32(qreg[it], cb[4 * it], s, 0, 0, 0);
-        s2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qreg[it + 1], cb[4 * it + 4], s2, 0, 0, 0);
-      }
-      s += s2;
+  for (int x = 0; x < NB; ++x) {
+    const int d = 16 * (wave + 4 * x) + 4 * g4;
+    if (VEC) {
+      if (d < r) *reinterpret_cast<f32x4u*>(dst + d) = acc[x] * inv;
+    } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) Sp[(wave * 16 + 4 * g4 + i) * LDS_S + c16] = s[i];
-    }
-    lds_barrier();
-    float p[4], corr[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int o = (4 * g4 + i) * LDS_S + c16;
-      float sc = (Sp[o] + Sp[16 * LDS_S + o]) + (Sp[32 * LDS_S + o] + Sp[48 * LDS_S + o]);
-      if (key0 + c16 >= mylen[i]) sc = -INFINITY;
-      const float mnew = fmaxf(mrun[i], row16_max(sc));
-      p[i] = (sc == -INFINITY) ? 0.f : fast_exp(sc - mnew);
-      corr[i] = (mrun[i] == -INFINITY) ? 0.f : fast_exp(mrun[i] - mnew);
-      lrun[i] = lrun[i] * corr[i] + row16_sum(p[i]);
-      mrun[i] = mnew;
-      if (wave == 0) Pl[(4 * g4 + i) * LDP + c16] = p[i];
-    }
-#pragma unroll
-    for (int b = 0; b < NBW; ++b)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[b][i] *= corr[i];
-    lds_barrier();
-    // step t multiplies keys t, t + 4, t + 8, t + 12 (lane group g4 holds key t + 4 g4): with the row stride 4 mod 32 their rows
-    // start 16 banks apart pairwise, so the 64 lanes' reads spread two per bank — consecutive keys would pile four on some
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float pa = Pl[c16 * LDP + t + 4 * g4];
-      const float* cb = Cl + (t + 4 * g4) * LDC + 16 * wave + c16;
-#pragma unroll
-      for (int b = 0; b < NBW; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, cb[64 * b], acc[b], 0, 0, 0);
+      for (int e = 0; e < 4; ++e)
+        if (d + e < r) dst[d + e] = acc[x][e] * inv;
     }
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int qv = qv0 + 4 * g4 + i;
-    if (qv >= nqv) continue;
-    const int64_t o = (int64_t)(row0 + qv / H) * H + qv % H;
-    const float inv = 1.0f / lrun[i];
-#pragma unroll
-    for (int b = 0; b < NBW; ++b) {
-      const int d = 16 * (wave + 4 * b) + c16;
-      if (d >= r) continue;
-      if (KS == 1) lat[o * r + d] = acc[b][i] * inv;
-      else part_acc[((int64_t)blockIdx.z * M * H + o) * r + d] = acc[b][i];
-    }
-    if (KS > 1 && wave == 0 && c16 == 0) {
-      const int64_t po = (int64_t)blockIdx.z * M * H + o;
-      part_ml[po * 2] = mrun[i];
-      part_ml[po * 2 + 1] = lrun[i];
-    }
+  if (KS > 1 && wave == 0 && g4 == 0) {
+    const int64_t po = (int64_t)blockIdx.z * M * H + o;
+    part_ml[po * 2] = mrun;
+    part_ml[po * 2 + 1] = lrun;
   }
 }
 
@@ -926,7 +841,10 @@ extern "C" int mn_gemm_f32_batched(const float* A, int64_t lda, int64_t a_bs, co
 
 // rows of a workgroup (consecutive rows of one sequence) and the key-tile length for latent size r
 extern "C" int mn_latent_attn_block_rows(void) { return 4; }
-static inline int latent_kt(int r, int variant) { return variant == MN_LATENT_ATTN_VALU ? (r <= 256 ? 64 : r <= 512 ? 32 : 16) : 16; }   // VALU: the tile [KT][r + 1] fp32 stays below 66 KiB
+static inline int latent_kt(int r, int variant) {
+  // VALU: the tile [KT][r + 1] fp32 stays below 66 KiB; MFMA: 32 keys while two such tiles fit a CU's LDS
+  return variant == MN_LATENT_ATTN_VALU ? (r <= 256 ? 64 : r <= 512 ? 32 : 16) : (r <= 512 ? 32 : 16);
+}
 
 extern "C" int mn_latent_attn_splits(int n_blk, int max_len, int r) {
   const int tiles = (int)mn_cdiv(max_len > 0 ? max_len : 1, 16);
@@ -958,24 +876,17 @@ extern "C" int mn_latent_attn_ex(const float* qabs, const float* arena, const in
   hipStream_t st = mn_stream(stream);
   if (variant == MN_LATENT_ATTN_MFMA) {
     const int nbw = (int)mn_cdiv(r, 64);
-    const int inst = nbw <= 4 ? nbw : nbw <= 6 ? 6 : nbw <= 8 ? 8 : nbw <= 12 ? 12 : 16;      // instantiated paddings: 64 .. 256, 384, 512, 768, 1024
-    const size_t lds = ((size_t)16 * (64 * inst + 4) + 4 * 16 * 17 + 16 * 20) * sizeof(float);
-    const dim3 grid((unsigned)n_blk, (unsigned)mn_cdiv(RB * H, 16), (unsigned)ks);
-    MN_CHECK_ARG(grid.y <= 65535 && ks <= 64, "mn_latent_attn: too many heads or key splits");
-#define MN_LM(N_)                                                                                                                   \
-  do {                                                                                                                              \
-    static bool attr_set = false;                                                                                                   \
-    if (!attr_set) {                                                                                                                \
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(latent_attn_mfma_kernel<N_>), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                144 * 1024);                                                                                        \
-      attr_set = true;                                                                                                              \
-    }                                                                                                                               \
-    hipLaunchKernelGGL((latent_attn_mfma_kernel<N_>), grid, dim3(256), lds, st, qabs, arena, row_seq, row_len, blk_tab, H, r, t_max, tps, \
-                       lat, pacc, pml, ks, M);                                                                                      \
-  } while (0)
-    switch (inst) {
-      case 1: MN_LM(1); break; case 2: MN_LM(2); break; case 3: MN_LM(3); break; case 4: MN_LM(4); break;
-      case 6: MN_LM(6); break; case 8: MN_LM(8); break; case 12: MN_LM(12); break; default: MN_LM(16); break;
+    // as many runs as rows: one row each (workgroups for the rows a run does not have still wait for their LDS: 3 of 4 in a decode step)
+    const dim3 grid((unsigned)n_blk, (unsigned)mn_cdiv((n_blk == M ? 1 : RB) * H, 16), (unsigned)ks);
+    MN_CHECK_ARG(mn_cdiv(RB * H, 16) <= 65535 && ks <= 64, "mn_latent_attn: too many heads or key splits");
+#define MN_LM(N_, F_, V_)                                                                                                           \
+  hipLaunchKernelGGL((latent_attn_mfma_kernel<N_, F_, V_>), grid, dim3(256), 0, st, qabs, arena, row_seq, row_len, blk_tab, H, r, t_max, tps, lat, pacc, \
+                     pml, ks, M)
+    if (r & 3) {                                         // (latents of any size but a multiple of 4 go value by value)
+      if (nbw <= 2) MN_LM(2, 2, false); else if (nbw <= 8) MN_LM(8, 2, false); else MN_LM(16, 1, false);
+    } else {                                             // instantiated paddings: 64 .. 256, 384, 512, 768, 1024
+      if (nbw == 1) MN_LM(1, 2, true); else if (nbw == 2) MN_LM(2, 2, true); else if (nbw == 3) MN_LM(3, 2, true); else if (nbw == 4) MN_LM(4, 2, true);
+      else if (nbw <= 6) MN_LM(6, 2, true); else if (nbw <= 8) MN_LM(8, 2, true); else if (nbw <= 12) MN_LM(12, 1, true); else MN_LM(16, 1, true);
     }
 #undef MN_LM
   } else {

@@ -756,128 +756,6 @@ __global__ __launch_bounds__(256) void window_attn_tiled_kernel(AttnTArgs a) {
   }
 }
 
-// Latent attention of decode rows on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: scores and weights stay 32-bit): the values are the first
-// columns of the keys (one key/value head whose value arena is a view of the key arena).  Workgroup b of 4 waves takes row b and up to
-// 16 of its query heads and walks the row's keys in tiles of 16, staged through registers into LDS while the previous tile is multiplied:
-//   scores   S[16 q, 16 keys] = Q K^T: every wave multiplies its quarter of the head's values (its slice of Q stays in registers),
-//            the partial tiles are summed through LDS, so all four waves hold the same scores, apply the same per-(row, key)
-//            visibility and keep the same running maximum / sum
-//   values   O[16 q, vdim] += P V from the same staged tile: the weights go through LDS into the A-operand layout, wave w owns the 16-column
-//            blocks w, w + 4, ..
-// NBD: 64-value blocks of a key (zero padded).  Key splits write the same partial layout as the tiled form.  (Runs of rows: attn_rows.inl.)
-template <int NBD>
-__global__ __launch_bounds__(256) void window_attn_mfma_kernel(AttnTArgs a) {
-  constexpr int NBV = NBD, KT = 16, LDP = 20, LDS_S = 17, DP = 64 * NBD, LDK = DP + 4, LDV = LDK, DQ = DP / 4, AQ = 16;
-  extern __shared__ float lds[];
-  const int tid = threadIdx.x, b = blockIdx.x, gy = blockIdx.y, sp = blockIdx.z;
-  const int rep = a.H / a.G, chunks = (rep + a.hpc - 1) / a.hpc;
-  const int g = gy / chunks, h0 = g * rep + (gy % chunks) * a.hpc;
-  const int Rc = min(a.hpc, g * rep + rep - h0);
-  const int nqv = Rc, seq = a.row_seq[b], pos = a.row_slot[b], tF = first_key(a, pos);
-  const int nk = pos - tF + 1;
-  const int ntile = (nk + KT - 1) / KT, tps = (ntile + a.nsplit - 1) / a.nsplit;
-  const int t0 = sp * tps, t1 = min(ntile, t0 + tps);
-  float* Kl = lds;                       // [16 keys][LDK]
-  float* Sp = Kl + KT * LDK;             // [4 waves][16 q][LDS_S] partial scores
-  float* Pl = Sp + 4 * 16 * LDS_S;       // [16 q][LDP] weights
-  const int wave = tid >> 6, lane = tid & 63, c16 = lane & 15, g4 = lane >> 4;
-  // the A operands of this wave's score products stay in registers for the whole key walk: query c16, values wave DQ + 4 it + g4
-  float qreg[DQ / 4];
-  {
-    const int qv = min(c16, nqv - 1);
-    const float* src = a.q + (int64_t)b * a.ldq + (int64_t)(h0 + qv) * a.dim;
-#pragma unroll
-    for (int it = 0; it < DQ / 4; ++it) {
-      const int d = wave * DQ + 4 * it + g4;
-      const float t = src[d < a.dim ? d : 0];
-      qreg[it] = (c16 < nqv && d < a.dim) ? t : 0.f;
-    }
-  }
-  float mrun[4], lrun[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) { mrun[i] = -INFINITY; lrun[i] = 0.f; }
-  f32x4 acc[NBV];
-#pragma unroll
-  for (int c = 0; c < NBV; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const float* kb = a.k + ((int64_t)seq * a.t_max + tF) * a.ldk + (int64_t)g * a.dim;
-  f32x4 vk[NBD];
-  auto fetch = [&](int tile) {
-    const int k0 = tile * KT;
-    load16<NBD>(vk, a.dim, tid, [&](int j) { return kb + (int64_t)min(k0 + j, nk - 1) * a.ldk; }, [&](int j) { return k0 + j < nk; });
-  };
-  if (t0 < t1) fetch(t0);
-  for (int tile = t0; tile < t1; ++tile) {
-    const int key0 = tile * KT;
-    lds_barrier();                                             // the previous tile's keys, values and weights are consumed
-    store16<NBD, LDK>(Kl, vk, tid);
-    if (tile + 1 < t1) fetch(tile + 1);                          // in flight while this tile is multiplied
-    lds_barrier();
-    {                                                            // partial scores over this wave's quarter of the head's values
-      f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f}, s2 = f32x4{0.f, 0.f, 0.f, 0.f};
-      const float* cb = Kl + c16 * LDK + wave * DQ + g4;
-#pragma unroll
-      for (int it = 0; it < DQ / 4; it += 2) {
-        s = __builtin_amdgcn_mfma_f32_16x16x4f32(qreg[it], cb[4 * it], s, 0, 0, 0);
-        s2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qreg[it + 1], cb[4 * it + 4], s2, 0, 0, 0);
-      }
-      s += s2;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) Sp[(wave * 16 + 4 * g4 + i) * LDS_S + c16] = s[i];
-    }
-    lds_barrier();
-    float corr[4];
-    const int j = key0 + c16;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int o = (4 * g4 + i) * LDS_S + c16;
-      float sc = soft_cap((Sp[o] + Sp[16 * LDS_S + o]) + (Sp[32 * LDS_S + o] + Sp[48 * LDS_S + o]), a.cap);
-      if (j >= nk || 4 * g4 + i >= nqv) sc = -INFINITY;
-      const float mnew = fmaxf(mrun[i], row16_max(sc));
-      const float p = (sc == -INFINITY) ? 0.f : fast_exp(sc - mnew);
-      corr[i] = (mrun[i] == -INFINITY) ? 0.f : fast_exp(mrun[i] - mnew);
-      lrun[i] = lrun[i] * corr[i] + row16_sum(p);
-      mrun[i] = mnew;
-      if (wave == 0) Pl[(4 * g4 + i) * LDP + c16] = p;
-    }
-#pragma unroll
-    for (int c = 0; c < NBV; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[c][i] *= corr[i];
-    lds_barrier();
-    // step t multiplies keys t, t + 4, t + 8, t + 12 (lane group g4 holds key t + 4 g4): with the row stride 4 mod 32 their rows
-    // start 16 banks apart pairwise
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float pa = Pl[c16 * LDP + t + 4 * g4];
-      const float* cb = Kl + (t + 4 * g4) * LDV + 16 * wave + c16;
-#pragma unroll
-      for (int c = 0; c < NBV; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, cb[64 * c], acc[c], 0, 0, 0);
-    }
-  }
-  float* part_out = a.nsplit > 1 ? a.part + (((int64_t)b * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)AQ * (2 + a.vdim)) : nullptr;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int qv = 4 * g4 + i;
-    if (qv >= nqv) continue;
-    const int row = b;
-    const int64_t col0 = (int64_t)(h0 + qv) * a.vdim;
-    const float inv = a.out_scale * softmax_inv(mrun[i], lrun[i], a.sink, h0 + qv);
-#pragma unroll
-    for (int c = 0; c < NBV; ++c) {
-      const int d = 16 * (wave + 4 * c) + c16;
-      if (d >= a.vdim) continue;
-      if (part_out) {
-        part_out[2 * AQ + (int64_t)qv * a.vdim + d] = acc[c][i];
-      } else {
-        const float val = gated(a, acc[c][i] * inv, row, col0 + d);
-        if (a.out) a.out[(int64_t)row * a.ldo + col0 + d] = val;
-        if (a.out16) a.out16[(int64_t)row * a.ldo16 + col0 + d] = f32_to_bf16(val);
-      }
-    }
-    if (part_out && wave == 0 && c16 == 0) { part_out[qv] = mrun[i]; part_out[AQ + qv] = lrun[i]; }
-  }
-}
-
 #include "attn_rows.inl"
 
 // grid (n_blk, G * chunks, ceil(vdim / MERGE_COLS)): the splits' statistics and sums of every vector become its result; a workgroup
@@ -1338,7 +1216,7 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
                "mn_window_pool_attn_blocks: the matrix-core kernel takes runs of rows with dim, vdim <= 256, or values inside keys of dim <= 640");
   if (variant == MN_WINDOW_ATTN_MFMA) {
     hipStream_t stm = mn_stream(stream);
-    const int nb = dim <= 256 ? (dim + 63) / 64 : (dim <= 320 ? 5 : (dim <= 384 ? 6 : (dim <= 512 ? 8 : 10)));
+    
     if (!one_row) {                                    // runs of rows: 64 query vectors per workgroup
       const int hv = attn_rows_heads(H / G);
       dim3 gridr((unsigned)mn_cdiv(n_blk, attn_rows_runs(H / G)), (unsigned)(G * sh.chunks), (unsigned)nsplit);
@@ -1379,18 +1257,23 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
 #undef MN_WL
 #undef MN_WR
     } else {                                           // decode rows whose values lie inside the keys
+      const int nb = dim <= 384 ? (dim + 63) / 64 : (dim <= 512 ? 8 : (dim <= 576 ? 9 : 10));
       const dim3 gridm((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)nsplit);
-      const size_t ldsm = ((size_t)16 * (64 * nb + 4) + 4 * 16 * 17 + 16 * 20) * sizeof(float);
-#define MN_WK(D_) hipLaunchKernelGGL((window_attn_mfma_kernel<D_>), gridm, dim3(256), ldsm, stm, a)
-      switch (nb) {
-        case 1: MN_WK(1); break;
-        case 2: MN_WK(2); break;
-        case 3: MN_WK(3); break;
-        case 4: MN_WK(4); break;
-        case 5: MN_WK(5); break;
-        case 6: MN_WK(6); break;
-        case 8: MN_WK(8); break;
-        default: MN_WK(10); break;
+#define MN_WK(D_, F_, E_) hipLaunchKernelGGL((attn_latent_decode_kernel<D_, F_, E_>), gridm, dim3(256), 0, stm, a)
+      if ((dim | vdim) & 3) {                          // (rows of any size but a multiple of 4 go value by value)
+        if (nb <= 2) MN_WK(2, 2, false); else if (nb <= 5) MN_WK(5, 2, false); else MN_WK(10, 1, false);
+      } else {
+        switch (nb) {                                  // 32 keys a tile while two such tiles fit a CU's LDS, else 16
+          case 1: MN_WK(1, 2, true); break;
+          case 2: MN_WK(2, 2, true); break;
+          case 3: MN_WK(3, 2, true); break;
+          case 4: MN_WK(4, 2, true); break;
+          case 5: MN_WK(5, 2, true); break;
+          case 6: MN_WK(6, 2, true); break;
+          case 8: MN_WK(8, 2, true); break;
+          case 9: MN_WK(9, 1, true); break;
+          default: MN_WK(10, 1, true); break;
+        }
       }
 #undef MN_WK
     }

@@ -65,3 +65,46 @@ def test_three_splits_of_many_groups():
     """More than 256 workgroups in a head and split: every group exactly once whatever the launch order."""
     run([(0, 700, 0), (1, 700, 0), (2, 700, 0)], 5, 1, 16, 16, 0, 0.0, 0, False, 3, 704)
     run([(0, 700, 0), (1, 701, 0)], 4, 1, 32, 32, 0, 0.0, 0, True, 3, 704)
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 32, 33, 300])
+@pytest.mark.parametrize("H,r,e", [(4, 64, 48), (16, 128, 128), (7, 35, 19), (1, 200, 200), (20, 256, 192), (5, 442, 442), (16, 512, 448), (9, 576, 512), (3, 640, 512),
+                                   (2, 700, 0), (17, 1024, 0), (1, 33, 0), (2, 130, 0), (2, 513, 0), (2, 1022, 0)])
+def test_decode_rows_over_latents(n, H, r, e):
+    """One row a sequence, values inside the keys: n, n + 1 and 1 keys, with and without key splits, a window and a soft cap, heads beyond 16.  e = 0:
+    only mn_latent_attn takes the size."""
+    from ming_univision_amd._lib import check, current_stream, lib, ptr
+    L = lib()
+    g = torch.Generator().manual_seed(n + H + r)
+    lens, t_max = [n, n + 1, 1], 304
+    k = torch.randn(3, t_max, r, generator=g)
+    q = torch.randn(3, H * r, generator=g) * r ** -0.5
+    kd, qd = k.cuda(), q.cuda()
+    seq, ln = torch.arange(3, dtype=torch.int32, device="cuda"), torch.tensor(lens, dtype=torch.int32, device="cuda")
+    slot = ln - 1
+    blk = torch.stack([seq, torch.ones_like(seq)], 1).contiguous()
+
+    def want(cols, window=0, cap=0.0):
+        out = []
+        for i, m in enumerate(lens):
+            first = max(0, m - window) if window else 0
+            s = q[i].reshape(H, r).double() @ k[i, first:m].double().T
+            s = cap * torch.tanh(s / cap) if cap else s
+            out.append(torch.softmax(s, -1) @ k[i, first:m, :cols].double())
+        return torch.stack(out)
+
+    for ks in (1, 3):
+        lat = torch.full((4, H, r), 7.0, device="cuda")
+        ws = torch.empty(max(16, L.mn_latent_attn_workspace_bytes(3, H, r, ks)), dtype=torch.uint8, device="cuda")
+        check(L.mn_latent_attn(ptr(qd), ptr(kd), ptr(seq), ptr(ln), ptr(blk), 3, 3, H, r, t_max, n + 1, ks, ptr(lat), ptr(ws), ws.numel(), current_stream()), "latent")
+        ref = want(r)
+        assert bool((lat[3] == 7.0).all()) and float((lat[:3].double().cpu() - ref).abs().max() / ref.abs().max()) < 1e-5
+    if not e:
+        return
+    for window, cap, ns in ((0, 0.0, 1), (20, 5.0, 1), (0, 5.0, 3), (40, 0.0, 2)):
+        ws = torch.empty(max(16, L.mn_window_attn_workspace_bytes(3, H, 1, e, 1, ns)), dtype=torch.uint8, device="cuda")
+        out = torch.full((4, H * e), 7.0, device="cuda")
+        check(L.mn_window_pool_attn_blocks_gate(ptr(qd), H * r, ptr(kd), r, ptr(kd), r, None, None, None, cap, 0, None, 0, ptr(seq), ptr(slot), None, 3, 1, H, 1, r, e,
+                                                t_max, 1, window, 0, 1.0, ptr(out), H * e, None, 0, ns, ptr(ws), ws.numel(), -1, current_stream()), "attn")
+        ref = want(e, window, cap).reshape(3, -1)
+        assert bool((out[3] == 7.0).all()) and float((out[:3].double().cpu() - ref).abs().max() / ref.abs().max()) < 1e-5

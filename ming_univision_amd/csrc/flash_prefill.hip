@@ -1,13 +1,13 @@
 // flash_prefill.hip — flash attention of the batch / prefill passes (bf16 MFMA, fp32 online softmax), 64-key tiles.
 //
 //   SRC 0  flash_attn_func on packed qkv, head dim 64 (mingtok/vision_tower/layers/attention.py:78-108 full, :177-239 causal):
-//          q / k / v bf16 inside qkv [B, T, 3, nh, 64]; a workgroup = 128 queries of one (image, head), 32 per wave.
+//          q / k / v bf16 inside qkv [B, T, 3, nh, 64]; a workgroup = 64 QG queries of one (image, head), 16 QG per wave.
 //   SRC 1  BailingMoeFlashAttention2 on a long prompt (modeling_bailing_moe.py:848-1045; bottom-right causal, :844-846), head
 //          dim 128, GQA 4:1: q bf16 [rows, n_q, 128] (RoPE'd, pre-scaled), K / V read from the fp32 KV arena the decode
-//          kernels use; a workgroup = 32 queries x the 4 query heads of one KV head (one head per wave), so a staged K / V
-//          tile serves 128 query rows in both forms; several prompts per launch through a (sequence, first row, length) table.
+//          kernels use; a workgroup = 16 QG queries x the 4 query heads of one KV head (one head per wave), so a staged K / V
+//          tile serves 64 QG query rows in both forms; several prompts per launch through a (sequence, first row, length) table.
 //
-// Per 64-key tile, with q = lane & 15 (a query COLUMN), g = lane >> 4, two 16-query groups per wave:
+// Per 64-key tile, with q = lane & 15 (a query COLUMN), g = lane >> 4, QG 16-query groups per wave:
 //   S^T[key, q] = sum_d K[key, d] Q[q, d]      A = K fragment (ds_read_b128 from the row-major tile, rows padded by 16 B),
 //                                              B = Q fragment (registers, loaded once)
 //     -> accumulator reg r of key fragment f holds key 16 f + 4 g + r for query q
@@ -20,13 +20,15 @@
 //     i/4, i/4 + 4, i/4 + 8, i/4 + 12 — measured, tools/exp/tr_probe.hip) from the ROW-major V tile, so V is staged like K with
 //     16-byte writes and never transposed by stores.  V rows are padded by 32 B: a 16-lane group reads 4 keys x 32 B and the
 //     eight groups of two waves tile the 64 banks.
+// KS 2: two groups of four waves walk the tiles 0, 2, .. and 1, 3, .. of the same queries; maxima, sums and accumulators meet in LDS at the end.
+// QG: 16-query groups per wave (the hi/lo form at head dim 128 has one: q, o, s, p hi + lo would not fit 256 registers).
 // The staging of tile t+1 is issued to registers before tile t is computed and written to LDS after it (one tile in flight).
 //
 // HILO (round 4; SRC 0 only): the fp32-class regime's attention — q / k / v are FP32 inside qkv, every operand is carried as a bf16
 // hi + lo pair (x = hi + lo to 2^-17) and every product as three MFMAs (hi hi + hi lo + lo hi; the lo lo term is 2^-16 of the
 // product), scores / softmax / accumulators fp32, output fp32 and / or the next GEMM's hi / lo operand.  It replaces the per-row
 // decode kernels the regime borrowed before (every query row re-reading all of K and V through L2: 8.5 ms of the 14.8 ms a
-// 1024^2 image spends in MingTok) with the tiled form: a staged 64-key tile serves 128 query rows.
+// 1024^2 image spends in MingTok) with the tiled form: a staged 64-key tile serves 64 or 128 query rows.
 #include "common.h"
 
 typedef short bf16x8 __attribute__((ext_vector_type(8)));
@@ -54,28 +56,32 @@ struct FlashP {
   int mask_per_row;                                // (unused with key_mask == NULL)
 };
 
-template <int HD, int SRC, bool HILO = false>
-__global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const FlashP p) {
-  // query groups (16 queries each) per wave: the hi/lo form at head dim 128 keeps one (q, o, s, p hi + lo would not fit 256 registers)
-  constexpr int QG = (HILO && HD == 128) ? 1 : 2, QW = 16 * QG;
+template <int HD, int SRC, bool HILO, int QG, int KS>
+__global__ __launch_bounds__(256 * KS, QG == 1 && KS == 2 && HD == 64 ? 4 : 2) void flash_prefill_kernel(const FlashP p) {
+  constexpr int QW = 16 * QG;
   constexpr int KROW = HD + 8, VROW = HD + 16, NKK = HD / 32, NDT = HD / 16;
   constexpr int ESZ = (SRC == 0 && !HILO) ? 2 : 4, PPR = HD * ESZ / 16, KPP = 256 / PPR, NP = FKT / KPP;
-  __shared__ __attribute__((aligned(16))) bf16_t ks[FKT * KROW * (HILO ? 2 : 1)];     // HILO: the hi tile, then the lo tile
-  __shared__ __attribute__((aligned(16))) bf16_t vs[FKT * VROW * (HILO ? 2 : 1)];
-  constexpr int KLO = FKT * KROW, VLO = FKT * VROW;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int KLO = FKT * KROW, VLO = FKT * VROW, TILE = (KLO + VLO) * (HILO ? 2 : 1);
+  constexpr int PART = QG * (NDT * 4 + 2) * 256;                                        // floats a key group hands over
+  constexpr int SMEM = KS > 1 && (KS - 1) * PART * 2 > KS * TILE ? (KS - 1) * PART * 2 : KS * TILE;
+  __shared__ __attribute__((aligned(16))) bf16_t smem[SMEM];
+  const int kg = KS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;    // key group: the tiles kg, kg + KS, ..
+  bf16_t* ks = smem + kg * TILE;                                                        // HILO: the hi tile, then the lo tile
+  bf16_t* vs = ks + KLO * (HILO ? 2 : 1);
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int i16 = lane & 15, g = lane >> 4;
   int T = p.T, q0, q_hi_wg;
   int past = p.past;
+  const int qblk = p.causal ? (int)(gridDim.y - 1 - blockIdx.y) : (int)blockIdx.y;      // causal: the long walks first
   int64_t o_off;                                    // element offset of the (image | span, head)'s first output
   const bf16_t* qb;
   bf16_t* ob;
   const char *kb, *vb;
   const uint8_t* km = p.key_mask;
   if (SRC == 0) {
-    const int head = blockIdx.y, b = blockIdx.z;
-    q0 = blockIdx.x * 128 + wave * 32;
-    q_hi_wg = blockIdx.x * 128 + 127;
+    const int head = blockIdx.x, b = blockIdx.z;
+    q0 = qblk * 4 * QW + wave * QW;
+    q_hi_wg = qblk * 4 * QW + 4 * QW - 1;
     qb = p.q + (b * p.q_bs + head * p.q_hs) * (HILO ? 2 : 1);          // HILO: q is fp32 (pointer arithmetic in bf16 units)
     o_off = b * p.o_bs + head * HD;
     ob = p.out + o_off;
@@ -89,8 +95,8 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const FlashP p) {
       seq = te[0]; r0 = te[1]; T = te[2];
       if (p.tab_w > 3) past = te[3];
     }
-    const int kvh = blockIdx.y, head = kvh * 4 + wave;
-    q0 = blockIdx.x * QW;
+    const int kvh = blockIdx.x, head = kvh * 4 + wave;
+    q0 = qblk * QW;
     q_hi_wg = q0 + QW - 1;
     if (q0 >= T) return;                                   // uniform per workgroup
     qb = p.q + ((int64_t)r0 * p.q_rs + head * p.q_hs) * (HILO ? 2 : 1);
@@ -186,13 +192,13 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const FlashP p) {
   const bf16_t* kfr = &ks[i16 * KROW + g * 8];
   const bf16_t* vfr = &vs[(g * 4 + (i16 >> 2)) * VROW + 4 * (i16 & 3)];
 
-  fetch(0);
-  for (int kt = 0; kt < ntile; ++kt) {
-    const int k0 = kt * FKT;
+  fetch(kg * FKT);                         // (clamped to the last key)
+  for (int kt0 = 0; kt0 < ntile; kt0 += KS) {
+    const int k0 = (kt0 + kg) * FKT;
     __syncthreads();                       // the previous tile's fragments are read
     park();
     __syncthreads();                       // tile kt visible
-    if (kt + 1 < ntile) fetch(k0 + FKT);   // in flight under this tile's MFMAs
+    if (kt0 + kg + KS < ntile) fetch(k0 + KS * FKT);   // in flight under this tile's MFMAs
     if (!wave_on || k0 >= wave_kmax) continue;
 
     f32x4 s[QG][4];
@@ -305,12 +311,45 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const FlashP p) {
         }
       }
   }
+#pragma unroll
+  for (int qg = 0; qg < QG; ++qg) {
+    l_run[qg] += __shfl_xor(l_run[qg], 16, 64);
+    l_run[qg] += __shfl_xor(l_run[qg], 32, 64);
+  }
+  if constexpr (KS > 1) {                  // the key groups' maxima, sums and accumulators meet in LDS
+    float* mine = reinterpret_cast<float*>(smem) + (kg - 1) * PART + tid;
+    __syncthreads();                       // every tile is read
+    if (kg > 0) {
+#pragma unroll
+      for (int qg = 0; qg < QG; ++qg) {
+        mine[(qg * (NDT * 4 + 2)) * 256] = m_run[qg];
+        mine[(qg * (NDT * 4 + 2) + 1) * 256] = l_run[qg];
+#pragma unroll
+        for (int x = 0; x < NDT * 4; ++x) mine[(qg * (NDT * 4 + 2) + 2 + x) * 256] = o[qg][x >> 2][x & 3];
+      }
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int w = 1; w < KS; ++w) {
+      const float* other = reinterpret_cast<const float*>(smem) + (w - 1) * PART + tid;
+#pragma unroll
+      for (int qg = 0; qg < QG; ++qg) {
+        constexpr float LOG2E = 1.4426950408889634f;
+        const float m2 = other[(qg * (NDT * 4 + 2)) * 256], l2 = other[(qg * (NDT * 4 + 2) + 1) * 256], m = fmaxf(m_run[qg], m2);
+        const float a1 = m_run[qg] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_run[qg] - m) * LOG2E);
+        const float a2 = m2 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m2 - m) * LOG2E);
+        m_run[qg] = m;
+        l_run[qg] = l_run[qg] * a1 + l2 * a2;
+#pragma unroll
+        for (int x = 0; x < NDT * 4; ++x) o[qg][x >> 2][x & 3] = o[qg][x >> 2][x & 3] * a1 + other[(qg * (NDT * 4 + 2) + 2 + x) * 256] * a2;
+      }
+    }
+  }
   if (!wave_on) return;
 #pragma unroll
   for (int qg = 0; qg < QG; ++qg) {
-    float l = l_run[qg];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    const float l = l_run[qg];
     if (q_idx[qg] >= T) continue;
     const float inv = l > 0.f ? 1.0f / l : 0.f;   // no attended key: 0, not NaN
     if constexpr (HILO) {
@@ -336,6 +375,38 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_kernel(const FlashP p) {
     }
   }
 }
+// Which form (measured on MI355X, us; T tokens x heads x images, "hi/lo" the fp32-class operands).  A workgroup walks its key tiles one after the
+// other at 2 .. 3 us a tile, most of it latency, so a launch that does not fill the chip takes 64 instead of 128 queries a workgroup and two key
+// groups (KS 2: 8 waves, each group every other tile):
+//   1024 x 16 x 1 bf16 25.0 -> 13.8; 1025 x 16 x 1 hi/lo causal 41.3 -> 24, 1025 x 12 hi/lo 41 -> 24; 257 x 16 10.6 -> 7.1; 2500 x 16 hi/lo causal 99.6 -> 68
+// A causal launch has half the work and goes longest walk first, so it takes them up to 2.5 workgroups a CU (1088 of 64 queries: no form
+// is better).  A full launch of more than one a CU has a second round; 128 queries in two key groups avoid it (1025 x 16 hi/lo: 34 against 38 and 46 us).
+// Launches that fill the chip walk alone (64 x 256 x 16 bf16: 38 us, in key groups 55), 64 queries a workgroup where 128 would leave much
+// of the last one empty (64 x 65 x 16: 14.1 -> 11.0, 64 x 257 x 12: 46 -> 43).  Heads are the fastest grid dimension: an XCD then sees few heads' keys
+// (2500 x 16 hi/lo, 128 queries: 126 -> 100 us).
+template <bool HILO>
+void flash_hd64(const FlashP& p, int T, int n_heads, int B, hipStream_t st) {
+  const int64_t cu = mn_num_cus(), hb = (int64_t)n_heads * B, w64 = mn_cdiv(T, 64) * hb, w128 = mn_cdiv(T, 128) * hb;
+#define MN_FL(QG_, KS_) hipLaunchKernelGGL((flash_prefill_kernel<64, 0, HILO, QG_, KS_>), dim3(n_heads, mn_cdiv(T, 64 * (QG_)), B), dim3(256 * (KS_)), 0, st, p)
+  if (T > 64 && w64 <= (p.causal ? 5 * cu / 2 : cu)) MN_FL(1, 2);
+  else if (T > 64 && w128 <= cu) MN_FL(2, 2);
+  else if (((T - 1) & 127) < 80) MN_FL(1, 1);
+  else MN_FL(2, 1);
+#undef MN_FL
+}
+
+// Head dim 128, causal: 16 queries x 4 heads in two key groups up to two workgroups a CU (1062 tokens x 4 key heads hi/lo 55 -> 42 us, bf16 45 -> 26; 64 tokens
+// behind 2000: 94 -> 68, 82 -> 42; 608 workgroups of 8 spans of 300: 31 -> 36, so not there); bf16 rows beyond that take 32 queries, in key groups
+// where the walks are long (4000 tokens: 156 -> 125 us; 8 spans of 300: 23 -> 27).
+template <bool HILO, int QG>
+void flash_hd128(const FlashP& p, int T, int past, int n_kv, int n, hipStream_t st) {
+  const int64_t cu = mn_num_cus(), w16 = mn_cdiv(T, 16) * (int64_t)n_kv * n, w32 = mn_cdiv(T, 32) * (int64_t)n_kv * n;
+#define MN_FL(QG_, KS_) hipLaunchKernelGGL((flash_prefill_kernel<128, 1, HILO, QG_, KS_>), dim3(n_kv, mn_cdiv(T, 16 * (QG_)), n), dim3(256 * (KS_)), 0, st, p)
+  if (w16 <= 2 * cu) MN_FL(1, 2);
+  else if (QG == 2 && w32 <= 2 * cu && past + T >= 1024) MN_FL(QG, 2);
+  else MN_FL(QG, 1);
+#undef MN_FL
+}
 }  // namespace
 
 // flash_attn_func on packed qkv bf16 [B, T, 3, nh, 64] -> out bf16 [B, T, nh * 64]  (mingtok attention.py:78-108, 177-239)
@@ -347,7 +418,7 @@ extern "C" int mn_attn_prefill_hd64(const uint16_t* qkv, uint16_t* out, int B, i
   p.q_rs = rs; p.q_hs = 64; p.kv_rs = rs; p.kv_hs = 64; p.o_rs = (int64_t)n_heads * 64;
   p.q_bs = (int64_t)T * rs; p.kv_bs = (int64_t)T * rs; p.o_bs = (int64_t)T * n_heads * 64;
   p.T = T; p.past = 0; p.causal = causal;
-  hipLaunchKernelGGL((flash_prefill_kernel<64, 0>), dim3(mn_cdiv(T, 128), n_heads, B), dim3(256), 0, mn_stream(stream), p);
+  flash_hd64<false>(p, T, n_heads, B, mn_stream(stream));
   MN_CHECK_LAUNCH("mn_attn_prefill_hd64");
   return MN_OK;
 }
@@ -363,7 +434,7 @@ extern "C" int mn_attn_prefill_hd64_f32(const float* qkv, float* out, uint16_t* 
   p.q_rs = rs; p.q_hs = 64; p.kv_rs = rs; p.kv_hs = 64; p.o_rs = (int64_t)n_heads * 64;
   p.q_bs = (int64_t)T * rs; p.kv_bs = (int64_t)T * rs; p.o_bs = (int64_t)T * n_heads * 64;
   p.T = T; p.past = 0; p.causal = causal;
-  hipLaunchKernelGGL((flash_prefill_kernel<64, 0, true>), dim3(mn_cdiv(T, 128), n_heads, B), dim3(256), 0, mn_stream(stream), p);
+  flash_hd64<true>(p, T, n_heads, B, mn_stream(stream));
   MN_CHECK_LAUNCH("mn_attn_prefill_hd64_f32");
   return MN_OK;
 }
@@ -375,7 +446,7 @@ extern "C" int mn_flash_prefill_gqa_hd128_one(const uint16_t* q, const float* kv
   p.q = q; p.k = kv_seq; p.v = kv_seq + (int64_t)n_kv * t_max * 128; p.out = out;
   p.q_rs = (int64_t)n_q * 128; p.q_hs = 128; p.kv_rs = 128; p.kv_hs = t_max * 128; p.o_rs = (int64_t)n_q * 128;
   p.T = T; p.past = past; p.causal = 1; p.key_mask = key_mask;
-  hipLaunchKernelGGL((flash_prefill_kernel<128, 1>), dim3(mn_cdiv(T, 32), n_kv, 1), dim3(256), 0, mn_stream(stream), p);
+  flash_hd128<false, 2>(p, T, past, n_kv, 1, mn_stream(stream));
   MN_CHECK_LAUNCH("mn_attn_prefill_gqa_hd128");
   return MN_OK;
 }
@@ -394,7 +465,7 @@ extern "C" int mn_flash_prefill_gqa_hd128_f32(const float* q, const float* kv_la
   p.q_rs = (int64_t)n_q * 128; p.q_hs = 128; p.kv_rs = 128; p.kv_hs = t_max * 128; p.o_rs = (int64_t)n_q * 128;
   p.T = max_len; p.past = 0; p.causal = 1;
   p.seq_tab = span_tab; p.tab_w = 4; p.kv_seq_stride = (int64_t)2 * n_kv * t_max * 128;
-  hipLaunchKernelGGL((flash_prefill_kernel<128, 1, true>), dim3(mn_cdiv(max_len, 16), n_kv, n_spans), dim3(256), 0, mn_stream(stream), p);
+  flash_hd128<true, 1>(p, max_len, 0, n_kv, n_spans, mn_stream(stream));
   MN_CHECK_LAUNCH("mn_flash_prefill_gqa_hd128_f32");
   return MN_OK;
 }
@@ -413,7 +484,7 @@ extern "C" int mn_flash_prefill_gqa_hd128(const uint16_t* q, const float* kv_lay
   p.q_rs = (int64_t)n_q * 128; p.q_hs = 128; p.kv_rs = 128; p.kv_hs = t_max * 128; p.o_rs = (int64_t)n_q * 128;
   p.T = max_len; p.past = past; p.causal = 1; p.key_mask = key_mask; p.mask_bs = mask_stride;
   p.seq_tab = seq_tab; p.tab_w = 3; p.kv_seq_stride = (int64_t)2 * n_kv * t_max * 128;
-  hipLaunchKernelGGL((flash_prefill_kernel<128, 1>), dim3(mn_cdiv(max_len, 32), n_kv, n_spans), dim3(256), 0, mn_stream(stream), p);
+  flash_hd128<false, 2>(p, max_len, past, n_kv, n_spans, mn_stream(stream));
   MN_CHECK_LAUNCH("mn_flash_prefill_gqa_hd128");
   return MN_OK;
 }

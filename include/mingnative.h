@@ -533,6 +533,16 @@ MN_API int mn_llm_step_spans(const mn_llm* m, const float* x, int64_t ldx, int M
  * device-resident row_slot / row_pos / row_len arrays between autoregressive steps without a host round trip. */
 MN_API int mn_rows_advance(int32_t* a, int32_t* b, int32_t* c, int M, int delta, void* stream);
 
+/* The blocks of a vision transformer (mingtok/vision_tower/layers/block.py:80-105, 301-327) on the fp32 residual stream x [B * T, dim], heads of 64, one call
+ * for the stack's launches.  w: HOST array of 12 device pointers a block: norm1 g, b; qkv w [3 dim, dim], b; proj w, b; norm2 g, b; up w, b; down w
+ * [dim, hidden], b.  gelu 0: up = [2 hidden, dim] gate rows then up rows (SwiGLU); 1: up [hidden, dim] (exact-erf GELU).
+ * precise 0: bf16 operands; out bf16 [B * T, dim] = LayerNorm(x; fin_g, fin_b), then GELU if fin_gelu.  precise 1: hi / lo operands (fp32-class), hidden a
+ * multiple of 64, out NULL (the caller norms x).  workspace: mn_vit_blocks_workspace_bytes, 256-byte aligned. */
+MN_API size_t mn_vit_blocks_workspace_bytes(int B, int T, int dim, int hidden, int gelu, int precise);
+MN_API int mn_vit_blocks(float* x, int B, int T, int dim, int depth, const uint16_t* const* w, int hidden, int gelu, int causal, int precise, float eps,
+                         const uint16_t* fin_g, const uint16_t* fin_b, int fin_gelu, uint16_t* out, void* workspace, size_t workspace_bytes,
+                         void* stream);
+
 /* MingTok semantic decoder, cached causal decode step for M <= 64 rows of ONE sequence each
  * (MingTok.forward_feature_decoder, modeling_mingtok.py:165-174 -> TransformerDecoder.forward_features,
  * vision_transformer.py:382-451) followed by linear_proj (modeling_bailingmm.py:111-115). */

@@ -84,59 +84,40 @@ class MingTok:
     def _w(self, k):
         return self.sd[k]
 
-    def _resid_linear(self, a, w, bias, x, next_norm):
-        """x (fp32 residual stream) += a @ w^T + bias; returns bf16 next_norm(x) when it was fused into the tail, else None.
-        next_norm: None or (weight, bias, gelu).  With few rows (a 256 x 256-tile GEMM would fill under half the chip) the
-        product runs split-K and ONE launch reduces the slabs, updates the stream and applies the consumer's LayerNorm."""
-        ks = ops.splitk_plan(a.shape[0], w.shape[0], a.shape[1])
-        if ks and lib().mn_gemm256_supported(a.shape[1], 0, w.stride(0), w.shape[0], a.shape[0], w.shape[0], a.shape[1]):
-            P = ops.gemm256_splitk_bf16(a, w, bias, ks)
-            if next_norm is None:
-                return ops.slab_resid_norm(P, x, norm=False)
-            return ops.slab_resid_norm(P, x, next_norm[0], next_norm[1], gelu=next_norm[2])
-        ops.gemm_bf16(a, w, bias, "f32_resid", out=x)
-        return None
-
-    def _block(self, x, prefix, D, B, T, causal, xn=None, next_norm=None):
-        """Block.forward / CausalBlock.forward (layers/block.py:80-105, 301-327) on the fp32 residual x [B*T, D].
-        xn: bf16 norm1(x) when the previous block's tail already produced it; next_norm = (weight, bias, gelu) of the LayerNorm
-        that consumes this block's output.  Returns that LayerNorm's bf16 output when it was fused into the tail, else None."""
-        nh = D // 64
-        if xn is None:
-            xn = ops.layernorm_bf16(x, self._w(prefix + ".norm1.weight"), self._w(prefix + ".norm1.bias"))
-        qkv = ops.gemm_bf16(xn, self._w(prefix + ".attn.qkv.weight"), self._w(prefix + ".attn.qkv.bias"))
-        att = ops.attn_prefill_hd64(qkv, B, T, nh, causal)
-        xn = self._resid_linear(att, self._w(prefix + ".attn.proj.weight"), self._w(prefix + ".attn.proj.bias"), x,
-                                (self._w(prefix + ".norm2.weight"), self._w(prefix + ".norm2.bias"), False))
-        if xn is None:
-            xn = ops.layernorm_bf16(x, self._w(prefix + ".norm2.weight"), self._w(prefix + ".norm2.bias"))
-        if (prefix + ".mlp.w12.weight") in self.sd:
-            w12, b12, w3 = self._w(prefix + ".mlp.w12.weight"), self._w(prefix + ".mlp.w12.bias"), self._w(prefix + ".mlp.w3.weight")
-            if prefix.startswith("semantic_decoder.blocks.0."):
-                # the zero-padded copies (hidden 2736 -> 2752): whole 64-k tiles for w3, results unchanged
-                self._semdec()
-                li = int(prefix.rsplit(".", 1)[1])
-                w12, b12, w3 = self._sem_pad[0][li], self._sem_pad[1][li], self._sem_pad[2][li]
-            hid = w12.shape[0] // 2
-            if hid % 4 == 0 and D % 64 == 0:
-                h = ops.gemm256_swiglu(xn, w12, b12)                 # SwiGLU in the GEMM epilogue: no [M, 2*hidden] round trip
-            else:
-                h = ops.swiglu_bf16(ops.gemm_bf16(xn, w12, b12))
-            return self._resid_linear(h, w3, self._w(prefix + ".mlp.w3.bias"), x, next_norm)
-        h = ops.gemm_bf16(xn, self._w(prefix + ".mlp.fc1.weight"), self._w(prefix + ".mlp.fc1.bias"), "bf16_gelu")
-        return self._resid_linear(h, self._w(prefix + ".mlp.fc2.weight"), self._w(prefix + ".mlp.fc2.bias"), x, next_norm)
-
-    def _blocks(self, x, stem, depth, D, B, T, causal, final_norm):
-        """`depth` blocks `stem`.i in sequence; final_norm = (weight, bias, gelu) of the LayerNorm after the last one.
-        Returns its bf16 output.  Each block's tail is asked for the next LayerNorm (fused when the tail runs split-K)."""
-        xn = None
+    def _blocks(self, x, stem, depth, D, B, T, causal, final_norm=None, fp32=False):
+        """`depth` blocks `stem`.i (Block.forward / CausalBlock.forward, layers/block.py:80-105, 301-327) on the fp32 residual x [B*T, D], in place, one
+        native call (mn_vit_blocks).  bf16 regime: final_norm = (weight, bias, gelu) of the LayerNorm after the last block, whose bf16 output is
+        returned; fp32: hi / lo operands, nothing returned.  The weights are looked up and checked on every call."""
+        sd, M = self.sd, B * T
+        if depth == 0:
+            return None if fp32 else ops.layernorm_bf16(x, final_norm[0], final_norm[1], gelu=final_norm[2])
+        swiglu = f"{stem}.0.mlp.w12.weight" in sd
+        up, down = (".mlp.w12", ".mlp.w3") if swiglu else (".mlp.fc1", ".mlp.fc2")
+        table, hidden = (C.c_void_p * (12 * depth))(), None
+        n = 0
         for i in range(depth):
-            nxt = (final_norm if i + 1 == depth else
-                   (self._w(f"{stem}.{i + 1}.norm1.weight"), self._w(f"{stem}.{i + 1}.norm1.bias"), False))
-            xn = self._block(x, f"{stem}.{i}", D, B, T, causal, xn=xn, next_norm=nxt)
-        if xn is None:
-            xn = ops.layernorm_bf16(x, final_norm[0], final_norm[1], gelu=final_norm[2])
-        return xn
+            p = f"{stem}.{i}"
+            # SwiGLU widths zero-padded to whole 64-k tiles of w3 (results unchanged): every stack of the fp32 regime, and the semantic decoder's
+            if swiglu and (fp32 or stem.startswith("semantic_decoder.blocks.0")):
+                wu, bu, wd = self._swiglu_padded(p)
+            else:
+                wu, bu, wd = sd[p + up + ".weight"], sd[p + up + ".bias"], sd[p + down + ".weight"]
+            hidden = hidden or wd.shape[1]
+            rows = 2 * hidden if swiglu else hidden
+            for t, shape in ((sd[p + ".norm1.weight"], (D,)), (sd[p + ".norm1.bias"], (D,)), (sd[p + ".attn.qkv.weight"], (3 * D, D)), (sd[p + ".attn.qkv.bias"], (3 * D,)),
+                             (sd[p + ".attn.proj.weight"], (D, D)), (sd[p + ".attn.proj.bias"], (D,)), (sd[p + ".norm2.weight"], (D,)), (sd[p + ".norm2.bias"], (D,)),
+                             (wu, (rows, D)), (bu, (rows,)), (wd, (D, hidden)), (sd[p + down + ".bias"], (D,))):
+                if t.dtype != torch.bfloat16 or t.shape != shape or not t.is_cuda or not t.is_contiguous():
+                    raise TypeError(f"{p}: expected a contiguous bf16 tensor {shape} on the GPU, got {t.dtype} {tuple(t.shape)} on {t.device}")
+                table[n] = t.data_ptr()
+                n += 1
+        assert x.is_contiguous() and x.shape == (M, D) and x.dtype == torch.float32 and x.is_cuda
+        ws = torch.empty(lib().mn_vit_blocks_workspace_bytes(B, T, D, hidden, int(not swiglu), int(fp32)), dtype=torch.uint8, device=x.device)
+        out = None if fp32 else torch.empty(M, D, dtype=torch.bfloat16, device=x.device)
+        g, b, act = final_norm or (None, None, False)
+        check(lib().mn_vit_blocks(ptr(x), B, T, D, depth, C.cast(table, _lib.PP), hidden, int(not swiglu), int(causal), int(fp32), 1e-6, ptr(g), ptr(b), int(act),
+                                  ptr(out), ptr(ws), ws.numel(), current_stream()), "mn_vit_blocks")
+        return out
 
     def _pos_embed(self, npatch, w, h):
         """interpolate_pos_encoding (vision_transformer.py:183-215) — cached per resolution (load-time table)."""
@@ -183,34 +164,6 @@ class MingTok:
                 self._pos_cache[key] = (a, bb, c)
         return self._pos_cache[key]
 
-    def _attention_fp32(self, qkv, B, T, nh, causal):
-        """softmax(q k^T / 8) v per (image, head), fp32-class: the hi/lo flash kernel (mn_attn_prefill_hd64_f32: operands as bf16
-        hi + lo pairs, three MFMAs per product, fp32 softmax).  qkv fp32 [B*T, 3*nh*64] in the reshape of attention.py:83 -> the
-        hi/lo pair bf16 [2, B*T, nh*64] of the result (the projection's operand).  (Round 3 borrowed the per-row decode kernels
-        over a scratch arena: every query row re-read all keys — 8.5 of the 14.8 ms a 1024^2 image spent in MingTok.)"""
-        return ops.attn_prefill_hd64_f32(qkv, B, T, nh, causal)
-
-    def _block_fp32(self, x, prefix, D, B, T, causal):
-        """Block.forward / CausalBlock.forward (layers/block.py:80-105, 301-327) on the fp32 residual x [B*T, D], fp32-class."""
-        nh = D // 64
-        xn, _ = ops.norm_act_split(x, "ln", self._w(prefix + ".norm1.weight"), self._w(prefix + ".norm1.bias"))
-        qkv = ops.linear_hilo(xn, self._w(prefix + ".attn.qkv.weight"), self._w(prefix + ".attn.qkv.bias"))
-        att = self._attention_fp32(qkv, B, T, nh, causal)
-        ops.linear_hilo(att, self._w(prefix + ".attn.proj.weight"), self._w(prefix + ".attn.proj.bias"), out=x, resid=True)
-        xn, _ = ops.norm_act_split(x, "ln", self._w(prefix + ".norm2.weight"), self._w(prefix + ".norm2.bias"))
-        if (prefix + ".mlp.w12.weight") in self.sd:
-            w12, b12, w3 = self._swiglu_padded(prefix)
-            h = ops.gemm256_swiglu_split(xn, w12, b12)
-            ops.linear_hilo(h, w3, self._w(prefix + ".mlp.w3.bias"), out=x, resid=True)
-        else:
-            h = ops.linear_hilo(xn, self._w(prefix + ".mlp.fc1.weight"), self._w(prefix + ".mlp.fc1.bias"))
-            hs, _ = ops.norm_act_split(h, "none", gelu=True)
-            ops.linear_hilo(hs, self._w(prefix + ".mlp.fc2.weight"), self._w(prefix + ".mlp.fc2.bias"), out=x, resid=True)
-
-    def _blocks_fp32(self, x, stem, depth, D, B, T, causal):
-        for i in range(depth):
-            self._block_fp32(x, f"{stem}.{i}", D, B, T, causal)
-
     # ---- encoder ---------------------------------------------------------------------------
     def encode(self, x, precision=None):
         """low_level_encoder(x) -> RAW latent fp32 [B, N+1, latent_dim] (vision_transformer.py:225-233)."""
@@ -232,7 +185,7 @@ class MingTok:
         xf = ops.tokens_assemble(tok, self._w("low_level_encoder.cls_token").reshape(D), pe, B, N).reshape(B * T, D)
         # blocks, then forward_out_layer (:173-178) whose LayerNorm + GELU rides the last block's tail
         if fp32:
-            self._blocks_fp32(xf, "low_level_encoder.blocks.0", self.enc_depth, D, B, T, False)
+            self._blocks(xf, "low_level_encoder.blocks.0", self.enc_depth, D, B, T, False, fp32=True)
             xn, _ = ops.norm_act_split(xf, "ln", self._w("low_level_encoder.out_norm.weight"), self._w("low_level_encoder.out_norm.bias"), gelu=True)
             y = ops.linear_hilo(xn, self._w("low_level_encoder.out_proj.weight"), self._w("low_level_encoder.out_proj.bias"))
         else:
@@ -259,7 +212,7 @@ class MingTok:
         x = torch.empty_like(y)
         check(lib().mn_repeat_add(ptr(y), ptr(lat), ptr(x), B * T, D, Cin, 1.0, 0.0, current_stream()), "mn_repeat_add")
         if fp32:
-            self._blocks_fp32(x, "semantic_decoder.blocks.0", self.sem_depth, D, B, T, True)
+            self._blocks(x, "semantic_decoder.blocks.0", self.sem_depth, D, B, T, True, fp32=True)
             _, out = ops.norm_act_split(x, "ln", self._w("semantic_decoder.norm.weight"), self._w("semantic_decoder.norm.bias"),
                                         want_split=False, want_f32=True)
             return out.reshape(B, T, D)
@@ -296,7 +249,7 @@ class MingTok:
         x = ops.subtoken_rearrange(y, B, h, w, r, Dp)           # "b (h w) (x y c) -> b (h x w y) c" in one pass
         T = N * r * r
         if fp32:
-            self._blocks_fp32(x, "pixel_decoder.blocks.0", self.pix_depth, Dp, B, T, False)
+            self._blocks(x, "pixel_decoder.blocks.0", self.pix_depth, Dp, B, T, False, fp32=True)
             xn, _ = ops.norm_act_split(x, "ln", self._w("pixel_decoder.norm.weight"), self._w("pixel_decoder.norm.bias"))
             o = ops.linear_hilo(xn, self._w("pixel_decoder.head.weight"), self._w("pixel_decoder.head.bias"))
         else:

@@ -110,13 +110,13 @@ __device__ __forceinline__ float dpp_f(float v) {
 __device__ __forceinline__ float lane_f(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
-__device__ __forceinline__ float row16_sum(float v) {
-  v += dpp_f<0x140>(v);
-  v += dpp_f<0x141>(v);
-  v += dpp_f<0x4E>(v);
-  v += dpp_f<0xB1>(v);
-  return v;
+// v + its partner's v: zero as the value of a partner that does not run lets the compiler fold the move into v_add_f32_dpp (one instruction of
+// three; a chain of sums is all there is in a one-row kernel's tail)
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
+__device__ __forceinline__ float row16_sum(float v) { return dpp_add<0xB1>(dpp_add<0x4E>(dpp_add<0x141>(dpp_add<0x140>(v)))); }
 __device__ __forceinline__ float row16_max(float v) {
   v = fmaxf(v, dpp_f<0x140>(v));
   v = fmaxf(v, dpp_f<0x141>(v));

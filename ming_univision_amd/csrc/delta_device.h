@@ -10,10 +10,34 @@ __device__ __forceinline__ float silu_x(float z) { return z / (1.0f + expf(-z));
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.0f ? z : log1pf(expf(z)); }
 
 __device__ __forceinline__ float sum8(float v) {                    // over the 8 lanes of an aligned group; every lane gets the sum
-  v += dpp_f<0xB1>(v);
-  v += dpp_f<0x4E>(v);
-  v += dpp_f<0x141>(v);
-  return v;
+  return dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(v)));
+}
+
+// First row of the step's sequence j (its rows' row_back counts 0, 1, ..), -1 if the step has fewer: 256 threads, the same result in all of them.
+// A launch of sequences x channels whose workgroups look theirs up beats one workgroup a row of which most find nothing to do: 1409 rows x 64
+// workgroups with 35 KB of LDS each took 33 us to come and go.
+__device__ __forceinline__ int sequence_start(const int32_t* __restrict__ row_back, int M, int j, uint64_t (&mask)[32]) {
+  const int tid = threadIdx.x;
+  for (int base = 0; base < M; base += 2048) {
+    __syncthreads();                            // the masks of the rows (or the call) before are read
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int m = base + 256 * k + tid;
+      const uint64_t b = __ballot(m < M && row_back[m < M ? m : 0] == 0);
+      if ((tid & 63) == 0) mask[4 * k + (tid >> 6)] = b;
+    }
+    __syncthreads();
+    for (int i = 0; i < 32; ++i) {
+      uint64_t b = mask[i];
+      const int c = __popcll(b);
+      if (j < c) {
+        for (; j > 0; --j) b &= b - 1;
+        return base + 64 * i + __ffsll((unsigned long long)b) - 1;
+      }
+      j -= c;
+    }
+  }
+  return -1;
 }
 
 // Gated delta rule, preparation of a row: channels [q: G dim ; k: G dim ; v: H vdim] of the raw projections go through their causal

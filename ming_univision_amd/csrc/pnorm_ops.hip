@@ -393,122 +393,133 @@ __global__ __launch_bounds__(256) void delta_rows_kernel(DeltaArgs a) {
   }
 }
 
-// The same walk for heads of at most 256 state rows, without a branch in the step: grid (H * ceil(vdim / CPB), M) — the workgroups that
-// work (those of a sequence's first row) are neighbours in the launch order and land on different CUs.  LPC lanes share a value column
+// The same walk for heads of at most 256 state rows, without a branch in the step: grid (H * ceil(vdim / CPB), S):
+// workgroup y takes the step's sequences y, y + S, ..  LPC lanes share a value column
 // (CPB = 256 / LPC columns a workgroup); a lane holds the state rows 4 (s + LPC jj) + t, t < 4, jj < NS / 4, so that q and k come from
 // LDS in 16-byte reads; LDS rows are padded with zeros to DP = NS * LPC values, under which the padded state rows stay zero.
+// A serial chain: what bounds it is the instructions of a step.  Four steps are unrolled with the operands in alternating registers (no moves), the sums are
+// DPP additions, outputs stay in a lane until LPC of them are written at once.  1409 rows in 5 sequences (the longest 470), 8 heads of 128 + 128: 106 us
+// (195 with a workgroup per row and 830 cycles a step).
 template <int NS, int LPC, int DBT>
 __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
   constexpr int CPB = 256 / LPC, DP = NS * LPC, NQ = DBT * 2 * DP / 256, NV = (DBT * CPB + 255) / 256;
   extern __shared__ float lds[];             // [DBT][2 DP] q, k; [DBT][CPB] v; [DBT] beta, decay, k . q; [DBT][CPB] outputs
-  const int m0 = blockIdx.y, ncb = (a.vdim + CPB - 1) / CPB, h = blockIdx.x / ncb, cb = blockIdx.x - h * ncb;
+  const int ncb = (a.vdim + CPB - 1) / CPB, h = blockIdx.x / ncb, cb = blockIdx.x - h * ncb;
   const int tid = threadIdx.x, s = tid % LPC, cl = tid / LPC, c = cb * CPB + cl;
-  if (a.row_back[m0] != 0) return;
   const int d = a.dim, kvh = h / (a.H / a.G);
   const bool on = c < a.vdim;
-  int n = 1;
-  for (;;) {
-    const int m = m0 + n + tid;
-    const int cnt = __syncthreads_count(m < a.M && a.row_back[m] == m - m0);
-    n += cnt;
-    if (cnt < 256) break;
-  }
-  float* sp = a.state + (((int64_t)a.row_seq[m0] * a.H + h) * d) * a.vdim + (on ? c : 0);
-  const bool fresh = a.row_slot[m0] == 0;
-  float S[NS];
-#pragma unroll
-  for (int j = 0; j < NS; ++j) {
-    const int i = 4 * (s + LPC * (j >> 2)) + (j & 3);
-    S[j] = (on && !fresh && i < d) ? sp[(int64_t)i * a.vdim] : 0.f;
-  }
-  float* qk = lds;                           // row r: q at r * 2 DP, k at r * 2 DP + DP
-  float* vs = qk + DBT * 2 * DP;
-  float* bs = vs + DBT * CPB;
-  float* os = bs + 3 * DBT;                   // [DBT][CPB] the batch's outputs
-  float rq[NQ], rv[NV], rb = 0.f;
-  // element e of a batch's q / k block: row e / (2 DP), value e % (2 DP) (q below DP, k from DP on)
-  auto fetch = [&](int b0) {
-    const int rows = min(DBT, n - b0);
-#pragma unroll
-    for (int t = 0; t < NQ; ++t) {
-      const int e = tid + 256 * t, r = e / (2 * DP), i = e % (2 * DP), ii = i % DP;
-      rq[t] = (r < rows && ii < d) ? a.qkv[(int64_t)(m0 + b0 + r) * a.ld + (i < DP ? 0 : a.G * d) + (int64_t)kvh * d + ii] : 0.f;
+  __shared__ uint64_t mask[32];
+  for (int seq = blockIdx.y;; seq += gridDim.y) {
+    const int m0 = __builtin_amdgcn_readfirstlane(sequence_start(a.row_back, a.M, seq, mask));
+    if (m0 < 0) return;
+    int n = 1;
+    for (;;) {
+      const int m = m0 + n + tid;
+      const int cnt = __syncthreads_count(m < a.M && a.row_back[m] == m - m0);
+      n += cnt;
+      if (cnt < 256) break;
     }
-#pragma unroll
-    for (int t = 0; t < NV; ++t) {
-      const int e = tid + 256 * t, r = e / CPB, cc = cb * CPB + e % CPB;
-      rv[t] = (r < rows && cc < a.vdim) ? a.qkv[(int64_t)(m0 + b0 + r) * a.ld + 2 * a.G * d + (int64_t)h * a.vdim + cc] : 0.f;
-    }
-    if (tid < 2 * DBT) {
-      const int r = tid % DBT;
-      rb = r < rows ? a.bd[(int64_t)(m0 + b0 + r) * a.ldbd + (tid < DBT ? 0 : a.H) + h] : 0.f;
-    }
-  };
-  fetch(0);
-  for (int b0 = 0; b0 < n; b0 += DBT) {
-    const int rows = min(DBT, n - b0);
-    lds_barrier();                           // the previous batch's steps have read their rows
-#pragma unroll
-    for (int t = 0; t < NQ; ++t) qk[tid + 256 * t] = rq[t];
-#pragma unroll
-    for (int t = 0; t < NV; ++t) { const int e = tid + 256 * t; if (e < DBT * CPB) vs[e] = rv[t]; }
-    if (tid < 2 * DBT) bs[tid] = rb;
-    lds_barrier();
-    if (b0 + DBT < n) fetch(b0 + DBT);         // in flight while this batch is computed
-    for (int r = tid >> 4; r < DBT; r += 16) {   // k . q of every row: 16 threads a row
-      const int l = tid & 15;
-      float t = 0.f;
-#pragma unroll
-      for (int i = l; i < DP; i += 16) t = fmaf(qk[r * 2 * DP + i], qk[r * 2 * DP + DP + i], t);
-      t = row16_sum(t);
-      if (l == 0) bs[2 * DBT + r] = t;
-    }
-    lds_barrier();                           // orders LDS only: the next batch's loads stay in flight
-    // the operands of step r + 1 are read from LDS before step r is computed: they do not depend on the state
-    float kk[NS], qq[NS], v, beta, g, kq;
-    auto load_row = [&](int r, float (&k_)[NS], float (&q_)[NS], float& v_, float& b_, float& g_, float& kq_) {
-      const float* q = qk + r * 2 * DP + 4 * s;
-#pragma unroll
-      for (int jj = 0; jj < NS / 4; ++jj) {
-        const float4 k4 = *reinterpret_cast<const float4*>(q + DP + 4 * LPC * jj), q4 = *reinterpret_cast<const float4*>(q + 4 * LPC * jj);
-        k_[4 * jj] = k4.x; k_[4 * jj + 1] = k4.y; k_[4 * jj + 2] = k4.z; k_[4 * jj + 3] = k4.w;
-        q_[4 * jj] = q4.x; q_[4 * jj + 1] = q4.y; q_[4 * jj + 2] = q4.z; q_[4 * jj + 3] = q4.w;
-      }
-      v_ = vs[r * CPB + cl]; b_ = bs[r]; g_ = bs[DBT + r]; kq_ = bs[2 * DBT + r];
-    };
-    load_row(0, kk, qq, v, beta, g, kq);
-#pragma unroll 2
-    for (int r = 0; r < rows; ++r) {
-      float kn[NS], qn[NS], vn, bn, gn, kqn;
-      load_row(min(r + 1, DBT - 1), kn, qn, vn, bn, gn, kqn);
-      float pk = 0.f, pq = 0.f, pk2 = 0.f, pq2 = 0.f;
-#pragma unroll
-      for (int j = 0; j < NS; j += 2) {
-        pk = fmaf(S[j], kk[j], pk); pk2 = fmaf(S[j + 1], kk[j + 1], pk2);
-        pq = fmaf(S[j], qq[j], pq); pq2 = fmaf(S[j + 1], qq[j + 1], pq2);
-      }
-      pk += pk2; pq += pq2;
-      if (LPC == 16) { pk = row16_sum(pk); pq = row16_sum(pq); } else { pk = sum8(pk); pq = sum8(pq); }
-      const float u = beta * (v - g * pk);
-#pragma unroll
-      for (int j = 0; j < NS; ++j) S[j] = fmaf(g, S[j], kk[j] * u);
-      if (s == 0) os[r * CPB + cl] = fmaf(g, pq, u * kq);
-#pragma unroll
-      for (int j = 0; j < NS; ++j) { kk[j] = kn[j]; qq[j] = qn[j]; }
-      v = vn; beta = bn; g = gn; kq = kqn;
-    }
-    lds_barrier();
-#pragma unroll
-    for (int t = 0; t < NV; ++t) {           // the batch's outputs, a row's columns side by side
-      const int e = tid + 256 * t, r = e / CPB, cc = cb * CPB + e % CPB;
-      if (r < rows && cc < a.vdim) a.out[(int64_t)(m0 + b0 + r) * a.ldo + (int64_t)h * a.vdim + cc] = os[e];
-    }
-  }
-  if (on) {
+    float* sp = a.state + (((int64_t)a.row_seq[m0] * a.H + h) * d) * a.vdim + (on ? c : 0);
+    const bool fresh = a.row_slot[m0] == 0;
+    float S[NS];
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
       const int i = 4 * (s + LPC * (j >> 2)) + (j & 3);
-      if (i < d) sp[(int64_t)i * a.vdim] = S[j];
+      S[j] = (on && !fresh && i < d) ? sp[(int64_t)i * a.vdim] : 0.f;
+    }
+    float* qk = lds;                           // row r: q at r * 2 DP, k at r * 2 DP + DP
+    float* vs = qk + DBT * 2 * DP;
+    float* bs = vs + DBT * CPB;
+    float* os = bs + 3 * DBT;                   // [DBT][CPB] the batch's outputs
+    float rq[NQ], rv[NV], rb = 0.f;
+    // element e of a batch's q / k block: row e / (2 DP), value e % (2 DP) (q below DP, k from DP on)
+    auto fetch = [&](int b0) {
+      const int rows = min(DBT, n - b0);
+#pragma unroll
+      for (int t = 0; t < NQ; ++t) {
+        const int e = tid + 256 * t, r = e / (2 * DP), i = e % (2 * DP), ii = i % DP;
+        rq[t] = (r < rows && ii < d) ? a.qkv[(int64_t)(m0 + b0 + r) * a.ld + (i < DP ? 0 : a.G * d) + (int64_t)kvh * d + ii] : 0.f;
+      }
+#pragma unroll
+      for (int t = 0; t < NV; ++t) {
+        const int e = tid + 256 * t, r = e / CPB, cc = cb * CPB + e % CPB;
+        rv[t] = (r < rows && cc < a.vdim) ? a.qkv[(int64_t)(m0 + b0 + r) * a.ld + 2 * a.G * d + (int64_t)h * a.vdim + cc] : 0.f;
+      }
+      if (tid < 2 * DBT) {
+        const int r = tid % DBT;
+        rb = r < rows ? a.bd[(int64_t)(m0 + b0 + r) * a.ldbd + (tid < DBT ? 0 : a.H) + h] : (tid < DBT ? 0.f : 1.f);
+      }
+    };
+    fetch(0);
+    for (int b0 = 0; b0 < n; b0 += DBT) {
+      const int rows = min(DBT, n - b0);
+      lds_barrier();                           // the previous batch's steps have read their rows
+#pragma unroll
+      for (int t = 0; t < NQ; ++t) qk[tid + 256 * t] = rq[t];
+#pragma unroll
+      for (int t = 0; t < NV; ++t) { const int e = tid + 256 * t; if (e < DBT * CPB) vs[e] = rv[t]; }
+      if (tid < 2 * DBT) bs[tid] = rb;
+      lds_barrier();
+      if (b0 + DBT < n) fetch(b0 + DBT);         // in flight while this batch is computed
+      for (int r = tid >> 4; r < DBT; r += 16) {   // k . q of every row: 16 threads a row
+        const int l = tid & 15;
+        float t = 0.f;
+#pragma unroll
+        for (int i = l; i < DP; i += 16) t = fmaf(qk[r * 2 * DP + i], qk[r * 2 * DP + DP + i], t);
+        t = row16_sum(t);
+        if (l == 0) bs[2 * DBT + r] = t;
+      }
+      lds_barrier();                           // orders LDS only: the next batch's loads stay in flight
+      // the operands of step r + 1 are read from LDS before step r is computed: they do not depend on the state.  (The read behind the last row stays
+      // inside the LDS block; rows up to the next multiple of 4 are zeros with decay 1.)
+      float kk[2][NS], qq[2][NS], v[2], beta[2], g[2], kq[2];
+      auto load_row = [&](int r, int b) {
+        const float* q = qk + r * 2 * DP + 4 * s;
+#pragma unroll
+        for (int jj = 0; jj < NS / 4; ++jj) {
+          const float4 k4 = *reinterpret_cast<const float4*>(q + DP + 4 * LPC * jj), q4 = *reinterpret_cast<const float4*>(q + 4 * LPC * jj);
+          kk[b][4 * jj] = k4.x; kk[b][4 * jj + 1] = k4.y; kk[b][4 * jj + 2] = k4.z; kk[b][4 * jj + 3] = k4.w;
+          qq[b][4 * jj] = q4.x; qq[b][4 * jj + 1] = q4.y; qq[b][4 * jj + 2] = q4.z; qq[b][4 * jj + 3] = q4.w;
+        }
+        v[b] = vs[r * CPB + cl]; beta[b] = bs[r]; g[b] = bs[DBT + r]; kq[b] = bs[2 * DBT + r];
+      };
+      load_row(0, 0);
+      for (int rb = 0; rb < rows; rb += LPC) {
+        float keep = 0.f;                      // lane s: the output of row rb + s
+        for (int r0 = rb; r0 < min(rows, rb + LPC); r0 += 4) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int b = j & 1;
+            load_row(r0 + j + 1, b ^ 1);
+            float pk = 0.f, pq = 0.f, pk2 = 0.f, pq2 = 0.f;
+#pragma unroll
+            for (int i = 0; i < NS; i += 2) {
+              pk = fmaf(S[i], kk[b][i], pk); pk2 = fmaf(S[i + 1], kk[b][i + 1], pk2);
+              pq = fmaf(S[i], qq[b][i], pq); pq2 = fmaf(S[i + 1], qq[b][i + 1], pq2);
+            }
+            pk += pk2; pq += pq2;
+            if (LPC == 16) { pk = row16_sum(pk); pq = row16_sum(pq); } else { pk = sum8(pk); pq = sum8(pq); }
+            const float u = beta[b] * (v[b] - g[b] * pk);
+#pragma unroll
+            for (int i = 0; i < NS; ++i) S[i] = fmaf(g[b], S[i], kk[b][i] * u);
+            keep = s == r0 + j - rb ? fmaf(g[b], pq, u * kq[b]) : keep;
+          }
+        }
+        os[(rb + s) * CPB + cl] = keep;
+      }
+      lds_barrier();
+#pragma unroll
+      for (int t = 0; t < NV; ++t) {           // the batch's outputs, a row's columns side by side
+        const int e = tid + 256 * t, r = e / CPB, cc = cb * CPB + e % CPB;
+        if (r < rows && cc < a.vdim) a.out[(int64_t)(m0 + b0 + r) * a.ldo + (int64_t)h * a.vdim + cc] = os[e];
+      }
+    }
+    if (on) {
+#pragma unroll
+      for (int j = 0; j < NS; ++j) {
+        const int i = 4 * (s + LPC * (j >> 2)) + (j & 3);
+        if (i < d) sp[(int64_t)i * a.vdim] = S[j];
+      }
     }
   }
 }
@@ -692,8 +703,10 @@ extern "C" int mn_gated_delta_rows(const float* qkv, int64_t ld, const float* bd
   }
   if (dim <= 256) {
     MN_CHECK_ARG(M <= 65535 && (int64_t)H * mn_cdiv(vdim, 16) < ((int64_t)1 << 31), "mn_gated_delta_rows: too many rows or columns");
+    // sequences walked side by side: two workgroups a CU (what LDS lets in), the rest one after the other
+    auto slots = [&](int64_t gx) { const int64_t y = 2 * (int64_t)mn_num_cus() / gx; return (unsigned)(y < 1 ? 1 : (y < M ? y : M)); };
 #define MN_DF(NS_, LPC_, DB_)                                                                                                                 \
-  hipLaunchKernelGGL((delta_rows_fast_kernel<NS_, LPC_, DB_>), dim3((unsigned)(H * mn_cdiv(vdim, 256 / LPC_)), (unsigned)M), dim3(256),  \
+  hipLaunchKernelGGL((delta_rows_fast_kernel<NS_, LPC_, DB_>), dim3((unsigned)(H * mn_cdiv(vdim, 256 / LPC_)), slots(H * mn_cdiv(vdim, 256 / LPC_))), dim3(256),  \
                      ((size_t)DB_ * 2 * NS_ * LPC_ + 2 * DB_ * (256 / LPC_) + 3 * DB_) * sizeof(float), st, a)
     if (dim <= 32) MN_DF(4, 8, 32); else if (dim <= 64) MN_DF(4, 16, 32); else if (dim <= 128) MN_DF(8, 16, 32); else MN_DF(16, 16, 16);
 #undef MN_DF

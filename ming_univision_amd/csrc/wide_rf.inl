@@ -1,6 +1,5 @@
-// wide_rf.inl — RectifiedFlowLoss.sample (diff_loss_rf_swiglu.py:103-181) for 65..2048 CFG rows advancing in lock-step
-// (textually part of engine.hip).  Same arithmetic as the <= 64-row route of mn_rf_sample; at this width the launches are
-// MFMA-bound, so every Linear is a gemm256 launch on bf16 hi/lo operands (fp32-class products) and the work between two
+// wide_rf.inl — RectifiedFlowLoss.sample (diff_loss_rf_swiglu.py:103-181) for 24..2048 CFG rows advancing in lock-step
+// (textually part of engine.hip).  Same arithmetic as the streaming route of mn_rf_sample; every Linear is a gemm256 launch on bf16 hi/lo operands (fp32-class products) and the work between two
 // Linears is one wide_glue launch:
 //
 //   per visual token   vis_head Linear -> LayerNorm -> cond_embed           (modeling_bailing_moe.py:1571-1574, diff_loss:374)
@@ -10,12 +9,17 @@
 //                      w3 GEMM, split-K partial slabs
 //                      [slab reduce + b3 + gated residual + next in_ln / final LN + modulate]   (diff_loss:270-272, 290)
 //                      final Linear (split-K) -> bias -> CFG combine + Euler step              (diff_loss:144-179, 291)
-// First row count that takes the wide route, per stage (measured crossovers); mn_wide_tune is the A/B hook.
-static int g_wide_min_llm = 65, g_wide_min_rf = 41, g_wide_min_sem = 65;
+// First row count that takes the wide route, per stage (measured crossovers); mn_wide_tune is the A/B hook.  The flow head's bf16 weights go by tiles
+// from 24 rows on: 64 x 64 tiles pay the same for 12 and for 64 rows (w12 of 3072 x 16384 with its SwiGLU 27 us, w3 16 us at 36 rows), the streaming
+// kernels and the launches between them do not (26.6 + 5.5, 19.3 us).  A token of 36 rows: 20.9 -> 19.4 ms; 30 rows 18.3 -> 18.0; 24 rows 17.4 -> 17.2; 16
+// rows 15.0 against 15.7.  Weight-only formats are expanded to bf16 once per call on this route and keep their line at 41.
+// The semantic decoder likewise (a token of 12 rows the same, 24 rows 17.3 -> 16.9 ms, 36 rows 19.4 -> 19.0, 64 rows 22.8 -> 22.3); the language model's experts
+// keep the streaming kernels up to 64 rows (64 rows of 1100 tokens: 10.8 against 11.1 ms).
+static int g_wide_min_llm = 65, g_wide_min_rf = 24, g_wide_min_rf_w8 = 41, g_wide_min_sem = 16;
 #ifdef MN_DEV_HOOKS
 extern "C" MN_DEV_API void mn_wide_tune(int llm_min_rows, int rf_min_rows, int sem_min_rows) {
   if (llm_min_rows > 0) g_wide_min_llm = llm_min_rows;
-  if (rf_min_rows > 0) g_wide_min_rf = rf_min_rows;
+  if (rf_min_rows > 0) g_wide_min_rf = g_wide_min_rf_w8 = rf_min_rows;
   if (sem_min_rows > 0) g_wide_min_sem = sem_min_rows;
 }
 #endif
@@ -106,9 +110,10 @@ static size_t rf_wide_carve(const mn_rf_head* h, int rows, void* ws, size_t cap,
   Carver cv(ws, cap, ws == nullptr);
   const int64_t SR = (int64_t)h->steps * rows;
   const int A = h->depth * 3 * h->w + 2 * h->w;
-  // w12: the SwiGLU epilogue needs the whole K sum, i.e. cdiv(rows, 128) * hidden / 128 workgroups; below a chip's worth of them
-  // the plain split-K form + rf_swiglu_slabs_kernel is the faster pair (128 rows: 69 -> 3x us per block)
-  o->ks12 = mn_cdiv(rows, 128) * (h->hidden / 128) >= 256 ? 1 : rf_wide_ksplit(rows, 2 * h->hidden, h->w);
+  // w12: the SwiGLU epilogue needs the whole K sum.  Up to 64 rows one row of 64 x 64 tiles reads every weight byte once and fills the chip from 4096
+  // hidden units on (64 rows x 3072 x 16384: 30.3 us; in two K-slices 29.6 + 8 for the launch behind them); above, cdiv(rows, 128) * hidden / 128
+  // workgroups, and below a chip's worth of them the split-K form + rf_swiglu_slabs_kernel is the faster pair (96 rows: 41.8 against 31 + 8)
+  o->ks12 = (rows <= 64 && h->hidden >= 4096) || mn_cdiv(rows, 128) * (h->hidden / 128) >= 256 ? 1 : rf_wide_ksplit(rows, 2 * h->hidden, h->w);
   o->ks3 = rf_wide_ksplit(rows, h->w, h->hidden);
   o->ksf = rf_wide_ksplit(rows, h->target, h->w);
   const size_t p3 = (size_t)mn_gemm256_slices(h->hidden, o->ks3) * rows * h->w;
@@ -135,7 +140,7 @@ static size_t rf_wide_carve(const mn_rf_head* h, int rows, void* ws, size_t cap,
 
 static bool rf_wide_ok(const mn_rf_head* h, int rows) {
   const bool fmt_ok = h->wfmt == MN_W_BF16 || ((h->wfmt == MN_W_FP8_E4M3 || h->wfmt == MN_W_INT8 || h->wfmt == MN_W_NF4) && h->w12_scale && h->w3_scale && h->ada_w);
-  return fmt_ok && rows >= g_wide_min_rf && rows <= 2048 && wide_glue_ok(h->w) && wide_glue_ok(h->z_dim) && wide_glue_ok(h->llm_hidden) &&
+  return fmt_ok && rows >= (h->wfmt ? g_wide_min_rf_w8 : g_wide_min_rf) && rows <= 2048 && wide_glue_ok(h->w) && wide_glue_ok(h->z_dim) && wide_glue_ok(h->llm_hidden) &&
          (h->w % 64) == 0 && (h->hidden % 64) == 0 && (h->z_dim % 64) == 0 && (h->llm_hidden % 64) == 0 && h->target <= 64 &&
          (h->target % 4) == 0;
 }

@@ -1,0 +1,159 @@
+// rows_kc.inl — a Linear of 2 .. 32 rows in one launch (included inside skinny_gemm.hip's anonymous namespace).
+//
+// The three-launch form (split the rows into hi / lo, stream the weights in K-slices, sum the slices) pays 4 .. 6 us for each of its small launches; at
+// the sizes of a decoder's projections that is more than the product.  Here a workgroup owns NT tiles of 16 columns with ALL of K: its 8 waves take
+// 64-value chunks of K in turn, read weights and fp32 rows straight into MFMA operands (lane l: row / column l & 15, values 8 (l >> 4) .. + 7
+// of every 32), split the rows there into three bf16 parts (24 bits: products of all of an fp32 value, 2e-7 of the result off 64 bits where hi + lo is
+// 2.5e-6; the third part costs 2 %) and meet once, in LDS, for the sum of the eight waves' tiles and the epilogue.  Every workgroup
+// reads all rows (M K 4 bytes, from L2), every weight byte is read once; the next chunk's loads are in flight during a chunk's products.  What bounds it is the load and
+// conversion of the rows (0.85 us + 0.042 a row for each 512 values of K; weights two or four chunks ahead, or 8-byte pieces that coalesce better, changed
+// nothing or cost 25 %).  2048 x 2048: 5.5 us at 2 rows, 7.9 at 16, 11.7 at 32 (10.0, 11.3, 13.7 as three launches); 4096 x 1024 4.2, 5.4, 7.6 (9.6, 10.9, 13.1).
+// RMSNorm: the gain multiplies the values, 1 / rms the sums (each wave adds up the squares of its chunks).
+// Paired epilogues (gate, up): tile t < NT / 2 holds gate columns, tile t + NT / 2 the up columns of the same units.
+typedef short bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));      // rows start at any float: a 16-byte load needs 4-byte alignment here
+
+// a pair of values as three pairs of bf16, 24 bits: all of an fp32 value
+__device__ __forceinline__ void split3_pk_bf16(float a, float b, u32x4 (&part)[3], int at) {
+  uint32_t h = cvt_pk_bf16(a, b);
+  part[0][at] = h;
+  a -= bf16lo_to_f32(h); b -= bf16hi_to_f32(h);
+  h = cvt_pk_bf16(a, b);
+  part[1][at] = h;
+  part[2][at] = cvt_pk_bf16(a - bf16lo_to_f32(h), b - bf16hi_to_f32(h));
+}
+
+template <int MT, int NT, int PRO>
+__global__ __launch_bounds__(512) void rows_kc_kernel(const mn_skinny_args a, int paired) {
+  constexpr int NW = 8, CK = 64, R = MT * NT * 4;
+  __shared__ float red[NW][R][64];
+  __shared__ float sq[PRO == MN_PRO_RMSNORM ? NW : 1][16 * MT];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int K = a.K, M = a.M, N = a.N, G = paired ? NT / 2 : NT;             // G: tiles of units per workgroup
+  const int n0 = blockIdx.x * 16 * G;
+  const bf16_t* wp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wp[t] = a.w + (int64_t)(min(n0 + 16 * (t % G) + r, N - 1) + (t >= G ? N : 0)) * K + 8 * q;
+  const float *xp[MT], *pp[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = min(16 * i + r, M - 1);
+    xp[i] = a.x + (int64_t)m * a.ldx + 8 * q;
+    pp[i] = PRO == MN_PRO_ADD_SILU ? a.pro_a + (int64_t)m * a.ld_pro_a + 8 * q : nullptr;
+  }
+  f32x4 acc[MT][NT], xf[MT][2][2];
+  u32x4 wf[NT][2];
+  float ss[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    ss[i] = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // K is a multiple of 8: a lane's 8 values are all inside K or all beyond it, where it reads its row's start and both operands become zeros
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int k = k0 + 32 * s, kk = k + 8 * q < K ? k : -8 * q;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wf[t][s] = *reinterpret_cast<const u32x4*>(wp[t] + kk);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        xf[i][s][0] = *reinterpret_cast<const f32x4u*>(xp[i] + kk);
+        xf[i][s][1] = *reinterpret_cast<const f32x4u*>(xp[i] + kk + 4);
+      }
+    }
+  };
+  if (wave * CK < K) fetch(wave * CK);
+  for (int k0 = wave * CK; k0 < K; k0 += NW * CK) {
+    f32x4 cx[MT][2][2];
+    u32x4 cw[NT][2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) cw[t][s] = wf[t][s];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) { cx[i][s][0] = xf[i][s][0]; cx[i][s][1] = xf[i][s][1]; }
+    }
+    if (k0 + NW * CK < K) fetch(k0 + NW * CK);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int k = k0 + 32 * s + 8 * q;
+      const bool in = k < K;
+      f32x4 g0, g1;
+      if (PRO == MN_PRO_RMSNORM) {
+        const u32x4 gw = *reinterpret_cast<const u32x4*>(a.ln_g + (in ? k : 0));
+        g0 = f32x4{bf16lo_to_f32(gw.x), bf16hi_to_f32(gw.x), bf16lo_to_f32(gw.y), bf16hi_to_f32(gw.y)};
+        g1 = f32x4{bf16lo_to_f32(gw.z), bf16hi_to_f32(gw.z), bf16lo_to_f32(gw.w), bf16hi_to_f32(gw.w)};
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        f32x4 v0 = cx[i][s][0], v1 = cx[i][s][1];
+        if (PRO == MN_PRO_ADD_SILU) {
+          const int kk = in ? k - 8 * q : -8 * q;
+          v0 += *reinterpret_cast<const f32x4u*>(pp[i] + kk);
+          v1 += *reinterpret_cast<const f32x4u*>(pp[i] + kk + 4);
+        }
+        if (PRO == MN_PRO_SILU || PRO == MN_PRO_ADD_SILU) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { v0[e] = silu_f(v0[e]); v1[e] = silu_f(v1[e]); }
+        }
+        if (!in) v0 = v1 = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (PRO == MN_PRO_RMSNORM) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) ss[i] = fmaf(v0[e], v0[e], fmaf(v1[e], v1[e], ss[i]));
+          v0 *= g0; v1 *= g1;
+        }
+        u32x4 part[3];
+        split3_pk_bf16(v0[0], v0[1], part, 0);
+        split3_pk_bf16(v0[2], v0[3], part, 1);
+        split3_pk_bf16(v1[0], v1[1], part, 2);
+        split3_pk_bf16(v1[2], v1[3], part, 3);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const bf16x8 w = __builtin_bit_cast(bf16x8, in ? cw[t][s] : u32x4{0, 0, 0, 0});
+#pragma unroll
+          for (int p = 2; p >= 0; --p) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, part[p]), w, acc[i][t], 0, 0, 0);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) red[wave][(i * 4 + e) * NT + t][lane] = acc[i][t][e];
+    if (PRO == MN_PRO_RMSNORM) {
+      ss[i] += __shfl_xor(ss[i], 16);
+      ss[i] += __shfl_xor(ss[i], 32);
+      if (q == 0) sq[wave][16 * i + r] = ss[i];
+    }
+  }
+  __syncthreads();
+  for (int j = wave; j < 4 * MT; j += NW) {                                  // row 16 (j / 4) + 4 q + j % 4 of every tile
+    const int ml = 16 * (j >> 2) + 4 * q + (j & 3);
+    float rstd = 1.f;
+    if (PRO == MN_PRO_RMSNORM) {
+      float t = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) t += sq[w][ml];
+      rstd = rsqrtf(t / (float)K + a.eps);
+    }
+    float y[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) v += red[w][j * NT + t][lane];
+      y[t] = PRO == MN_PRO_RMSNORM ? v * rstd : v;
+    }
+    if (ml >= M) continue;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int n = n0 + 16 * t + r;
+      if (t >= G || n >= N) continue;
+      medium_finish(a, ml, n, y[t], NT > 1 ? y[NT > 1 && paired ? t + NT / 2 : 0] : 0.f);
+    }
+  }
+}

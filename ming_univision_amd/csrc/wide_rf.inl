@@ -13,9 +13,9 @@
 // from 24 rows on: 64 x 64 tiles pay the same for 12 and for 64 rows (w12 of 3072 x 16384 with its SwiGLU 27 us, w3 16 us at 36 rows), the streaming
 // kernels and the launches between them do not (26.6 + 5.5, 19.3 us).  A token of 36 rows: 20.9 -> 19.4 ms; 30 rows 18.3 -> 18.0; 24 rows 17.4 -> 17.2; 16
 // rows 15.0 against 15.7.  Weight-only formats are expanded to bf16 once per call on this route and keep their line at 41.
-// The semantic decoder likewise (a token of 12 rows the same, 24 rows 17.3 -> 16.9 ms, 36 rows 19.4 -> 19.0, 64 rows 22.8 -> 22.3); the language model's experts
+// The semantic decoder likewise beyond the 32 rows whose projections are one launch (a token of 64 rows 22.8 -> 22.3 ms); the language model's experts
 // keep the streaming kernels up to 64 rows (64 rows of 1100 tokens: 10.8 against 11.1 ms).
-static int g_wide_min_llm = 65, g_wide_min_rf = 24, g_wide_min_rf_w8 = 41, g_wide_min_sem = 16;
+static int g_wide_min_llm = 65, g_wide_min_rf = 24, g_wide_min_rf_w8 = 41, g_wide_min_sem = 33;
 #ifdef MN_DEV_HOOKS
 extern "C" MN_DEV_API void mn_wide_tune(int llm_min_rows, int rf_min_rows, int sem_min_rows) {
   if (llm_min_rows > 0) g_wide_min_llm = llm_min_rows;

@@ -1,0 +1,79 @@
+"""A Linear of 2 .. 32 rows as one launch (rows_kc.inl) around its edges: one and two row tiles, columns that fill no tile, one and two tiles a workgroup, K that
+ends inside a chunk or leaves waves without one, every prologue and epilogue it takes, rows in wider buffers, and calls it must leave to the three
+launches (output over the input, LayerNorm, more rows).  The reference is float64; hi / lo rows (the three launches) carry 17 bits:
+2^-16 of the summed magnitudes."""
+import ctypes as C
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+F = torch.nn.functional
+
+
+def call(x, ldx, w, out, ldo, M, N, K, ws, **kw):
+    from ming_univision_amd._lib import SkinnyArgs, check, current_stream, lib
+    a = SkinnyArgs()
+    a.x, a.ldx, a.w, a.ldw, a.out, a.ldo, a.M, a.N, a.K = x, ldx, w.data_ptr(), K, out, ldo, M, N, K
+    a.ws, a.ws_bytes = ws.data_ptr(), ws.numel()
+    for k, v in kw.items():
+        setattr(a, k, v.data_ptr() if torch.is_tensor(v) else v)
+    check(lib().mn_skinny_gemm(C.byref(a), current_stream()), "skinny")
+
+
+@pytest.mark.parametrize("M", [2, 3, 16, 17, 32, 33])
+@pytest.mark.parametrize("N,K", [(1, 8), (66, 200), (16, 512), (250, 1032), (1024, 1024), (4097, 504), (4500, 1024), (2048, 2048)])
+def test_forms(M, N, K):
+    from ming_univision_amd._lib import lib
+    g = torch.Generator().manual_seed(M + N + K)
+    w = (torch.randn(2 * N, K, generator=g)).bfloat16().cuda()
+    bias, gain = torch.randn(2 * N, generator=g).bfloat16().cuda(), (1 + 0.2 * torch.randn(K, generator=g)).bfloat16().cuda()
+    beta = (0.2 * torch.randn(K, generator=g)).bfloat16().cuda()
+    xb, pb = (torch.randn(M, K + 3, generator=g) + 0.3).cuda(), torch.randn(M, K + 5, generator=g).cuda()
+    x, add = xb[:, 1:1 + K].double(), pb[:, 2:2 + K].double()
+    res, gate = torch.randn(M, N + 1, generator=g).cuda(), torch.randn(M, N, generator=g).cuda()
+    L = lib()
+    L.mn_skinny_workspace_bytes.restype = C.c_size_t
+    rows = {0: x, 1: F.silu(x), 2: F.silu(x + add), 3: x * torch.rsqrt((x * x).mean(1, keepdim=True) + 1e-6) * gain.double(),
+            4: F.layer_norm(x, (K,), gain.double(), beta.double(), 1e-6)}
+    for pro, epi, with_bias in ((0, 0, 0), (0, 0, 1), (1, 1, 1), (2, 2, 1), (3, 0, 0), (3, 3, 1), (0, 3, 0), (0, 4, 1), (0, 5, 1), (0, 6, 0), (4, 0, 1)):
+        pair = epi in (3, 6)
+        r, wd, bd = rows[pro], w[:2 * N if pair else N].double(), bias[:2 * N if pair else N].double() * with_bias
+        y, mag = r @ wd.T + bd, r.abs() @ wd.abs().T + bd.abs()
+        room = mag[:, :N].clone()
+        if pair:
+            up, act = y[:, N:], F.silu(y[:, :N]) if epi == 3 else F.gelu(y[:, :N], approximate="tanh")
+            room = 1.2 * mag[:, :N] * up.abs() + mag[:, N:] * act.abs()      # both activations are 1.13-Lipschitz
+            y = act * up
+        elif epi in (1, 2):
+            y, room = (F.silu(y) if epi == 1 else F.gelu(y)), 1.2 * room
+        elif epi == 4:
+            y, room = y + res[:, :N].double(), room + res[:, :N].double().abs()
+        elif epi == 5:
+            room = room * gate.double().abs() + res[:, :N].double().abs()
+            y = res[:, :N].double() + gate.double() * y
+        ws = torch.empty(L.mn_skinny_workspace_bytes(M, N, K, epi), dtype=torch.uint8, device="cuda")
+        out = torch.full((M + 1, N + 2), 7.0, device="cuda")
+        kw = dict(prologue=pro, epilogue=epi, eps=1e-6, ln_g=gain, ln_b=beta, pro_a=pb.data_ptr() + 8, ld_pro_a=K + 5, res=res, ldres=N + 1, gate=gate, ldgate=N)
+        if with_bias:
+            kw["bias"] = bias
+        call(xb.data_ptr() + 4, K + 3, w, out.data_ptr(), N + 2, M, N, K, ws, **kw)
+        assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+        assert float(((out[:M, :N].double() - y).abs() / (room + 1e-3)).max()) < 2.0 ** -15, (pro, epi)
+
+
+def test_output_over_the_input():
+    """The rows are all read before any is written: out = x, and out between the rows of x."""
+    from ming_univision_amd._lib import lib
+    g = torch.Generator().manual_seed(3)
+    M, N = 12, 512
+    w = (torch.randn(N, N, generator=g) * N ** -0.5).bfloat16().cuda()
+    ws = torch.empty(lib().mn_skinny_workspace_bytes(M, N, N, 0), dtype=torch.uint8, device="cuda")
+    for ld, at in ((N, 0), (2 * N, N), (N + 64, 32)):
+        buf = torch.randn(M + 1, ld, generator=g).cuda()
+        flat = buf.reshape(-1)
+        x = torch.stack([flat[i * ld:i * ld + N] for i in range(M)]).double()
+        call(buf.data_ptr(), ld, w, buf.data_ptr() + 4 * at, ld, M, N, N, ws)
+        got = torch.stack([flat[i * ld + at:i * ld + at + N] for i in range(M)]).double()
+        want = x @ w.double().T
+        assert float((got - want).abs().max() / want.abs().max()) < 1e-5

@@ -132,6 +132,12 @@ __device__ __forceinline__ float wave_max(float v) {
   v = row16_max(v);
   return fmaxf(fmaxf(lane_f(v, 0), lane_f(v, 16)), fmaxf(lane_f(v, 32), lane_f(v, 48)));
 }
+// s + l += v, s rounded, l collecting what the rounding left
+__device__ __forceinline__ void two_sum(float& s, float& l, float v) {
+  const float t = s + v, b = t - s;
+  l += (s - (t - b)) + (v - b);
+  s = t;
+}
 // Block-wide sum; `red` is LDS scratch of >= blockDim.x/64 floats. All threads get the result.
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);

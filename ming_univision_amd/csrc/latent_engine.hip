@@ -174,7 +174,9 @@ extern "C" int mn_seq_step(const mn_seq_model* m, const mn_seq_state* st, const 
     // absorb: qabs[m, h, :] = scale * q[m, h, :] W_uk[h]   (W_ukT[h] is [kv_rank, dim])
     MN_TRY(mn_gemm_f32_batched(qp, ldq, l.dim, l.w_ukT, l.dim, (int64_t)l.kv_rank * l.dim, nullptr, qabs, d.hr, l.kv_rank, nullptr, 0, 0,
                                nullptr, 0, 0, M, l.kv_rank, l.dim, l.heads, l.scale, stream));
-    const int ks = mn_latent_attn_splits(n_blk, max_len, l.kv_rank);
+    // (16 vectors a workgroup: a run of several rows is several workgroups, and needs its keys split that much less.  1500 prompt rows of 16 heads: two splits
+    // nobody needed cost 42 us of merging a layer)
+    const int ks = mn_latent_attn_splits(n_blk * (int)mn_cdiv((M > n_blk ? mn_latent_attn_block_rows() : 1) * l.heads, 16), max_len, l.kv_rank);
     MN_TRY(mn_latent_attn(qabs, arena, row_seq, row_len, blk_tab, n_blk, M, l.heads, l.kv_rank, st->t_max, max_len, ks, lat, attn_ws,
                           p.attn_ws, stream));
     // expand: att[m, h, :] = W_uv[h] lat[m, h, :]  (* sigmoid(gate))

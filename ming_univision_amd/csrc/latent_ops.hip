@@ -256,13 +256,6 @@ __device__ __forceinline__ void f32_store(const GemmF32& a, int z, int m, int n,
 // one 16-byte read of each operand, in an order of K that both share.  Values past K enter as zeros.  V4: rows of A are 16-byte, rows
 // of W 8-byte aligned; else value by value.
 
-// s + l += v, s rounded, l collecting what the rounding left
-__device__ __forceinline__ void two_sum(float& s, float& l, float v) {
-  const float t = s + v, b = t - s;
-  l += (s - (t - b)) + (v - b);
-  s = t;
-}
-
 // Few tiles: 32 x 16 outputs a workgroup, whose four waves split K; operands straight from memory, the next 32 values in flight during
 // the products.  Latency bounds it (32 rows x 16 heads of 512 x 128: 5 us here, 45 us as one wave a column and 8 rows).  A block of 32
 // values is summed as a tree of single products and added to the running sum with its rounding error kept (two-sum), so the

@@ -3,21 +3,24 @@
 // The three-launch form (split the rows into hi / lo, stream the weights in K-slices, sum the slices) pays 4 .. 6 us for each of its small launches; at
 // the sizes of a decoder's projections that is more than the product.  Here a workgroup owns NT tiles of 16 columns with ALL of K: its 8 waves take
 // 64-value chunks of K in turn, read weights and fp32 rows straight into MFMA operands (lane l: row / column l & 15, values 8 (l >> 4) .. + 7
-// of every 32), split the rows there into three bf16 parts (24 bits: products of all of an fp32 value, 2e-7 of the result off 64 bits where hi + lo is
-// 2.5e-6; the third part costs 2 %) and meet once, in LDS, for the sum of the eight waves' tiles and the epilogue.  Every workgroup
-// reads all rows (M K 4 bytes, from L2), every weight byte is read once; the next chunk's loads are in flight during a chunk's products.  What bounds it is the load and
-// conversion of the rows (0.85 us + 0.042 a row for each 512 values of K; weights two or four chunks ahead, or 8-byte pieces that coalesce better, changed
-// nothing or cost 25 %).  2048 x 2048: 5.5 us at 2 rows, 7.9 at 16, 11.7 at 32 (10.0, 11.3, 13.7 as three launches); 4096 x 1024 4.2, 5.4, 7.6 (9.6, 10.9, 13.1).
+// of every 32), split the rows there into three bf16 parts (24 bits: products of all of an fp32 value) and meet once, in LDS, for the sum of the eight
+// waves' tiles and the epilogue.  A chunk's sum joins the running one with its rounding kept (two-sum): 1.5e-8 of the summed magnitudes off 64 bits at
+// the most, 2.0e-8 on the fp32 FMA kernel, 4e-7 as hi + lo.  Every workgroup reads all rows (M K 4 bytes, from L2), every weight byte is read once; the
+// next chunk's loads are in flight during a chunk's products.  What bounds it is the load and conversion of the rows (0.85 us + 0.042 a row for each 512
+// values of K; weights two or four chunks ahead, or 8-byte pieces that coalesce better, changed nothing or cost 25 %).  2048 x 2048: 6.2 us at 2 rows, 8.2 at
+// 16, 12.1 at 32 (10.0, 11.3, 13.7 as three launches); 4096 x 1024 4.6, 5.7, 8.0 (9.6, 10.9, 13.1).
 // RMSNorm: the gain multiplies the values, 1 / rms the sums (each wave adds up the squares of its chunks).
 // Paired epilogues (gate, up): tile t < NT / 2 holds gate columns, tile t + NT / 2 the up columns of the same units.
 typedef short bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));      // rows start at any float: a 16-byte load needs 4-byte alignment here
 
-// a pair of values as three pairs of bf16, 24 bits: all of an fp32 value
+// a pair of values as three pairs of bf16, 24 bits: all of an fp32 value (ODD: of a value that may be infinite; what is left of it is nothing, not inf - inf)
+template <bool ODD>
 __device__ __forceinline__ void split3_pk_bf16(float a, float b, u32x4 (&part)[3], int at) {
   uint32_t h = cvt_pk_bf16(a, b);
   part[0][at] = h;
   a -= bf16lo_to_f32(h); b -= bf16hi_to_f32(h);
+  if (ODD) { a = a == a ? a : 0.f; b = b == b ? b : 0.f; }
   h = cvt_pk_bf16(a, b);
   part[1][at] = h;
   part[2][at] = cvt_pk_bf16(a - bf16lo_to_f32(h), b - bf16hi_to_f32(h));
@@ -41,14 +44,14 @@ __global__ __launch_bounds__(512) void rows_kc_kernel(const mn_skinny_args a, in
     xp[i] = a.x + (int64_t)m * a.ldx + 8 * q;
     pp[i] = PRO == MN_PRO_ADD_SILU ? a.pro_a + (int64_t)m * a.ld_pro_a + 8 * q : nullptr;
   }
-  f32x4 acc[MT][NT], xf[MT][2][2];
+  f32x4 acc[MT][NT], low[MT][NT], xf[MT][2][2];
   u32x4 wf[NT][2];
   float ss[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     ss[i] = 0.f;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT; ++t) acc[i][t] = low[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   // K is a multiple of 8: a lane's 8 values are all inside K or all beyond it, where it reads its row's start and both operands become zeros
   auto fetch = [&](int k0) {
@@ -76,6 +79,11 @@ __global__ __launch_bounds__(512) void rows_kc_kernel(const mn_skinny_args a, in
       for (int i = 0; i < MT; ++i) { cx[i][s][0] = xf[i][s][0]; cx[i][s][1] = xf[i][s][1]; }
     }
     if (k0 + NW * CK < K) fetch(k0 + NW * CK);
+    f32x4 sum[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) sum[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const int k = k0 + 32 * s + 8 * q;
@@ -105,25 +113,44 @@ __global__ __launch_bounds__(512) void rows_kc_kernel(const mn_skinny_args a, in
           v0 *= g0; v1 *= g1;
         }
         u32x4 part[3];
-        split3_pk_bf16(v0[0], v0[1], part, 0);
-        split3_pk_bf16(v0[2], v0[3], part, 1);
-        split3_pk_bf16(v1[0], v1[1], part, 2);
-        split3_pk_bf16(v1[2], v1[3], part, 3);
+        float most = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) most = fmaxf(most, fmaxf(fabsf(v0[e]), fabsf(v1[e])));
+        if (__ballot(most == INFINITY) == 0) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) { split3_pk_bf16<false>(v0[2 * e], v0[2 * e + 1], part, e); split3_pk_bf16<false>(v1[2 * e], v1[2 * e + 1], part, 2 + e); }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) { split3_pk_bf16<true>(v0[2 * e], v0[2 * e + 1], part, e); split3_pk_bf16<true>(v1[2 * e], v1[2 * e + 1], part, 2 + e); }
+        }
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           const bf16x8 w = __builtin_bit_cast(bf16x8, in ? cw[t][s] : u32x4{0, 0, 0, 0});
 #pragma unroll
-          for (int p = 2; p >= 0; --p) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, part[p]), w, acc[i][t], 0, 0, 0);
+          for (int p = 2; p >= 0; --p) sum[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, part[p]), w, sum[i][t], 0, 0, 0);
         }
       }
     }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float a0 = acc[i][t][e], l0 = low[i][t][e];
+          two_sum(a0, l0, sum[i][t][e]);
+          acc[i][t][e] = a0; low[i][t][e] = l0;
+        }
   }
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) red[wave][(i * 4 + e) * NT + t][lane] = acc[i][t][e];
+      for (int e = 0; e < 4; ++e) {
+        const float v = acc[i][t][e] + low[i][t][e];
+        red[wave][(i * 4 + e) * NT + t][lane] = v == v ? v : acc[i][t][e];   // a sum at infinity has no error term
+      }
     if (PRO == MN_PRO_RMSNORM) {
       ss[i] += __shfl_xor(ss[i], 16);
       ss[i] += __shfl_xor(ss[i], 32);
@@ -143,9 +170,10 @@ __global__ __launch_bounds__(512) void rows_kc_kernel(const mn_skinny_args a, in
     float y[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      float v = 0.f;
+      float p[NW];
 #pragma unroll
-      for (int w = 0; w < NW; ++w) v += red[w][j * NT + t][lane];
+      for (int w = 0; w < NW; ++w) p[w] = red[w][j * NT + t][lane];
+      const float v = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
       y[t] = PRO == MN_PRO_RMSNORM ? v * rstd : v;
     }
     if (ml >= M) continue;

@@ -333,13 +333,15 @@ extern "C" size_t mn_skinny_workspace_bytes_w8(int M, int N, int K, int epilogue
   return mn_skinny_workspace_bytes_wq(MN_W_FP8_E4M3, M, N, K, epilogue);
 }
 
-// One launch (rows_kc.inl) for up to 32 rows of bf16 weights, where it is estimated faster than three: 2.2 us + 0.85 + 0.042 M for every 512 values of K
-// (x 1.7 with two tiles a workgroup, x 1.4 behind an RMSNorm) in one round over the CUs, against 8.8 + 0.08 M + 0.2 a megabyte of weights.  The lines this draws, both sides measured: 32
-// rows of 2048 x 2048 11.7 / 13.7, of 1024 x 4096 20.1 / 14.8, of 8192 x 2048 (two tiles) 17.2 / 22.4, of 3072 x 3072 17.7 / 17.2, of 3072 x 2048 behind an
-// RMSNorm 17.4 / 16.2; 2 rows of 2048 x 8192 16.3 / 16.9;
-// 16 rows of 32 x 3072 9.5 / 8.7.  Not where the output overlaps what is read (three launches read the rows before they write) and not behind a LayerNorm
-// (its mean has to be known before the split).
-static bool rows_kc(const mn_skinny_args& a, hipStream_t st) {
+// One launch (rows_kc.inl) for up to 32 rows of bf16 weights, where it is estimated faster than the three launches (`fma` false) or the fp32 FMA kernel of
+// 2 .. 8 rows: 2.5 us + (0.85 + 0.042 M) for every 512 values of K (x 1.7 with two tiles a workgroup, x 1.4 behind an RMSNorm) and round over the CUs, or 0.22 a
+// megabyte of weights, against
+// 8.8 + 0.08 M + 0.2 a megabyte of weights, or 3.2 + 0.19 a megabyte + 0.3 per 1024 of K and as much again a row (8 rows at once; 5 .. 7 as 4 + the rest).  The lines
+// this draws, both sides measured: 32 rows of 2048 x 2048 11.9 / 13.7, of 1024 x 4096 20.1 / 14.8, of 8192 x 2048 (two tiles) 18.8 / 22.4, of 3072 x 3072 17.7 /
+// 17.2, of 3072 x 2048 behind an RMSNorm 17.4 / 16.2; 16 rows of 32 x 3072 9.5 / 8.7; against FMA 2 rows of 2048 x 2048 6.2 / 5.4, of 4096 x 1024 4.6 / 5.3; 4 rows of
+// 2048 x 2048 6.3 / 7.1; 5 rows of it 6.2 / 11.8; 8 rows of 8192 x 2048 11.8 / 22.5; 2 rows of 32000 x 2048 32.0 / 28.2, 3 rows 33.6 / 36.0.  Not where the output overlaps what is read (the other forms read a row
+// before they write it) and not behind a LayerNorm (its mean has to be known before the split).
+static bool rows_kc(const mn_skinny_args& a, bool fma, hipStream_t st) {
   const bool paired = mn_epi_pairs(a.epilogue);
   auto apart = [&](const float* p, int64_t ld) {
     return p + (int64_t)(a.M - 1) * ld + a.K <= a.out || a.out + (int64_t)(a.M - 1) * a.ldo + a.N <= p;
@@ -350,8 +352,11 @@ static bool rows_kc(const mn_skinny_args& a, hipStream_t st) {
   const int64_t tiles = mn_cdiv(a.N, 16);
   const int nt = paired || tiles > mn_num_cus() ? 2 : 1;
   const int64_t g = paired ? tiles : mn_cdiv(a.N, 16 * nt);
-  const double mb = (paired ? 2.0 : 1.0) * a.N * a.K * 2e-6;
-  if (g > mn_num_cus() || 2.2 + mn_cdiv(a.K, 512) * (0.85 + 0.042 * a.M) * (nt == 2 ? 1.7 : 1.0) * (a.prologue == MN_PRO_RMSNORM ? 1.4 : 1.0) >= 8.8 + 0.08 * a.M + 0.2 * mb) return false;
+  const double mb = (paired ? 2.0 : 1.0) * a.N * a.K * 2e-6, kk = a.K / 1024.0;
+  const double here = 2.5 + fmax(0.22 * mb, mn_cdiv(a.K, 512) * (0.85 + 0.042 * a.M) * (nt == 2 ? 1.7 : 1.0) * (a.prologue == MN_PRO_RMSNORM ? 1.4 : 1.0) * mn_cdiv(g, mn_num_cus()));
+  const double row = 0.4 + 0.25 * kk + 0.02 * mb, once = 3.2 + 0.19 * mb + 0.3 * kk;
+  const double there = !fma ? 8.8 + 0.08 * a.M + 0.2 * mb : (a.M > 4 && a.M < 8 ? 2 * once + (a.M - 2) * row : once + (a.M - 1) * row) / 1.15;
+  if (g > (fma ? 4 : 1) * mn_num_cus() || here >= there) return false;
 #define MN_KC(MT_, NT_, P_) hipLaunchKernelGGL((rows_kc_kernel<MT_, NT_, P_>), dim3((unsigned)g), dim3(512), 0, st, a, paired ? 1 : 0)
 #define MN_KC_P(MT_, NT_)                                              \
   do {                                                                 \
@@ -382,7 +387,7 @@ static int skinny_medium(const mn_skinny_args& a, void* stream) {
   bf16_t* Y = reinterpret_cast<bf16_t*>(a.ws);
   float* P = reinterpret_cast<float*>(reinterpret_cast<char*>(a.ws) + (((size_t)2 * a.M * a.K * sizeof(bf16_t) + 255) & ~(size_t)255));
   hipStream_t st = mn_stream(stream);
-  if (!w8 && rows_kc(a, st)) {
+  if (!w8 && rows_kc(a, false, st)) {
     MN_CHECK_LAUNCH("mn_skinny_gemm(rows)");
     return MN_OK;
   }
@@ -436,6 +441,10 @@ extern "C" int mn_skinny_gemm(const mn_skinny_args* args, void* stream) {
   MN_CHECK_ARG(a.epilogue != MN_EPI_RESID_GATE || a.gate, "mn_skinny_gemm: RESID_GATE needs gate");
   MN_CHECK_ARG((((uintptr_t)a.w) & 15) == 0 && ((a.w_batch_stride | a.seg_w_stride) % 8) == 0,
                "mn_skinny_gemm: weights must be 16-byte aligned");
+  if (a.M >= 2 && ka.batch == 1 && ka.nseg == 1 && a.ldw == a.K && rows_kc(a, true, mn_stream(stream))) {
+    MN_CHECK_LAUNCH("mn_skinny_gemm(rows)");
+    return MN_OK;
+  }
   ka.nchunk = (a.K + 511) / 512;
   ka.inv_nchunk = (65536 + ka.nchunk - 1) / ka.nchunk;
   MN_CHECK_ARG((int64_t)ka.nseg * ka.nchunk < 4096 && ka.nseg <= 64, "mn_skinny_gemm: too many K chunks / segments");

@@ -15,7 +15,8 @@ def call(x, ldx, w, out, ldo, M, N, K, ws, **kw):
     from ming_univision_amd._lib import SkinnyArgs, check, current_stream, lib
     a = SkinnyArgs()
     a.x, a.ldx, a.w, a.ldw, a.out, a.ldo, a.M, a.N, a.K = x, ldx, w.data_ptr(), K, out, ldo, M, N, K
-    a.ws, a.ws_bytes = ws.data_ptr(), ws.numel()
+    if ws is not None:
+        a.ws, a.ws_bytes = ws.data_ptr(), ws.numel()
     for k, v in kw.items():
         setattr(a, k, v.data_ptr() if torch.is_tensor(v) else v)
     check(lib().mn_skinny_gemm(C.byref(a), current_stream()), "skinny")
@@ -60,6 +61,26 @@ def test_forms(M, N, K):
         call(xb.data_ptr() + 4, K + 3, w, out.data_ptr(), N + 2, M, N, K, ws, **kw)
         assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
         assert float(((out[:M, :N].double() - y).abs() / (room + 1e-3)).max()) < 2.0 ** -15, (pro, epi)
+
+
+@pytest.mark.parametrize("M,with_ws", [(2, False), (5, False), (8, False), (5, True), (20, True)])
+def test_small_steps_and_infinities(M, with_ws):
+    """2 .. 8 rows without scratch are held to the fp32 kernel's error (2^-24 a step of sums of trees: 1e-7 of the summed magnitudes); an infinite value
+    makes its row's outputs infinite with the weights' signs, two of opposite sign NaN, and no other row sees them."""
+    from ming_univision_amd._lib import lib
+    g = torch.Generator().manual_seed(M)
+    for N, K in ((1024, 1024), (4096, 1032), (100, 520)):
+        w = torch.randn(N, K, generator=g).bfloat16().cuda()
+        x = torch.randn(M, K, generator=g).cuda()
+        ws = torch.empty(lib().mn_skinny_workspace_bytes(M, N, K, 0), dtype=torch.uint8, device="cuda") if with_ws else None
+        out = torch.empty(M, N, device="cuda")
+        call(x.data_ptr(), K, w, out.data_ptr(), N, M, N, K, ws)
+        assert float(((out.double() - x.double() @ w.double().T).abs() / (x.double().abs() @ w.double().abs().T)).max()) < 1e-7
+        x[1, 7] = float("inf")
+        x[0, 3], x[0, K - 1] = float("inf"), -float("inf")
+        call(x.data_ptr(), K, w, out.data_ptr(), N, M, N, K, ws)
+        want = x.double() @ w.double().T
+        assert torch.equal(out[1].double(), want[1]) and bool((torch.isnan(out[0]) == torch.isnan(want[0])).all()) and bool(torch.isfinite(out[2:]).all())
 
 
 def test_output_over_the_input():

@@ -507,7 +507,7 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
   }
 }
 
-// GQA form for many rows: one wave per (row, KV head, split) serves all G = n_q / n_kv query heads of its group, so every
+// GQA form from 8 rows on: one wave per (row, KV head, split) serves all G = n_q / n_kv query heads of its group, so every
 // K / V line is loaded ONCE per group instead of once per query head (the per-head kernel above re-reads them through L1:
 // 4x the load instructions at G = 4).  Same partial layout, same combine kernel.  Block = 4 waves = 4 KV heads of one row.
 template <int HD, int G>
@@ -860,7 +860,9 @@ __global__ __launch_bounds__(1024) void attn_decode_one_kernel(
 
 // Key-range splits (flash-decoding): enough workgroups to fill the chip at few rows, none needed at hundreds of rows;
 // one split never holds more than 4096 keys (its scores live in LDS).
-static bool attn_use_gqa(int M, int n_q, int n_kv, int hd) { return M > 64 && hd == 128 && n_q == 4 * n_kv; }
+// One wave a (row, KV head, split) reads every key once for its four heads; from 8 rows on there are enough of them (a step of 64 rows at 1100 keys 10.8 ->
+// 10.3 ms, 40 rows at 1800 10.5 -> 9.7, 20 rows at 1100 7.53 -> 7.39, 8 rows at 1500 5.26 -> 5.16; 3 rows at 1800 3.80 against 3.90)
+static bool attn_use_gqa(int M, int n_q, int n_kv, int hd) { return M >= 8 && hd == 128 && n_q == 4 * n_kv; }
 // the one-launch form: <= g_one_rows rows whose caches hold <= 1024 keys (dev-library A/B: mn_attn_tune_one)
 static int g_one_rows = 16;
 #ifdef MN_DEV_HOOKS
@@ -951,8 +953,8 @@ extern "C" int mn_attn_decode_split(const float* q, int M, int n_q, int n_kv, in
 
 // Internal (engine.hip): RoPE + q scale + KV append + masked decode attention in ONE split launch (+ the combine) from the raw QKV
 // projection (optionally as nz K-slice partial slabs): what mn_rope_kv_append_3d / mn_rope_kv_from_partials followed by
-// mn_attn_decode_split compute, one launch fewer per layer and step and no q round trip.  Needs row_len == row_slot + 1, at most 64
-// rows (the many-row GQA kernel keeps the separate append) and n_q / n_kv in {1, 2, 4}; mn_attn_fused_ok says whether a shape qualifies.
+// mn_attn_decode_split compute, one launch fewer per layer and step and no q round trip.  Needs row_len == row_slot + 1, the
+// one-launch form or one row, and n_q / n_kv in {1, 2, 4}; mn_attn_fused_ok says whether a shape qualifies.
 // Where the append rides the attention launch (tools/exp/attn_fused_ab.py, profiles/r04_attn_fused_ab.txt): always in the one-launch form
 // (every row count it serves gains 1-2 %: each workgroup keeps the new key in LDS, no hazard, no redundant reads worth counting); in
 // the split form at ONE row only (2.00 -> 1.92 ms per 28-layer step; from 2 rows on every split re-reduces the QKV slabs: 2.59 -> 2.74).
@@ -964,7 +966,7 @@ extern "C" int mn_attn_fused_ok(int M, int n_q, int n_kv, int hd, int64_t t_max)
   if (g_kv_round_bf16 || !g_attn_fuse) return 0;     // the bf16-KV measurement hook lives in the stand-alone append kernel
   if (!attn_use_one(M, t_max) && M > 1) return 0;
   const int ratio = n_kv > 0 && n_q % n_kv == 0 ? n_q / n_kv : 0;
-  return M >= 1 && !attn_use_gqa(M, n_q, n_kv, hd) && (hd == 64 || hd == 128) && (ratio == 1 || ratio == 2 || ratio == 4);
+  return M >= 1 && (hd == 64 || hd == 128) && (ratio == 1 || ratio == 2 || ratio == 4);
 }
 extern "C" int mn_attn_decode_fused(const float* qkv, int64_t ldqkv, int nz, int64_t slab, int M, int n_q, int n_kv, int hd, int rope,
                                     const float* cos_tab, const float* sin_tab, const int32_t* row_seq, const int32_t* row_slot,

@@ -443,7 +443,7 @@ extern "C" MN_DEV_API void mn_gemm256_tune_order(int group_m, int group_list) { 
 // with the constants measured on MI355X (weights cycling through HBM, graph of 48 launches; us): a workgroup alone on its CU needs `alone` per
 // K-tile, rising to `full` when every CU holds one and to `two` when every CU holds two (forms that fit twice); beyond that `per` for each
 // workgroup of a CU, or whole rounds of `full` (forms that fit once: per = 0).  The fixed part is launch, first round trip and epilogue: 4 us
-// for the small tiles, + 3 per further round of the form that fits once, 11 us + 7 per further round for the 256-tile kernel.
+// for the small tiles, 11 us + 7 per further round for the 256-tile kernel.
 // Where the lines then lie, both sides measured: 65 x 3072 x 1024 bf16: 7.3 us (64 x 64) against 23.7 (256); 256 x 4096 x 1024: 8.2 against
 // 32.1; 1025 hi/lo rows x 1024 x 1024: 12.4 against 25.0; x 3072: 20.5 (128 x 128) against 27.5; 2048 x 2048 x 8192: 79.6 (128 x 128) against 136.6;
 // 16384 x 1024 x 1024: 37.2 (256) against 54.2 (128 x 128); 1025 hi/lo rows x 2752 SwiGLU: 29.9 (256) against 37.8.
@@ -461,7 +461,7 @@ static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bo
   else if (f.per == 0) per_tile = f.full * rounds;
   else if (w <= 2.0) per_tile = f.full + (f.two - f.full) * (w - 1.0);
   else per_tile = f.per * w > f.two ? f.per * w : f.two;
-  return f.fixed + (f.per == 0 ? (f.form == 0 ? 7.0 : 3.0) * (rounds - 1.0) : 0.0) + k_tiles * per_tile;
+  return f.fixed + (f.form == 0 ? 7.0 * (rounds - 1.0) : 0.0) + k_tiles * per_tile;
 }
 
 // the form of a dense M x N x K launch in nz K-slices of Kc, and the estimate of its time

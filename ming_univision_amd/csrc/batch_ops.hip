@@ -247,13 +247,14 @@ extern "C" int mn_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, i
   // 65 x 3072 x 1024 bf16 7.3 us against 23.6 on the 128 x 128 tiles below, 2048 x 2048 x 14336 140 against 220); anything else stays
   // on the 128-tile kernel with its scalar epilogue (gemm256's stores 4 consecutive columns per lane and loads the bias 8 bytes at a time)
   const bool f32_out = epilogue == MN_GEMM_F32 || epilogue == MN_GEMM_F32_RESID;
-  if (g_gemm_route256 && (K % 64) == 0 && (N % 4) == 0 &&
+  // gemm256 addresses its operands with 32-bit byte offsets: an activation matrix beyond 4 GiB goes in chunks of 256 rows and more; rows so far
+  // apart that fewer fit (one token of each of a batch of long sequences) stay on the 128-tile kernel's 64-bit addresses
+  int64_t chunk = lda > 0 ? ((((int64_t)1 << 31) - 1 - K) / lda + 1) : (lda == 0 ? M : 0);
+  chunk = chunk >= M ? M : chunk / 256 * 256;
+  if (g_gemm_route256 && (K % 64) == 0 && (N % 4) == 0 && chunk > 0 && ldw >= 0 &&
       (int64_t)N * ldw * 2 < ((int64_t)1 << 32) && epilogue >= MN_GEMM_BF16 && epilogue <= MN_GEMM_F32_RESID &&
       (ldc % 4) == 0 && ((uintptr_t)C & (f32_out ? 15 : 7)) == 0 && ((uintptr_t)bias & 7) == 0) {
     static const int map[4] = {MN_G256_BF16, MN_G256_BF16_GELU, MN_G256_F32, MN_G256_F32_RESID};
-    // gemm256 addresses its operands with 32-bit byte offsets: an activation matrix beyond 4 GiB goes in row chunks
-    int64_t chunk = ((((int64_t)1 << 32) - 1) / (lda * 2)) / 256 * 256;
-    if (chunk >= M) chunk = M;
     const int64_t c_elt = (epilogue == MN_GEMM_F32 || epilogue == MN_GEMM_F32_RESID) ? 4 : 2;
     for (int64_t m0 = 0; m0 < M; m0 += chunk) {
       mn_g256 a;

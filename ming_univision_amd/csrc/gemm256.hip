@@ -609,7 +609,7 @@ static bool g256_shape_ok(const void* A, int64_t lda, int64_t a_lo_off, const vo
                           int K) {
   // whole K-tiles; 16-byte aligned rows; every per-lane source offset fits 32 bits; 4 output columns per lane
   return M >= 1 && N >= 4 && (N % 4) == 0 && K >= BK && (K % BK) == 0 && (lda % 8) == 0 && (ldw % 8) == 0 && (a_lo_off % 8) == 0 &&
-         (((uintptr_t)A | (uintptr_t)W) & 15) == 0 && ((int64_t)M * lda + a_lo_off) * 2 < ((int64_t)1 << 32) &&
+         lda >= 0 && ldw >= 0 && a_lo_off >= 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0 && ((int64_t)M * lda + a_lo_off) * 2 < ((int64_t)1 << 32) &&
          w_rows * ldw * 2 < ((int64_t)1 << 32);
 }
 

@@ -118,3 +118,17 @@ def test_lightning_scan(T, H, d, e):
                 assert float((out[t].double().cpu() - ref).abs().max() / ref.abs().max()) < 1e-5, t
         assert rel(state[seq], S) < 1e-5
         r += n
+
+
+@pytest.mark.parametrize("M,lda", [(3, 0), (300, 0), (3, 1 << 23), (130, 1 << 24), (600, 1 << 22)])
+def test_rows_far_apart(M, lda):
+    """One row for all (stride 0), one token of each sequence of a long batch, rows of which fewer than M and than 256 fit under 4 GiB, chunks of 256 rows and more."""
+    from ming_univision_amd import ops
+    N, K = 132, 192
+    g = torch.Generator(device="cuda").manual_seed(M)
+    buf = torch.empty((M - 1) * lda + K, dtype=torch.bfloat16, device="cuda")
+    a = buf.as_strided((M, K), (lda, 1))
+    (a if lda else buf).copy_(torch.randn(*((M, K) if lda else (K,)), generator=g, device="cuda"))
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    ref = a.double() @ w.double().T
+    assert rel(ops.gemm_bf16(a, w, None, "f32"), ref) < 3e-5 and rel(ops.gemm_bf16(a, w, None, "bf16"), ref) < 2 ** -8

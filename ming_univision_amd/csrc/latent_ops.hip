@@ -642,39 +642,40 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
   using Walk = LatentWalk<NB, KF, VEC, PlainScore>;
   __shared__ __attribute__((aligned(16))) float lds[Walk::LDS_FLOATS];
   const int row0 = blk_tab[2 * blockIdx.x], nrows = blk_tab[2 * blockIdx.x + 1];
-  const int nqv = nrows * H, qv0 = blockIdx.y * 16;
-  if (qv0 >= nqv) return;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
-  const int64_t seq = row_seq[row0];
-  const int len = row_len[row0 + nrows - 1];
-  const bool on = qv0 + c < nqv;
-  const int qv = on ? qv0 + c : nqv - 1;
-  const int64_t o = (int64_t)(row0 + qv / H) * H + qv % H;
-  f32x4 q[NB], acc[NB];
+  const int nqv = nrows * H, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
+  // (one pass unless the grid was cut for runs of one row and this one is longer)
+  for (int qv0 = blockIdx.y * 16; qv0 < nqv; qv0 += 16 * gridDim.y) {
+    const int64_t seq = row_seq[row0];
+    const int len = row_len[row0 + nrows - 1];
+    const bool on = qv0 + c < nqv;
+    const int qv = on ? qv0 + c : nqv - 1;
+    const int64_t o = (int64_t)(row0 + qv / H) * H + qv % H;
+    f32x4 q[NB], acc[NB];
 #pragma unroll
-  for (int it = 0; it < NB; ++it) q[it] = load4<VEC>(qabs + o * r, wave * 16 * NB + 16 * it + 4 * g4, r, on);
-  const int n_tiles = (len + Walk::KT - 1) / Walk::KT;
-  const int t0 = blockIdx.z * tiles_per_split, t1 = min(t0 + tiles_per_split, n_tiles);
-  float mrun, lrun;
-  Walk::run(lds, arena + seq * t_max * r, r, r, len, on ? row_len[row0 + qv / H] : len, t0, t1, q, PlainScore{}, mrun, lrun, acc);
-  if (!on) return;
-  const float inv = KS == 1 ? 1.0f / lrun : 1.0f;
-  float* dst = KS == 1 ? lat + o * r : part_acc + ((int64_t)blockIdx.z * M * H + o) * r;
+    for (int it = 0; it < NB; ++it) q[it] = load4<VEC>(qabs + o * r, wave * 16 * NB + 16 * it + 4 * g4, r, on);
+    const int n_tiles = (len + Walk::KT - 1) / Walk::KT;
+    const int t0 = blockIdx.z * tiles_per_split, t1 = min(t0 + tiles_per_split, n_tiles);
+    float mrun, lrun;
+    Walk::run(lds, arena + seq * t_max * r, r, r, len, on ? row_len[row0 + qv / H] : len, t0, t1, q, PlainScore{}, mrun, lrun, acc);
+    if (!on) continue;
+    const float inv = KS == 1 ? 1.0f / lrun : 1.0f;
+    float* dst = KS == 1 ? lat + o * r : part_acc + ((int64_t)blockIdx.z * M * H + o) * r;
 #pragma unroll
-  for (int x = 0; x < NB; ++x) {
-    const int d = 16 * (wave + 4 * x) + 4 * g4;
-    if (VEC) {
-      if (d < r) *reinterpret_cast<f32x4u*>(dst + d) = acc[x] * inv;
-    } else {
+    for (int x = 0; x < NB; ++x) {
+      const int d = 16 * (wave + 4 * x) + 4 * g4;
+      if (VEC) {
+        if (d < r) *reinterpret_cast<f32x4u*>(dst + d) = acc[x] * inv;
+      } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (d + e < r) dst[d + e] = acc[x][e] * inv;
+        for (int e = 0; e < 4; ++e)
+          if (d + e < r) dst[d + e] = acc[x][e] * inv;
+      }
     }
-  }
-  if (KS > 1 && wave == 0 && g4 == 0) {
-    const int64_t po = (int64_t)blockIdx.z * M * H + o;
-    part_ml[po * 2] = mrun;
-    part_ml[po * 2 + 1] = lrun;
+    if (KS > 1 && wave == 0 && g4 == 0) {
+      const int64_t po = (int64_t)blockIdx.z * M * H + o;
+      part_ml[po * 2] = mrun;
+      part_ml[po * 2 + 1] = lrun;
+    }
   }
 }
 
@@ -869,7 +870,8 @@ extern "C" int mn_latent_attn_ex(const float* qabs, const float* arena, const in
   hipStream_t st = mn_stream(stream);
   if (variant == MN_LATENT_ATTN_MFMA) {
     const int nbw = (int)mn_cdiv(r, 64);
-    // as many runs as rows: one row each (workgroups for the rows a run does not have still wait for their LDS: 3 of 4 in a decode step)
+    // as many runs as rows: one row each, or longer ones beside empty ones, whose workgroups go round again (workgroups for the rows a run does not have
+    // still wait for their LDS: 3 of 4 in a decode step)
     const dim3 grid((unsigned)n_blk, (unsigned)mn_cdiv((n_blk == M ? 1 : RB) * H, 16), (unsigned)ks);
     MN_CHECK_ARG(mn_cdiv(RB * H, 16) <= 65535 && ks <= 64, "mn_latent_attn: too many heads or key splits");
 #define MN_LM(N_, F_, V_)                                                                                                           \

@@ -108,3 +108,20 @@ def test_decode_rows_over_latents(n, H, r, e):
                                                 t_max, 1, window, 0, 1.0, ptr(out), H * e, None, 0, ns, ptr(ws), ws.numel(), -1, current_stream()), "attn")
         ref = want(e, window, cap).reshape(3, -1)
         assert bool((out[3] == 7.0).all()) and float((out[:3].double().cpu() - ref).abs().max() / ref.abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("H,r,ks", [(16, 64, 1), (5, 256, 3), (20, 512, 1), (33, 35, 2)])
+def test_as_many_runs_as_rows_of_uneven_length(H, r, ks):
+    """Runs of three and two rows beside empty ones: the launch is cut for runs of one row."""
+    from ming_univision_amd._lib import check, current_stream, lib, ptr
+    L = lib()
+    g = torch.Generator().manual_seed(H + r)
+    k, q = torch.randn(2, 48, r, generator=g), torch.randn(5, H * r, generator=g) * r ** -0.5
+    seq, ln = torch.tensor([0, 0, 0, 1, 1], dtype=torch.int32), torch.tensor([38, 39, 40, 1, 2], dtype=torch.int32)
+    blk = torch.tensor([[0, 3], [0, 0], [3, 2], [0, 0], [0, 0]], dtype=torch.int32)
+    kd, qd, sd, ld, bd = k.cuda(), q.cuda(), seq.cuda(), ln.cuda(), blk.cuda()
+    lat = torch.full((6, H, r), 7.0, device="cuda")
+    ws = torch.empty(max(16, L.mn_latent_attn_workspace_bytes(5, H, r, ks)), dtype=torch.uint8, device="cuda")
+    check(L.mn_latent_attn(ptr(qd), ptr(kd), ptr(sd), ptr(ld), ptr(bd), 5, 5, H, r, 48, 40, ks, ptr(lat), ptr(ws), ws.numel(), current_stream()), "latent")
+    ref = torch.stack([torch.softmax(q[m].reshape(H, r).double() @ k[seq[m], :ln[m]].double().T, -1) @ k[seq[m], :ln[m]].double() for m in range(5)])
+    assert bool((lat[5] == 7.0).all()) and float((lat[:5].double().cpu() - ref).abs().max() / ref.abs().max()) < 1e-5

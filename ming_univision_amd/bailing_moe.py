@@ -601,7 +601,11 @@ class BailingMoeDecoder:
         if hidden.shape[0] > 8 and self.lm_head.data_ptr() % 16 == 0 and lib().mn_gemm256_supported(
                 hidden.shape[1], 8, self.lm_head.stride(0), self.lm_head.shape[0], hidden.shape[0], self.lm_head.shape[0], hidden.shape[1]):
             # one pass over the vocabulary matrix (the 8-row chunks below read it once each) on the same hi/lo operands
-            return ops.gemm256(ops.split_hilo(hidden.contiguous()), self.lm_head, None, "f32")
+            hidden = hidden.contiguous()
+            out = ops.gemm256(ops.split_hilo(hidden), self.lm_head, None, "f32")
+            if hidden.shape[0] <= MAX_ROWS and hidden.shape[0] % 8 == 1:
+                ops.skinny_gemm(hidden[-1:], self.lm_head, out=out[-1:])      # the row that is a chunk of its own below: fp32 products
+            return out
         outs = [ops.skinny_gemm(hidden[i:i + 8].contiguous(), self.lm_head) for i in range(0, hidden.shape[0], 8)]
         return torch.cat(outs, 0)
 

@@ -98,3 +98,18 @@ def test_output_over_the_input():
         got = torch.stack([flat[i * ld + at:i * ld + at + N] for i in range(M)]).double()
         want = x @ w.double().T
         assert float((got - want).abs().max() / want.abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("M", [9, 17, 57, 16, 65])
+def test_logits_of_a_row_by_itself(M):
+    """One row more than whole chunks of eight (up to 64 rows): that row's logits are fp32 products (1e-7 of the summed magnitudes, as above), the others hi / lo."""
+    from ming_univision_amd import configuration as cfgs
+    from ming_univision_amd.bailing_moe import BailingMoeDecoder
+    cfg = cfgs.BailingMoeConfig(vocab_size=512, hidden_size=256, num_hidden_layers=1, num_attention_heads=4, num_key_value_heads=2, head_dim=128, use_bias=False,
+                                rope_theta=600000.0, num_experts=8, num_shared_experts=2, num_experts_per_tok=3, moe_intermediate_size=64, multi_gate=True,
+                                num_image_tokens_for_gen=16, image_start_token=500)
+    dec = BailingMoeDecoder.synthetic(cfg, "cuda", seed=1, t_max=16, n_seq=1)
+    h = torch.randn(M, 256, generator=torch.Generator().manual_seed(M)).cuda()
+    want, mag = h.double() @ dec.lm_head.double().T, h.double().abs() @ dec.lm_head.double().abs().T
+    off = (dec.logits(h).double() - want).abs() / mag
+    assert float(off.max()) < 2.0 ** -16 and (M % 8 != 1 or M > 64 or float(off[-1].max()) < 1e-7)

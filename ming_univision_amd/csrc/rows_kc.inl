@@ -3,7 +3,8 @@
 // The three-launch form (split the rows into hi / lo, stream the weights in K-slices, sum the slices) pays 4 .. 6 us for each of its small launches; at
 // the sizes of a decoder's projections that is more than the product.  Here a workgroup owns NT tiles of 16 columns with ALL of K: its 8 waves take
 // 64-value chunks of K in turn, read weights and fp32 rows straight into MFMA operands (lane l: row / column l & 15, values 8 (l >> 4) .. + 7
-// of every 32), split the rows there into three bf16 parts (24 bits: products of all of an fp32 value) and meet once, in LDS, for the sum of the eight
+// of every 32), split the rows there into three bf16 parts (24 bits: products of all of an fp32 value of 2^-110 and more; the last bits of
+// smaller ones fall off bf16's subnormals: 1e-7 of the summed magnitudes at rows around 2^-114, 2e-6 at 2^-118) and meet once, in LDS, for the sum of the eight
 // waves' tiles and the epilogue.  A chunk's sum joins the running one with its rounding kept (two-sum): 1.5e-8 of the summed magnitudes off 64 bits at
 // the most, 2.0e-8 on the fp32 FMA kernel, 4e-7 as hi + lo.  Every workgroup reads all rows (M K 4 bytes, from L2), every weight byte is read once; the
 // next chunk's loads are in flight during a chunk's products.  What bounds it is the load and conversion of the rows (0.85 us + 0.042 a row for each 512
@@ -14,10 +15,13 @@
 typedef short bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));      // rows start at any float: a 16-byte load needs 4-byte alignment here
 
-// a pair of values as three pairs of bf16, 24 bits: all of an fp32 value (ODD: of a value that may be infinite; what is left of it is nothing, not inf - inf)
+// a pair of values as three pairs of bf16, 24 bits.  ODD: of values that bf16 rounds to infinity; a finite one starts from the largest finite
+// bf16, what is left of an infinite one is nothing (not inf - inf).
+constexpr float BF16_TO_INF = 0x1.ffp127f, BF16_MAX = 0x1.fep127f;
 template <bool ODD>
 __device__ __forceinline__ void split3_pk_bf16(float a, float b, u32x4 (&part)[3], int at) {
-  uint32_t h = cvt_pk_bf16(a, b);
+  uint32_t h = ODD ? cvt_pk_bf16(fabsf(a) < INFINITY ? fminf(fmaxf(a, -BF16_MAX), BF16_MAX) : a, fabsf(b) < INFINITY ? fminf(fmaxf(b, -BF16_MAX), BF16_MAX) : b)
+                   : cvt_pk_bf16(a, b);
   part[0][at] = h;
   a -= bf16lo_to_f32(h); b -= bf16hi_to_f32(h);
   if (ODD) { a = a == a ? a : 0.f; b = b == b ? b : 0.f; }
@@ -116,7 +120,7 @@ __global__ __launch_bounds__(512) void rows_kc_kernel(const mn_skinny_args a, in
         float most = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) most = fmaxf(most, fmaxf(fabsf(v0[e]), fabsf(v1[e])));
-        if (__ballot(most == INFINITY) == 0) {
+        if (__ballot(most >= BF16_TO_INF) == 0) {
 #pragma unroll
           for (int e = 0; e < 2; ++e) { split3_pk_bf16<false>(v0[2 * e], v0[2 * e + 1], part, e); split3_pk_bf16<false>(v1[2 * e], v1[2 * e + 1], part, 2 + e); }
         } else {

@@ -83,6 +83,27 @@ def test_small_steps_and_infinities(M, with_ws):
         assert torch.equal(out[1].double(), want[1]) and bool((torch.isnan(out[0]) == torch.isnan(want[0])).all()) and bool(torch.isfinite(out[2:]).all())
 
 
+@pytest.mark.parametrize("M,with_ws", [(2, False), (8, False), (5, True), (20, True)])
+def test_range_of_fp32(M, with_ws):
+    """Finite values that bf16 rounds to infinity, and tiny ones: products of all their bits (1e-7 of the summed magnitudes) from 2^-100 on."""
+    from ming_univision_amd._lib import lib
+    g = torch.Generator().manual_seed(M)
+    N, K = 1024, 1024
+    w = torch.randn(N, K, generator=g).bfloat16().cuda()
+    x = torch.randn(M, K, generator=g)
+    x[0], x[1] = 0.0, x[1] * 2.0 ** -98
+    x[0, 3], x[0, K - 1] = 3.4e38, -3.3999e38
+    x = x.cuda()
+    w[:, K - 1] = (w[:, 3].float() * 0.5).bfloat16()              # (sums stay finite)
+    w[:, 3] = w[:, 3].clamp(-0.75, 0.75)
+    w[:, K - 1] = w[:, K - 1].clamp(-0.125, 0.125)
+    ws = torch.empty(lib().mn_skinny_workspace_bytes(M, N, K, 0), dtype=torch.uint8, device="cuda") if with_ws else None
+    out = torch.empty(M, N, device="cuda")
+    call(x.data_ptr(), K, w, out.data_ptr(), N, M, N, K, ws)
+    off = (out.double() - x.double() @ w.double().T).abs() / (x.double().abs() @ w.double().abs().T)
+    assert float(off.max()) < 1e-7
+
+
 def test_output_over_the_input():
     """The rows are all read before any is written: out = x, and out between the rows of x."""
     from ming_univision_amd._lib import lib

@@ -30,6 +30,29 @@ __device__ __forceinline__ void rows_table(const AttnTArgs& a, int b0, int nb, i
   __syncthreads();
 }
 
+// An infinite or NaN value at a key that a query does not see would meet its weight 0 there and turn into NaN (the rows of a workgroup share the walk).  So
+// such values stay out of the tiles, one product by zero a value says whether there are any, and a workgroup that met some looks its keys
+// over again behind the walk: every query then takes them as they are from the keys it sees.  (It costs 0 .. 2.5 % of either kernel: 16 heads of 256 375 -> 384 us,
+// of 128 as before; keys of 576 744 -> 761.)
+template <int NF, int NB>
+__device__ __forceinline__ void finite_only(f32x4 (&v)[NF][NB], int& met) {
+  float z[2] = {0.f, 0.f};
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int x = 0; x < NB; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z[e & 1] = fmaf(v[f][x][e], 0.f, z[e & 1]);
+  if (__ballot(z[0] + z[1] != 0.f) == 0) return;
+  met = 1;
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int x = 0; x < NB; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[f][x][e] = fabsf(v[f][x][e]) < INFINITY ? v[f][x][e] : 0.f;
+}
+
 // values d .. d + 3 of one query vector's result
 __device__ __forceinline__ void emit4(const AttnTArgs& a, f32x4 v, int row, int64_t col0, int d, bool vec) {
 #pragma unroll
@@ -62,9 +85,10 @@ template <int NBD, int NBV, bool VEC>
 __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_blk, int hv) {
   constexpr int KT = NBD + NBV > 4 ? 16 : 32, KF = KT / 16, AQ = 16, LDK = 64 * NBD + 4, LDV = 64 * NBV + 4, TILE = KT * (LDK + LDV);
   __shared__ __attribute__((aligned(16))) float lds[2 * TILE];        // [2][K tile | V tile]
-  __shared__ int tab[16][4];
+  __shared__ int tab[16][4], met;                      // met: an infinite or NaN value
   const int tid = threadIdx.x, gy = blockIdx.y, sp = blockIdx.z;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, g4 = lane >> 4;
+  if (tid == 0) met = 0;
   const int rep = a.H / a.G, chunks = (rep + a.hpc - 1) / a.hpc;
   const int g = gy / chunks, h0 = g * rep + (gy % chunks) * a.hpc;
   const int Rc = min(a.hpc, g * rep + rep - h0);
@@ -121,6 +145,7 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_bl
     };
     auto put = [&](int tile, int buf) {
       float* K = lds + buf * TILE;
+      finite_only(vv, met);
 #pragma unroll
       for (int f = 0; f < KF; ++f) {
         const bool ok = tile * KT + 16 * f + fj < nk;
@@ -230,6 +255,26 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_bl
             if (d + e < a.vdim) part[2 * AQ + (int64_t)qv * a.vdim + d + e] = r[e];
         }
       if (part && g4 == 0) { part[qv] = mrun; part[AQ + qv] = lrun; }
+      if (met) {
+#pragma unroll 1
+        for (int x = 0; x < 16 * NBV; ++x) {           // this lane's columns again: what is not finite among the seen keys' values
+          const int d = 64 * (x >> 4) + 16 * g4 + (x & 15);
+          if (d >= a.vdim) continue;
+          float odd = 0.f;
+#pragma unroll 1
+          for (int j = t0 * KT; j < min(nk, t1 * KT); ++j) {
+            const float v = (j < nbL ? pvb + (int64_t)j * Gv : vb_ + (int64_t)(j - nbL) * a.ldv)[d];
+            const bool see = ((j < nbL) & (j < my_nb)) | ((j >= lo) & (j <= hi));
+            odd += see && !(fabsf(v) < INFINITY) ? v : 0.f;
+          }
+          if (odd == 0.f) continue;
+          odd *= inv;
+          if (part) { part[2 * AQ + (int64_t)qv * a.vdim + d] = odd; continue; }
+          odd = gated(a, odd, row, col0 + d);
+          if (a.out) a.out[(int64_t)row * a.ldo + col0 + d] = odd;
+          if (a.out16) a.out16[(int64_t)row * a.ldo16 + col0 + d] = f32_to_bf16(odd);
+        }
+      }
     }
     s0 = s1;
   }
@@ -240,15 +285,16 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_bl
 // values, a quarter of the columns.  The four partial score tiles meet in LDS, each wave sums them and takes the same softmax: 144 MFMAs of
 // 32 cycles per wave and 16-key tile at 576 + 512 values stand against three barriers, and two or three workgroups share a CU.  (64 vectors
 // at 512 registers and one wave per SIMD: 1450 us on the case below, nothing covers the barriers and 129 registers spill.)
-// 2048 tokens, 16 heads, keys of 576 and values of 512, window 1024 (54.8 GF): 1674 us in the form before, 746 us here.
+// 2048 tokens, 16 heads, keys of 576 and values of 512, window 1024 (54.8 GF): 1674 us in the form before, 761 us here.
 template <int NB, bool VEC>
 __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, int n_blk, int hv) {
   constexpr int KT = 16, AQ = 16, QF = 2, LDK = 64 * NB + 4, LDS_S = 20;
   __shared__ __attribute__((aligned(16))) float K[KT * LDK];
   __shared__ __attribute__((aligned(16))) float Sp[4][16 * QF * LDS_S];     // [wave][query][16 keys]: partial scores
-  __shared__ int tab[16][4];
+  __shared__ int tab[16][4], met;
   const int tid = threadIdx.x, gy = blockIdx.y, sp = blockIdx.z;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, g4 = lane >> 4;
+  if (tid == 0) met = 0;
   const int rep = a.H / a.G, h0 = gy * a.hpc;
   const int Rc = min(a.hpc, rep - h0);
   const int rf = 16 / hv, nbw = rf * QF / a.rows_per_blk;               // rows per 16-vector fragment; runs per workgroup
@@ -290,10 +336,10 @@ __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, i
     for (int o = 1; o < 16; o <<= 1) { lo_all = max(lo_all, __shfl_xor(lo_all, o)); hi_all = min(hi_all, __shfl_xor(hi_all, o)); }
     lo_all = __builtin_amdgcn_readfirstlane(lo_all); hi_all = __builtin_amdgcn_readfirstlane(hi_all);
     const float* kb = a.k + ((int64_t)seq * a.t_max + tF) * a.ldk;
-    f32x4 vk[NB];
+    f32x4 vk[1][NB];
     const int fj = tid >> 4, fc = tid & 15;
-    auto fetch = [&](int tile) { rows_fetch<NB, VEC>(vk, kb + (int64_t)min(tile * KT + fj, nk - 1) * a.ldk, a.dim, fc); };
-    auto put = [&](int tile) { rows_put<NB, LDK, VEC>(K, vk, a.dim, fj, fc, tile * KT + fj < nk); };
+    auto fetch = [&](int tile) { rows_fetch<NB, VEC>(vk[0], kb + (int64_t)min(tile * KT + fj, nk - 1) * a.ldk, a.dim, fc); };
+    auto put = [&](int tile) { rows_put<NB, LDK, VEC>(K, vk[0], a.dim, fj, fc, tile * KT + fj < nk); };
     float mrun[QF], lrun[QF];
     f32x4 acc[QF][NB];
 #pragma unroll
@@ -306,6 +352,7 @@ __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, i
     if (t0 < t1) fetch(t0);
     for (int tile = t0; tile < t1; ++tile) {
       const int key0 = tile * KT;
+      finite_only(vk, met);
       lds_barrier();                                   // the previous tile's values and partial scores are read
       put(tile);
       if (tile + 1 < t1) fetch(tile + 1);              // in flight while this tile is multiplied
@@ -373,6 +420,17 @@ __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, i
 #pragma unroll
           for (int f = 0; f < QF; ++f) acc[f][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[x], p[f][i], acc[f][x], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);             // (all four steps' reads at once would not fit the registers)
+      }
+    }
+    if (met) {                                         // a key that is not finite has no finite score either: nothing of a row that sees it is known
+#pragma unroll 1
+      for (int j = t0 * KT; j < min(nk, t1 * KT); ++j) {
+        bool odd = false;
+#pragma unroll 1
+        for (int d = lane; d < a.dim; d += 64) odd |= !(fabsf(kb[(int64_t)j * a.ldk + d]) < INFINITY);
+        if (__ballot(odd) == 0) continue;
+#pragma unroll
+        for (int f = 0; f < QF; ++f) lrun[f] = j >= lo[f] && j <= hi[f] ? NAN : lrun[f];
       }
     }
     const bool vec = emit_vec(a);

@@ -61,6 +61,54 @@ def test_values_inside_keys(spans, H, d, e):
         run(spans, H, 1, d, e, window, cap, chunk, True, ns, 256)
 
 
+@pytest.mark.parametrize("vk", [False, True])
+@pytest.mark.parametrize("H,G,d,e", [(8, 2, 128, 128), (4, 4, 64, 64), (6, 3, 72, 136), (3, 1, 200, 256), (5, 1, 34, 33), (16, 1, 576, 512)])
+def test_values_that_are_not_finite(H, G, d, e, vk):
+    """An infinite value at one key and a NaN at a later one: no row sees them before their keys or after they have left its window, every row between has
+    them in their columns and the other columns as they are (values inside the keys: the scores are not
+    finite either, and nothing of a row that sees the NaN is)."""
+    from ming_univision_amd._lib import check, current_stream, lib, ptr
+    from ming_univision_amd.sequences import rows_of_spans
+    if vk:
+        G, e = 1, min(d, e)
+    elif d > 256:
+        return
+    L = lib()
+    T, at, nan_at = 90, 37, 40
+    g = torch.Generator().manual_seed(H + d)
+    tabs = rows_of_spans([(0, T, 0)], L.mn_window_attn_block_rows())
+    dev = {x: torch.from_numpy(np.ascontiguousarray(y)).cuda() for x, y in tabs.items() if x != "max_len"}
+    q, k = torch.randn(T, H * d, generator=g) * d ** -0.5, torch.randn(T, G, d, generator=g)
+    v = k[..., :e] if vk else torch.randn(T, G, e, generator=g)
+    qd, kd = q.cuda(), k.cuda()
+    vd = kd if vk else v.cuda()
+    vd[at, :, 1], vd[nan_at, :, 3] = float("inf"), float("nan")
+    n_blk = dev["blk_tab"].shape[0]
+    for window, ns in ((0, 1), (20, 1), (0, 3)):
+        ws = torch.empty(max(16, L.mn_window_attn_workspace_bytes(n_blk, H, G, e, 0, ns)), dtype=torch.uint8, device="cuda")
+        out = torch.empty(T, H * e, device="cuda")
+        check(L.mn_window_pool_attn_blocks_gate(ptr(qd), H * d, ptr(kd), G * d, ptr(vd), G * (d if vk else e), None, None, None, 0.0, 0, None, 0, ptr(dev["row_seq"]),
+                                                ptr(dev["row_slot"]), ptr(dev["blk_tab"]), n_blk, 0, H, G, d, e, T, 1, window, 0, 1.0, ptr(out), H * e,
+                                                None, 0, ns, ptr(ws), ws.numel(), -1, current_stream()), "attn")
+        got = out.view(T, H, e).cpu().double()
+        i, j = torch.arange(T)[:, None], torch.arange(T)[None]
+        see = (j <= i) & ((i - j < window) if window else True)
+        for h in range(H):
+            c = h // (H // G)
+            p = torch.softmax((q.view(T, H, d)[:, h].double() @ k[:, c].double().T).masked_fill(~see, -float("inf")), -1)
+            mine, ref = got[:, h], p @ v[:, c].double()
+            if vk:
+                hit = see[:, at] | see[:, nan_at]
+                fin = torch.isfinite(mine)
+                assert not bool(fin[see[:, nan_at]].any()) and not bool(fin[hit, 1].any()) and bool(fin[~hit].all())
+                mine, ref = mine[~hit], ref[~hit]
+            else:
+                for col, key, odd in ((1, at, torch.isposinf), (3, nan_at, torch.isnan)):
+                    assert torch.equal(odd(mine[:, col]), see[:, key]), (h, col)
+                    ref[see[:, key], col], mine[see[:, key], col] = 0.0, 0.0
+            assert float((mine - ref).abs().max() / ref.abs().max()) < 1e-5
+
+
 def test_three_splits_of_many_groups():
     """More than 256 workgroups in a head and split: every group exactly once whatever the launch order."""
     run([(0, 700, 0), (1, 700, 0), (2, 700, 0)], 5, 1, 16, 16, 0, 0.0, 0, False, 3, 704)

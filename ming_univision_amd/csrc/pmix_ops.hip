@@ -54,7 +54,7 @@ __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x));
 
 // ---------------------------------------------------------------------------------------------------------------------------
 // one wave per row: x += mult * y, then RMS norm with a weight
-__global__ __launch_bounds__(256) void axpy_rms_kernel(float* __restrict__ x, int64_t ldx, const float* __restrict__ y, int64_t ldy,
+__global__ __launch_bounds__(256) void axpy_rms_kernel(float* __restrict__ x, int64_t ldx, const float* __restrict__ y, int64_t ldy, int nz, int64_t zs,
                                                        float mult, const bf16_t* __restrict__ w, float eps, float* __restrict__ nout,
                                                        int64_t ldn, bf16_t* __restrict__ n16, int64_t ldn16, int M, int n) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -63,7 +63,12 @@ __global__ __launch_bounds__(256) void axpy_rms_kernel(float* __restrict__ x, in
   float s = 0.f;
   for (int i = lane; i < n; i += 64) {
     float v = xr[i];
-    if (y) { v += mult * y[(int64_t)row * ldy + i]; xr[i] = v; }
+    if (y) {
+      float t = y[(int64_t)row * ldy + i];
+      for (int z = 1; z < nz; ++z) t += y[(int64_t)row * ldy + i + z * zs];
+      v += mult * t;
+      xr[i] = v;
+    }
     s += v * v;
   }
   if (!nout && !n16) return;
@@ -977,20 +982,20 @@ extern "C" int mn_axpy_rms_rows(float* x, int64_t ldx, const float* y, int64_t l
   return mn_axpy_rms_rows_slabs(x, ldx, y, ldy, 1, 0, mult, w, eps, n_out, ldn, n16, ldn16, M, n, stream);
 }
 
-// the same with y = the sum of nz slabs zs values apart (nz > 1: rows the register form takes)
+// the same with y = the sum of nz slabs zs values apart
 extern "C" int mn_axpy_rms_rows_slabs(float* x, int64_t ldx, const float* y, int64_t ldy, int nz, int64_t zs, float mult, const uint16_t* w, float eps,
                                       float* n_out, int64_t ldn, uint16_t* n16, int64_t ldn16, int M, int n, void* stream) {
   MN_CHECK_ARG(x && M >= 1 && n >= 1 && (w || (!n_out && !n16)), "mn_axpy_rms_rows: bad args");
   hipStream_t st = mn_stream(stream);
   const bool vec = (n % 4) == 0 && n <= 8192 && (ldx % 4) == 0 && (!y || (ldy % 4) == 0) && (!n_out || (ldn % 4) == 0) && (!n16 || (ldn16 % 4) == 0) &&
-                   (((uintptr_t)x | (uintptr_t)y | (uintptr_t)n_out) & 15) == 0 && (((uintptr_t)n16 | (uintptr_t)w) & 7) == 0;
-  MN_CHECK_ARG(nz == 1 || (nz > 1 && y && vec && (zs % 4) == 0), "mn_axpy_rms_rows: slabs need rows of at most 8192 values, a multiple of 4, 16-byte aligned");
+                   (((uintptr_t)x | (uintptr_t)y | (uintptr_t)n_out) & 15) == 0 && (((uintptr_t)n16 | (uintptr_t)w) & 7) == 0 && (nz == 1 || (zs % 4) == 0);
+  MN_CHECK_ARG(nz == 1 || (nz > 1 && y), "mn_axpy_rms_rows: bad slabs");
 #define MN_AR(V_) hipLaunchKernelGGL((axpy_rms_reg_kernel<V_>), dim3((unsigned)M), dim3(256), 0, st, x, ldx, y, ldy, nz, zs, mult, w, eps, n_out, ldn, n16, ldn16, n)
   if (vec && n <= 1024) MN_AR(1);
   else if (vec && n <= 2048) MN_AR(2);
   else if (vec && n <= 4096) MN_AR(4);
   else if (vec) MN_AR(8);
-  else hipLaunchKernelGGL(axpy_rms_kernel, dim3((unsigned)mn_cdiv(M, 4)), dim3(256), 0, st, x, ldx, y, ldy, mult, w, eps, n_out, ldn, n16, ldn16, M, n);
+  else hipLaunchKernelGGL(axpy_rms_kernel, dim3((unsigned)mn_cdiv(M, 4)), dim3(256), 0, st, x, ldx, y, ldy, nz, zs, mult, w, eps, n_out, ldn, n16, ldn16, M, n);
 #undef MN_AR
   MN_CHECK_LAUNCH("mn_axpy_rms_rows");
   return MN_OK;

@@ -70,6 +70,45 @@ def test_activations_in_the_products_epilogue(M, width, ff):
         assert rel(out[0], out[1]) < 3e-2                # two layers of products on bf16 operands (2^-9 each, some ten of them, of values up to 4 rms)
 
 
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("M", [65, 130, 300])
+def test_output_product_in_slabs(M, off):
+    """A hybrid prompt pass whose joined output product comes as split-K slabs, summed by the next layer's norm, the final norm and the trace's sum: against the
+    same layers in fp32 arithmetic; off: the caller's result and the norms' gains lie where no vector access may go."""
+    from ming_univision_amd._lib import lib
+    from ming_univision_amd.configuration import ZuzenexConfig
+    from ming_univision_amd.sequences import rows_of_spans
+    from ming_univision_amd.zuzenex import ZuzenexDecoder
+    W, ff = 128, 448
+    assert lib().mn_gemm256_plan_ksplit(M, W, 64 + ff, 0) > 1
+    mlp = dict(kind="dense", ff=ff)
+    cfg = ZuzenexConfig(width=W, vocab=40, norm=dict(eps=1e-6), layers=[
+        dict(type="attention", mixer=dict(heads=2, kv_heads=1, dim=32, vdim=32, scale=0.2), mlp=mlp),
+        dict(type="lightning", mixer=dict(heads=2, dim=32, vdim=32, decay=[0.9, 0.99]), mlp=mlp)])
+    got = []
+    for arith in ("bf16", "f32"):
+        dec = ZuzenexDecoder.synthetic(cfg, "cuda", t_max=M, n_seq=1, arith=arith)
+        x = dec.embed(torch.arange(M, device="cuda") % 40)
+        tabs = {k: torch.from_numpy(v).cuda() for k, v in rows_of_spans([(0, M, 0)], dec.block_rows, dec.chunk_rows).items() if k != "max_len"}
+        keep = []
+        if off and arith == "bf16":
+            for s, name in [(dec._layers[0], "norm1"), (dec._layers[1], "norm1"), (dec.struct, "final_w")]:
+                src = next(t for t in dec._keep if t.data_ptr() == getattr(s, name))
+                keep.append(torch.empty(W + 1, dtype=torch.bfloat16, device="cuda"))
+                keep[-1][1:] = src
+                setattr(s, name, keep[-1].data_ptr() + 2)
+        buf = torch.full((M * W + 2,), 7.0, device="cuda")
+        out, trace = buf[off:off + M * W].view(M, W), torch.empty(dec.n_trace, M, W, device="cuda")
+        for tr in (None, trace):
+            dec.step(x, tabs["row_seq"], tabs["row_slot"], tabs["row_back"], blk_tab=tabs["blk_tab"], max_len=M, out=out, trace=tr, chunk_tab=tabs["chunk_tab"])
+            got.append(out.clone())
+        got.append(trace)
+        assert bool((buf[off + M * W:] == 7.0).all())
+    assert rel(got[0], got[1]) < 1e-6                    # the trace takes the slabs in a launch of its own
+    for a, b in zip(got[:3], got[3:]):
+        assert rel(a, b) < 3e-2                          # (as above)
+
+
 @pytest.mark.parametrize("M,n", [(1, 4), (3, 1020), (5, 1024), (2, 1028), (70, 2048), (4, 4100), (3, 8192), (2, 8196), (3, 33)])
 def test_residual_and_rms_rows(M, n):
     """x += m y, RMS norm: rows in registers and the walking form (odd or very wide rows)."""

@@ -273,10 +273,12 @@ __device__ __forceinline__ void stage_silu(float* __restrict__ dst, int ld, cons
       for (int u = 0; u < 4; ++u) {
         const int x = x0 + 256 * u, j = x / lq, i = 4 * (x - j * lq);
         if (x >= cnt) break;
-        const float w = j < n ? f(j) : 0.f;
-        f32x4 r;
+        f32x4 r = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (j < n && i < d) {                          // (a chunk of a few rows: most waves have none)
+          const float w = f(j);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = j < n && i < d ? silu32(t[u][e]) * w : 0.f;
+          for (int e = 0; e < 4; ++e) r[e] = silu32(t[u][e]) * w;
+        }
         *reinterpret_cast<f32x4*>(dst + j * ld + i) = r;
       }
     }
@@ -330,48 +332,85 @@ __global__ __launch_bounds__(256) void light_scan_kv_mfma_kernel(LightScanArgs s
   }
 }
 
-// grid (ceil(dim vdim / 256), H): a thread walks its state value through all chunks of the pass, one sequence after the other.  The chunks' table entries
-// come through LDS, 256 at a time, and 16 chunks' sums are requested before the first is used: with a chain of dependent reads per
-// chunk the walk took 45 us for 64 chunks of 16 heads of 128 x 128 (134 MB), 38 us here.
-__global__ __launch_bounds__(256) void light_scan_carry_kernel(LightScanArgs s) {
+// grid (ceil(dim vdim / 256), H, Z): a thread walks its state value through the chunks of the sequences that start in its part of the pass (chunks
+// z per .. z per + per - 1), one sequence after the other.  The chunks' table entries come through LDS, 256 at a time, and 16 chunks' sums and start states are
+// requested before the first is used: with a chain of dependent reads per chunk the walk took 45 us for 64 chunks of 16 heads of 128 x 128 (134 MB), 38 us here.
+// Z: as many parts as give 16 workgroups a CU, so that small states (or heads) of many sequences go side by side.
+__global__ __launch_bounds__(256) void light_scan_carry_kernel(LightScanArgs s, int per) {
   constexpr int PRE = 16, TAB = 256;
   __shared__ int2 tab[TAB];                            // per chunk: rows; the cache sequence that starts here (-1: none; -2 - seq: it starts from zero)
+  __shared__ int first, stop;                          // of the table: the first chunk that starts a sequence, the first that starts one of the next part
   const LightArgs& a = s.b;
-  const int x = blockIdx.x * 256 + threadIdx.x, h = blockIdx.y, de = a.dim * a.vdim;
+  const int x = blockIdx.x * 256 + threadIdx.x, h = blockIdx.y, de = a.dim * a.vdim, tid = threadIdx.x;
+  const int beg = blockIdx.z * per, end = min(s.n_chunks, beg + per);
   const bool on = x < de;
   const float lam = a.decay[h], ll = lam > 0.f ? logf(lam) : 0.f;
   const int64_t step = (int64_t)a.H * de;
   float* sp = nullptr;
   float S = 0.f;
-  for (int c0 = 0; c0 < s.n_chunks; c0 += TAB) {
+  bool walking = false;
+  for (int c0 = beg; c0 < (walking ? s.n_chunks : end); c0 += TAB) {
     const int nc = min(TAB, s.n_chunks - c0);
     __syncthreads();
-    if ((int)threadIdx.x < nc) {
-      const int row = s.chunk_tab[2 * (c0 + threadIdx.x)], seq = a.row_seq[row];
-      tab[threadIdx.x] = int2{s.chunk_tab[2 * (c0 + threadIdx.x) + 1], a.row_back[row] != 0 ? -1 : (a.row_slot[row] != 0 ? seq : -2 - seq)};
+    if (tid == 0) first = stop = nc;
+    __syncthreads();
+    if (tid < nc) {
+      const int row = s.chunk_tab[2 * (c0 + tid)], seq = a.row_seq[row], y = a.row_back[row] != 0 ? -1 : (a.row_slot[row] != 0 ? seq : -2 - seq);
+      tab[tid] = int2{s.chunk_tab[2 * (c0 + tid) + 1], y};
+      if (y != -1) atomicMin(c0 + tid < end ? &first : &stop, tid);
     }
     __syncthreads();
-    if (!on) continue;
-    for (int ch = 0; ch < nc; ch += PRE) {
+    const int last = stop;
+    int ch = walking ? 0 : min(first, last);
+    walking = walking || ch < last;
+    for (; ch < last && on; ch += PRE) {
       float* w = s.ws + ((int64_t)(c0 + ch) * a.H + h) * de + x;
-      float kv[PRE];
-#pragma unroll
-      for (int u = 0; u < PRE; ++u) kv[u] = w[(int64_t)(min(ch + u, nc - 1) - ch) * step];
+      float kv[PRE], st[PRE];
 #pragma unroll
       for (int u = 0; u < PRE; ++u) {
-        if (ch + u >= nc) break;
+        kv[u] = st[u] = 0.f;
+        if (ch + u >= last) continue;
+        const int seq = tab[ch + u].y;
+        kv[u] = w[(int64_t)u * step];
+        if (seq >= 0) st[u] = a.state[((int64_t)seq * a.H + h) * de + x];
+      }
+#pragma unroll
+      for (int u = 0; u < PRE; ++u) {
+        if (ch + u >= last) break;
         const int2 t = tab[ch + u];
         if (t.y != -1) {                               // uniform: a sequence starts here
           if (sp) *sp = S;
           sp = a.state + ((int64_t)(t.y >= 0 ? t.y : -2 - t.y) * a.H + h) * de + x;
-          S = t.y >= 0 ? *sp : 0.f;
+          S = st[u];
         }
         w[(int64_t)u * step] = S;
         S = fmaf(powi32(lam, ll, t.x), S, kv[u]);
       }
     }
+    if (last < nc) break;                              // the next part's first sequence
   }
   if (sp) *sp = S;
+}
+
+// The same as a workgroup a chunk, of which the ones of a sequence's first chunk walk that sequence: passes of mostly one-chunk sequences (decode steps with a few
+// drafted tokens), where the table and the batches above are all overhead: 64 sequences of two rows, 4 heads of 64 x 64 6.8 us (14 as parts), 1024 of one row, 2
+// heads of 16 x 16 4.5 (10).
+__global__ __launch_bounds__(256) void light_scan_carry_short_kernel(LightScanArgs s) {
+  const LightArgs& a = s.b;
+  const int x = blockIdx.x * 256 + threadIdx.x, h = blockIdx.y, c0 = blockIdx.z, de = a.dim * a.vdim;
+  const int r0 = s.chunk_tab[2 * c0];
+  if (a.row_back[r0] != 0 || x >= de) return;
+  const float lam = a.decay[h], ll = lam > 0.f ? logf(lam) : 0.f;
+  float* sp = a.state + ((int64_t)a.row_seq[r0] * a.H + h) * de + x;
+  float S = a.row_slot[r0] == 0 ? 0.f : *sp;
+  for (int ch = c0; ch < s.n_chunks; ++ch) {
+    if (ch > c0 && a.row_back[s.chunk_tab[2 * ch]] == 0) break;      // the next sequence starts here
+    float* w = s.ws + ((int64_t)ch * a.H + h) * de + x;
+    const float kv = *w;
+    *w = S;
+    S = fmaf(powi32(lam, ll, s.chunk_tab[2 * ch + 1]), S, kv);
+  }
+  *sp = S;
 }
 
 template <int CV>
@@ -826,20 +865,31 @@ extern "C" int mn_lightning_rows_scan_ex(const float* qkv, int64_t ldqkv, int M,
   const bool v4 = (vdim % 4) == 0 && (((uintptr_t)workspace) & 15) == 0;
   // quadruples of 16-byte aligned values throughout the rows: vector staging
   const bool r4 = ((dim | vdim) % 4) == 0 && ((ldqkv | ldo) % 4) == 0 && (((uintptr_t)qkv | (uintptr_t)out | (uintptr_t)workspace) & 15) == 0;
+  // chunks half empty on average: most are sequences of their own, of a few rows.  Their own sums go by rows (64 chunks of two, 16 heads of 128 x 128: 14 us, 27 as
+  // tiles of 32 rows; 1024 of one row, 2 heads of 16 x 16 6.4 either way), the walk over the chunks by chunks.
+  const bool few = (int64_t)n_chunks * (LCH / 2) >= M && n_chunks <= 65535;
   const int ldk1 = ((dim + 15) / 16 * 16 + 47) / 64 * 64 + 16, ldv1 = ((vdim + 15) / 16 * 16 + 47) / 64 * 64 + 16;      // 16 mod 64: the four rows of an operand read fall in banks of their own
   const size_t lds1 = (size_t)LCH * (ldk1 + ldv1) * sizeof(float);
-  if (variant == MN_LIGHTNING_SCAN_MFMA && lds1 <= 64 * 1024) {
+  if (variant == MN_LIGHTNING_SCAN_MFMA && lds1 <= 64 * 1024 && !few) {
     if (r4) hipLaunchKernelGGL((light_scan_kv_mfma_kernel<true>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), lds1, st, s, ldk1, ldv1);
     else hipLaunchKernelGGL((light_scan_kv_mfma_kernel<false>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), lds1, st, s, ldk1, ldv1);
   } else if (v4) hipLaunchKernelGGL((light_scan_kv_kernel<4>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), (size_t)LCH * (dim + vdim) * sizeof(float), st, s);
   else hipLaunchKernelGGL((light_scan_kv_kernel<1>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), (size_t)LCH * (dim + vdim) * sizeof(float), st, s);
   MN_CHECK_LAUNCH("mn_lightning_rows_scan(sums)");
-  hipLaunchKernelGGL(light_scan_carry_kernel, dim3((unsigned)mn_cdiv((int64_t)dim * vdim, 256), (unsigned)H), dim3(256), 0, st, s);
+  const int64_t de256 = mn_cdiv((int64_t)dim * vdim, 256);
+  if (few) {
+    hipLaunchKernelGGL(light_scan_carry_short_kernel, dim3((unsigned)de256, (unsigned)H, (unsigned)n_chunks), dim3(256), 0, st, s);
+  } else {
+    const int64_t want = mn_cdiv(16 * (int64_t)mn_num_cus(), de256 * H);
+    const int per = (int)mn_cdiv(n_chunks, want < n_chunks ? want : n_chunks);
+    hipLaunchKernelGGL(light_scan_carry_kernel, dim3((unsigned)de256, (unsigned)H, (unsigned)mn_cdiv(n_chunks, per)), dim3(256), 0, st, s, per);
+  }
   MN_CHECK_LAUNCH("mn_lightning_rows_scan(carry)");
   if (variant == MN_LIGHTNING_SCAN_MFMA) {
     MN_CHECK_ARG(scan_mfma_lds(dim, vdim) <= 64 * 1024, "mn_lightning_rows_scan: heads of %d + %d values do not fit the matrix-core pass", dim, vdim);
-    if (r4) hipLaunchKernelGGL((light_scan_out_mfma_kernel<true>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), scan_mfma_lds(dim, vdim), st, s,
-                               scan_ldq(dim), scan_ldv(vdim));
+    // (the vector form deals out 64 columns at a time to four waves a SIMD, where the other has six: 1024 chunks of one row, 2 heads of 16 x 16: 19.5 against 12.5 us)
+    if (r4 && vdim > 32) hipLaunchKernelGGL((light_scan_out_mfma_kernel<true>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), scan_mfma_lds(dim, vdim), st, s,
+                                            scan_ldq(dim), scan_ldv(vdim));
     else hipLaunchKernelGGL((light_scan_out_mfma_kernel<false>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), scan_mfma_lds(dim, vdim), st, s,
                             scan_ldq(dim), scan_ldv(vdim));
   } else if (v4) hipLaunchKernelGGL((light_scan_out_kernel<4>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), lds3, st, s);

@@ -127,7 +127,7 @@ def test_residual_and_rms_rows(M, n):
 
 @pytest.mark.parametrize("T,H,d,e", [(65, 2, 16, 16), (100, 3, 20, 36), (1000, 2, 128, 128), (2100, 1, 64, 100), (70, 2, 6, 10)])
 def test_lightning_scan(T, H, d, e):
-    """The chunked recurrence around its batches of eight chunks, two sequences in one pass (one continuing), vector and scalar staging, against the
+    """The chunked recurrence around its batches of 16 chunks, two sequences in one pass (one continuing), vector and scalar staging, against the
     recurrence in float64."""
     import numpy as np
     from ming_univision_amd._lib import check, current_stream, lib, ptr
@@ -171,3 +171,40 @@ def test_rows_far_apart(M, lda):
     w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
     ref = a.double() @ w.double().T
     assert rel(ops.gemm_bf16(a, w, None, "f32"), ref) < 3e-5 and rel(ops.gemm_bf16(a, w, None, "bf16"), ref) < 2 ** -8
+
+
+@pytest.mark.parametrize("H,d,e", [(2, 16, 16), (3, 20, 36), (16, 128, 128)])
+@pytest.mark.parametrize("lens", [[2] * 64, [1, 33, 64, 1, 1, 700, 2] * 2, [1] * 300 + [40, 3] + [2] * 20, [8300]])
+def test_lightning_scan_of_many_sequences(H, d, e, lens):
+    """The walk over the chunks cut into parts: sequences of one chunk and of many, begun before and behind a part's end, new and continuing, more chunks than the
+    256 of a table; the states carried, against the recurrence in float64."""
+    import numpy as np
+    from ming_univision_amd._lib import check, current_stream, lib, ptr
+    from ming_univision_amd.sequences import rows_of_spans
+    if H == 16 and len(lens) > 100:
+        return
+    L, g = lib(), torch.Generator(device="cuda").manual_seed(H + len(lens))
+    n = len(lens)
+    order = [(7 * i + 3) % n if n % 7 else i for i in range(n)]
+    spans = [(order[i], m, 5 * (i % 3)) for i, m in enumerate(lens)]
+    tabs = rows_of_spans(spans, 4, L.mn_lightning_chunk_rows())
+    dev = {k: torch.from_numpy(np.ascontiguousarray(v)).cuda() for k, v in tabs.items() if k != "max_len"}
+    T, n_ch = sum(lens), dev["chunk_tab"].shape[0]
+    qkv, S0 = torch.randn(T, H * (2 * d + e), generator=g, device="cuda"), torch.randn(n, H, d, e, generator=g, device="cuda")
+    decay = torch.tensor([0.5, 0.97, 0.999] * 6)[:H].cuda()
+    state, out = S0.clone(), torch.empty(T, H * e, device="cuda")
+    ws = torch.empty(L.mn_lightning_scan_workspace_bytes(n_ch, H, d, e), dtype=torch.uint8, device="cuda")
+    check(L.mn_lightning_rows_scan(ptr(qkv), qkv.shape[1], T, H, d, e, ptr(decay), ptr(state), ptr(dev["row_seq"]), ptr(dev["row_slot"]), ptr(dev["row_back"]),
+                                   ptr(dev["chunk_tab"]), n_ch, ptr(out), H * e, ptr(ws), ws.numel(), current_stream()), "scan")
+    act, r = F.silu(qkv.double()), 0
+    for seq, m, past in spans:
+        S = S0[seq].double() * (past != 0)
+        q, k, v = act[r:r + m, :H * d].reshape(m, H, d), act[r:r + m, H * d:2 * H * d].reshape(m, H, d), act[r:r + m, 2 * H * d:].reshape(m, H, e)
+        pw = decay.double()[:, None] ** torch.arange(m - 1, -1, -1, device="cuda", dtype=torch.float64)[None]
+        end = decay.double()[:, None, None] ** m * S + ((k * pw.T[..., None]).permute(1, 2, 0).contiguous() @ v.permute(1, 0, 2).contiguous())
+        assert rel(state[seq], end) < 1e-5
+        first = ((decay.double()[:, None, None] * S + k[0, :, :, None] * v[0, :, None, :]) * q[0, :, :, None]).sum(1).reshape(-1)
+        assert float((out[r].double() - first).abs().max() / first.abs().max()) < 1e-5
+        last = (end * q[m - 1, :, :, None]).sum(1).reshape(-1)
+        assert float((out[r + m - 1].double() - last).abs().max() / last.abs().max()) < 1e-5
+        r += m

@@ -15,7 +15,7 @@ __device__ __forceinline__ float sum8(float v) {                    // over the 
 
 // First row of the step's sequence j (its rows' row_back counts 0, 1, ..), -1 if the step has fewer: 256 threads, the same result in all of them.
 // A launch of sequences x channels whose workgroups look theirs up beats one workgroup a row of which most find nothing to do: 1409 rows x 64
-// workgroups with 35 KB of LDS each took 33 us to come and go.
+// workgroups with 35 KB of LDS each took 33 us to come and go.  (Rows beyond sequence_starts's table.)
 __device__ __forceinline__ int sequence_start(const int32_t* __restrict__ row_back, int M, int j, uint64_t (&mask)[32]) {
   const int tid = threadIdx.x;
   for (int base = 0; base < M; base += 2048) {
@@ -38,6 +38,35 @@ __device__ __forceinline__ int sequence_start(const int32_t* __restrict__ row_ba
     }
   }
   return -1;
+}
+
+// The step's sequences at once, where its rows are at most 2048: first[j] = sequence j's first row, first[count] = M; the count comes back (256 threads)
+__device__ __forceinline__ int sequence_starts(const int32_t* __restrict__ row_back, int M, uint64_t (&mask)[32], uint16_t (&first)[2049]) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int m = 256 * k + tid;
+    const uint64_t b = __ballot(m < M && row_back[m < M ? m : 0] == 0);
+    if (lane == 0) mask[4 * k + wave] = b;
+  }
+  __syncthreads();
+  const int own = lane < 32 ? __popcll(mask[lane & 31]) : 0;
+  int upto = own;
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) {
+    const int t = __shfl_up(upto, o, 64);
+    upto += lane >= o ? t : 0;
+  }
+  const int count = __shfl(upto, 31, 64);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const uint64_t b = mask[4 * k + wave];
+    const int before = __shfl(upto - own, 4 * k + wave, 64);
+    if ((b >> lane) & 1) first[before + __popcll(b & (((uint64_t)1 << lane) - 1))] = (uint16_t)(256 * k + tid);
+  }
+  if (tid == 0) first[count] = (uint16_t)M;
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(count);
 }
 
 // Gated delta rule, preparation of a row: channels [q: G dim ; k: G dim ; v: H vdim] of the raw projections go through their causal

@@ -394,13 +394,13 @@ __global__ __launch_bounds__(256) void delta_rows_kernel(DeltaArgs a) {
 }
 
 // The same walk for heads of at most 256 state rows, without a branch in the step: grid (H * ceil(vdim / CPB), S):
-// workgroup y takes the step's sequences y, y + S, ..  LPC lanes share a value column
+// workgroup y takes the step's sequences y, y + S, .., from a table of their first rows that it makes once (TABLE: at most 2048 rows).  LPC lanes share a value column
 // (CPB = 256 / LPC columns a workgroup); a lane holds the state rows 4 (s + LPC jj) + t, t < 4, jj < NS / 4, so that q and k come from
 // LDS in 16-byte reads; LDS rows are padded with zeros to DP = NS * LPC values, under which the padded state rows stay zero.
 // A serial chain: what bounds it is the instructions of a step.  Four steps are unrolled with the operands in alternating registers (no moves), the sums are
-// DPP additions, outputs stay in a lane until LPC of them are written at once.  1409 rows in 5 sequences (the longest 470), 8 heads of 128 + 128: 106 us
-// (195 with a workgroup per row and 830 cycles a step).
-template <int NS, int LPC, int DBT>
+// DPP additions, outputs stay in a lane until LPC of them are written at once.  1409 rows in 5 sequences (the longest 470), 8 heads of 128 + 128: 101 us
+// (195 with a workgroup per row and 830 cycles a step); 512 sequences of two rows 374 (431; 493 with every sequence looked for from the step's first row).
+template <int NS, int LPC, int DBT, bool TABLE>
 __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
   constexpr int CPB = 256 / LPC, DP = NS * LPC, NQ = DBT * 2 * DP / 256, NV = (DBT * CPB + 255) / 256;
   extern __shared__ float lds[];             // [DBT][2 DP] q, k; [DBT][CPB] v; [DBT] beta, decay, k . q; [DBT][CPB] outputs
@@ -409,15 +409,23 @@ __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
   const int d = a.dim, kvh = h / (a.H / a.G);
   const bool on = c < a.vdim;
   __shared__ uint64_t mask[32];
-  for (int seq = blockIdx.y;; seq += gridDim.y) {
-    const int m0 = __builtin_amdgcn_readfirstlane(sequence_start(a.row_back, a.M, seq, mask));
-    if (m0 < 0) return;
-    int n = 1;
-    for (;;) {
-      const int m = m0 + n + tid;
-      const int cnt = __syncthreads_count(m < a.M && a.row_back[m] == m - m0);
-      n += cnt;
-      if (cnt < 256) break;
+  __shared__ uint16_t first[2049];
+  const int count = TABLE ? sequence_starts(a.row_back, a.M, mask, first) : a.M;
+  for (int seq = blockIdx.y; seq < count; seq += gridDim.y) {
+    int m0, n;
+    if constexpr (TABLE) {
+      m0 = __builtin_amdgcn_readfirstlane(first[seq]);
+      n = __builtin_amdgcn_readfirstlane(first[seq + 1]) - m0;
+    } else {
+      m0 = __builtin_amdgcn_readfirstlane(sequence_start(a.row_back, a.M, seq, mask));
+      if (m0 < 0) return;
+      n = 1;
+      for (;;) {
+        const int m = m0 + n + tid;
+        const int cnt = __syncthreads_count(m < a.M && a.row_back[m] == m - m0);
+        n += cnt;
+        if (cnt < 256) break;
+      }
     }
     float* sp = a.state + (((int64_t)a.row_seq[m0] * a.H + h) * d) * a.vdim + (on ? c : 0);
     const bool fresh = a.row_slot[m0] == 0;
@@ -703,13 +711,16 @@ extern "C" int mn_gated_delta_rows(const float* qkv, int64_t ld, const float* bd
   }
   if (dim <= 256) {
     MN_CHECK_ARG(M <= 65535 && (int64_t)H * mn_cdiv(vdim, 16) < ((int64_t)1 << 31), "mn_gated_delta_rows: too many rows or columns");
-    // sequences walked side by side: two workgroups a CU (what LDS lets in), the rest one after the other
-    auto slots = [&](int64_t gx) { const int64_t y = 2 * (int64_t)mn_num_cus() / gx; return (unsigned)(y < 1 ? 1 : (y < M ? y : M)); };
-#define MN_DF(NS_, LPC_, DB_)                                                                                                                 \
-  hipLaunchKernelGGL((delta_rows_fast_kernel<NS_, LPC_, DB_>), dim3((unsigned)(H * mn_cdiv(vdim, 256 / LPC_)), slots(H * mn_cdiv(vdim, 256 / LPC_))), dim3(256),  \
+    // sequences walked side by side: four workgroups a CU, the rest one after the other (64 sequences of two rows, 8 heads of 128 x 128 53 us with four, 51 with two, 61
+    // with three; 4 heads of 64 x 64 10.4, 12.1, 11.6; 1024 sequences of one row, 2 heads of 16 x 16 10.8, 13.5, 11.2)
+    auto slots = [&](int64_t gx) { const int64_t y = 4 * (int64_t)mn_num_cus() / gx; return (unsigned)(y < 1 ? 1 : (y < M ? y : M)); };
+#define MN_DFT(NS_, LPC_, DB_, T_)                                                                                                                 \
+  hipLaunchKernelGGL((delta_rows_fast_kernel<NS_, LPC_, DB_, T_>), dim3((unsigned)(H * mn_cdiv(vdim, 256 / LPC_)), slots(H * mn_cdiv(vdim, 256 / LPC_))), dim3(256),  \
                      ((size_t)DB_ * 2 * NS_ * LPC_ + 2 * DB_ * (256 / LPC_) + 3 * DB_) * sizeof(float), st, a)
+#define MN_DF(NS_, LPC_, DB_) do { if (M <= 2048) MN_DFT(NS_, LPC_, DB_, true); else MN_DFT(NS_, LPC_, DB_, false); } while (0)
     if (dim <= 32) MN_DF(4, 8, 32); else if (dim <= 64) MN_DF(4, 16, 32); else if (dim <= 128) MN_DF(8, 16, 32); else MN_DF(16, 16, 16);
 #undef MN_DF
+#undef MN_DFT
   } else {
     const size_t lds = ((size_t)DB * 2 * dim + DB * 32 + 3 * DB) * sizeof(float);    // 16 rows of q and k: 64 KiB at dim 512
     if (lds > 64 * 1024) {

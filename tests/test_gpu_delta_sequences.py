@@ -40,3 +40,33 @@ def test_many_sequences(H, G, d, e, lens):
         assert err(out[sl].reshape(-1, H, e), torch.stack(ref)) < 2e-5, i
         assert err(sd[order[i]], S) < 2e-5, i
         r0 += lens[i]
+
+
+@pytest.mark.parametrize("H,G,d,e,n,m", [(1, 1, 8, 4, 2048, 1), (2, 1, 36, 16, 682, 3), (3, 3, 130, 20, 1023, 2), (1, 1, 8, 16, 2049, 1), (2, 2, 70, 33, 64, 32)])
+def test_tables_of_sequences(H, G, d, e, n, m):
+    """Up to 2048 rows the step's sequences come from one table, filled to its last entry; more rows are looked through.  Here n sequences of m rows.  A row whose
+    k . q is next to nothing has a result next to nothing: the errors are held to 2e-5 of the pass's largest value, of which every sum's terms are a part."""
+    check, stream, L, ptr = _api()
+    g = torch.Generator().manual_seed(n + d)
+    M = n * m
+    q, k, v, beta, dec = delta_inputs(g, M, H, G, d, e)
+    state = torch.randn(n, H, d, e, generator=g) * 0.3
+    past = torch.arange(n) % 2 * 5
+    sd = state.cuda()
+    r = _rows([(n - 1 - i, m, int(past[i])) for i in range(n)])
+    qkv = torch.cat([q.reshape(M, -1), k.reshape(M, -1), v.reshape(M, -1)], 1)
+    out = torch.full((M + 1, H * e), 7.0, device="cuda")
+    check(L.mn_gated_delta_rows(ptr(D(qkv)), qkv.shape[1], ptr(D(torch.cat([beta, dec], 1))), 2 * H, M, H, G, d, e, ptr(sd), ptr(r["row_seq"]), ptr(r["row_slot"]),
+                                ptr(r["row_back"]), 0, ptr(out), H * e, stream()))
+    assert bool((out[M] == 7.0).all())
+    S = state.flip(0).double() * (past > 0).double()[:, None, None, None]
+    ref = torch.empty(n, m, H, e, dtype=torch.float64)
+    rows = lambda t, w: t.double().reshape(n, m, *w)  # noqa: E731
+    qq, kk = (rows(t, (G, d)).repeat_interleave(H // G, 2) for t in (q, k))
+    vv, bb, dd = rows(v, (H, e)), rows(beta, (H,)), rows(dec, (H,))
+    for t in range(m):
+        S = dd[:, t, :, None, None] * S
+        u = bb[:, t, :, None] * (vv[:, t] - (S * kk[:, t, :, :, None]).sum(2))
+        S = S + kk[:, t, :, :, None] * u[:, :, None]
+        ref[:, t] = (S * qq[:, t, :, :, None]).sum(2)
+    assert err(out[:M].reshape(n, m, H, e), ref) < 2e-5 and err(sd.flip(0), S) < 2e-5

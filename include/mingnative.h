@@ -261,6 +261,8 @@ MN_API int mn_gemm_bf16_grouped(const uint16_t* A, int64_t lda, const uint16_t* 
  * epilogue: enum mn_gemm_epilogue. */
 /* Slices to ask of a split-K launch on these sizes (hilo: a is a bf16 hi/lo pair), 0: one slice is best. */
 MN_API int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo);
+/* The same for mn_gemm256_f8's product (at least 1). */
+MN_API int mn_gemm256_f8_plan_ksplit(int M, int N, int K);
 MN_API int mn_gemm256_supported(int64_t lda, int64_t a_lo_off, int64_t ldw, int64_t w_rows, int M, int N, int K);
 MN_API int mn_gemm256(const uint16_t* A, int64_t lda, int64_t a_lo_off, const uint16_t* W, int64_t ldw, const uint16_t* bias,
                void* C, int64_t ldc, int M, int N, int K, int epilogue, void* stream);

@@ -304,6 +304,7 @@ SYMBOLS = {
     "mn_moe_combine": (_i, [_p, _i64, _p, _p, _i, _p, _i64, _i, _i, _p]),
     "mn_gemm_bf16_grouped": (_i, [_p, _i64, _p, _i64, _i64, _p, _p, _i, _p, _i64, _i, _i, _i, _i, _p]),
     "mn_gemm256_plan_ksplit": (_i, [_i, _i, _i, _i]),
+    "mn_gemm256_f8_plan_ksplit": (_i, [_i, _i, _i]),
     "mn_gemm256_supported": (_i, [_i64, _i64, _i64, _i64, _i, _i, _i]),
     "mn_gemm256": (_i, [_p, _i64, _i64, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _p]),
     "mn_gemm256_splitk": (_i, [_p, _i64, _i64, _p, _i64, _p, _p, _i, _i, _i, _i, _p]),

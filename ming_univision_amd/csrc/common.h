@@ -200,3 +200,4 @@ extern "C" int mn_gemm256_slices(int K, int ksplit);
 extern "C" int mn_axpy_rms_rows_slabs(float* x, int64_t ldx, const float* y, int64_t ldy, int nz, int64_t zs, float mult, const uint16_t* w, float eps,
                                       float* n_out, int64_t ldn, uint16_t* n16, int64_t ldn16, int M, int n, void* stream);
 extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo);
+extern "C" int mn_gemm256_f8_plan_ksplit(int M, int N, int K);

@@ -599,6 +599,20 @@ extern "C" int mn_gemm256_slices(int K, int ksplit) {
   const int Kc = (int)(mn_cdiv(mn_cdiv(K, ksplit), 2 * BK) * 2 * BK);
   return (int)mn_cdiv(K, Kc);
 }
+// The e4m3 product has the 256 x 256 form alone, with half the K-tiles of the same K: its own request, rounds of workgroups x (K-tiles of a slice at 1.9 us
+// a 64 values + 10 us) + the slabs at 4 TB/s.  3072 x 8192, product and the slabs' read, at this request against the one of the forms above: 41 rows (16 / 8 slices)
+// 16.8 / 18.3 us, 128 (16 / 5) 28.2 / 31.1, 300 (7 / 4) 33.8 / 37.1, 384 (7 / 3) 35.9 / 41.1, 768 (3 / 3) 47.4.
+extern "C" int mn_gemm256_f8_plan_ksplit(int M, int N, int K) {
+  const double tiles = (double)(mn_cdiv(M, 128) * mn_cdiv(N, 256));
+  const int kt = K / BK;
+  int best = 1;
+  double tb = 1e30;
+  for (int ks = 1; ks <= 16 && kt / ks >= 4; ++ks) {
+    const double t = (double)mn_cdiv((int64_t)(tiles * ks), 256) * ((double)mn_cdiv(kt, ks) * 1.9 + 10.0) + (ks > 1 ? (double)ks * M * N * 8.0 / 4.0e6 : 0.0);
+    if (t < tb) { tb = t; best = ks; }
+  }
+  return best;
+}
 extern "C" int mn_gemm256_f8_slices(int K, int ksplit) {      // the fp8 regime: 128 k per K-tile
   if (ksplit <= 1) return 1;
   const int Kc = (int)(mn_cdiv(mn_cdiv(K, ksplit), 4 * BK) * 4 * BK);

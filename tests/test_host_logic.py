@@ -131,6 +131,19 @@ def test_splitk_plan_for_few_row_residual_gemms():
         assert 2 <= ks <= 8 and K // ks >= 256 and tiles * ks <= 512, (M, N, K, ks)
 
 
+def test_split_of_the_e4m3_product_follows_its_own_tiles():
+    """mn_gemm256_f8_plan_ksplit: 256 x 256 tiles alone, so few rows want as many K-slices as keep four 64-value tiles (3072 x 8192 and 1024 x 4096, where 16 slices
+    of 41 .. 128 rows measured fastest, 6 .. 8 of 300 .. 384, one of 2048), and every slice of a request is a whole number of its 128-value tiles."""
+    import ctypes
+    from ming_univision_amd import _lib
+    L = ctypes.CDLL(_lib.LIB_PATH)
+    plan, cut = L.mn_gemm256_f8_plan_ksplit, L.mn_gemm256_f8_slices
+    for rows, least, most in ((41, 12, 16), (65, 12, 16), (96, 8, 16), (128, 8, 16), (192, 8, 12), (300, 6, 8), (384, 6, 8), (768, 3, 5), (1024, 2, 4), (2048, 1, 1)):
+        ks = plan(rows, 3072, 8192)
+        assert least <= ks <= most and 1 <= cut(8192, ks) <= ks, (rows, ks)
+    assert plan(41, 1024, 4096) == 16 and 1 <= plan(2048, 1024, 4096) <= 6 and plan(64, 256, 128) == 1
+
+
 def test_config_shapes_and_sizes():
     cfg = C.MingUniVisionConfig.ming_univision_16b_a3b()
     n_llm = sum(int(torch.tensor(s).prod()) for s in C.llm_param_shapes(cfg.llm_config).values())

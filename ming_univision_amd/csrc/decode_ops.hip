@@ -507,7 +507,7 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
   }
 }
 
-// GQA form from 8 rows on: one wave per (row, KV head, split) serves all G = n_q / n_kv query heads of its group, so every
+// GQA form from some 40 (row, KV head) pairs on: one wave per (row, KV head, split) serves all G = n_q / n_kv query heads of its group, so every
 // K / V line is loaded ONCE per group instead of once per query head (the per-head kernel above re-reads them through L1:
 // 4x the load instructions at G = 4).  Same partial layout, same combine kernel.  Block = 4 waves = 4 KV heads of one row.
 template <int HD, int G>
@@ -860,9 +860,13 @@ __global__ __launch_bounds__(1024) void attn_decode_one_kernel(
 
 // Key-range splits (flash-decoding): enough workgroups to fill the chip at few rows, none needed at hundreds of rows;
 // one split never holds more than 4096 keys (its scores live in LDS).
-// One wave a (row, KV head, split) reads every key once for its four heads; from 8 rows on there are enough of them (a step of 64 rows at 1100 keys 10.8 ->
-// 10.3 ms, 40 rows at 1800 10.5 -> 9.7, 20 rows at 1100 7.53 -> 7.39, 8 rows at 1500 5.26 -> 5.16; 3 rows at 1800 3.80 against 3.90)
-static bool attn_use_gqa(int M, int n_q, int n_kv, int hd) { return M >= 8 && hd == 128 && n_q == 4 * n_kv; }
+// One wave a (row, KV head, split) reads every key once for its four heads, where there are enough (row, KV head) pairs: 40, with two KV heads 48 (cold caches, us,
+// this form against one wave a head: 12 rows x 4 KV heads 28 / 32, 64 x 4 65 / 90, 24 x 2 33 / 38, 16 x 3 23 / 25; but 8 x 4 25.6 / 23.9, 20 x 2 22.9 / 21.7, 12 x 3
+// 26.5 / 26.1; a step of 28 layers with 11 rows 5.82 / 5.92 ms, with 8 5.28 / 5.24).  With one KV head three of a workgroup's four waves repeat the fourth's
+// work (64 x 1 37 / 29).
+static bool attn_use_gqa(int M, int n_q, int n_kv, int hd) {
+  return (M > 64 || (n_kv >= 2 && M * n_kv >= (n_kv == 2 ? 48 : 40))) && hd == 128 && n_q == 4 * n_kv;
+}
 // the one-launch form: <= g_one_rows rows whose caches hold <= 1024 keys (dev-library A/B: mn_attn_tune_one)
 static int g_one_rows = 16;
 #ifdef MN_DEV_HOOKS

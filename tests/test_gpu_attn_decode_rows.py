@@ -1,4 +1,4 @@
-"""Decode attention around the row count from which one wave serves a key head's four query heads (8 rows), past the caches the one-launch form takes: rows of
+"""Decode attention around the row counts from which one wave serves a key head's four query heads (40 pairs of row and key head, 48 with two), past the caches the one-launch form takes: rows of
 1 .. t_max keys, splits that hold no key of a row, holes in the mask, fp32 and hi / lo outputs.  The reference is float64; fp32 sums of at most 1300 products: 1e-5
 of the largest value."""
 import pytest

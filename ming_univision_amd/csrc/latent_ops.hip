@@ -634,9 +634,9 @@ __global__ __launch_bounds__(1024) void latent_attn_kernel(const float* __restri
 // 18 here).
 struct PlainScore { __device__ __forceinline__ float operator()(float s) const { return s; } };
 template <int NB, int KF, bool VEC>
-__global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __restrict__ qabs, const float* __restrict__ arena,
+__global__ __launch_bounds__(256, VEC && NB <= 8 ? 2 : 1) void latent_attn_mfma_kernel(const float* __restrict__ qabs, const float* __restrict__ arena,
                                                                const int32_t* __restrict__ row_seq, const int32_t* __restrict__ row_len,
-                                                               const int32_t* __restrict__ blk_tab, int H, int r, int t_max,
+                                                               const int32_t* __restrict__ blk_tab, int H, int r_, int t_max,
                                                                int tiles_per_split, float* __restrict__ lat, float* __restrict__ part_acc,
                                                                float* __restrict__ part_ml, int KS, int M) {
   using Walk = LatentWalk<NB, KF, VEC, PlainScore>;
@@ -645,6 +645,8 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const float* __re
   const int nqv = nrows * H, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
   // (one pass unless the grid was cut for runs of one row and this one is longer)
   for (int qv0 = blockIdx.y * 16; qv0 < nqv; qv0 += 16 * gridDim.y) {
+    int r = r_;
+    asm("" : "+s"(r));                     // (what depends on it is not held over the passes: it would cost half the waves)
     const int64_t seq = row_seq[row0];
     const int len = row_len[row0 + nrows - 1];
     const bool on = qv0 + c < nqv;

@@ -83,7 +83,7 @@ __device__ __forceinline__ bool emit_vec(const AttnTArgs& a) {
 // VEC: dim and vdim are multiples of 4.
 template <int NBD, int NBV, bool VEC>
 __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_blk, int hv) {
-  constexpr int KT = NBD + NBV > 4 ? 16 : 32, KF = KT / 16, AQ = 16, LDK = 64 * NBD + 4, LDV = 64 * NBV + 4, TILE = KT * (LDK + LDV);
+  constexpr int KT = NBD + NBV > 4 ? 16 : 32, KF = KT / 16, LDK = 64 * NBD + 4, LDV = 64 * NBV + 4, TILE = KT * (LDK + LDV);
   __shared__ __attribute__((aligned(16))) float lds[2 * TILE];        // [2][K tile | V tile]
   __shared__ int tab[16][4], met;                      // met: an infinite or NaN value
   const int tid = threadIdx.x, gy = blockIdx.y, sp = blockIdx.z;
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_bl
     lrun += __shfl_xor(lrun, 32);
     if (mine) {
       const int qv = rin * Rc + hc;                    // the vector's place in its run's partial slab
-      float* part = a.nsplit > 1 ? a.part + (((int64_t)(b0 + run) * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)AQ * (2 + a.vdim)) : nullptr;
+      float* part = a.nsplit > 1 ? a.part + (((int64_t)(b0 + run) * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)a.sq * (2 + a.vdim)) : nullptr;
       const int64_t col0 = (int64_t)(h0 + hc) * a.vdim;
       const float inv = part ? 1.f : a.out_scale * softmax_inv(mrun, lrun, a.sink, h0 + hc);
       const bool vec = emit_vec(a);
@@ -252,9 +252,9 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_bl
           if (!part) { emit4(a, r, row, col0, d, vec); continue; }
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            if (d + e < a.vdim) part[2 * AQ + (int64_t)qv * a.vdim + d + e] = r[e];
+            if (d + e < a.vdim) part[2 * a.sq + (int64_t)qv * a.vdim + d + e] = r[e];
         }
-      if (part && g4 == 0) { part[qv] = mrun; part[AQ + qv] = lrun; }
+      if (part && g4 == 0) { part[qv] = mrun; part[a.sq + qv] = lrun; }
       if (met) {
 #pragma unroll 1
         for (int x = 0; x < 16 * NBV; ++x) {           // this lane's columns again: what is not finite among the seen keys' values
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_bl
           }
           if (odd == 0.f) continue;
           odd *= inv;
-          if (part) { part[2 * AQ + (int64_t)qv * a.vdim + d] = odd; continue; }
+          if (part) { part[2 * a.sq + (int64_t)qv * a.vdim + d] = odd; continue; }
           odd = gated(a, odd, row, col0 + d);
           if (a.out) a.out[(int64_t)row * a.ldo + col0 + d] = odd;
           if (a.out16) a.out16[(int64_t)row * a.ldo16 + col0 + d] = f32_to_bf16(odd);
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_bl
 // 2048 tokens, 16 heads, keys of 576 and values of 512, window 1024 (54.8 GF): 1674 us in the form before, 761 us here.
 template <int NB, bool VEC>
 __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, int n_blk, int hv) {
-  constexpr int KT = 16, AQ = 16, QF = 2, LDK = 64 * NB + 4, LDS_S = 20;
+  constexpr int KT = 16, QF = 2, LDK = 64 * NB + 4, LDS_S = 20;
   __shared__ __attribute__((aligned(16))) float K[KT * LDK];
   __shared__ __attribute__((aligned(16))) float Sp[4][16 * QF * LDS_S];     // [wave][query][16 keys]: partial scores
   __shared__ int tab[16][4], met;
@@ -440,7 +440,7 @@ __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, i
       lrun[f] += __shfl_xor(lrun[f], 32);
       if (hi[f] < 0) continue;                         // not of this sequence
       const int qv = (row[f] - tab[run[f]][0]) * Rc + hc;
-      float* part = a.nsplit > 1 ? a.part + (((int64_t)(b0 + run[f]) * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)AQ * (2 + a.vdim)) : nullptr;
+      float* part = a.nsplit > 1 ? a.part + (((int64_t)(b0 + run[f]) * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)a.sq * (2 + a.vdim)) : nullptr;
       const int64_t col0 = (int64_t)(h0 + hc) * a.vdim;
       const float inv = part ? 1.f : a.out_scale * softmax_inv(mrun[f], lrun[f], a.sink, h0 + hc);
 #pragma unroll
@@ -451,9 +451,9 @@ __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, i
         if (!part) { emit4(a, r, row[f], col0, d, vec); continue; }
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (d + e < a.vdim) part[2 * AQ + (int64_t)qv * a.vdim + d + e] = r[e];
+          if (d + e < a.vdim) part[2 * a.sq + (int64_t)qv * a.vdim + d + e] = r[e];
       }
-      if (part && wave == 0 && g4 == 0) { part[qv] = mrun[f]; part[AQ + qv] = lrun[f]; }
+      if (part && wave == 0 && g4 == 0) { part[qv] = mrun[f]; part[a.sq + qv] = lrun[f]; }
     }
     s0 = s1;
   }
@@ -464,7 +464,7 @@ struct SoftCap { float cap; __device__ __forceinline__ float operator()(float s)
 template <int NB, int KF, bool VEC>
 __global__ __launch_bounds__(256) void attn_latent_decode_kernel(AttnTArgs a) {
   using Walk = LatentWalk<NB, KF, VEC, SoftCap>;
-  constexpr int KT = Walk::KT, AQ = 16;
+  constexpr int KT = Walk::KT;
   __shared__ __attribute__((aligned(16))) float lds[Walk::LDS_FLOATS];
   const int tid = threadIdx.x, b = blockIdx.x, gy = blockIdx.y, sp = blockIdx.z;
   const int rep = a.H / a.G, chunks = (rep + a.hpc - 1) / a.hpc;
@@ -482,7 +482,7 @@ __global__ __launch_bounds__(256) void attn_latent_decode_kernel(AttnTArgs a) {
   float mrun, lrun;
   Walk::run(lds, a.k + ((int64_t)seq * a.t_max + tF) * a.ldk + (int64_t)g * a.dim, a.ldk, a.dim, nk, nk, t0, t1, q, SoftCap{a.cap}, mrun, lrun, acc);
   if (c >= Rc) return;
-  float* part = a.nsplit > 1 ? a.part + (((int64_t)b * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)AQ * (2 + a.vdim)) : nullptr;
+  float* part = a.nsplit > 1 ? a.part + (((int64_t)b * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)a.sq * (2 + a.vdim)) : nullptr;
   const bool vec = emit_vec(a);
   const int64_t col0 = (int64_t)(h0 + c) * a.vdim;
   const float inv = part ? 1.f : a.out_scale * softmax_inv(mrun, lrun, a.sink, h0 + c);
@@ -494,7 +494,7 @@ __global__ __launch_bounds__(256) void attn_latent_decode_kernel(AttnTArgs a) {
     if (!part) { emit4(a, r, b, col0, d, vec); continue; }
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (d + e < a.vdim) part[2 * AQ + (int64_t)c * a.vdim + d + e] = r[e];
+      if (d + e < a.vdim) part[2 * a.sq + (int64_t)c * a.vdim + d + e] = r[e];
   }
-  if (part && wave == 0 && g4 == 0) { part[c] = mrun; part[AQ + c] = lrun; }
+  if (part && wave == 0 && g4 == 0) { part[c] = mrun; part[a.sq + c] = lrun; }
 }

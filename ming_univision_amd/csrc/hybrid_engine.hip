@@ -102,7 +102,7 @@ HPlan make_plan(const mn_hyb_model* m, int M) {
     if (d.n_gate > p.gate) p.gate = d.n_gate;
     if (d.n_beta > p.beta) p.beta = d.n_beta;
     if (l.kind == MN_HYB_ATTENTION) {
-      const size_t aw = (size_t)4 * mn_num_cus() * 64 * (2 + (size_t)l.vdim) * sizeof(float);
+      const size_t aw = mn_window_attn_scratch_bytes(M, l.heads, l.kv_heads, l.dim, l.vdim, 0);
       if (aw > p.attn_ws) p.attn_ws = aw;
     } else if (l.kind == MN_HYB_TALK_ATTENTION) {                // (runs x splits) of a launch stay near two workgroups per compute unit
       const size_t aw = mn_talk_attn_workspace_bytes(mn_num_cus(), l.heads, l.kv_heads, l.dim, M > 1 && m->block_rows > 0 ? m->block_rows : 1, 2);
@@ -296,7 +296,7 @@ extern "C" int mn_hyb_step(const mn_hyb_model* m, const mn_hyb_state* st, const 
     if (attn) {
       MN_TRY(mn_head_norm_temp_append(pin, d.n_in, M, l.heads, l.kv_heads, l.dim, l.vdim, l.q_norm, l.k_norm, m->eps, l.scale, l.temp_coef,
                                       l.temp_every, row_seq, row_slot, qf, d.cq, st->k[ri], st->v[ri], st->t_max, stream));
-      int ns = mn_window_attn_splits(n_blk, l.heads, l.kv_heads, one_row, max_len);
+      int ns = mn_window_attn_splits_heads(n_blk, l.heads, l.kv_heads, one_row, max_len, 64, l.dim, l.vdim, 0);
       while (ns > 1 && mn_window_attn_workspace_bytes(n_blk, l.heads, l.kv_heads, l.vdim, one_row, ns) > p.attn_ws) --ns;
       MN_TRY(mn_window_pool_attn_blocks_sink(qf, d.cq, st->k[ri], st->v[ri], nullptr, nullptr, l.sink, row_seq, row_slot, blk_tab, n_blk, one_row,
                                              l.heads, l.kv_heads, l.dim, l.vdim, st->t_max, 1, 0, 0, 1.0f, cat, d.n_cat, cath, d.n_cat, ns, aws,

@@ -64,8 +64,7 @@ MPlan make_plan(const mn_ms_model* m, int M) {
     const MDims d = mdims(l);
     up(p.n_in, d.n_in); up(p.cq, d.cq); up(p.cv, d.cv); up(p.hv, d.hv); up(p.n_router, d.n_router);
     if (l.experts > 0) { up(p.top, l.top); up(p.ff, l.expert_ff); up(p.experts, l.experts); }
-    // key splits are chosen so that a launch has about two workgroups per compute unit: (workgroups of 64 query vectors x splits) stays below four
-    const size_t aw = (size_t)4 * mn_num_cus() * 64 * (2 + (size_t)l.vdim) * sizeof(float);
+    const size_t aw = mn_window_attn_scratch_bytes(M, l.heads, l.kv_heads, l.dim, l.vdim, 0);
     if (aw > p.attn_ws) p.attn_ws = aw;
     if (m->arith == MN_SEQ_ARITH_BF16 && M > 8 && M <= 64) {       // scratch of the weight-streaming MFMA route: the largest product of the stack
       const int W = m->width;
@@ -200,7 +199,7 @@ extern "C" int mn_ms_step(const mn_ms_model* m, const mn_ms_state* st, const flo
     int keys = max_len;
     if (l.window > 0 && l.window + 3 < keys) keys = l.window + 3;
     if (l.chunk > 0 && l.chunk + 3 < keys) keys = l.chunk + 3;
-    int ns = mn_window_attn_splits(n_blk, H, G, one_row, keys);
+    int ns = mn_window_attn_splits_heads(n_blk, H, G, one_row, keys, 64, l.dim, l.vdim, 0);
     while (ns > 1 && mn_window_attn_workspace_bytes(n_blk, H, G, l.vdim, one_row, ns) > p.attn_ws) --ns;
     const bool cat16_only = cath && mfma_ok(l.w_o, d.hv);
     MN_TRY(mn_window_pool_attn_blocks_gate(qf, d.cq, st->k[li], 0, st->v[li], 0, nullptr, nullptr, l.sink, 0.0f, l.chunk,

@@ -59,8 +59,7 @@ PPlan make_plan(const mn_pmix_model* m, int M) {
     if (l.top > p.top) p.top = l.top;
     if (l.ff > p.ff) p.ff = l.ff;
     if (l.experts > p.experts) p.experts = l.experts;
-    // key splits are chosen so that a launch has about two workgroups per compute unit: (workgroups of 64 query vectors x splits) stays below four
-    const size_t aw = (size_t)4 * mn_num_cus() * 64 * (2 + (size_t)l.vdim) * sizeof(float);
+    const size_t aw = mn_window_attn_scratch_bytes(M, l.heads, l.kv_heads, l.dim, l.vdim, 0);
     if (aw > p.attn_ws) p.attn_ws = aw;
     const size_t gw = mn_mingru_scan_workspace_bytes(M, l.gru);
     if (gw > p.gru_ws) p.gru_ws = gw;
@@ -243,7 +242,7 @@ extern "C" int mn_pmix_step(const mn_pmix_model* m, const mn_pmix_state* st, con
         max_keys = l.window + rb - 1 < max_len ? l.window + rb - 1 : max_len;
         if (l.pool > 0) max_keys += max_len / l.pool;
       }
-      int ns = mn_window_attn_splits(n_blk, l.heads, l.kv_heads, one_row, max_keys);
+      int ns = mn_window_attn_splits_heads(n_blk, l.heads, l.kv_heads, one_row, max_keys, 64, l.dim, l.vdim, 0);
       while (ns > 1 && mn_window_attn_workspace_bytes(n_blk, l.heads, l.kv_heads, l.vdim, one_row, ns) > p.attn_ws) --ns;
       MN_TRY(mn_window_pool_attn_blocks(qf, d.cq, st->k[ri], st->v[ri], st->pk[ri], st->pv[ri], row_seq, row_slot, blk_tab, n_blk, one_row,
                                         l.heads, l.kv_heads, l.dim, l.vdim, st->t_max, st->n_pool_max, l.window, l.pool, l.left_scale, cat,

@@ -562,6 +562,7 @@ struct AttnTArgs {
   int64_t ldk, ldv;     // row strides of the key and value arenas (>= G * dim, G * vdim): a value arena may be a view into the key arena
   int chunk;            // > 0: a position sees only its own chunk of `chunk` positions, counted from position 0 of the sequence
   const float* gate; int64_t ldg;   // optional [M, H * vdim]: every result is multiplied by the sigmoid of its gate
+  int sq;               // query vectors of a run's slab of partial results (rows x heads of a chunk): [sq] maxima, [sq] sums, [sq][vdim]
 };
 
 __device__ __forceinline__ float gated(const AttnTArgs& a, float val, int row, int64_t col) {
@@ -731,8 +732,8 @@ __global__ __launch_bounds__(256) void window_attn_tiled_kernel(AttnTArgs a) {
     __syncthreads();
   }
   // ---- the key shares of a column meet in LDS; then the result, or this split's part of it ----
-  float* part_out = a.nsplit > 1 ? a.part + (((int64_t)b * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)AQ * (2 + a.vdim)) : nullptr;
-  if (part_out && tid < AQ) { part_out[tid] = st_m[tid]; part_out[AQ + tid] = st_l[tid]; }
+  float* part_out = a.nsplit > 1 ? a.part + (((int64_t)b * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)a.sq * (2 + a.vdim)) : nullptr;
+  if (part_out && tid < a.sq) { part_out[tid] = st_m[tid]; part_out[a.sq + tid] = st_l[tid]; }
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb) {
     const int c0 = cb * 256;
@@ -748,7 +749,7 @@ __global__ __launch_bounds__(256) void window_attn_tiled_kernel(AttnTArgs a) {
       float t = 0.f;
       for (int u = 0; u < nsub; ++u) t += red[(u * AQ + i) * cw + cc];
       if (part_out) {
-        part_out[2 * AQ + (int64_t)i * a.vdim + c0 + cc] = t;
+        part_out[2 * a.sq + (int64_t)i * a.vdim + c0 + cc] = t;
       } else {
         const int64_t col = (int64_t)(h0 + i % Rc) * a.vdim + c0 + cc;
         const int row = r0 + i / Rc;
@@ -775,16 +776,16 @@ __global__ __launch_bounds__(256) void window_attn_merge_kernel(AttnTArgs a) {
   const int r0 = a.blk_tab ? a.blk_tab[2 * b] : b;
   const int nr = a.blk_tab ? min(a.blk_tab[2 * b + 1], a.rows_per_blk) : 1;
   const int nqv = nr * Rc;
-  const int64_t stride = (int64_t)AQ * (2 + a.vdim);
+  const int64_t stride = (int64_t)a.sq * (2 + a.vdim);
   const float* base = a.part + ((int64_t)b * gridDim.y + gy) * a.nsplit * stride;
   // the weight of every (vector, split) once per workgroup: exp(its maximum - the overall maximum), and the vectors' normalisers
   __shared__ float wgt[AQ * 64];
   __shared__ float Ls[AQ], Ms[AQ];
-  for (int i = tid >> 6; i < AQ; i += 4) {            // one wave per vector, one lane per split (at most 64)
+  for (int i = tid >> 6; i < a.sq; i += 4) {          // one wave per vector, one lane per split (at most 64)
     const int lane = tid & 63;
     const bool on = lane < a.nsplit;
     const float ms = on ? base[lane * stride + i] : -INFINITY;
-    const float ls = on ? base[lane * stride + AQ + i] : 0.f;
+    const float ls = on ? base[lane * stride + a.sq + i] : 0.f;
     const float mx = wave_max(ms);
     const float w = ms == -INFINITY ? 0.f : expf(ms - mx);
     wgt[i * 64 + lane] = w;
@@ -795,7 +796,7 @@ __global__ __launch_bounds__(256) void window_attn_merge_kernel(AttnTArgs a) {
   const int c0 = blockIdx.z * MERGE_COLS, cw = min(MERGE_COLS, a.vdim - c0);     // this workgroup's slice of the value columns
   for (int e = tid; e < nqv * cw; e += 256) {
     const int i = e / cw, c = c0 + e - i * cw;
-    const float* src = base + 2 * AQ + (int64_t)i * a.vdim + c;
+    const float* src = base + 2 * a.sq + (int64_t)i * a.vdim + c;
     float t = 0.f;
 #pragma unroll 4
     for (int s = 0; s < a.nsplit; ++s) t = fmaf(src[s * stride], wgt[i * 64 + s], t);
@@ -1106,7 +1107,7 @@ extern "C" int mn_window_pool_attn(const float* q, int64_t ldq, const float* k_a
 extern "C" int mn_window_attn_block_rows(void) { return 4; }
 
 namespace {
-struct AttnShape { int aq, rows, hpc, chunks; };
+struct AttnShape { int aq, rows, hpc, chunks, sq; };
 AttnShape attn_shape(int H, int G, int one_row) {
   AttnShape s;
   const int rep = H / G;
@@ -1114,6 +1115,7 @@ AttnShape attn_shape(int H, int G, int one_row) {
   s.aq = (one_row && rep <= 4) ? 4 : 16;
   s.hpc = s.aq / s.rows;
   s.chunks = (rep + s.hpc - 1) / s.hpc;
+  s.sq = s.rows * (rep < s.hpc ? rep : s.hpc);
   return s;
 }
 // attn_rows.inl: heads side by side in a wave's 16 query vectors, and the runs of a workgroup
@@ -1121,17 +1123,28 @@ int attn_rows_heads(int rep) { return rep >= 3 ? 4 : rep; }
 int attn_rows_runs(int rep) { return 4 * (16 / attn_rows_heads(rep)) / 4; }
 }  // namespace
 
+// query vectors of a workgroup on runs of rows: 64 on the matrix cores (32 where the values lie inside the keys), a run on the FMA kernel
+static int attn_run_vectors(int dim, int vdim, int vk) { return vk ? (dim <= 640 ? 32 : 16) : (dim <= 256 && vdim <= 256 ? 64 : 16); }
+
 extern "C" int mn_window_attn_splits(int n_blk, int H, int G, int one_row, int max_keys) {
   return mn_window_attn_splits_tile(n_blk, H, G, one_row, max_keys, AKT);
 }
-
 extern "C" int mn_window_attn_splits_tile(int n_blk, int H, int G, int one_row, int max_keys, int key_tile) {
+  return mn_window_attn_splits_heads(n_blk, H, G, one_row, max_keys, key_tile, 64, 64, 0);
+}
+
+// Two workgroups a CU.  What a workgroup is follows from the kernel that serves such heads (us by splits, the request marked: keys of 320, 16 heads, 353 runs of
+// 5 prompts 1: 120*, 2: 150, 3: 156; 8 heads 1: 96, 2: 96*, 3: 90; 4 heads x 2048 tokens 1: 313, 2: 186*, 4: 220; one prompt of 600, 8 heads 3: 64, 4: 62*, 6: 70;
+// heads of 64, 8 of 1000 tokens 3: 43, 4: 39*, 6: 44).
+extern "C" int mn_window_attn_splits_heads(int n_blk, int H, int G, int one_row, int max_keys, int key_tile, int dim, int vdim, int vk) {
   if (n_blk < 1 || H < 1 || G < 1 || (H % G) != 0 || max_keys < 1 || key_tile < 1) return 1;
   const AttnShape sh = attn_shape(H, G, one_row);
-  const int64_t wgs = mn_cdiv(n_blk, one_row ? 1 : attn_rows_runs(H / G)) * G * sh.chunks, tiles = mn_cdiv(max_keys, key_tile);
+  const int vec = one_row ? 16 : attn_run_vectors(dim, vdim, vk);
+  const int64_t runs = vec == 16 ? 1 : attn_rows_runs(H / G) * vec / 64;
+  const int64_t wgs = mn_cdiv(n_blk, runs) * G * sh.chunks, tiles = mn_cdiv(max_keys, key_tile);
   int64_t ns = mn_cdiv(2 * (int64_t)mn_num_cus(), wgs);
-  // (a workgroup of 64 vectors has some 10 us of its own: a split of its walk below 128 keys costs more than it saves)
-  const int64_t most = one_row ? tiles : mn_cdiv(max_keys, 128);
+  // (a workgroup of 32 or 64 vectors has some 10 us of its own: a split of its walk below 128 keys costs more than it saves)
+  const int64_t most = vec == 16 ? tiles : mn_cdiv(max_keys, 128);
   if (ns > most) ns = most;
   if (ns > tiles) ns = tiles;
   if (ns > 64) ns = 64;
@@ -1141,7 +1154,16 @@ extern "C" int mn_window_attn_splits_tile(int n_blk, int H, int G, int one_row, 
 extern "C" size_t mn_window_attn_workspace_bytes(int n_blk, int H, int G, int vdim, int one_row, int nsplit) {
   if (nsplit <= 1 || n_blk < 1 || H < 1 || G < 1 || (H % G) != 0) return 0;
   const AttnShape sh = attn_shape(H, G, one_row);
-  return (size_t)n_blk * G * sh.chunks * nsplit * sh.aq * (2 + (size_t)vdim) * sizeof(float);
+  return (size_t)n_blk * G * sh.chunks * nsplit * sh.sq * (2 + (size_t)vdim) * sizeof(float);
+}
+
+// What the request above needs at most in a step of M rows: workgroups x splits stay below four a CU (and splits at 64), a workgroup's vectors are a slab each.
+extern "C" size_t mn_window_attn_scratch_bytes(int M, int H, int G, int dim, int vdim, int vk) {
+  if (M < 1 || H < 1 || G < 1 || (H % G) != 0) return 0;
+  const AttnShape run = attn_shape(H, G, 0), one = attn_shape(H, G, 1);
+  const size_t rows = (size_t)M * G * 64, a = rows * run.chunks * run.sq, b = rows * one.chunks * one.sq;
+  const size_t most = (size_t)4 * mn_num_cus() * attn_run_vectors(dim, vdim, vk), need = a > b ? a : b;
+  return (need < most ? need : most) * (2 + (size_t)vdim) * sizeof(float);
 }
 
 extern "C" int mn_window_pool_attn_blocks(const float* q, int64_t ldq, const float* k_arena, const float* v_arena, const float* pk,
@@ -1212,7 +1234,7 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
                "mn_window_pool_attn_blocks: workspace too small");
   AttnTArgs a{q, ldq, k_arena, v_arena, pool ? pk : nullptr, pool ? pv : nullptr, row_seq, row_slot, one_row ? nullptr : blk_tab, H, G, dim, vdim,
               t_max, n_pool_max, window, pool, sh.rows, sh.hpc, nsplit, out_scale, out, ldo, out16, ldo16, (float*)workspace, sink, softcap, ldk, ldv,
-              chunk, gate, ldgate};
+              chunk, gate, ldgate, sh.sq};
   // values that are a view of the keys (one key/value head, the same arena and stride): the matrix-core kernel stages one tile for both
   const bool vk = G == 1 && k_arena == v_arena && ldk == ldv && vdim <= dim && !pool;
   const bool mfma_fits = vk ? (dim <= 640 && sh.aq == 16) : (!one_row && dim <= 256 && vdim <= 256);

@@ -68,7 +68,7 @@ PPlan make_plan(const mn_pn_model* m, int M) {
     const PDims d = pdims(l);
     up(p.n_in, d.n_in); up(p.nq, d.nq); up(p.nmid, d.nmid); up(p.hv, d.hv); up(p.ff, l.ff); up(p.side, pad8(l.side)); up(p.heads, l.heads);
     if (l.kind != MN_PN_DELTA) {
-      const size_t aw = (size_t)4 * mn_num_cus() * 64 * (2 + (size_t)d.avd) * sizeof(float);
+      const size_t aw = mn_window_attn_scratch_bytes(M, l.heads, l.kind == MN_PN_LATENT ? 1 : l.kv_heads, d.akd, d.avd, l.kind == MN_PN_LATENT);
       if (aw > p.attn_ws) p.attn_ws = aw;
     }
     if (m->arith == MN_SEQ_ARITH_BF16 && M > 8 && M <= 64) {       // scratch of the weight-streaming MFMA route: the largest product of the stack
@@ -185,7 +185,7 @@ extern "C" int mn_pn_step(const mn_pn_model* m, const mn_pn_state* st, const flo
       int keys = max_len;
       if (l.window > 0 && l.window + 3 < keys) keys = l.window + 3;
       // latent attention's decode rows run on the matrix-core kernel (all heads of a row in one workgroup): its key tiles hold 16 keys
-      int ns = mn_window_attn_splits_tile(n_blk, H, G, one_row, keys, latent && one_row ? 16 : 64);
+      int ns = mn_window_attn_splits_heads(n_blk, H, G, one_row, keys, latent && one_row ? 16 : 64, d.akd, d.avd, latent);
       if (latent && one_row && (int64_t)ns * d.avd > 16384) ns = 16384 / d.avd > 1 ? 16384 / d.avd : 1;   // the merge reads ns x 16 x avd partial sums a row
       while (ns > 1 && mn_window_attn_workspace_bytes(n_blk, H, G, d.avd, one_row, ns) > p.attn_ws) --ns;
       const bool gate = attn && l.has_gate;

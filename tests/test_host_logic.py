@@ -144,6 +144,33 @@ def test_split_of_the_e4m3_product_follows_its_own_tiles():
     assert plan(41, 1024, 4096) == 16 and 1 <= plan(2048, 1024, 4096) <= 6 and plan(64, 256, 128) == 1
 
 
+def test_key_splits_of_attention_runs_and_their_scratch():
+    """mn_window_attn_splits_heads counts the workgroups of the kernel that serves the heads (64 query vectors, 32 where the values lie inside the keys, a run of 4 rows
+    beyond 256 values): one split once they are two a CU, more below; mn_window_attn_scratch_bytes holds what the request needs whatever the heads a key head, and a
+    workspace for more rows serves fewer."""
+    import ctypes
+    from ming_univision_amd import _lib
+    L = ctypes.CDLL(_lib.LIB_PATH)
+    L.mn_window_attn_scratch_bytes.restype = L.mn_window_attn_workspace_bytes.restype = ctypes.c_size_t
+    splits, need, have = L.mn_window_attn_splits_heads, L.mn_window_attn_workspace_bytes, L.mn_window_attn_scratch_bytes
+    assert splits(353, 16, 1, 0, 470, 64, 320, 256, 1) == 1 and splits(353, 8, 1, 0, 470, 64, 320, 256, 1) == 2         # 708 and 354 workgroups of 32
+    assert splits(353, 8, 8, 0, 470, 64, 320, 320, 0) == 1 and splits(20, 4, 1, 0, 1000, 64, 320, 320, 0) == 16         # runs of their own: by their count, down to 64 keys
+    assert splits(353, 16, 4, 0, 470, 64, 128, 128, 0) == 2 and splits(353, 16, 4, 0, 200, 64, 128, 128, 0) == 2        # 356 of 64
+    assert splits(512, 16, 1, 0, 2048, 64, 128, 128, 0) == L.mn_window_attn_splits(512, 16, 1, 0, 2048)
+    last = {}
+    for H, G, d, e, vk in ((16, 16, 64, 64, 0), (16, 8, 128, 128, 0), (16, 4, 128, 128, 0), (12, 4, 96, 200, 0), (5, 1, 64, 512, 1), (16, 1, 576, 512, 1), (2, 1, 320, 256, 1),
+                           (8, 2, 300, 512, 0), (1, 1, 64, 64, 0), (20, 1, 128, 128, 0)):
+        for M in (1, 2, 5, 33, 64, 65, 130, 300, 511, 1000, 2048, 5000):
+            got = have(M, H, G, d, e, vk)
+            assert got >= last.get((H, G, d, e, vk), 0)
+            last[(H, G, d, e, vk)] = got
+            for n_blk, one_row in ((-(-M // 4), 0), (M, 0), (M, 1)):
+                for keys in (1, 100, 2048, 100000):
+                    for tile in (16, 64):
+                        ns = splits(n_blk, H, G, one_row, keys, tile, d, e, vk)
+                        assert 1 <= ns <= 64 and need(n_blk, H, G, e, one_row, ns) <= got, (H, G, d, e, vk, M, n_blk, one_row, keys, ns)
+
+
 def test_config_shapes_and_sizes():
     cfg = C.MingUniVisionConfig.ming_univision_16b_a3b()
     n_llm = sum(int(torch.tensor(s).prod()) for s in C.llm_param_shapes(cfg.llm_config).values())

@@ -57,9 +57,10 @@ HDims hdims(const mn_hyb_layer& l) {
   return d;
 }
 
-// rows of the joined output product's buffer where it may come in slabs: as many for every row count, so that a workspace for more rows serves fewer
+// rows of the joined output product's buffer where it may come in slabs: 16 slabs (the most that are asked for), up to 8192 rows in all; never fewer for more rows,
+// so that a workspace for more rows serves fewer
 constexpr int SLAB_ROWS = 8192;
-inline size_t out_rows(bool slabs, int M) { return slabs && M < SLAB_ROWS ? (size_t)SLAB_ROWS : (size_t)M; }
+inline int out_rows(bool slabs, int M) { return !slabs || M >= SLAB_ROWS ? M : (M > SLAB_ROWS / 16 ? SLAB_ROWS : 16 * M); }
 
 struct HPlan {
   int n_in = 1, cq = 1, hv = 1, n_cat = 1, top = 1, eff = 1, eup = 1, experts = 1, dec = 1, gate = 1, beta = 1;
@@ -149,7 +150,7 @@ extern "C" size_t mn_hyb_workspace_bytes(const mn_hyb_model* m, int M) {
   n += al(R * p.cq * 4);                               // queries
   n += al(R * p.hv * 4);                               // the recurrence's heads before their norm
   n += al(R * p.n_cat * 4) + al(R * p.n_cat * 2);      // [mixer | activation] + bf16
-  n += al(out_rows(p.slabs, M) * W * 4);               // their joined output product
+  n += al((size_t)out_rows(p.slabs, M) * W * 4);               // their joined output product
   n += 2 * al(Z * 4);                                  // chosen experts, weights
   n += al(Z * p.eup * 4);                              // [gate ; up] or up of the pairs
   n += al(Z * p.eff * 4) + al(Z * p.eff * 2);          // their activation + bf16
@@ -190,7 +191,7 @@ extern "C" int mn_hyb_step(const mn_hyb_model* m, const mn_hyb_state* st, const 
   float* lo = (float*)take(R * p.hv * 4);
   float* cat = (float*)take(R * p.n_cat * 4);
   uint16_t* cath = (uint16_t*)take(R * p.n_cat * 2);
-  float* yf = (float*)take(out_rows(p.slabs, M) * W * 4);
+  float* yf = (float*)take((size_t)out_rows(p.slabs, M) * W * 4);
   int32_t* tidx = (int32_t*)take(Zmax * 4);
   float* tw = (float*)take(Zmax * 4);
   float* gu = (float*)take(Zmax * p.eup * 4);
@@ -363,7 +364,7 @@ extern "C" int mn_hyb_step(const mn_hyb_model* m, const mn_hyb_state* st, const 
     }
     int nz = 0;
     if (!layer_norm && !moe && p.slabs)
-      MN_TRY(linear_slabs(arith, M, cath, d.n_cat, l.w_out, W, d.n_cat, linear_slices(arith, M, W, d.n_cat, SLAB_ROWS / M), yf, stream, &nz));
+      MN_TRY(linear_slabs(arith, M, cath, d.n_cat, l.w_out, W, d.n_cat, linear_slices(arith, M, W, d.n_cat, out_rows(true, M) / M), yf, stream, &nz));
     if (nz == 0) MN_TRY(linear(arith, M, cat, d.n_cat, cath, d.n_cat, l.w_out, W, d.n_cat, nullptr, yf, W, gws, gwb, stream));
     pend.y = yf;
     pend.nz = nz > 0 ? nz : 1;

@@ -171,6 +171,26 @@ def test_key_splits_of_attention_runs_and_their_scratch():
                         assert 1 <= ns <= 64 and need(n_blk, H, G, e, one_row, ns) <= got, (H, G, d, e, vk, M, n_blk, one_row, keys, ns)
 
 
+def test_scratch_of_a_hybrid_prompt_grows_with_its_rows():
+    """mn_hyb_workspace_bytes: the output product's slabs are 16 times the step's rows up to 8192 in all, not 8192 rows from 65 on; never less for more prompt
+    rows."""
+    import ctypes
+    from ming_univision_amd import _lib
+    L = ctypes.CDLL(_lib.LIB_PATH)
+    L.mn_hyb_workspace_bytes.restype = ctypes.c_size_t
+    layer = (_lib.HybLayer * 1)()
+    ly, W = layer[0], 2048
+    ly.kind, ly.heads, ly.kv_heads, ly.dim, ly.vdim, ly.ff_kind, ly.ff = 0, 16, 4, 128, 128, 1, 4096
+    m = _lib.HybModel(width=W, n_layers=1, n_runs=1, arith=0, norm=0, block_rows=4)
+    m.layers = ctypes.cast(layer, ctypes.POINTER(_lib.HybLayer))
+    m.run_layer = (ctypes.c_int32 * 1)(0)
+    size = [L.mn_hyb_workspace_bytes(ctypes.byref(m), M) for M in (1, 64, 65, 100, 511, 512, 513, 2048, 8191, 8192, 8193)]
+    assert size[:2] == sorted(size[:2]) and size[2:] == sorted(size[2:]) and size[0] > 0      # (up to 64 rows there is the streaming products' scratch instead)
+    m.arith = 1                                           # fp32 arithmetic has no slabs: what is left of the difference is the bf16 copies
+    plain = [L.mn_hyb_workspace_bytes(ctypes.byref(m), M) for M in (64, 65, 512)]
+    assert size[2] - plain[1] < 16 * 65 * W * 4 + (4 << 20) and size[5] - plain[2] > 8192 * W * 4 - 512 * W * 4
+
+
 def test_config_shapes_and_sizes():
     cfg = C.MingUniVisionConfig.ming_univision_16b_a3b()
     n_llm = sum(int(torch.tensor(s).prod()) for s in C.llm_param_shapes(cfg.llm_config).values())

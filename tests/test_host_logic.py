@@ -188,7 +188,7 @@ def test_scratch_of_a_hybrid_prompt_grows_with_its_rows():
     assert size[:2] == sorted(size[:2]) and size[2:] == sorted(size[2:]) and size[0] > 0      # (up to 64 rows there is the streaming products' scratch instead)
     m.arith = 1                                           # fp32 arithmetic has no slabs: what is left of the difference is the bf16 copies
     plain = [L.mn_hyb_workspace_bytes(ctypes.byref(m), M) for M in (64, 65, 512)]
-    assert size[2] - plain[1] < 16 * 65 * W * 4 + (4 << 20) and size[5] - plain[2] > 8192 * W * 4 - 512 * W * 4
+    assert size[2] - plain[1] < 16 * 65 * W * 4 + (4 << 20) and size[5] - plain[2] >= 8192 * W * 4 - 512 * W * 4
 
 
 def test_config_shapes_and_sizes():

@@ -540,6 +540,8 @@ MN_API int mn_rows_advance(int32_t* a, int32_t* b, int32_t* c, int M, int delta,
  * [dim, hidden], b.  gelu 0: up = [2 hidden, dim] gate rows then up rows (SwiGLU); 1: up [hidden, dim] (exact-erf GELU).
  * precise 0: bf16 operands; out bf16 [B * T, dim] = LayerNorm(x; fin_g, fin_b), then GELU if fin_gelu.  precise 1: hi / lo operands (fp32-class), hidden a
  * multiple of 64, out NULL (the caller norms x).  workspace: mn_vit_blocks_workspace_bytes, 256-byte aligned. */
+/* Split-K slices of a block's product onto the residual stream whose 256 x 256 tiles would leave more than half of the chip idle; 0: one launch adds to the stream. */
+MN_API int mn_vit_resid_slices(int M, int N, int K);
 MN_API size_t mn_vit_blocks_workspace_bytes(int B, int T, int dim, int hidden, int gelu, int precise);
 MN_API int mn_vit_blocks(float* x, int B, int T, int dim, int depth, const uint16_t* const* w, int hidden, int gelu, int causal, int precise, float eps,
                          const uint16_t* fin_g, const uint16_t* fin_b, int fin_gelu, uint16_t* out, void* workspace, size_t workspace_bytes,

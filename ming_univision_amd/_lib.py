@@ -368,6 +368,7 @@ SYMBOLS = {
     "mn_lmhead_argmax_workspace_bytes": (_sz, [_i, _i, _i]),
     "mn_lmhead_argmax": (_i, [_p, _i64, _i, _p, _i64, _i, _i, _i64, _p, _p, _p, _sz, _p]),
     "mn_sample_logits": (_i, [_p, _i64, _i, _i, _f, _i, _f, _p, _i64, _p, _p, _p]),
+    "mn_vit_resid_slices": (_i, [_i, _i, _i]),
     "mn_vit_blocks_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _i]),
     "mn_vit_blocks": (_i, [_p, _i, _i, _i, _i, PP, _i, _i, _i, _i, _f, _p, _p, _i, _p, _p, _sz, _p]),
     "mn_semdec_workspace_bytes": (_sz, [C.POINTER(SemDec), _i, _i64]),

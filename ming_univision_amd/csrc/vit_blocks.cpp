@@ -7,7 +7,7 @@ namespace {
 
 size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-// Slices of a residual product whose 256 x 256 tiles would leave more than half of the chip idle, 0: one launch adds to the stream
+// Slices of a residual product (mn_vit_resid_slices), for any number of rows
 int resid_slices(int64_t M, int N, int K) {
   const int64_t tiles = mn_cdiv(M, 256) * mn_cdiv(N, 256);
   if (tiles >= 128 || K < 512 || (K % 64) || (N % 4)) return 0;
@@ -40,6 +40,8 @@ Plan plan(int64_t M, int dim, int hidden, int gelu, int precise) {
 #define TRY(e) do { const int rc_ = (e); if (rc_ < 0) return rc_; } while (0)
 
 }  // namespace
+
+extern "C" int mn_vit_resid_slices(int M, int N, int K) { return M < 1 || N < 1 || K < 1 ? 0 : resid_slices(M, N, K); }
 
 extern "C" size_t mn_vit_blocks_workspace_bytes(int B, int T, int dim, int hidden, int gelu, int precise) {
   return B < 1 || T < 1 || dim < 1 || hidden < 1 ? 0 : plan((int64_t)B * T, dim, hidden, gelu, precise).total;

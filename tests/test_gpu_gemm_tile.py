@@ -7,7 +7,7 @@ import torch.nn.functional as F
 
 pytestmark = pytest.mark.gpu
 
-# (M, N, K): each of the plain forms (64 x 64, 64 x 128, 128 x 128 once and twice per CU) and of the hi/lo ones is the choice of one of them
+# (M, N, K): what the rule makes of them (64 x 64, 64 x 128 and two-per-CU 128 x 128 tiles; 128 x 128 of eight waves for SwiGLU only); test_every_form has the rest
 SHAPES = [(1, 4, 64), (63, 60, 128), (64, 64, 192), (65, 68, 256), (65, 3072, 320), (129, 132, 576), (200, 1028, 1024), (300, 3076, 512),
           (520, 2736, 1024), (1025, 1024, 1024), (1025, 3072, 256), (1409, 3200, 128), (2048, 3072, 192), (2100, 2052, 2048), (33, 32004, 64)]
 
@@ -49,6 +49,45 @@ def test_forms(M, N, K):
         else:
             assert rel(ops.gemm256_swiglu(a1, w, b), act) < 2 ** -8
 
+
+
+@pytest.fixture
+def dev_lib():
+    """The same code with the switches of mingnative_dev.h, in the place of the product library."""
+    import ctypes
+    import os
+    from ming_univision_amd import _lib
+    shipped = _lib.lib()
+    handle = ctypes.CDLL(os.path.join(os.path.dirname(_lib.LIB_PATH), "libmingnative_dev.so"))
+    for name, (res, args) in _lib.SYMBOLS.items():
+        fn = getattr(handle, name)
+        fn.restype, fn.argtypes = res, args
+    _lib._lib = handle
+    yield handle
+    handle.mn_gemm_tile_tune(-1)
+    _lib._lib = shipped
+
+
+@pytest.mark.parametrize("form", [0, 1, 2, 3, 4])
+def test_every_form(dev_lib, form):
+    """Each tile form in turn (0: 256 x 256) on rows and columns that end inside its tiles, one to five K-tiles and more than its pipeline holds, and the activations in
+    the epilogues with a tail that begins and ends inside a tile.  (Hi / lo rows have no form 4: the 256-tile kernel takes them.)"""
+    dev_lib.mn_gemm_tile_tune(form)
+    for M, N, K in ((1, 4, 64), (63, 60, 128), (65, 68, 192), (129, 132, 256), (257, 260, 320), (300, 516, 64), (200, 1028, 1024)):
+        test_forms(M, N, K)
+    for M, width, ff in ((65, 64, 96), (130, 128, 516), (300, 64, 1028)):
+        test_activations_in_the_products_epilogue(M, width, ff)
+
+
+def test_activations_on_the_large_tiles():
+    """A prompt wide enough for the 256 x 256 tiles under the rule."""
+    test_activations_in_the_products_epilogue(2048, 2048, 4096)
+
+
+@pytest.mark.parametrize("M,N,K", [(16380, 1020, 1024), (4100, 4100, 2048)])
+def test_rule_picks_the_large_tiles(M, N, K):
+    """A round of 256 x 256 tiles and more with ragged last rows and columns, every epilogue."""
+    test_forms(M, N, K)
 
 
 @pytest.mark.parametrize("M,width,ff", [(65, 64, 96), (130, 128, 516), (300, 64, 1028), (70, 128, 102)])

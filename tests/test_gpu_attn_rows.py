@@ -1,5 +1,5 @@
 """Attention of runs of rows (attn_rows.inl) at the sizes where its grouping can go wrong: row counts around 16 / 32 / 64 vectors, several sequences
-and cached tokens in one workgroup, head groups of every width, windows, chunks, pooled blocks' tiles, key splits, values inside keys.  The
+and cached tokens in one workgroup, head groups of every width, windows, chunks, tiles of pooled blocks, key splits, values inside keys.  The
 reference is a plain float64 softmax; fp32 products of up to 600 terms and exponentials at 1e-6: 1e-5 of the largest value."""
 import numpy as np
 import pytest
@@ -8,7 +8,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def run(spans, H, G, d, e, window, cap, chunk, vk, nsplit, t_max):
+def run(spans, H, G, d, e, window, cap, chunk, vk, nsplit, t_max, pool=0):
     from ming_univision_amd._lib import check, current_stream, lib, ptr
     from ming_univision_amd.sequences import rows_of_spans
     L = lib()
@@ -19,26 +19,33 @@ def run(spans, H, G, d, e, window, cap, chunk, vk, nsplit, t_max):
     q = torch.randn(M, H * d, generator=g) * d ** -0.5
     k = torch.randn(n_seq, t_max, G * d, generator=g)
     v = k if vk else torch.randn(n_seq, t_max, G * e, generator=g)
+    n_pool = t_max // pool if pool else 1
+    means = [x[:, :n_pool * pool].reshape(n_seq, n_pool, pool, -1).mean(2) for x in (k, v)] if pool else None
     ref, r = torch.empty(M, H, e, dtype=torch.float64), 0
     for s, n, past in spans:
         i, j = torch.arange(past, past + n)[:, None], torch.arange(past + n)[None]
         see = (j <= i) & ((i - j < window) if window else True) & ((i // chunk == j // chunk) if chunk else True)
+        keys, vals = k[s, :past + n], v[s, :past + n]
+        if pool:                                                    # the means of whole blocks before the window
+            see = torch.cat([torch.arange(n_pool)[None] < (i - window + 1).clamp(min=0) // pool, see], 1)
+            keys, vals = torch.cat([means[0][s], keys]), torch.cat([means[1][s], vals])
         for h in range(H):
             c = h // (H // G)
-            sc = q[r:r + n].reshape(n, H, d)[:, h].double() @ k[s, :past + n].reshape(-1, G, d)[:, c].double().T
+            sc = q[r:r + n].reshape(n, H, d)[:, h].double() @ keys.reshape(-1, G, d)[:, c].double().T
             sc = cap * torch.tanh(sc / cap) if cap else sc
-            vv = k[s, :past + n].reshape(-1, G, d)[:, c, :e] if vk else v[s, :past + n].reshape(-1, G, e)[:, c]
+            vv = vals.reshape(-1, G, d)[:, c, :e] if vk else vals.reshape(-1, G, e)[:, c]
             ref[r:r + n, h] = torch.softmax(sc.masked_fill(~see, -float("inf")), -1) @ vv.double()
         r += n
     kd, qd = k.cuda(), q.cuda()
     vd = kd if vk else v.cuda()
+    pk, pv = [x.contiguous().cuda() for x in means] if pool else (None, None)
     n_blk, ldv = dev["blk_tab"].shape[0], G * d if vk else G * e
     ns = nsplit or L.mn_window_attn_splits(n_blk, H, G, 0, tabs["max_len"])
     ws = torch.empty(max(16, L.mn_window_attn_workspace_bytes(n_blk, H, G, e, 0, ns)), dtype=torch.uint8, device="cuda")
     out = torch.full((M + 1, H * e), 7.0, device="cuda")
-    check(L.mn_window_pool_attn_blocks_gate(ptr(qd), H * d, ptr(kd), G * d, ptr(vd), ldv, None, None, None, cap, chunk, None, 0, ptr(dev["row_seq"]),
-                                            ptr(dev["row_slot"]), ptr(dev["blk_tab"]), n_blk, 0, H, G, d, e, t_max, 1, window, 0, 1.0, ptr(out), H * e,
-                                            None, 0, ns, ptr(ws), ws.numel(), -1, current_stream()), "attn")
+    check(L.mn_window_pool_attn_blocks_gate(ptr(qd), H * d, ptr(kd), G * d, ptr(vd), ldv, ptr(pk), ptr(pv), None, cap, chunk, None, 0, ptr(dev["row_seq"]),
+                                            ptr(dev["row_slot"]), ptr(dev["blk_tab"]), n_blk, 0, H, G, d, e, t_max, n_pool, window, pool, 1.0, ptr(out),
+                                            H * e, None, 0, ns, ptr(ws), ws.numel(), -1, current_stream()), "attn")
     assert bool((out[M] == 7.0).all())
     err = float((out[:M].double().cpu() - ref.reshape(M, -1)).abs().max() / ref.abs().max())
     assert err < 1e-5, err
@@ -52,6 +59,14 @@ SPANS = [[(0, 1, 0)], [(0, 63, 0)], [(0, 65, 7)], [(0, 3, 0), (1, 70, 0), (2, 1,
 def test_runs(spans, H, G, d, e):
     for window, cap, chunk, ns in ((0, 0.0, 0, 0), (33, 20.0, 0, 3), (0, 0.0, 48, 2), (200, 0.0, 0, 1)):
         run(spans, H, G, d, e, window, cap, chunk, False, ns, 256)
+
+
+@pytest.mark.parametrize("spans", SPANS)
+@pytest.mark.parametrize("H,G,d,e", [(4, 1, 64, 64), (8, 2, 128, 128), (6, 3, 72, 136), (5, 1, 34, 50)])
+def test_runs_with_pooled_blocks(spans, H, G, d, e):
+    """Block means before the window: tiles of means alone, of means and tokens, and rows of one tile that see different numbers of either."""
+    for window, pool, ns in ((33, 4, 0), (17, 16, 1), (40, 3, 3), (1, 1, 2)):
+        run(spans, H, G, d, e, window, 0.0, 0, False, ns, 256, pool)
 
 
 @pytest.mark.parametrize("spans", SPANS)

@@ -969,8 +969,8 @@ MN_API int mn_window_pool_attn_blocks(const float* q, int64_t ldq, const float* 
                                       float out_scale, float* out, int64_t ldo, uint16_t* out16, int64_t ldo16, int nsplit, void* workspace,
                                       size_t workspace_bytes, void* stream);
 /* The same with the kernel named: MN_WINDOW_ATTN_MFMA (what mn_window_pool_attn_blocks runs for runs of rows with dim, vdim <= 256) =
- * scores and weighted sums on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands and accumulation), 16-key tiles with
- * keys and values staged in LDS; MN_WINDOW_ATTN_VALU = the fp32 FMA kernel (decode rows, larger heads). */
+ * scores and weighted sums on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands and accumulation), 64 query vectors of a
+ * key/value head a workgroup, tiles of 16 or 32 keys and values staged in LDS; MN_WINDOW_ATTN_VALU = the fp32 FMA kernel (decode rows, larger heads). */
 enum { MN_WINDOW_ATTN_MFMA = 0, MN_WINDOW_ATTN_VALU = 1 };
 MN_API int mn_window_pool_attn_blocks_ex(const float* q, int64_t ldq, const float* k_arena, const float* v_arena, const float* pk,
                                          const float* pv, const int32_t* row_seq, const int32_t* row_slot, const int32_t* blk_tab, int n_blk,

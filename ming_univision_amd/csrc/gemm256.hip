@@ -445,7 +445,7 @@ extern "C" MN_DEV_API void mn_gemm256_tune_order(int group_m, int group_list) { 
 // workgroup of a CU, or whole rounds of `full` (forms that fit once: per = 0).  The fixed part is launch, first round trip and epilogue: 4 us
 // for the small tiles, 11 us + 7 per further round for the 256-tile kernel.
 // Where the lines then lie, both sides measured: 65 x 3072 x 1024 bf16: 7.3 us (64 x 64) against 23.7 (256); 256 x 4096 x 1024: 8.2 against
-// 32.1; 1025 hi/lo rows x 1024 x 1024: 12.4 against 25.0; x 3072: 20.5 (128 x 128) against 27.5; 2048 x 2048 x 8192: 79.6 (128 x 128) against 136.6;
+// 32.1; 1025 hi/lo rows x 1024 x 1024: 10.9 (64 x 64) against 22.3; x 3072: 20.0 (64 x 128) against 26.0; 2048 x 2048 x 8192: 79.6 (128 x 128) against 136.6;
 // 16384 x 1024 x 1024: 37.2 (256) against 54.2 (128 x 128); 1025 hi/lo rows x 2752 SwiGLU: 29.9 (256) against 37.8.
 struct TileForm { int form, bm, bn; double fixed, alone, full, two, per; };
 static const TileForm tile_plain[] = {{1, 64, 64, 3.6, 0.23, 0.26, 0.42, 0.30}, {2, 64, 128, 3.9, 0.37, 0.40, 0.75, 0.48}, {3, 128, 128, 4.2, 0.50, 0.61, 0, 0},

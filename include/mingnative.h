@@ -972,6 +972,10 @@ MN_API int mn_window_pool_attn_blocks(const float* q, int64_t ldq, const float* 
  * scores and weighted sums on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands and accumulation), 64 query vectors of a
  * key/value head a workgroup, tiles of 16 or 32 keys and values staged in LDS; MN_WINDOW_ATTN_VALU = the fp32 FMA kernel (decode rows, larger heads). */
 enum { MN_WINDOW_ATTN_MFMA = 0, MN_WINDOW_ATTN_VALU = 1 };
+/* Below 0: the kernel that mn_window_pool_attn_blocks chooses; MN_WINDOW_ATTN_AUTO_RUNS: and, on the matrix cores, every run in a workgroup of its own whatever their
+ * number, for steps whose sequences are shorter than the groups that runs share otherwise (mn_window_attn_form says so for the longest one's keys). */
+enum { MN_WINDOW_ATTN_AUTO = -1, MN_WINDOW_ATTN_AUTO_RUNS = -2 };
+MN_API int mn_window_attn_form(int H, int G, int vk, int max_len);
 MN_API int mn_window_pool_attn_blocks_ex(const float* q, int64_t ldq, const float* k_arena, const float* v_arena, const float* pk,
                                          const float* pv, const int32_t* row_seq, const int32_t* row_slot, const int32_t* blk_tab, int n_blk,
                                          int one_row, int H, int G, int dim, int vdim, int t_max, int n_pool_max, int window, int pool,

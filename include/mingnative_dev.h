@@ -45,6 +45,8 @@ MN_DEV_API void mn_lo_drop_mask(unsigned mask);
 MN_DEV_API void mn_gemm256_tune_thin(int on);
 /* The form of every dense gemm256 launch: -1 the rule, 0 the 256 x 256 tiles, 1 .. the small-tile forms of gemm_tile.inl. */
 MN_DEV_API void mn_gemm_tile_tune(int form);
+/* Matrix-core attention of runs of rows: -1 the rule, 0 in groups, 1 every run in a workgroup of its own. */
+MN_DEV_API void mn_attn_rows_tune(int form);
 /* Measurement only: K / V rows are rounded to bf16 when appended to the (fp32) cache — the values a bf16 KV cache would hold. */
 MN_DEV_API void mn_kv_round_bf16(int on);
 

@@ -417,6 +417,7 @@ SYMBOLS = {
     "mn_window_attn_splits": (_i, [_i, _i, _i, _i, _i]),
     "mn_window_attn_splits_tile": (_i, [_i, _i, _i, _i, _i, _i]),
     "mn_window_attn_splits_heads": (_i, [_i] * 9),
+    "mn_window_attn_form": (_i, [_i] * 4),
     "mn_window_attn_scratch_bytes": (_sz, [_i] * 6),
     "mn_window_attn_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _i]),
     "mn_window_pool_attn_blocks": (_i, [_p, _i64, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _f, _p, _i64, _p, _i64, _i,

@@ -301,7 +301,7 @@ extern "C" int mn_hyb_step(const mn_hyb_model* m, const mn_hyb_state* st, const 
       while (ns > 1 && mn_window_attn_workspace_bytes(n_blk, l.heads, l.kv_heads, l.vdim, one_row, ns) > p.attn_ws) --ns;
       MN_TRY(mn_window_pool_attn_blocks_sink(qf, d.cq, st->k[ri], st->v[ri], nullptr, nullptr, l.sink, row_seq, row_slot, blk_tab, n_blk, one_row,
                                              l.heads, l.kv_heads, l.dim, l.vdim, st->t_max, 1, 0, 0, 1.0f, cat, d.n_cat, cath, d.n_cat, ns, aws,
-                                             p.attn_ws, -1, stream));
+                                             p.attn_ws, mn_window_attn_form(l.heads, l.kv_heads, 0, max_len), stream));
     } else if (talk) {
       const int ck = l.kv_heads * l.dim, rows = one_row ? 1 : m->block_rows;
       MN_TRY(mn_rope_unit_append_from(pin, d.n_in, M, l.heads, l.kv_heads, l.dim, l.dim, l.heads * l.dim, l.rot_dims, l.rot_freq, 1.0f, 1, m->eps,

@@ -205,7 +205,7 @@ extern "C" int mn_ms_step(const mn_ms_model* m, const mn_ms_state* st, const flo
     MN_TRY(mn_window_pool_attn_blocks_gate(qf, d.cq, st->k[li], 0, st->v[li], 0, nullptr, nullptr, l.sink, 0.0f, l.chunk,
                                            l.has_gate ? pin + d.off_g : nullptr, d.n_in, row_seq, row_slot, blk_tab, n_blk, one_row, H, G, l.dim,
                                            l.vdim, st->t_max, 1, l.window, 0, 1.0f, cat16_only ? nullptr : cat, d.hv, cath, d.hv, ns, aws,
-                                           p.attn_ws, -1, stream));
+                                           p.attn_ws, mn_window_attn_form(H, G, 0, max_len), stream));
     MN_TRY(linear(arith, M, cat, d.hv, cath, d.hv, l.w_o, W, d.hv, nullptr, yf, W, gws, gwb, stream));
     sa.mix = l.hc1_mix; sa.out = l.hc1_out; sa.y = yf; sa.ldy = W;
     // ---- experts ----

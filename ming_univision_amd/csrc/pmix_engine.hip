@@ -244,9 +244,9 @@ extern "C" int mn_pmix_step(const mn_pmix_model* m, const mn_pmix_state* st, con
       }
       int ns = mn_window_attn_splits_heads(n_blk, l.heads, l.kv_heads, one_row, max_keys, 64, l.dim, l.vdim, 0);
       while (ns > 1 && mn_window_attn_workspace_bytes(n_blk, l.heads, l.kv_heads, l.vdim, one_row, ns) > p.attn_ws) --ns;
-      MN_TRY(mn_window_pool_attn_blocks(qf, d.cq, st->k[ri], st->v[ri], st->pk[ri], st->pv[ri], row_seq, row_slot, blk_tab, n_blk, one_row,
-                                        l.heads, l.kv_heads, l.dim, l.vdim, st->t_max, st->n_pool_max, l.window, l.pool, l.left_scale, cat,
-                                        d.n_cat, cath, d.n_cat, ns, aws, p.attn_ws, stream));
+      MN_TRY(mn_window_pool_attn_blocks_ex(qf, d.cq, st->k[ri], st->v[ri], st->pk[ri], st->pv[ri], row_seq, row_slot, blk_tab, n_blk, one_row,
+                                           l.heads, l.kv_heads, l.dim, l.vdim, st->t_max, st->n_pool_max, l.window, l.pool, l.left_scale, cat,
+                                           d.n_cat, cath, d.n_cat, ns, aws, p.attn_ws, mn_window_attn_form(l.heads, l.kv_heads, 0, max_len), stream));
     }
     const int hv = l.heads * l.vdim;
     if (gru_in_rows) {

@@ -1121,10 +1121,27 @@ AttnShape attn_shape(int H, int G, int one_row) {
 // attn_rows.inl: heads side by side in a wave's 16 query vectors, and the runs of a workgroup
 int attn_rows_heads(int rep) { return rep >= 3 ? 4 : rep; }
 int attn_rows_runs(int rep) { return 4 * (16 / attn_rows_heads(rep)) / 4; }
+int64_t attn_run_wgs(int n_blk, int H, int G) { return (int64_t)n_blk * G * attn_shape(H, G, 0).chunks; }
+// Every run by itself (attn_run) or in groups: by itself while that makes at most four workgroups a CU, key splits included.  A launch of more fills the chip with
+// groups, which read the keys a fourth as often (us, in groups / by runs: heads of 128, 8 over two key heads: 256 rows 28 / 16, 400 30 / 27, 700 49 / 49; 16 over
+// four: 256 30 / 22, 700 67 / 73; 16 over 16: 160 24 / 23, 256 32 / 48, 64 behind 2000 keys 39 / 92).
+bool attn_runs_alone(int n_blk, int H, int G, int nsplit) { return attn_run_wgs(n_blk, H, G) * nsplit <= 4 * (int64_t)mn_num_cus(); }
 }  // namespace
+
+static int g_attn_rows_form = -1;                      // runs of rows: 0 groups, 1 every run by itself, -1 the rule
+#ifdef MN_DEV_HOOKS
+extern "C" MN_DEV_API void mn_attn_rows_tune(int form) { g_attn_rows_form = form; }
+#endif
 
 // query vectors of a workgroup on runs of rows: 64 on the matrix cores (32 where the values lie inside the keys), a run on the FMA kernel
 static int attn_run_vectors(int dim, int vdim, int vk) { return vk ? (dim <= 640 ? 32 : 16) : (dim <= 256 && vdim <= 256 ? 64 : 16); }
+
+// Sequences of at most half the rows of a group would leave most groups to several of them, run by run (16 heads of 128, 64 sequences of 16 rows: 51 us, 35 without
+// groups, over eight key heads 28, 19; of 30 rows over eight key heads, a group each, 21, 36 without)
+extern "C" int mn_window_attn_form(int H, int G, int vk, int max_len) {
+  if (H < 1 || G < 1 || (H % G) != 0) return MN_WINDOW_ATTN_AUTO;
+  return max_len * attn_rows_heads(H / G) <= (vk ? 16 : 32) ? MN_WINDOW_ATTN_AUTO_RUNS : MN_WINDOW_ATTN_AUTO;
+}
 
 extern "C" int mn_window_attn_splits(int n_blk, int H, int G, int one_row, int max_keys) {
   return mn_window_attn_splits_tile(n_blk, H, G, one_row, max_keys, AKT);
@@ -1140,15 +1157,13 @@ extern "C" int mn_window_attn_splits_heads(int n_blk, int H, int G, int one_row,
   if (n_blk < 1 || H < 1 || G < 1 || (H % G) != 0 || max_keys < 1 || key_tile < 1) return 1;
   const AttnShape sh = attn_shape(H, G, one_row);
   const int vec = one_row ? 16 : attn_run_vectors(dim, vdim, vk);
-  const int64_t runs = vec == 16 ? 1 : attn_rows_runs(H / G) * vec / 64;
-  const int64_t wgs = mn_cdiv(n_blk, runs) * G * sh.chunks, tiles = mn_cdiv(max_keys, key_tile);
-  int64_t ns = mn_cdiv(2 * (int64_t)mn_num_cus(), wgs);
-  // (a workgroup of 32 or 64 vectors has some 10 us of its own: a split of its walk below 128 keys costs more than it saves)
-  const int64_t most = vec == 16 ? tiles : mn_cdiv(max_keys, 128);
-  if (ns > most) ns = most;
-  if (ns > tiles) ns = tiles;
-  if (ns > 64) ns = 64;
-  return ns < 1 ? 1 : (int)ns;
+  const int64_t runs = vec == 16 ? 1 : attn_rows_runs(H / G) * vec / 64, tiles = mn_cdiv(max_keys, key_tile);
+  auto want = [&](int64_t wgs, int64_t most) { const int64_t ns = mn_cdiv(2 * (int64_t)mn_num_cus(), wgs); return ns < most ? (ns < 64 ? (int)ns : 64) : (most < 64 ? (int)most : 64); };
+  const int by_runs = want((int64_t)n_blk * G * sh.chunks, tiles);
+  if (vec == 16) return by_runs;
+  // (a group of 32 or 64 vectors has some 10 us of its own: a split of its walk below 128 keys costs more than it saves)
+  const int by_groups = want(mn_cdiv(n_blk, runs) * G * sh.chunks, mn_cdiv(max_keys, 128) < tiles ? mn_cdiv(max_keys, 128) : tiles);
+  return attn_runs_alone(n_blk, H, G, by_groups) ? by_runs : by_groups;
 }
 
 extern "C" size_t mn_window_attn_workspace_bytes(int n_blk, int H, int G, int vdim, int one_row, int nsplit) {
@@ -1220,7 +1235,7 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
   MN_CHECK_ARG(ldk >= (int64_t)G * dim && ldv >= (int64_t)G * vdim && ((dim % 4) != 0 || (ldk % 4) == 0) && ((vdim % 4) != 0 || (ldv % 4) == 0) &&
                    softcap >= 0.0f,
                "mn_window_pool_attn_blocks: arena row strides below a row, or no multiple of 4 under heads that are; or a negative soft cap");
-  const bool variant_auto = variant < 0;
+  const bool variant_auto = variant < 0, runs_alone = variant == MN_WINDOW_ATTN_AUTO_RUNS;
   MN_CHECK_ARG(q && k_arena && v_arena && row_seq && row_slot && (out || out16) && n_blk >= 1 && H >= 1 && G >= 1 && (H % G) == 0 && dim >= 1 &&
                    vdim >= 1 && vdim <= 512 && t_max >= 1 && window >= 0 && pool >= 0 && nsplit >= 1 && nsplit <= 64,
                "mn_window_pool_attn_blocks: bad args (vdim=%d: at most 512; nsplit=%d: at most 64)", vdim, nsplit);
@@ -1243,15 +1258,24 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
                "mn_window_pool_attn_blocks: the matrix-core kernel takes runs of rows with dim, vdim <= 256, or values inside keys of dim <= 640");
   if (variant == MN_WINDOW_ATTN_MFMA) {
     hipStream_t stm = mn_stream(stream);
-    
-    if (!one_row) {                                    // runs of rows: 64 query vectors per workgroup
-      const int hv = attn_rows_heads(H / G);
-      dim3 gridr((unsigned)mn_cdiv(n_blk, attn_rows_runs(H / G)), (unsigned)(G * sh.chunks), (unsigned)nsplit);
-#define MN_WR(D_, V_, E_) hipLaunchKernelGGL((attn_rows_kernel<D_, V_, E_>), gridr, dim3(256), 0, stm, a, n_blk, hv)
-#define MN_WL(D_, E_) hipLaunchKernelGGL((attn_latent_rows_kernel<D_, E_>), gridr, dim3(256), 0, stm, a, n_blk, hv)
+    if (!one_row) {                                    // runs of rows: groups of 64 (values inside keys: 32) query vectors, and every run by itself behind them
+      const bool alone = g_attn_rows_form >= 0 ? g_attn_rows_form == 1 : runs_alone || attn_runs_alone(n_blk, H, G, nsplit);
+      const int hv = attn_rows_heads(H / G), runs = vk ? attn_rows_runs(H / G) / 2 : attn_rows_runs(H / G), groups = (int)mn_cdiv(n_blk, runs);
+      const int64_t tasks = attn_run_wgs(n_blk, H, G) * nsplit, two = 2 * mn_num_cus();
+      MN_CHECK_ARG(tasks < ((int64_t)1 << 29), "mn_window_pool_attn_blocks: too many rows");
+      const dim3 gridr((unsigned)((int64_t)groups * G * sh.chunks * nsplit + (tasks < two ? tasks : two))), grid1((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)nsplit);
+#define MN_WR(D_, V_, E_)                                                                                                                     \
+  do {                                                                                                                                       \
+    if (alone) hipLaunchKernelGGL((attn_runs_kernel<D_, V_, (D_ + V_ > 4 ? 1 : 2), E_, false>), grid1, dim3(256), 0, stm, a);                    \
+    else hipLaunchKernelGGL((attn_rows_kernel<D_, V_, E_>), gridr, dim3(256), 0, stm, a, n_blk, hv, groups);                                 \
+  } while (0)
+#define MN_WL(D_, E_)                                                                                                                        \
+  do {                                                                                                                                       \
+    if (alone) hipLaunchKernelGGL((attn_runs_kernel<D_, D_, (D_ > 4 ? 1 : 2), E_, true>), grid1, dim3(256), 0, stm, a);                          \
+    else hipLaunchKernelGGL((attn_latent_rows_kernel<D_, E_>), gridr, dim3(256), 0, stm, a, n_blk, hv, groups);                              \
+  } while (0)
       const bool vec4 = ((dim | vdim) & 3) == 0;       // (rows of any other size go value by value)
       if (vk) {
-        gridr.x = (unsigned)mn_cdiv(n_blk, attn_rows_runs(H / G) / 2);      // 32 vectors per workgroup
         const int nbl = (dim + 63) / 64;
         if (!vec4) {
           if (nbl <= 2) MN_WL(2, false);

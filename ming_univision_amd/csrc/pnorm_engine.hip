@@ -191,7 +191,7 @@ extern "C" int mn_pn_step(const mn_pn_model* m, const mn_pn_state* st, const flo
       const bool gate = attn && l.has_gate;
       MN_TRY(mn_window_pool_attn_blocks_cap(qf, d.nq, karena, ldk, varena, ldv, nullptr, nullptr, nullptr, l.softcap, row_seq, row_slot, blk_tab,
                                             n_blk, one_row, H, G, d.akd, d.avd, st->t_max, 1, l.window, 0, 1.0f, att, ldatt,
-                                            (attn && !gate) ? cath : nullptr, d.hv, ns, aws, p.attn_ws, -1, stream));
+                                            (attn && !gate) ? cath : nullptr, d.hv, ns, aws, p.attn_ws, mn_window_attn_form(H, G, latent, max_len), stream));
       if (gate) MN_TRY(mn_head_sigmoid_gate_rows(cat, d.hv, pin + d.off_g, d.n_in, cath, d.hv, M, H, l.vdim, stream));
       if (latent)                                        // every head's value = W_uv[h] (its attended latent)
         MN_TRY(mn_gemm_f32_batched(mid, d.nmid, l.kv_rank, l.w_uv, l.kv_rank, (int64_t)l.vdim * l.kv_rank, nullptr, cat, d.hv, l.vdim, cath, d.hv,

@@ -124,6 +124,44 @@ def test_values_that_are_not_finite(H, G, d, e, vk):
             assert float((mine - ref).abs().max() / ref.abs().max()) < 1e-5
 
 
+@pytest.fixture
+def dev_lib():
+    """The same code with the switches of mingnative_dev.h, in the place of the product library."""
+    import ctypes
+    import os
+    from ming_univision_amd import _lib
+    shipped = _lib.lib()
+    handle = ctypes.CDLL(os.path.join(os.path.dirname(_lib.LIB_PATH), "libmingnative_dev.so"))
+    for name, (res, args) in _lib.SYMBOLS.items():
+        fn = getattr(handle, name)
+        fn.restype, fn.argtypes = res, args
+    _lib._lib = handle
+    yield handle
+    handle.mn_attn_rows_tune(-1)
+    _lib._lib = shipped
+
+
+# sequences that end inside a group, begin inside one, fill one, and many in one; rows alone, drafted rows and prompts beside each other
+MIXED = SPANS + [[(i, 16, 0) for i in range(9)], [(0, 61, 3)] + [(1 + i, 2, 30 + i) for i in range(21)] + [(30, 70, 0)], [(i, 1 + i % 5, 7 * i) for i in range(30)]]
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("H,G,d,e,vk", [(4, 1, 64, 64, 0), (8, 2, 128, 128, 0), (6, 6, 16, 40, 0), (6, 3, 72, 136, 0), (5, 1, 34, 50, 0), (3, 1, 200, 256, 0), (4, 1, 64, 48, 1),
+                                        (16, 1, 576, 512, 1), (1, 1, 320, 256, 1), (2, 1, 35, 19, 1)])
+def test_either_form(dev_lib, form, H, G, d, e, vk):
+    """Groups of 64 (32) query vectors and runs in workgroups of their own, whatever the rule would take."""
+    dev_lib.mn_attn_rows_tune(form)
+    for spans in MIXED:
+        for window, cap, chunk, ns, pool in ((0, 0.0, 0, 1, 0), (33, 20.0, 0, 3, 0), (0, 0.0, 48, 2, 0), (17, 0.0, 0, 1, 0 if vk else 4)):
+            run(spans, H, G, d, e, window, cap, chunk, bool(vk), ns, 256, pool)
+    test_values_that_are_not_finite(H, G, d, e, bool(vk))
+
+
+def test_more_runs_than_the_groups_workgroups_look_at_together():
+    """36000 (run, head, split) tasks of groups that hold several sequences."""
+    run([(i, 1 + i % 2, 5) for i in range(600)], 20, 20, 16, 16, 0, 0.0, 0, False, 3, 16)
+
+
 def test_three_splits_of_many_groups():
     """More than 256 workgroups in a head and split: every group exactly once whatever the launch order."""
     run([(0, 700, 0), (1, 700, 0), (2, 700, 0)], 5, 1, 16, 16, 0, 0.0, 0, False, 3, 704)

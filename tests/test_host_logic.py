@@ -171,6 +171,19 @@ def test_key_splits_of_attention_runs_and_their_scratch():
                         assert 1 <= ns <= 64 and need(n_blk, H, G, e, one_row, ns) <= got, (H, G, d, e, vk, M, n_blk, one_row, keys, ns)
 
 
+def test_form_of_attention_runs():
+    """mn_window_attn_form: no groups where the longest sequence has at most half a group's rows (64 query vectors, 32 where the values lie inside the keys); the split
+    request of few runs counts them one by one, down to 64 keys."""
+    import ctypes
+    from ming_univision_amd import _lib
+    L = ctypes.CDLL(_lib.LIB_PATH)
+    form, splits = L.mn_window_attn_form, L.mn_window_attn_splits_heads
+    for H, G, vk, rows in ((16, 16, 0, 32), (16, 8, 0, 16), (16, 4, 0, 8), (12, 4, 0, 8), (16, 1, 1, 4), (2, 1, 1, 8), (1, 1, 1, 16)):
+        assert form(H, G, vk, rows) == -2 and form(H, G, vk, rows + 1) == -1 and form(H, G, vk, 1) == -2
+    assert splits(8, 8, 2, 0, 502, 64, 128, 128, 0) == 8 and splits(4, 16, 4, 0, 516, 64, 128, 128, 0) == 9          # 16 workgroups a split, however the keys allow
+    assert splits(100, 8, 2, 0, 400, 64, 128, 128, 0) == 3 and splits(175, 16, 16, 0, 700, 64, 128, 128, 0) == 3     # 200 runs; 704 groups
+
+
 def test_scratch_of_a_hybrid_prompt_grows_with_its_rows():
     """mn_hyb_workspace_bytes: the output product's slabs are 16 times the step's rows up to 8192 in all, not 8192 rows from 65 on; never less for more prompt
     rows."""

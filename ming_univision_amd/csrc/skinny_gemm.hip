@@ -339,7 +339,10 @@ extern "C" size_t mn_skinny_workspace_bytes_w8(int M, int N, int K, int epilogue
 // 8.8 + 0.08 M + 0.2 a megabyte of weights, or 3.2 + 0.19 a megabyte + 0.3 per 1024 of K and as much again a row (8 rows at once; 5 .. 7 as 4 + the rest).  The lines
 // this draws, both sides measured: 32 rows of 2048 x 2048 11.9 / 13.7, of 1024 x 4096 20.1 / 14.8, of 8192 x 2048 (two tiles) 18.8 / 22.4, of 3072 x 3072 17.7 /
 // 17.2, of 3072 x 2048 behind an RMSNorm 17.4 / 16.2; 16 rows of 32 x 3072 9.5 / 8.7; against FMA 2 rows of 2048 x 2048 6.2 / 5.4, of 4096 x 1024 4.6 / 5.3; 4 rows of
-// 2048 x 2048 6.3 / 7.1; 5 rows of it 6.2 / 11.8; 8 rows of 8192 x 2048 11.8 / 22.5; 2 rows of 32000 x 2048 32.0 / 28.2, 3 rows 33.6 / 36.0.  Not where the output overlaps what is read (the other forms read a row
+// 2048 x 2048 6.3 / 7.1; 5 rows of it 6.2 / 11.8; 8 rows of 8192 x 2048 11.8 / 22.5; 2 rows of 32000 x 2048 32.0 / 28.2, 3 rows 33.6 / 36.0.  Two rows stay on FMA,
+// and three of plain products of more than 4096 columns and up to 1024 values: the launch itself is shorter here (7424 x 1024 6.4 / 8.4), but the ones behind it are
+// longer by as much and more (decode steps of 2 rows, four layers of width 1024: 208 / 189, 302 / 280, 191 / 184 us, of 3 rows of such products 211 / 198; of width
+// 2048 alike).  Not where the output overlaps what is read (the other forms read a row
 // before they write it) and not behind a LayerNorm (its mean has to be known before the split).
 static bool rows_kc(const mn_skinny_args& a, bool fma, hipStream_t st) {
   const bool paired = mn_epi_pairs(a.epilogue);
@@ -356,6 +359,7 @@ static bool rows_kc(const mn_skinny_args& a, bool fma, hipStream_t st) {
   const double here = 2.5 + fmax(0.22 * mb, mn_cdiv(a.K, 512) * (0.85 + 0.042 * a.M) * (nt == 2 ? 1.7 : 1.0) * (a.prologue == MN_PRO_RMSNORM ? 1.4 : 1.0) * mn_cdiv(g, mn_num_cus()));
   const double row = 0.4 + 0.25 * kk + 0.02 * mb, once = 3.2 + 0.19 * mb + 0.3 * kk;
   const double there = !fma ? 8.8 + 0.08 * a.M + 0.2 * mb : (a.M > 4 && a.M < 8 ? 2 * once + (a.M - 2) * row : once + (a.M - 1) * row) / 1.15;
+  if (fma && (a.M == 2 || (a.M == 3 && nt == 2 && !paired && a.K <= 1024))) return false;
   if (g > (fma ? 4 : 1) * mn_num_cus() || here >= there) return false;
 #define MN_KC(MT_, NT_, P_) hipLaunchKernelGGL((rows_kc_kernel<MT_, NT_, P_>), dim3((unsigned)g), dim3(512), 0, st, a, paired ? 1 : 0)
 #define MN_KC_P(MT_, NT_)                                              \

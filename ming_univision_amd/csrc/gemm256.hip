@@ -443,7 +443,8 @@ extern "C" MN_DEV_API void mn_gemm256_tune_order(int group_m, int group_list) { 
 // with the constants measured on MI355X (weights cycling through HBM, graph of 48 launches; us): a workgroup alone on its CU needs `alone` per
 // K-tile, rising to `full` when every CU holds one and to `two` when every CU holds two (forms that fit twice); beyond that `per` for each
 // workgroup of a CU, or whole rounds of `full` (forms that fit once: per = 0).  The fixed part is launch, first round trip and epilogue: 4 us
-// for the small tiles, 11 us + 7 per further round for the 256-tile kernel.
+// for the small tiles, 11 us + 7 per further round for the 256-tile kernel, 4.2 per round of the other form that fits once; many workgroups of the forms that fit
+// twice pay for their epilogues from 6 (hi/lo 3) a CU on: 4100 x 6000 x 768 hi/lo 93 (256) against 122, 4096 x 4096 x 512 45 against 60.
 // Where the lines then lie, both sides measured: 65 x 3072 x 1024 bf16: 7.3 us (64 x 64) against 23.7 (256); 256 x 4096 x 1024: 8.2 against
 // 32.1; 1025 hi/lo rows x 1024 x 1024: 10.9 (64 x 64) against 22.3; x 3072: 20.0 (64 x 128) against 26.0; 2048 x 2048 x 8192: 79.6 (128 x 128) against 136.6;
 // 16384 x 1024 x 1024: 37.2 (256) against 54.2 (128 x 128); 1025 hi/lo rows x 2752 SwiGLU: 29.9 (256) against 37.8.
@@ -453,7 +454,7 @@ static const TileForm tile_plain[] = {{1, 64, 64, 3.6, 0.23, 0.26, 0.42, 0.30}, 
 static const TileForm tile_hilo[] = {{1, 64, 64, 3.8, 0.41, 0.42, 0.60, 0.41}, {2, 64, 128, 4.0, 0.64, 0.66, 1.00, 0.58}, {3, 128, 128, 4.2, 0.93, 1.04, 0, 0},
                                      {0, 128, 256, 11.0, 0.87, 1.25, 0, 0}};
 
-static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bool paired) {
+static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bool hilo, bool paired) {
   const double w = (double)(mn_cdiv(M, f.bm) * mn_cdiv(N, paired ? f.bn / 2 : f.bn) * nz) / 256.0;
   const double rounds = w > 1.0 ? (double)(int64_t)(w + 0.999) : 1.0;
   double per_tile;
@@ -461,7 +462,8 @@ static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bo
   else if (f.per == 0) per_tile = f.full * rounds;
   else if (w <= 2.0) per_tile = f.full + (f.two - f.full) * (w - 1.0);
   else per_tile = f.per * w > f.two ? f.per * w : f.two;
-  return f.fixed + (f.form == 0 ? 7.0 * (rounds - 1.0) : 0.0) + k_tiles * per_tile;
+  const double ends = f.form == 0 ? 7.0 * (rounds - 1.0) : f.per == 0 ? 4.2 * (rounds - 1.0) : hilo ? 1.8 * fmax(w - 3.0, 0.0) : 1.0 * fmax(w - 6.0, 0.0);
+  return f.fixed + ends + k_tiles * per_tile;
 }
 
 // the form of a dense M x N x K launch in nz K-slices of Kc, and the estimate of its time
@@ -472,7 +474,7 @@ static int tile_form(int M, int N, int Kc, int nz, bool hilo, bool paired, bool 
   double tb = 1e30;
   for (int i = 0; i < n; ++i) {
     if (t[i].form == 0 && !may256) continue;
-    const double e = tile_time(t[i], M, N, Kc / BK, nz, paired);
+    const double e = tile_time(t[i], M, N, Kc / BK, nz, hilo, paired);
     if (e < tb) { tb = e; best = t[i].form; }
   }
   if (us) *us = tb;
@@ -531,9 +533,10 @@ static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
     else hipLaunchKernelGGL((gemm256_kernel<E_SWIGLU_BF16, false, true>), grid, dim3(512), 0, st, p);
     return nz;
   }
-  // (the 256-tile kernel's GELU is the 1.5e-7 polynomial: it serves the problems of 128 tiles and more)
+  // (the 256-tile kernel's GELU is the 1.5e-7 polynomial: it serves the problems of 128 tiles and more, where erff in the small tiles' epilogue costs more than they save:
+  // 4096 x 4096 x 256 26.9 us against 38.6, 8000 x 4000 x 192 45 against 69)
   const bool may256 = epi != E_BF16_GELU || mn_cdiv(p.M, 256) * mn_cdiv(p.N, 256) >= 128;
-  const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : tile_form(p.M, p.N, p.Kc, nz, hilo, paired, may256, nullptr);
+  const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : epi == E_BF16_GELU && may256 ? 0 : tile_form(p.M, p.N, p.Kc, nz, hilo, paired, may256, nullptr);
 #define G256_GO(E)                                                                          \
   do {                                                                                      \
     if (form > 0 && tile_launch<E>(p, form, nz, hilo, st)) break;                           \

@@ -381,8 +381,9 @@ __global__ __launch_bounds__(256 * KS, QG == 1 && KS == 2 && HD == 64 ? 4 : 2) v
 //   1024 x 16 x 1 bf16 25.0 -> 13.8; 1025 x 16 x 1 hi/lo causal 41.3 -> 24, 1025 x 12 hi/lo 41 -> 24; 257 x 16 10.6 -> 7.1; 2500 x 16 hi/lo causal 99.6 -> 68
 // A causal launch has half the work and goes longest walk first, so it takes them up to 2.5 workgroups a CU (1088 of 64 queries: no form
 // is better).  A full launch of more than one a CU has a second round; 128 queries in two key groups avoid it (1025 x 16 hi/lo: 34 against 38 and 46 us).
-// Launches that fill the chip walk alone (64 x 256 x 16 bf16: 38 us, in key groups 55), 64 queries a workgroup where 128 would leave much
-// of the last one empty (64 x 65 x 16: 14.1 -> 11.0, 64 x 257 x 12: 46 -> 43).  Heads are the fastest grid dimension: an XCD then sees few heads' keys
+// Launches that fill the chip walk alone (64 x 256 x 16 bf16: 38 us, in key groups 55), 64 queries a workgroup where causal (64 x 200 x 16: 36 -> 30, 1 x 4096 x 16: 87
+// -> 69), where 128 would leave an eighth and more of the queries empty (64 x 257 x 12: 47 -> 44) or some CUs a second workgroup (1 x 2500 x 16: 72 -> 62); else 128
+// (1 x 4000 x 16 hi/lo: 264 -> 210, 16 x 1025 x 12 221 -> 197, 64 x 65 x 16 28 -> 25).  Heads are the fastest grid dimension: an XCD then sees few heads' keys
 // (2500 x 16 hi/lo, 128 queries: 126 -> 100 us).
 template <bool HILO>
 void flash_hd64(const FlashP& p, int T, int n_heads, int B, hipStream_t st) {
@@ -390,7 +391,7 @@ void flash_hd64(const FlashP& p, int T, int n_heads, int B, hipStream_t st) {
 #define MN_FL(QG_, KS_) hipLaunchKernelGGL((flash_prefill_kernel<64, 0, HILO, QG_, KS_>), dim3(n_heads, mn_cdiv(T, 64 * (QG_)), B), dim3(256 * (KS_)), 0, st, p)
   if (T > 64 && w64 <= (p.causal ? 5 * cu / 2 : cu)) MN_FL(1, 2);
   else if (T > 64 && w128 <= cu) MN_FL(2, 2);
-  else if (((T - 1) & 127) < 80) MN_FL(1, 1);
+  else if (p.causal || 2 * w128 <= 3 * cu || 100 * w128 >= 58 * w64) MN_FL(1, 1);
   else MN_FL(2, 1);
 #undef MN_FL
 }

@@ -366,24 +366,27 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(GemmF32 a) {
         if (k < a.K) { fa[t] = *reinterpret_cast<const f32x4*>(ap + k); fw[t] = *reinterpret_cast<const ushort4*>(wp + k); }
       } else {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) if (k + c < a.K) fa[t][c] = ap[k + c];
-        if (k < a.K) fw[t].x = wp[k];
-        if (k + 1 < a.K) fw[t].y = wp[k + 1];
-        if (k + 2 < a.K) fw[t].z = wp[k + 2];
-        if (k + 3 < a.K) fw[t].w = wp[k + 3];
+        for (int c = 0; c < 4; ++c) fa[t][c] = ap[min(k + c, a.K - 1)];          // (what is past K becomes zero on the way to LDS: a branch here is a wait)
+        fw[t] = ushort4{wp[min(k, a.K - 1)], wp[min(k + 1, a.K - 1)], wp[min(k + 2, a.K - 1)], wp[min(k + 3, a.K - 1)]};
       }
     }
   };
-  auto put = [&](int b) {
+  auto put = [&](int b, int k0) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int e = tid + 256 * t, at = (e >> 3) * LD + 4 * (e & 7);
+      if (!V4) {
+        const int left = a.K - k0 - 4 * (e & 7);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) fa[t][c] = c < left ? fa[t][c] : 0.f;
+        fw[t] = ushort4{left > 0 ? fw[t].x : (unsigned short)0, left > 1 ? fw[t].y : (unsigned short)0, left > 2 ? fw[t].z : (unsigned short)0, left > 3 ? fw[t].w : (unsigned short)0};
+      }
       *reinterpret_cast<f32x4*>(&As[b][at]) = fa[t];
       *reinterpret_cast<f32x4*>(&Ws[b][at]) = f32x4{bf16_to_f32(fw[t].x), bf16_to_f32(fw[t].y), bf16_to_f32(fw[t].z), bf16_to_f32(fw[t].w)};
     }
   };
   fetch(0);
-  put(0);
+  put(0, 0);
   int b = 0;
   for (int k0 = 0; k0 < a.K; k0 += 32, b ^= 1) {
     const bool more = k0 + 32 < a.K;
@@ -404,7 +407,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(GemmF32 a) {
 #pragma unroll
           for (int j = 0; j < 2; ++j) acc[u][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[i][t], rw[j][t], acc[u][i][j], 0, 0, 0);
     }
-    if (more) put(b ^ 1);                                     // the buffer that every wave left before this step's barrier
+    if (more) put(b ^ 1, k0 + 32);                                     // the buffer that every wave left before this step's barrier
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)

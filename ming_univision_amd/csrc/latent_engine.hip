@@ -7,6 +7,9 @@
 // The per-head absorb (q W_uk) and expand (latent W_uv^T) products are batched over heads in fp32 (mn_gemm_f32_batched) in both modes.
 #include "seq_linear.h"
 
+extern "C" int mn_rms_rows_pair(const float* xa, const uint16_t* wa, float* ya, int64_t ldya, uint16_t* ya16, int64_t ldya16, int na, const float* xb, const uint16_t* wb,
+                                float* yb, const int32_t* row_seq, const int32_t* row_slot, int t_max, int nb, int64_t ldx, float eps, int M, void* stream);
+
 extern "C" size_t mn_sizeof_seq_layer(void) { return sizeof(mn_seq_layer); }
 extern "C" size_t mn_sizeof_seq_model(void) { return sizeof(mn_seq_model); }
 extern "C" size_t mn_sizeof_seq_state(void) { return sizeof(mn_seq_state); }
@@ -162,13 +165,17 @@ extern "C" int mn_seq_step(const mn_seq_model* m, const mn_seq_state* st, const 
     MN_TRY(linear(arith, M, hf, W, hh, W, l.w_in, d.n_in, W, nullptr, pin, d.n_in, gws, gwb, stream));
     const float* qp; int64_t ldq; const float* gp = nullptr; int kv_off;
     if (l.kind == MN_SEQ_MIX_LATENT_Q) {
-      MN_TRY(mn_rms_rows(pin, d.n_in, l.q_norm, m->eps, cq, l.q_rank, cqh, l.q_rank, nullptr, nullptr, 0, M, l.q_rank, stream));
+      if (l.writes_arena)
+        MN_TRY(mn_rms_rows_pair(pin, l.q_norm, cq, l.q_rank, cqh, l.q_rank, l.q_rank, pin + l.q_rank, l.kv_norm, arena, row_seq, row_slot, st->t_max, l.kv_rank,
+                                d.n_in, m->eps, M, stream));
+      else
+        MN_TRY(mn_rms_rows(pin, d.n_in, l.q_norm, m->eps, cq, l.q_rank, cqh, l.q_rank, nullptr, nullptr, 0, M, l.q_rank, stream));
       MN_TRY(linear(arith, M, cq, l.q_rank, cqh, l.q_rank, l.w_uq, d.hd, l.q_rank, nullptr, qf, d.hd, gws, gwb, stream));
       qp = qf; ldq = d.hd; kv_off = l.q_rank;
     } else {
       qp = pin; ldq = d.n_in; gp = pin + d.hd; kv_off = d.hd + d.hv;
     }
-    if (l.writes_arena)
+    if (l.writes_arena && l.kind != MN_SEQ_MIX_LATENT_Q)
       MN_TRY(mn_rms_rows(pin + kv_off, d.n_in, l.kv_norm, m->eps, arena, l.kv_rank, nullptr, 0, row_seq, row_slot, st->t_max, M, l.kv_rank,
                          stream));
     // absorb: qabs[m, h, :] = scale * q[m, h, :] W_uk[h]   (W_ukT[h] is [kv_rank, dim])

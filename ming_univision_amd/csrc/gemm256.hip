@@ -453,6 +453,13 @@ static const TileForm tile_plain[] = {{1, 64, 64, 3.6, 0.23, 0.26, 0.42, 0.30}, 
                                       {4, 128, 128, 4.2, 0.55, 0.85, 1.16, 0.85}, {0, 256, 256, 11.0, 0.85, 1.30, 0, 0}};
 static const TileForm tile_hilo[] = {{1, 64, 64, 3.8, 0.41, 0.42, 0.60, 0.41}, {2, 64, 128, 4.0, 0.64, 0.66, 1.00, 0.58}, {3, 128, 128, 4.2, 0.93, 1.04, 0, 0},
                                      {0, 128, 256, 11.0, 0.87, 1.25, 0, 0}};
+// Up to 64 hi/lo rows: one row of tiles, so every weight byte comes from HBM, and what a CU takes in (rows and weights alike, 45 .. 50 GB/s of them however
+// many loads are in flight) is the time.  So tiles no taller than the rows: 3072 x 16384 with its SwiGLU at 16 rows 19.7 us (32-row tiles) against 28.3 (64), at 36
+// 25.2 (48-row tiles, gate and up in one fragment) against 29.5; and wider ones where slices of K leave enough of them: 8192 x 3072 at 36 rows 13.8 us
+// (64 x 128, 8 slices) against 15.8, at 16 rows 11.5 (32 x 64, 5 slices) against 14.4.  max_m: 0 or the most rows the form takes; split: the split SwiGLU alone.
+struct FewForm { TileForm f; int max_m; bool split; };
+static const FewForm tile_few[] = {{{5, 32, 64, 3.8, 0.28, 0.36, 0.74, 0.40}, 32, false}, {{6, 48, 64, 3.8, 0.40, 0.44, 0.90, 0.50}, 48, true},
+                                   {{1, 64, 64, 3.8, 0.46, 0.53, 0.95, 0.55}, 64, false}, {{7, 64, 128, 4.0, 0.50, 0.72, 0, 0}, 64, false}};
 
 static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bool hilo, bool paired) {
   const double w = (double)(mn_cdiv(M, f.bm) * mn_cdiv(N, paired ? f.bn / 2 : f.bn) * nz) / 256.0;
@@ -467,7 +474,19 @@ static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bo
 }
 
 // the form of a dense M x N x K launch in nz K-slices of Kc, and the estimate of its time
-static int tile_form(int M, int N, int Kc, int nz, bool hilo, bool paired, bool may256, double* us) {
+static int tile_form(int M, int N, int Kc, int nz, bool hilo, int epi, bool may256, double* us) {
+  const bool paired = epi_paired(epi);
+  if (hilo && M <= 64) {
+    int best = 0;
+    double tb = 1e30;
+    for (const FewForm& t : tile_few) {
+      if (M > t.max_m || (t.split && epi != E_SWIGLU_SPLIT)) continue;
+      const double e = tile_time(t.f, M, N, Kc / BK, nz, true, paired);
+      if (e < tb) { tb = e; best = t.f.form; }
+    }
+    if (us) *us = tb;
+    return best;
+  }
   const TileForm* t = hilo ? tile_hilo : tile_plain;
   const int n = hilo ? (int)(sizeof(tile_hilo) / sizeof(TileForm)) : (int)(sizeof(tile_plain) / sizeof(TileForm));
   int best = 0;
@@ -507,6 +526,11 @@ static bool tile_launch(const G256& p, int form, int nz, bool hilo, hipStream_t 
     case 1: tile_go<EPI, 64, 64, 2, 2, 3, true>(p, nz, st); return true;
     case 2: tile_go<EPI, 64, 128, 2, 2, 2, true>(p, nz, st); return true;
     case 3: tile_go<EPI, 128, 128, 2, 4, 3, true>(p, nz, st); return true;
+    case 5: tile_go<EPI, 32, 64, 2, 2, 5, true>(p, nz, st); return true;
+    case 6:
+      if constexpr (EPI == E_SWIGLU_SPLIT) { tile_go<EPI, 48, 64, 1, 4, 4, true>(p, nz, st); return true; }
+      return false;
+    case 7: tile_go<EPI, 64, 128, 4, 2, 3, true>(p, nz, st); return true;
     default: return false;
   }
 }
@@ -536,7 +560,7 @@ static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
   // (the 256-tile kernel's GELU is the 1.5e-7 polynomial: it serves the problems of 128 tiles and more, where erff in the small tiles' epilogue costs more than they save:
   // 4096 x 4096 x 256 26.9 us against 38.6, 8000 x 4000 x 192 45 against 69)
   const bool may256 = epi != E_BF16_GELU || mn_cdiv(p.M, 256) * mn_cdiv(p.N, 256) >= 128;
-  const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : epi == E_BF16_GELU && may256 ? 0 : tile_form(p.M, p.N, p.Kc, nz, hilo, paired, may256, nullptr);
+  const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : epi == E_BF16_GELU && may256 ? 0 : tile_form(p.M, p.N, p.Kc, nz, hilo, epi, may256, nullptr);
 #define G256_GO(E)                                                                          \
   do {                                                                                      \
     if (form > 0 && tile_launch<E>(p, form, nz, hilo, st)) break;                           \
@@ -589,8 +613,9 @@ extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo) {
     const int Kc = ks == 1 ? K : (int)(mn_cdiv(mn_cdiv(K, ks), 2 * BK) * 2 * BK), nz = (int)mn_cdiv(K, Kc);
     if (nz != ks) continue;
     double t;
-    tile_form(M, N, Kc, nz, hilo != 0, false, true, &t);
+    tile_form(M, N, Kc, nz, hilo != 0, E_F32, true, &t);
     t += nz * (double)M * N * 8.0 / 4.5e6;
+    if (hilo && M <= 64) t += 0.25 * nz * fmin(1.0, N / 2048.0);         // (a few rows' slabs are read by a few workgroups)
     if (t < tb - 1e-9) { tb = t; best = ks; }
   }
   return best > 1 ? best : 0;

@@ -29,7 +29,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
   constexpr int NW = WM * WN, AR = HILO ? 2 * BM : BM, QA = AR / 8 / NW, QW = BN / 8 / NW, STAGE = (AR + BN) * 128;
   constexpr int MI = BM / WM / 16, NJ = BN / WN / 16, AI = HILO ? 2 * MI : MI;
   constexpr bool paired = epi_paired(EPI);
-  static_assert(QA * 8 * NW == AR && QW * 8 * NW == BN && MI >= 1 && NJ >= (paired ? 2 : 1), "whole instructions and fragments per wave");
+  constexpr bool quads = paired && NJ == 1;            // gate and up of a unit within one fragment: a lane's 4 columns are 2 gates, then their 2 ups
+  static_assert(QA * 8 * NW == AR && QW * 8 * NW == BN && MI >= 1 && NJ >= 1 && (!quads || EPI == E_SWIGLU_SPLIT), "whole instructions and fragments per wave");
   static_assert((QA + QW) * (S - 2) < 64 && S * STAGE <= 160 * 1024, "vmcnt range, LDS");
   __shared__ __attribute__((aligned(1024))) char lds[S * STAGE];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -60,7 +61,9 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
   for (int q = 0; q < QW; ++q) {
     const int L = (wave * QW + q) * 8 + rin;
     int gn;
-    if (paired) {                                      // a wave's columns: its gate rows, then the up rows of the same units
+    if (quads) {
+      gn = min(n0 + (L >> 4) * 8 + ((L >> 2) & 3) * 2 + (L & 1), p.N - 1) + (L & 2 ? (int)p.w_pair_rows : 0);
+    } else if (paired) {                               // a wave's columns: its gate rows, then the up rows of the same units
       constexpr int WC = BN / WN, half = WC / 2;
       const int w = L / WC, r = L % WC;
       gn = min(n0 + w * half + (r % half), p.N - 1) + (r >= half ? (int)p.w_pair_rows : 0);
@@ -119,6 +122,27 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
 
   char* Cz = reinterpret_cast<char*>(p.C);
   if (EPI == E_F32) Cz += (int64_t)blockIdx.y * p.c_zstride * 4;
+  if constexpr (quads) {
+    const int n = n0 + wn * 8 + fq * 2;                // two units (N % 4 == 0: both in or both out)
+    float bg[2] = {0.f, 0.f}, bu[2] = {0.f, 0.f};
+    if (p.bias && n < p.N) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) { bg[e] = bf16_to_f32(p.bias[n + e]); bu[e] = bf16_to_f32(p.bias[p.w_pair_rows + n + e]); }
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int m = m0 + i * 16 + fr;
+      if (m >= p.M || n >= p.N) continue;
+      f32x4 v = acc[i][0];
+      if (HILO) v += acc[(i + MI) % AI][0];
+      uint32_t hi, lo;
+      split_pk_bf16(silu_f(v.x + bg[0]) * (v.z + bu[0]), silu_f(v.y + bg[1]) * (v.w + bu[1]), hi, lo);
+      bf16_t* c = reinterpret_cast<bf16_t*>(p.C) + (int64_t)m * p.ldc + n;
+      *reinterpret_cast<uint32_t*>(c) = hi;
+      *reinterpret_cast<uint32_t*>(c + p.c_lo_off) = lo;
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int m = m0 + wm * (BM / WM) + i * 16 + fr;

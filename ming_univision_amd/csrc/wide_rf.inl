@@ -1,4 +1,4 @@
-// wide_rf.inl — RectifiedFlowLoss.sample (diff_loss_rf_swiglu.py:103-181) for 24..2048 CFG rows advancing in lock-step
+// wide_rf.inl — RectifiedFlowLoss.sample (diff_loss_rf_swiglu.py:103-181) for 5..2048 CFG rows advancing in lock-step
 // (textually part of engine.hip).  Same arithmetic as the streaming route of mn_rf_sample; every Linear is a gemm256 launch on bf16 hi/lo operands (fp32-class products) and the work between two
 // Linears is one wide_glue launch:
 //
@@ -10,12 +10,13 @@
 //                      [slab reduce + b3 + gated residual + next in_ln / final LN + modulate]   (diff_loss:270-272, 290)
 //                      final Linear (split-K) -> bias -> CFG combine + Euler step              (diff_loss:144-179, 291)
 // First row count that takes the wide route, per stage (measured crossovers); mn_wide_tune is the A/B hook.  The flow head's bf16 weights go by tiles
-// from 24 rows on: 64 x 64 tiles pay the same for 12 and for 64 rows (w12 of 3072 x 16384 with its SwiGLU 27 us, w3 16 us at 36 rows), the streaming
-// kernels and the launches between them do not (26.6 + 5.5, 19.3 us).  A token of 36 rows: 20.9 -> 19.4 ms; 30 rows 18.3 -> 18.0; 24 rows 17.4 -> 17.2; 16
-// rows 15.0 against 15.7.  Weight-only formats are expanded to bf16 once per call on this route and keep their line at 41.
+// from 5 rows on: with tiles no taller than the rows w12 and its SwiGLU run at the weights' rate (20 us up to 32 rows, 24 at 36, for 101 MB), the streaming kernels
+// and the launches between them do not (26.6 + 5.5 us).  A sampler call, streaming kernels against tiles, ms: 4 rows 7.57 / 7.76, 5 rows 8.29 / 7.73, 8 rows
+// 8.41 / 7.80, 16 rows 8.92 / 8.07, 24 rows 10.23 / 8.47, 36 rows 12.40 / 9.94, 64 rows 13.50 / 11.66 (with 64-row tiles alone the line was 24 rows).
+// Weight-only formats are expanded to bf16 once per call on this route and keep their line at 41.
 // The semantic decoder likewise beyond the 32 rows whose projections are one launch (a token of 64 rows 22.8 -> 22.3 ms); the language model's experts
 // keep the streaming kernels up to 64 rows (64 rows of 1100 tokens: 10.8 against 11.1 ms).
-static int g_wide_min_llm = 65, g_wide_min_rf = 24, g_wide_min_rf_w8 = 41, g_wide_min_sem = 33;
+static int g_wide_min_llm = 65, g_wide_min_rf = 5, g_wide_min_rf_w8 = 41, g_wide_min_sem = 33;
 #ifdef MN_DEV_HOOKS
 extern "C" MN_DEV_API void mn_wide_tune(int llm_min_rows, int rf_min_rows, int sem_min_rows) {
   if (llm_min_rows > 0) g_wide_min_llm = llm_min_rows;
@@ -39,6 +40,7 @@ struct RfWideWs {
   float* pbuf_stream;    // tp.inl, <= 64 rows: K-slice slabs of the weight-streaming kernels
   float* pbuf_stream3;   // tp.inl, <= 4 rows: w3's slabs when its prologue reads w12's (stream_fuse.h)
   bf16_t *hs, *zs, *y, *ya, *yb;
+  int64_t lda;           // elements between the rows of ya
   bf16_t *wq12, *wq3;    // weight-only modes: the blocks' weights de-quantised once per call, [depth][2 hidden][w] / [depth][w][hidden]
   float* f8s;            // fp8-MFMA regime: the activations' row scales — [steps * rows] adaLN operand, [rows] w12 operand, [rows] w3 operand
   int ks12, ks3, ksf;    // split-K requests of the w12 (1 = SwiGLU in the GEMM epilogue), w3 and final GEMMs
@@ -129,7 +131,10 @@ static size_t rf_wide_carve(const mn_rf_head* h, int rows, void* ws, size_t cap,
   o->hs = cv.take<bf16_t>((size_t)2 * rows * h->llm_hidden);
   o->zs = cv.take<bf16_t>((size_t)2 * rows * h->z_dim);
   o->y = cv.take<bf16_t>((size_t)2 * SR * h->w);
-  o->ya = cv.take<bf16_t>((size_t)2 * rows * h->w);
+  // up to 64 rows, whose tiles' loads bound w12: an odd number of 128-byte lines a row, so that the rows of a K-tile meet every L2 channel (rows
+  // of 6144 bytes: 36 rows 29 .. 32 us against 26 .. 29; nothing at 1536 rows)
+  o->lda = rows <= 64 && !rf_f8_mfma(h) && (h->w / 64) % 2 == 0 ? h->w + 64 : h->w;
+  o->ya = cv.take<bf16_t>((size_t)2 * rows * o->lda);
   o->yb = cv.take<bf16_t>((size_t)2 * rows * h->hidden);
   const bool f8 = rf_f8_mfma(h);                          // (the e4m3 bytes ARE the operands: no bf16 expansion of the blocks)
   o->wq12 = cv.take<bf16_t>(h->wfmt && !f8 ? (size_t)h->depth * 2 * h->hidden * h->w : 0);
@@ -211,14 +216,14 @@ static int rf_sample_wide(const mn_rf_head* h, const float* hidden, int64_t ld_h
     }
   }
   const float step = 1.0f / (float)h->steps;
-  const int64_t lo_a = (int64_t)rows * W, lo_b = (int64_t)rows * HID;
+  const int64_t LA = w.lda, lo_a = (int64_t)rows * LA, lo_b = (int64_t)rows * HID;
   for (int s = 0; s < h->steps; ++s) {
     const float* ada = w.ada + (int64_t)s * rows * A;
     // h = input_proj(x); ya = split(in_ln_0(h) * (1 + scale_0) + shift_0)
     memset(&g, 0, sizeof(g));
     g.xin = w.x; g.kin = T; g.win = h->in_w; g.bin = h->in_b; g.h_out = w.hh; g.ldho = W;
     g.norm = 2; g.ng = h->ln_g[0]; g.nb = h->ln_b[0]; g.eps = 1e-6f; g.shift = ada; g.scale = ada + W; g.ldmod = A;
-    g.Y = w.ya; g.ldy = W; g.y_lo_off = lo_a; g.M = rows; g.D = W;
+    g.Y = w.ya; g.ldy = LA; g.y_lo_off = lo_a; g.M = rows; g.D = W;
     if (f8) { g.y_lo_off = 0; g.Y8 = reinterpret_cast<uint8_t*>(w.ya + lo_a); g.y8_scale = s_a; }
     wide_glue(g, st);
     for (int b = 0; b < h->depth; ++b) {
@@ -246,20 +251,20 @@ static int rf_sample_wide(const mn_rf_head* h, const float* hidden, int64_t ld_h
         g.gate = mod + 2 * W; g.ldgate = A; g.h_out = w.hh; g.ldho = W;
         g.norm = 2; g.ng = last8 ? nullptr : h->ln_g[b + 1]; g.nb = last8 ? nullptr : h->ln_b[b + 1]; g.eps = 1e-6f;
         g.shift = nmod8; g.scale = nmod8 + W; g.ldmod = A;
-        g.Y = w.ya; g.ldy = W; g.y_lo_off = lo_a; g.M = rows; g.D = W;
+        g.Y = w.ya; g.ldy = LA; g.y_lo_off = lo_a; g.M = rows; g.D = W;
         if (!last8) { g.y_lo_off = 0; g.Y8 = ya8; g.y8_scale = s_a; }      // the next block multiplies e4m3: hi rows (unused, kept for inspection) + bytes; the last one feeds the hi/lo final layer
         wide_glue(g, st);
         continue;
       }
       if (w.ks12 > 1) {
-        a = g256_hilo(w.ya, W, lo_at(LO_RF_W12, lo_a), w12b, W, nullptr, w.pbuf, 2 * HID, rows, 2 * HID, W);
+        a = g256_hilo(w.ya, LA, lo_at(LO_RF_W12, lo_a), w12b, W, nullptr, w.pbuf, 2 * HID, rows, 2 * HID, W);
         a.c_zstride = (int64_t)rows * 2 * HID;
         const int nz12 = mn_gemm256_ex(&a, MN_G256_F32, w.ks12, stream);
         if (nz12 < 0) return nz12;
         hipLaunchKernelGGL(rf_swiglu_slabs_kernel, dim3(mn_cdiv((int64_t)rows * (HID / 4), 256)), dim3(256), 0, st, w.pbuf, nz12,
                            (int64_t)rows * 2 * HID, h->b12[b], w.yb, lo_b, rows, HID);
       } else {
-        a = g256_hilo(w.ya, W, lo_at(LO_RF_W12, lo_a), w12b, W, h->b12[b], w.yb, HID, rows, HID, W);
+        a = g256_hilo(w.ya, LA, lo_at(LO_RF_W12, lo_a), w12b, W, h->b12[b], w.yb, HID, rows, HID, W);
         a.w_pair_rows = HID; a.c_lo_off = lo_b;
         MN_TRYZ(mn_gemm256_ex(&a, MN_G256_SWIGLU_SPLIT, 1, stream));
       }
@@ -274,10 +279,10 @@ static int rf_sample_wide(const mn_rf_head* h, const float* hidden, int64_t ld_h
       g.gate = mod + 2 * W; g.ldgate = A; g.h_out = w.hh; g.ldho = W;
       g.norm = 2; g.ng = last ? nullptr : h->ln_g[b + 1]; g.nb = last ? nullptr : h->ln_b[b + 1]; g.eps = 1e-6f;
       g.shift = nmod; g.scale = nmod + W; g.ldmod = A;
-      g.Y = w.ya; g.ldy = W; g.y_lo_off = lo_a; g.M = rows; g.D = W;
+      g.Y = w.ya; g.ldy = LA; g.y_lo_off = lo_a; g.M = rows; g.D = W;
       wide_glue(g, st);
     }
-    a = g256_hilo(w.ya, W, lo_at(LO_RF_FIN, lo_a), h->fin_w, W, nullptr, w.pbuf, T, rows, T, W);
+    a = g256_hilo(w.ya, LA, lo_at(LO_RF_FIN, lo_a), h->fin_w, W, nullptr, w.pbuf, T, rows, T, W);
     a.c_zstride = (int64_t)rows * T;
     const int nz = mn_gemm256_ex(&a, MN_G256_F32, w.ksf, stream);
     if (nz < 0) return nz;

@@ -1,0 +1,42 @@
+"""Hi/lo products of up to 64 rows (tiles of 32, 48 and 64 rows, 64 and 128 columns): edges of the tiles in rows and columns, one K-tile up to more than
+the LDS pipelines hold, every epilogue; and the flow sampler on both sides of the row counts its routes change at.  Tolerances as in test_gpu_gemm_tile."""
+import pytest
+import torch
+
+from tests import test_gpu_gemm_tile as G
+
+pytestmark = pytest.mark.gpu
+dev_lib = G.dev_lib
+
+
+@pytest.mark.parametrize("M", [1, 16, 31, 32, 33, 47, 48, 49, 63, 64])
+def test_rule(M):
+    for N, K in ((4, 64), (60, 128), (132, 448), (1028, 1024), (8196, 320)):
+        G.test_forms(M, N, K)
+
+
+@pytest.mark.parametrize("form", [5, 6, 7])
+def test_forms_in_turn(dev_lib, form):
+    dev_lib.mn_gemm_tile_tune(form)
+    for M, N, K in ((1, 4, 64), (31, 28, 128), (33, 36, 192), (48, 60, 256), (49, 68, 320), (65, 132, 384), (97, 516, 1024)):
+        G.test_forms(M, N, K)
+
+
+@pytest.mark.parametrize("rows, images", [(5, 5), (6, 3), (6, 2), (23, 23), (32, 16), (33, 11), (64, 32)])
+def test_sampler(rows, images):
+    """A flow head of whole tiles: the batch's rows against the same rows two images at a time."""
+    from ming_univision_amd import configuration as C
+    from ming_univision_amd.rf_head import RectifiedFlowHead
+    from ming_univision_amd.synth import synth_state_dict
+    w = 384                                          # six K-tiles a row: the rows of w12's operand lie seven apart
+    shapes = {"vis_head.0.weight": (w, 128), "vis_head.0.bias": (w,), "vis_head.1.weight": (w,), "vis_head.1.bias": (w,)}
+    shapes.update(C.rf_param_shapes(w, 2, w))
+    sd = {k: v.to("cuda", torch.bfloat16) for k, v in synth_state_dict(shapes, 3).items()}
+    head = RectifiedFlowHead(sd, 128, dict(diffloss_w=w, diffloss_d=2, num_sampling_steps="4", gen_method="flow_matching_swiglu-4", vis_head_arch="linear2-norm"))
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    per = rows // images
+    hid, noise = torch.randn(rows, 128, generator=g, device="cuda"), torch.randn(images, 32, generator=g, device="cuda")
+    whole = head.sample(hid, noise, text_cfg=3.0, image_cfg=1.1, n_images=images)
+    for i in range(images):
+        one = head.sample(hid[i * per:(i + 1) * per].contiguous(), noise[i:i + 1].contiguous(), text_cfg=3.0, image_cfg=1.1, n_images=1)
+        assert float((whole[i] - one[0]).norm() / one.norm()) < 1e-4

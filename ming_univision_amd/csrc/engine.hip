@@ -763,43 +763,86 @@ extern "C" int mn_rf_sample(const mn_rf_head* h, const float* hidden, int64_t ld
 // ===========================================================================================
 // Bailing-MoE decoder stack step
 // ===========================================================================================
-// ---- grouped expert path (rows >= 5): every distinct expert's weights are streamed once on the matrix cores ----
-// Block 0 sorts the (row, slot) pairs by expert — off[g] .. off[g+1] are the sorted positions of group g, a pair's
-// rank inside its group is its pair index order, so the layout is deterministic; blocks 1..M split row m-1 of the
-// normalised activations into bf16 hi / lo halves for the MFMA kernel.
+// ---- grouped expert path: every distinct expert's weights are streamed once on the matrix cores ----
+// Sorts the P <= 1024 (row, slot) pairs by expert (G <= 256 groups): off[g] .. off[g + 1] are the sorted positions of group g, a pair's rank inside its group is
+// its pair index order, so the layout is deterministic.  64 pairs at a time match their groups bit by bit; what they count is summed over the chunks
+// before.  (A pair that looks at every pair before it: 13.4 us at 64 rows of 8 slots, 8.0 at 36; here 4.5, as little as a launch takes.)
+template <int NT>
+__device__ __forceinline__ void sort_pairs(const int32_t* __restrict__ topk_idx, int P, int n_slot, int G, int32_t* __restrict__ off, int32_t* __restrict__ xrows,
+                                           int32_t* __restrict__ pair_pos) {
+  constexpr int NW = NT / 64, CW = 16 / NW;                  // chunks of 64 pairs per wave
+  __shared__ int32_t cnt[16][256], s_off[257], s_wave[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int i = tid; i < 16 * 256; i += NT) cnt[i >> 8][i & 255] = 0;
+  int e[CW], rank[CW];
+#pragma unroll
+  for (int j = 0; j < CW; ++j) {                             // (a row of NaN logits has no top-k: its pairs go to some group)
+    const int p = 64 * (j * NW + wave) + lane;
+    e[j] = p < P ? min((int)min((uint32_t)topk_idx[p], (uint32_t)0x7fffffff), G - 1) : 0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < CW; ++j) {
+    const int c = j * NW + wave, p = 64 * c + lane;
+    uint64_t same = __ballot(p < P);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const uint64_t set = __ballot((e[j] >> b) & 1);
+      same &= ((e[j] >> b) & 1) ? set : ~set;
+    }
+    rank[j] = __popcll(same & (((uint64_t)1 << lane) - 1));
+    if (p < P && rank[j] == 0) cnt[c][e[j]] = __popcll(same);
+  }
+  __syncthreads();
+  int total = 0;
+  if (tid < 256) {
+#pragma unroll
+    for (int c = 0; c < 16; ++c) { const int t = cnt[c][tid]; cnt[c][tid] = total; total += t; }
+    int upto = total;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(upto, o, 64);
+      upto += lane >= o ? t : 0;
+    }
+    if (lane == 63) s_wave[wave] = upto;
+    s_off[tid + 1] = upto;
+    if (tid == 0) s_off[0] = 0;
+  }
+  __syncthreads();
+  if (tid < 256) {
+    int before = 0;
+    for (int w = 0; w < wave; ++w) before += s_wave[w];
+    s_off[tid + 1] += before;
+  }
+  __syncthreads();
+  for (int g = tid; g <= G; g += NT) off[g] = s_off[g];
+#pragma unroll
+  for (int j = 0; j < CW; ++j) {
+    const int c = j * NW + wave, p = 64 * c + lane;
+    if (p >= P) continue;
+    const int pos = s_off[e[j]] + cnt[c][e[j]] + rank[j];
+    xrows[pos] = p / n_slot;
+    pair_pos[p] = pos;
+  }
+}
+
+__global__ __launch_bounds__(1024) void moe_sort_pairs_kernel(const int32_t* __restrict__ topk_idx, int P, int n_slot, int G, int32_t* __restrict__ off,
+                                                              int32_t* __restrict__ xrows, int32_t* __restrict__ pair_pos) {
+  sort_pairs<1024>(topk_idx, P, n_slot, G, off, xrows, pair_pos);
+}
+
+// Block 0 sorts; blocks 1..M split row m-1 of the normalised activations into bf16 hi / lo halves for the MFMA kernel.
 __global__ __launch_bounds__(256) void moe_group_split_kernel(const int32_t* __restrict__ topk_idx, int M, int n_slot, int G,
                                                               int32_t* __restrict__ off, int32_t* __restrict__ xrows,
                                                               int32_t* __restrict__ pair_pos, const float* __restrict__ xn,
                                                               int H, bf16_t* __restrict__ Y) {
-  __shared__ int32_t s_idx[1024];
-  __shared__ int32_t s_off[257];
-  const int tid = threadIdx.x;
-  if (blockIdx.x > 0) {
-    const int m = blockIdx.x - 1;
-    for (int k = tid; k < H; k += 256) {
-      const float v = xn[(int64_t)m * H + k];
-      const bf16_t hi = f32_to_bf16(v);
-      Y[(int64_t)m * H + k] = hi;
-      Y[(int64_t)(M + m) * H + k] = f32_to_bf16(v - bf16_to_f32(hi));
-    }
-    return;
-  }
-  const int P = M * n_slot;                         // <= 1024 pairs, G <= 256 groups (checked by the caller)
-  for (int p = tid; p < P; p += 256) s_idx[p] = topk_idx[p];
-  for (int g = tid; g <= G; g += 256) s_off[g] = 0;
-  __syncthreads();
-  for (int p = tid; p < P; p += 256) atomicAdd(&s_off[s_idx[p] + 1], 1);
-  __syncthreads();
-  if (tid == 0) for (int g = 0; g < G; ++g) s_off[g + 1] += s_off[g];
-  __syncthreads();
-  for (int g = tid; g <= G; g += 256) off[g] = s_off[g];
-  for (int p = tid; p < P; p += 256) {
-    const int e = s_idx[p];
-    int rank = 0;
-    for (int q = 0; q < p; ++q) rank += (s_idx[q] == e);
-    const int pos = s_off[e] + rank;
-    xrows[pos] = p / n_slot;
-    pair_pos[p] = pos;
+  if (blockIdx.x == 0) { sort_pairs<256>(topk_idx, M * n_slot, n_slot, G, off, xrows, pair_pos); return; }
+  const int m = blockIdx.x - 1;
+  for (int k = threadIdx.x; k < H; k += 256) {
+    const float v = xn[(int64_t)m * H + k];
+    const bf16_t hi = f32_to_bf16(v);
+    Y[(int64_t)m * H + k] = hi;
+    Y[(int64_t)(M + m) * H + k] = f32_to_bf16(v - bf16_to_f32(hi));
   }
 }
 
@@ -856,13 +899,17 @@ __global__ __launch_bounds__(1024) void llm_glue_kernel(int mode, const float* _
       v = *reinterpret_cast<const f4*>(h + (int64_t)m * H + col);
       if (mode == 1) {
         const float* pp = P + (int64_t)m * H + col;
+        f4 y = {0.f, 0.f, 0.f, 0.f};                // (the small sum first: the stream is rounded once)
         for (int z0 = 0; z0 < nz; z0 += 8) {        // eight slabs' loads in flight (a one-by-one loop is nz dependent round trips)
           f4 t[8];
 #pragma unroll
           for (int j = 0; j < 8; ++j) t[j] = z0 + j < nz ? *reinterpret_cast<const f4*>(pp + (int64_t)(z0 + j) * slab) : f4{0.f, 0.f, 0.f, 0.f};
-          for (int j = 0; j < 8; ++j) v += t[j];                      // (the one-by-one loop's order: same bits)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) y += t[j];
         }
+        v += y;
       } else if (mode == 2) {
+        f4 sum = {0.f, 0.f, 0.f, 0.f};
         for (int s = 0; s < n_slot; s += 4) {       // four slots x nz slabs of independent 16-byte loads in flight
           const float* pp[4];
           float wv[4];
@@ -878,8 +925,9 @@ __global__ __launch_bounds__(1024) void llm_glue_kernel(int mode, const float* _
             for (int j = 0; j < 4; ++j) y[j] += *reinterpret_cast<const f4*>(pp[j] + z * slab);
           }
 #pragma unroll
-          for (int j = 0; j < 4; ++j) v += wv[j] * y[j];
+          for (int j = 0; j < 4; ++j) sum += wv[j] * y[j];
         }
+        v += sum;
       }
     }
     if (mode != 3) *reinterpret_cast<f4*>(h + (int64_t)m * H + col) = v;
@@ -902,67 +950,6 @@ __global__ __launch_bounds__(1024) void llm_glue_kernel(int mode, const float* _
       *reinterpret_cast<u2*>(Y + (int64_t)m * H + col) = u2{(uint32_t)hi[0] | ((uint32_t)hi[1] << 16), (uint32_t)hi[2] | ((uint32_t)hi[3] << 16)};
       *reinterpret_cast<u2*>(Y + (int64_t)(M + m) * H + col) = u2{(uint32_t)lo[0] | ((uint32_t)lo[1] << 16), (uint32_t)lo[2] | ((uint32_t)lo[3] << 16)};
     }
-  }
-}
-
-// Router tail in ONE workgroup: reduce the gate GEMV's K-slice partials, softmax + top-k + renormalise per row (one wave
-// per row, 64 experts = 64 lanes; BailingMoeGate.forward :505-520), append the shared pseudo-experts, and — when off is
-// given — sort the (row, slot) pairs by expert for the grouped expert GEMMs (same layout as moe_group_split_kernel).
-__global__ __launch_bounds__(1024) void moe_route_group_kernel(const float* __restrict__ P, int nz, int M, int E, int top_k,
-                                                               int norm_topk_prob, int n_shared, float* __restrict__ topk_w,
-                                                               int32_t* __restrict__ topk_idx, int G, int32_t* __restrict__ off,
-                                                               int32_t* __restrict__ xrows, int32_t* __restrict__ pair_pos) {
-  __shared__ int32_t s_idx[1024];
-  __shared__ int32_t s_off[257];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int n_slot = top_k + n_shared;
-  for (int m = wave; m < M; m += 16) {
-    float s = -INFINITY;
-    if (lane < E) {
-      s = 0.f;
-      for (int z0 = 0; z0 < nz; z0 += 8) {          // eight slabs' loads in flight
-        float t[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) t[j] = z0 + j < nz ? P[((int64_t)(z0 + j) * M + m) * E + lane] : 0.f;
-        for (int j = 0; j < 8; ++j) s += t[j];                    // (the one-by-one loop's order: same bits)
-      }
-    }
-    const float mx = wave_max(s);
-    float p = lane < E ? __expf(s - mx) : 0.f;
-    p = p / wave_sum(p);
-    float cur = lane < E ? p : -1.f, wsum = 0.f, myw = 0.f;
-    int myidx = 0;
-    for (int k = 0; k < top_k; ++k) {             // iterative arg-max; ties -> lowest expert index
-      const float best = wave_max(cur);
-      const int sel = __ffsll((long long)__ballot(cur == best)) - 1;
-      if (lane == k) { myw = best; myidx = sel; }
-      if (lane == sel) cur = -1.f;
-      wsum += best;
-    }
-    if (lane < n_slot) {
-      const int idx = lane < top_k ? myidx : E + (lane - top_k);
-      const float wv = lane < top_k ? ((norm_topk_prob && top_k > 1) ? myw / wsum : myw) : 1.0f;
-      topk_idx[m * n_slot + lane] = idx;
-      topk_w[m * n_slot + lane] = wv;
-      s_idx[m * n_slot + lane] = idx;
-    }
-  }
-  if (!off) return;
-  const int Pn = M * n_slot;
-  for (int g = tid; g <= G; g += 1024) s_off[g] = 0;
-  __syncthreads();
-  for (int p = tid; p < Pn; p += 1024) atomicAdd(&s_off[s_idx[p] + 1], 1);
-  __syncthreads();
-  if (tid == 0) for (int g = 0; g < G; ++g) s_off[g + 1] += s_off[g];
-  __syncthreads();
-  for (int g = tid; g <= G; g += 1024) off[g] = s_off[g];
-  for (int p = tid; p < Pn; p += 1024) {
-    const int e = s_idx[p];
-    int rank = 0;
-    for (int q = 0; q < p; ++q) rank += (s_idx[q] == e);
-    const int pos = s_off[e] + rank;
-    xrows[pos] = p / n_slot;
-    pair_pos[p] = pos;
   }
 }
 
@@ -1027,22 +1014,23 @@ static bool moe_mfma_ok(const mn_llm* m, int rows) {
          m->n_experts + m->n_shared_slots <= 256 && (m->hidden % 8) == 0 && (m->moe_inter % 8) == 0;   // % 4: vector glue
 }
 
-// 2..32 rows run the decoder stack as a chain of weight-streaming launches and fused glue kernels (4 columns per thread,
+// 2..64 rows run the decoder stack as a chain of weight-streaming launches and fused glue kernels (4 columns per thread,
 // one wave per router row: 64 experts at most).  Measured end to end against the unfused sequence (same box, tokens/s):
-// 2 rows 78.5 vs 76.5, 8 rows 254 vs 247, 16 rows 451 vs 442, 32 rows 699 vs 698; at 64 rows the one-workgroup-per-row
-// glue kernels lose to the wider unfused ones (1084 vs 1122), so the chain stops at 32.
-static int g_chain_max_rows = 32, g_chain_router = 1, g_chain_fuse_ln1 = 1;
+// 2 rows 78.5 vs 76.5, 8 rows 254 vs 247, 16 rows 451 vs 442; with the router as a launch of a workgroup a row (moe_router_rows) and the sort that matches 64 pairs at a
+// time, eleven launches a layer instead of eighteen: a decode step and logits of 64 rows over 1100
+// tokens 9.90 -> 9.09 ms, a visual token of 36 rows 18.2 -> 17.9 (with a one-workgroup router and sort the chain stopped at 32 rows).
+static int g_chain_max_rows = 64, g_chain_fuse_ln1 = 1;
 static int g_moe_gate_up = 1, g_moe_gate_up_rows = 1, g_moe_gate_up_chain_rows = 2, g_moe_gate_up_chain_all = 0;      // (chain: int8 / NF4 by default — bf16 / e4m3 keep the pair launches: 2.25 vs 2.64 ms, 1.71 vs 1.84)      // the one-launch router + gate/up of 1-row steps (dev-library A/B: mn_moe_tune_gate_up)
 bool moe_router_rows_ok(int M, int H, int E);
 int moe_router_rows(float* h, const float* P, int nz, const uint16_t* norm_w, float eps, const uint16_t* gate_w, int M, int H, int E, int top_k,
-                    int norm_topk_prob, int n_shared_slots, float* x_norm, int32_t* topk_idx, float* topk_w, float* logits_ws, void* stream);
+                    int norm_topk_prob, int n_shared_slots, float* x_norm, uint16_t* y, int32_t* topk_idx, float* topk_w, float* logits_ws, void* stream);
 #ifdef MN_DEV_HOOKS
 extern "C" MN_DEV_API void mn_moe_tune_gate_up(int on, int max_rows) { g_moe_gate_up = on; g_moe_gate_up_rows = max_rows & 0xff; g_moe_gate_up_chain_rows = (max_rows >> 8) & 0xff; g_moe_gate_up_chain_all = (max_rows >> 16) & 1; }
-extern "C" MN_DEV_API void mn_llm_tune_chain(int max_rows) { g_chain_max_rows = max_rows & 0xffff; g_chain_router = (max_rows >> 16) & 1 ? 0 : 1; g_chain_fuse_ln1 = (max_rows >> 17) & 1 ? 0 : 1; }   // A/B hook (tools/): bit 16 = the one-launch router of the chain OFF, bit 17 = RMSNorm(ln1) as its own glue launch
+extern "C" MN_DEV_API void mn_llm_tune_chain(int max_rows) { g_chain_max_rows = max_rows & 0xffff; g_chain_fuse_ln1 = (max_rows >> 17) & 1 ? 0 : 1; }   // A/B hook (tools/): bit 17 = RMSNorm(ln1) as its own glue launch
 #endif
 static bool llm_chain_ok(const mn_llm* m, int rows) {
   return rows >= 2 && rows <= g_chain_max_rows && (m->hidden % 8) == 0 && m->hidden <= 4096 && ((m->n_q * m->head_dim) % 8) == 0 &&
-         m->n_experts <= 64 && rows * (m->top_k + m->n_shared_slots) <= 1024 && m->n_experts + m->n_shared_slots <= 256;
+         m->n_experts <= 64 && m->top_k + m->n_shared_slots <= 64 && rows * (m->top_k + m->n_shared_slots) <= 1024;
 }
 
 struct LlmWs {
@@ -1228,7 +1216,7 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
   // append ride the attention launch
   const bool fuse_attn = (flags & MN_STEP_DISTINCT_SEQUENCES) && mn_attn_fused_ok(M, nq, nkv, hd, t_max);
   if (llm_chain_ok(m, M) && !(image_mask && m->image_gate)) {
-    // ---- chain path: 12 launches per layer instead of 18 (2 rows: 6 — QKV with the RMSNorm prologue, attention with RoPE + KV append, dense,
+    // ---- chain path: 11 launches per layer instead of 18 (2 rows: 6 — QKV with the RMSNorm prologue, attention with RoPE + KV append, dense,
     // the one-launch router, the expert pairs' gate/up, the down projection into h).  glue = llm_glue_kernel.
     const int E = m->n_experts, S = m->n_shared_slots, G = E + S, ad = nq * hd, P = M * n_slot;
     // 2 rows (the CFG rows of one image): the experts run as router + gate/up in ONE launch and the wave-segmented down projection,
@@ -1283,25 +1271,11 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
         nz2 = 0;
         continue;
       }
-      // <= 4 rows on the fp32-FMA expert kernels: residual + RMSNorm(ln2) + gate + top-k in ONE launch (decode_ops.hip) instead of glue,
-      // gate launch and the one-workgroup top-k
-      if (!grouped && g_chain_router && moe_router_rows_ok(M, H, E)) {
-        MN_TRY(moe_router_rows(w.h, w.pp, nz, m->ln2[l], m->rms_eps, m->gate[l], M, H, E, m->top_k, m->norm_topk_prob, S, w.xn, w.ti, w.tw,
-                               w.logits, stream));
-        route_capture(l, w.ti, M, n_slot, st);
-        goto experts_2rows;
-      }
-      // glue: h += dense partials; RMSNorm(ln2) -> xn (fp32 for the 2-row expert kernels) and yh (gate + expert operand)
-      hipLaunchKernelGGL(llm_glue_kernel, dim3(M), dim3(gt), 0, st, 1, (const float*)nullptr, (int64_t)0, 1, (const float*)w.pp, nz,
-                         (int64_t)M * H, (const int32_t*)nullptr, (const float*)nullptr, n_slot, w.h, M, H, m->ln2[l],
-                         m->rms_eps, grouped ? (float*)nullptr : w.xn, w.yh);
-      // gate launch -> partials; ONE workgroup does softmax / top-k / expert sort  (:505-520, 565-592)
-      nz = mn_stream_mfma(w.yh, m->gate[l], w.pp, M, E, H, stream);
-      if (nz < 0) return nz;
-      hipLaunchKernelGGL(moe_route_group_kernel, dim3(1), dim3(1024), 0, st, (const float*)w.pp, nz, M, E, m->top_k,
-                         m->norm_topk_prob, S, w.tw, w.ti, G, grouped ? w.moe.off : (int32_t*)nullptr, w.moe.xrows,
-                         w.moe.pair_pos);
+      // residual + RMSNorm(ln2) + gate + top-k in ONE launch (decode_ops.hip): -> xn (fp32, the pair kernels) or yh (the grouped experts' operand)  (:505-520, 565-592)
+      MN_TRY(moe_router_rows(w.h, w.pp, nz, m->ln2[l], m->rms_eps, m->gate[l], M, H, E, m->top_k, m->norm_topk_prob, S, grouped ? (float*)nullptr : w.xn,
+                             grouped ? w.yh : (uint16_t*)nullptr, w.ti, w.tw, w.logits, stream));
       route_capture(l, w.ti, M, n_slot, st);
+      if (grouped) hipLaunchKernelGGL(moe_sort_pairs_kernel, dim3(1), dim3(1024), 0, st, w.ti, P, n_slot, G, w.moe.off, w.moe.xrows, w.moe.pair_pos);
       if (grouped) {
         nz = stream_grouped(m->wfmt, w.yh, M, m->w_gate_up[l], (int64_t)2 * I * H, m->wfmt ? m->w_gate_up_scale[l] : nullptr, 2 * I,
                             w.moe.p1, P, w.moe.off, w.moe.xrows, G, M, 2 * I, H, stream);
@@ -1312,7 +1286,6 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
                              w.moe.off, nullptr, G, M, H, I, stream);
         if (nz2 < 0) return nz2;
       } else {   // 2 rows: (row, expert) pairs on the fp32-FMA kernels, accumulated straight into h
-      experts_2rows:
         mn_skinny_args a = sk(w.xn, H, m->w_gate_up[l], H, nullptr, w.hmid, I, 1, I, H);
         a.epilogue = MN_EPI_SWIGLU;
         a.batch = M * n_slot; a.w_index = w.ti; a.w_batch_stride = (int64_t)2 * I * H;

@@ -189,3 +189,149 @@ __global__ __launch_bounds__(512) void rows_kc_kernel(const mn_skinny_args a, in
     }
   }
 }
+
+// The same with rows and weights on their way through LDS: a wave instruction fetches whole 64- or 128-byte pieces of a row (64 bytes a cycle and CU), where
+// operands read straight from memory, 16 rows apart lane by lane, come at a quarter of that (38 GB/s a CU: 7 of 12 us for 32 rows of 2048).  Each wave has a ring of
+// its own, so nothing but the sum at the end is a barrier.  What is left is the split (130 vector instructions for 32 values of 32 rows, 4 us of the
+// 2048).  Rows of 16-byte aligned values; 2048 x 2048 at 32 rows 14.5 -> 11.1 us.
+template <int MT, int NT, int PRO>
+__global__ __launch_bounds__(512) void rows_kc_lds_kernel(const mn_skinny_args a, int paired) {
+  constexpr int NW = 8, CK = 64, R = MT * NT * 4, S = 3, XB = MT * 2048, SUB = XB + NT * 1024;      // a ring holds S pieces of 32 values of K: rows of 128 bytes, then weights of 64
+  constexpr int BYTES = NW * S * SUB > NW * R * 256 ? NW * S * SUB : NW * R * 256;
+  __shared__ __attribute__((aligned(1024))) char lds[BYTES];
+  float (*red)[R][64] = reinterpret_cast<float (*)[R][64]>(lds);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const int K = a.K, M = a.M, N = a.N, G = paired ? NT / 2 : NT;             // G: tiles of units per workgroup
+  const int n0 = blockIdx.x * 16 * G;
+  // what this lane fetches: row 8 i + lane / 8 of the rows (16 bytes: slot lane % 8, in the order that leaves no bank twice), row lane / 4 of every weight tile
+  typedef const __attribute__((address_space(1))) void gptr;
+  typedef __attribute__((address_space(3))) void lptr;
+  const int xr = lane >> 3, wr = lane >> 2;
+  const float* xp[2 * MT];
+  int xk[2 * MT];
+#pragma unroll
+  for (int i = 0; i < 2 * MT; ++i) {
+    const int row = 8 * i + xr;
+    xk[i] = 4 * ((lane & 7) ^ ((row >> 1) & 7));
+    xp[i] = a.x + (int64_t)min(row, M - 1) * a.ldx;
+  }
+  const int wk = 8 * ((lane & 3) ^ ((wr >> 2) & 3));
+  const bf16_t* wp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wp[t] = a.w + (int64_t)(min(n0 + 16 * (t % G) + wr, N - 1) + (t >= G ? N : 0)) * K;
+  char* ring = lds + wave * (S * SUB);
+  f32x4 acc[MT][NT], low[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[i][t] = low[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // K is a multiple of 8: 8 values are all inside K or all beyond it, where the row's start is fetched and both operands become zeros
+  const int pieces = wave * CK < K ? 2 * ((K - wave * CK + NW * CK - 1) / (NW * CK)) : 0;
+  auto fetch = [&](int c, int buf) {
+    const int k0 = (wave + NW * (c >> 1)) * CK + 32 * (c & 1);
+    char* dst = ring + buf * SUB;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) __builtin_amdgcn_global_load_lds((gptr*)(wp[t] + (k0 + wk < K ? k0 + wk : 0)), (lptr*)(dst + XB + t * 1024), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) __builtin_amdgcn_global_load_lds((gptr*)(xp[i] + (k0 + xk[i] < K ? k0 + xk[i] : 0)), (lptr*)(dst + i * 1024), 16, 0, 0);
+  };
+#pragma unroll
+  for (int c = 0; c < S; ++c)
+    if (c < pieces) fetch(c, c);
+  int buf = 0;
+  for (int c0 = 0; c0 < pieces; c0 += 2) {
+    const int k0 = (wave + NW * (c0 >> 1)) * CK;
+    f32x4 sum[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) sum[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int k = k0 + 32 * s + 8 * q, left = pieces - 1 - c0 - s;
+      const bool in = k < K;
+      if (left >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (2 * MT + NT)) : "memory");
+      else if (left == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * MT + NT) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      f32x4 cx[MT][2];
+      u32x4 cw[NT];
+      const char* src = ring + buf * SUB;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) cx[i][h] = *reinterpret_cast<const f32x4*>(src + (16 * i + r) * 128 + (((2 * q + h) ^ ((r >> 1) & 7)) << 4));
+#pragma unroll
+      for (int t = 0; t < NT; ++t) cw[t] = *reinterpret_cast<const u32x4*>(src + XB + t * 1024 + r * 64 + ((q ^ ((r >> 2) & 3)) << 4));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (c0 + s + S < pieces) fetch(c0 + s + S, buf);           // the piece is in registers
+      buf = buf + 1 == S ? 0 : buf + 1;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        f32x4 v0 = cx[i][0], v1 = cx[i][1];
+        if (PRO == MN_PRO_SILU) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { v0[e] = silu_f(v0[e]); v1[e] = silu_f(v1[e]); }
+        }
+        if (!in) v0 = v1 = f32x4{0.f, 0.f, 0.f, 0.f};
+        u32x4 part[3];
+        float most = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) most = fmaxf(most, fmaxf(fabsf(v0[e]), fabsf(v1[e])));
+        if (__ballot(most >= BF16_TO_INF) == 0) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) { split3_pk_bf16<false>(v0[2 * e], v0[2 * e + 1], part, e); split3_pk_bf16<false>(v1[2 * e], v1[2 * e + 1], part, 2 + e); }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) { split3_pk_bf16<true>(v0[2 * e], v0[2 * e + 1], part, e); split3_pk_bf16<true>(v1[2 * e], v1[2 * e + 1], part, 2 + e); }
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const bf16x8 w = __builtin_bit_cast(bf16x8, in ? cw[t] : u32x4{0, 0, 0, 0});
+#pragma unroll
+          for (int p = 2; p >= 0; --p) sum[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, part[p]), w, sum[i][t], 0, 0, 0);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float a0 = acc[i][t][e], l0 = low[i][t][e];
+          two_sum(a0, l0, sum[i][t][e]);
+          acc[i][t][e] = a0; low[i][t][e] = l0;
+        }
+  }
+  __syncthreads();                                     // the rings are read: the tiles' sums take their place
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = acc[i][t][e] + low[i][t][e];
+        red[wave][(i * 4 + e) * NT + t][lane] = v == v ? v : acc[i][t][e];   // a sum at infinity has no error term
+      }
+  }
+  __syncthreads();
+  for (int j = wave; j < 4 * MT; j += NW) {                                  // row 16 (j / 4) + 4 q + j % 4 of every tile
+    const int ml = 16 * (j >> 2) + 4 * q + (j & 3);
+    float y[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      float p[NW];
+#pragma unroll
+      for (int w = 0; w < NW; ++w) p[w] = red[w][j * NT + t][lane];
+      y[t] = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+    }
+    if (ml >= M) continue;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int n = n0 + 16 * t + r;
+      if (t >= G || n >= N) continue;
+      medium_finish(a, ml, n, y[t], NT > 1 ? y[NT > 1 && paired ? t + NT / 2 : 0] : 0.f);
+    }
+  }
+}

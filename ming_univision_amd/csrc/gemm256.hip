@@ -453,13 +453,14 @@ static const TileForm tile_plain[] = {{1, 64, 64, 3.6, 0.23, 0.26, 0.42, 0.30}, 
                                       {4, 128, 128, 4.2, 0.55, 0.85, 1.16, 0.85}, {0, 256, 256, 11.0, 0.85, 1.30, 0, 0}};
 static const TileForm tile_hilo[] = {{1, 64, 64, 3.8, 0.41, 0.42, 0.60, 0.41}, {2, 64, 128, 4.0, 0.64, 0.66, 1.00, 0.58}, {3, 128, 128, 4.2, 0.93, 1.04, 0, 0},
                                      {0, 128, 256, 11.0, 0.87, 1.25, 0, 0}};
-// Up to 64 hi/lo rows: one row of tiles, so every weight byte comes from HBM, and what a CU takes in (rows and weights alike, 45 .. 50 GB/s of them however
+// Up to 128 hi/lo rows: one or two rows of tiles, so every weight byte comes from HBM, and what a CU takes in (rows and weights alike, 45 .. 50 GB/s of them however
 // many loads are in flight) is the time.  So tiles no taller than the rows: 3072 x 16384 with its SwiGLU at 16 rows 19.7 us (32-row tiles) against 28.3 (64), at 36
 // 25.2 (48-row tiles, gate and up in one fragment) against 29.5; and wider ones where slices of K leave enough of them: 8192 x 3072 at 36 rows 13.8 us
-// (64 x 128, 8 slices) against 15.8, at 16 rows 11.5 (32 x 64, 5 slices) against 14.4.  max_m: 0 or the most rows the form takes; split: the split SwiGLU alone.
+// (64 x 128, 8 slices) against 15.8, at 16 rows 11.5 (32 x 64, 5 slices) against 14.4.  At 96 rows 3072 x 16384 with its SwiGLU 33.0 us (64 x 128) against 42.4 (64 x 64)
+// and 51 (128 x 128), 8192 x 3072 20.1 (5 slices) against 24.3 and 29.5.  max_m: 0 or the most rows the form takes; split: the split SwiGLU alone.
 struct FewForm { TileForm f; int max_m; bool split; };
 static const FewForm tile_few[] = {{{5, 32, 64, 3.8, 0.28, 0.36, 0.74, 0.40}, 32, false}, {{6, 48, 64, 3.8, 0.40, 0.44, 0.90, 0.50}, 48, true},
-                                   {{1, 64, 64, 3.8, 0.46, 0.53, 0.95, 0.55}, 64, false}, {{7, 64, 128, 4.0, 0.50, 0.72, 0, 0}, 64, false}};
+                                   {{1, 64, 64, 3.8, 0.46, 0.53, 0.95, 0.55}, 128, false}, {{7, 64, 128, 4.0, 0.50, 0.72, 0, 0}, 128, false}};
 
 static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bool hilo, bool paired) {
   const double w = (double)(mn_cdiv(M, f.bm) * mn_cdiv(N, paired ? f.bn / 2 : f.bn) * nz) / 256.0;
@@ -476,7 +477,7 @@ static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bo
 // the form of a dense M x N x K launch in nz K-slices of Kc, and the estimate of its time
 static int tile_form(int M, int N, int Kc, int nz, bool hilo, int epi, bool may256, double* us) {
   const bool paired = epi_paired(epi);
-  if (hilo && M <= 64) {
+  if (hilo && M <= 128) {
     int best = 0;
     double tb = 1e30;
     for (const FewForm& t : tile_few) {
@@ -615,7 +616,7 @@ extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo) {
     double t;
     tile_form(M, N, Kc, nz, hilo != 0, E_F32, true, &t);
     t += nz * (double)M * N * 8.0 / 4.5e6;
-    if (hilo && M <= 64) t += 0.25 * nz * fmin(1.0, N / 2048.0);         // (a few rows' slabs are read by a few workgroups)
+    if (hilo && M <= 128) t += 0.25 * nz * fmin(1.0, N / 2048.0);         // (a few rows' slabs are read by a few workgroups)
     if (t < tb - 1e-9) { tb = t; best = ks; }
   }
   return best > 1 ? best : 0;

@@ -112,10 +112,10 @@ static size_t rf_wide_carve(const mn_rf_head* h, int rows, void* ws, size_t cap,
   Carver cv(ws, cap, ws == nullptr);
   const int64_t SR = (int64_t)h->steps * rows;
   const int A = h->depth * 3 * h->w + 2 * h->w;
-  // w12: the SwiGLU epilogue needs the whole K sum.  Up to 64 rows one row of 64 x 64 tiles reads every weight byte once and fills the chip from 4096
-  // hidden units on (64 rows x 3072 x 16384: 30.3 us; in two K-slices 29.6 + 8 for the launch behind them); above, cdiv(rows, 128) * hidden / 128
-  // workgroups, and below a chip's worth of them the split-K form + rf_swiglu_slabs_kernel is the faster pair (96 rows: 41.8 against 31 + 8)
-  o->ks12 = (rows <= 64 && h->hidden >= 4096) || mn_cdiv(rows, 128) * (h->hidden / 128) >= 256 ? 1 : rf_wide_ksplit(rows, 2 * h->hidden, h->w);
+  // w12: the SwiGLU epilogue needs the whole K sum.  Up to 128 rows a row or two of tiles reads every weight byte once and fills the chip from 4096 hidden
+  // units on (96 rows x 3072 x 16384: 33 us; in two K-slices 31 + 8 for the launch behind them); above, cdiv(rows, 128) * hidden / 128
+  // workgroups, and below a chip's worth of them the split-K form + rf_swiglu_slabs_kernel is the faster pair
+  o->ks12 = (rows <= 128 && h->hidden >= 4096) || mn_cdiv(rows, 128) * (h->hidden / 128) >= 256 ? 1 : rf_wide_ksplit(rows, 2 * h->hidden, h->w);
   o->ks3 = rf_f8_mfma(h) ? mn_gemm256_f8_plan_ksplit(rows, h->w, h->hidden) : rf_wide_ksplit(rows, h->w, h->hidden);
   o->ksf = rf_wide_ksplit(rows, h->target, h->w);
   const size_t p3 = (size_t)mn_gemm256_slices(h->hidden, o->ks3) * rows * h->w;

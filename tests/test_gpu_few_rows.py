@@ -1,4 +1,4 @@
-"""Hi/lo products of up to 64 rows (tiles of 32, 48 and 64 rows, 64 and 128 columns): edges of the tiles in rows and columns, one K-tile up to more than
+"""Hi/lo products of up to 128 rows (tiles of 32, 48 and 64 rows, 64 and 128 columns): edges of the tiles in rows and columns, one K-tile up to more than
 the LDS pipelines hold, every epilogue; and the flow sampler on both sides of the row counts its routes change at.  Tolerances as in test_gpu_gemm_tile."""
 import pytest
 import torch
@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 dev_lib = G.dev_lib
 
 
-@pytest.mark.parametrize("M", [1, 16, 31, 32, 33, 47, 48, 49, 63, 64])
+@pytest.mark.parametrize("M", [1, 16, 31, 32, 33, 47, 48, 49, 63, 64, 65, 128, 129])
 def test_rule(M):
     for N, K in ((4, 64), (60, 128), (132, 448), (1028, 1024), (8196, 320)):
         G.test_forms(M, N, K)
@@ -22,7 +22,7 @@ def test_forms_in_turn(dev_lib, form):
         G.test_forms(M, N, K)
 
 
-@pytest.mark.parametrize("rows, images", [(5, 5), (6, 3), (6, 2), (23, 23), (32, 16), (33, 11), (64, 32)])
+@pytest.mark.parametrize("rows, images", [(5, 5), (6, 3), (6, 2), (23, 23), (32, 16), (33, 11), (64, 32), (128, 64), (129, 43)])
 def test_sampler(rows, images):
     """A flow head of whole tiles: the batch's rows against the same rows two images at a time."""
     from ming_univision_amd import configuration as C

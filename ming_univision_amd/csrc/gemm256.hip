@@ -138,94 +138,181 @@ __device__ __forceinline__ float gelu_erf_bf16out(float x) {
   return 0.5f * x * one_plus_erf;
 }
 
-// Epilogue of one output tile.  A lane holds, per (i, j), output row 16 i + fr and the 4 CONSECUTIVE columns 16 j + 4 fq .. +3.
-// One lane's 4 CONSECUTIVE output columns n..n+3 of row m (u: the paired "up" values): bias, epilogue, store.
+__host__ __device__ constexpr bool epi_split(int epi) { return epi == E_SWIGLU_SPLIT; }
+__host__ __device__ constexpr bool epi_f32(int epi) { return epi == E_F32 || epi == E_F32_RESID || epi == E_F32_RESID_GATE || epi == E_F32_TAIL_RELU2; }
+
+__device__ __forceinline__ f32x4 bf16x4_f32(u32x2 b) { return f32x4{bf16lo_to_f32(b.x), bf16hi_to_f32(b.x), bf16lo_to_f32(b.y), bf16hi_to_f32(b.y)}; }
+
+// 4 consecutive output columns as bf16 (u: the paired "up" values; lo: the rest of a hi/lo pair).
 // EXACT_GELU: erff itself (the small-tile kernels, whose lanes hold 16 .. 32 values)
-template <int EPI, bool EXACT_GELU = false>
-__device__ __forceinline__ void g256_emit(const G256& p, char* Cz, int m, int n, f32x4 v, f32x4 u, int zslice) {
-  constexpr bool paired = epi_paired(EPI);
-  if (p.bias && zslice == 0) {
-    const u32x2 b = *reinterpret_cast<const u32x2*>(p.bias + n);
-    v += f32x4{bf16lo_to_f32(b.x), bf16hi_to_f32(b.x), bf16lo_to_f32(b.y), bf16hi_to_f32(b.y)};
-    if (paired) {
-      const u32x2 b2 = *reinterpret_cast<const u32x2*>(p.bias + p.w_pair_rows + n);
-      u += f32x4{bf16lo_to_f32(b2.x), bf16hi_to_f32(b2.x), bf16lo_to_f32(b2.y), bf16hi_to_f32(b2.y)};
-    }
+template <int EPI, bool EXACT_GELU>
+__device__ __forceinline__ void g256_pack(f32x4 v, f32x4 u, u32x2& hi, u32x2& lo) {
+  if (EPI == E_BF16_GELU && EXACT_GELU) v = f32x4{gelu_erf_f(v.x), gelu_erf_f(v.y), gelu_erf_f(v.z), gelu_erf_f(v.w)};
+  else if (EPI == E_BF16_GELU) v = f32x4{gelu_erf_bf16out(v.x), gelu_erf_bf16out(v.y), gelu_erf_bf16out(v.z), gelu_erf_bf16out(v.w)};
+  else if (EPI == E_GEGLU_BF16) v = f32x4{gelu_tanh_f(v.x) * u.x, gelu_tanh_f(v.y) * u.y, gelu_tanh_f(v.z) * u.z, gelu_tanh_f(v.w) * u.w};
+  else if (epi_paired(EPI)) v = f32x4{silu_f(v.x) * u.x, silu_f(v.y) * u.y, silu_f(v.z) * u.z, silu_f(v.w) * u.w};
+  if (EPI == E_BF16_RELU2) {                           // the squared relu of a feed-forward's hidden units
+    const f32x4 r = f32x4{fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f)};
+    v = r * r;
   }
-  if (EPI == E_F32) {
-    *reinterpret_cast<f32x4*>(Cz + ((int64_t)m * p.ldc + n) * 4) = v;
-  } else if (EPI == E_F32_TAIL_RELU2) {                // a feed-forward's hidden units beside other projections of the same rows
-    if (n >= p.tail0 && n < p.tail1) {
-      const f32x4 r = f32x4{fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f)};
-      v = r * r;
-      *reinterpret_cast<u32x2*>(p.C2 + (int64_t)m * p.ldc2 + (n - p.tail0)) = u32x2{cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w)};
-    } else {
-      *reinterpret_cast<f32x4*>(Cz + ((int64_t)m * p.ldc + n) * 4) = v;
-    }
-  } else if (EPI == E_GEGLU_BF16) {
-    *reinterpret_cast<u32x2*>(Cz + ((int64_t)m * p.ldc + n) * 2) =
-        u32x2{cvt_pk_bf16(gelu_tanh_f(v.x) * u.x, gelu_tanh_f(v.y) * u.y), cvt_pk_bf16(gelu_tanh_f(v.z) * u.z, gelu_tanh_f(v.w) * u.w)};
-  } else if (EPI == E_F32_RESID) {
-    f32x4* c = reinterpret_cast<f32x4*>(Cz + ((int64_t)m * p.ldc + n) * 4);
-    *c += v;
-  } else if (EPI == E_F32_RESID_GATE) {
-    f32x4* c = reinterpret_cast<f32x4*>(Cz + ((int64_t)m * p.ldc + n) * 4);
-    const f32x4 g = *reinterpret_cast<const f32x4*>(p.gate + (int64_t)m * p.ldgate + n);
-    *c += g * v;
-  } else if (EPI == E_BF16 || EPI == E_BF16_GELU || EPI == E_BF16_RELU2) {
-    if (EPI == E_BF16_GELU && EXACT_GELU) v = f32x4{gelu_erf_f(v.x), gelu_erf_f(v.y), gelu_erf_f(v.z), gelu_erf_f(v.w)};
-    else if (EPI == E_BF16_GELU) v = f32x4{gelu_erf_bf16out(v.x), gelu_erf_bf16out(v.y), gelu_erf_bf16out(v.z), gelu_erf_bf16out(v.w)};
-    if (EPI == E_BF16_RELU2) {                         // the squared relu of a feed-forward's hidden units
-      const f32x4 r = f32x4{fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f)};
-      v = r * r;
-    }
-    *reinterpret_cast<u32x2*>(Cz + ((int64_t)m * p.ldc + n) * 2) = u32x2{cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w)};
-  } else if (EPI == E_SWIGLU_BF16 || EPI == E_SWIGLU_BF16_SCALED) {   // y = silu(gate) * up as plain bf16 (the batched bf16 path)
-    if (EPI == E_SWIGLU_BF16_SCALED) {                 // the input row's factor, applied to its products
-      const float rs = p.row_scale[m];
-      v *= rs; u *= rs;
-    }
-    *reinterpret_cast<u32x2*>(Cz + ((int64_t)m * p.ldc + n) * 2) =
-        u32x2{cvt_pk_bf16(silu_f(v.x) * u.x, silu_f(v.y) * u.y), cvt_pk_bf16(silu_f(v.z) * u.z, silu_f(v.w) * u.w)};
-  } else {  // E_SWIGLU_SPLIT: y = silu(gate) * up, stored as bf16 hi rows and lo rows
+  if (epi_split(EPI)) {
     uint32_t h0, l0, h1, l1;
-    split_pk_bf16(silu_f(v.x) * u.x, silu_f(v.y) * u.y, h0, l0);
-    split_pk_bf16(silu_f(v.z) * u.z, silu_f(v.w) * u.w, h1, l1);
-    bf16_t* c = reinterpret_cast<bf16_t*>(Cz) + (int64_t)m * p.ldc + n;
-    *reinterpret_cast<u32x2*>(c) = u32x2{h0, h1};
-    *reinterpret_cast<u32x2*>(c + p.c_lo_off) = u32x2{l0, l1};
+    split_pk_bf16(v.x, v.y, h0, l0);
+    split_pk_bf16(v.z, v.w, h1, l1);
+    hi = u32x2{h0, h1};
+    lo = u32x2{l0, l1};
+  } else {
+    hi = u32x2{cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w)};
   }
 }
 
-// Epilogue of one output tile of the 8-wave kernel.  A lane holds, per (i, j), output row 16 i + fr and the 4 CONSECUTIVE
-// columns 16 j + 4 fq .. +3.
+// Lanes 16 apart hold 4 columns each of fragments j (a) and j + 1 (b): the even one comes out with both lanes' 4 of j, the odd one with both lanes' 4 of j + 1.
+__device__ __forceinline__ u32x4 pair_lanes16(u32x2 a, u32x2 b) {
+  const auto x = __builtin_amdgcn_permlane16_swap(a.x, b.x, false, false), y = __builtin_amdgcn_permlane16_swap(a.y, b.y, false, false);
+  return u32x4{x[0], y[0], x[1], y[1]};
+}
+
+// Epilogue of a wave's MI x NJ fragments.  A lane holds, per (i, j), output row row(i) and the 4 CONSECUTIVE columns col(j) .. +3, col(j) = col(0) + 16 j (val
+// gives them, u: the paired "up" values).  What bounds it is latency: read where it is used, the bias (or the residual) of a fragment cannot be asked for before the
+// fragment before it has been stored, as the two might be the same memory, and its wait takes the store in too; so everything an epilogue reads is asked for
+// ahead of the stores: bias and scales of all columns at once, the residual a fragment row before it is added (two rows ahead measured the same, four spend
+// registers: 4112 x 1024 x 1024 21.1 and 22.1 us against 20.8).  With a bias, us, at its use -> ahead: residual 16384 x 1024 x 1024 48.3 -> 44.1, 16448 x 1024 x 4096
+// 181 -> 172, hi/lo 1025 x 768 x 768 9.5 -> 8.9; bf16 16384 x 3072 x 1024 110 -> 96, with GELU x 4096 162 -> 157.
+// bf16 results leave 16 bytes a lane where rows are of whole 16 bytes: two fragments' columns between lanes 16 apart (2048 x 3072 x 1024 21.8 -> 18.9); the 8-wave
+// kernel's gated units leave one fragment at a time (1409 x 4096 x 1024 of them 31.3 us, in pairs 32.4).
+template <int EPI, bool EXACT_GELU, bool F8, int MI, int NJ, class Row, class Col, class Val>
+__device__ __forceinline__ void g256_out_b(const G256& p, char* Cz, const bool biased, int row0, int Mg, int grp, Row row, Col col, Val val) {
+  constexpr bool paired = epi_paired(EPI), resid = EPI == E_F32_RESID || EPI == E_F32_RESID_GATE, gated = EPI == E_F32_RESID_GATE;
+  constexpr bool at_once = paired && !epi_split(EPI) && MI == 8, pairs = !epi_f32(EPI) && NJ % 2 == 0 && !at_once;
+  constexpr int AHEAD = resid && MI == 2 ? 2 : 1;
+  f32x4 b[NJ], b2[NJ], ws[NJ], ws2[NJ], res[AHEAD][NJ], gt[AHEAD][NJ];
+  float rs[MI], sa[MI];
+  const auto m_of = [&](int i) { return row0 + min(row(i), Mg - 1); };      // (rows and columns past the end are not stored, and read nothing past it)
+  const auto n_of = [&](int j) { return min(col(j), p.N - 4); };
+  const auto ahead = [&](int i) {
+    const int64_t m = m_of(i);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      if (resid) res[i % AHEAD][j] = *reinterpret_cast<const f32x4*>(Cz + (m * p.ldc + n_of(j)) * 4);
+      if (gated) gt[i % AHEAD][j] = *reinterpret_cast<const f32x4*>(p.gate + m * p.ldgate + n_of(j));
+    }
+  };
+  if (resid) {
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) ahead(i);
+  }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) b[j] = b2[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (biased) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      b[j] = bf16x4_f32(*reinterpret_cast<const u32x2*>(p.bias + n_of(j)));
+      if (paired) b2[j] = bf16x4_f32(*reinterpret_cast<const u32x2*>(p.bias + p.w_pair_rows + n_of(j)));
+    }
+  }
+  if constexpr (F8) {                                  // e4m3 operands: the row scales of both sides (before bias and epilogue)
+    const float* wsc = p.w_scale + (int64_t)grp * p.w_sstride;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      ws[j] = *reinterpret_cast<const f32x4*>(wsc + n_of(j));
+      if (paired) ws2[j] = *reinterpret_cast<const f32x4*>(wsc + p.w_pair_rows + n_of(j));
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) sa[i] = p.a_scale[p.a_rows ? p.a_rows[m_of(i)] : m_of(i)];      // (the operand row this output row was multiplied from)
+  }
+  if (EPI == E_SWIGLU_BF16_SCALED) {                   // the input row's factor, applied to its products
+#pragma unroll
+    for (int i = 0; i < MI; ++i) rs[i] = p.row_scale[m_of(i)];
+  }
+  const bool wide = pairs && ((p.N | p.ldc | (epi_split(EPI) ? p.c_lo_off : 0)) & 7) == 0 && ((uintptr_t)Cz & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int64_t m = row0 + row(i);
+    const bool m_ok = row(i) < Mg;
+    if (__builtin_amdgcn_ballot_w64(m_ok) == 0) continue;
+    f32x4 v[NJ];
+    u32x2 hi[NJ], lo[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      if (at_once) __builtin_amdgcn_sched_barrier(0);
+      f32x4 u = {0.f, 0.f, 0.f, 0.f};
+      val(i, j, v[j], u);
+      if constexpr (F8) {
+        v[j] *= ws[j] * sa[i];
+        if (paired) u *= ws2[j] * sa[i];
+      }
+      if (biased) {
+        asm volatile("");                              // (a branch, where it is not known: the activation is not to be moved across fragments)
+        v[j] += b[j];
+        if (paired) u += b2[j];
+      }
+      if (EPI == E_SWIGLU_BF16_SCALED) { v[j] *= rs[i]; u *= rs[i]; }
+      if (gated) v[j] = res[i % AHEAD][j] + gt[i % AHEAD][j] * v[j];
+      else if (resid) v[j] = res[i % AHEAD][j] + v[j];
+      if (!epi_f32(EPI)) g256_pack<EPI, EXACT_GELU>(v[j], u, hi[j], lo[j]);
+      if (at_once && m_ok && col(j) < p.N) *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(Cz) + m * p.ldc + col(j)) = hi[j];
+    }
+    if (resid && i + AHEAD < MI) ahead(i + AHEAD);
+    if constexpr (pairs) {
+      if (wide) {
+        const int odd = (threadIdx.x >> 4) & 1;
+#pragma unroll
+        for (int j = 0; j < NJ; j += 2) {
+          const u32x4 h = pair_lanes16(hi[j], hi[j + 1]);
+          u32x4 l;
+          if (epi_split(EPI)) l = pair_lanes16(lo[j], lo[j + 1]);
+          const int n = odd ? col(j + 1) - 4 : col(j);             // (N % 8 == 0: the 8 columns are all in or all out)
+          if (!m_ok || n >= p.N) continue;
+          bf16_t* c = reinterpret_cast<bf16_t*>(Cz) + m * p.ldc + n;
+          *reinterpret_cast<u32x4*>(c) = h;
+          if (epi_split(EPI)) *reinterpret_cast<u32x4*>(c + p.c_lo_off) = l;
+        }
+        continue;
+      }
+    }
+    if (at_once) continue;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int n = col(j);
+      if (!m_ok || n >= p.N) continue;                 // N % 4 == 0 (host check): the 4 columns are all in or all out
+      if (EPI == E_F32_TAIL_RELU2 && n >= p.tail0 && n < p.tail1) {  // a feed-forward's hidden units beside other projections of the same rows
+        f32x4 r = f32x4{fmaxf(v[j].x, 0.f), fmaxf(v[j].y, 0.f), fmaxf(v[j].z, 0.f), fmaxf(v[j].w, 0.f)};
+        r = r * r;
+        *reinterpret_cast<u32x2*>(p.C2 + m * p.ldc2 + (n - p.tail0)) = u32x2{cvt_pk_bf16(r.x, r.y), cvt_pk_bf16(r.z, r.w)};
+      } else if (epi_f32(EPI)) {
+        *reinterpret_cast<f32x4*>(Cz + (m * p.ldc + n) * 4) = v[j];
+      } else {
+        bf16_t* c = reinterpret_cast<bf16_t*>(Cz) + m * p.ldc + n;
+        *reinterpret_cast<u32x2*>(c) = hi[j];
+        if (epi_split(EPI)) *reinterpret_cast<u32x2*>(c + p.c_lo_off) = lo[j];
+      }
+    }
+  }
+}
+
+template <int EPI, bool EXACT_GELU, bool F8, int MI, int NJ, class Row, class Col, class Val>
+__device__ __forceinline__ void g256_out(const G256& p, char* Cz, int zslice, int row0, int Mg, int grp, Row row, Col col, Val val) {
+  const bool biased = p.bias && zslice == 0;
+  constexpr bool one = MI == 8 || epi_paired(EPI);     // one copy of the code (two spill accumulators of the 8-wave kernel)
+  if (one || !biased) g256_out_b<EPI, EXACT_GELU, F8, MI, NJ>(p, Cz, one && biased, row0, Mg, grp, row, col, val);
+  else g256_out_b<EPI, EXACT_GELU, F8, MI, NJ>(p, Cz, true, row0, Mg, grp, row, col, val);
+}
+
+// Epilogue of one output tile of the 8-wave kernel.
 template <int EPI, bool HILO, bool F8 = false>
 __device__ __forceinline__ void g256_epilogue(const G256& p, const f32x4 (&acc)[8][4], int wr, int wc, int fr, int fq, int m0,
                                               int n0, int row0, int Mg, int zslice, int grp = 0) {
   constexpr bool hilo = HILO, paired = epi_paired(EPI);
   char* Cz = reinterpret_cast<char*>(p.C);
   if (EPI == E_F32) Cz += (int64_t)zslice * p.c_zstride * 4;
-  constexpr int mi_n = hilo ? 4 : 8, nj_n = paired ? 2 : 4;
-#pragma unroll
-  for (int i = 0; i < mi_n; ++i) {
-    const int ml = hilo ? m0 + wr * 64 + i * 16 + fr : m0 + wr * 128 + i * 16 + fr;
-#pragma unroll
-    for (int j = 0; j < nj_n; ++j) {
-      const int n = paired ? n0 + wc * 32 + j * 16 + fq * 4 : n0 + wc * 64 + j * 16 + fq * 4;
-      if (ml >= Mg || n >= p.N) continue;           // N % 4 == 0 (host check): the 4 columns are all in or all out
-      f32x4 v = acc[i][j];
-      if (hilo) v += acc[(i + 4) & 7][j];
-      f32x4 u = {0.f, 0.f, 0.f, 0.f};
-      if (paired) { u = acc[i][(j + 2) & 3]; if (hilo) u += acc[(i + 4) & 7][(j + 2) & 3]; }
-      if constexpr (F8) {                              // e4m3 operands: the row scales of both sides (before bias and epilogue)
-        const float sa = p.a_scale[p.a_rows ? p.a_rows[row0 + ml] : row0 + ml];      // (the operand row this output row was multiplied from)
-        const float* wsc = p.w_scale + (int64_t)grp * p.w_sstride;
-        v *= *reinterpret_cast<const f32x4*>(wsc + n) * sa;
-        if (paired) u *= *reinterpret_cast<const f32x4*>(wsc + p.w_pair_rows + n) * sa;
-      }
-      g256_emit<EPI>(p, Cz, row0 + ml, n, v, u, zslice);
-    }
-  }
+  g256_out<EPI, false, F8, hilo ? 4 : 8, paired ? 2 : 4>(
+      p, Cz, zslice, row0, Mg, grp, [&](int i) { return m0 + wr * (hilo ? 64 : 128) + i * 16 + fr; },
+      [&](int j) { return n0 + wc * (paired ? 32 : 64) + j * 16 + fq * 4; },
+      [&](int i, int j, f32x4& v, f32x4& u) {
+        v = acc[i][j];
+        if (hilo) v += acc[(i + 4) & 7][j];
+        if (paired) { u = acc[i][(j + 2) & 3]; if (hilo) u += acc[(i + 4) & 7][(j + 2) & 3]; }
+      });
 }
 
 template <int EPI, bool HILO, bool F8 = false>

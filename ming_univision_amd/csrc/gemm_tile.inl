@@ -143,17 +143,11 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
     }
     return;
   }
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int m = m0 + wm * (BM / WM) + i * 16 + fr;
-#pragma unroll
-    for (int j = 0; j < (paired ? NJ / 2 : NJ); ++j) {
-      const int n = n0 + wn * (cols / WN) + j * 16 + fq * 4;
-      if (m >= p.M || n >= p.N) continue;              // N % 4 == 0 (host check): the 4 columns are all in or all out
-      f32x4 v = acc[i][j], u = {0.f, 0.f, 0.f, 0.f};
-      if (HILO) v += acc[(i + MI) % AI][j];
-      if (paired) { u = acc[i][(j + NJ / 2) % NJ]; if (HILO) u += acc[(i + MI) % AI][(j + NJ / 2) % NJ]; }
-      g256_emit<EPI, true>(p, Cz, m, n, v, u, blockIdx.y);
-    }
-  }
+  g256_out<EPI, true, false, MI, paired ? (NJ + 1) / 2 : NJ>(
+      p, Cz, blockIdx.y, 0, p.M, 0, [&](int i) { return m0 + wm * (BM / WM) + i * 16 + fr; }, [&](int j) { return n0 + wn * (cols / WN) + j * 16 + fq * 4; },
+      [&](int i, int j, f32x4& v, f32x4& u) {
+        v = acc[i][j];
+        if (HILO) v += acc[(i + MI) % AI][j];
+        if (paired) { u = acc[i][(j + NJ / 2) % NJ]; if (HILO) u += acc[(i + MI) % AI][(j + NJ / 2) % NJ]; }
+      });
 }

@@ -194,7 +194,8 @@ enum { MN_G256_F32 = 0, MN_G256_BF16 = 1, MN_G256_BF16_GELU = 2, MN_G256_F32_RES
        MN_G256_F32_RESID_GATE = 5, MN_G256_SWIGLU_BF16 = 6, MN_G256_BF16_RELU2 = 7,
        MN_G256_SWIGLU_BF16_SCALED = 8,
        MN_G256_F32_TAIL_RELU2 = 9,                     // fp32, but columns [tail0, tail1) go squared-relu'd to C2 as bf16 (column tail0 of the product = column 0 of C2)
-       MN_G256_GEGLU_BF16 = 10 };                       // gelu(gate) * up, tanh form, as bf16 (paired like SWIGLU_BF16)
+       MN_G256_GEGLU_BF16 = 10,                        // gelu(gate) * up, tanh form, as bf16 (paired like SWIGLU_BF16)
+       MN_G256_BF16_SPLIT = 11 };                      // the fp32 result as bf16 hi rows and lo rows (c_lo_off elements further); hi/lo rows only
 extern "C" int mn_gemm256_ex(const mn_g256* a, int epi, int ksplit, void* stream);
 extern "C" int mn_gemm256_slices(int K, int ksplit);
 extern "C" int mn_axpy_rms_rows_slabs(float* x, int64_t ldx, const float* y, int64_t ldy, int nz, int64_t zs, float mult, const uint16_t* w, float eps,

@@ -54,13 +54,18 @@ struct FlashP {
   const int32_t* seq_tab; int64_t kv_seq_stride;   // SRC 1: [n][tab_w] = (cache sequence, first q / out row, span length[, past]); NULL: (0, 0, T)
   int tab_w;                                       // 3, or 4 = every span brings its own `past`
   int mask_per_row;                                // (unused with key_mask == NULL)
+  int64_t lo_off;                                  // SRC 2: elements from a hi value of qkv to its lo value
 };
 
 template <int HD, int SRC, bool HILO, int QG, int KS>
-__global__ __launch_bounds__(256 * KS, QG == 1 && KS == 2 && HD == 64 ? 4 : 2) void flash_prefill_kernel(const FlashP p) {
+__global__ __launch_bounds__(256 * KS, KS == 4 || (QG == 1 && KS == 2 && HD == 64) ? 4 : 2) void flash_prefill_kernel(const FlashP p) {
   constexpr int QW = 16 * QG;
   constexpr int KROW = HD + 8, VROW = HD + 16, NKK = HD / 32, NDT = HD / 16;
-  constexpr int ESZ = (SRC == 0 && !HILO) ? 2 : 4, PPR = HD * ESZ / 16, KPP = 256 / PPR, NP = FKT / KPP;
+  static_assert(SRC != 2 || HILO, "hi and lo planes");
+  constexpr bool PACKED = SRC == 0 || SRC == 2, PLANES = SRC == 2;                       // qkv [B, T, 3, nh, 64]; as a bf16 hi and a bf16 lo plane
+  // log2 of a score's exponential: PLANES takes head dim 64's 0.125 here, the others in q (a power of two: the same bits)
+  constexpr float LOG2E = 1.4426950408889634f * (PLANES ? 0.125f : 1.0f);
+  constexpr int ESZ = (SRC == 0 && !HILO) || PLANES ? 2 : 4, PPR = HD * ESZ / 16, KPP = 256 / PPR, NP = FKT / KPP;
   constexpr int KLO = FKT * KROW, VLO = FKT * VROW, TILE = (KLO + VLO) * (HILO ? 2 : 1);
   constexpr int PART = QG * (NDT * 4 + 2) * 256;                                        // floats a key group hands over
   constexpr int SMEM = KS > 1 && (KS - 1) * PART * 2 > KS * TILE ? (KS - 1) * PART * 2 : KS * TILE;
@@ -78,11 +83,11 @@ __global__ __launch_bounds__(256 * KS, QG == 1 && KS == 2 && HD == 64 ? 4 : 2) v
   bf16_t* ob;
   const char *kb, *vb;
   const uint8_t* km = p.key_mask;
-  if (SRC == 0) {
+  if (PACKED) {
     const int head = blockIdx.x, b = blockIdx.z;
     q0 = qblk * 4 * QW + wave * QW;
     q_hi_wg = qblk * 4 * QW + 4 * QW - 1;
-    qb = p.q + (b * p.q_bs + head * p.q_hs) * (HILO ? 2 : 1);          // HILO: q is fp32 (pointer arithmetic in bf16 units)
+    qb = p.q + (b * p.q_bs + head * p.q_hs) * (ESZ / 2);               // (fp32 q: pointer arithmetic in bf16 units)
     o_off = b * p.o_bs + head * HD;
     ob = p.out + o_off;
     kb = reinterpret_cast<const char*>(p.k) + (b * p.kv_bs + head * p.kv_hs) * ESZ;
@@ -117,7 +122,15 @@ __global__ __launch_bounds__(256 * KS, QG == 1 && KS == 2 && HD == 64 ? 4 : 2) v
 #pragma unroll
   for (int qg = 0; qg < QG; ++qg) {
     q_idx[qg] = q0 + qg * 16 + i16;
-    if constexpr (HILO) {
+    if constexpr (PLANES) {
+      const bf16_t* qr = qb + (int64_t)min(q_idx[qg], T - 1) * p.q_rs + g * 8;
+#pragma unroll
+      for (int kk = 0; kk < NKK; ++kk) {
+        qf[qg][kk] = *reinterpret_cast<const bf16x8*>(qr + kk * 32);
+        qfl[qg][kk] = *reinterpret_cast<const bf16x8*>(qr + p.lo_off + kk * 32);
+      }
+      continue;
+    } else if constexpr (HILO) {
       const float* qr = reinterpret_cast<const float*>(qb) + (int64_t)min(q_idx[qg], T - 1) * p.q_rs + g * 8;
 #pragma unroll
       for (int kk = 0; kk < NKK; ++kk) {
@@ -155,7 +168,7 @@ __global__ __launch_bounds__(256 * KS, QG == 1 && KS == 2 && HD == 64 ? 4 : 2) v
 
   // staging: piece = 16 source bytes; a pass of the workgroup covers KPP whole key rows (coalesced)
   const int piece = tid % PPR, krow = tid / PPR;
-  u32x4 rk[NP], rv[NP];
+  u32x4 rk[PLANES ? 2 * NP : NP], rv[PLANES ? 2 * NP : NP];                              // PLANES: hi pieces, then lo
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int ps = 0; ps < NP; ++ps) {
@@ -163,13 +176,22 @@ __global__ __launch_bounds__(256 * KS, QG == 1 && KS == 2 && HD == 64 ? 4 : 2) v
       const int64_t off = (int64_t)kr * p.kv_rs * ESZ + piece * 16;
       rk[ps] = *reinterpret_cast<const u32x4*>(kb + off);
       rv[ps] = *reinterpret_cast<const u32x4*>(vb + off);
+      if constexpr (PLANES) {
+        rk[NP + ps] = *reinterpret_cast<const u32x4*>(kb + off + p.lo_off * 2);
+        rv[NP + ps] = *reinterpret_cast<const u32x4*>(vb + off + p.lo_off * 2);
+      }
     }
   };
   auto park = [&]() {
 #pragma unroll
     for (int ps = 0; ps < NP; ++ps) {
       const int key = ps * KPP + krow;
-      if constexpr (HILO) {
+      if constexpr (PLANES) {
+        *reinterpret_cast<u32x4*>(&ks[key * KROW + piece * 8]) = rk[ps];
+        *reinterpret_cast<u32x4*>(&ks[KLO + key * KROW + piece * 8]) = rk[NP + ps];
+        *reinterpret_cast<u32x4*>(&vs[key * VROW + piece * 8]) = rv[ps];
+        *reinterpret_cast<u32x4*>(&vs[VLO + key * VROW + piece * 8]) = rv[NP + ps];
+      } else if constexpr (HILO) {
         const f32x4 a = __builtin_bit_cast(f32x4, rk[ps]), b = __builtin_bit_cast(f32x4, rv[ps]);
         u32x2 h, l;
         { const HL t_ = spl(a.x, a.y); h.x = t_.h; l.x = t_.l; } { const HL t_ = spl(a.z, a.w); h.y = t_.h; l.y = t_.l; }
@@ -255,7 +277,6 @@ __global__ __launch_bounds__(256 * KS, QG == 1 && KS == 2 && HD == 64 ? 4 : 2) v
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float m_new = fmaxf(m_run[qg], mx);
       // exp(x - m) = 2^(x log2e - m log2e): one fma + v_exp_f32 per score; a row with no visible key yet keeps m = -inf, p = 0
-      constexpr float LOG2E = 1.4426950408889634f;
       const float mb = m_new == -INFINITY ? 0.f : m_new * LOG2E;
       float e[16], psum = 0.f;
 #pragma unroll
@@ -335,7 +356,6 @@ __global__ __launch_bounds__(256 * KS, QG == 1 && KS == 2 && HD == 64 ? 4 : 2) v
       const float* other = reinterpret_cast<const float*>(smem) + (w - 1) * PART + tid;
 #pragma unroll
       for (int qg = 0; qg < QG; ++qg) {
-        constexpr float LOG2E = 1.4426950408889634f;
         const float m2 = other[(qg * (NDT * 4 + 2)) * 256], l2 = other[(qg * (NDT * 4 + 2) + 1) * 256], m = fmaxf(m_run[qg], m2);
         const float a1 = m_run[qg] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_run[qg] - m) * LOG2E);
         const float a2 = m2 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m2 - m) * LOG2E);
@@ -385,11 +405,16 @@ __global__ __launch_bounds__(256 * KS, QG == 1 && KS == 2 && HD == 64 ? 4 : 2) v
 // -> 69), where 128 would leave an eighth and more of the queries empty (64 x 257 x 12: 47 -> 44) or some CUs a second workgroup (1 x 2500 x 16: 72 -> 62); else 128
 // (1 x 4000 x 16 hi/lo: 264 -> 210, 16 x 1025 x 12 221 -> 197, 64 x 65 x 16 28 -> 25).  Heads are the fastest grid dimension: an XCD then sees few heads' keys
 // (2500 x 16 hi/lo, 128 queries: 126 -> 100 us).
-template <bool HILO>
+// Hi/lo operands of 450 tokens and more whose 64-query workgroups are about one a CU or fewer walk in four key groups (16 waves):
+// a key group of half the tiles ends sooner, and the groups meet once (hi/lo planes, us, two -> four groups: 1 x 1025 x 16 causal 23.0 -> 20.8, x 12 24.5 -> 22.9,
+// 730 x 16 17.8 -> 16.5, 500 x 16 13.4 -> 13.0; 257 x 16 9.4 -> 9.9 and 2 x 1025 x 16 33.1 -> 35.3 stay with two).  Planes against fp32 rows that every workgroup
+// splits for itself: 1 x 1025 x 16 26.0 -> 23.0 in two groups, 257 x 12 11.9 -> 10.8, 8 x 257 x 16 22.8 -> 18.8: the split was a third of a tile's vector work.
+template <int SRC, bool HILO>
 void flash_hd64(const FlashP& p, int T, int n_heads, int B, hipStream_t st) {
   const int64_t cu = mn_num_cus(), hb = (int64_t)n_heads * B, w64 = mn_cdiv(T, 64) * hb, w128 = mn_cdiv(T, 128) * hb;
-#define MN_FL(QG_, KS_) hipLaunchKernelGGL((flash_prefill_kernel<64, 0, HILO, QG_, KS_>), dim3(n_heads, mn_cdiv(T, 64 * (QG_)), B), dim3(256 * (KS_)), 0, st, p)
-  if (T > 64 && w64 <= (p.causal ? 5 * cu / 2 : cu)) MN_FL(1, 2);
+#define MN_FL(QG_, KS_) hipLaunchKernelGGL((flash_prefill_kernel<64, SRC, HILO, QG_, KS_>), dim3(n_heads, mn_cdiv(T, 64 * (QG_)), B), dim3(256 * (KS_)), 0, st, p)
+  if (HILO && T >= 450 && w64 <= (p.causal ? 5 * cu / 4 : cu)) MN_FL(1, HILO ? 4 : 2);
+  else if (T > 64 && w64 <= (p.causal ? 5 * cu / 2 : cu)) MN_FL(1, 2);
   else if (T > 64 && w128 <= cu) MN_FL(2, 2);
   else if (p.causal || 2 * w128 <= 3 * cu || 100 * w128 >= 58 * w64) MN_FL(1, 1);
   else MN_FL(2, 1);
@@ -419,7 +444,7 @@ extern "C" int mn_attn_prefill_hd64(const uint16_t* qkv, uint16_t* out, int B, i
   p.q_rs = rs; p.q_hs = 64; p.kv_rs = rs; p.kv_hs = 64; p.o_rs = (int64_t)n_heads * 64;
   p.q_bs = (int64_t)T * rs; p.kv_bs = (int64_t)T * rs; p.o_bs = (int64_t)T * n_heads * 64;
   p.T = T; p.past = 0; p.causal = causal;
-  flash_hd64<false>(p, T, n_heads, B, mn_stream(stream));
+  flash_hd64<0, false>(p, T, n_heads, B, mn_stream(stream));
   MN_CHECK_LAUNCH("mn_attn_prefill_hd64");
   return MN_OK;
 }
@@ -435,8 +460,24 @@ extern "C" int mn_attn_prefill_hd64_f32(const float* qkv, float* out, uint16_t* 
   p.q_rs = rs; p.q_hs = 64; p.kv_rs = rs; p.kv_hs = 64; p.o_rs = (int64_t)n_heads * 64;
   p.q_bs = (int64_t)T * rs; p.kv_bs = (int64_t)T * rs; p.o_bs = (int64_t)T * n_heads * 64;
   p.T = T; p.past = 0; p.causal = causal;
-  flash_hd64<true>(p, T, n_heads, B, mn_stream(stream));
+  flash_hd64<0, true>(p, T, n_heads, B, mn_stream(stream));
   MN_CHECK_LAUNCH("mn_attn_prefill_hd64_f32");
+  return MN_OK;
+}
+
+// The same on qkv as a product writes it for this kernel (MN_G256_BF16_SPLIT): a bf16 hi plane [B, T, 3, nh, 64] and its lo plane lo_off elements further.  What the
+// fp32 form splits once for every 64 queries that meet a tile was split once.
+extern "C" int mn_attn_prefill_hd64_planes(const uint16_t* qkv, int64_t lo_off, uint16_t* split, int B, int T, int n_heads, int causal, void* stream) {
+  MN_CHECK_ARG(qkv && split && B >= 1 && T >= 1 && n_heads >= 1 && (lo_off % 8) == 0 && ((uintptr_t)qkv & 15) == 0, "mn_attn_prefill_hd64_planes: bad args");
+  FlashP p{};
+  const int64_t rs = (int64_t)3 * n_heads * 64;
+  p.q = qkv; p.k = qkv + (int64_t)n_heads * 64; p.v = qkv + (int64_t)2 * n_heads * 64; p.lo_off = lo_off;
+  p.out_split = split; p.split_lo_off = (int64_t)B * T * n_heads * 64;
+  p.q_rs = rs; p.q_hs = 64; p.kv_rs = rs; p.kv_hs = 64; p.o_rs = (int64_t)n_heads * 64;
+  p.q_bs = (int64_t)T * rs; p.kv_bs = (int64_t)T * rs; p.o_bs = (int64_t)T * n_heads * 64;
+  p.T = T; p.past = 0; p.causal = causal;
+  flash_hd64<2, true>(p, T, n_heads, B, mn_stream(stream));
+  MN_CHECK_LAUNCH("mn_attn_prefill_hd64_planes");
   return MN_OK;
 }
 

@@ -84,7 +84,7 @@ typedef mn_g256 G256;
 enum { E_F32 = MN_G256_F32, E_BF16 = MN_G256_BF16, E_BF16_GELU = MN_G256_BF16_GELU, E_F32_RESID = MN_G256_F32_RESID,
        E_SWIGLU_SPLIT = MN_G256_SWIGLU_SPLIT, E_F32_RESID_GATE = MN_G256_F32_RESID_GATE, E_SWIGLU_BF16 = MN_G256_SWIGLU_BF16,
        E_BF16_RELU2 = MN_G256_BF16_RELU2, E_SWIGLU_BF16_SCALED = MN_G256_SWIGLU_BF16_SCALED,
-       E_F32_TAIL_RELU2 = MN_G256_F32_TAIL_RELU2, E_GEGLU_BF16 = MN_G256_GEGLU_BF16 };
+       E_F32_TAIL_RELU2 = MN_G256_F32_TAIL_RELU2, E_GEGLU_BF16 = MN_G256_GEGLU_BF16, E_BF16_SPLIT = MN_G256_BF16_SPLIT };
 __host__ __device__ constexpr bool epi_paired(int epi) {
   return epi == E_SWIGLU_SPLIT || epi == E_SWIGLU_BF16 || epi == E_SWIGLU_BF16_SCALED || epi == E_GEGLU_BF16;
 }
@@ -138,7 +138,7 @@ __device__ __forceinline__ float gelu_erf_bf16out(float x) {
   return 0.5f * x * one_plus_erf;
 }
 
-__host__ __device__ constexpr bool epi_split(int epi) { return epi == E_SWIGLU_SPLIT; }
+__host__ __device__ constexpr bool epi_split(int epi) { return epi == E_SWIGLU_SPLIT || epi == E_BF16_SPLIT; }
 __host__ __device__ constexpr bool epi_f32(int epi) { return epi == E_F32 || epi == E_F32_RESID || epi == E_F32_RESID_GATE || epi == E_F32_TAIL_RELU2; }
 
 __device__ __forceinline__ f32x4 bf16x4_f32(u32x2 b) { return f32x4{bf16lo_to_f32(b.x), bf16hi_to_f32(b.x), bf16lo_to_f32(b.y), bf16hi_to_f32(b.y)}; }
@@ -178,7 +178,7 @@ __device__ __forceinline__ u32x4 pair_lanes16(u32x2 a, u32x2 b) {
 // ahead of the stores: bias and scales of all columns at once, the residual a fragment row before it is added (two rows ahead measured the same, four spend
 // registers: 4112 x 1024 x 1024 21.1 and 22.1 us against 20.8).  With a bias, us, at its use -> ahead: residual 16384 x 1024 x 1024 48.3 -> 44.1, 16448 x 1024 x 4096
 // 181 -> 172, hi/lo 1025 x 768 x 768 9.5 -> 8.9; bf16 16384 x 3072 x 1024 110 -> 96, with GELU x 4096 162 -> 157.
-// bf16 results leave 16 bytes a lane where rows are of whole 16 bytes: two fragments' columns between lanes 16 apart (2048 x 3072 x 1024 21.8 -> 18.9); the 8-wave
+// bf16 results leave 16 bytes a lane where rows are of whole 16 bytes: two fragments' columns between lanes 16 apart (hi/lo rows of 1025 x 3072: 23.7 -> 21.7 us; 2048 x 3072 x 1024 21.8 -> 18.9); the 8-wave
 // kernel's gated units leave one fragment at a time (1409 x 4096 x 1024 of them 31.3 us, in pairs 32.4).
 template <int EPI, bool EXACT_GELU, bool F8, int MI, int NJ, class Row, class Col, class Val>
 __device__ __forceinline__ void g256_out_b(const G256& p, char* Cz, const bool biased, int row0, int Mg, int grp, Row row, Col col, Val val) {
@@ -672,6 +672,10 @@ static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
       } else {
         if (!(form > 0 && tile_launch_plain<E_F32_TAIL_RELU2>(p, form, nz, st))) hipLaunchKernelGGL((gemm256_kernel<E_F32_TAIL_RELU2, false>), grid, dim3(512), 0, st, p);
       }
+      break;
+    case E_BF16_SPLIT:
+      if (!hilo || a.g_off || nz > 1) { mn_set_error("gemm256: epilogue %d takes one dense product of hi/lo rows", epi); return MN_EINVAL; }
+      if (!(form > 0 && tile_launch<E_BF16_SPLIT>(p, form, nz, true, st))) hipLaunchKernelGGL((gemm256_kernel<E_BF16_SPLIT, true>), grid, dim3(512), 0, st, p);
       break;
     case E_SWIGLU_BF16_SCALED:
       if (hilo || !a.row_scale) { mn_set_error("gemm256: the scaled SwiGLU epilogue takes plain rows and their factors"); return MN_EINVAL; }

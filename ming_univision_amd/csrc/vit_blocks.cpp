@@ -3,6 +3,8 @@
 // one call per launch from Python costs more than the launch runs: 60 blocks took 5.1 ms of host time over 3.1 ms of kernels.
 #include "common.h"
 
+extern "C" int mn_attn_prefill_hd64_planes(const uint16_t* qkv, int64_t lo_off, uint16_t* split, int B, int T, int n_heads, int causal, void* stream);
+
 namespace {
 
 size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -65,8 +67,17 @@ extern "C" int mn_vit_blocks(float* x, int B, int T, int dim, int depth, const u
     MN_CHECK_ARG((hidden % 64) == 0, "mn_vit_blocks: hidden=%d must be a multiple of 64 (pad with zeros)", hidden);
     for (int i = 0; i < depth; ++i, w += 12) {
       TRY(mn_norm_act_split(x, dim, 2, w[0], w[1], eps, 0, xs, dim, dlo, nullptr, 0, M, dim, stream));
-      TRY(mn_gemm256(xs, dim, dlo, w[2], dim, w[3], wide, 3 * (int64_t)dim, M, 3 * dim, dim, MN_GEMM_F32, stream));
-      TRY(mn_attn_prefill_hd64_f32(wide, nullptr, att, B, T, nh, causal, stream));
+      if (mn_gemm256_supported(dim, dlo, dim, 3 * (int64_t)dim, M, 3 * dim, dim) && ((uintptr_t)w[2] & 15) == 0 && ((uintptr_t)w[3] & 7) == 0) {
+        // q, k, v as a bf16 hi and a bf16 lo plane, where attention would split them for every 64 queries
+        mn_g256 qkv{};
+        qkv.A = xs; qkv.lda = dim; qkv.a_lo_off = dlo; qkv.W = w[2]; qkv.ldw = dim; qkv.bias = w[3]; qkv.C = wide; qkv.ldc = 3 * (int64_t)dim;
+        qkv.c_lo_off = 3 * dlo; qkv.M = M; qkv.N = 3 * dim; qkv.K = dim;
+        TRY(mn_gemm256_ex(&qkv, MN_G256_BF16_SPLIT, 1, stream));
+        TRY(mn_attn_prefill_hd64_planes(reinterpret_cast<const uint16_t*>(wide), 3 * dlo, att, B, T, nh, causal, stream));
+      } else {                                 // (refused with the product's reasons)
+        TRY(mn_gemm256(xs, dim, dlo, w[2], dim, w[3], wide, 3 * (int64_t)dim, M, 3 * dim, dim, MN_GEMM_F32, stream));
+        TRY(mn_attn_prefill_hd64_f32(wide, nullptr, att, B, T, nh, causal, stream));
+      }
       TRY(mn_gemm256(att, dim, dlo, w[4], dim, w[5], x, dim, M, dim, dim, MN_GEMM_F32_RESID, stream));
       TRY(mn_norm_act_split(x, dim, 2, w[6], w[7], eps, 0, xs, dim, dlo, nullptr, 0, M, dim, stream));
       if (gelu) {

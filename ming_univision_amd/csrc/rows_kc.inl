@@ -193,10 +193,12 @@ __global__ __launch_bounds__(512) void rows_kc_kernel(const mn_skinny_args a, in
 // The same with rows and weights on their way through LDS: a wave instruction fetches whole 64- or 128-byte pieces of a row (64 bytes a cycle and CU), where
 // operands read straight from memory, 16 rows apart lane by lane, come at a quarter of that (38 GB/s a CU: 7 of 12 us for 32 rows of 2048).  Each wave has a ring of
 // its own, so nothing but the sum at the end is a barrier.  What is left is the split (130 vector instructions for 32 values of 32 rows, 4 us of the
-// 2048).  Rows of 16-byte aligned values; 2048 x 2048 at 32 rows 14.5 -> 11.1 us.
-template <int MT, int NT, int PRO>
+// 2048).  Rows of 16-byte aligned values; 2048 x 2048 at 32 rows 14.5 -> 11.1 us.  NX eights of rows are fetched, as many as there are: with sixteen of them always, 5 rows of
+// 32000 x 1024 took 23.4 us beside other work, with eight 16.5.
+template <int NX, int NT, int PRO>
 __global__ __launch_bounds__(512) void rows_kc_lds_kernel(const mn_skinny_args a, int paired) {
-  constexpr int NW = 8, CK = 64, R = MT * NT * 4, S = 3, XB = MT * 2048, SUB = XB + NT * 1024;      // a ring holds S pieces of 32 values of K: rows of 128 bytes, then weights of 64
+  constexpr int MT = (NX + 1) / 2;                     // NX: eights of rows that are fetched
+  constexpr int NW = 8, CK = 64, R = MT * NT * 4, S = 3, XB = NX * 1024, SUB = XB + NT * 1024;      // a ring holds S pieces of 32 values of K: rows of 128 bytes, then weights of 64
   constexpr int BYTES = NW * S * SUB > NW * R * 256 ? NW * S * SUB : NW * R * 256;
   __shared__ __attribute__((aligned(1024))) char lds[BYTES];
   float (*red)[R][64] = reinterpret_cast<float (*)[R][64]>(lds);
@@ -207,10 +209,10 @@ __global__ __launch_bounds__(512) void rows_kc_lds_kernel(const mn_skinny_args a
   typedef const __attribute__((address_space(1))) void gptr;
   typedef __attribute__((address_space(3))) void lptr;
   const int xr = lane >> 3, wr = lane >> 2;
-  const float* xp[2 * MT];
-  int xk[2 * MT];
+  const float* xp[NX];
+  int xk[NX];
 #pragma unroll
-  for (int i = 0; i < 2 * MT; ++i) {
+  for (int i = 0; i < NX; ++i) {
     const int row = 8 * i + xr;
     xk[i] = 4 * ((lane & 7) ^ ((row >> 1) & 7));
     xp[i] = a.x + (int64_t)min(row, M - 1) * a.ldx;
@@ -234,7 +236,7 @@ __global__ __launch_bounds__(512) void rows_kc_lds_kernel(const mn_skinny_args a
 #pragma unroll
     for (int t = 0; t < NT; ++t) __builtin_amdgcn_global_load_lds((gptr*)(wp[t] + (k0 + wk < K ? k0 + wk : 0)), (lptr*)(dst + XB + t * 1024), 16, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 2 * MT; ++i) __builtin_amdgcn_global_load_lds((gptr*)(xp[i] + (k0 + xk[i] < K ? k0 + xk[i] : 0)), (lptr*)(dst + i * 1024), 16, 0, 0);
+    for (int i = 0; i < NX; ++i) __builtin_amdgcn_global_load_lds((gptr*)(xp[i] + (k0 + xk[i] < K ? k0 + xk[i] : 0)), (lptr*)(dst + i * 1024), 16, 0, 0);
   };
 #pragma unroll
   for (int c = 0; c < S; ++c)
@@ -251,8 +253,8 @@ __global__ __launch_bounds__(512) void rows_kc_lds_kernel(const mn_skinny_args a
     for (int s = 0; s < 2; ++s) {
       const int k = k0 + 32 * s + 8 * q, left = pieces - 1 - c0 - s;
       const bool in = k < K;
-      if (left >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (2 * MT + NT)) : "memory");
-      else if (left == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * MT + NT) : "memory");
+      if (left >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (NX + NT)) : "memory");
+      else if (left == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NX + NT) : "memory");
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       f32x4 cx[MT][2];
       u32x4 cw[NT];
@@ -260,7 +262,7 @@ __global__ __launch_bounds__(512) void rows_kc_lds_kernel(const mn_skinny_args a
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) cx[i][h] = *reinterpret_cast<const f32x4*>(src + (16 * i + r) * 128 + (((2 * q + h) ^ ((r >> 1) & 7)) << 4));
+        for (int h = 0; h < 2; ++h) cx[i][h] = *reinterpret_cast<const f32x4*>(src + (2 * i + 1 < NX ? 16 * i + r : 16 * i + (r & 7)) * 128 + (((2 * q + h) ^ ((r >> 1) & (2 * i + 1 < NX ? 7 : 3))) << 4));
 #pragma unroll
       for (int t = 0; t < NT; ++t) cw[t] = *reinterpret_cast<const u32x4*>(src + XB + t * 1024 + r * 64 + ((q ^ ((r >> 2) & 3)) << 4));
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

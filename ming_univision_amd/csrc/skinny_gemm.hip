@@ -361,12 +361,17 @@ static bool rows_kc(const mn_skinny_args& a, bool fma, hipStream_t st) {
   const double there = !fma ? 8.8 + 0.08 * a.M + 0.2 * mb : (a.M > 4 && a.M < 8 ? 2 * once + (a.M - 2) * row : once + (a.M - 1) * row) / 1.15;
   if (fma && (a.M == 2 || (a.M == 3 && nt == 2 && !paired && a.K <= 1024))) return false;
   if (g > (fma ? 4 : 1) * mn_num_cus() || here >= there) return false;
-  // through LDS from 5 rows on, where the rows' loads are the launch (us straight from memory / through LDS: 2048 x 2048 at 4 rows 6.9 / 7.0, 8 rows 7.3 / 7.1, 16
-  // rows 8.8 / 7.6, 32 rows 14.5 / 11.1; 8192 x 2048 at 2 rows 10.7 / 11.9, 8 rows 11.9 / 12.2, 32 rows 20.0 / 17.2); a norm's gain or a second row would be a load
-  // that waits for the pieces in flight behind it
-  const bool lds = a.M > 4 && (a.prologue == MN_PRO_NONE || a.prologue == MN_PRO_SILU) && ((uintptr_t)a.x & 15) == 0 && (a.ldx % 4) == 0;
+  // through LDS from 5 rows on, where the rows' loads are the launch (us straight from memory / through LDS: 2048 x 2048 at 4 rows 6.9 / 7.0, 8 rows 7.3 / 7.0, 16
+  // rows 8.8 / 7.6, 32 rows 14.5 / 11.1; 1024 x 1024 at 5 rows 4.6 / 4.3, 24 rows 7.5 / 6.4; 32000 x 1024 at 5 rows 19.1 / 19.1), from 7 with two tiles a workgroup
+  // and more than 1024 values, whose weights are more (8192 x 2048 at 2 rows 10.7 / 11.9, 6 rows 11.3 / 11.9, 8 rows 12.0 / 11.9, 32 rows 19.6 / 16.3); a norm's gain
+  // or a second row would be a load that waits for the pieces in flight behind it
+  const bool lds = a.M > (nt == 2 && a.K > 1024 ? 6 : 4) && (a.prologue == MN_PRO_NONE || a.prologue == MN_PRO_SILU) && ((uintptr_t)a.x & 15) == 0 && (a.ldx % 4) == 0;
 #define MN_KC(MT_, NT_, P_) hipLaunchKernelGGL((rows_kc_kernel<MT_, NT_, P_>), dim3((unsigned)g), dim3(512), 0, st, a, paired ? 1 : 0)
-#define MN_KCL(MT_, NT_, P_) hipLaunchKernelGGL((rows_kc_lds_kernel<MT_, NT_, P_>), dim3((unsigned)g), dim3(512), 0, st, a, paired ? 1 : 0)
+#define MN_KCL(MT_, NT_, P_)                                                                                                                          \
+  do {                                                                                                                                               \
+    if (a.M <= 16 * (MT_) - 8) hipLaunchKernelGGL((rows_kc_lds_kernel<2 * (MT_) - 1, NT_, P_>), dim3((unsigned)g), dim3(512), 0, st, a, paired ? 1 : 0); \
+    else hipLaunchKernelGGL((rows_kc_lds_kernel<2 * (MT_), NT_, P_>), dim3((unsigned)g), dim3(512), 0, st, a, paired ? 1 : 0);                          \
+  } while (0)
 #define MN_KC_P(MT_, NT_)                                              \
   do {                                                                 \
     switch (lds ? 16 + a.prologue : a.prologue) {                      \

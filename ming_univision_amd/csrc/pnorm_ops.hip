@@ -393,17 +393,26 @@ __global__ __launch_bounds__(256) void delta_rows_kernel(DeltaArgs a) {
   }
 }
 
+typedef float f4 __attribute__((ext_vector_type(4)));
+// own + the value `other` of the lane CTRL names
+template <int CTRL>
+__device__ __forceinline__ float dpp_add_to(float own, float other) {
+  return own + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(other), CTRL, 0xf, 0xf, true));
+}
+
 // The same walk for heads of at most 256 state rows, without a branch in the step: grid (H * ceil(vdim / CPB), S):
 // workgroup y takes the step's sequences y, y + S, .., from a table of their first rows that it makes once (TABLE: at most 2048 rows).  LPC lanes share a value column
 // (CPB = 256 / LPC columns a workgroup); a lane holds the state rows 4 (s + LPC jj) + t, t < 4, jj < NS / 4, so that q and k come from
 // LDS in 16-byte reads; LDS rows are padded with zeros to DP = NS * LPC values, under which the padded state rows stay zero.
-// A serial chain: what bounds it is the instructions of a step.  Four steps are unrolled with the operands in alternating registers (no moves), the sums are
-// DPP additions, outputs stay in a lane until LPC of them are written at once.  1409 rows in 5 sequences (the longest 470), 8 heads of 128 + 128: 101 us
-// (195 with a workgroup per row and 830 cycles a step); 512 sequences of two rows 374 (431; 493 with every sequence looked for from the step's first row).
-template <int NS, int LPC, int DBT, bool TABLE>
+// A serial chain on one wave a SIMD: what bounds it is the instructions of a step and of a batch.  Four steps are unrolled with the operands in alternating registers (no
+// moves); the output is the updated state's product with q, a partial sum a lane whose exchange waits for four rows of them (11 instructions for four rows, 32 one by
+// one); VEC (heads of exactly DP values in 16-byte rows) brings q and k 16 bytes a load with no branch.  1409 rows in 5 sequences (the longest 470), 8 heads of
+// 128 + 128: 74 us (98 with loads of 4 bytes and sums row by row, 83 with the wide loads alone); one sequence of 2048 rows 288 (397); 300 rows, 2 heads of 256 + 128 78
+// (110); 256 sequences of two rows 152 (181).  Operands read two rows ahead took 87 for 83, four rows solved at once (their products with each other made beforehand) 105.
+template <int NS, int LPC, int DBT, bool TABLE, bool VEC>
 __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
   constexpr int CPB = 256 / LPC, DP = NS * LPC, NQ = DBT * 2 * DP / 256, NV = (DBT * CPB + 255) / 256;
-  extern __shared__ float lds[];             // [DBT][2 DP] q, k; [DBT][CPB] v; [DBT] beta, decay, k . q; [DBT][CPB] outputs
+  extern __shared__ float lds[];             // [DBT][2 DP] q, k; [DBT][CPB] v; [DBT] beta, decay; [DBT][CPB] outputs
   const int ncb = (a.vdim + CPB - 1) / CPB, h = blockIdx.x / ncb, cb = blockIdx.x - h * ncb;
   const int tid = threadIdx.x, s = tid % LPC, cl = tid / LPC, c = cb * CPB + cl;
   const int d = a.dim, kvh = h / (a.H / a.G);
@@ -438,11 +447,18 @@ __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
     float* qk = lds;                           // row r: q at r * 2 DP, k at r * 2 DP + DP
     float* vs = qk + DBT * 2 * DP;
     float* bs = vs + DBT * CPB;
-    float* os = bs + 3 * DBT;                   // [DBT][CPB] the batch's outputs
-    float rq[NQ], rv[NV], rb = 0.f;
+    float* os = bs + 2 * DBT;                   // [DBT][CPB] the batch's outputs
+    float rq[VEC ? 1 : NQ], rv[NV], rb = 0.f;
+    constexpr int NX = VEC ? NQ / 4 : 1, PER = DP / 2, RT = 256 / PER;            // 16-byte loads a thread, of them a row, rows the workgroup loads at once
+    f4 rx[NX];
+    const float* xp = a.qkv + (int64_t)m0 * a.ld + (tid % PER < PER / 2 ? 0 : (a.G - 1) * d) + (int64_t)kvh * d + 4 * (tid % PER);
     // element e of a batch's q / k block: row e / (2 DP), value e % (2 DP) (q below DP, k from DP on)
     auto fetch = [&](int b0) {
-      const int rows = min(DBT, n - b0);
+      [[maybe_unused]] const int rows = min(DBT, n - b0);
+      if constexpr (VEC) {                     // (rows past the end are the last one again, until they become zeros on their way to LDS)
+#pragma unroll
+        for (int t = 0; t < NX; ++t) rx[t] = *reinterpret_cast<const f4*>(xp + (int64_t)min(b0 + tid / PER + RT * t, n - 1) * a.ld);
+      } else
 #pragma unroll
       for (int t = 0; t < NQ; ++t) {
         const int e = tid + 256 * t, r = e / (2 * DP), i = e % (2 * DP), ii = i % DP;
@@ -451,7 +467,8 @@ __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
 #pragma unroll
       for (int t = 0; t < NV; ++t) {
         const int e = tid + 256 * t, r = e / CPB, cc = cb * CPB + e % CPB;
-        rv[t] = (r < rows && cc < a.vdim) ? a.qkv[(int64_t)(m0 + b0 + r) * a.ld + 2 * a.G * d + (int64_t)h * a.vdim + cc] : 0.f;
+        if constexpr (VEC) rv[t] = a.qkv[(int64_t)(m0 + min(b0 + r, n - 1)) * a.ld + 2 * a.G * d + (int64_t)h * a.vdim + min(cc, a.vdim - 1)];
+        else rv[t] = (r < rows && cc < a.vdim) ? a.qkv[(int64_t)(m0 + b0 + r) * a.ld + 2 * a.G * d + (int64_t)h * a.vdim + cc] : 0.f;
       }
       if (tid < 2 * DBT) {
         const int r = tid % DBT;
@@ -462,25 +479,27 @@ __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
     for (int b0 = 0; b0 < n; b0 += DBT) {
       const int rows = min(DBT, n - b0);
       lds_barrier();                           // the previous batch's steps have read their rows
+      if constexpr (VEC) {
+        if (rows < DBT) {
 #pragma unroll
-      for (int t = 0; t < NQ; ++t) qk[tid + 256 * t] = rq[t];
+          for (int t = 0; t < NX; ++t) if (tid / PER + RT * t >= rows) rx[t] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int t = 0; t < NV; ++t) if ((tid + 256 * t) / CPB >= rows) rv[t] = 0.f;
+        }
+#pragma unroll
+        for (int t = 0; t < NX; ++t) *reinterpret_cast<f4*>(qk + 4 * (tid + 256 * t)) = rx[t];
+      } else {
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) qk[tid + 256 * t] = rq[t];
+      }
 #pragma unroll
       for (int t = 0; t < NV; ++t) { const int e = tid + 256 * t; if (e < DBT * CPB) vs[e] = rv[t]; }
       if (tid < 2 * DBT) bs[tid] = rb;
       lds_barrier();
       if (b0 + DBT < n) fetch(b0 + DBT);         // in flight while this batch is computed
-      for (int r = tid >> 4; r < DBT; r += 16) {   // k . q of every row: 16 threads a row
-        const int l = tid & 15;
-        float t = 0.f;
-#pragma unroll
-        for (int i = l; i < DP; i += 16) t = fmaf(qk[r * 2 * DP + i], qk[r * 2 * DP + DP + i], t);
-        t = row16_sum(t);
-        if (l == 0) bs[2 * DBT + r] = t;
-      }
-      lds_barrier();                           // orders LDS only: the next batch's loads stay in flight
       // the operands of step r + 1 are read from LDS before step r is computed: they do not depend on the state.  (The read behind the last row stays
       // inside the LDS block; rows up to the next multiple of 4 are zeros with decay 1.)
-      float kk[2][NS], qq[2][NS], v[2], beta[2], g[2], kq[2];
+      float kk[2][NS], qq[2][NS], v[2], beta[2], g[2];
       auto load_row = [&](int r, int b) {
         const float* q = qk + r * 2 * DP + 4 * s;
 #pragma unroll
@@ -489,31 +508,35 @@ __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
           kk[b][4 * jj] = k4.x; kk[b][4 * jj + 1] = k4.y; kk[b][4 * jj + 2] = k4.z; kk[b][4 * jj + 3] = k4.w;
           qq[b][4 * jj] = q4.x; qq[b][4 * jj + 1] = q4.y; qq[b][4 * jj + 2] = q4.z; qq[b][4 * jj + 3] = q4.w;
         }
-        v[b] = vs[r * CPB + cl]; beta[b] = bs[r]; g[b] = bs[DBT + r]; kq[b] = bs[2 * DBT + r];
+        v[b] = vs[r * CPB + cl]; beta[b] = bs[r]; g[b] = bs[DBT + r];
       };
       load_row(0, 0);
-      for (int rb = 0; rb < rows; rb += LPC) {
-        float keep = 0.f;                      // lane s: the output of row rb + s
-        for (int r0 = rb; r0 < min(rows, rb + LPC); r0 += 4) {
+      for (int r0 = 0; r0 < rows; r0 += 4) {
+        float o[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int b = j & 1;
-            load_row(r0 + j + 1, b ^ 1);
-            float pk = 0.f, pq = 0.f, pk2 = 0.f, pq2 = 0.f;
+        for (int j = 0; j < 4; ++j) {
+          const int b = j & 1;
+          load_row(r0 + j + 1, b ^ 1);
+          float pk = 0.f, pk2 = 0.f, pq = 0.f, pq2 = 0.f;
 #pragma unroll
-            for (int i = 0; i < NS; i += 2) {
-              pk = fmaf(S[i], kk[b][i], pk); pk2 = fmaf(S[i + 1], kk[b][i + 1], pk2);
-              pq = fmaf(S[i], qq[b][i], pq); pq2 = fmaf(S[i + 1], qq[b][i + 1], pq2);
-            }
-            pk += pk2; pq += pq2;
-            if (LPC == 16) { pk = row16_sum(pk); pq = row16_sum(pq); } else { pk = sum8(pk); pq = sum8(pq); }
-            const float u = beta[b] * (v[b] - g[b] * pk);
+          for (int i = 0; i < NS; i += 2) { pk = fmaf(S[i], kk[b][i], pk); pk2 = fmaf(S[i + 1], kk[b][i + 1], pk2); }
+          pk += pk2;
+          if (LPC == 16) pk = row16_sum(pk); else pk = sum8(pk);
+          const float u = beta[b] * (v[b] - g[b] * pk);
 #pragma unroll
-            for (int i = 0; i < NS; ++i) S[i] = fmaf(g[b], S[i], kk[b][i] * u);
-            keep = s == r0 + j - rb ? fmaf(g[b], pq, u * kq[b]) : keep;
-          }
+          for (int i = 0; i < NS; ++i) S[i] = fmaf(g[b], S[i], kk[b][i] * u);
+#pragma unroll
+          for (int i = 0; i < NS; i += 2) { pq = fmaf(S[i], qq[b][i], pq); pq2 = fmaf(S[i + 1], qq[b][i + 1], pq2); }
+          o[j] = pq + pq2;
         }
-        os[(rb + s) * CPB + cl] = keep;
+        // four rows' outputs at once: lanes that hold the sums of one row each after two exchanges (with the lane mirrored in 16, then in 8; of 8 lanes: in 8, then in 4)
+        const bool hi1 = LPC == 16 ? (s & 8) != 0 : (s & 4) != 0, hi2 = LPC == 16 ? (s & 4) != 0 : (s & 2) != 0;
+        constexpr int M1 = LPC == 16 ? 0x140 : 0x141, M2 = LPC == 16 ? 0x141 : 0x1B;
+        const float x = dpp_add_to<M1>(hi1 ? o[1] : o[0], hi1 ? o[0] : o[1]), y = dpp_add_to<M1>(hi1 ? o[3] : o[2], hi1 ? o[2] : o[3]);
+        float z = dpp_add_to<M2>(hi2 ? y : x, hi2 ? x : y);
+        if (LPC == 16) z = dpp_add<0x4E>(z);
+        z = dpp_add<0xB1>(z);
+        os[(r0 + (hi1 ? 1 : 0) + (hi2 ? 2 : 0)) * CPB + cl] = z;
       }
       lds_barrier();
 #pragma unroll
@@ -714,10 +737,15 @@ extern "C" int mn_gated_delta_rows(const float* qkv, int64_t ld, const float* bd
     // sequences walked side by side: four workgroups a CU, the rest one after the other (64 sequences of two rows, 8 heads of 128 x 128 53 us with four, 51 with two, 61
     // with three; 4 heads of 64 x 64 10.4, 12.1, 11.6; 1024 sequences of one row, 2 heads of 16 x 16 10.8, 13.5, 11.2)
     auto slots = [&](int64_t gx) { const int64_t y = 4 * (int64_t)mn_num_cus() / gx; return (unsigned)(y < 1 ? 1 : (y < M ? y : M)); };
-#define MN_DFT(NS_, LPC_, DB_, T_)                                                                                                                 \
-  hipLaunchKernelGGL((delta_rows_fast_kernel<NS_, LPC_, DB_, T_>), dim3((unsigned)(H * mn_cdiv(vdim, 256 / LPC_)), slots(H * mn_cdiv(vdim, 256 / LPC_))), dim3(256),  \
-                     ((size_t)DB_ * 2 * NS_ * LPC_ + 2 * DB_ * (256 / LPC_) + 3 * DB_) * sizeof(float), st, a)
-#define MN_DF(NS_, LPC_, DB_) do { if (M <= 2048) MN_DFT(NS_, LPC_, DB_, true); else MN_DFT(NS_, LPC_, DB_, false); } while (0)
+#define MN_DFT(NS_, LPC_, DB_, T_, V_)                                                                                                             \
+  hipLaunchKernelGGL((delta_rows_fast_kernel<NS_, LPC_, DB_, T_, V_>), dim3((unsigned)(H * mn_cdiv(vdim, 256 / LPC_)), slots(H * mn_cdiv(vdim, 256 / LPC_))), dim3(256),  \
+                     ((size_t)DB_ * 2 * NS_ * LPC_ + 2 * DB_ * (256 / LPC_) + 2 * DB_) * sizeof(float), st, a)
+#define MN_DF(NS_, LPC_, DB_)                                                                                            \
+  do {                                                                                                                   \
+    const bool vec = dim == NS_ * LPC_ && (ld % 4) == 0 && ((uintptr_t)qkv & 15) == 0;      /* 16-byte loads of whole heads */ \
+    if (M <= 2048) { if (vec) MN_DFT(NS_, LPC_, DB_, true, true); else MN_DFT(NS_, LPC_, DB_, true, false); }            \
+    else { if (vec) MN_DFT(NS_, LPC_, DB_, false, true); else MN_DFT(NS_, LPC_, DB_, false, false); }                    \
+  } while (0)
     if (dim <= 32) MN_DF(4, 8, 32); else if (dim <= 64) MN_DF(4, 16, 32); else if (dim <= 128) MN_DF(8, 16, 32); else MN_DF(16, 16, 16);
 #undef MN_DF
 #undef MN_DFT

@@ -10,6 +10,11 @@
 extern "C" int mn_rms_rows_pair(const float* xa, const uint16_t* wa, float* ya, int64_t ldya, uint16_t* ya16, int64_t ldya16, int na, const float* xb, const uint16_t* wb,
                                 float* yb, const int32_t* row_seq, const int32_t* row_slot, int t_max, int nb, int64_t ldx, float eps, int M, void* stream);
 
+extern "C" int mn_gated_norm_filter_rows_split(float* x, int64_t ldx, const float* g, int64_t ldg, const float* y, int64_t ldy, const uint16_t* wa, const uint16_t* ba,
+                                               const uint16_t* wb, const uint16_t* bb, float eps, float* n_out, int64_t ldn, const uint16_t* taps_w, int taps, float* state,
+                                               const int32_t* row_seq, const int32_t* row_slot, float* h, int64_t ldh, uint16_t* y16, int M, int n, void* stream);
+extern "C" int mn_polynorm_rows_split(const float* z, int64_t ldz, const uint16_t* coef, float eps, uint16_t* y16, int M, int n, void* stream);
+
 extern "C" size_t mn_sizeof_seq_layer(void) { return sizeof(mn_seq_layer); }
 extern "C" size_t mn_sizeof_seq_model(void) { return sizeof(mn_seq_model); }
 extern "C" size_t mn_sizeof_seq_state(void) { return sizeof(mn_seq_state); }
@@ -135,12 +140,13 @@ extern "C" int mn_seq_step(const mn_seq_model* m, const mn_seq_state* st, const 
   // operators run one by one.  `pend` is a sublayer end that has not been applied to x yet.
   const bool fuse = (flags & MN_SEQ_ROWS_DISTINCT) && !want16 && W <= 4096 && m->taps <= 8 && !trace;
   struct Pending { const float* g = nullptr; int64_t ldg = 0; const uint16_t *w = nullptr, *b = nullptr; } pend;
-  // n_out = LN(x; wb, bb) after applying `pend`; with tstate / h_out also h = n + filter(n) and the state update
+  // n_out = LN(x; wb, bb) after applying `pend`; with tstate / h_out also h = n + filter(n) and the state update.  last_split (`fuse` only): the last of the two as the
+  // hi/lo rows of the product behind it
   auto norm_stage = [&](const uint16_t* wb, const uint16_t* bb, float* n_out, uint16_t* n16, const uint16_t* taps_w, float* tstate,
-                        float* h_out, uint16_t* h16) -> int {
+                        float* h_out, uint16_t* h16, uint16_t* last_split) -> int {
     if (fuse) {
-      const int rc2 = mn_gated_norm_filter_rows(xr, W, pend.g, pend.ldg, yf, W, pend.w, pend.b, wb, bb, m->eps, n_out, W, taps_w, m->taps, tstate,
-                                                row_seq, row_slot, h_out, W, M, W, stream);
+      const int rc2 = mn_gated_norm_filter_rows_split(xr, W, pend.g, pend.ldg, yf, W, pend.w, pend.b, wb, bb, m->eps, n_out, W, taps_w, m->taps, tstate,
+                                                row_seq, row_slot, h_out, W, last_split, M, W, stream);
       pend = Pending();
       return rc2;
     }
@@ -160,9 +166,12 @@ extern "C" int mn_seq_step(const mn_seq_model* m, const mn_seq_state* st, const 
     float* arena = st->latent[l.arena];
     float* tstate = st->taps ? st->taps + (size_t)li * taps_layer : nullptr;
     // ---- mixer sublayer ----
-    MN_TRY(norm_stage(l.norm1_w, l.norm1_b, n1, n1h, l.taps_w, tstate, hf, hh));
+    mn_skinny_args pa;
+    uint16_t* split = fuse ? linear_operand(arith, M, hf, W, l.w_in, d.n_in, W, nullptr, pin, d.n_in, gws, gwb, &pa) : nullptr;
+    MN_TRY(norm_stage(l.norm1_w, l.norm1_b, n1, n1h, l.taps_w, tstate, hf, hh, split));
+    if (split) MN_TRY(mn_skinny_gemm_presplit(&pa, stream));
+    else MN_TRY(linear(arith, M, hf, W, hh, W, l.w_in, d.n_in, W, nullptr, pin, d.n_in, gws, gwb, stream));
     MN_TRY(linear(arith, M, n1, W, n1h, W, l.rg1_w, W, W, l.rg1_b, g1, W, gws, gwb, stream));
-    MN_TRY(linear(arith, M, hf, W, hh, W, l.w_in, d.n_in, W, nullptr, pin, d.n_in, gws, gwb, stream));
     const float* qp; int64_t ldq; const float* gp = nullptr; int kv_off;
     if (l.kind == MN_SEQ_MIX_LATENT_Q) {
       if (l.writes_arena)
@@ -194,10 +203,18 @@ extern "C" int mn_seq_step(const mn_seq_model* m, const mn_seq_state* st, const 
     // ---- feed-forward sublayer ----
     if (l.ff > 0) {
       const int nf = W + l.ff;
-      MN_TRY(norm_stage(l.norm2_w, l.norm2_b, n1, n1h, nullptr, nullptr, nullptr, nullptr));
-      MN_TRY(linear(arith, M, n1, W, n1h, W, l.w_ff_in, nf, W, l.b_ff_in, fin, nf, gws, gwb, stream));
-      MN_TRY(mn_polynorm_rows(fin + W, nf, l.act, m->eps, af, l.ff, afh, l.ff, M, l.ff, stream));
-      MN_TRY(linear(arith, M, af, l.ff, afh, l.ff, l.w_down, W, l.ff, nullptr, yf, W, gws, gwb, stream));
+      split = fuse ? linear_operand(arith, M, n1, W, l.w_ff_in, nf, W, l.b_ff_in, fin, nf, gws, gwb, &pa) : nullptr;
+      MN_TRY(norm_stage(l.norm2_w, l.norm2_b, n1, n1h, nullptr, nullptr, nullptr, nullptr, split));
+      if (split) MN_TRY(mn_skinny_gemm_presplit(&pa, stream));
+      else MN_TRY(linear(arith, M, n1, W, n1h, W, l.w_ff_in, nf, W, l.b_ff_in, fin, nf, gws, gwb, stream));
+      split = l.ff >= 512 && l.ff <= 8192 ? linear_operand(arith, M, af, l.ff, l.w_down, W, l.ff, nullptr, yf, W, gws, gwb, &pa) : nullptr;
+      if (split) {
+        MN_TRY(mn_polynorm_rows_split(fin + W, nf, l.act, m->eps, split, M, l.ff, stream));
+        MN_TRY(mn_skinny_gemm_presplit(&pa, stream));
+      } else {
+        MN_TRY(mn_polynorm_rows(fin + W, nf, l.act, m->eps, af, l.ff, afh, l.ff, M, l.ff, stream));
+        MN_TRY(linear(arith, M, af, l.ff, afh, l.ff, l.w_down, W, l.ff, nullptr, yf, W, gws, gwb, stream));
+      }
       pend.g = fin; pend.ldg = nf; pend.w = l.norm2b_w; pend.b = l.norm2b_b;
     }
     if (trace) {                                       // the trace wants x after the whole layer: apply the layer's last sublayer end now
@@ -207,7 +224,7 @@ extern "C" int mn_seq_step(const mn_seq_model* m, const mn_seq_state* st, const 
       if (e != hipSuccess) { mn_set_error("mn_seq_step: trace copy: %s", hipGetErrorString(e)); return MN_ELAUNCH; }
     }
   }
-  MN_TRY(norm_stage(m->final_w, m->final_b, out, nullptr, nullptr, nullptr, nullptr, nullptr));
+  MN_TRY(norm_stage(m->final_w, m->final_b, out, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr));
 #undef MN_TRY
   return MN_OK;
 }

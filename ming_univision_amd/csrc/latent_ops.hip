@@ -170,6 +170,7 @@ struct RowArgs {
   float* out; int64_t ldo;
   bf16_t* out16; int64_t ldo16;
   int n;
+  int64_t lo16;                          // polynorm: out16 as hi rows, lo rows lo16 values further (0: plain bf16)
 };
 
 template <int VPT, int MODE>
@@ -208,7 +209,11 @@ __global__ __launch_bounds__(256) void row_block_kernel(RowArgs a) {
       if (c >= n) continue;
       const float v2 = v[i] * v[i], o = ca * v[i] + cb * v2 + cc * (v2 * v[i]) + ce;
       if (a.out) a.out[(int64_t)row * a.ldo + c] = o;
-      if (a.out16) a.out16[(int64_t)row * a.ldo16 + c] = f32_to_bf16(o);
+      if (a.out16) {
+        const bf16_t hi = f32_to_bf16(o);
+        a.out16[(int64_t)row * a.ldo16 + c] = hi;
+        if (a.lo16) a.out16[a.lo16 + (int64_t)row * a.ldo16 + c] = f32_to_bf16(o - bf16_to_f32(hi));
+      }
     }
     return;
   }
@@ -487,7 +492,13 @@ struct FusedRowArgs {
   float* state; const int32_t* row_seq; const int32_t* row_slot;
   float* h; int64_t ldh;
   int n;
+  bf16_t* y16; int64_t y_lo;             // optional: the last of the outputs (h, or n_out without a filter) as dense bf16 hi rows, lo rows y_lo values further
 };
+__device__ __forceinline__ void store_hilo(bf16_t* y, int64_t lo, float v) {
+  const bf16_t hi = f32_to_bf16(v);
+  y[0] = hi;
+  y[lo] = f32_to_bf16(v - bf16_to_f32(hi));
+}
 
 constexpr int FUSED_MAX_TAPS = 8;
 
@@ -549,6 +560,7 @@ __global__ __launch_bounds__(256) void row_fused_kernel(FusedRowArgs a) {
     if (c >= n) continue;
     const float nv = (xv[i] - mean) * rstd * bf16_to_f32(a.wb[c]) + bf16_to_f32(a.bb[c]);
     a.n_out[(int64_t)row * a.ldn + c] = nv;
+    if (!FILTER && a.y16) store_hilo(a.y16 + (int64_t)row * n + c, a.y_lo, nv);
     if (FILTER) {
       const bf16_t* tw = a.taps_w + (int64_t)c * a.taps;
       float acc = nv + bf16_to_f32(tw[a.taps - 1]) * nv;
@@ -556,6 +568,7 @@ __global__ __launch_bounds__(256) void row_fused_kernel(FusedRowArgs a) {
       for (int k = 1; k < FUSED_MAX_TAPS; ++k)
         if (k < a.taps && slot - k >= 0) acc += bf16_to_f32(tw[a.taps - 1 - k]) * sv[i][k - 1];
       a.h[(int64_t)row * a.ldh + c] = acc;
+      if (a.y16) store_hilo(a.y16 + (int64_t)row * n + c, a.y_lo, acc);
       float* st = st0 + c;
 #pragma unroll
       for (int k = FUSED_MAX_TAPS - 2; k >= 1; --k)
@@ -610,7 +623,15 @@ __global__ __launch_bounds__(1024) void row_fused_vec_kernel(FusedRowArgs a) {
   }
   const f32x4 nv = norm(x, wb, bb);
   if (!on) return;
+  auto split = [&](const f32x4& v) {
+    ushort4 hi = {f32_to_bf16(v.x), f32_to_bf16(v.y), f32_to_bf16(v.z), f32_to_bf16(v.w)};
+    const f32x4 r = v - wide(hi);
+    bf16_t* y = a.y16 + (int64_t)row * n + c;
+    *reinterpret_cast<ushort4*>(y) = hi;
+    *reinterpret_cast<ushort4*>(y + a.y_lo) = ushort4{f32_to_bf16(r.x), f32_to_bf16(r.y), f32_to_bf16(r.z), f32_to_bf16(r.w)};
+  };
   *reinterpret_cast<f32x4*>(a.n_out + (int64_t)row * a.ldn + c) = nv;
+  if (TAPS == 0 && a.y16) split(nv);
   if (TAPS > 0) {
     float t[4 * TW];
 #pragma unroll
@@ -624,6 +645,7 @@ __global__ __launch_bounds__(1024) void row_fused_vec_kernel(FusedRowArgs a) {
         if (slot - k >= 0) h[j] += t[j * TW + TW - 1 - k] * sv[k - 1][j];
     }
     *reinterpret_cast<f32x4*>(a.h + (int64_t)row * a.ldh + c) = h;
+    if (a.y16) split(h);
 #pragma unroll
     for (int k = TAPS - 2; k >= 1; --k) *reinterpret_cast<f32x4*>(st0 + (int64_t)k * n) = sv[k - 1];
     if (TAPS > 1) *reinterpret_cast<f32x4*>(st0) = nv;
@@ -635,7 +657,7 @@ bool row_fused_vec_ok(const FusedRowArgs& a) {
   auto f = [](const float* p, int64_t ld) { return !p || (((uintptr_t)p & 15) == 0 && (ld % 4) == 0); };
   auto h = [](const bf16_t* p) { return ((uintptr_t)p & 7) == 0; };
   return (a.n % 4) == 0 && f(a.x, a.ldx) && f(a.g, a.ldg) && f(a.y, a.ldy) && f(a.n_out, a.ldn) && f(a.h, a.ldh) && f(a.state, 0) && h(a.wa) && h(a.ba) && h(a.wb) &&
-         h(a.bb) && h(a.taps_w);
+         h(a.bb) && h(a.taps_w) && h(a.y16) && (a.y_lo % 4) == 0;
 }
 
 // C[z][m, n] = alpha * A[z][m, :] . W[z][n, :] (+ bias) (* sigmoid(G)) for at most MM rows: one wave per output column, lanes over K
@@ -835,7 +857,7 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(const float* __restri
 extern "C" int mn_affine_ln_rows(const float* x, int64_t ldx, const uint16_t* w, const uint16_t* b, float eps, float* y, int64_t ldy,
                                  uint16_t* y16, int64_t ldy16, int M, int n, void* stream) {
   MN_CHECK_ARG(x && w && b && (y || y16) && M >= 1 && n >= 1, "mn_affine_ln_rows: bad args");
-  const RowArgs ra{x, ldx, nullptr, 0, nullptr, 0, w, b, eps, y, ldy, y16, ldy16, n};
+  const RowArgs ra{x, ldx, nullptr, 0, nullptr, 0, w, b, eps, y, ldy, y16, ldy16, n, 0};
   if (!launch_row_block<ROW_LN>(ra, M, mn_stream(stream)))
     hipLaunchKernelGGL(affine_ln_kernel, dim3((unsigned)mn_cdiv(M, 4)), dim3(256), 0, mn_stream(stream), x, ldx, w, b, eps, y, ldy, y16, ldy16,
                        M, n);
@@ -846,7 +868,7 @@ extern "C" int mn_affine_ln_rows(const float* x, int64_t ldx, const uint16_t* w,
 extern "C" int mn_gated_ln_residual(float* x, int64_t ldx, const float* g, int64_t ldg, const float* y, int64_t ldy, const uint16_t* w,
                                     const uint16_t* b, float eps, int M, int n, void* stream) {
   MN_CHECK_ARG(x && g && y && w && b && M >= 1 && n >= 1, "mn_gated_ln_residual: bad args");
-  const RowArgs ra{nullptr, 0, g, ldg, y, ldy, w, b, eps, x, ldx, nullptr, 0, n};
+  const RowArgs ra{nullptr, 0, g, ldg, y, ldy, w, b, eps, x, ldx, nullptr, 0, n, 0};
   if (!launch_row_block<ROW_GATED_LN_RESIDUAL>(ra, M, mn_stream(stream)))
     hipLaunchKernelGGL(gated_ln_residual_kernel, dim3((unsigned)mn_cdiv(M, 4)), dim3(256), 0, mn_stream(stream), x, ldx, g, ldg, y, ldy, w, b,
                        eps, M, n);
@@ -886,10 +908,19 @@ extern "C" int mn_rms_rows_pair(const float* xa, const uint16_t* wa, float* ya, 
 extern "C" int mn_polynorm_rows(const float* z, int64_t ldz, const uint16_t* coef, float eps, float* y, int64_t ldy, uint16_t* y16,
                                 int64_t ldy16, int M, int n, void* stream) {
   MN_CHECK_ARG(z && coef && (y || y16) && M >= 1 && n >= 1, "mn_polynorm_rows: bad args");
-  const RowArgs ra{z, ldz, nullptr, 0, nullptr, 0, coef, nullptr, eps, y, ldy, y16, ldy16, n};
+  const RowArgs ra{z, ldz, nullptr, 0, nullptr, 0, coef, nullptr, eps, y, ldy, y16, ldy16, n, 0};
   if (!launch_row_block<ROW_POLYNORM>(ra, M, mn_stream(stream)))
     hipLaunchKernelGGL(polynorm_kernel, dim3((unsigned)M), dim3(256), 0, mn_stream(stream), z, ldz, coef, eps, y, ldy, y16, ldy16, n);
   MN_CHECK_LAUNCH("mn_polynorm_rows");
+  return MN_OK;
+}
+
+// The same with its rows as bf16 hi rows, then lo rows (y16 [2, M, n] dense): the operand of a product on such rows; rows of 512 .. 8192 values
+extern "C" int mn_polynorm_rows_split(const float* z, int64_t ldz, const uint16_t* coef, float eps, uint16_t* y16, int M, int n, void* stream) {
+  MN_CHECK_ARG(z && coef && y16 && M >= 1 && n >= 512 && n <= 8192, "mn_polynorm_rows_split: bad args");
+  const RowArgs ra{z, ldz, nullptr, 0, nullptr, 0, coef, nullptr, eps, nullptr, 0, y16, n, n, (int64_t)M * n};
+  launch_row_block<ROW_POLYNORM>(ra, M, mn_stream(stream));
+  MN_CHECK_LAUNCH("mn_polynorm_rows_split");
   return MN_OK;
 }
 
@@ -926,15 +957,16 @@ extern "C" int mn_tap_state_update(const float* x, int64_t ldx, int taps, float*
   return MN_OK;
 }
 
-extern "C" int mn_gated_norm_filter_rows(float* x, int64_t ldx, const float* g, int64_t ldg, const float* y, int64_t ldy, const uint16_t* wa,
+// y16 (optional): mn_gated_norm_filter_rows with its last output also as bf16 hi rows, then lo rows ([2, M, n] dense)
+extern "C" int mn_gated_norm_filter_rows_split(float* x, int64_t ldx, const float* g, int64_t ldg, const float* y, int64_t ldy, const uint16_t* wa,
                                          const uint16_t* ba, const uint16_t* wb, const uint16_t* bb, float eps, float* n_out, int64_t ldn,
                                          const uint16_t* taps_w, int taps, float* state, const int32_t* row_seq, const int32_t* row_slot,
-                                         float* h, int64_t ldh, int M, int n, void* stream) {
+                                         float* h, int64_t ldh, uint16_t* y16, int M, int n, void* stream) {
   MN_CHECK_ARG(x && wb && bb && n_out && M >= 1 && n >= 1 && n <= 4096, "mn_gated_norm_filter_rows: bad args (rows of at most 4096 values)");
   MN_CHECK_ARG(!g || (y && wa && ba), "mn_gated_norm_filter_rows: the gated stage needs y and its norm");
   MN_CHECK_ARG(!h || (taps_w && taps >= 1 && taps <= FUSED_MAX_TAPS && (state || taps == 1) && row_seq && row_slot),
                "mn_gated_norm_filter_rows: the filter stage needs its state and at most %d taps", FUSED_MAX_TAPS);
-  const FusedRowArgs a{x, ldx, g, ldg, y, ldy, wa, ba, wb, bb, eps, n_out, ldn, taps_w, taps, state, row_seq, row_slot, h, ldh, n};
+  const FusedRowArgs a{x, ldx, g, ldg, y, ldy, wa, ba, wb, bb, eps, n_out, ldn, taps_w, taps, state, row_seq, row_slot, h, ldh, n, y16, (int64_t)M * n};
   const int vpt = (n + 255) / 256;
   hipStream_t st = mn_stream(stream);
   if (row_fused_vec_ok(a)) {
@@ -954,6 +986,13 @@ extern "C" int mn_gated_norm_filter_rows(float* x, int64_t ldx, const float* g, 
 #undef MN_RF
   MN_CHECK_LAUNCH("mn_gated_norm_filter_rows");
   return MN_OK;
+}
+
+extern "C" int mn_gated_norm_filter_rows(float* x, int64_t ldx, const float* g, int64_t ldg, const float* y, int64_t ldy, const uint16_t* wa,
+                                         const uint16_t* ba, const uint16_t* wb, const uint16_t* bb, float eps, float* n_out, int64_t ldn,
+                                         const uint16_t* taps_w, int taps, float* state, const int32_t* row_seq, const int32_t* row_slot,
+                                         float* h, int64_t ldh, int M, int n, void* stream) {
+  return mn_gated_norm_filter_rows_split(x, ldx, g, ldg, y, ldy, wa, ba, wb, bb, eps, n_out, ldn, taps_w, taps, state, row_seq, row_slot, h, ldh, nullptr, M, n, stream);
 }
 
 extern "C" int mn_softcap_rows(float* z, int64_t ld, int M, int n, float cap, void* stream) {

@@ -8,6 +8,9 @@
 
 #include "common.h"
 
+extern "C" uint16_t* mn_skinny_operand(const mn_skinny_args* a);
+extern "C" int mn_skinny_gemm_presplit(const mn_skinny_args* a, void* stream);
+
 namespace {
 
 inline size_t al(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -32,6 +35,17 @@ inline int linear(int arith, int M, const float* A, int64_t lda, const uint16_t*
   if (arith == MN_SEQ_ARITH_BF16 && A16 && mfma_ok(W, K) && (lda16 % 8) == 0 && (((uintptr_t)A16) & 15) == 0)
     return mn_gemm_bf16(A16, lda16, W, K, bias, C, ldc, M, N, K, MN_GEMM_F32, stream);
   return mn_gemm_f32_batched(A, lda, 0, W, K, 0, bias, C, ldc, 0, nullptr, 0, 0, nullptr, 0, 0, M, N, K, 1, 1.0f, stream);
+}
+
+// Where the kernel that makes the rows A of linear()'s call may leave them as bf16 hi rows and lo rows ([2, M, K], at the start of gws) for linear_presplit to take up: a
+// step's launch less (32 rows of 2048: 5.2 us).  NULL: linear() takes another route.  Nothing else may use gws in between.
+inline uint16_t* linear_operand(int arith, int M, const float* A, int64_t lda, const uint16_t* W, int N, int K, const uint16_t* bias, float* C, int64_t ldc, void* gws,
+                                size_t gws_bytes, mn_skinny_args* a) {
+  if (arith != MN_SEQ_ARITH_BF16 || M <= 8 || M > 64 || !mfma_ok(W, K)) return nullptr;
+  memset(a, 0, sizeof(*a));
+  a->x = A; a->ldx = lda; a->w = W; a->ldw = K; a->bias = bias; a->out = C; a->ldo = ldc;
+  a->M = M; a->N = N; a->K = K; a->ws = gws; a->ws_bytes = gws_bytes;
+  return mn_skinny_operand(a);
 }
 
 // act fp32 [M, N] = gelu_tanh(A Wg^T) * (A Wu^T) with W = [Wg ; Wu] (2N rows) as the EPILOGUE of the weight-streaming product, for steps

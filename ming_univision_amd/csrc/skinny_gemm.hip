@@ -344,7 +344,8 @@ extern "C" size_t mn_skinny_workspace_bytes_w8(int M, int N, int K, int epilogue
 // longer by as much and more (decode steps of 2 rows, four layers of width 1024: 208 / 189, 302 / 280, 191 / 184 us, of 3 rows of such products 211 / 198; of width
 // 2048 alike).  Not where the output overlaps what is read (the other forms read a row
 // before they write it) and not behind a LayerNorm (its mean has to be known before the split).
-static bool rows_kc(const mn_skinny_args& a, bool fma, hipStream_t st) {
+// (ask: the answer alone, nothing is launched)
+static bool rows_kc(const mn_skinny_args& a, bool fma, hipStream_t st, bool ask = false) {
   const bool paired = mn_epi_pairs(a.epilogue);
   auto apart = [&](const float* p, int64_t ld) {
     return p + (int64_t)(a.M - 1) * ld + a.K <= a.out || a.out + (int64_t)(a.M - 1) * a.ldo + a.N <= p;
@@ -361,6 +362,7 @@ static bool rows_kc(const mn_skinny_args& a, bool fma, hipStream_t st) {
   const double there = !fma ? 8.8 + 0.08 * a.M + 0.2 * mb : (a.M > 4 && a.M < 8 ? 2 * once + (a.M - 2) * row : once + (a.M - 1) * row) / 1.15;
   if (fma && (a.M == 2 || (a.M == 3 && nt == 2 && !paired && a.K <= 1024))) return false;
   if (g > (fma ? 4 : 1) * mn_num_cus() || here >= there) return false;
+  if (ask) return true;
   // through LDS from 5 rows on, where the rows' loads are the launch (us straight from memory / through LDS: 2048 x 2048 at 4 rows 6.9 / 7.0, 8 rows 7.3 / 7.0, 16
   // rows 8.8 / 7.6, 32 rows 14.5 / 11.1; 1024 x 1024 at 5 rows 4.6 / 4.3, 24 rows 7.5 / 6.4; 32000 x 1024 at 5 rows 19.1 / 19.1), from 7 with two tiles a workgroup
   // and more than 1024 values, whose weights are more (8192 x 2048 at 2 rows 10.7 / 11.9, 6 rows 11.3 / 11.9, 8 rows 12.0 / 11.9, 32 rows 19.6 / 16.3); a norm's gain
@@ -391,7 +393,8 @@ static bool rows_kc(const mn_skinny_args& a, bool fma, hipStream_t st) {
   return true;
 }
 
-static int skinny_medium(const mn_skinny_args& a, void* stream) {
+// presplit: the rows lie in the workspace already, as the prologue would leave them
+static int skinny_medium(const mn_skinny_args& a, void* stream, bool presplit = false) {
   MN_CHECK_ARG(a.M <= 64, "mn_skinny_gemm: M=%d out of range [1,64]", a.M);
   MN_CHECK_ARG((a.batch <= 1) && (a.nseg <= 1), "mn_skinny_gemm: batch/nseg forms need M <= 8");
   MN_CHECK_ARG(a.ldw == a.K, "mn_skinny_gemm: M > 8 needs densely packed weights (ldw == K)");
@@ -404,17 +407,32 @@ static int skinny_medium(const mn_skinny_args& a, void* stream) {
   bf16_t* Y = reinterpret_cast<bf16_t*>(a.ws);
   float* P = reinterpret_cast<float*>(reinterpret_cast<char*>(a.ws) + (((size_t)2 * a.M * a.K * sizeof(bf16_t) + 255) & ~(size_t)255));
   hipStream_t st = mn_stream(stream);
-  if (!w8 && rows_kc(a, false, st)) {
+  if (!presplit && !w8 && rows_kc(a, false, st)) {
     MN_CHECK_LAUNCH("mn_skinny_gemm(rows)");
     return MN_OK;
   }
-  hipLaunchKernelGGL(medium_prologue_kernel, dim3(a.M), dim3(1024), 0, st, a, Y);
+  if (!presplit) hipLaunchKernelGGL(medium_prologue_kernel, dim3(a.M), dim3(1024), 0, st, a, Y);
   const int nz = w8 ? mn_stream_mfma_wq(Y, reinterpret_cast<const uint8_t*>(a.w), a.wscale, P, a.M, Ntot, a.K, a.wfmt, stream)
                     : mn_stream_mfma(Y, a.w, P, a.M, Ntot, a.K, stream);
   if (nz < 0) return nz;
   hipLaunchKernelGGL(medium_epilogue_kernel, dim3((unsigned)mn_cdiv((int64_t)a.M * a.N, 256)), dim3(256), 0, st, a, P, nz, Ntot);
   MN_CHECK_LAUNCH("mn_skinny_gemm(medium)");
   return MN_OK;
+}
+
+// A plain product of 9 .. 64 dense bf16-weight rows that mn_skinny_gemm would take in three launches: where its first one leaves the rows ([2, M, K] bf16, hi rows
+// then lo rows, the start of the workspace), so that the kernel that makes the rows can; NULL: another route, or a call that is refused.
+extern "C" uint16_t* mn_skinny_operand(const mn_skinny_args* a) {
+  if (a->M <= 8 || a->M > 64 || a->N < 1 || a->K < 8 || (a->K % 8) || a->ldw != a->K || !a->x || !a->w || !a->out || a->prologue != MN_PRO_NONE || a->epilogue < 0 ||
+      a->epilogue > MN_EPI_GEGLU_TANH || a->wfmt != MN_W_BF16 || a->batch > 1 || a->nseg > 1 || !a->ws ||
+      a->ws_bytes < mn_skinny_workspace_bytes(a->M, a->N, a->K, a->epilogue) || rows_kc(*a, false, nullptr, true))
+    return nullptr;
+  return reinterpret_cast<uint16_t*>(a->ws);
+}
+// the same product from rows that lie there
+extern "C" int mn_skinny_gemm_presplit(const mn_skinny_args* a, void* stream) {
+  MN_CHECK_ARG(a && mn_skinny_operand(a), "mn_skinny_gemm_presplit: not a product of three launches");
+  return skinny_medium(*a, stream, true);
 }
 
 // Tuning overrides for micro-benchmarks (0 = heuristic). Not part of the stable ABI.

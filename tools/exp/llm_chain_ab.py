@@ -42,5 +42,5 @@ for rows in (2, 3, 4):
           f"chain with router + gate/up in ONE launch {min(t for t, _ in res[32]):.3f} ms ({', '.join('%.3f' % t for t, _ in res[32])}); "
           f"fp32-FMA sequence {min(t for t, _ in res[1]):.3f} ms ({', '.join('%.3f' % t for t, _ in res[1])}); "
           f"fp32-FMA sequence with the one-launch router + gate/up {min(t for t, _ in res[2]):.3f} ms ({', '.join('%.3f' % t for t, _ in res[2])}); hidden states differ by {d:.1e}", flush=True)
-L.mn_llm_tune_chain(32)
+L.mn_llm_tune_chain(64)
 L.mn_moe_tune_gate_up(1, 1 | (2 << 8))

@@ -35,4 +35,4 @@ for rows in (2, 3, 4):
     a, b = res[32 | (1 << 17)], res[32]
     print(f"{weights} {rows} rows: glue launch + QKV {min(t for t, _ in a):.3f} ms ({', '.join('%.3f' % t for t, _ in a)});  QKV with the RMSNorm prologue "
           f"{min(t for t, _ in b):.3f} ms ({', '.join('%.3f' % t for t, _ in b)});  same bits {torch.equal(a[0][1], b[0][1])} (max diff {((a[0][1] - b[0][1]).abs().max() / a[0][1].abs().max()).item():.1e}), finite {bool(torch.isfinite(b[0][1]).all())}", flush=True)
-L.mn_llm_tune_chain(32)
+L.mn_llm_tune_chain(64)

@@ -40,3 +40,23 @@ def test_sampler(rows, images):
     for i in range(images):
         one = head.sample(hid[i * per:(i + 1) * per].contiguous(), noise[i:i + 1].contiguous(), text_cfg=3.0, image_cfg=1.1, n_images=1)
         assert float((whole[i] - one[0]).norm() / one.norm()) < 1e-4
+
+
+@pytest.mark.parametrize("w, hidden, steps", [(384, 128, 4), (64, 1024, 1), (128, 256, 2)])
+@pytest.mark.parametrize("images", [3, 8, 11, 16])
+def test_condition(images, w, hidden, steps):
+    """The products before the blocks as one launch on fp32 rows, whose scratch is the modulations' memory, and on hi/lo rows where heads of one block and one step leave it
+    too small: two rows an image against each image alone."""
+    from ming_univision_amd import configuration as C
+    from ming_univision_amd.rf_head import RectifiedFlowHead
+    from ming_univision_amd.synth import synth_state_dict
+    shapes = {"vis_head.0.weight": (w, hidden), "vis_head.0.bias": (w,), "vis_head.1.weight": (w,), "vis_head.1.bias": (w,)}
+    shapes.update(C.rf_param_shapes(w, 1, w))
+    sd = {k: v.to("cuda", torch.bfloat16) for k, v in synth_state_dict(shapes, 5).items()}
+    head = RectifiedFlowHead(sd, hidden, dict(diffloss_w=w, diffloss_d=1, num_sampling_steps=str(steps), gen_method="flow_matching_swiglu-4", vis_head_arch="linear2-norm"))
+    g = torch.Generator(device="cuda").manual_seed(images)
+    hid, noise = torch.randn(2 * images, hidden, generator=g, device="cuda"), torch.randn(images, 32, generator=g, device="cuda")
+    whole = head.sample(hid, noise, text_cfg=3.0, image_cfg=1.1, n_images=images)
+    for i in range(images):
+        one = head.sample(hid[2 * i:2 * i + 2].contiguous(), noise[i:i + 1].contiguous(), text_cfg=3.0, image_cfg=1.1, n_images=1)
+        assert float((whole[i] - one[0]).norm() / one.norm()) < 1e-4

@@ -174,15 +174,15 @@ static int rf_sample_wide(const mn_rf_head* h, const float* hidden, int64_t ld_h
   const int W = h->w, HID = h->hidden, T = h->target, A = h->depth * 3 * W + 2 * W, rpi = rows / n_images;
   const int64_t SR = (int64_t)h->steps * rows;
 
-  // z = vis_head Linear(hidden);  c = cond_embed(LayerNorm(z)).  Every block's modulation comes from them, so up to 32 rows, where one launch does it, z keeps the fp32
-  // rows' every bit (and c up to 8), which hi/lo rows cut to 17: errors of the latents against 64 bits at 16 rows 2.3e-5 with hi/lo rows, 1.9e-5 without.
-  // (the modulations' memory is not written before both are done; heads of so few blocks that it is too small take hi/lo rows)
+  // z = vis_head Linear(hidden);  c = cond_embed(LayerNorm(z)).  Every block's modulation comes from them.  Up to 32 rows z is mn_skinny_gemm's, whose one-launch form
+  // keeps the fp32 rows' every bit where it is the faster one (2048 -> 3072: always), which hi/lo rows cut to 17: errors of the latents against 64 bits at 30 rows
+  // 9.8e-6 with hi/lo rows, 8.0e-6 without.  Its scratch is the modulations' memory, which is written behind it; heads of so few blocks that it is too small take
+  // hi/lo rows.  c, behind the LayerNorm, is a product of hi/lo rows on either route.
   const size_t ada_bytes = (size_t)SR * A * sizeof(float);
-  const bool z_rows = rows <= 32 && mn_skinny_workspace_bytes(rows, h->z_dim, h->llm_hidden, MN_EPI_NONE) <= ada_bytes, c_rows = z_rows && rows <= 8;
-  t_sk_ws = reinterpret_cast<char*>(w.ada); t_sk_ws_bytes = ada_bytes;
   WideGlue g;
   mn_g256 a;
-  if (z_rows) {
+  if (rows <= 32 && mn_skinny_workspace_bytes(rows, h->z_dim, h->llm_hidden, MN_EPI_NONE) <= ada_bytes) {
+    t_sk_ws = reinterpret_cast<char*>(w.ada); t_sk_ws_bytes = ada_bytes;
     mn_skinny_args k = sk(hidden, ld_hidden, h->vis_w, h->llm_hidden, h->vis_b, w.z, h->z_dim, rows, h->z_dim, h->llm_hidden);
     MN_TRYZ(mn_skinny_gemm(&k, stream));
   } else {
@@ -194,18 +194,12 @@ static int rf_sample_wide(const mn_rf_head* h, const float* hidden, int64_t ld_h
                           h->z_dim, h->llm_hidden);
     MN_TRYZ(mn_gemm256_ex(&a, MN_G256_F32, 1, stream));
   }
-  if (c_rows) {
-    mn_skinny_args k = sk(w.z, h->z_dim, h->cond_w, h->z_dim, h->cond_b, w.c, W, rows, W, h->z_dim);
-    k.prologue = MN_PRO_LN; k.ln_g = h->vis_ln_g; k.ln_b = h->vis_ln_b; k.eps = 1e-6f;
-    MN_TRYZ(mn_skinny_gemm(&k, stream));
-  } else {
-    memset(&g, 0, sizeof(g));
-    g.h = w.z; g.ldh = h->z_dim; g.norm = 2; g.ng = h->vis_ln_g; g.nb = h->vis_ln_b; g.eps = 1e-6f;
-    g.Y = w.zs; g.ldy = h->z_dim; g.y_lo_off = (int64_t)rows * h->z_dim; g.M = rows; g.D = h->z_dim;
-    wide_glue(g, st);
-    a = g256_hilo(w.zs, h->z_dim, lo_at(LO_RF_COND, (int64_t)rows * h->z_dim), h->cond_w, h->z_dim, h->cond_b, w.c, W, rows, W, h->z_dim);
-    MN_TRYZ(mn_gemm256_ex(&a, MN_G256_F32, 1, stream));
-  }
+  memset(&g, 0, sizeof(g));
+  g.h = w.z; g.ldh = h->z_dim; g.norm = 2; g.ng = h->vis_ln_g; g.nb = h->vis_ln_b; g.eps = 1e-6f;
+  g.Y = w.zs; g.ldy = h->z_dim; g.y_lo_off = (int64_t)rows * h->z_dim; g.M = rows; g.D = h->z_dim;
+  wide_glue(g, st);
+  a = g256_hilo(w.zs, h->z_dim, lo_at(LO_RF_COND, (int64_t)rows * h->z_dim), h->cond_w, h->z_dim, h->cond_b, w.c, W, rows, W, h->z_dim);
+  MN_TRYZ(mn_gemm256_ex(&a, MN_G256_F32, 1, stream));
 
   hipLaunchKernelGGL(rf_init_x_kernel, dim3(mn_cdiv(rows * T, 256)), dim3(256), 0, st, noise, temperature, w.x, rows, T, rpi);
   // modulations of every Euler step: [steps * rows, w] x [w, depth*3w + 2w], adaLN weights read once per token

@@ -42,11 +42,12 @@ def test_sampler(rows, images):
         assert float((whole[i] - one[0]).norm() / one.norm()) < 1e-4
 
 
-@pytest.mark.parametrize("w, hidden, steps", [(384, 128, 4), (64, 1024, 1), (128, 256, 2)])
+@pytest.mark.parametrize("w, hidden, steps", [(384, 128, 4), (64, 1024, 1), (128, 256, 2), (384, 1024, 1), (960, 128, 1)])
 @pytest.mark.parametrize("images", [3, 8, 11, 16])
 def test_condition(images, w, hidden, steps):
-    """The products before the blocks as one launch on fp32 rows, whose scratch is the modulations' memory, and on hi/lo rows where heads of one block and one step leave it
-    too small: two rows an image against each image alone."""
+    """The product before the blocks as one launch on fp32 rows, whose scratch is the modulations' memory, and on hi/lo rows where heads of one block and one step leave it
+    too small (384 behind 1024 values; of 960 behind 128 it holds this product's scratch and not the next one's; widths of 64 and 128 have no whole tiles and take the
+    streaming kernels): two rows an image against each image alone."""
     from ming_univision_amd import configuration as C
     from ming_univision_amd.rf_head import RectifiedFlowHead
     from ming_univision_amd.synth import synth_state_dict

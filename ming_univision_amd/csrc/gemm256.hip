@@ -588,10 +588,10 @@ static int tile_form(int M, int N, int Kc, int nz, bool hilo, int epi, bool may2
   return best;
 }
 
-template <int EPI, int BM, int BN, int WM, int WN, int S, bool HILO>
+template <int EPI, int BM, int BN, int WM, int WN, int S, bool HILO, bool TWO = false>
 static void tile_go(const G256& p, int nz, hipStream_t st) {
   const dim3 grid((unsigned)(mn_cdiv(p.M, BM) * mn_cdiv(p.N, epi_paired(EPI) ? BN / 2 : BN)), nz);
-  hipLaunchKernelGGL((gemm_tile_kernel<EPI, HILO, BM, BN, WM, WN, S>), grid, dim3(WM * WN * 64), 0, st, p);
+  hipLaunchKernelGGL((gemm_tile_kernel<EPI, HILO, BM, BN, WM, WN, S, TWO>), grid, dim3(WM * WN * 64), 0, st, p);
 }
 
 // stages: as many K-tiles as leave room for two workgroups of the 64-row forms on a CU (64 x 64 hi/lo: 3 x 24 KiB; 64 x 128: 3 x 24, hi/lo
@@ -614,11 +614,11 @@ static bool tile_launch(const G256& p, int form, int nz, bool hilo, hipStream_t 
     case 1: tile_go<EPI, 64, 64, 2, 2, 3, true>(p, nz, st); return true;
     case 2: tile_go<EPI, 64, 128, 2, 2, 2, true>(p, nz, st); return true;
     case 3: tile_go<EPI, 128, 128, 2, 4, 3, true>(p, nz, st); return true;
-    case 5: tile_go<EPI, 32, 64, 2, 2, 5, true>(p, nz, st); return true;
+    case 5: tile_go<EPI, 32, 64, 2, 2, 5, true, true>(p, nz, st); return true;
     case 6:
       if constexpr (EPI == E_SWIGLU_SPLIT) { tile_go<EPI, 48, 64, 1, 4, 4, true>(p, nz, st); return true; }
       return false;
-    case 7: tile_go<EPI, 64, 128, 4, 2, 3, true>(p, nz, st); return true;
+    case 7: tile_go<EPI, 64, 128, 4, 2, 3, true, true>(p, nz, st); return true;
     default: return false;
   }
 }

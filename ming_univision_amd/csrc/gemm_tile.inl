@@ -10,6 +10,9 @@
 //     buffer the loads of K-tile t + S - 1 may then overwrite.
 // HILO: the LDS image of a K-tile holds BM hi rows, then the same rows' lo parts; both are multiplied into accumulators of their own (the
 // sum is taken once, in the epilogue, as in the 256-tile kernel).
+// TWO: the hi products of a K-tile's halves go to two accumulators, so that a chain of fp32 additions is half as long, as it is in the K-slices that the flow head's few
+// rows had before these tiles: latents against 64 bits at 16 rows, 2 x 96 draws, 7.59e-6 and 7.73e-6 with one chain, 7.49e-6 and 7.56e-6 with two (slices: 7.50e-6
+// and 7.63e-6); the time is the same (a sampler call of 16 rows 8.13 ms; a total every 8 K-tiles instead of a second accumulator 8.25).
 template <int N>
 __device__ __forceinline__ void wait_vm_n() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory"); }
 
@@ -24,7 +27,7 @@ __device__ __forceinline__ void wait_tiles(int rem) {
   }
 }
 
-template <int EPI, bool HILO, int BM, int BN, int WM, int WN, int S>
+template <int EPI, bool HILO, int BM, int BN, int WM, int WN, int S, bool TWO = false>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
   constexpr int NW = WM * WN, AR = HILO ? 2 * BM : BM, QA = AR / 8 / NW, QW = BN / 8 / NW, STAGE = (AR + BN) * 128;
   constexpr int MI = BM / WM / 16, NJ = BN / WN / 16, AI = HILO ? 2 * MI : MI;
@@ -92,6 +95,13 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
   for (int i = 0; i < AI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 odd[TWO ? MI : 1][NJ];
+  if constexpr (TWO) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) odd[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
 #pragma unroll
   for (int t = 0; t < S - 1; ++t)
@@ -114,10 +124,20 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
 #pragma unroll
       for (int i = 0; i < AI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < NJ; ++j) {
+          f32x4& c = TWO && kk == 1 && i < MI ? odd[TWO ? i % MI : 0][j] : acc[i][j];
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], c, 0, 0, 0);
+        }
     }
     buf = buf + 1 == S ? 0 : buf + 1;
     nbuf = nbuf + 1 == S ? 0 : nbuf + 1;
+  }
+
+  if constexpr (TWO) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] += odd[i][j];
   }
 
   char* Cz = reinterpret_cast<char*>(p.C);

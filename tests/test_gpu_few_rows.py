@@ -61,3 +61,20 @@ def test_condition(images, w, hidden, steps):
     for i in range(images):
         one = head.sample(hid[2 * i:2 * i + 2].contiguous(), noise[i:i + 1].contiguous(), text_cfg=3.0, image_cfg=1.1, n_images=1)
         assert float((whole[i] - one[0]).norm() / one.norm()) < 1e-4
+
+
+@pytest.mark.parametrize("M, N, K", [(16, 256, 8192), (32, 68, 4096), (23, 512, 3072), (96, 16384, 3072)])
+def test_sums_in_two_chains(M, N, K):
+    """Positive operands, whose partial sums grow: a sum over all of K in one chain of fp32 additions (eight products at a time, as the matrix instruction rounds) is off
+    by twice what two chains of half the length are.  The tiles that took the flow head's few rows over from K-slices may not fall back to one."""
+    from ming_univision_amd import ops
+    g = torch.Generator().manual_seed(3)
+    x, w = ((0.5 + 0.5 * torch.rand(r, K, generator=g)).to(torch.bfloat16) for r in (M, N))
+    got = ops.gemm256(torch.stack([x, torch.zeros_like(x)]).cuda(), w.cuda(), None, "f32").cpu()
+    off = lambda v, ref: float(((v.double() - ref) / ref).pow(2).mean().sqrt())  # noqa: E731
+    few = min(N, 64)
+    parts = torch.einsum("mbk,nbk->bmn", x.double().reshape(M, -1, 8), w[:few].double().reshape(few, -1, 8)).float()
+    chain = torch.zeros(M, few)
+    for p in parts:
+        chain = chain + p
+    assert off(got, x.double() @ w.double().T) < 0.75 * off(chain, x.double() @ w[:few].double().T)

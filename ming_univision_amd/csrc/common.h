@@ -132,6 +132,19 @@ __device__ __forceinline__ float wave_max(float v) {
   v = row16_max(v);
   return fmaxf(fmaxf(lane_f(v, 0), lane_f(v, 16)), fmaxf(lane_f(v, 32), lane_f(v, 48)));
 }
+// Round k of a router's top-k over the experts of lanes [0, E): the best score, out of the running from then on, and its lane (the lowest of equal ones).  Scores of
+// NaN (a row of NaN is all NaN) are none: slot k then names expert k with a NaN weight, as every slot has to name an expert and no expert two slots of a row — a group of
+// more pairs than there are rows is one that the grouped products pass over, for all of its rows.
+__device__ __forceinline__ int topk_round(float& cur, int E, int k, float& best) {
+  best = wave_max(cur);
+  const int sel = __ffsll((long long)__ballot(cur == best)) - 1;
+  if ((uint32_t)sel >= (uint32_t)E) {
+    best = __builtin_nanf("");
+    return k;
+  }
+  if ((int)(threadIdx.x & 63) == sel) cur = -1.f;
+  return sel;
+}
 // s + l += v, s rounded, l collecting what the rounding left
 __device__ __forceinline__ void two_sum(float& s, float& l, float v) {
   const float t = s + v, b = t - s;

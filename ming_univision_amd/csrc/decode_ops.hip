@@ -18,10 +18,10 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // one 256-thread block per row writes the normalised row (input of the experts) and wave 0 does
 // the fp32 softmax + iterative arg-max top-k + renormalisation.
 //
-// TIE RULE (every router of this library: this kernel, moe_router_row_kernel below,
+// TIE RULE (topk_round in common.h, which every router of this library goes by: this kernel, moe_router_row_kernel below, moe_gate_up.hip,
 // moe_topk_logits_kernel in prefill_ops.hip and the wide route's top-k in wide_llm.inl): expert e lives in lane e; a round takes the
 // wave maximum and `__ffsll(__ballot(cur == best))`, i.e. among EQUAL scores the LOWEST expert id wins, and the picked slots are in
-// descending score / ascending id order.  The reference calls `torch.topk` (modeling_bailing_moe.py:512), whose order among equal
+// descending score / ascending id order; a row of NaN scores gets experts 0 .. top_k - 1 with NaN weights.  The reference calls `torch.topk` (modeling_bailing_moe.py:512), whose order among equal
 // values is unspecified; exact ties need two identical gate rows (fp32 scores of real weights tie with probability zero).
 // Pinned by tests/test_gpu_router_ties.py.
 // -------------------------------------------------------------------------------------------
@@ -52,11 +52,9 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(
     int myidx = 0;
     const int n_slot = top_k + n_shared;
     for (int k = 0; k < top_k; ++k) {
-      const float best = wave_max(cur);
-      const unsigned long long ball = __ballot(cur == best);
-      const int sel = __ffsll((long long)ball) - 1;
+      float best;
+      const int sel = topk_round(cur, E, k, best);
       if (lane == k) { myw = best; myidx = sel; }
-      if (lane == sel) cur = -1.f;
       wsum += best;
     }
     if (lane < top_k) {
@@ -199,10 +197,9 @@ __global__ __launch_bounds__(1024) void moe_router_row_kernel(
     int myidx = 0;
     const int n_slot = top_k + n_shared;
     for (int k = 0; k < top_k; ++k) {
-      const float best = wave_max(cur);
-      const int sel = __ffsll((long long)__ballot(cur == best)) - 1;
+      float best;
+      const int sel = topk_round(cur, E, k, best);
       if (lane == k) { myw = best; myidx = sel; }
-      if (lane == sel) cur = -1.f;
       wsum += best;
     }
     if (lane < top_k) {

@@ -776,9 +776,9 @@ __device__ __forceinline__ void sort_pairs(const int32_t* __restrict__ topk_idx,
   for (int i = tid; i < 16 * 256; i += NT) cnt[i >> 8][i & 255] = 0;
   int e[CW], rank[CW];
 #pragma unroll
-  for (int j = 0; j < CW; ++j) {                             // (a row of NaN logits has no top-k: its pairs go to some group)
+  for (int j = 0; j < CW; ++j) {
     const int p = 64 * (j * NW + wave) + lane;
-    e[j] = p < P ? min((int)min((uint32_t)topk_idx[p], (uint32_t)0x7fffffff), G - 1) : 0;
+    e[j] = p < P ? (int)min((uint32_t)topk_idx[p], (uint32_t)(G - 1)) : 0;
   }
   __syncthreads();
 #pragma unroll

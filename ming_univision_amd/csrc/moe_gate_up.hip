@@ -163,11 +163,10 @@ __global__ __launch_bounds__(GU_WAVES * 64) void moe_gate_up_routed_kernel(const
   float cur = lane < E ? pr : -1.f, wsum = 0.f, myw = 0.f;
   int myidx = 0, slot_e = E + (s - a.top_k);
   for (int k = 0; k < a.top_k; ++k) {
-    const float best = wave_max(cur);
-    const int sel = __ffsll((long long)__ballot(cur == best)) - 1;
+    float best;
+    const int sel = topk_round(cur, E, k, best);
     if (lane == k) { myw = best; myidx = sel; }
     if (k == s) slot_e = sel;
-    if (lane == sel) cur = -1.f;
     wsum += best;
   }
   if (blockIdx.x == 0 && s == 0) {                   // one workgroup per row publishes the routing (the down projection reads it)

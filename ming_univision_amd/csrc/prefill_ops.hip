@@ -276,10 +276,9 @@ __global__ __launch_bounds__(256) void moe_topk_logits_kernel(const float* __res
   int myidx = 0;
   const int n_slot = top_k + n_shared;
   for (int k = 0; k < top_k; ++k) {
-    const float best = wave_max(cur);
-    const int sel = __ffsll((long long)__ballot(cur == best)) - 1;
+    float best;
+    const int sel = topk_round(cur, E, k, best);
     if (lane == k) { myw = best; myidx = sel; }
-    if (lane == sel) cur = -1.f;
     wsum += best;
   }
   if (lane < top_k) {

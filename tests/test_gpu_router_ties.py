@@ -6,7 +6,7 @@ tie has measure zero; it only happens when two experts carry the same gate row. 
 
     among equal scores the LOWEST expert id wins   (expert e = lane e; a round picks `__ffsll(__ballot(cur == wave_max(cur)))`)
 
-— decode_ops.hip `moe_topk_kernel` / `moe_router_row_kernel` (the rule is written down there), engine.hip `moe_route_group_kernel`,
+— decode_ops.hip `moe_topk_kernel` / `moe_router_row_kernel` (the rule is written down there), moe_gate_up.hip,
 prefill_ops.hip `moe_topk_logits_kernel`, the wide route's top-k in wide_llm.inl.  These tests pin that rule: experts 3 and 40 (and 11, 52) share a gate row,
 so every row ties exactly, and the tie sits at the top-k boundary for many rows; the oracle is run with a stable descending sort
 (= lowest id first among equals), and the device must agree on all three routes (2 rows: chain; 40 rows: unfused <= 64-row route;

@@ -544,10 +544,16 @@ static const TileForm tile_hilo[] = {{1, 64, 64, 3.8, 0.41, 0.42, 0.60, 0.41}, {
 // many loads are in flight) is the time.  So tiles no taller than the rows: 3072 x 16384 with its SwiGLU at 16 rows 19.7 us (32-row tiles) against 28.3 (64), at 36
 // 25.2 (48-row tiles, gate and up in one fragment) against 29.5; and wider ones where slices of K leave enough of them: 8192 x 3072 at 36 rows 13.8 us
 // (64 x 128, 8 slices) against 15.8, at 16 rows 11.5 (32 x 64, 5 slices) against 14.4.  At 96 rows 3072 x 16384 with its SwiGLU 33.0 us (64 x 128) against 42.4 (64 x 64)
-// and 51 (128 x 128), 8192 x 3072 20.1 (5 slices) against 24.3 and 29.5.  max_m: 0 or the most rows the form takes; split: the split SwiGLU alone.
-struct FewForm { TileForm f; int max_m; bool split; };
-static const FewForm tile_few[] = {{{5, 32, 64, 3.8, 0.28, 0.36, 0.74, 0.40}, 32, false}, {{6, 48, 64, 3.8, 0.40, 0.44, 0.90, 0.50}, 48, true},
-                                   {{1, 64, 64, 3.8, 0.46, 0.53, 0.95, 0.55}, 128, false}, {{7, 64, 128, 4.0, 0.50, 0.72, 0, 0}, 128, false}};
+// and 51 (128 x 128), 8192 x 3072 20.1 (5 slices) against 24.3 and 29.5.  Where two rows of 64 are more workgroups than one round, one row of 128 reads the weights once:
+// 65 and 128 rows x 32000 x 1024 20.6 and 22.7 us (128 x 128) against 24.6 and 27.9 (64 x 128), x 65536 x 3072 86 and 100 (256 x 256) against 123 and 142, x 116736 x
+// 3072 153 and 179 against 231 and 270.  Up to 32 rows several rounds of 32 x 64 lose to 64 x 128: 16 and 32 rows x 32000 x 1024 14.9 and 16.2 against 14.0 and 14.7, x
+// 116736 x 3072 140 and 159 against 136 and 144.  The 48-row tiles gain where they are a workgroup a CU (above); 48 rows x 1152 units x 768 8.0 against 7.4 (64 x 64), x
+// 12288 units x 1024 17.2 against 14.0 (64 x 128).  The rows from min_m to max_m; split: the split SwiGLU alone.
+struct FewForm { TileForm f; int min_m, max_m; bool split; };
+static const FewForm tile_few[] = {{{5, 32, 64, 3.8, 0.28, 0.36, 0.76, 0.44}, 1, 32, false},     {{6, 48, 64, 3.8, 0.48, 0.48, 1.05, 0.55}, 33, 48, true},
+                                   {{1, 64, 64, 3.8, 0.46, 0.53, 0.95, 0.55}, 1, 128, false},    {{7, 64, 128, 4.0, 0.50, 0.72, 0, 0}, 1, 64, false},
+                                   {{7, 64, 128, 4.0, 0.50, 0.62, 0, 0}, 65, 128, false},        {{3, 128, 128, 4.2, 0.90, 1.08, 0, 0}, 65, 128, false},
+                                   {{0, 128, 256, 11.0, 0.95, 1.55, 0, 0}, 65, 128, false}};
 
 static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bool hilo, bool paired) {
   const double w = (double)(mn_cdiv(M, f.bm) * mn_cdiv(N, paired ? f.bn / 2 : f.bn) * nz) / 256.0;
@@ -568,7 +574,7 @@ static int tile_form(int M, int N, int Kc, int nz, bool hilo, int epi, bool may2
     int best = 0;
     double tb = 1e30;
     for (const FewForm& t : tile_few) {
-      if (M > t.max_m || (t.split && epi != E_SWIGLU_SPLIT)) continue;
+      if (M < t.min_m || M > t.max_m || (t.split && epi != E_SWIGLU_SPLIT) || (t.f.form == 0 && !may256)) continue;
       const double e = tile_time(t.f, M, N, Kc / BK, nz, true, paired);
       if (e < tb) { tb = e; best = t.f.form; }
     }

@@ -15,6 +15,13 @@ def test_rule(M):
         G.test_forms(M, N, K)
 
 
+@pytest.mark.parametrize("M", [1, 32, 33, 65, 127, 128])
+def test_rule_of_many_columns(M):
+    """More workgroups than a round of the few-row tiles: 64 x 128, and from 65 rows 128 x 128 (32004 columns) and 256 x 256 ones (65532)."""
+    for N, K in ((32004, 128), (65532, 512)):
+        G.test_forms(M, N, K)
+
+
 @pytest.mark.parametrize("form", [5, 6, 7])
 def test_forms_in_turn(dev_lib, form):
     dev_lib.mn_gemm_tile_tune(form)

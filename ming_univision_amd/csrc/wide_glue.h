@@ -260,8 +260,9 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(const WideGlue p) {
 inline bool wide_glue_ok(int D) { return D >= 4 && (D % 4) == 0 && D <= 4096; }
 
 inline void wide_glue(const WideGlue& g, hipStream_t st) {
-  // from six rows a CU on (1024 values, us, a workgroup / a wave a row: 512 rows 3.4 / 3.8, 1025 4.0 / 4.0, 1500 4.8 / 4.3, 2048 5.8 / 4.5)
-  if (g.norm == 2 && !g.x && !g.xin && !g.P && !g.cy && !g.h_out && !g.scale && !g.Y8 && !g.wait_flags && g.D <= 1024 && g.M >= 6 * mn_num_cus()) {
+  // from six rows a CU on (1024 values, us, a workgroup / a wave a row: 512 rows 3.4 / 3.8, 1025 4.0 / 4.0, 1500 4.8 / 4.3, 2048 5.8 / 4.5), of more than 256 values, where
+  // a row is more than one wave's (1536 rows of 512 3.6 / 3.6, 4096 5.8 / 4.9; of 256 3.1 / 3.3, 4.0 / 4.0)
+  if (g.norm == 2 && !g.x && !g.xin && !g.P && !g.cy && !g.h_out && !g.scale && !g.Y8 && !g.wait_flags && g.D > 256 && g.D <= 1024 && g.M >= 6 * mn_num_cus()) {
     hipLaunchKernelGGL(ln_rows_kernel<4>, dim3((unsigned)std::min<int64_t>(mn_cdiv(g.M, 4), 4 * mn_num_cus())), dim3(256), 0, st, g);
     return;
   }

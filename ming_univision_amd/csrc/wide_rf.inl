@@ -215,9 +215,11 @@ static int rf_sample_wide(const mn_rf_head* h, const float* hidden, int64_t ld_h
     MN_TRYZ(mn_quant_fp8_rows(w.y, W, y8, W, s_ada, SR, W, stream));
     a = g256_f8(y8, W, s_ada, h->ada_q, W, h->ada_scale, h->ada_b, w.ada, A, (int)SR, A, W);
     MN_TRYZ(mn_gemm256_ex(&a, MN_G256_F32, 1, stream));
-  } else {
+  } else if (mn_gemm256_supported(W, SR * W, W, A, (int)SR, A, W)) {
     a = g256_hilo(w.y, W, lo_at(LO_RF_ADA, SR * W), h->ada_w, W, h->ada_b, w.ada, A, (int)SR, A, W);
     MN_TRYZ(mn_gemm256_ex(&a, MN_G256_F32, 1, stream));
+  } else {                       // operands beyond 4 GiB (3072 wide: 76 blocks and more)
+    MN_TRYZ(mn_gemm_bf16_hilo(w.y, W, SR * W, h->ada_w, W, h->ada_b, w.ada, A, (int)SR, A, W, stream));
   }
 
   if (h->wfmt && !f8) {          // weight-only mode: W' of every block, once per call

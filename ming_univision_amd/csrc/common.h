@@ -213,5 +213,16 @@ extern "C" int mn_gemm256_ex(const mn_g256* a, int epi, int ksplit, void* stream
 extern "C" int mn_gemm256_slices(int K, int ksplit);
 extern "C" int mn_axpy_rms_rows_slabs(float* x, int64_t ldx, const float* y, int64_t ldy, int nz, int64_t zs, float mult, const uint16_t* w, float eps,
                                       float* n_out, int64_t ldn, uint16_t* n16, int64_t ldn16, int M, int n, void* stream);
+// rows that a producer leaves as the next product's bf16 hi and lo planes: where mn_skinny_gemm reads them (NULL: no product of three launches), that product from them, and
+// the producers (latent_ops.hip); q, k, v planes (MN_G256_BF16_SPLIT) into attention (flash_prefill.hip)
+extern "C" uint16_t* mn_skinny_operand(const mn_skinny_args* a);
+extern "C" int mn_skinny_gemm_presplit(const mn_skinny_args* a, void* stream);
+extern "C" int mn_gated_norm_filter_rows_split(float* x, int64_t ldx, const float* g, int64_t ldg, const float* y, int64_t ldy, const uint16_t* wa, const uint16_t* ba,
+                                               const uint16_t* wb, const uint16_t* bb, float eps, float* n_out, int64_t ldn, const uint16_t* taps_w, int taps, float* state,
+                                               const int32_t* row_seq, const int32_t* row_slot, float* h, int64_t ldh, uint16_t* y16, int M, int n, void* stream);
+extern "C" int mn_polynorm_rows_split(const float* z, int64_t ldz, const uint16_t* coef, float eps, uint16_t* y16, int M, int n, void* stream);
+extern "C" int mn_rms_rows_pair(const float* xa, const uint16_t* wa, float* ya, int64_t ldya, uint16_t* ya16, int64_t ldya16, int na, const float* xb, const uint16_t* wb,
+                                float* yb, const int32_t* row_seq, const int32_t* row_slot, int t_max, int nb, int64_t ldx, float eps, int M, void* stream);
+extern "C" int mn_attn_prefill_hd64_planes(const uint16_t* qkv, int64_t lo_off, uint16_t* split, int B, int T, int n_heads, int causal, void* stream);
 extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo);
 extern "C" int mn_gemm256_f8_plan_ksplit(int M, int N, int K);

@@ -99,8 +99,8 @@ __global__ __launch_bounds__(1024) void moe_router_row_kernel(
         if (e < E && k < H) gw[i][j] = *reinterpret_cast<const u4*>(G + (int64_t)e * H + k);
       }
   }
-  // P != NULL (the decoder chain at <= 4 rows): the row is h + the nz K-slice partial slabs of the attention output projection, summed
-  // here (in slab order, like llm_glue_kernel) and written back to h_out — the residual glue launch and the gate launch fold into this one
+  // P != NULL (the decoder chain, up to 64 rows): the row is h + the sum of the nz K-slice partial slabs of the attention output projection (the slabs first, in slab order, as
+  // llm_glue_kernel does), written back to h_out — the residual glue launch and the gate launch fold into this one
   float xv[4], add[4] = {0.f, 0.f, 0.f, 0.f};     // H <= 4096: columns tid, tid + 1024, ...
   float ss = 0.f;
 #pragma unroll

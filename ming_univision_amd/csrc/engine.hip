@@ -1038,7 +1038,7 @@ struct LlmWs {
   int32_t* ti;
   MoeWs moe;
   bf16_t *yh, *ya;      // chain: bf16 hi/lo operands of width H and n_q * head_dim
-  float* pp;            // chain: K-slice partials of the QKV / dense / gate launches
+  float* pp;            // chain: K-slice partials of the QKV / dense launches
   void* attn_ws;
   size_t attn_ws_bytes;
   char* sk_ws;
@@ -1069,9 +1069,7 @@ static size_t llm_carve(const mn_llm* m, int rows, int64_t t_max, void* ws, size
     o->ya = cv.take<bf16_t>((size_t)2 * rows * ad);
     size_t pmax = (size_t)mn_stream_mfma_slices(rows, qkv_dim, m->hidden) * qkv_dim;
     const size_t p2 = (size_t)mn_stream_mfma_slices(rows, m->hidden, ad) * m->hidden;
-    const size_t p3 = (size_t)mn_stream_mfma_slices(rows, m->n_experts, m->hidden) * m->n_experts;
     if (p2 > pmax) pmax = p2;
-    if (p3 > pmax) pmax = p3;
     o->pp = cv.take<float>(pmax * rows);
   }
   return cv.off;

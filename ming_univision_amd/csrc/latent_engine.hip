@@ -7,14 +7,6 @@
 // The per-head absorb (q W_uk) and expand (latent W_uv^T) products are batched over heads in fp32 (mn_gemm_f32_batched) in both modes.
 #include "seq_linear.h"
 
-extern "C" int mn_rms_rows_pair(const float* xa, const uint16_t* wa, float* ya, int64_t ldya, uint16_t* ya16, int64_t ldya16, int na, const float* xb, const uint16_t* wb,
-                                float* yb, const int32_t* row_seq, const int32_t* row_slot, int t_max, int nb, int64_t ldx, float eps, int M, void* stream);
-
-extern "C" int mn_gated_norm_filter_rows_split(float* x, int64_t ldx, const float* g, int64_t ldg, const float* y, int64_t ldy, const uint16_t* wa, const uint16_t* ba,
-                                               const uint16_t* wb, const uint16_t* bb, float eps, float* n_out, int64_t ldn, const uint16_t* taps_w, int taps, float* state,
-                                               const int32_t* row_seq, const int32_t* row_slot, float* h, int64_t ldh, uint16_t* y16, int M, int n, void* stream);
-extern "C" int mn_polynorm_rows_split(const float* z, int64_t ldz, const uint16_t* coef, float eps, uint16_t* y16, int M, int n, void* stream);
-
 extern "C" size_t mn_sizeof_seq_layer(void) { return sizeof(mn_seq_layer); }
 extern "C" size_t mn_sizeof_seq_model(void) { return sizeof(mn_seq_model); }
 extern "C" size_t mn_sizeof_seq_state(void) { return sizeof(mn_seq_state); }

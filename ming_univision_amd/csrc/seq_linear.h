@@ -8,9 +8,6 @@
 
 #include "common.h"
 
-extern "C" uint16_t* mn_skinny_operand(const mn_skinny_args* a);
-extern "C" int mn_skinny_gemm_presplit(const mn_skinny_args* a, void* stream);
-
 namespace {
 
 inline size_t al(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -37,8 +34,8 @@ inline int linear(int arith, int M, const float* A, int64_t lda, const uint16_t*
   return mn_gemm_f32_batched(A, lda, 0, W, K, 0, bias, C, ldc, 0, nullptr, 0, 0, nullptr, 0, 0, M, N, K, 1, 1.0f, stream);
 }
 
-// Where the kernel that makes the rows A of linear()'s call may leave them as bf16 hi rows and lo rows ([2, M, K], at the start of gws) for linear_presplit to take up: a
-// step's launch less (32 rows of 2048: 5.2 us).  NULL: linear() takes another route.  Nothing else may use gws in between.
+// Where the kernel that makes the rows A of linear()'s call may leave them as bf16 hi rows and lo rows ([2, M, K], at the start of gws) for mn_skinny_gemm_presplit to take
+// up: a launch less a product (32 rows of 2048: 5.2 us).  NULL: linear() takes another route.  Nothing else may use gws in between.
 inline uint16_t* linear_operand(int arith, int M, const float* A, int64_t lda, const uint16_t* W, int N, int K, const uint16_t* bias, float* C, int64_t ldc, void* gws,
                                 size_t gws_bytes, mn_skinny_args* a) {
   if (arith != MN_SEQ_ARITH_BF16 || M <= 8 || M > 64 || !mfma_ok(W, K)) return nullptr;

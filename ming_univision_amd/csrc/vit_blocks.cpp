@@ -3,8 +3,6 @@
 // one call per launch from Python costs more than the launch runs: 60 blocks took 5.1 ms of host time over 3.1 ms of kernels.
 #include "common.h"
 
-extern "C" int mn_attn_prefill_hd64_planes(const uint16_t* qkv, int64_t lo_off, uint16_t* split, int B, int T, int n_heads, int causal, void* stream);
-
 namespace {
 
 size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }

@@ -37,6 +37,17 @@ Plan plan(int64_t M, int dim, int hidden, int gelu, int precise) {
   return p;
 }
 
+// the products that take their LayerNorm or residual with them (vit_rows.hip): few rows, 16-byte weights, 8-byte biases and norm parameters
+bool rows_ok(const float* x, const uint16_t* const* w, int depth, int64_t M, int dim, int hidden, int gelu) {
+  if (!mn_vit_rows_ok((int)M, dim, hidden, gelu) || ((uintptr_t)x & 15)) return false;
+  for (int i = 0; i < 12 * depth; ++i) {
+    const int k = i % 12;
+    const uintptr_t mask = k == 2 || k == 4 || k == 8 || k == 10 ? 15 : 7;
+    if ((uintptr_t)w[i] & mask) return false;
+  }
+  return true;
+}
+
 #define TRY(e) do { const int rc_ = (e); if (rc_ < 0) return rc_; } while (0)
 
 }  // namespace
@@ -90,6 +101,16 @@ extern "C" int mn_vit_blocks(float* x, int B, int T, int dim, int depth, const u
   }
   uint16_t *qkv = reinterpret_cast<uint16_t*>(base), *h = qkv, *xn = reinterpret_cast<uint16_t*>(base + p.b), *att = reinterpret_cast<uint16_t*>(base + p.c);
   float* slabs = reinterpret_cast<float*>(base + p.p);
+  if (rows_ok(x, w, depth, M, dim, hidden, gelu)) {
+    for (int i = 0; i < depth; ++i, w += 12) {
+      TRY(mn_ln_gemm_rows(x, dim, w[0], w[1], eps, w[2], dim, w[3], 0, 0, qkv, 3 * (int64_t)dim, M, 3 * dim, dim, stream));
+      TRY(mn_attn_prefill_hd64(qkv, att, B, T, nh, causal, stream));
+      TRY(mn_resid_gemm_rows(att, dim, w[4], dim, w[5], x, dim, M, dim, dim, stream));
+      TRY(mn_ln_gemm_rows(x, dim, w[6], w[7], eps, w[8], dim, w[9], gelu, !gelu, h, hidden, M, hidden, dim, stream));
+      TRY(mn_resid_gemm_rows(h, hidden, w[10], hidden, w[11], x, dim, M, dim, hidden, stream));
+    }
+    return mn_layernorm_bf16(x, dim, fin_g, fin_b, eps, out, dim, M, dim, fin_gelu, stream);
+  }
   bool normed = false;                         // xn holds the next product's input: the tail of the product before wrote it
   // x += A W^T + b, and the LayerNorm behind it where the product runs split-K (one launch sums the slabs, updates the stream and norms its rows)
   auto resid = [&](const uint16_t* A, int K, const uint16_t* W, const uint16_t* b, const uint16_t* g, const uint16_t* be, int act, uint16_t* y) -> int {

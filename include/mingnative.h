@@ -512,8 +512,8 @@ MN_API int mn_llm_route_capture(int32_t* capture);
 
 /* mn_llm_step with flags.  MN_STEP_DISTINCT_SEQUENCES: every row belongs to a different cache sequence and row_len == row_slot + 1
  * (a decode step of independent conversations / CFG rows — NOT a prefill chunk, whose rows attend each other's new K / V lines): the
- * rotary embedding and the K / V append then ride the attention launch (one launch fewer per layer; <= 64 rows, n_q / n_kv in
- * {1, 2, 4}).  Results are identical to mn_llm_step. */
+ * rotary embedding and the K / V append then ride the attention launch (two launches fewer per layer; n_q / n_kv in {1, 2, 4}).
+ * Results are those of mn_llm_step up to the order of fp32 sums. */
 #define MN_STEP_DISTINCT_SEQUENCES 1
 MN_API int mn_llm_step_ex(const mn_llm* m, const float* x, int64_t ldx, int x_row_div, int M, const uint8_t* image_mask,
                    const int32_t* row_seq, const int32_t* row_slot, const int32_t* row_pos, const int32_t* row_len,

@@ -372,11 +372,8 @@ extern "C" int mn_rope_kv_append(const float* qkv, int64_t ldqkv, int M, int n_q
 // cover 4 consecutive q heads (= one GQA group when n_q/n_kv == 4, so K/V lines are shared in L1).
 // partial layout: [M][n_q][S][HD + 2]  (acc[HD], m, l)
 // -------------------------------------------------------------------------------------------
-// FUSED (round 4): the launch takes the RAW QKV projection instead of q — the rotary embedding of the row's q and new k, the
-// q scale and the K / V append of the new token (rope_kv_append_kernel, one launch per layer and step before) happen here: every
-// wave rotates its own q head into LDS; in the split that holds the new key, the first q head of each KV group writes the group's
-// K / V line into the arena (n_q / n_kv in {1, 2, 4}: the 4 heads of a block never straddle a KV group, so the line's readers are
-// waves of the SAME workgroup, ordered by vmcnt(0) + the barrier; the vector L1 holds no older copy of a line nobody read yet).
+// What mn_attn_decode_fused's launch takes instead of q: the RAW QKV projection; the rotary embedding of the row's q and new k, the q scale and the K / V append of the new token
+// happen in the attention launch.
 struct AttnFuse {
   const float* qkv; int64_t ldqkv; int nz; int64_t slab;        // raw QKV rows [(n_q + 2 n_kv) * HD], optionally nz K-slice partial slabs
   int rope; const float* cos_tab; const float* sin_tab;          // [n_pos, HD / 2]
@@ -384,13 +381,12 @@ struct AttnFuse {
   float* kv_cache_w;                                              // the arena, writable
 };
 
-template <int HD, bool FUSED>
+template <int HD>
 __global__ __launch_bounds__(256) void attn_decode_split_kernel(
     const float* __restrict__ q, int n_q, int n_kv, const float* __restrict__ kv_cache, int64_t t_max,
     const int32_t* __restrict__ row_seq, const int32_t* __restrict__ row_len, const uint8_t* __restrict__ key_mask,
-    int64_t ld_mask, int S, int chunk_cap, float* __restrict__ partial, const AttnFuse fz) {
+    int64_t ld_mask, int S, int chunk_cap, float* __restrict__ partial) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
-  __shared__ __attribute__((aligned(16))) float qs[FUSED ? 4 * HD : 4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = blockIdx.x, s = blockIdx.z;
   const int h_raw = blockIdx.y * 4 + wave;
@@ -409,50 +405,12 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
   const uint8_t* mk = key_mask ? key_mask + (int64_t)m * ld_mask : nullptr;
   float* out = partial + (((int64_t)m * n_q + h) * S + s) * (HD + 2);
 
-  if constexpr (FUSED) {
-    constexpr int half = HD / 2;
-    const float* row = fz.qkv + (int64_t)m * fz.ldqkv;
-    auto fetch = [&](int head, int i) {                 // element i of projection head `head` (q heads, then k heads, then v heads)
-      const float* p_ = row + (int64_t)head * HD + i;
-      float v = p_[0];
-      for (int z = 1; z < fz.nz; ++z) v += p_[z * fz.slab];
-      return v;
-    };
-    float c = 1.f, sn = 0.f;
-    if (lane < half && fz.rope) {
-      const int stream = fz.sec_t <= 0 ? 0 : (lane < fz.sec_t ? 0 : (lane < fz.sec_t + fz.sec_h ? 1 : 2));
-      const int pos = fz.row_pos[stream * fz.M + m];
-      c = fz.cos_tab[(int64_t)pos * half + lane];
-      sn = fz.sin_tab[(int64_t)pos * half + lane];
-    }
-    if (lane < half) {                                  // this wave's q head: rotate, scale, park in LDS
-      const float x1 = fetch(h, lane), x2 = fetch(h, lane + half);
-      qs[wave * HD + lane] = (x1 * c - x2 * sn) * fz.q_scale;
-      qs[wave * HD + lane + half] = (x2 * c + x1 * sn) * fz.q_scale;
-    }
-    const int slot = fz.row_slot[m];
-    const int ratio = n_q / n_kv;
-    // the new token's K / V line: written once per KV group, by the group's first q head, in the split that will read it
-    if (active && h % ratio == 0 && slot >= j0 && slot < j0 + chunk && (uint64_t)slot < (uint64_t)t_max && lane < half) {
-      const float k1 = fetch(n_q + kvh, lane), k2 = fetch(n_q + kvh, lane + half);
-      float* kd = fz.kv_cache_w + (((seq * 2 + 0) * n_kv + kvh) * t_max + slot) * HD;
-      float* vd = fz.kv_cache_w + (((seq * 2 + 1) * n_kv + kvh) * t_max + slot) * HD;
-      kd[lane] = k1 * c - k2 * sn;
-      kd[lane + half] = k2 * c + k1 * sn;
-      vd[lane] = fetch(n_q + n_kv + kvh, lane);
-      vd[lane + half] = fetch(n_q + n_kv + kvh, lane + half);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    // (callers pass row_len = row_slot + 1: the split that contains `slot` always exists)
-  }
-
   // ---- scores: 16 lanes per key, 4 keys per wave-iteration
   constexpr int PER = HD / 16;  // floats per lane (8 for 128, 4 for 64)
   const int sub = lane & 15, kq = lane >> 4;
   float qv[PER];
 #pragma unroll
-  for (int i = 0; i < PER; ++i) qv[i] = FUSED ? qs[wave * HD + sub * PER + i] : qr[sub * PER + i];
+  for (int i = 0; i < PER; ++i) qv[i] = qr[sub * PER + i];
   float mx = -INFINITY;
   for (int j = j0 + kq; j < j0 + chunk; j += 4) {
     float d = 0.f;
@@ -697,25 +655,19 @@ __global__ void attn_decode_combine_kernel(const float* __restrict__ partial, in
 // the semantic decoder's row; <= 1024 keys): one 16-wave workgroup per (row, q head).  The key range is split over the WAVES of the
 // workgroup, their (acc, max, sum) partials meet in LDS — no partial round trip through memory and no combine launch (split 9.8 us +
 // combine 4.7 us per layer at 2 rows before).  Scores and PV run on 16 / 8 keys' loads in flight per wave.
-// FUSED: as in the split kernel the launch takes the raw QKV row; here every workgroup rotates its q head AND the new key of its KV
-// group into LDS and attends to that key from there (the first q head of the group also writes the K / V line into the arena: no
-// workgroup reads the new line from memory in this launch, so the heads of a group need no ordering among themselves).
 // (A form with ALL of a wave's K and V loads issued before the first score — <= 24 keys per wave, 123 VGPRs — measured no faster:
 // 2.046 vs 2.059 ms per 28-layer step at 1 row / 296 keys, slower at 40 keys; removed.  profiles/r04_attn_fused_ab.txt)
-template <int HD, bool FUSED>
+template <int HD>
 __global__ __launch_bounds__(1024) void attn_decode_one_kernel(
     const float* __restrict__ q, int n_q, int n_kv, const float* __restrict__ kv_cache, int64_t t_max,
     const int32_t* __restrict__ row_seq, const int32_t* __restrict__ row_len, const uint8_t* __restrict__ key_mask,
-    int64_t ld_mask, int chunk_cap, float* __restrict__ out, bf16_t* __restrict__ split, int M, const AttnFuse fz) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];      // [16][chunk_cap] scores, [16][HD + 2] partials, [3][HD] q / new k / new v
+    int64_t ld_mask, int chunk_cap, float* __restrict__ out, bf16_t* __restrict__ split, int M) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];      // [16][chunk_cap] scores, [16][HD + 2] partials
   constexpr int NW = 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = blockIdx.x, h = blockIdx.y;
   float* sc = sm + wave * chunk_cap;
   float* part = sm + NW * chunk_cap;
-  float* qs = part + NW * (HD + 2);
-  float* knew = qs + HD;
-  float* vnew = knew + HD;
   const int len = row_len[m];
   int chunk = (len + NW - 1) / NW;
   chunk = (chunk + 3) & ~3;
@@ -725,41 +677,6 @@ __global__ __launch_bounds__(1024) void attn_decode_one_kernel(
   const float* Kb = kv_cache + ((seq * 2 + 0) * n_kv + kvh) * t_max * HD;
   const float* Vb = kv_cache + ((seq * 2 + 1) * n_kv + kvh) * t_max * HD;
   const uint8_t* mk = key_mask ? key_mask + (int64_t)m * ld_mask : nullptr;
-  int slot = -1;                                 // FUSED: the new key lives in LDS, not in the arena
-  if constexpr (FUSED) {
-    constexpr int half = HD / 2;
-    slot = fz.row_slot[m];
-    if (wave < 3 && lane < half) {               // wave 0: q head h, wave 1: the group's new k, wave 2: its new v
-      const float* row = fz.qkv + (int64_t)m * fz.ldqkv;
-      const int head = wave == 0 ? h : (wave == 1 ? n_q + kvh : n_q + n_kv + kvh);
-      const float* p_ = row + (int64_t)head * HD + lane;
-      float x1 = 0.f, x2 = 0.f;
-      for (int z0 = 0; z0 < fz.nz; z0 += 8) {      // eight slabs' loads in flight
-        float a1[8], a2[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          a1[j] = z0 + j < fz.nz ? p_[(int64_t)(z0 + j) * fz.slab] : 0.f;
-          a2[j] = z0 + j < fz.nz ? p_[(int64_t)(z0 + j) * fz.slab + half] : 0.f;
-        }
-        for (int j = 0; j < 8; ++j) x1 += a1[j];                    // (the one-by-one loop's order: same bits)
-        for (int j = 0; j < 8; ++j) x2 += a2[j];
-      }
-      if (fz.rope && wave < 2) {
-        const int stream = fz.sec_t <= 0 ? 0 : (lane < fz.sec_t ? 0 : (lane < fz.sec_t + fz.sec_h ? 1 : 2));
-        const int pos = fz.row_pos[stream * fz.M + m];
-        const float c = fz.cos_tab[(int64_t)pos * half + lane], sn = fz.sin_tab[(int64_t)pos * half + lane];
-        rotate_pair(x1, x2, c, sn);
-      }
-      if (wave == 0) { x1 *= fz.q_scale; x2 *= fz.q_scale; }
-      float* dst = wave == 0 ? qs : (wave == 1 ? knew : vnew);
-      dst[lane] = x1; dst[lane + half] = x2;
-      if (wave > 0 && h % (n_q / n_kv) == 0 && (uint64_t)slot < (uint64_t)t_max) {     // the arena line, once per KV group
-        float* ad = fz.kv_cache_w + (((seq * 2 + (wave - 1)) * n_kv + kvh) * t_max + slot) * HD;
-        ad[lane] = x1; ad[lane + half] = x2;
-      }
-    }
-    __syncthreads();
-  }
   // ---- scores: 16 lanes per key, 4 keys per step, 4 steps' loads in flight
   constexpr int PER = HD / 16;
   constexpr int DPL = HD / 64;
@@ -767,7 +684,7 @@ __global__ __launch_bounds__(1024) void attn_decode_one_kernel(
   const int n = max(0, j1 - j0);
   float qv[PER];
 #pragma unroll
-  for (int i = 0; i < PER; ++i) qv[i] = FUSED ? qs[sub * PER + i] : q[((int64_t)m * n_q + h) * HD + sub * PER + i];
+  for (int i = 0; i < PER; ++i) qv[i] = q[((int64_t)m * n_q + h) * HD + sub * PER + i];
   float mx = -INFINITY;
   for (int jb = j0; jb < j0 + chunk; jb += 16) {
     f32x4 kv[4][PER / 4];
@@ -777,10 +694,7 @@ __global__ __launch_bounds__(1024) void attn_decode_one_kernel(
 #pragma unroll
       for (int i = 0; i < PER / 4; ++i) {
         kv[u][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (j < j1) {
-          if (FUSED && j == slot) kv[u][i] = *reinterpret_cast<const f32x4*>(knew + sub * PER + i * 4);
-          else kv[u][i] = *reinterpret_cast<const f32x4*>(Kb + (int64_t)j * HD + sub * PER + i * 4);
-        }
+        if (j < j1) kv[u][i] = *reinterpret_cast<const f32x4*>(Kb + (int64_t)j * HD + sub * PER + i * 4);
       }
     }
 #pragma unroll
@@ -821,7 +735,7 @@ __global__ __launch_bounds__(1024) void attn_decode_one_kernel(
       for (int i = 0; i < DPL; ++i) {
         const int j = j0 + jb + u;
         v[u][i] = 0.f;
-        if (jb + u < n) v[u][i] = (FUSED && j == slot) ? vnew[lane * DPL + i] : Vb[(int64_t)j * HD + lane * DPL + i];
+        if (jb + u < n) v[u][i] = Vb[(int64_t)j * HD + lane * DPL + i];
       }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -854,7 +768,7 @@ __global__ __launch_bounds__(1024) void attn_decode_one_kernel(
     v = at / lt;
   } else {      // no attended key: uniform over the row's keys (see attn_decode_combine_kernel)
     float sum = 0.f;
-    for (int j = 0; j < len; ++j) sum += (FUSED && j == slot) ? vnew[d] : Vb[(int64_t)j * HD + d];
+    for (int j = 0; j < len; ++j) sum += Vb[(int64_t)j * HD + d];
     v = len > 0 ? sum / (float)len : 0.f;
   }
   const int64_t o = ((int64_t)m * n_q + h) * HD + d;
@@ -863,6 +777,243 @@ __global__ __launch_bounds__(1024) void attn_decode_one_kernel(
     const bf16_t hi = f32_to_bf16(v);
     split[o] = hi;
     split[(int64_t)M * n_q * HD + o] = f32_to_bf16(v - bf16_to_f32(hi));
+  }
+}
+
+// -------------------------------------------------------------------------------------------
+// One launch for a few rows over caches of any length: a workgroup per (row, KV head, key split), all G query heads of the group from one read of K and V, RoPE and the K / V
+// append of the new token with it (as in the one-workgroup form above), and the last split of a (row, KV head) to arrive joins them all.
+// What bounds it is latency: the kernel's arguments, the row's numbers, K and V together, the partial results, the arrival, the join are one round trip each.
+//   * a lane group of 16 owns a key; it keeps its own running maximum, sum and G outputs, so that nothing crosses lanes inside the key loop but the score itself;
+//   * K and V of U keys a group are asked for at once, before the query is rotated;
+//   * a split is at least `keys` long: a short row is one split, which needs no join (the grid is sized for the cache, the row's length is known here);
+//   * partials leave write-through (agent scope) and are drained before the arrival is counted; the last arrival (one counter a (row, KV head), zero between launches)
+//     reads them past its L1 in split order: the result does not depend on who is last.
+// -------------------------------------------------------------------------------------------
+template <int HD, int G, int NW, int U, int WPE>
+__global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q, int n_kv, int64_t t_max, const int32_t* __restrict__ row_seq, const int32_t* __restrict__ row_len,
+                                                                   const uint8_t* __restrict__ key_mask, int64_t ld_mask, int S_max, int keys, float* __restrict__ partial,
+                                                                   uint32_t* __restrict__ arrived, float* __restrict__ out, bf16_t* __restrict__ split, const AttnFuse fz) {
+  constexpr int half = HD / 2, PER = HD / 16, V4 = PER / 4, GR = 4 * NW, N = G * PER, TH = NW * 64;
+  __shared__ __attribute__((aligned(16))) float qs[G * HD], knew[HD], vnew[HD];
+  __shared__ __attribute__((aligned(16))) float part[NW][G * HD], mw[NW][G], lw[NW][G];
+  __shared__ uint32_t last;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), sub = lane & 15, row4 = lane >> 4, grp = wave * 4 + row4;
+  const int m = blockIdx.x, kvh = blockIdx.y, s = blockIdx.z;
+  const int len = row_len[m], slot = fz.row_slot[m];
+  const int64_t seq = row_seq[m];
+  const int S = len <= keys + keys / 2 ? 1 : min(S_max, (len + keys - 1) / keys);
+  if (s >= S) return;                                    // uniform
+  const int chunk = (len + S - 1) / S, j0 = s * chunk, j1 = min(len, j0 + chunk);
+  const float* Kb = fz.kv_cache_w + ((seq * 2 + 0) * n_kv + kvh) * t_max * HD + sub * PER;
+  const float* Vb = fz.kv_cache_w + ((seq * 2 + 1) * n_kv + kvh) * t_max * HD + sub * PER;
+  const uint8_t* mk = key_mask ? key_mask + (int64_t)m * ld_mask : nullptr;
+  f32x4 k[U][V4], v[U][V4];
+  bool keep[U];
+  auto fetch = [&](int jb) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = jb + u * GR + grp, jc = min(j, j1 - 1);
+      keep[u] = j < j1;
+      if (keep[u] && mk) keep[u] = mk[j] != 0;
+#pragma unroll
+      for (int i = 0; i < V4; ++i) {
+        k[u][i] = *reinterpret_cast<const f32x4*>(Kb + (int64_t)jc * HD + i * 4);
+        v[u][i] = *reinterpret_cast<const f32x4*>(Vb + (int64_t)jc * HD + i * 4);
+      }
+    }
+  };
+  if (j0 < j1) fetch(j0);
+  // ---- the row's query heads of this group, and the new key and value where the split holds them: slabs summed, rotated, into LDS ----
+  const bool fresh = slot >= j0 && slot < j1;
+  {
+    const float* row = fz.qkv + (int64_t)m * fz.ldqkv;
+    for (int t = tid; t < (fresh ? G + 2 : G) * half; t += TH) {
+      const int hh = t / half, i = t % half, head = hh < G ? kvh * G + hh : n_q + (hh - G) * n_kv + kvh;
+      const float* p_ = row + (int64_t)head * HD + i;
+      float x1 = 0.f, x2 = 0.f, c = 1.f, sn = 0.f;
+      const bool rot = fz.rope && hh <= G;
+      if (rot) {
+        const int stream = fz.sec_t <= 0 ? 0 : (i < fz.sec_t ? 0 : (i < fz.sec_t + fz.sec_h ? 1 : 2));
+        const int pos = fz.row_pos[stream * fz.M + m];
+        c = fz.cos_tab[(int64_t)pos * half + i];
+        sn = fz.sin_tab[(int64_t)pos * half + i];
+      }
+      for (int z0 = 0; z0 < fz.nz; z0 += 8) {            // eight slabs' loads in flight, added in slab order
+        float a1[8], a2[8];
+#pragma unroll
+        for (int z = 0; z < 8; ++z) {
+          a1[z] = z0 + z < fz.nz ? p_[(int64_t)(z0 + z) * fz.slab] : 0.f;
+          a2[z] = z0 + z < fz.nz ? p_[(int64_t)(z0 + z) * fz.slab + half] : 0.f;
+        }
+#pragma unroll
+        for (int z = 0; z < 8; ++z) { x1 += a1[z]; x2 += a2[z]; }
+      }
+      if (rot) rotate_pair(x1, x2, c, sn);
+      if (hh < G) { x1 *= fz.q_scale; x2 *= fz.q_scale; }
+      float* dst = hh < G ? qs + hh * HD : hh == G ? knew : vnew;
+      dst[i] = x1;
+      dst[i + half] = x2;
+      if (hh >= G && (uint64_t)slot < (uint64_t)t_max) {   // the new token's line of the arena
+        float* ad = fz.kv_cache_w + (((seq * 2 + (hh - G)) * n_kv + kvh) * t_max + slot) * HD;
+        ad[i] = x1;
+        ad[i + half] = x2;
+      }
+    }
+  }
+  __syncthreads();
+  f32x4 q[G][V4];
+  float acc[N], mx[G], l[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    mx[g] = -INFINITY;
+    l[g] = 0.f;
+#pragma unroll
+    for (int i = 0; i < V4; ++i) q[g][i] = *reinterpret_cast<const f32x4*>(qs + g * HD + sub * PER + i * 4);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) acc[i] = 0.f;
+  for (int jb = j0; jb < j1; jb += U * GR) {
+    if (jb > j0) fetch(jb);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (fresh && jb + u * GR + grp == slot) {
+#pragma unroll
+        for (int i = 0; i < V4; ++i) {
+          k[u][i] = *reinterpret_cast<const f32x4*>(knew + sub * PER + i * 4);
+          v[u][i] = *reinterpret_cast<const f32x4*>(vnew + sub * PER + i * 4);
+        }
+      }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float d[U], top = mx[g];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        float a = 0.f;
+#pragma unroll
+        for (int i = 0; i < V4; ++i) {
+          a = fmaf(k[u][i].x, q[g][i].x, a); a = fmaf(k[u][i].y, q[g][i].y, a);
+          a = fmaf(k[u][i].z, q[g][i].z, a); a = fmaf(k[u][i].w, q[g][i].w, a);
+        }
+        a = row16_sum(a);
+        d[u] = keep[u] ? a : -INFINITY;
+        top = fmaxf(top, d[u]);
+      }
+      const float f = mx[g] == -INFINITY ? 0.f : __expf(mx[g] - top);
+      l[g] *= f;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) acc[g * PER + i] *= f;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float p = d[u] == -INFINITY ? 0.f : __expf(d[u] - top);
+        l[g] += p;
+        if (keep[u]) {                                   // (a key that is not attended may hold anything)
+#pragma unroll
+          for (int i = 0; i < PER; ++i) acc[g * PER + i] = fmaf(p, v[u][i / 4][i % 4], acc[g * PER + i]);
+        }
+      }
+      mx[g] = top;
+    }
+  }
+  // ---- a wave's four groups: one maximum, then a sum that leaves each group a quarter of the outputs (values i + N / 4 (row4 >> 1) + N / 2 (row4 & 1)) ----
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    float top = fmaxf(mx[g], __shfl_xor(mx[g], 16));
+    top = fmaxf(top, __shfl_xor(top, 32));
+    const float f = mx[g] == -INFINITY ? 0.f : __expf(mx[g] - top);
+    float a = l[g] * f;
+    a += __shfl_xor(a, 16);
+    a += __shfl_xor(a, 32);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) acc[g * PER + i] *= f;
+    if (lane == 0) { mw[wave][g] = top; lw[wave][g] = a; }
+  }
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i]), __float_as_uint(acc[i + N / 2]), false, false);
+    acc[i] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) {
+    const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i]), __float_as_uint(acc[i + N / 4]), false, false);
+    const int at = i + N / 4 * (row4 >> 1) + N / 2 * (row4 & 1);
+    part[wave][at / PER * HD + sub * PER + at % PER] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+  }
+  __syncthreads();
+  // ---- the waves' results meet in LDS; they are the row's (one split) or leave as the split's ----
+  float* base = partial + ((int64_t)m * n_q + kvh * G) * S_max * (HD + 2);
+  auto put = [&](int g, int d, float lt, float at) {
+    float val;
+    if (lt > 0.f) {
+      val = at / lt;
+    } else {                                             // no attended key: uniform over the row's keys (see attn_decode_combine_kernel)
+      const float* Vd = fz.kv_cache_w + ((seq * 2 + 1) * n_kv + kvh) * t_max * HD + d;
+      const float* vp = fz.qkv + (int64_t)m * fz.ldqkv + (int64_t)(n_q + n_kv + kvh) * HD + d;
+      float sum = 0.f;
+      for (int j = 0; j < len; ++j) {
+        float y = 0.f;
+        if (j == slot) for (int z = 0; z < fz.nz; ++z) y += vp[(int64_t)z * fz.slab];      // (the arena's line of it may be another split's to write)
+        else y = Vd[(int64_t)j * HD];
+        sum += y;
+      }
+      val = len > 0 ? sum / (float)len : 0.f;
+    }
+    const int64_t o = ((int64_t)m * n_q + kvh * G + g) * HD + d;
+    if (out) out[o] = val;
+    if (split) {
+      const bf16_t hi = f32_to_bf16(val);
+      split[o] = hi;
+      split[(int64_t)fz.M * n_q * HD + o] = f32_to_bf16(val - bf16_to_f32(hi));
+    }
+  };
+  for (int t = tid; t < G * HD; t += TH) {
+    const int g = t / HD, d = t % HD;
+    float top = -INFINITY, lt = 0.f, at = 0.f;
+#pragma unroll
+    for (int r = 0; r < NW; ++r) top = fmaxf(top, mw[r][g]);
+#pragma unroll
+    for (int r = 0; r < NW; ++r) {
+      const float f = mw[r][g] == -INFINITY ? 0.f : __expf(mw[r][g] - top);
+      lt = fmaf(f, lw[r][g], lt);
+      at = fmaf(f, part[r][t], at);
+    }
+    if (S == 1) {
+      put(g, d, lt, at);
+      continue;
+    }
+    float* o = base + ((int64_t)g * S_max + s) * (HD + 2);
+    __hip_atomic_store(o + d, at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (d == 0) {
+      __hip_atomic_store(o + HD, top, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(o + HD + 1, lt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (S == 1) return;                                    // uniform
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  uint32_t* cnt = arrived + (int64_t)m * n_kv + kvh;
+  if (tid == 0) last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)S - 1;
+  __syncthreads();
+  if (!last) return;
+  if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int t = tid; t < G * HD; t += TH) {               // (whole waves of one head; S <= 64: lane z holds split z's statistics)
+    const int g = t / HD, d = t % HD;
+    const float* p = base + (int64_t)g * S_max * (HD + 2);
+    auto ld = [&](int z, int i) { return __hip_atomic_load(p + (int64_t)z * (HD + 2) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    float ms = -INFINITY, ls = 0.f, x[16], a = 0.f;
+    if (lane < S) { ms = ld(lane, HD); ls = ld(lane, HD + 1); }
+#pragma unroll
+    for (int z = 0; z < 16; ++z) x[z] = z < S ? ld(z, d) : 0.f;
+    const float top = wave_max(ms), f = ms == -INFINITY ? 0.f : __expf(ms - top), lt = wave_sum(f * ls);
+#pragma unroll
+    for (int z = 0; z < 16; ++z) a = fmaf(lane_f(f, z), x[z], a);
+    for (int z0 = 16; z0 < S; z0 += 16) {
+#pragma unroll
+      for (int z = 0; z < 16; ++z) x[z] = z0 + z < S ? ld(z0 + z, d) : 0.f;
+#pragma unroll
+      for (int z = 0; z < 16; ++z) a = fmaf(lane_f(f, (z0 + z) & 63), x[z], a);
+    }
+    put(g, d, lt, a);
   }
 }
 
@@ -896,21 +1047,17 @@ extern "C" size_t mn_attn_decode_workspace_bytes(int M, int n_q, int hd, int64_t
   return (size_t)M * n_q * attn_splits(M, n_q, t_max) * (hd + 2) * sizeof(float);
 }
 
-static int attn_decode_launch(const float* q, const AttnFuse* fz, int M, int n_q, int n_kv, int hd, const float* kv_cache, int64_t t_max,
+static int attn_decode_launch(const float* q, int M, int n_q, int n_kv, int hd, const float* kv_cache, int64_t t_max,
                               const int32_t* row_seq, const int32_t* row_len, const uint8_t* key_mask, int64_t ld_mask, float* out,
                               uint16_t* split, void* workspace, size_t workspace_bytes, void* stream) {
   hipStream_t st0 = mn_stream(stream);
   if (attn_use_one(M, t_max)) {                 // a few rows, short caches: one launch, the key split lives inside the workgroup
     int cc = (int)mn_cdiv(t_max, 16);
     cc = (cc + 3) & ~3;
-    const size_t lds1 = ((size_t)16 * cc + 16 * (hd + 2) + 3 * hd) * sizeof(float);
-    const AttnFuse nf{};
-    const AttnFuse& fa = fz ? *fz : nf;
+    const size_t lds1 = ((size_t)16 * cc + 16 * (hd + 2)) * sizeof(float);
     const dim3 g1(M, n_q), b1(1024);
-#define MN_ONE(HD_, F_) hipLaunchKernelGGL((attn_decode_one_kernel<HD_, F_>), g1, b1, lds1, st0, q, n_q, n_kv, kv_cache, t_max, row_seq, row_len, \
-                                           key_mask, ld_mask, cc, out, split, M, fa)
-    if (hd == 128) { if (fz) MN_ONE(128, true); else MN_ONE(128, false); }
-    else           { if (fz) MN_ONE(64, true); else MN_ONE(64, false); }
+#define MN_ONE(HD_) hipLaunchKernelGGL(attn_decode_one_kernel<HD_>, g1, b1, lds1, st0, q, n_q, n_kv, kv_cache, t_max, row_seq, row_len, key_mask, ld_mask, cc, out, split, M)
+    if (hd == 128) MN_ONE(128); else MN_ONE(64);
 #undef MN_ONE
     MN_CHECK_LAUNCH("mn_attn_decode(one launch)");
     return MN_OK;
@@ -924,23 +1071,15 @@ static int attn_decode_launch(const float* q, const AttnFuse* fz, int M, int n_q
   float* partial = reinterpret_cast<float*>(workspace);
   dim3 grid(M, (n_q + 3) / 4, S);
   hipStream_t st = mn_stream(stream);
-  const AttnFuse none{};
-  if (fz) {
-    if (hd == 128)
-      hipLaunchKernelGGL((attn_decode_split_kernel<128, true>), grid, dim3(256), lds, st, q, n_q, n_kv, kv_cache, t_max, row_seq, row_len,
-                         key_mask, ld_mask, S, chunk_cap, partial, *fz);
-    else
-      hipLaunchKernelGGL((attn_decode_split_kernel<64, true>), grid, dim3(256), lds, st, q, n_q, n_kv, kv_cache, t_max, row_seq, row_len,
-                         key_mask, ld_mask, S, chunk_cap, partial, *fz);
-  } else if (attn_use_gqa(M, n_q, n_kv, hd)) {
+  if (attn_use_gqa(M, n_q, n_kv, hd)) {
     hipLaunchKernelGGL((attn_decode_gqa_kernel<128, 4>), dim3(M, (n_kv + 3) / 4, S), dim3(256), lds * 4, st, q, n_q, n_kv, kv_cache,
                        t_max, row_seq, row_len, key_mask, ld_mask, S, chunk_cap, partial);
   } else if (hd == 128) {
-    hipLaunchKernelGGL((attn_decode_split_kernel<128, false>), grid, dim3(256), lds, st, q, n_q, n_kv, kv_cache, t_max, row_seq,
-                       row_len, key_mask, ld_mask, S, chunk_cap, partial, none);
+    hipLaunchKernelGGL(attn_decode_split_kernel<128>, grid, dim3(256), lds, st, q, n_q, n_kv, kv_cache, t_max, row_seq,
+                       row_len, key_mask, ld_mask, S, chunk_cap, partial);
   } else {
-    hipLaunchKernelGGL((attn_decode_split_kernel<64, false>), grid, dim3(256), lds, st, q, n_q, n_kv, kv_cache, t_max, row_seq,
-                       row_len, key_mask, ld_mask, S, chunk_cap, partial, none);
+    hipLaunchKernelGGL(attn_decode_split_kernel<64>, grid, dim3(256), lds, st, q, n_q, n_kv, kv_cache, t_max, row_seq,
+                       row_len, key_mask, ld_mask, S, chunk_cap, partial);
   }
   if (hd == 128)
     hipLaunchKernelGGL(attn_decode_combine_kernel<128>, dim3(M, n_q), dim3(128), 0, st, partial, n_q, S, out, split, M, kv_cache, n_kv, t_max,
@@ -959,41 +1098,75 @@ extern "C" int mn_attn_decode_split(const float* q, int M, int n_q, int n_kv, in
                                     size_t workspace_bytes, void* stream) {
   MN_CHECK_ARG(M >= 1 && n_q >= 1 && n_kv >= 1 && n_q % n_kv == 0 && (hd == 64 || hd == 128), "mn_attn_decode: bad shape");
   MN_CHECK_ARG(q && kv_cache && row_seq && row_len && (out || split) && workspace, "mn_attn_decode: null pointer");
-  return attn_decode_launch(q, nullptr, M, n_q, n_kv, hd, kv_cache, t_max, row_seq, row_len, key_mask, ld_mask, out, split, workspace,
+  return attn_decode_launch(q, M, n_q, n_kv, hd, kv_cache, t_max, row_seq, row_len, key_mask, ld_mask, out, split, workspace,
                             workspace_bytes, stream);
 }
 
-// Internal (engine.hip): RoPE + q scale + KV append + masked decode attention in ONE split launch (+ the combine) from the raw QKV
-// projection (optionally as nz K-slice partial slabs): what mn_rope_kv_append_3d / mn_rope_kv_from_partials followed by
-// mn_attn_decode_split compute, one launch fewer per layer and step and no q round trip.  Needs row_len == row_slot + 1, the
-// one-launch form or one row, and n_q / n_kv in {1, 2, 4}; mn_attn_fused_ok says whether a shape qualifies.
-// Where the append rides the attention launch (tools/exp/attn_fused_ab.py, profiles/r04_attn_fused_ab.txt): always in the one-launch form
-// (every row count it serves gains 1-2 %: each workgroup keeps the new key in LDS, no hazard, no redundant reads worth counting); in
-// the split form at ONE row only (2.00 -> 1.92 ms per 28-layer step; from 2 rows on every split re-reduces the QKV slabs: 2.59 -> 2.74).
+// Internal (engine.hip): RoPE + q scale + KV append + masked decode attention in ONE launch from the raw QKV projection (optionally as nz K-slice partial slabs): what
+// mn_rope_kv_append_3d / mn_rope_kv_from_partials followed by mn_attn_decode_split compute.  Rows of distinct sequences with row_len == row_slot + 1; n_q / n_kv in {1, 2, 4}.
+// Splits of a row: as many as make one round of the CUs with the other rows, 16 at most; arrived: mn_attn_arrivals' counters, zero (they are left zero), or NULL for one split a row.
+// us a launch over 24 layers' caches, the launches before (one workgroup a head up to 16 rows over 1024 keys; else the append, a launch of 32 splits and one that joins them; from
+// 40 (row, key head) pairs on a wave a key head) / this one.  16 heads of 128 over 4: 1 row of 80 keys 6.5 / 6.4, 330 13.1 / 7.7, 1100 13.0 / 9.7, 1900 16.9 / 9.9; 4 rows 7.1 / 7.5,
+// 13.3 / 8.9, 19.7 / 14.3, 27.0 / 15.7; 10 rows 7.7 / 7.6, 18.0 / 11.0, 25.7 / 16.4, 35.7 / 21.4; 36 rows 18.9 / 10.1, 22.8 / 18.0, 43.5 / 37.4, 64 / 57; 64 rows 19.6 / 11.3, 27.2 / 22.8,
+// 69.6 / 55.5 (5.2 TB/s), 110 / 89; 200 rows 26.7 / 23.1, 66 / 60, 192 / 169; 1536 rows of 80 147 / 127.  16 heads of 64: 1 row of 40 keys 4.4 / 3.3, 250 6.9 / 5.8, 600 10.7 / 7.1;
+// 16 rows 5.9 / 4.7, 11.2 / 10.1, 19.3 / 18.4; 64 rows 16.8 / 9.6, 37.3 / 27.3, 71 / 58.
 static int g_attn_fuse = 1;                          // dev-library A/B switch: 0 = never fused
 #ifdef MN_DEV_HOOKS
 extern "C" MN_DEV_API void mn_attn_tune_fuse(int on) { g_attn_fuse = on; }
 #endif
-extern "C" int mn_attn_fused_ok(int M, int n_q, int n_kv, int hd, int64_t t_max) {
+extern "C" int mn_attn_fused_ok(int M, int n_q, int n_kv, int hd) {
   if (g_kv_round_bf16 || !g_attn_fuse) return 0;     // the bf16-KV measurement hook lives in the stand-alone append kernel
-  if (!attn_use_one(M, t_max) && M > 1) return 0;
   const int ratio = n_kv > 0 && n_q % n_kv == 0 ? n_q / n_kv : 0;
   return M >= 1 && (hd == 64 || hd == 128) && (ratio == 1 || ratio == 2 || ratio == 4);
+}
+// a split of 64 KB of K and V: what a workgroup asks for at once
+static int attn_join_keys(int hd) { return 64 * 128 / hd; }
+static int attn_join_splits(int M, int n_kv, int hd, int64_t t_max) {
+  const int64_t most = mn_cdiv(t_max, attn_join_keys(hd)), fill = mn_num_cus() / ((int64_t)M * n_kv);
+  const int64_t s = most < fill ? most : fill;
+  return s < 1 ? 1 : (s > 16 ? 16 : (int)s);
+}
+// The arrival counters of mn_attn_decode_fused, behind the partials in the scratch that mn_attn_decode_workspace_bytes sizes (its 32 splits of 32 keys are more than these): [M][n_kv],
+// to be zeroed once before a step's first layer (*n words); NULL: one split a row, which needs none.
+extern "C" uint32_t* mn_attn_arrivals(int M, int n_q, int n_kv, int hd, int64_t t_max, void* workspace, size_t workspace_bytes, int* n) {
+  const int S = attn_join_splits(M, n_kv, hd, t_max);
+  const size_t part = (size_t)M * n_q * S * (hd + 2) * sizeof(float), need = part + (size_t)M * n_kv * sizeof(uint32_t);
+  *n = 0;
+  if (S == 1 || !workspace || need > workspace_bytes) return nullptr;
+  *n = M * n_kv;
+  return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(workspace) + part);
 }
 extern "C" int mn_attn_decode_fused(const float* qkv, int64_t ldqkv, int nz, int64_t slab, int M, int n_q, int n_kv, int hd, int rope,
                                     const float* cos_tab, const float* sin_tab, const int32_t* row_seq, const int32_t* row_slot,
                                     const int32_t* row_pos, int sec_t, int sec_h, float q_scale, float* kv_cache, int64_t t_max,
                                     const int32_t* row_len, const uint8_t* key_mask, int64_t ld_mask, float* out, uint16_t* split,
-                                    void* workspace, size_t workspace_bytes, void* stream) {
-  MN_CHECK_ARG(mn_attn_fused_ok(M, n_q, n_kv, hd, t_max) && nz >= 1, "mn_attn_decode_fused: unsupported shape");
-  MN_CHECK_ARG(qkv && kv_cache && row_seq && row_slot && row_len && (out || split) && workspace, "mn_attn_decode_fused: null pointer");
+                                    void* workspace, uint32_t* arrived, void* stream) {
+  MN_CHECK_ARG(mn_attn_fused_ok(M, n_q, n_kv, hd) && nz >= 1, "mn_attn_decode_fused: unsupported shape");
+  MN_CHECK_ARG(qkv && kv_cache && row_seq && row_slot && row_len && (out || split) && (workspace || !arrived), "mn_attn_decode_fused: null pointer");
   MN_CHECK_ARG(!rope || (cos_tab && sin_tab && row_pos), "mn_attn_decode_fused: rope needs tables and positions");
   MN_CHECK_ARG(sec_t >= 0 && sec_h >= 0 && sec_t + sec_h <= hd / 2, "mn_attn_decode_fused: bad rotary sections %d/%d", sec_t, sec_h);
   AttnFuse fz;
   fz.qkv = qkv; fz.ldqkv = ldqkv; fz.nz = nz; fz.slab = slab; fz.rope = rope; fz.cos_tab = cos_tab; fz.sin_tab = sin_tab;
   fz.row_slot = row_slot; fz.row_pos = row_pos; fz.sec_t = sec_t; fz.sec_h = sec_h; fz.q_scale = q_scale; fz.M = M; fz.kv_cache_w = kv_cache;
-  return attn_decode_launch(nullptr, &fz, M, n_q, n_kv, hd, kv_cache, t_max, row_seq, row_len, key_mask, ld_mask, out, split, workspace,
-                            workspace_bytes, stream);
+  const int S = arrived ? attn_join_splits(M, n_kv, hd, t_max) : 1, keys = attn_join_keys(hd);
+  const int64_t pairs = (int64_t)M * n_kv, cu = mn_num_cus();
+  float* partial = reinterpret_cast<float*>(workspace);
+  const dim3 grid(M, n_kv, S);
+  hipStream_t st = mn_stream(stream);
+#define MN_JOIN(HD_, G_, NW_, U_, W_) hipLaunchKernelGGL((attn_decode_join_kernel<HD_, G_, NW_, U_, W_>), grid, dim3(NW_ * 64), 0, st, n_q, n_kv, t_max, row_seq, row_len, key_mask, \
+                                                         ld_mask, S, keys, partial, arrived, out, split, fz)
+  // from a workgroup a CU on: with one key a group in flight two of them fit a CU (1536 rows of 80 keys 195 -> 127 us, 64 rows 57 -> 55.5; 36 rows 37.4 -> 47); heads of 64, from four a
+  // CU on: four waves each (64 rows of 40 keys 10.7 -> 9.6 us; 32 rows 9.9 -> 10.4)
+#define MN_JOIN_HD128(G_) do { if (pairs >= cu) MN_JOIN(128, G_, 8, 1, 4); else MN_JOIN(128, G_, 8, 2, 2); } while (0)
+#define MN_JOIN_HD64(G_) do { if (pairs >= 4 * cu) MN_JOIN(64, G_, 4, 2, 4); else MN_JOIN(64, G_, 8, 2, 2); } while (0)
+  const int ratio = n_q / n_kv;
+  if (hd == 128) { if (ratio == 4) MN_JOIN_HD128(4); else if (ratio == 2) MN_JOIN_HD128(2); else MN_JOIN_HD128(1); }
+  else           { if (ratio == 4) MN_JOIN_HD64(4); else if (ratio == 2) MN_JOIN_HD64(2); else MN_JOIN_HD64(1); }
+#undef MN_JOIN_HD128
+#undef MN_JOIN_HD64
+#undef MN_JOIN
+  MN_CHECK_LAUNCH("mn_attn_decode_fused");
+  return MN_OK;
 }
 
 extern "C" int mn_attn_decode(const float* q, int M, int n_q, int n_kv, int hd, const float* kv_cache,

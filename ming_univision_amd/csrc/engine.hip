@@ -24,14 +24,15 @@ extern "C" int mn_rope_kv_from_partials(const float* qkv, int64_t ldqkv, int nz,
 extern "C" int mn_attn_decode_split(const float* q, int M, int n_q, int n_kv, int hd, const float* kv_cache, int64_t t_max,
                                     const int32_t* row_seq, const int32_t* row_len, const uint8_t* key_mask, int64_t ld_mask,
                                     float* out, uint16_t* split, void* workspace, size_t workspace_bytes, void* stream);
-extern "C" int mn_attn_fused_ok(int M, int n_q, int n_kv, int hd, int64_t t_max);
+extern "C" int mn_attn_fused_ok(int M, int n_q, int n_kv, int hd);
+extern "C" uint32_t* mn_attn_arrivals(int M, int n_q, int n_kv, int hd, int64_t t_max, void* workspace, size_t workspace_bytes, int* n);
 extern "C" int mn_flash_prefill_gqa_hd128_f32(const float* q, const float* kv_layer, int64_t t_max, int n_q, int n_kv, const int32_t* span_tab,
                                               int n_spans, int max_len, float* out, uint16_t* split, int64_t split_lo_off, void* stream);
 extern "C" int mn_attn_decode_fused(const float* qkv, int64_t ldqkv, int nz, int64_t slab, int M, int n_q, int n_kv, int hd, int rope,
                                     const float* cos_tab, const float* sin_tab, const int32_t* row_seq, const int32_t* row_slot,
                                     const int32_t* row_pos, int sec_t, int sec_h, float q_scale, float* kv_cache, int64_t t_max,
                                     const int32_t* row_len, const uint8_t* key_mask, int64_t ld_mask, float* out, uint16_t* split,
-                                    void* workspace, size_t workspace_bytes, void* stream);
+                                    void* workspace, uint32_t* arrived, void* stream);
 extern "C" int mn_stream_mfma_grouped(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P,
                                       int p_rows, const int32_t* off, const int32_t* xrows, int G, int max_rows,
                                       int Ntot, int K, void* stream);
@@ -431,10 +432,17 @@ __global__ __launch_bounds__(1024) void rf_step_boundary_kernel(
 
 // semantic decoder input: de-normalise, Linear(in_dim -> D) + channel-repeat shortcut
 // (modeling_mingtok.py:168; vision_transformer.py:373-380)
+// (zero: n_zero words that the step's attention launches count arrivals in, here and in the two other kernels that start a step)
+__device__ __forceinline__ void zero_words(uint32_t* zero, int n_zero) {
+  if (blockIdx.x == 0 && blockIdx.y == 0)
+    for (int i = threadIdx.x; i < n_zero; i += blockDim.x) zero[i] = 0u;
+}
+
 __global__ void semdec_in_kernel(const float* __restrict__ latent, int in_dim, float scale, float mean,
                                  const bf16_t* __restrict__ w, const bf16_t* __restrict__ b, float* __restrict__ out,
-                                 int D) {
+                                 int D, uint32_t* __restrict__ zero, int n_zero) {
   const int m = blockIdx.y, n = blockIdx.x * blockDim.x + threadIdx.x;
+  zero_words(zero, n_zero);
   if (n >= D) return;
   const float* lr = latent + (int64_t)m * in_dim;
   float acc = bf16_to_f32(b[n]);
@@ -456,7 +464,8 @@ __global__ void rf_gather_latent_kernel(const float* __restrict__ x, float* __re
 
 // rows copy: b[m] = a[(m / row_div) * lda]  (lda == 0 broadcasts one row; row_div > 1 shares one source row
 // between the CFG rows of an image)
-__global__ void copy_rows_f32_kernel(const float* __restrict__ a, int64_t lda, int row_div, float* __restrict__ b, int M, int D) {
+__global__ void copy_rows_f32_kernel(const float* __restrict__ a, int64_t lda, int row_div, float* __restrict__ b, int M, int D, uint32_t* __restrict__ zero, int n_zero) {
+  zero_words(zero, n_zero);
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < (int64_t)M * D) b[i] = a[((i / D) / row_div) * lda + (i % D)];
 }
@@ -883,12 +892,13 @@ __global__ __launch_bounds__(1024) void llm_glue_kernel(int mode, const float* _
                                                         const int32_t* __restrict__ pair_pos, const float* __restrict__ tw,
                                                         int n_slot, float* __restrict__ h, int M, int H,
                                                         const bf16_t* __restrict__ norm_w, float eps,
-                                                        float* __restrict__ xn_out, bf16_t* __restrict__ Y) {
+                                                        float* __restrict__ xn_out, bf16_t* __restrict__ Y, uint32_t* __restrict__ zero, int n_zero) {
   __shared__ float red[32];
   typedef float f4 __attribute__((ext_vector_type(4)));
   typedef uint32_t u2 __attribute__((ext_vector_type(2)));
   const int m = blockIdx.x, col = threadIdx.x * 4;
   const bool act = col < H;
+  zero_words(zero, n_zero);
   f4 v = {0.f, 0.f, 0.f, 0.f};
   u2 nw2 = {0u, 0u};                               // the norm weights of this thread's columns, requested with the row (not behind the barrier)
   if (act && norm_w) nw2 = *reinterpret_cast<const u2*>(norm_w + col);
@@ -1200,7 +1210,7 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
                "mn_llm_step: quantised experts need scale tables, widths %% 16 == 0 (NF4: %% 64) and <= 64 rows or the wide route's shapes (M = %d)", M);
   if (llm_wide_ok(m, M))
     return llm_step_wide(m, x, ldx, x_row_div, M, image_mask, row_seq, row_slot, row_pos, row_len, key_mask, ld_mask, kv_cache, n_seq, t_max,
-                         hidden_out, workspace, workspace_bytes, stream, span_tab, n_spans, span_max_len);
+                         hidden_out, workspace, workspace_bytes, flags, stream, span_tab, n_spans, span_max_len);
   LlmWs w{};
   const size_t need = llm_carve(m, M, t_max, workspace, workspace_bytes, &w);
   if (need > workspace_bytes) { mn_set_error("mn_llm_step: workspace %zu < %zu", workspace_bytes, need); return MN_ENOSPACE; }
@@ -1212,7 +1222,9 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
   t_sk_ws = w.sk_ws; t_sk_ws_bytes = w.sk_ws_bytes;
   // rows of DISTINCT cache sequences (decode steps; not a prefill chunk, whose rows read each other's new K / V lines): RoPE + KV
   // append ride the attention launch
-  const bool fuse_attn = (flags & MN_STEP_DISTINCT_SEQUENCES) && mn_attn_fused_ok(M, nq, nkv, hd, t_max);
+  const bool fuse_attn = (flags & MN_STEP_DISTINCT_SEQUENCES) && mn_attn_fused_ok(M, nq, nkv, hd);
+  int n_zero = 0;
+  uint32_t* arrived = fuse_attn ? mn_attn_arrivals(M, nq, nkv, hd, t_max, w.attn_ws, w.attn_ws_bytes, &n_zero) : nullptr;
   if (llm_chain_ok(m, M) && !(image_mask && m->image_gate)) {
     // ---- chain path: 11 launches per layer instead of 18 (2 rows: 6 — QKV with the RMSNorm prologue, attention with RoPE + KV append, dense,
     // the one-launch router, the expert pairs' gate/up, the down projection into h).  glue = llm_glue_kernel.
@@ -1232,11 +1244,11 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
       if (l == 0)
         hipLaunchKernelGGL(llm_glue_kernel, dim3(M), dim3(gt), 0, st, 0, x, ldx, x_row_div, (const float*)nullptr, 0, (int64_t)0,
                            (const int32_t*)nullptr, (const float*)nullptr, n_slot, w.h, M, H, m->ln1[l], m->rms_eps,
-                           (float*)nullptr, w.yh);
+                           (float*)nullptr, w.yh, arrived, n_zero);
       else if (!(ln1_fused = !grouped && g_chain_fuse_ln1 && stream_rmsnorm_ok(M, qkv_dim, H)))
         hipLaunchKernelGGL(llm_glue_kernel, dim3(M), dim3(gt), 0, st, grouped ? 2 : 3, (const float*)nullptr, (int64_t)0, 1,
                            (const float*)w.moe.p2, nz2, (int64_t)P * H, (const int32_t*)w.moe.pair_pos, (const float*)w.tw,
-                           n_slot, w.h, M, H, m->ln1[l], m->rms_eps, (float*)nullptr, w.yh);
+                           n_slot, w.h, M, H, m->ln1[l], m->rms_eps, (float*)nullptr, w.yh, (uint32_t*)nullptr, 0);
       // QKV launch -> partials; RoPE + KV append reduce them  (:743-789).  With the experts already summed into h (2-4 rows) the
       // launch normalises h itself (stream_mfma.hip FUSE_RMSNORM: the glue launch's arithmetic in every workgroup's staging pass)
       int nz = ln1_fused ? stream_rmsnorm(m->wqkv[l], w.pp, M, qkv_dim, H, w.h, m->ln1[l], m->rms_eps, stream)
@@ -1245,7 +1257,7 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
       if (fuse_attn) {
         MN_TRY(mn_attn_decode_fused(w.pp, qkv_dim, nz, (int64_t)M * qkv_dim, M, nq, nkv, hd, 1, m->cos_tab, m->sin_tab, row_seq, row_slot,
                                     row_pos, m->mrope_sec_t, m->mrope_sec_h, q_scale, kv_l, t_max, row_len, key_mask, ld_mask, nullptr,
-                                    w.ya, w.attn_ws, w.attn_ws_bytes, stream));
+                                    w.ya, w.attn_ws, arrived, stream));
       } else {
         MN_TRY(mn_rope_kv_from_partials(w.pp, qkv_dim, nz, (int64_t)M * qkv_dim, M, nq, nkv, hd, 1, m->cos_tab, m->sin_tab,
                                         row_seq, row_slot, row_pos, m->mrope_sec_t, m->mrope_sec_h, q_scale, w.q, kv_l, t_max,
@@ -1306,11 +1318,11 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
     // last experts' combine + residual -> final RMSNorm -> hidden_out
     hipLaunchKernelGGL(llm_glue_kernel, dim3(M), dim3(gt), 0, st, grouped ? 2 : 3, (const float*)nullptr, (int64_t)0, 1,
                        (const float*)w.moe.p2, nz2, (int64_t)P * H, (const int32_t*)w.moe.pair_pos, (const float*)w.tw, n_slot,
-                       w.h, M, H, m->final_norm, m->rms_eps, hidden_out, (bf16_t*)nullptr);
+                       w.h, M, H, m->final_norm, m->rms_eps, hidden_out, (bf16_t*)nullptr, (uint32_t*)nullptr, 0);
     MN_CHECK_LAUNCH("mn_llm_step");
     return MN_OK;
   }
-  hipLaunchKernelGGL(copy_rows_f32_kernel, dim3(mn_cdiv((int64_t)M * H, 256)), dim3(256), 0, st, x, ldx, x_row_div, w.h, M, H);
+  hipLaunchKernelGGL(copy_rows_f32_kernel, dim3(mn_cdiv((int64_t)M * H, 256)), dim3(256), 0, st, x, ldx, x_row_div, w.h, M, H, arrived, n_zero);
   for (int l = 0; l < m->n_layers; ++l) {
     float* kv_l = kv_cache + (int64_t)l * layer_kv;
     // attention: RMSNorm -> QKV -> RoPE/KV append -> masked GQA -> dense + residual  (:1204-1215, :743-829)
@@ -1320,7 +1332,7 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
     if (fuse_attn) {
       MN_TRY(mn_attn_decode_fused(w.qkv, qkv_dim, 1, 0, M, nq, nkv, hd, 1, m->cos_tab, m->sin_tab, row_seq, row_slot, row_pos,
                                   m->mrope_sec_t, m->mrope_sec_h, q_scale, kv_l, t_max, row_len, key_mask, ld_mask, w.attn, nullptr,
-                                  w.attn_ws, w.attn_ws_bytes, stream));
+                                  w.attn_ws, arrived, stream));
     } else {
       MN_TRY(mn_rope_kv_append_3d(w.qkv, qkv_dim, M, nq, nkv, hd, 1, m->cos_tab, m->sin_tab, row_seq, row_slot, row_pos,
                                   m->mrope_sec_t, m->mrope_sec_h, q_scale, w.q, kv_l, t_max, stream));
@@ -1439,16 +1451,20 @@ extern "C" int mn_semdec_step(const mn_semdec* s, const float* latent_norm, int 
   const int D = s->dim, nh = s->n_heads;
   const int64_t layer_kv = (int64_t)n_seq * 2 * nh * t_max * 64;
   t_sk_ws = w.sk_ws; t_sk_ws_bytes = w.sk_ws_bytes;
+  // (more than 16 rows may share a sequence, as its rows in a chunk do: their append is a launch before)
+  const bool fuse_attn = ((M <= 16 && t_max <= 1024) || M == 1) && mn_attn_fused_ok(M, nh, nh, 64);
+  int n_zero = 0;
+  uint32_t* arrived = fuse_attn ? mn_attn_arrivals(M, nh, nh, 64, t_max, w.attn_ws, w.attn_ws_bytes, &n_zero) : nullptr;
   hipLaunchKernelGGL(semdec_in_kernel, dim3(mn_cdiv(D, 256), M), dim3(256), 0, st, latent_norm, s->in_dim, s->scale,
-                     s->mean, s->in_w, s->in_b, w.h, D);
+                     s->mean, s->in_w, s->in_b, w.h, D, arrived, n_zero);
   for (int l = 0; l < s->depth; ++l) {
     float* kv_l = kv_cache + (int64_t)l * layer_kv;
     mn_skinny_args a = sk(w.h, D, s->wqkv[l], D, s->bqkv[l], w.qkv, 3 * D, M, 3 * D, D);
     a.prologue = MN_PRO_LN; a.ln_g = s->ln1_g[l]; a.ln_b = s->ln1_b[l]; a.eps = 1e-6f;
     MN_TRY(mn_skinny_gemm(&a, stream));
-    if (mn_attn_fused_ok(M, nh, nh, 64, t_max)) {     // one row (batch 1): the K / V append rides the attention launch (see mn_llm_step_ex)
+    if (fuse_attn) {                                 // the K / V append rides the attention launch (see mn_llm_step_ex)
       MN_TRY(mn_attn_decode_fused(w.qkv, 3 * D, 1, 0, M, nh, nh, 64, 0, nullptr, nullptr, row_seq, row_slot, nullptr, 0, 0, 0.125f, kv_l,
-                                  t_max, row_len, nullptr, 0, w.attn, nullptr, w.attn_ws, w.attn_ws_bytes, stream));
+                                  t_max, row_len, nullptr, 0, w.attn, nullptr, w.attn_ws, arrived, stream));
     } else {
       MN_TRY(mn_rope_kv_append(w.qkv, 3 * D, M, nh, nh, 64, 0, nullptr, nullptr, row_seq, row_slot, nullptr, 0.125f,
                                w.q, kv_l, t_max, stream));

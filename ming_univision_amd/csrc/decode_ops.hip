@@ -84,6 +84,7 @@ __global__ __launch_bounds__(1024) void moe_router_row_kernel(
   const bool img = image_mask && image_gate_w && image_mask[m];
   const bf16_t* G = img ? image_gate_w : gate_w;
   typedef float f4 __attribute__((ext_vector_type(4)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
   float acc[4] = {0.f, 0.f, 0.f, 0.f};          // experts wave, wave + 16, wave + 32, wave + 48: four weight rows in flight per lane
   // H <= 2048 (the 16B-A3B width): this lane's 16 weight slots do not depend on x — requested FIRST, so the launch is one memory round
   // trip (x and the gate rows together) + the reductions, not two dependent ones
@@ -100,47 +101,55 @@ __global__ __launch_bounds__(1024) void moe_router_row_kernel(
       }
   }
   // P != NULL (the decoder chain, up to 64 rows): the row is h + the sum of the nz K-slice partial slabs of the attention output projection (the slabs first, in slab order, as
-  // llm_glue_kernel does), written back to h_out — the residual glue launch and the gate launch fold into this one
-  float xv[4], add[4] = {0.f, 0.f, 0.f, 0.f};     // H <= 4096: columns tid, tid + 1024, ...
+  // llm_glue_kernel does), written back to h_out — the residual glue launch and the gate launch fold into this one.  Two columns a thread, the norm's weights with them: all that
+  // the row needs is asked for before the first of it is waited for (sixteen slabs at once, one round trip).
+  f2 xv[2] = {{0.f, 0.f}, {0.f, 0.f}}, add[2] = {{0.f, 0.f}, {0.f, 0.f}};     // H <= 4096: columns 2 tid, 2 tid + 2048
+  uint32_t nw[2] = {0u, 0u};
   float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) xv[i] = tid + 1024 * i < H ? xr[tid + 1024 * i] : 0.f;
+  for (int i = 0; i < 2; ++i) {
+    const int k = 2 * tid + 2048 * i;
+    if (k >= H) continue;
+    xv[i] = f2{xr[k], xr[k + 1]};
+    nw[i] = (uint32_t)norm_w[k] | (uint32_t)norm_w[k + 1] << 16;
+  }
   if (P) {
-    const float* pp = P + (int64_t)m * H + tid;
-    for (int z0 = 0; z0 < nz; z0 += 8) {          // eight slabs of all columns in flight
-      float t[4][8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2; ++i) {
+      const int k = 2 * tid + 2048 * i;
+      if (k >= H) continue;
+      const float* pp = P + (int64_t)m * H + k;
+      for (int z0 = 0; z0 < nz; z0 += 16) {
+        f2 t[16];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) t[i][j] = z0 + j < nz && tid + 1024 * i < H ? pp[(int64_t)(z0 + j) * slab + 1024 * i] : 0.f;
+        for (int j = 0; j < 16; ++j) t[j] = z0 + j < nz ? *reinterpret_cast<const f2*>(pp + (int64_t)(z0 + j) * slab) : f2{0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) add[i] += t[i][j];
+        for (int j = 0; j < 16; ++j) add[i] += t[j];
+      }
     }
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = tid + 1024 * i;
+  for (int i = 0; i < 2; ++i) {
+    const int k = 2 * tid + 2048 * i;
     if (k >= H) continue;
     xv[i] += add[i];                              // (the small sum first: the stream is rounded once)
-    if (P) h_out[(int64_t)m * H + k] = xv[i];
-    ss += xv[i] * xv[i];
+    if (P) *reinterpret_cast<f2*>(h_out + (int64_t)m * H + k) = xv[i];
+    ss += xv[i].x * xv[i].x + xv[i].y * xv[i].y;
   }
   ss = block_sum(ss, red);
   const float rstd = rsqrtf(ss / (float)H + eps);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = tid + 1024 * i;
-    if (k < H) {
-      const float v = xv[i] * rstd * bf16_to_f32(norm_w[k]);
-      xs[k] = v;
-      if (x_norm) x_norm[(int64_t)m * H + k] = v;
-      if (Y) {                                    // the grouped experts' operand: hi rows, then lo rows
-        const bf16_t hi = f32_to_bf16(v);
-        Y[(int64_t)m * H + k] = hi;
-        Y[(int64_t)(M + m) * H + k] = f32_to_bf16(v - bf16_to_f32(hi));
-      }
+  for (int i = 0; i < 2; ++i) {
+    const int k = 2 * tid + 2048 * i;
+    if (k >= H) continue;
+    const f2 v = f2{xv[i].x * rstd * bf16lo_to_f32(nw[i]), xv[i].y * rstd * bf16hi_to_f32(nw[i])};
+    *reinterpret_cast<f2*>(&xs[k]) = v;
+    if (x_norm) *reinterpret_cast<f2*>(x_norm + (int64_t)m * H + k) = v;
+    if (Y) {                                      // the grouped experts' operand: hi rows, then lo rows
+      uint32_t hi, lo;
+      split_pk_bf16(v.x, v.y, hi, lo);
+      *reinterpret_cast<uint32_t*>(Y + (int64_t)m * H + k) = hi;
+      *reinterpret_cast<uint32_t*>(Y + (int64_t)(M + m) * H + k) = lo;
     }
   }
   __syncthreads();
@@ -218,8 +227,8 @@ extern "C" MN_DEV_API void mn_moe_router_tune(int max_rows) { g_router_rows = ma
 #endif
 
 // The decoder chain's form (engine.hip): h[m] += sum of the nz partial slabs P [nz][M][H]; RMSNorm -> x_norm and / or Y (bf16 hi rows, lo rows); gate;
-// top-k — one launch.  A row is a workgroup, which reads the gate (256 KB at 64 x 2048) from its XCD's L2: 12.9 us at 64 rows, where the norm, the gate's product
-// and a one-workgroup top-k and sort took 6 + 5 + 13.
+// top-k — one launch.  A row is a workgroup, which reads the gate (256 KB at 64 x 2048) and its slabs (131 KB) from its XCD's L2: 10.7 us at 64 rows (11.8 with eight slabs a round
+// trip and the norm's weights behind the sum; 2 rows 11.0 -> 9.9), where the norm, the gate's product and a one-workgroup top-k and sort took 6 + 5 + 13.
 bool moe_router_rows_ok(int M, int H, int E) { return M >= 1 && M <= 64 && H <= 4096 && (H % 8) == 0 && E <= 64; }
 int moe_router_rows(float* h, const float* P, int nz, const uint16_t* norm_w, float eps, const uint16_t* gate_w, int M, int H, int E, int top_k,
                     int norm_topk_prob, int n_shared_slots, float* x_norm, uint16_t* y, int32_t* topk_idx, float* topk_w, float* logits_ws, void* stream) {

@@ -16,7 +16,9 @@
 extern "C" size_t mn_attn_decode_workspace_bytes(int M, int n_q, int hd, int64_t t_max);
 extern "C" int mn_stream_mfma(const uint16_t* Y, const uint16_t* W, float* P, int M, int Ntot, int K, void* stream);
 extern "C" int mn_stream_mfma_slices(int M, int Ntot, int K);
-extern "C" int mn_stream_mfma_grouped_slices(int G, int max_rows, int Ntot, int K);
+extern "C" int mn_stream_kwalk_slices(int max_rows, int K);
+extern "C" int mn_stream_kwalk_grouped(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G,
+                                       int max_rows, int Ntot, int K, void* stream);
 extern "C" int mn_rope_kv_from_partials(const float* qkv, int64_t ldqkv, int nz, int64_t slab, int M, int n_q, int n_kv, int hd,
                                         int rope, const float* cos_tab, const float* sin_tab, const int32_t* row_seq,
                                         const int32_t* row_slot, const int32_t* row_pos, int sec_t, int sec_h, float q_scale,
@@ -60,8 +62,8 @@ static inline int stream_grouped(int wfmt, const uint16_t* Y, int y_rows, const 
                                  void* stream) {
   return wfmt ? mn_stream_mfma_grouped_wq(Y, y_rows, reinterpret_cast<const uint8_t*>(W), w_stride, wscale,
                                           s_stride * mn_wq_scales_per_row(wfmt, K), P, p_rows, off, xrows, G, max_rows, Ntot, K, wfmt, stream)
-              : mn_stream_mfma_grouped(Y, y_rows, reinterpret_cast<const uint16_t*>(W), w_stride, P, p_rows, off, xrows, G, max_rows, Ntot,
-                                       K, stream);
+              : mn_stream_kwalk_grouped(Y, y_rows, reinterpret_cast<const uint16_t*>(W), w_stride, P, p_rows, off, xrows, G, max_rows, Ntot,
+                                        K, stream);
 }
 
 namespace {
@@ -989,8 +991,8 @@ static size_t moe_carve(Carver& cv, int rows, int H, int I, int G, int n_slot, M
   o->pair_pos = cv.take<int32_t>(P);
   o->y1 = cv.take<bf16_t>((size_t)2 * rows * H);
   o->y2 = cv.take<bf16_t>(2 * P * I);
-  o->p1 = cv.take<float>((size_t)mn_stream_mfma_grouped_slices(G, rows, 2 * I, H) * P * 2 * I);
-  o->p2 = cv.take<float>((size_t)mn_stream_mfma_grouped_slices(G, rows, H, I) * P * H);
+  o->p1 = cv.take<float>((size_t)mn_stream_kwalk_slices(rows, H) * P * 2 * I);
+  o->p2 = cv.take<float>((size_t)mn_stream_kwalk_slices(rows, I) * P * H);
   return cv.off - before;
 }
 

@@ -285,6 +285,123 @@ __global__ __launch_bounds__(KW * 64, (WQ == 1 && MT == 4 && NT == 2) ? 4 : 1) v
   }
 }
 
+// ---- the walk of bf16 groups ---------------------------------------------------------------------------------------------------
+// In the grid form above a workgroup is a column tile and a K-range of a group, two fit a CU, and a round of them that is not full costs a whole one: 66 experts of 2048 x 1408
+// in two ranges are 1056 workgroups on 512 places and stream at 4.9 TB/s, of 5632 x 2048 1452 and 5.8.  Here a resident set of workgroups, two a CU, takes the chunks of
+// all live groups' tiles (16 rows x 256 columns) one behind the other in equal shares, so that all end together whatever the number of live groups, which only the device knows.
+// A tile spans at most nz workgroups (a share is no less than a tile / (nz - 1)); each writes its part into a slab of its own, the one that ends a tile zeros in the slabs behind.  Weights and rows of the
+// next tile are asked for while the last one is multiplied: the loads in flight do not end at a tile's end.
+constexpr int WALK_MAX = 1024;       // blocks of 16 rows: 256 groups of at most 64 rows
+struct WalkBlock { int row0; short group, rows; };
+__global__ __launch_bounds__(KW * 64, 4) void stream_kwalk_kernel(const bf16_t* __restrict__ Y, int64_t y_lo, const bf16_t* __restrict__ W, float* __restrict__ P, int64_t p_slab,
+                                                                  int Ntot, int K, int nz, int G, KGroups g) {
+  constexpr int CK = 64, ROWB = 128, XB = 32 * ROWB, COLS = KW * 32, D = 2;        // D: chunks in flight a wave (three: the same; four spill)
+  __shared__ __attribute__((aligned(16))) char xs[2 * XB], ws[KW * 32 * ROWB];      // x: [2 buffers][16 hi rows, 16 lo rows][64 k]; w: [wave][32 rows][64 k]
+  __shared__ WalkBlock list[WALK_MAX];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, fq = lane >> 4;
+  int n_blk = 0;
+  for (int e0 = 0; e0 < G; e0 += 64) {                                  // every wave scans the groups, wave 0 writes the list
+    const int e = e0 + lane, o = e < G ? g.off[e] : 0, n = e < G ? g.off[e + 1] - o : 0;
+    const int nb = n > g.row_lo && n <= g.row_hi ? (n + 15) >> 4 : 0;
+    int at = nb;                                                        // inclusive prefix over the lanes
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(at, d);
+      if (lane >= d) at += v;
+    }
+    if (wave == 0)
+      for (int j = 0; j < nb; ++j) list[n_blk + at - nb + j] = WalkBlock{o + 16 * j, (short)e, (short)min(16, n - 16 * j)};
+    n_blk += __builtin_amdgcn_readlane(at, 63);
+  }
+  __syncthreads();
+  const int nch = (K + CK - 1) / CK, tb = (Ntot + COLS - 1) / COLS, total = n_blk * tb * nch;
+  const int share = max((total + (int)gridDim.x - 1) / (int)gridDim.x, nz > 1 ? (nch + nz - 2) / (nz - 1) : nch);
+  const int begin = blockIdx.x * share, n = min(total, begin + share) - begin;
+  if (n <= 0) return;                                                   // uniform
+
+  // ---- the loads' side: chunk pc of tile pt next ----
+  int pt = begin / nch, pc = begin - pt * nch;
+  const int slot = lane & 7;
+  const bf16_t *wp[4], *xp = nullptr;
+  auto open = [&](int tile) {
+    const WalkBlock b = list[tile / tb];
+    const int grp = __builtin_amdgcn_readfirstlane(b.group), n0 = (tile % tb) * COLS + wave * 32 + (lane >> 3);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wp[i] = W + (int64_t)grp * g.w_stride + (int64_t)min(n0 + i * 8, Ntot - 1) * K;
+    const int h = tid >> 7, m = (tid >> 3) & 15;                        // threads 0 .. 255: row m's hi or lo part, slot
+    xp = nullptr;
+    if (tid < 256 && m < b.rows) xp = Y + h * y_lo + (int64_t)(g.xrows ? g.xrows[b.row0 + m] : b.row0 + m) * K + slot * 8;
+  };
+  u32x4 wr[D][4], xr[D];
+  auto load = [&](u32x4 (&w)[4], u32x4& x) {
+    const int k = min(pc * CK + slot * 8, K - 8);                       // beyond K the x image is zero: any finite value will do
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp[i] + k));
+    x = u32x4{0u, 0u, 0u, 0u};
+    if (xp && pc * CK + slot * 8 < K) x = *reinterpret_cast<const u32x4*>(xp + pc * CK);
+    if (++pc == nch) { pc = 0; if (++pt < n_blk * tb) open(pt); }
+  };
+  auto put_x = [&](const u32x4& x, int buf) {
+    if (tid < 256) *reinterpret_cast<u32x4*>(xs + buf * XB + cslot<CK>(tid >> 3, slot)) = x;
+  };
+  open(pt);
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d < n) load(wr[d], xr[d]);
+  put_x(xr[0], 0);
+  __syncthreads();
+
+  // ---- the products' side: chunk c of tile ct ----
+  int ct = begin / nch, c = begin - ct * nch, buf = 0;
+  char* wt = ws + wave * 32 * ROWB;
+  f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  for (int jb = 0; jb < n; jb += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int j = jb + d;
+      if (j < n) {                                                      // uniform
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(wt + cslot<CK>(i * 8 + (lane >> 3), slot)) = wr[d][i];
+        if (j + D < n) load(wr[d], xr[d]);                              // (x of this chunk is in LDS since the one before)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const bf16x8 ah = *reinterpret_cast<const bf16x8*>(xs + buf * XB + cslot<CK>(fr, s * 4 + fq));
+          const bf16x8 al = *reinterpret_cast<const bf16x8*>(xs + buf * XB + cslot<CK>(16 + fr, s * 4 + fq));
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const bf16x8 w = *reinterpret_cast<const bf16x8*>(wt + cslot<CK>(t * 16 + fr, s * 4 + fq));
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, w, acc[t], 0, 0, 0);
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, w, acc[t], 0, 0, 0);
+          }
+        }
+        if (++c == nch || j + 1 == n) {                                 // this workgroup's part of the tile is done
+          const WalkBlock b = list[ct / tb];
+          const int z = blockIdx.x - ct * nch / share, zeros = c == nch ? nz - 1 - z : 0;      // (a tile's parts are consecutive workgroups')
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const int nn = (ct % tb) * COLS + wave * 32 + t * 16 + fr;
+            if (nn < Ntot) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                if (fq * 4 + r < b.rows) {
+                  float* p_ = P + (int64_t)z * p_slab + (int64_t)(b.row0 + fq * 4 + r) * Ntot + nn;
+                  *p_ = acc[t][r];
+                  for (int e = 1; e <= zeros; ++e) p_[e * p_slab] = 0.f;
+                }
+            }
+            acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+          c = 0;
+          ++ct;
+        }
+        if (j + 1 < n) put_x(xr[(d + 1) % D], buf ^ 1);                 // (its readers passed the barrier before)
+        buf ^= 1;
+        __syncthreads();
+      }
+    }
+  }
+}
+
 int g_kl_nz = 0, g_kl_depth = 0, g_kl_nt = 0, g_kl_ck = 0;
 
 // k per chunk: 64 (x double buffer 32 KiB + weight tiles 32 KiB at 64 rows: two workgroups fit a CU, also one of another
@@ -419,6 +536,28 @@ extern "C" int mn_stream_kloop_grouped(const uint16_t* Y, int y_rows, const uint
   const KGroups g{off, xrows, w_stride, row_lo, max_rows, 0, 0};
   kloop_dispatch(G, max_rows, nz, Y, (int64_t)y_rows * K, W, nullptr, P, (int64_t)p_rows * Ntot, 0, Ntot, K, g, mn_stream(stream));
   MN_CHECK_LAUNCH("mn_stream_kloop_grouped");
+  return nz;
+}
+
+// The grouped bf16 product of the decoder's steps, and the slabs it may write (the callers' buffers).  us, an expert layer's gate and up (5632 x 2048) / down (2048 x 1408) of 64 experts,
+// 6 a row, and two that all rows share, grid in two ranges -> walk: 3 rows 46.7 -> 36.7 / 22.1 -> 21.5, 3 rows with the same experts 25.1 -> 19.2 / 17.3 -> 13.5, 4 51.1 -> 47.7 / 32.9 -> 26.1
+// (four slabs), 6 64.3 -> 58.4 / 36.2 -> 31.7, 8 77.1 -> 76.5 / 40.7 -> 38.9, 16 103 -> 100 / 55.6 -> 52.3, 20 126 -> 116 / 65.6 -> 59.7, 24 rows of 12 sets of experts 89.8 -> 83.0 / 51.0 -> 43.3
+// (three; with two a share is no less than a tile: 98.7 / 48.2).  Above 32 rows the blocks of 16 read the shared experts four times: 33 rows 119 -> 128 / 72.3 -> 65.8, 48 127 -> 133 /
+// 74.8 -> 71.3, 64 131 -> 141 / 76.9 -> 74.6 (two), so there only where the grid's last round would be mostly empty.
+extern "C" int mn_stream_kwalk_slices(int max_rows, int K) {
+  const int nch = (K + 63) / 64, want = max_rows <= 4 ? 4 : (max_rows <= 32 ? 3 : 2);
+  return nch < want ? nch : want;
+}
+extern "C" int mn_stream_kwalk_grouped(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G,
+                                       int max_rows, int Ntot, int K, void* stream) {
+  const int nz = mn_stream_kwalk_slices(max_rows, K);
+  MN_CHECK_ARG(Y && W && P && off && G >= 1 && max_rows >= 1 && max_rows <= 64 && Ntot >= 1 && K >= 8 && (K % 8) == 0, "mn_stream_kwalk_grouped: bad args");
+  const int64_t places = 2 * (int64_t)mn_num_cus(), wgs = mn_cdiv(mn_cdiv(Ntot, 16), 2 * KW) * nz * G;
+  if (G > 256 || (max_rows > 32 && 5 * wgs >= 4 * mn_cdiv(wgs, places) * places))
+    return mn_stream_kloop_grouped(Y, y_rows, W, w_stride, P, p_rows, off, xrows, G, max_rows, 0, nz, Ntot, K, stream);
+  const KGroups g{off, xrows, w_stride, 0, max_rows, 0, 0};
+  hipLaunchKernelGGL(stream_kwalk_kernel, dim3((unsigned)places), dim3(KW * 64), 0, mn_stream(stream), Y, (int64_t)y_rows * K, W, P, (int64_t)p_rows * Ntot, Ntot, K, nz, G, g);
+  MN_CHECK_LAUNCH("mn_stream_kwalk_grouped");
   return nz;
 }
 

@@ -300,8 +300,8 @@ static size_t llm_tp_carve(const mn_llm* m, const mn_llm_tp* tp, int rows, int64
     const size_t s3 = (size_t)stream_slices(m->wfmt, rows, H, SIc) * rows * H;
     if (s3 > psh) psh = s3;
     o->pps = cv.take<float>(pmax * rows);
-    o->p1 = cv.take<float>((size_t)mn_stream_mfma_grouped_slices(m->n_experts, rows, 2 * I, H) * Pn * 2 * I);
-    o->p2 = cv.take<float>((size_t)mn_stream_mfma_grouped_slices(m->n_experts, rows, H, I) * Pn * H);
+    o->p1 = cv.take<float>((size_t)mn_stream_kwalk_slices(rows, H) * Pn * 2 * I);
+    o->p2 = cv.take<float>((size_t)mn_stream_kwalk_slices(rows, I) * Pn * H);
   }
   o->psh = cv.take<float>(psh);
   return off + cv.off;

@@ -62,13 +62,9 @@ def test_replayed():
     dec.kv_cache.normal_()
     length, out = slot + 1, torch.empty(M, 256, device="cuda")
     want = dec.step(x, seq, slot, slot, length, distinct_sequences=True).clone()
-    s = torch.cuda.Stream()
-    s.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(s):
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
         dec.step(x, seq, slot, slot, length, out=out, distinct_sequences=True)
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=s):
-            dec.step(x, seq, slot, slot, length, out=out, distinct_sequences=True)
     torch.cuda.synchronize()
     for _ in range(4):
         out.zero_()

@@ -224,10 +224,11 @@ extern "C" int mn_polynorm_rows_split(const float* z, int64_t ldz, const uint16_
 extern "C" int mn_rms_rows_pair(const float* xa, const uint16_t* wa, float* ya, int64_t ldya, uint16_t* ya16, int64_t ldya16, int na, const float* xb, const uint16_t* wb,
                                 float* yb, const int32_t* row_seq, const int32_t* row_slot, int t_max, int nb, int64_t ldx, float eps, int M, void* stream);
 extern "C" int mn_attn_prefill_hd64_planes(const uint16_t* qkv, int64_t lo_off, uint16_t* split, int B, int T, int n_heads, int causal, void* stream);
-// the products of a vision block on few rows (vit_rows.hip): LayerNorm in front, or the residual behind, in the same launch
+// the products of a vision block on few rows (rows_gemm.hip): LayerNorm in front, or the residual behind, in the same launch
 extern "C" int mn_vit_rows_ok(int M, int dim, int hidden, int gelu);
 extern "C" int mn_ln_gemm_rows(const float* x, int64_t ldx, const uint16_t* g, const uint16_t* b, float eps, const uint16_t* W, int64_t ldw, const uint16_t* bias, int gelu, int pair,
                                uint16_t* C, int64_t ldc, int M, int N, int K, void* stream);
 extern "C" int mn_resid_gemm_rows(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t ldw, const uint16_t* bias, float* x, int64_t ldx, int M, int N, int K, void* stream);
+extern "C" int mn_rows_gemm(const mn_g256* a, int epi, double tile_us, void* stream);
 extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo);
 extern "C" int mn_gemm256_f8_plan_ksplit(int M, int N, int K);

@@ -654,7 +654,9 @@ static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
   // (the 256-tile kernel's GELU is the 1.5e-7 polynomial: it serves the problems of 128 tiles and more, where erff in the small tiles' epilogue costs more than they save:
   // 4096 x 4096 x 256 26.9 us against 38.6, 8000 x 4000 x 192 45 against 69)
   const bool may256 = epi != E_BF16_GELU || mn_cdiv(p.M, 256) * mn_cdiv(p.N, 256) >= 128;
-  const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : epi == E_BF16_GELU && may256 ? 0 : tile_form(p.M, p.N, p.Kc, nz, hilo, epi, may256, nullptr);
+  double us = 0;
+  const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : epi == E_BF16_GELU && may256 ? 0 : tile_form(p.M, p.N, p.Kc, nz, hilo, epi, may256, &us);
+  if (us > 0 && nz == 1 && mn_rows_gemm(&p, epi, us, st)) return 1;       // few tiles: forms whose waves split K (rows_gemm.hip)
 #define G256_GO(E)                                                                          \
   do {                                                                                      \
     if (form > 0 && tile_launch<E>(p, form, nz, hilo, st)) break;                           \

@@ -1,13 +1,15 @@
-// vit_rows.hip — the products of a vision-transformer block on few rows (a picture's 65 encoder tokens, its 256 pixel-decoder tokens): LayerNorm in front of the product
-// and the residual behind it in the same launch, so that a block is five launches and not seven (block.py:80-105, mlp.py:34-40, swiglu_ffn.py:27-34).
+// rows_gemm.hip — bf16 products whose tiles are one round of the CUs at most (gfx950): a vision block's on few rows (a picture's 65 encoder tokens, its 256 pixel-decoder tokens),
+// with LayerNorm in front or the residual behind in the same launch, so that a block is five launches and not seven (block.py:80-105, mlp.py:34-40, swiglu_ffn.py:27-34), and the
+// sequence models' prompts of a few hundred rows.
 //
 //   mn_ln_gemm_rows      C = act(bf16(LayerNorm(x)) W^T + b)      x fp32, act: none, exact GELU, SwiGLU; C bf16
 //   mn_resid_gemm_rows   x += A W^T + b                           A bf16, x fp32
+//   mn_rows_gemm         gemm256.hip's dense products of plain or hi/lo rows, where it estimates these forms faster than its tiles
 //
-// What bounds such a launch is latency, a launch boundary (1.5 us) and then one memory round trip after another, not bytes (6 MB of weights are 1.3 us at HBM rate)
-// and not the matrix cores.  So:
-//   * a workgroup asks for all it needs at once: its rows' LayerNorm input into registers, its weights by global_load_lds into up to 96 KiB of LDS, bias and residual;
-//   * 32-row tiles by 16 .. 128 columns, the columns chosen so that the tiles are one round of the CUs;
+// What bounds such a launch is latency, a launch boundary (1.5 us) and then one memory round trip after another, and what a CU can take in (64 B a cycle), not HBM (6 MB of weights are
+// 1.3 us) and not the matrix cores.  So:
+//   * a workgroup asks for all it needs at once: its rows' LayerNorm input into registers, rows and weights by global_load_lds into up to 160 KiB of LDS, bias and residual;
+//   * tiles of 16 .. 64 rows by 16 .. 128 columns, the ones that bring a workgroup the fewest bytes while all of them are one round of the CUs;
 //   * LayerNorm is done again by every workgroup of a row tile (32 rows x 4 KB from its XCD's L2): that costs less than a launch of its own with its round trips, and
 //     no split-K slabs have to be summed by anyone: the eight waves split K inside the workgroup and meet in LDS once.
 // us a launch with cold weights, these against a 64 x 64 tile launch and the launch that norms its rows or sums its slabs: 65 rows, 1024 -> 3072 7.5 / 7.7 + 4.6,
@@ -32,9 +34,10 @@ struct RowsGemm {
   const bf16_t* A; int64_t lda;                                                  // else
   const bf16_t* W; int64_t ldw; const bf16_t* bias; int64_t pair;                // pair: row distance from a unit's gate to its up
   void* C; int64_t ldc; int M, N, K;
+  int64_t a_lo, c_lo;                                                            // HILO: elements from a row's hi part to its lo part; split results likewise
   uint32_t tiles_m, magic;                                                       // magic: ceil(2^32 / tiles_m)
 };
-enum { R_BF16, R_GELU, R_SWIGLU, R_RESID };
+enum { R_BF16, R_GELU, R_SWIGLU, R_RESID, R_F32, R_SPLIT, R_SWIGLU_SPLIT };
 
 __device__ __forceinline__ f32x4 bf16x4(u32x2 b) { return f32x4{bf16lo_to_f32(b.x), bf16hi_to_f32(b.x), bf16lo_to_f32(b.y), bf16hi_to_f32(b.y)}; }
 
@@ -53,15 +56,15 @@ __device__ __forceinline__ void wait_stages(int rem) {
 
 constexpr int KMAX = 1024;
 
-// NJ: fragments of 16 weight rows a tile; KW: waves along K (a stage is KW k-steps of 32), 8 / KW waves along the columns; S: stages of LDS
-template <int EPI, bool NORM, int BM, int NJ, int KW, int S>
+// HILO: A is a bf16 hi row and, a_lo elements further, the same row's lo part, both multiplied.  NJ: fragments of 16 weight rows a tile; KW: waves along K (a stage is KW k-steps of 32), 8 / KW waves along the columns; S: stages of LDS
+template <int EPI, bool NORM, bool HILO, int BM, int NJ, int KW, int S>
 __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
   constexpr int MI = BM / 16, RW = BM / 8, BN = 16 * NJ, WN = 8 / KW, NW = NJ / WN, ROWB = KW * 64, SLOTS = ROWB / 16, RPI = 1024 / ROWB;
-  constexpr bool paired = EPI == R_SWIGLU, resid = EPI == R_RESID;
-  constexpr int AB = NORM ? BM * KMAX * 2 : 0, ROWS = BN + (NORM ? 0 : BM), STAGE = ROWS * ROWB, Q = STAGE / 1024 / 8;
+  constexpr bool paired = EPI == R_SWIGLU || EPI == R_SWIGLU_SPLIT, resid = EPI == R_RESID, f32 = resid || EPI == R_F32, split = EPI == R_SPLIT || EPI == R_SWIGLU_SPLIT;
+  constexpr int AB = NORM ? BM * KMAX * 2 : 0, AR = NORM ? 0 : HILO ? 2 * BM : BM, ROWS = BN + AR, STAGE = ROWS * ROWB, Q = STAGE / 1024 / 8;
   constexpr int OC = paired ? BN / 2 : BN, RS = BN + 4, RED = KW * BM * RS * 4, GROUPS = BM * OC / 4, T = (GROUPS + 511) / 512;
   constexpr int LDS = AB + S * STAGE > RED ? AB + S * STAGE : RED;
-  static_assert(NJ % WN == 0 && Q * 1024 * 8 == STAGE && Q * (S - 1) < 64 && LDS <= 160 * 1024, "whole fragments and instructions a wave, vmcnt range, LDS");
+  static_assert(!(NORM && HILO) && NJ % WN == 0 && Q * 1024 * 8 == STAGE && Q * (S - 1) < 64 && LDS <= 160 * 1024, "whole fragments and instructions a wave, vmcnt range, LDS");
   __shared__ __attribute__((aligned(1024))) char lds[LDS];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kw = wave % KW, wn = wave / KW, fr = lane & 15, fq = lane >> 4;
@@ -102,7 +105,7 @@ __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
     const int L = (wave * Q + q) * RPI + rin;
     kin[q] = (uint32_t)((slot ^ (L & 15)) << 4);
     if (!NORM && L >= BN) {
-      src[q] = (uint32_t)min(m0 + L - BN, p.M - 1) * ((uint32_t)p.lda * 2u);
+      src[q] = (uint32_t)min(m0 + (L - BN) % BM, p.M - 1) * ((uint32_t)p.lda * 2u) + (HILO && L - BN >= BM ? (uint32_t)p.a_lo * 2u : 0u);
     } else if (paired) {
       src[q] = (uint32_t)(min(n0 + L % OC, p.N - 1) + (L >= OC ? (int)p.pair : 0)) * ((uint32_t)p.ldw * 2u);
     } else {
@@ -189,6 +192,15 @@ __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
 #pragma unroll
     for (int i = 0; i < MI; ++i)
       af[i] = *reinterpret_cast<const bf16x8*>(NORM ? lds + (i * 16 + fr) * p.K * 2 + (((t * KW + kw) * 4 + fq) ^ fr) * 16 : w + (BN + i * 16 + fr) * ROWB + sl);
+    if constexpr (HILO) {
+      bf16x8 al[MI];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) al[i] = *reinterpret_cast<const bf16x8*>(w + (BN + BM + i * 16 + fr) * ROWB + sl);
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NW; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], al[i], acc[i][j], 0, 0, 0);
+    }
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -240,34 +252,83 @@ __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
       a = f32x4{silu_f(a.x) * u.x, silu_f(a.y) * u.y, silu_f(a.z) * u.z, silu_f(a.w) * u.w};
     }
     if (EPI == R_GELU) a = f32x4{gelu_erf_f(a.x), gelu_erf_f(a.y), gelu_erf_f(a.z), gelu_erf_f(a.w)};
-    if (resid) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.C) + om[t] * p.ldc + on[t]) = rv[t] + a;
-    else *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(p.C) + om[t] * p.ldc + on[t]) = u32x2{cvt_pk_bf16(a.x, a.y), cvt_pk_bf16(a.z, a.w)};
+    if (f32) {
+      if (resid) a += rv[t];
+      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.C) + om[t] * p.ldc + on[t]) = a;
+    } else {
+      bf16_t* c = reinterpret_cast<bf16_t*>(p.C) + om[t] * p.ldc + on[t];
+      if (split) {
+        uint32_t h0, h1, l0, l1;
+        split_pk_bf16(a.x, a.y, h0, l0);
+        split_pk_bf16(a.z, a.w, h1, l1);
+        *reinterpret_cast<u32x2*>(c) = u32x2{h0, h1};
+        *reinterpret_cast<u32x2*>(c + p.c_lo) = u32x2{l0, l1};
+      } else {
+        *reinterpret_cast<u32x2*>(c) = u32x2{cvt_pk_bf16(a.x, a.y), cvt_pk_bf16(a.z, a.w)};
+      }
+    }
   }
 }
 
-template <int EPI, bool NORM, int BM, int NJ, int KW, int S>
+template <int EPI, bool NORM, bool HILO, int BM, int NJ, int KW, int S>
 void go(RowsGemm p, hipStream_t st) {
   p.tiles_m = (uint32_t)mn_cdiv(p.M, BM);
   p.magic = (uint32_t)mn_cdiv((int64_t)1 << 32, p.tiles_m);
-  const int64_t tiles = p.tiles_m * mn_cdiv(p.N, EPI == R_SWIGLU ? NJ * 8 : NJ * 16);
-  hipLaunchKernelGGL((rows_gemm_kernel<EPI, NORM, BM, NJ, KW, S>), dim3((unsigned)tiles), dim3(512), 0, st, p);
+  const int64_t tiles = p.tiles_m * mn_cdiv(p.N, EPI == R_SWIGLU || EPI == R_SWIGLU_SPLIT ? NJ * 8 : NJ * 16);
+  hipLaunchKernelGGL((rows_gemm_kernel<EPI, NORM, HILO, BM, NJ, KW, S>), dim3((unsigned)tiles), dim3(512), 0, st, p);
 }
 
-// A tile form and what a workgroup of it takes, us: a launch and its prologue, LayerNorm of its rows (five vector instructions a value), its bytes at what a CU takes in
-// (45 KB/us of rows its L2 holds and weights from HBM).
-struct Form { int bm, nj, kw; };
-double form_time(const Form& f, bool norm, int M, int64_t wrows, int K) {
-  const double rounds = (double)mn_cdiv(mn_cdiv(M, f.bm) * mn_cdiv(wrows, 16 * f.nj), mn_num_cus());
-  return 1.9 + rounds * ((norm ? (0.25 + 0.05 * f.bm) * K / 1024 : 0.5) + (f.bm * (norm ? 4 : 2) + 32.0 * f.nj) * K / 45e3);
-}
-template <int N>
-int best_form(const Form (&forms)[N], bool norm, int M, int64_t wrows, int K) {
+struct Form { int bm, nj; };
+int64_t form_tiles(const Form& f, int M, int64_t wrows) { return mn_cdiv(M, f.bm) * mn_cdiv(wrows, 16 * f.nj); }
+template <int N, class Time>
+int best_form(const Form (&forms)[N], Time time, double* us) {
   int best = 0;
-  for (int i = 1; i < N; ++i)
-    if (form_time(forms[i], norm, M, wrows, K) < form_time(forms[best], norm, M, wrows, K)) best = i;
+  double tb = 1e30;
+  for (int i = 0; i < N; ++i) {
+    const double t = time(forms[i]);
+    if (t < tb) { tb = t; best = i; }
+  }
+  if (us) *us = tb;
   return best;
 }
-constexpr Form ln_forms[] = {{16, 4, 8}, {16, 8, 4}, {32, 3, 8}, {32, 6, 4}, {32, 8, 4}}, res_forms[] = {{32, 1, 8}, {16, 2, 8}, {32, 2, 8}, {32, 4, 8}};
+// What a workgroup takes, us.  Behind a LayerNorm: a launch and its prologue, the norm of its rows (five vector instructions a value), its bytes, rows from its L2 and
+// weights from HBM (45 KB/us); more rounds than one where there is nothing else.
+constexpr Form ln_forms[] = {{16, 4}, {16, 8}, {32, 3}, {32, 6}, {32, 8}};
+double ln_time(const Form& f, int M, int64_t wrows, int K) {
+  const double rounds = (double)mn_cdiv(form_tiles(f, M, wrows), mn_num_cus());
+  return 1.9 + rounds * ((0.25 + 0.05 * f.bm) * K / 1024 + (f.bm * 4 + 32.0 * f.nj) * K / 45e3);
+}
+// Plain: 2.3 us and 68 KB/us, one round or nothing.  us, measured / this: 32 x 16 tiles of K = 1024 3.7 / 3.7, 32 x 32 of 1024 4.2 / 4.2, of 4096 9.7 / 10.0, of 8192 15.6 / 17.7, 64 x 32 of 1024
+// 5.0 / 5.2, of 8192 20.4 / 25.4, 64 x 64 of 4096 16.6 / 17.7, 64 x 128 of 2048 15.9 / 13.9, of 8192 46.7 / 48.5.
+constexpr Form forms[] = {{32, 1}, {16, 2}, {32, 2}, {32, 4}, {64, 2}, {64, 4}, {64, 8}}, hilo_forms[] = {{16, 2}, {32, 1}, {32, 2}, {32, 4}, {32, 6}, {32, 8}, {64, 2}, {64, 4}};
+double rows_time(const Form& f, bool hilo, int M, int64_t wrows, int K) {
+  return form_tiles(f, M, wrows) > mn_num_cus() ? 1e30 : 2.3 + (f.bm * (hilo ? 2 : 1) + 16 * f.nj) * (double)K / 34e3;
+}
+template <int EPI>
+void go_plain(int form, const RowsGemm& p, hipStream_t st) {
+  switch (form) {
+    case 0: go<EPI, false, false, 32, 1, 8, 6>(p, st); break;
+    case 1: go<EPI, false, false, 16, 2, 8, 6>(p, st); break;
+    case 2: go<EPI, false, false, 32, 2, 8, 5>(p, st); break;
+    case 3: go<EPI, false, false, 32, 4, 8, 3>(p, st); break;
+    case 4: go<EPI, false, false, 64, 2, 8, 3>(p, st); break;
+    case 5: go<EPI, false, false, 64, 4, 4, 5>(p, st); break;
+    default: go<EPI, false, false, 64, 8, 4, 3>(p, st); break;
+  }
+}
+template <int EPI>
+void go_hilo(int form, const RowsGemm& p, hipStream_t st) {
+  switch (form) {
+    case 0: go<EPI, false, true, 16, 2, 8, 5>(p, st); break;
+    case 1: go<EPI, false, true, 32, (EPI == R_SWIGLU_SPLIT ? 2 : 1), 8, 3>(p, st); break;
+    case 2: go<EPI, false, true, 32, 2, 8, 3>(p, st); break;
+    case 3: go<EPI, false, true, 32, 4, 4, 5>(p, st); break;
+    case 4: go<EPI, false, true, 32, 6, 4, 4>(p, st); break;
+    case 5: go<EPI, false, true, 32, 8, 4, 3>(p, st); break;
+    case 6: go<EPI, false, true, 64, 2, 4, 4>(p, st); break;
+    default: go<EPI, false, true, 64, 4, 4, 3>(p, st); break;
+  }
+}
 
 bool shape_ok(const void* A, int64_t lda, const void* W, int64_t ldw, int64_t wrows, const void* bias, const void* C, int64_t ldc, int M, int N, int K) {
   return M >= 1 && N >= 4 && N % 4 == 0 && K >= 64 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldc % 4 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15) == 0 &&
@@ -293,12 +354,12 @@ extern "C" int mn_ln_gemm_rows(const float* x, int64_t ldx, const uint16_t* g, c
   p.x = x; p.ldx = ldx; p.g = g; p.b = b; p.eps = eps; p.W = W; p.ldw = ldw; p.bias = bias; p.pair = pair ? N : 0; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K;
   hipStream_t st = mn_stream(stream);
 #define GO(E)                                                                              \
-  switch (best_form(ln_forms, true, M, pair ? 2 * (int64_t)N : N, K)) {                    \
-    case 0: go<E, true, 16, 4, 8, 4>(p, st); break;                                        \
-    case 1: go<E, true, 16, 8, 4, 4>(p, st); break;                                        \
-    case 2: go<E, true, 32, 3, 8, 4>(p, st); break;                                        \
-    case 3: go<E, true, 32, 6, 4, 4>(p, st); break;                                        \
-    default: go<E, true, 32, 8, 4, 3>(p, st); break;                                       \
+  switch (best_form(ln_forms, [&](const Form& f) { return ln_time(f, M, pair ? 2 * (int64_t)N : N, K); }, nullptr)) {          \
+    case 0: go<E, true, false, 16, 4, 8, 4>(p, st); break;                                        \
+    case 1: go<E, true, false, 16, 8, 4, 4>(p, st); break;                                        \
+    case 2: go<E, true, false, 32, 3, 8, 4>(p, st); break;                                        \
+    case 3: go<E, true, false, 32, 6, 4, 4>(p, st); break;                                        \
+    default: go<E, true, false, 32, 8, 4, 3>(p, st); break;                                       \
   }
   if (pair) { GO(R_SWIGLU) } else if (gelu) { GO(R_GELU) } else { GO(R_BF16) }
 #undef GO
@@ -310,13 +371,40 @@ extern "C" int mn_resid_gemm_rows(const uint16_t* A, int64_t lda, const uint16_t
   MN_CHECK_ARG(A && W && x && shape_ok(A, lda, W, ldw, N, bias, x, ldx, M, N, K), "mn_resid_gemm_rows: bad args");
   RowsGemm p{};
   p.A = A; p.lda = lda; p.W = W; p.ldw = ldw; p.bias = bias; p.C = x; p.ldc = ldx; p.M = M; p.N = N; p.K = K;
-  hipStream_t st = mn_stream(stream);
-  switch (best_form(res_forms, false, M, N, K)) {
-    case 0: go<R_RESID, false, 32, 1, 8, 6>(p, st); break;
-    case 1: go<R_RESID, false, 16, 2, 8, 6>(p, st); break;
-    case 2: go<R_RESID, false, 32, 2, 8, 5>(p, st); break;
-    default: go<R_RESID, false, 32, 4, 8, 3>(p, st); break;
-  }
+  double us;
+  int form = best_form(forms, [&](const Form& f) { return rows_time(f, false, M, N, K); }, &us);
+  if (us >= 1e30) form = 6;                              // more than one round of the largest
+  go_plain<R_RESID>(form, p, mn_stream(stream));
   MN_CHECK_LAUNCH("mn_resid_gemm_rows");
   return MN_OK;
+}
+
+// One dense product of gemm256.hip, of tile_us on its tiles by its estimate: taken (1) where a form here is estimated a tenth faster, else 0 and nothing is launched.
+// us, the tiles / these, cold weights, 40, 101, 256 and 600 rows: hi/lo 768 -> 768 7.5 / 3.8, 7.8 / 3.9, 7.9 / 4.7, 8.1 / 6.0; 2048 -> 768 15.3 / 5.9, 15.5 / 6.0, 15.7 / 7.1, 15.9 / 10.6;
+// 768 -> 2304 7.7 / 4.1, 7.9 / 5.8, 8.4 / 6.8, tiles; 4096 -> 1024 27.3 / 8.5, 27.9 / 8.8, 27.6 / 11.8, 28.4 / 21.8; 1024 -> 2 x 2752 gated 10.4 / 8.1, 10.5 / 9.4, tiles (14.1).  Plain rows, 70, 250, 450 and
+// 1000: 1024 -> 1024 6.9 / 3.8, 6.9 / 4.5, 7.1 / 5.6, tiles (7.4); 2048 -> 2048 10.5 / 6.1, 10.9 / 7.7, 11.2 / 10.5, 17.4 / 16.0; 8192 -> 2048 34.0 / 16.3, 36.7 / 25.9, 36.7 / 31.7, 57.9 / 51.4; 1024 -> 4096
+// 7.0 / 5.5, tiles (7.4).  The error is smaller throughout (eight sums of K / 8: 1.0e-7 for 1.9e-7 of 64 bits at K = 2048).
+extern "C" int mn_rows_gemm(const mn_g256* a, int epi, double tile_us, void* stream) {
+  const bool hilo = a->a_lo_off != 0, paired = epi == MN_G256_SWIGLU_SPLIT;
+  const bool known = epi == MN_G256_F32 || epi == MN_G256_F32_RESID || (hilo ? epi == MN_G256_BF16_SPLIT || paired : epi == MN_G256_BF16);
+  const int64_t wrows = paired ? a->w_pair_rows + a->N : a->N, rows = paired ? 2 * (int64_t)a->N : a->N;
+  if (!known || a->g_off || a->a_rows || a->f8 || (a->w_pair_rows != 0) != paired || ((uintptr_t)a->C & (epi == MN_G256_F32 || epi == MN_G256_F32_RESID ? 15 : 7)) || a->c_lo_off % 4 || a->w_pair_rows % 4 ||
+      !shape_ok(a->A, a->lda, a->W, a->ldw, wrows, a->bias, nullptr, a->ldc, a->M, a->N, a->K) || ((int64_t)a->M * a->lda + a->a_lo_off) * 2 >= ((int64_t)1 << 32) || a->a_lo_off % 8)
+    return 0;
+  double us;
+  const auto time = [&](const Form& f) { return (epi == MN_G256_SWIGLU_SPLIT && f.nj == 1) ? 1e30 : rows_time(f, hilo, a->M, rows, a->K); };
+  const int form = hilo ? best_form(hilo_forms, time, &us) : best_form(forms, time, &us);
+  if (us >= 0.9 * tile_us) return 0;
+  RowsGemm p{};
+  p.A = a->A; p.lda = a->lda; p.a_lo = a->a_lo_off; p.W = a->W; p.ldw = a->ldw; p.bias = a->bias; p.pair = a->w_pair_rows; p.C = a->C; p.ldc = a->ldc; p.c_lo = a->c_lo_off;
+  p.M = a->M; p.N = a->N; p.K = a->K;
+  hipStream_t st = mn_stream(stream);
+  switch (epi) {
+    case MN_G256_F32: hilo ? go_hilo<R_F32>(form, p, st) : go_plain<R_F32>(form, p, st); break;
+    case MN_G256_F32_RESID: hilo ? go_hilo<R_RESID>(form, p, st) : go_plain<R_RESID>(form, p, st); break;
+    case MN_G256_BF16: go_plain<R_BF16>(form, p, st); break;
+    case MN_G256_BF16_SPLIT: go_hilo<R_SPLIT>(form, p, st); break;
+    default: go_hilo<R_SWIGLU_SPLIT>(form, p, st); break;
+  }
+  return 1;
 }

@@ -37,7 +37,7 @@ Plan plan(int64_t M, int dim, int hidden, int gelu, int precise) {
   return p;
 }
 
-// the products that take their LayerNorm or residual with them (vit_rows.hip): few rows, 16-byte weights, 8-byte biases and norm parameters
+// the products that take their LayerNorm or residual with them (rows_gemm.hip): few rows, 16-byte weights, 8-byte biases and norm parameters
 bool rows_ok(const float* x, const uint16_t* const* w, int depth, int64_t M, int dim, int hidden, int gelu) {
   if (!mn_vit_rows_ok((int)M, dim, hidden, gelu) || ((uintptr_t)x & 15)) return false;
   for (int i = 0; i < 12 * depth; ++i) {

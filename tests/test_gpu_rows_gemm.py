@@ -1,0 +1,70 @@
+"""The dense products whose tiles are one round of the CUs: waves that split K inside a workgroup (rows_gemm.hip), behind the wide-row GEMM's entry points."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (rows, columns, K): each tile form of both operand kinds, one row, one fragment, columns and rows past the last tile, K of one k-step pair and no whole number of stages
+SHAPES = [(1, 4, 64), (15, 36, 192), (17, 100, 64), (33, 1024, 1024), (70, 1028, 320), (101, 2304, 768), (130, 1024, 4096), (250, 1020, 2752), (257, 2048, 576), (450, 1024, 1024), (600, 768, 2048),
+          (1000, 2048, 8192)]
+
+
+def rows(g, M, K, hilo, pad):
+    """fp32 values of M rows and their bf16 operand: plain, or hi and lo rows with `pad` columns between the rows."""
+    buf = torch.zeros(2, M, K + pad, dtype=torch.bfloat16, device="cuda")
+    x = torch.randn(M, K, device="cuda", generator=g)
+    buf[0, :, :K] = x
+    if hilo:
+        buf[1, :, :K] = x - buf[0, :, :K].float()
+    return buf, buf[0, :, :K].double() + buf[1, :, :K].double()
+
+
+@pytest.mark.parametrize("hilo", [0, 1])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_dense_epilogues(M, N, K, hilo):
+    from ming_univision_amd import _lib
+    from ming_univision_amd._lib import ptr
+    L = _lib.lib()
+    g = torch.Generator(device="cuda").manual_seed(M + N + K + hilo)
+    st = torch.cuda.current_stream().cuda_stream
+    pad = 8 if M % 2 else 0
+    A, a64 = rows(g, M, K, hilo, pad)
+    W = torch.empty(N, K + pad, dtype=torch.bfloat16, device="cuda").normal_(0, K ** -0.5, generator=g)
+    bias = torch.randn(N, device="cuda", generator=g).bfloat16() if M != 33 else None
+    w64 = W[:, :K].double()
+    prod = a64 @ w64.t() + (bias.double() if bias is not None else 0.0)
+    sums = a64.abs() @ w64.abs().t() + (bias.double().abs() if bias is not None else 0.0)
+    ldc = N + 4
+    for epi in (2, 3, 0):                                # fp32, fp32 added to what is there, bf16
+        C = torch.full((M + 1, ldc), 0.5, device="cuda", dtype=torch.bfloat16 if epi == 0 else torch.float32)
+        rc = L.mn_gemm256(ptr(A), K + pad, A[0].numel() if hilo else 0, ptr(W), K + pad, ptr(bias) if bias is not None else None, ptr(C), ldc, M, N, K, epi, st)
+        assert rc == 0
+        ref = prod + (0.5 if epi == 3 else 0.0)
+        # K products (twice for hi/lo) and the bias added in some order in fp32: 2^-24 of the sum of magnitudes each; one rounding to bf16: 2^-8
+        bound = (2 * K + 16) * 2.0 ** -24 * (sums + 0.5) + (2.0 ** -8 * ref.abs() if epi == 0 else 0.0)
+        assert bool(((C[:M, :N].double() - ref).abs() <= bound).all()), (epi, float((C[:M, :N].double() - ref).abs().max()))
+        assert bool((C[M:] == 0.5).all()) and bool((C[:, N:] == 0.5).all())
+
+
+@pytest.mark.parametrize("M,hidden,K", [(1, 4, 64), (17, 36, 192), (40, 2048, 768), (101, 2752, 1024), (128, 1028, 320), (256, 2048, 768)])
+def test_gated_hilo(M, hidden, K):
+    from ming_univision_amd import _lib
+    from ming_univision_amd._lib import ptr
+    L = _lib.lib()
+    g = torch.Generator(device="cuda").manual_seed(M + hidden + K)
+    A, a64 = rows(g, M, K, 1, 0)
+    W = torch.empty(2 * hidden, K, dtype=torch.bfloat16, device="cuda").normal_(0, K ** -0.5, generator=g)
+    b = torch.randn(2 * hidden, device="cuda", generator=g).bfloat16()
+    Y = torch.full((2, M + 1, hidden), 3.0, dtype=torch.bfloat16, device="cuda")
+    rc = L.mn_gemm256_swiglu_split(ptr(A), K, A[0].numel(), ptr(W), K, ptr(b), ptr(Y), hidden, Y[0].numel(), M, hidden, K, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    w64 = W.double()
+    z, s = a64 @ w64.t() + b.double(), a64.abs() @ w64.abs().t() + b.double().abs()
+    gate, up = z[:, :hidden], z[:, hidden:]
+    act = torch.nn.functional.silu(gate)
+    # the sums' error through the gate (slope of silu below 1.1) and the product, the fp32 silu (8 ulp) and the pair's 2^-17
+    dz = (2 * K + 16) * 2.0 ** -24 * s
+    bound = 1.1 * dz[:, :hidden] * up.abs() + dz[:, hidden:] * act.abs() + dz[:, :hidden] * dz[:, hidden:] + (2.0 ** -20 + 2.0 ** -16.5) * (act * up).abs() + 1e-30
+    got = Y[0, :M].double() + Y[1, :M].double()
+    assert bool(((got - act * up).abs() <= bound).all()), float((got - act * up).abs().max())
+    assert bool((Y[:, M:] == 3.0).all())

@@ -35,6 +35,7 @@ struct RowsGemm {
   const bf16_t* W; int64_t ldw; const bf16_t* bias; int64_t pair;                // pair: row distance from a unit's gate to its up
   void* C; int64_t ldc; int M, N, K;
   int64_t a_lo, c_lo;                                                            // HILO: elements from a row's hi part to its lo part; split results likewise
+  int once;                                                                      // HILO: the weights are read past the caches (below)
   uint32_t tiles_m, magic;                                                       // magic: ceil(2^32 / tiles_m)
 };
 enum { R_BF16, R_GELU, R_SWIGLU, R_RESID, R_F32, R_SPLIT, R_SWIGLU_SPLIT };
@@ -66,6 +67,7 @@ __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
   constexpr int LDS = AB + S * STAGE > RED ? AB + S * STAGE : RED;
   static_assert(!(NORM && HILO) && NJ % WN == 0 && Q * 1024 * 8 == STAGE && Q * (S - 1) < 64 && LDS <= 160 * 1024, "whole fragments and instructions a wave, vmcnt range, LDS");
   __shared__ __attribute__((aligned(1024))) char lds[LDS];
+  const bool once = HILO && p.once;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kw = wave % KW, wn = wave / KW, fr = lane & 15, fq = lane >> 4;
   // an XCD's tiles are consecutive, row tiles fastest: it reads its own part of the weights, and all of the rows
@@ -121,7 +123,9 @@ __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
       const int L0 = (wave * Q + q) * RPI;             // (an instruction's rows are all of A or all of W: 16 divides BN, RPI divides 16)
       const uint32_t k = min((uint32_t)kt * ROWB + kin[q], klast);      // past K: any value, the k-step is not multiplied
       const char* s = (!NORM && L0 >= BN ? Ab : Wb) + (src[q] + k);
-      __builtin_amdgcn_global_load_lds((glb_void*)s, (lds_void*)(lds + AB + buf * STAGE + (wave * Q + q) * 1024), 16, 0, 0);
+      lds_void* d = (lds_void*)(lds + AB + buf * STAGE + (wave * Q + q) * 1024);
+      if (once && L0 < BN) __builtin_amdgcn_global_load_lds((glb_void*)s, d, 16, 0, 2);       // non-temporal
+      else __builtin_amdgcn_global_load_lds((glb_void*)s, d, 16, 0, 0);
     }
   };
   // bias and residual of this thread's 4 outputs of a group
@@ -298,11 +302,18 @@ double ln_time(const Form& f, int M, int64_t wrows, int K) {
   const double rounds = (double)mn_cdiv(form_tiles(f, M, wrows), mn_num_cus());
   return 1.9 + rounds * ((0.25 + 0.05 * f.bm) * K / 1024 + (f.bm * 4 + 32.0 * f.nj) * K / 45e3);
 }
-// Plain: 2.3 us and 68 KB/us, one round or nothing.  us, measured / this: 32 x 16 tiles of K = 1024 3.7 / 3.7, 32 x 32 of 1024 4.2 / 4.2, of 4096 9.7 / 10.0, of 8192 15.6 / 17.7, 64 x 32 of 1024
-// 5.0 / 5.2, of 8192 20.4 / 25.4, 64 x 64 of 4096 16.6 / 17.7, 64 x 128 of 2048 15.9 / 13.9, of 8192 46.7 / 48.5.
-constexpr Form forms[] = {{32, 1}, {16, 2}, {32, 2}, {32, 4}, {64, 2}, {64, 4}, {64, 8}}, hilo_forms[] = {{16, 2}, {32, 1}, {32, 2}, {32, 4}, {32, 6}, {32, 8}, {64, 2}, {64, 4}};
+// Plain: 2.3 us, and 68 KB/us of its own or 5.3 TB/s of all weights (6.2 past the caches), whichever is longer, and somewhat more where they are near
+// each other; one round or nothing.  us, measured / this: 32 x 16 tiles of K = 1024 3.7 / 3.7, 32 x 32 of 1024 4.2 / 4.2, of 4096 9.7 / 10.0, of 8192 15.6 / 17.7, 64 x 32 of 1024 5.0 / 5.2, 64 x 64 of 4096
+// 16.6 / 17.7, 64 x 128 of 2048 15.9 / 13.9, of 8192 46.7 / 48.5; hi/lo, 16384 weight rows of 3072 (100 MB): 16 x 64 17.7 .. 18.2 / 19.4, 32 x 64 19.8 .. 20.9 / 20.3, 48 x 64 22.1 .. 23.8 / 21.7.
+constexpr Form forms[] = {{32, 1}, {16, 2}, {32, 2}, {32, 4}, {64, 2}, {64, 4}, {64, 8}}, hilo_forms[] = {{16, 2}, {32, 1}, {32, 2}, {32, 4}, {32, 6}, {32, 8}, {64, 2}, {64, 4}, {16, 4}, {48, 4}};
+double own_time(const Form& f, bool hilo, int K) { return (f.bm * (hilo ? 2 : 1) + 16 * f.nj) * (double)K / 34e3; }
+// One row tile's weights nobody reads again, and where they take longer than all else they stream faster as non-temporal loads (16384 x 3072: 16 rows 20.0 -> 18.2 us, 36 rows 23.3 -> 22.1); smaller
+// ones, whose round trips count, do not: 8 rows 1024 x 4096 8.2 -> 9.9, 2304 x 768 3.9 -> 4.5.
+bool read_once(const Form& f, bool hilo, int M, int64_t wrows, int K) { return hilo && f.bm >= M && (double)wrows * K / 2.65e6 > own_time(f, hilo, K); }
 double rows_time(const Form& f, bool hilo, int M, int64_t wrows, int K) {
-  return form_tiles(f, M, wrows) > mn_num_cus() ? 1e30 : 2.3 + (f.bm * (hilo ? 2 : 1) + 16 * f.nj) * (double)K / 34e3;
+  if (form_tiles(f, M, wrows) > mn_num_cus()) return 1e30;
+  const double own = own_time(f, hilo, K), all = (double)wrows * K / (read_once(f, hilo, M, wrows, K) ? 3.1e6 : 2.65e6), hi = fmax(own, all), lo = fmin(own, all);
+  return 2.3 + hi + 0.3 * lo * lo * lo / (hi * hi);
 }
 template <int EPI>
 void go_plain(int form, const RowsGemm& p, hipStream_t st) {
@@ -326,7 +337,9 @@ void go_hilo(int form, const RowsGemm& p, hipStream_t st) {
     case 4: go<EPI, false, true, 32, 6, 4, 4>(p, st); break;
     case 5: go<EPI, false, true, 32, 8, 4, 3>(p, st); break;
     case 6: go<EPI, false, true, 64, 2, 4, 4>(p, st); break;
-    default: go<EPI, false, true, 64, 4, 4, 3>(p, st); break;
+    case 7: go<EPI, false, true, 64, 4, 4, 3>(p, st); break;
+    case 8: go<EPI, false, true, 16, 4, 8, 3>(p, st); break;
+    default: go<EPI, false, true, 48, 4, 4, 4>(p, st); break;
   }
 }
 
@@ -388,14 +401,17 @@ extern "C" int mn_rows_gemm(const mn_g256* a, int epi, double tile_us, void* str
   const bool hilo = a->a_lo_off != 0, paired = epi == MN_G256_SWIGLU_SPLIT;
   const bool known = epi == MN_G256_F32 || epi == MN_G256_F32_RESID || (hilo ? epi == MN_G256_BF16_SPLIT || paired : epi == MN_G256_BF16);
   const int64_t wrows = paired ? a->w_pair_rows + a->N : a->N, rows = paired ? 2 * (int64_t)a->N : a->N;
-  if (!known || a->g_off || a->a_rows || a->f8 || (a->w_pair_rows != 0) != paired || ((uintptr_t)a->C & (epi == MN_G256_F32 || epi == MN_G256_F32_RESID ? 15 : 7)) || a->c_lo_off % 4 || a->w_pair_rows % 4 ||
+  if (!known || a->g_off || a->a_rows || a->f8 || (a->w_pair_rows != 0) != paired ||
+      ((uintptr_t)a->C & (epi == MN_G256_F32 || epi == MN_G256_F32_RESID ? 15 : 7)) || a->c_lo_off % 4 || a->w_pair_rows % 4 ||
       !shape_ok(a->A, a->lda, a->W, a->ldw, wrows, a->bias, nullptr, a->ldc, a->M, a->N, a->K) || ((int64_t)a->M * a->lda + a->a_lo_off) * 2 >= ((int64_t)1 << 32) || a->a_lo_off % 8)
     return 0;
   double us;
-  const auto time = [&](const Form& f) { return (epi == MN_G256_SWIGLU_SPLIT && f.nj == 1) ? 1e30 : rows_time(f, hilo, a->M, rows, a->K); };
+  const auto time = [&](const Form& f) { return (paired && f.nj == 1) ? 1e30 : rows_time(f, hilo, a->M, rows, a->K); };
   const int form = hilo ? best_form(hilo_forms, time, &us) : best_form(forms, time, &us);
-  if (us >= 0.9 * tile_us) return 0;
+  const bool once = hilo && read_once(hilo_forms[form], true, a->M, rows, a->K);
+  if (us >= (once ? 0.97 : 0.9) * tile_us) return 0;      // (the tiles' estimate takes them to read as others do)
   RowsGemm p{};
+  p.once = once;
   p.A = a->A; p.lda = a->lda; p.a_lo = a->a_lo_off; p.W = a->W; p.ldw = a->ldw; p.bias = a->bias; p.pair = a->w_pair_rows; p.C = a->C; p.ldc = a->ldc; p.c_lo = a->c_lo_off;
   p.M = a->M; p.N = a->N; p.K = a->K;
   hipStream_t st = mn_stream(stream);

@@ -193,6 +193,7 @@ typedef struct mn_g256 {
   // optional device-built list of the LIVE row tiles of the grouped form (mn_moe_sort_tiles): tile t = rows
   // [tile_m0[t], +128 or 256) of group tile_g[t], *n_tiles entries, at most max_mtiles; the grid then has no empty groups
   const int32_t* tile_g; const int32_t* tile_m0; const int32_t* n_tiles; int max_mtiles;
+  int tile_rows;                                         // hi/lo rows: the list's tiles are of 32 or 64 rows (mn_gemm256_group_rows); 0: of 128 or 256
   int group_m;                                           // set by the launcher: M-tiles per band of the tile order (0: tm fastest over all M-tiles)
   int thin;                                              // set by the launcher: tile lists skip the MFMAs / fragment reads of M-fragments without a live row
   // fp8-MFMA regime (f8 != 0; labelled reduced arithmetic, never the default): A and W point to OCP e4m3 BYTES (lda / ldw / K count
@@ -211,6 +212,7 @@ enum { MN_G256_F32 = 0, MN_G256_BF16 = 1, MN_G256_BF16_GELU = 2, MN_G256_F32_RES
        MN_G256_BF16_SPLIT = 11 };                      // the fp32 result as bf16 hi rows and lo rows (c_lo_off elements further); hi/lo rows only
 extern "C" int mn_gemm256_ex(const mn_g256* a, int epi, int ksplit, void* stream);
 extern "C" int mn_gemm256_slices(int K, int ksplit);
+extern "C" int mn_gemm256_group_rows(int rows, int picks, int n_experts);
 extern "C" int mn_axpy_rms_rows_slabs(float* x, int64_t ldx, const float* y, int64_t ldy, int nz, int64_t zs, float mult, const uint16_t* w, float eps,
                                       float* n_out, int64_t ldn, uint16_t* n16, int64_t ldn16, int M, int n, void* stream);
 // rows that a producer leaves as the next product's bf16 hi and lo planes: where mn_skinny_gemm reads them (NULL: no product of three launches), that product from them, and

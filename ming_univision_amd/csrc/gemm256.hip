@@ -629,6 +629,19 @@ static bool tile_launch(const G256& p, int form, int nz, bool hilo, hipStream_t 
   }
 }
 
+// The grouped products of few rows a group: row tiles of 32 or 64 of the list, rows and K-tiles as above.
+template <int EPI, int BM, int BN, int WM, int WN, int S, int GROUP>
+static void group_go(G256 p, hipStream_t st) {
+  p.group_m = 1;                                       // (bands of four row tiles: the same to 4 % slower)
+  const dim3 grid((unsigned)(p.max_mtiles * mn_cdiv(p.N, epi_paired(EPI) ? BN / 2 : BN)));
+  hipLaunchKernelGGL((gemm_tile_kernel<EPI, true, BM, BN, WM, WN, S, false, GROUP>), grid, dim3(WM * WN * 64), 0, st, p);
+}
+template <int EPI>
+static void group_launch(const G256& p, hipStream_t st) {
+  if (p.tile_rows == 32) group_go<EPI, 32, 128, 2, 2, 3, 2>(p, st);
+  else group_go<EPI, 64, 256, 2, 4, 3, 1>(p, st);
+}
+
 // Generic launcher.  Returns the number of split-K slices used (>= 1) or a negative error.
 static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
   const bool hilo = a.a_lo_off != 0, paired = a.w_pair_rows != 0;
@@ -650,6 +663,12 @@ static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
     if (epi == E_F32) hipLaunchKernelGGL((gemm256_kernel<E_F32, false, true>), grid, dim3(512), 0, st, p);
     else hipLaunchKernelGGL((gemm256_kernel<E_SWIGLU_BF16, false, true>), grid, dim3(512), 0, st, p);
     return nz;
+  }
+  if (a.tile_g && a.tile_rows) {
+    if (!hilo || (epi != E_F32 && epi != E_SWIGLU_SPLIT) || nz > 1 || (a.tile_rows != 32 && a.tile_rows != 64)) { mn_set_error("gemm256: row tiles of %d: hi/lo rows, epilogue F32 or SWIGLU_SPLIT", a.tile_rows); return MN_EINVAL; }
+    if (epi == E_F32) group_launch<E_F32>(p, st);
+    else group_launch<E_SWIGLU_SPLIT>(p, st);
+    return 1;
   }
   // (the 256-tile kernel's GELU is the 1.5e-7 polynomial: it serves the problems of 128 tiles and more, where erff in the small tiles' epilogue costs more than they save:
   // 4096 x 4096 x 256 26.9 us against 38.6, 8000 x 4000 x 192 45 against 69)
@@ -719,6 +738,15 @@ extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo) {
     if (t < tb - 1e-9) { tb = t; best = ks; }
   }
   return best > 1 ? best : 0;
+}
+
+// Row tile of the grouped hi/lo products of `rows` rows with `picks` of `n_experts` groups each (0: the 128 rows of the 256-tile kernel's).  That kernel brings in 128 rows' operands
+// for every 128 weight rows whatever is live, one workgroup a CU: 792 of them are four rounds of 256 CUs.  us, gate and up / down of a 64-expert layer, 256-tile kernel -> this: 70 rows
+// 153 / 90 -> 135 / 67, 100 154 / 93 -> 140 / 70, 170 156 / 90 -> 147 / 76, 260 177 / 93 -> 171 / 91 (32); 350 180 / 98 -> 176 / 93, 500 189 / 111 -> 182 / 99, 600 202 / 115 -> 181 / 105 (64);
+// 650 stays (192 / 112; 202 / 116).
+extern "C" int mn_gemm256_group_rows(int rows, int picks, int n_experts) {
+  const int64_t per = (int64_t)rows * picks;
+  return per <= 25 * (int64_t)n_experts ? 32 : per <= 57 * (int64_t)n_experts ? 64 : 0;
 }
 
 // slices mn_gemm256_ex will use for a ksplit request (whole pairs of K-tiles per slice)

@@ -27,11 +27,14 @@ __device__ __forceinline__ void wait_tiles(int rem) {
   }
 }
 
-template <int EPI, bool HILO, int BM, int BN, int WM, int WN, int S, bool TWO = false>
+// GROUP: the products of groups of rows with weights of their own (MoE experts), row tiles of BM from a device-built list.  2: the weights are read past the caches, where a group
+// is seldom more than one row tile: nobody reads them again, and lines that are let go at once stream faster (66 experts' 5632 x 2048 / 2048 x 1408 of 100 rows in tiles of
+// 32 x 128, 6 picks a row and two for all: 146 -> 140 us / 74 -> 70, 70 rows 146 -> 135 / 73 -> 67, 5.6 TB/s; 240 rows, where a third of the groups are two tiles, 162 -> 165 / 87 -> 89).
+template <int EPI, bool HILO, int BM, int BN, int WM, int WN, int S, bool TWO = false, int GROUP = 0>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
   constexpr int NW = WM * WN, AR = HILO ? 2 * BM : BM, QA = AR / 8 / NW, QW = BN / 8 / NW, STAGE = (AR + BN) * 128;
   constexpr int MI = BM / WM / 16, NJ = BN / WN / 16, AI = HILO ? 2 * MI : MI;
-  constexpr bool paired = epi_paired(EPI);
+  constexpr bool paired = epi_paired(EPI), GROUPED = GROUP != 0;
   constexpr bool quads = paired && NJ == 1;            // gate and up of a unit within one fragment: a lane's 4 columns are 2 gates, then their 2 ups
   static_assert(QA * 8 * NW == AR && QW * 8 * NW == BN && MI >= 1 && NJ >= 1 && (!quads || EPI == E_SWIGLU_SPLIT), "whole instructions and fragments per wave");
   static_assert((QA + QW) * (S - 2) < 64 && S * STAGE <= 160 * 1024, "vmcnt range, LDS");
@@ -42,12 +45,29 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
   constexpr int cols = paired ? BN / 2 : BN;
   const int tiles_m = (p.M + BM - 1) / BM;
   // XCD-aware order: an XCD's tiles are consecutive, row tiles fastest, so each XCD reads its own part of the weights and all of the rows
-  int bid = blockIdx.x;
+  int bid = blockIdx.x, nt = gridDim.x, nl = 0;
+  const int tiles_n = (p.N + cols - 1) / cols;
+  if constexpr (GROUPED) {
+    nl = *p.n_tiles;
+    nt = min(nt, nl * tiles_n);                        // the live tiles
+    if (bid >= nt) return;                             // uniform
+  }
   {
-    const int nt = gridDim.x, q = nt / 8, r = nt % 8, xcd = bid % 8, idx = bid / 8;
+    const int q = nt / 8, r = nt % 8, xcd = bid % 8, idx = bid / 8;
     bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + idx;
   }
-  const int m0 = (bid % tiles_m) * BM, n0 = (bid / tiles_m) * cols;
+  int m0, n0, row0 = 0, Mg = p.M, grp = 0;
+  if constexpr (GROUPED) {                             // bands of group_m row tiles of the list, row tile fastest
+    const int gb = p.group_m, band = bid / (gb * tiles_n), first = band * gb, r = bid - band * gb * tiles_n, gsz = min(nl - first, gb), t = first + r % gsz;
+    grp = p.tile_g[t];
+    m0 = p.tile_m0[t];
+    n0 = r / gsz * cols;
+    row0 = p.g_off[grp];
+    Mg = p.g_cnt[grp];
+  } else {
+    m0 = (bid % tiles_m) * BM;
+    n0 = (bid / tiles_m) * cols;
+  }
   const int kbeg = blockIdx.y * p.Kc, kend = min(p.K, kbeg + p.Kc);
   const int nk = (kend - kbeg) / BK;
 
@@ -57,7 +77,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
 #pragma unroll
   for (int q = 0; q < QA; ++q) {
     const int L = (wave * QA + q) * 8 + rin;
-    const int gm = min(m0 + (HILO && L >= BM ? L - BM : L), p.M - 1);
+    int gm = row0 + min(m0 + (HILO && L >= BM ? L - BM : L), Mg - 1);
+    if (GROUPED && p.a_rows) gm = p.a_rows[gm];
     srcA[q] = (uint32_t)(((int64_t)gm * p.lda + (HILO && L >= BM ? p.a_lo_off : 0) + kbeg) * 2 + (((lane & 7) ^ ((L >> 1) & 7)) << 4));
   }
 #pragma unroll
@@ -76,13 +97,13 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
     srcW[q] = (uint32_t)(((int64_t)gn * p.ldw + kbeg) * 2 + (((lane & 7) ^ ((L >> 1) & 7)) << 4));
   }
   const char* Ab = reinterpret_cast<const char*>(p.A);
-  const char* Wb = reinterpret_cast<const char*>(p.W);
+  const char* Wb = reinterpret_cast<const char*>(p.W) + (GROUPED ? (int64_t)grp * p.w_gstride * 2 : 0);
   auto stage = [&](int kt, int buf) {
     const uint32_t koff = (uint32_t)kt * (BK * 2);
     char* dst = &lds[buf * STAGE];
 #pragma unroll
     for (int q = 0; q < QW; ++q)
-      __builtin_amdgcn_global_load_lds((glb_void*)(Wb + (srcW[q] + koff)), (lds_void*)(dst + AR * 128 + (wave * QW + q) * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((glb_void*)(Wb + (srcW[q] + koff)), (lds_void*)(dst + AR * 128 + (wave * QW + q) * 1024), 16, 0, GROUP == 2 ? 2 : 0);
 #pragma unroll
     for (int q = 0; q < QA; ++q)
       __builtin_amdgcn_global_load_lds((glb_void*)(Ab + (srcA[q] + koff)), (lds_void*)(dst + (wave * QA + q) * 1024), 16, 0, 0);
@@ -113,6 +134,11 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
     __builtin_amdgcn_sched_barrier(0);
     if (t + S - 1 < nk) stage(t + S - 1, nbuf);
     const char* a = &lds[buf * STAGE + wm * (BM / WM) * 128];
+    if (GROUPED && m0 + wm * (BM / WM) >= Mg) {          // uniform: no row of this wave is live
+      buf = buf + 1 == S ? 0 : buf + 1;
+      nbuf = nbuf + 1 == S ? 0 : nbuf + 1;
+      continue;
+    }
     const char* w = &lds[buf * STAGE + AR * 128 + wn * (BN / WN) * 128];
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -164,7 +190,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
     return;
   }
   g256_out<EPI, true, false, MI, paired ? (NJ + 1) / 2 : NJ>(
-      p, Cz, blockIdx.y, 0, p.M, 0, [&](int i) { return m0 + wm * (BM / WM) + i * 16 + fr; }, [&](int j) { return n0 + wn * (cols / WN) + j * 16 + fq * 4; },
+      p, Cz, blockIdx.y, row0, Mg, grp, [&](int i) { return m0 + wm * (BM / WM) + i * 16 + fr; }, [&](int j) { return n0 + wn * (cols / WN) + j * 16 + fq * 4; },
       [&](int i, int j, f32x4& v, f32x4& u) {
         v = acc[i][j];
         if (HILO) v += acc[(i + MI) % AI][j];

@@ -50,6 +50,7 @@ struct LlmWideWs {
   bf16_t *wq_gu, *wq_dn;           // weight-only modes: ONE layer's expert weights de-quantised, [G][2 I][H] / [G][H][I] (wide_rf.inl)
   uint8_t* yh8; float *s_h, *s_y2; // fp8-MFMA regime: the experts' e4m3 operand [rows][H] + its row scales, the down projection's row scales [P]
   int32_t *ti, *cnt, *off, *perm, *slot_of, *tile_g, *tile_m0, *n_tiles;
+  int tile_rows;
   int max_mtiles;
   void* attn_ws;
   size_t attn_ws_bytes;
@@ -59,7 +60,7 @@ struct LlmWideWs {
 static bool llm_wide_ok(const mn_llm* m, int rows) {
   const int ad = m->n_q * m->head_dim, n_slot = m->top_k + m->n_shared_slots;
   const bool fmt_ok = m->wfmt == MN_W_BF16 || ((m->wfmt == MN_W_FP8_E4M3 || m->wfmt == MN_W_INT8 || m->wfmt == MN_W_NF4) && m->w_gate_up_scale && m->w_down_scale);
-  return fmt_ok && rows >= g_wide_min_llm && rows <= 2048 && wide_glue_ok(m->hidden) && (m->hidden % 64) == 0 && (ad % 64) == 0 && (m->moe_inter % 64) == 0 &&
+  return fmt_ok && rows >= (m->wfmt == MN_W_BF16 ? g_wide_min_llm : g_wide_min_llm_wq) && rows <= 2048 && wide_glue_ok(m->hidden) && (m->hidden % 64) == 0 && (ad % 64) == 0 && (m->moe_inter % 64) == 0 &&
          m->n_experts <= 64 && (m->n_experts % 4) == 0 && m->n_experts + m->n_shared_slots <= 128 && (int64_t)rows * n_slot <= 65536 &&
          (m->head_dim == 64 || m->head_dim == 128);
 }
@@ -96,7 +97,9 @@ static size_t llm_wide_carve(const mn_llm* m, int rows, int64_t t_max, void* ws,
   o->off = cv.take<int32_t>((size_t)G + 1);
   o->perm = cv.take<int32_t>(P);
   o->slot_of = cv.take<int32_t>(P);
-  o->max_mtiles = (int)(P / 128) + G;                   // sum_g ceil(cnt_g / 128) <= P / 128 + G
+  // (rows of plain bf16 or e4m3 operands keep the 256-tile kernel's list)
+  o->tile_rows = lo_at(LO_LLM_EXPERTS, 1) && !llm_f8_mfma(m) ? mn_gemm256_group_rows(rows, m->top_k, m->n_experts) : 0;
+  o->max_mtiles = (int)(P / (o->tile_rows ? o->tile_rows : 128)) + G;      // sum_g ceil(cnt_g / r) <= P / r + G
   o->tile_g = cv.take<int32_t>((size_t)o->max_mtiles);
   o->tile_m0 = cv.take<int32_t>((size_t)o->max_mtiles);
   o->n_tiles = cv.take<int32_t>(4);
@@ -188,7 +191,7 @@ static int llm_step_wide(const mn_llm* m, const float* x, int64_t ldx, int x_row
     hipLaunchKernelGGL(moe_topk_partials_kernel, dim3(mn_cdiv(M, 4)), dim3(256), 0, st, (const float*)w.pp, p_img, image_mask, nz,
                        (int64_t)M * E, M, E, m->top_k, m->norm_topk_prob, m->n_shared_slots, w.ti, w.tw);
     route_capture(l, w.ti, M, n_slot, st);
-    MN_TRY(mn_moe_sort_tiles(w.ti, M, n_slot, G, w.cnt, w.off, w.perm, w.slot_of, (lo_at(LO_LLM_EXPERTS, 1) && !f8) ? 128 : 256, w.tile_g, w.tile_m0,
+    MN_TRY(mn_moe_sort_tiles(w.ti, M, n_slot, G, w.cnt, w.off, w.perm, w.slot_of, w.tile_rows ? w.tile_rows : (lo_at(LO_LLM_EXPERTS, 1) && !f8) ? 128 : 256, w.tile_g, w.tile_m0,
                              w.n_tiles, stream));
     if (f8) {
       // fp8-MFMA regime: gate/up = e4m3(RMSNorm'd row, gathered by perm) x e4m3 expert bytes, SwiGLU in the epilogue -> bf16 [P, I];
@@ -222,11 +225,11 @@ static int llm_step_wide(const mn_llm* m, const float* x, int64_t ldx, int x_row
     a = g256_hilo(w.yh, H, lo_at(LO_LLM_EXPERTS, (int64_t)M * H), wgu, H, nullptr, w.y2, I, M, I, H);
     a.w_pair_rows = I; a.c_lo_off = P * I;
     a.g_off = w.off; a.g_cnt = w.cnt; a.w_gstride = (int64_t)2 * I * H; a.a_rows = w.perm; a.n_groups = G;
-    a.tile_g = w.tile_g; a.tile_m0 = w.tile_m0; a.n_tiles = w.n_tiles; a.max_mtiles = w.max_mtiles;
+    a.tile_g = w.tile_g; a.tile_m0 = w.tile_m0; a.n_tiles = w.n_tiles; a.max_mtiles = w.max_mtiles; a.tile_rows = w.tile_rows;
     MN_TRYZ(mn_gemm256_ex(&a, MN_G256_SWIGLU_SPLIT, 1, stream));
     a = g256_hilo(w.y2, I, lo_at(LO_LLM_EXPERTS, P * I), wdn, I, nullptr, w.yg, H, M, H, I);
     a.g_off = w.off; a.g_cnt = w.cnt; a.w_gstride = (int64_t)H * I; a.n_groups = G;
-    a.tile_g = w.tile_g; a.tile_m0 = w.tile_m0; a.n_tiles = w.n_tiles; a.max_mtiles = w.max_mtiles;
+    a.tile_g = w.tile_g; a.tile_m0 = w.tile_m0; a.n_tiles = w.n_tiles; a.max_mtiles = w.max_mtiles; a.tile_rows = w.tile_rows;
     MN_TRYZ(mn_gemm256_ex(&a, MN_G256_F32, 1, stream));
   }
   MN_CHECK_LAUNCH("mn_llm_step(wide)");

@@ -311,7 +311,7 @@ __device__ __forceinline__ void f32_store(const GemmF32& a, int z, int m, int n,
   if (a.C16) a.C16[(int64_t)z * a.c16_bs + (int64_t)m * a.ldc16 + n] = f32_to_bf16(v);
 }
 
-// More than 8 rows run on the fp32 matrix cores (v_mfma_f32_16x16x4f32: lane l holds row / column l & 15), fp32 rows and bf16 weights
+// More than 2 rows (8 where accesses go value by value) run on the fp32 matrix cores (v_mfma_f32_16x16x4f32: lane l holds row / column l & 15), fp32 rows and bf16 weights
 // widened on the way.  Both kernels give lane l the values 4 (l >> 4) .. + 3 of every 16 of K, so the four products of a 16-step take
 // one 16-byte read of each operand, in an order of K that both share.  Values past K enter as zeros.  V4: rows of A are 16-byte, rows
 // of W 8-byte aligned; else value by value.
@@ -319,7 +319,7 @@ __device__ __forceinline__ void f32_store(const GemmF32& a, int z, int m, int n,
 // Few tiles: 32 x 16 outputs a workgroup, whose four waves split K; operands straight from memory, the next 32 values in flight during
 // the products.  Latency bounds it (32 rows x 16 heads of 512 x 128: 5 us here, 45 us as one wave a column and 8 rows).  A block of 32
 // values is summed as a tree of single products and added to the running sum with its rounding error kept (two-sum), so the
-// result is as close to the exact sum as the tree over 64 lanes that <= 8 rows take (0.22e-7 and 0.46e-7 of the summed magnitudes at K 512).
+// result is as close to the exact sum as the tree over 64 lanes that one or two rows take (0.22e-7 and 0.46e-7 of the summed magnitudes at K 512).
 template <bool V4>
 __global__ __launch_bounds__(256) void gemm_f32_few_kernel(GemmF32 a) {
   __shared__ float red[4][16][64];
@@ -1008,16 +1008,18 @@ extern "C" int mn_gemm_f32_batched(const float* A, int64_t lda, int64_t a_bs, co
   MN_CHECK_ARG(A && W && (C || C16) && M >= 1 && N >= 1 && K >= 1 && batch >= 1 && batch <= 65535, "mn_gemm_f32_batched: bad args");
   GemmF32 a{A, lda, a_bs, W, ldw, w_bs, bias, C, ldc, c_bs, C16, ldc16, c16_bs, G, ldg, g_bs, M, N, K, alpha};
   hipStream_t st = mn_stream(stream);
-  if (M <= 8) {                                          // a few rows: one wave a column, lanes over K
+  const bool v4 = (K % 4) == 0 && (lda % 4) == 0 && (a_bs % 4) == 0 && ((uintptr_t)A & 15) == 0 && (ldw % 4) == 0 && (w_bs % 4) == 0 && ((uintptr_t)W & 7) == 0;
+  // One wave a column, lanes over K: one or two rows, and up to 8 value by value.  Its time grows with the rows, the matrix cores' does not.  us, this / those: 16 x 128 x 512 2 rows 4.4 / 5.9,
+  // 3 6.0 / 6.0, 6 8.3 / 6.0, 8 10.0 / 6.0; 16 x 512 x 128 2 rows 3.5 / 4.1, 3 4.5 / 4.1, 8 6.4 / 4.2; 2048 x 1024 3 rows 12.3 / 10.1, 8 19.6 / 10.1; value by value 64 x 4096 8 rows 57 / 73.  Error 0.8 .. 1.8e-7 / 0.7e-7.
+  if (M <= (v4 ? 2 : 8)) {
     if (M <= 2) hipLaunchKernelGGL((gemv_f32_kernel<2>), dim3((unsigned)mn_cdiv(N, 4), 1, (unsigned)batch), dim3(256), 0, st, a);
     else hipLaunchKernelGGL((gemv_f32_kernel<8>), dim3((unsigned)mn_cdiv(N, 4), 1, (unsigned)batch), dim3(256), 0, st, a);
     MN_CHECK_LAUNCH("mn_gemm_f32_batched");
     return MN_OK;
   }
   MN_CHECK_ARG(mn_cdiv(M, 64) <= 65535, "mn_gemm_f32_batched: too many rows");
-  const bool v4 = (K % 4) == 0 && (lda % 4) == 0 && (a_bs % 4) == 0 && ((uintptr_t)A & 15) == 0 && (ldw % 4) == 0 && (w_bs % 4) == 0 && ((uintptr_t)W & 7) == 0;
   const int64_t tiles = mn_cdiv(M, 64) * mn_cdiv(N, 64) * batch;
-  // 9 .. 64 rows always take the kernel that keeps its roundings (they are decode rows: error against 64 bits 0.2 .. 0.6e-7 of the summed
+  // up to 64 rows always take the kernel that keeps its roundings (they are decode rows: error against 64 bits 0.2 .. 0.6e-7 of the summed
   // magnitudes, the tiles' 2e-7).  More rows: 128 tiles are the break-even (256 rows x 16 x 128 x 512: 17 us either way; 128 rows x 16 x 512 x 128, 256
   // tiles: 10.6 and 7.3 us; 2048 rows x 4096 x 1024: 354 and 168 us, 292 us on FMA tiles before)
   if (M <= 64 || 2 * tiles < mn_num_cus()) {

@@ -295,7 +295,7 @@ class BailingMoeDecoder:
 
     def step(self, x, row_seq, row_slot, row_pos, row_len, key_mask=None, image_mask=None, out=None, rows=None,
              x_row_div=1, distinct_sequences=False, spans=None):
-        """One pass of the 28-layer stack over a few rows (weight-streaming kernels; up to 39 with bf16 weights, 64 with others) or up to 2048 (wide route).
+        """One pass of the 28-layer stack over M <= 64 rows (weight-streaming kernels) or 65..2048 rows (wide route).
         x fp32 [M,H]; or [1,H] with rows=M to broadcast; or [M / x_row_div, H] with rows=M when the x_row_div CFG
         rows of an image share one embedding.  int32 device arrays per row; key_mask uint8 [M, >=len].
         distinct_sequences: every row is a different cache sequence and row_len == row_slot + 1 (a decode step, not a prefill

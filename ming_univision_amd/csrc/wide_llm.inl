@@ -60,7 +60,7 @@ struct LlmWideWs {
 static bool llm_wide_ok(const mn_llm* m, int rows) {
   const int ad = m->n_q * m->head_dim, n_slot = m->top_k + m->n_shared_slots;
   const bool fmt_ok = m->wfmt == MN_W_BF16 || ((m->wfmt == MN_W_FP8_E4M3 || m->wfmt == MN_W_INT8 || m->wfmt == MN_W_NF4) && m->w_gate_up_scale && m->w_down_scale);
-  return fmt_ok && rows >= (m->wfmt == MN_W_BF16 ? g_wide_min_llm : g_wide_min_llm_wq) && rows <= 2048 && wide_glue_ok(m->hidden) && (m->hidden % 64) == 0 && (ad % 64) == 0 && (m->moe_inter % 64) == 0 &&
+  return fmt_ok && rows >= g_wide_min_llm && rows <= 2048 && wide_glue_ok(m->hidden) && (m->hidden % 64) == 0 && (ad % 64) == 0 && (m->moe_inter % 64) == 0 &&
          m->n_experts <= 64 && (m->n_experts % 4) == 0 && m->n_experts + m->n_shared_slots <= 128 && (int64_t)rows * n_slot <= 65536 &&
          (m->head_dim == 64 || m->head_dim == 128);
 }

@@ -14,14 +14,13 @@
 // and the launches between them do not (26.6 + 5.5 us).  A sampler call, streaming kernels against tiles, ms: 4 rows 7.57 / 7.76, 5 rows 8.29 / 7.73, 8 rows
 // 8.41 / 7.80, 16 rows 8.92 / 8.07, 24 rows 10.23 / 8.47, 36 rows 12.40 / 9.94, 64 rows 13.50 / 11.66 (with 64-row tiles alone the line was 24 rows).
 // Weight-only formats are expanded to bf16 once per call on this route and keep their line at 41.
-// The semantic decoder likewise beyond the 32 rows whose projections are one launch (a token of 64 rows 22.8 -> 22.3 ms); the language model's
-// experts leave the streaming kernels at 40 rows: their tiles (mn_gemm256_group_rows) write one fp32 result, gated already, where those write slabs.  us a step, streaming / tiles: rows of
-// sequences of their own 24 6995 / 6956, 33 7039 / 7108, 40 7272 / 7192, 48 7337 / 7307, 64 of 1100 tokens 8587 / 8542; a prompt of 20 rows 6530 / 6554, of 50 8138 / 7316.  Weight-only formats, expanded a
-// layer at a time, and e4m3 products keep their line at 65.
-static int g_wide_min_llm = 40, g_wide_min_llm_wq = 65, g_wide_min_rf = 5, g_wide_min_rf_w8 = 41, g_wide_min_sem = 33;
+// The semantic decoder likewise beyond the 32 rows whose projections are one launch (a token of 64 rows 22.8 -> 22.3 ms); the language model
+// keeps the streaming kernels up to 64 rows: the steps are as fast (rows of sequences of their own 40 7272 / 7192 us, 64 of 1100 tokens 8587 / 8542) and its router's logits are fp32 products there,
+// hi/lo ones here (hidden states of 48 rows against 64 bits 2.49e-6 / 2.51e-6).
+static int g_wide_min_llm = 65, g_wide_min_rf = 5, g_wide_min_rf_w8 = 41, g_wide_min_sem = 33;
 #ifdef MN_DEV_HOOKS
 extern "C" MN_DEV_API void mn_wide_tune(int llm_min_rows, int rf_min_rows, int sem_min_rows) {
-  if (llm_min_rows > 0) g_wide_min_llm = g_wide_min_llm_wq = llm_min_rows;
+  if (llm_min_rows > 0) g_wide_min_llm = llm_min_rows;
   if (rf_min_rows > 0) g_wide_min_rf = g_wide_min_rf_w8 = rf_min_rows;
   if (sem_min_rows > 0) g_wide_min_sem = sem_min_rows;
 }

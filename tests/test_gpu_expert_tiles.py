@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("hidden,inter,experts,top,shared,counts", [
-    (1024, 1408, 64, 6, 2, (40, 64, 65, 266, 267)), (256, 192, 8, 2, 1, (40, 100, 101, 228, 229)), (512, 320, 12, 12, 1, (40, 57, 65)), (256, 64, 16, 1, 0, (40, 129))])
+    (1024, 1408, 64, 6, 2, (65, 100, 266, 267)), (256, 192, 8, 2, 1, (65, 100, 101, 228, 229)), (512, 320, 12, 12, 1, (65, 80)), (256, 64, 16, 1, 0, (65, 129))])
 def test_rows_together_and_in_parts(hidden, inter, experts, top, shared, counts):
     from ming_univision_amd import configuration as C
     from ming_univision_amd._lib import check, lib, ptr

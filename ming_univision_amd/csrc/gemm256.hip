@@ -594,10 +594,10 @@ static int tile_form(int M, int N, int Kc, int nz, bool hilo, int epi, bool may2
   return best;
 }
 
-template <int EPI, int BM, int BN, int WM, int WN, int S, bool HILO, bool TWO = false>
+template <int EPI, int BM, int BN, int WM, int WN, int S, bool HILO, bool TWO = false, int GROUP = 0>
 static void tile_go(const G256& p, int nz, hipStream_t st) {
   const dim3 grid((unsigned)(mn_cdiv(p.M, BM) * mn_cdiv(p.N, epi_paired(EPI) ? BN / 2 : BN)), nz);
-  hipLaunchKernelGGL((gemm_tile_kernel<EPI, HILO, BM, BN, WM, WN, S, TWO>), grid, dim3(WM * WN * 64), 0, st, p);
+  hipLaunchKernelGGL((gemm_tile_kernel<EPI, HILO, BM, BN, WM, WN, S, TWO, GROUP>), grid, dim3(WM * WN * 64), 0, st, p);
 }
 
 // stages: as many K-tiles as leave room for two workgroups of the 64-row forms on a CU (64 x 64 hi/lo: 3 x 24 KiB; 64 x 128: 3 x 24, hi/lo
@@ -630,16 +630,16 @@ static bool tile_launch(const G256& p, int form, int nz, bool hilo, hipStream_t 
 }
 
 // The grouped products of few rows a group: row tiles of 32 or 64 of the list, rows and K-tiles as above.
-template <int EPI, int BM, int BN, int WM, int WN, int S, int GROUP>
+template <int EPI, int BM, int BN, int WM, int WN, int S, bool TWO, int GROUP>
 static void group_go(G256 p, hipStream_t st) {
   p.group_m = 1;                                       // (bands of four row tiles: the same to 4 % slower)
   const dim3 grid((unsigned)(p.max_mtiles * mn_cdiv(p.N, epi_paired(EPI) ? BN / 2 : BN)));
-  hipLaunchKernelGGL((gemm_tile_kernel<EPI, true, BM, BN, WM, WN, S, false, GROUP>), grid, dim3(WM * WN * 64), 0, st, p);
+  hipLaunchKernelGGL((gemm_tile_kernel<EPI, true, BM, BN, WM, WN, S, TWO, GROUP>), grid, dim3(WM * WN * 64), 0, st, p);
 }
 template <int EPI>
 static void group_launch(const G256& p, hipStream_t st) {
-  if (p.tile_rows == 32) group_go<EPI, 32, 128, 2, 2, 3, 2>(p, st);
-  else group_go<EPI, 64, 256, 2, 4, 3, 1>(p, st);
+  if (p.tile_rows == 32) group_go<EPI, 32, 128, 2, 2, 3, true, 2>(p, st);
+  else group_go<EPI, 64, 256, 2, 4, 3, false, 1>(p, st);
 }
 
 // Generic launcher.  Returns the number of split-K slices used (>= 1) or a negative error.
@@ -675,6 +675,14 @@ static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
   const bool may256 = epi != E_BF16_GELU || mn_cdiv(p.M, 256) * mn_cdiv(p.N, 256) >= 128;
   double us = 0;
   const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : epi == E_BF16_GELU && may256 ? 0 : tile_form(p.M, p.N, p.Kc, nz, hilo, epi, may256, &us);
+  // one row tile of a matrix that no cache holds (a vocabulary's logits): us at 126464 x 2048, the tiles below -> this: 5 rows 110 -> 86, 16 108 -> 91, 24 112 -> 98, 32 114 -> 102 (64 x 256 tiles
+  // like this 40 rows 118 -> 115, 64 129 -> 121; in the caches' reach the tiles below: 16384 x 3072 17 .. 20, this 23 .. 30)
+  if (us > 0 && nz == 1 && hilo && epi == E_F32 && a.M <= 64 && (int64_t)a.N * a.K * 2 >= (int64_t)256 << 20) {
+    if (a.M <= 16) tile_go<E_F32, 16, 128, 1, 4, 4, true, true, 3>(p, nz, st);
+    else if (a.M <= 32) tile_go<E_F32, 32, 128, 2, 2, 3, true, true, 3>(p, nz, st);
+    else tile_go<E_F32, 64, 256, 2, 4, 3, true, true, 3>(p, nz, st);
+    return 1;
+  }
   if (us > 0 && nz == 1 && mn_rows_gemm(&p, epi, us, st)) return 1;       // few tiles: forms whose waves split K (rows_gemm.hip)
 #define G256_GO(E)                                                                          \
   do {                                                                                      \

@@ -27,14 +27,15 @@ __device__ __forceinline__ void wait_tiles(int rem) {
   }
 }
 
-// GROUP: the products of groups of rows with weights of their own (MoE experts), row tiles of BM from a device-built list.  2: the weights are read past the caches, where a group
-// is seldom more than one row tile: nobody reads them again, and lines that are let go at once stream faster (66 experts' 5632 x 2048 / 2048 x 1408 of 100 rows in tiles of
-// 32 x 128, 6 picks a row and two for all: 146 -> 140 us / 74 -> 70, 70 rows 146 -> 135 / 73 -> 67, 5.6 TB/s; 240 rows, where a third of the groups are two tiles, 162 -> 165 / 87 -> 89).
+// GROUP 1, 2: the products of groups of rows with weights of their own (MoE experts), row tiles of BM from a device-built list.  2 and 3 (one dense product): the weights are read past
+// the caches, where all rows, or most groups, are one row tile: nobody reads them again, and lines that are let go at once stream faster (66 experts' 5632 x 2048 / 2048 x 1408 of 100
+// rows in tiles of 32 x 128, 6 picks a row and two for all: 146 -> 140 us / 74 -> 70, 70 rows 146 -> 135 / 73 -> 67, 5.6 TB/s; 240 rows, where a third of the groups are two tiles, 162 -> 165 /
+// 87 -> 89).
 template <int EPI, bool HILO, int BM, int BN, int WM, int WN, int S, bool TWO = false, int GROUP = 0>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
   constexpr int NW = WM * WN, AR = HILO ? 2 * BM : BM, QA = AR / 8 / NW, QW = BN / 8 / NW, STAGE = (AR + BN) * 128;
   constexpr int MI = BM / WM / 16, NJ = BN / WN / 16, AI = HILO ? 2 * MI : MI;
-  constexpr bool paired = epi_paired(EPI), GROUPED = GROUP != 0;
+  constexpr bool paired = epi_paired(EPI), GROUPED = GROUP == 1 || GROUP == 2;
   constexpr bool quads = paired && NJ == 1;            // gate and up of a unit within one fragment: a lane's 4 columns are 2 gates, then their 2 ups
   static_assert(QA * 8 * NW == AR && QW * 8 * NW == BN && MI >= 1 && NJ >= 1 && (!quads || EPI == E_SWIGLU_SPLIT), "whole instructions and fragments per wave");
   static_assert((QA + QW) * (S - 2) < 64 && S * STAGE <= 160 * 1024, "vmcnt range, LDS");
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
     char* dst = &lds[buf * STAGE];
 #pragma unroll
     for (int q = 0; q < QW; ++q)
-      __builtin_amdgcn_global_load_lds((glb_void*)(Wb + (srcW[q] + koff)), (lds_void*)(dst + AR * 128 + (wave * QW + q) * 1024), 16, 0, GROUP == 2 ? 2 : 0);
+      __builtin_amdgcn_global_load_lds((glb_void*)(Wb + (srcW[q] + koff)), (lds_void*)(dst + AR * 128 + (wave * QW + q) * 1024), 16, 0, GROUP >= 2 ? 2 : 0);
 #pragma unroll
     for (int q = 0; q < QA; ++q)
       __builtin_amdgcn_global_load_lds((glb_void*)(Ab + (srcA[q] + koff)), (lds_void*)(dst + (wave * QA + q) * 1024), 16, 0, 0);

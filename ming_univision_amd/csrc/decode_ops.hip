@@ -230,13 +230,12 @@ extern "C" MN_DEV_API void mn_moe_router_tune(int max_rows) { g_router_rows = ma
 // top-k — one launch.  A row is a workgroup, which reads the gate (256 KB at 64 x 2048) and its slabs (131 KB) from its XCD's L2: 10.7 us at 64 rows (11.8 with eight slabs a round
 // trip and the norm's weights behind the sum; 2 rows 11.0 -> 9.9), where the norm, the gate's product and a one-workgroup top-k and sort took 6 + 5 + 13.
 bool moe_router_rows_ok(int M, int H, int E) { return M >= 1 && M <= 64 && H <= 4096 && (H % 8) == 0 && E <= 64; }
-int moe_router_rows(float* h, const float* P, int nz, const uint16_t* norm_w, float eps, const uint16_t* gate_w, int M, int H, int E, int top_k,
-                    int norm_topk_prob, int n_shared_slots, float* x_norm, uint16_t* y, int32_t* topk_idx, float* topk_w, float* logits_ws, void* stream) {
+int moe_router_rows(float* h, const float* P, int nz, const uint16_t* norm_w, float eps, const uint16_t* gate_w, const uint16_t* image_gate_w, const uint8_t* image_mask, int M,
+                    int H, int E, int top_k, int norm_topk_prob, int n_shared_slots, float* x_norm, uint16_t* y, int32_t* topk_idx, float* topk_w, float* logits_ws, void* stream) {
   MN_CHECK_ARG(h && P && norm_w && gate_w && (x_norm || y) && topk_idx && topk_w && logits_ws && moe_router_rows_ok(M, H, E) && top_k >= 1 && top_k <= E &&
                top_k + n_shared_slots <= 64, "moe_router_rows: bad args");
   hipLaunchKernelGGL(moe_router_row_kernel, dim3(M), dim3(1024), 0, mn_stream(stream), (const float*)h, (int64_t)H, norm_w, eps, gate_w,
-                     (const bf16_t*)nullptr, (const uint8_t*)nullptr, M, H, E, top_k, norm_topk_prob, n_shared_slots, x_norm, topk_idx, topk_w,
-                     logits_ws, P, nz, (int64_t)M * H, h, y);
+                     image_gate_w, image_mask, M, H, E, top_k, norm_topk_prob, n_shared_slots, x_norm, topk_idx, topk_w, logits_ws, P, nz, (int64_t)M * H, h, y);
   MN_CHECK_LAUNCH("moe_router_rows");
   return MN_OK;
 }

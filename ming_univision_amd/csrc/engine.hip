@@ -1034,7 +1034,7 @@ static bool moe_mfma_ok(const mn_llm* m, int rows) {
 static int g_chain_max_rows = 64, g_chain_fuse_ln1 = 1;
 static int g_moe_gate_up = 1, g_moe_gate_up_rows = 1, g_moe_gate_up_chain_rows = 2, g_moe_gate_up_chain_all = 0;      // (chain: int8 / NF4 by default — bf16 / e4m3 keep the pair launches: 2.25 vs 2.64 ms, 1.71 vs 1.84)      // the one-launch router + gate/up of 1-row steps (dev-library A/B: mn_moe_tune_gate_up)
 bool moe_router_rows_ok(int M, int H, int E);
-int moe_router_rows(float* h, const float* P, int nz, const uint16_t* norm_w, float eps, const uint16_t* gate_w, int M, int H, int E, int top_k,
+int moe_router_rows(float* h, const float* P, int nz, const uint16_t* norm_w, float eps, const uint16_t* gate_w, const uint16_t* image_gate_w, const uint8_t* image_mask, int M, int H, int E, int top_k,
                     int norm_topk_prob, int n_shared_slots, float* x_norm, uint16_t* y, int32_t* topk_idx, float* topk_w, float* logits_ws, void* stream);
 #ifdef MN_DEV_HOOKS
 extern "C" MN_DEV_API void mn_moe_tune_gate_up(int on, int max_rows) { g_moe_gate_up = on; g_moe_gate_up_rows = max_rows & 0xff; g_moe_gate_up_chain_rows = (max_rows >> 8) & 0xff; g_moe_gate_up_chain_all = (max_rows >> 16) & 1; }
@@ -1227,14 +1227,15 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
   const bool fuse_attn = (flags & MN_STEP_DISTINCT_SEQUENCES) && mn_attn_fused_ok(M, nq, nkv, hd);
   int n_zero = 0;
   uint32_t* arrived = fuse_attn ? mn_attn_arrivals(M, nq, nkv, hd, t_max, w.attn_ws, w.attn_ws_bytes, &n_zero) : nullptr;
-  if (llm_chain_ok(m, M) && !(image_mask && m->image_gate)) {
+  const bool image_rows = image_mask && m->image_gate;         // rows of two gates: the router takes its own row's, the launches that route for themselves know one
+  if (llm_chain_ok(m, M)) {
     // ---- chain path: 11 launches per layer instead of 18 (2 rows: 6 — QKV with the RMSNorm prologue, attention with RoPE + KV append, dense,
     // the one-launch router, the expert pairs' gate/up, the down projection into h).  glue = llm_glue_kernel.
     const int E = m->n_experts, S = m->n_shared_slots, G = E + S, ad = nq * hd, P = M * n_slot;
     // 2 rows (the CFG rows of one image): the experts run as router + gate/up in ONE launch and the wave-segmented down projection,
     // straight into h (moe_gate_up.hip, moe_down.hip) — int8 / NF4 (2.26 -> 2.05 ms, 2.48 -> 2.38 per step against their grouped streaming launches;
     // bf16 / e4m3 keep the pair launches, which are faster there)
-    const bool gu_chain = g_moe_gate_up && M <= g_moe_gate_up_chain_rows && g_moe_down && moe_gate_up_ok(m->wfmt, H, I, E, m->top_k, S) &&
+    const bool gu_chain = g_moe_gate_up && !image_rows && M <= g_moe_gate_up_chain_rows && g_moe_down && moe_gate_up_ok(m->wfmt, H, I, E, m->top_k, S) &&
                           moe_down_ok(m->wfmt, n_slot, H, I) && (m->wfmt == MN_W_INT8 || m->wfmt == MN_W_NF4 || g_moe_gate_up_chain_all);
     const bool grouped = moe_mfma_ok(m, M) && !gu_chain;
     const int gt = ((H / 4 + 63) / 64) * 64;                           // threads of a glue workgroup
@@ -1284,7 +1285,7 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
         continue;
       }
       // residual + RMSNorm(ln2) + gate + top-k in ONE launch (decode_ops.hip): -> xn (fp32, the pair kernels) or yh (the grouped experts' operand)  (:505-520, 565-592)
-      MN_TRY(moe_router_rows(w.h, w.pp, nz, m->ln2[l], m->rms_eps, m->gate[l], M, H, E, m->top_k, m->norm_topk_prob, S, grouped ? (float*)nullptr : w.xn,
+      MN_TRY(moe_router_rows(w.h, w.pp, nz, m->ln2[l], m->rms_eps, m->gate[l], image_rows ? m->image_gate[l] : nullptr, image_mask, M, H, E, m->top_k, m->norm_topk_prob, S, grouped ? (float*)nullptr : w.xn,
                              grouped ? w.yh : (uint16_t*)nullptr, w.ti, w.tw, w.logits, stream));
       route_capture(l, w.ti, M, n_slot, st);
       if (grouped) hipLaunchKernelGGL(moe_sort_pairs_kernel, dim3(1), dim3(1024), 0, st, w.ti, P, n_slot, G, w.moe.off, w.moe.xrows, w.moe.pair_pos);
@@ -1346,7 +1347,7 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
     MN_TRY(mn_skinny_gemm(&a, stream));
     // one row: RMSNorm + router + the selected experts' gate/up in ONE launch (moe_gate_up.hip), then the down projection (moe_down.hip) — every
     // weight format (int8 / NF4 decode per element like the grouped MFMA launch they replace here: text decode int8 434 -> 699, int4 426 -> 619 tokens/s)
-    if (g_moe_gate_up && M <= g_moe_gate_up_rows && !(image_mask && m->image_gate) && g_moe_down &&
+    if (g_moe_gate_up && M <= g_moe_gate_up_rows && !image_rows && g_moe_down &&
         moe_gate_up_ok(m->wfmt, H, I, m->n_experts, m->top_k, m->n_shared_slots) && moe_down_ok(m->wfmt, n_slot, H, I)) {
       MN_TRY(moe_gate_up_routed(m->wfmt, w.h, H, m->ln2[l], m->rms_eps, m->gate[l], m->w_gate_up[l], (int64_t)2 * I * H,
                                 m->wfmt ? m->w_gate_up_scale[l] : nullptr, (int64_t)2 * I * mn_wq_scales_per_row(m->wfmt, H), M, H, I, m->n_experts, m->top_k,

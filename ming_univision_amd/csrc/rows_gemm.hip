@@ -305,8 +305,9 @@ double ln_time(const Form& f, int M, int64_t wrows, int K) {
 // Plain: 2.3 us, and 68 KB/us of its own or 5.3 TB/s of all weights (6.2 past the caches), whichever is longer, and somewhat more where they are near
 // each other; one round or nothing.  us, measured / this: 32 x 16 tiles of K = 1024 3.7 / 3.7, 32 x 32 of 1024 4.2 / 4.2, of 4096 9.7 / 10.0, of 8192 15.6 / 17.7, 64 x 32 of 1024 5.0 / 5.2, 64 x 64 of 4096
 // 16.6 / 17.7, 64 x 128 of 2048 15.9 / 13.9, of 8192 46.7 / 48.5; hi/lo, 16384 weight rows of 3072 (100 MB): 16 x 64 17.7 .. 18.2 / 19.4, 32 x 64 19.8 .. 20.9 / 20.3, 48 x 64 22.1 .. 23.8 / 21.7.
-constexpr Form forms[] = {{32, 1}, {16, 2}, {32, 2}, {32, 4}, {64, 2}, {64, 4}, {64, 8}}, hilo_forms[] = {{16, 2}, {32, 1}, {32, 2}, {32, 4}, {32, 6}, {32, 8}, {64, 2}, {64, 4}, {16, 4}, {48, 4}};
-double own_time(const Form& f, bool hilo, int K) { return (f.bm * (hilo ? 2 : 1) + 16 * f.nj) * (double)K / 34e3; }
+constexpr Form forms[] = {{32, 1}, {16, 2}, {32, 2}, {32, 4}, {64, 2}, {64, 4}, {64, 8}}, hilo_forms[] = {{16, 2}, {32, 1}, {32, 2}, {32, 4}, {32, 6}, {32, 8}, {64, 2}, {64, 4}, {16, 4}, {48, 4}, {48, 6}};
+// (hi/lo 48 x 96, the one form whose waves' LDS reads take longer than its bytes, is 1025 rows by 1024 columns in one round: K = 1024 10.3 us, 2752 22.2, 4096 29.0; 64 x 64 tiles, 272 of them, 11.3, 24.2, 32.9)
+double own_time(const Form& f, bool hilo, int K) { return (f.bm * (hilo ? 2 : 1) + 16 * f.nj) * (double)K / (hilo && f.bm * f.nj > 256 ? 31e3 : 34e3); }
 // One row tile's weights nobody reads again, and where they take longer than all else they stream faster as non-temporal loads (16384 x 3072: 16 rows 20.0 -> 18.2 us, 36 rows 23.3 -> 22.1); smaller
 // ones, whose round trips count, do not: 8 rows 1024 x 4096 8.2 -> 9.9, 2304 x 768 3.9 -> 4.5.
 bool read_once(const Form& f, bool hilo, int M, int64_t wrows, int K) { return hilo && f.bm >= M && (double)wrows * K / 2.65e6 > own_time(f, hilo, K); }
@@ -339,7 +340,8 @@ void go_hilo(int form, const RowsGemm& p, hipStream_t st) {
     case 6: go<EPI, false, true, 64, 2, 4, 4>(p, st); break;
     case 7: go<EPI, false, true, 64, 4, 4, 3>(p, st); break;
     case 8: go<EPI, false, true, 16, 4, 8, 3>(p, st); break;
-    default: go<EPI, false, true, 48, 4, 4, 4>(p, st); break;
+    case 9: go<EPI, false, true, 48, 4, 4, 4>(p, st); break;
+    default: go<EPI, false, true, 48, 6, 4, 3>(p, st); break;
   }
 }
 

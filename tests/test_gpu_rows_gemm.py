@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 
 # (rows, columns, K): each tile form of both operand kinds, one row, one fragment, columns and rows past the last tile, K of one k-step pair and no whole number of stages
 SHAPES = [(1, 4, 64), (15, 36, 192), (17, 100, 64), (33, 1024, 1024), (70, 1028, 320), (101, 2304, 768), (130, 1024, 4096), (250, 1020, 2752), (257, 2048, 576), (450, 1024, 1024), (600, 768, 2048),
-          (1000, 2048, 8192)]
+          (1025, 1020, 1088), (1000, 2048, 8192)]
 
 
 def rows(g, M, K, hilo, pad):

@@ -237,8 +237,8 @@ static int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* W, int64_
   return nz;
 }
 
-extern "C" int mn_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t ldw, const uint16_t* bias,
-                            void* C, int64_t ldc, int M, int N, int K, int epilogue, void* stream) {
+static int gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t ldw, const uint16_t* bias, void* C, int64_t ldc, int M, int N, int K, int epilogue, int k_parts,
+                     void* stream) {
   MN_CHECK_ARG(A && W && C, "mn_gemm_bf16: null pointer");
   MN_CHECK_ARG(M >= 1 && N >= 1 && K >= 8 && (K % 8) == 0, "mn_gemm_bf16: bad M=%d N=%d K=%d (K %% 8 == 0)", M, N, K);
   MN_CHECK_ARG((lda % 8) == 0 && (ldw % 8) == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0,
@@ -261,7 +261,7 @@ extern "C" int mn_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, i
       memset(&a, 0, sizeof(a));
       a.A = A + m0 * lda; a.lda = lda; a.W = W; a.ldw = ldw; a.bias = bias;
       a.C = reinterpret_cast<char*>(C) + m0 * ldc * c_elt; a.ldc = ldc;
-      a.M = (int)((M - m0) < chunk ? (M - m0) : chunk); a.N = N; a.K = K;
+      a.M = (int)((M - m0) < chunk ? (M - m0) : chunk); a.N = N; a.K = K; a.k_parts = k_parts;
       const int rc = mn_gemm256_ex(&a, map[epilogue], 1, stream);
       if (rc < 0) return rc;
     }
@@ -271,6 +271,13 @@ extern "C" int mn_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, i
   if (rc < 0) return rc;
   MN_CHECK_LAUNCH("mn_gemm_bf16");
   return MN_OK;
+}
+extern "C" int mn_gemm_bf16(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t ldw, const uint16_t* bias,
+                            void* C, int64_t ldc, int M, int N, int K, int epilogue, void* stream) {
+  return gemm_bf16(A, lda, W, ldw, bias, C, ldc, M, N, K, epilogue, 0, stream);
+}
+extern "C" int mn_gemm_bf16_parts(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t ldw, const uint16_t* bias, void* C, int64_t ldc, int M, int N, int K, int epilogue, void* stream) {
+  return gemm_bf16(A, lda, W, ldw, bias, C, ldc, M, N, K, epilogue, 1, stream);
 }
 
 // C fp32 [M,N] = (A_hi + A_lo) W^T + bias for activations split into bf16 hi and lo halves (A_lo = A_hi + a_lo_off

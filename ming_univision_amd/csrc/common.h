@@ -185,6 +185,8 @@ typedef struct mn_g256 {
   const bf16_t* bias;                                    // bf16 [N] (paired: gate bias at n, up bias at n + w_pair_rows) or NULL
   void* C; int64_t ldc; int64_t c_zstride;               // split-K: slice z writes C + z * c_zstride (F32 epilogue)
   int64_t c_lo_off;                                      // SWIGLU_SPLIT: lo rows c_lo_off elements after the hi rows
+  int k_parts;                                           // plain rows: K may be summed in parts where that is faster (mn_rows_gemm); 0: one chain whatever M is, so that a row's
+                                                         // result does not depend on the rows beside it
   const float* gate; int64_t ldgate;                     // F32_RESID_GATE: C += gate * (acc + bias)
   int M, N, K, Kc;                                       // Kc is set by the launcher (k per split-K slice)
   // grouped form: group g = blockIdx.z owns rows [g_off[g], g_off[g] + g_cnt[g]) (device arrays), weights W + g * w_gstride;
@@ -231,6 +233,8 @@ extern "C" int mn_vit_rows_ok(int M, int dim, int hidden, int gelu);
 extern "C" int mn_ln_gemm_rows(const float* x, int64_t ldx, const uint16_t* g, const uint16_t* b, float eps, const uint16_t* W, int64_t ldw, const uint16_t* bias, int gelu, int pair,
                                uint16_t* C, int64_t ldc, int M, int N, int K, void* stream);
 extern "C" int mn_resid_gemm_rows(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t ldw, const uint16_t* bias, float* x, int64_t ldx, int M, int N, int K, void* stream);
+// mn_gemm_bf16 where K may be summed in parts (mn_g256.k_parts)
+extern "C" int mn_gemm_bf16_parts(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t ldw, const uint16_t* bias, void* C, int64_t ldc, int M, int N, int K, int epilogue, void* stream);
 extern "C" int mn_rows_gemm(const mn_g256* a, int epi, double tile_us, void* stream);
 extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo);
 extern "C" int mn_gemm256_f8_plan_ksplit(int M, int N, int K);

@@ -403,7 +403,7 @@ extern "C" int mn_rows_gemm(const mn_g256* a, int epi, double tile_us, void* str
   const bool hilo = a->a_lo_off != 0, paired = epi == MN_G256_SWIGLU_SPLIT;
   const bool known = epi == MN_G256_F32 || epi == MN_G256_F32_RESID || (hilo ? epi == MN_G256_BF16_SPLIT || paired : epi == MN_G256_BF16);
   const int64_t wrows = paired ? a->w_pair_rows + a->N : a->N, rows = paired ? 2 * (int64_t)a->N : a->N;
-  if (!known || a->g_off || a->a_rows || a->f8 || (a->w_pair_rows != 0) != paired ||
+  if (!known || !(hilo || a->k_parts) || a->g_off || a->a_rows || a->f8 || (a->w_pair_rows != 0) != paired ||
       ((uintptr_t)a->C & (epi == MN_G256_F32 || epi == MN_G256_F32_RESID ? 15 : 7)) || a->c_lo_off % 4 || a->w_pair_rows % 4 ||
       !shape_ok(a->A, a->lda, a->W, a->ldw, wrows, a->bias, nullptr, a->ldc, a->M, a->N, a->K) || ((int64_t)a->M * a->lda + a->a_lo_off) * 2 >= ((int64_t)1 << 32) || a->a_lo_off % 8)
     return 0;

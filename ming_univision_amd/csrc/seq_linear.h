@@ -30,7 +30,7 @@ inline int linear(int arith, int M, const float* A, int64_t lda, const uint16_t*
     return mn_skinny_gemm(&a, stream);
   }
   if (arith == MN_SEQ_ARITH_BF16 && A16 && mfma_ok(W, K) && (lda16 % 8) == 0 && (((uintptr_t)A16) & 15) == 0)
-    return mn_gemm_bf16(A16, lda16, W, K, bias, C, ldc, M, N, K, MN_GEMM_F32, stream);
+    return mn_gemm_bf16_parts(A16, lda16, W, K, bias, C, ldc, M, N, K, MN_GEMM_F32, stream);
   return mn_gemm_f32_batched(A, lda, 0, W, K, 0, bias, C, ldc, 0, nullptr, 0, 0, nullptr, 0, 0, M, N, K, 1, 1.0f, stream);
 }
 

@@ -116,14 +116,14 @@ extern "C" int mn_vit_blocks(float* x, int B, int T, int dim, int depth, const u
   auto resid = [&](const uint16_t* A, int K, const uint16_t* W, const uint16_t* b, const uint16_t* g, const uint16_t* be, int act, uint16_t* y) -> int {
     const int ks = resid_slices(M, dim, K);
     normed = ks > 0 && mn_gemm256_supported(K, 0, K, dim, M, dim, K);
-    if (!normed) return mn_gemm_bf16(A, K, W, K, b, x, dim, M, dim, K, MN_GEMM_F32_RESID, stream);
+    if (!normed) return mn_gemm_bf16_parts(A, K, W, K, b, x, dim, M, dim, K, MN_GEMM_F32_RESID, stream);
     const int nz = mn_gemm256_splitk(A, K, 0, W, K, b, slabs, M, dim, K, ks, stream);
     return nz < 0 ? nz : mn_slab_resid_norm(slabs, nz, (int64_t)M * dim, x, dim, g, be, eps, act, y, dim, M, dim, stream);
   };
   for (int i = 0; i < depth; ++i, w += 12) {
     const bool last = i + 1 == depth;
     if (!normed) TRY(mn_layernorm_bf16(x, dim, w[0], w[1], eps, xn, dim, M, dim, 0, stream));
-    TRY(mn_gemm_bf16(xn, dim, w[2], dim, w[3], qkv, 3 * (int64_t)dim, M, 3 * dim, dim, MN_GEMM_BF16, stream));
+    TRY(mn_gemm_bf16_parts(xn, dim, w[2], dim, w[3], qkv, 3 * (int64_t)dim, M, 3 * dim, dim, MN_GEMM_BF16, stream));
     TRY(mn_attn_prefill_hd64(qkv, att, B, T, nh, causal, stream));
     TRY(resid(att, dim, w[4], w[5], w[6], w[7], 0, xn));
     if (!normed) TRY(mn_layernorm_bf16(x, dim, w[6], w[7], eps, xn, dim, M, dim, 0, stream));

@@ -1,4 +1,5 @@
-"""The dense products whose tiles are one round of the CUs: waves that split K inside a workgroup (rows_gemm.hip), behind the wide-row GEMM's entry points."""
+"""The dense products whose tiles are one round of the CUs: waves that split K inside a workgroup (rows_gemm.hip) for hi/lo rows, and for plain rows of prompts and pictures; plain rows
+of the wide-row GEMM's own entry points keep one chain of K."""
 import pytest
 import torch
 
@@ -44,6 +45,18 @@ def test_dense_epilogues(M, N, K, hilo):
         bound = (2 * K + 16) * 2.0 ** -24 * (sums + 0.5) + (2.0 ** -8 * ref.abs() if epi == 0 else 0.0)
         assert bool(((C[:M, :N].double() - ref).abs() <= bound).all()), (epi, float((C[:M, :N].double() - ref).abs().max()))
         assert bool((C[M:] == 0.5).all()) and bool((C[:, N:] == 0.5).all())
+
+
+@pytest.mark.parametrize("M,width", [(65, 1024), (257, 1024), (450, 512), (700, 256)])
+def test_plain_products_of_prompts(M, width):
+    """Prompts whose plain bf16 products are one round, against the fp32 arithmetic of the same layers (two layers of products on bf16 operands, 2^-9 each of some ten of them)."""
+    from ming_univision_amd.configuration import DaberaxConfig
+    from ming_univision_amd.daberax import DaberaxDecoder
+    cfg = DaberaxConfig(width=width, vocab=40, norm=dict(eps=1e-6), token_side=dict(dim=8), layers=[
+        dict(type="attention", mixer=dict(heads=4, kv_heads=2, dim=32, vdim=64, scale=0.2), mlp=dict(kind="dense", ff=2 * width + 64))] * 2)
+    ids = torch.arange(M, device="cuda") % 40
+    got, want = (DaberaxDecoder.synthetic(cfg, "cuda", t_max=M + 1, n_seq=1, arith=a).prefill(ids).double() for a in ("bf16", "f32"))
+    assert float((got - want).norm() / want.norm()) < 2e-2
 
 
 @pytest.mark.parametrize("M,hidden,K", [(1, 4, 64), (17, 36, 192), (40, 2048, 768), (101, 2752, 1024), (128, 1028, 320), (256, 2048, 768)])

@@ -630,16 +630,16 @@ static bool tile_launch(const G256& p, int form, int nz, bool hilo, hipStream_t 
 }
 
 // The grouped products of few rows a group: row tiles of 32 or 64 of the list, rows and K-tiles as above.
-template <int EPI, int BM, int BN, int WM, int WN, int S, bool TWO, int GROUP>
+template <int EPI, int BM, int BN, int WM, int WN, int S, int GROUP>
 static void group_go(G256 p, hipStream_t st) {
   p.group_m = 1;                                       // (bands of four row tiles: the same to 4 % slower)
   const dim3 grid((unsigned)(p.max_mtiles * mn_cdiv(p.N, epi_paired(EPI) ? BN / 2 : BN)));
-  hipLaunchKernelGGL((gemm_tile_kernel<EPI, true, BM, BN, WM, WN, S, TWO, GROUP>), grid, dim3(WM * WN * 64), 0, st, p);
+  hipLaunchKernelGGL((gemm_tile_kernel<EPI, true, BM, BN, WM, WN, S, false, GROUP>), grid, dim3(WM * WN * 64), 0, st, p);
 }
 template <int EPI>
 static void group_launch(const G256& p, hipStream_t st) {
-  if (p.tile_rows == 32) group_go<EPI, 32, 128, 2, 2, 3, true, 2>(p, st);
-  else group_go<EPI, 64, 256, 2, 4, 3, false, 1>(p, st);
+  if (p.tile_rows == 32) group_go<EPI, 32, 128, 2, 2, 3, 2>(p, st);
+  else group_go<EPI, 64, 256, 2, 4, 3, 1>(p, st);
 }
 
 // Generic launcher.  Returns the number of split-K slices used (>= 1) or a negative error.

@@ -1229,7 +1229,7 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
   uint32_t* arrived = fuse_attn ? mn_attn_arrivals(M, nq, nkv, hd, t_max, w.attn_ws, w.attn_ws_bytes, &n_zero) : nullptr;
   const bool image_rows = image_mask && m->image_gate;         // rows of two gates: the router takes its own row's, the launches that route for themselves know one
   if (llm_chain_ok(m, M)) {
-    // ---- chain path: 11 launches per layer instead of 18 (2 rows: 6 — QKV with the RMSNorm prologue, attention with RoPE + KV append, dense,
+    // ---- chain path: 9 launches per layer (11 where rows read each other's new keys) instead of 18 (2 rows: 6 — QKV with the RMSNorm prologue, attention with RoPE + KV append, dense,
     // the one-launch router, the expert pairs' gate/up, the down projection into h).  glue = llm_glue_kernel.
     const int E = m->n_experts, S = m->n_shared_slots, G = E + S, ad = nq * hd, P = M * n_slot;
     // 2 rows (the CFG rows of one image): the experts run as router + gate/up in ONE launch and the wave-segmented down projection,

@@ -675,13 +675,19 @@ static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
   const bool may256 = epi != E_BF16_GELU || mn_cdiv(p.M, 256) * mn_cdiv(p.N, 256) >= 128;
   double us = 0;
   const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : epi == E_BF16_GELU && may256 ? 0 : tile_form(p.M, p.N, p.Kc, nz, hilo, epi, may256, &us);
-  // one row tile of a matrix that no cache holds (a vocabulary's logits): us at 126464 x 2048, the tiles below -> this: 5 rows 110 -> 86, 16 108 -> 91, 24 112 -> 98, 32 114 -> 102 (64 x 256 tiles
-  // like this 40 rows 118 -> 115, 64 129 -> 121; in the caches' reach the tiles below: 16384 x 3072 17 .. 20, this 23 .. 30)
+  // one row tile of a matrix that no cache holds (a vocabulary's logits): us at 126464 x 2048, the tiles below -> this: 5 rows 110 -> 86, 16 108 -> 91, 24 112 -> 98, 32 114 -> 101; 30000 x 5120 5 rows 56 -> 46,
+  // 32 69 -> 53 (in the caches' reach the tiles below: 16384 x 3072 17 .. 20, this 23 .. 30).  Two workgroups a CU, and only where
+  // their rounds are 0.7 full or all tiles have a CU of their own (98304 x 2048, 0.75 16 rows 87 -> 71; 80000, 0.61 65 -> 65; 66000, 0.50 59 -> 62).  Above 32 rows 64 x 256 tiles, one a CU, where their rounds are 0.85 full:
+  // 126464 x 2048 40 rows 118 -> 115, 64 129 -> 120, 116736 x 3072 148 -> 136, 163 -> 144; 118 of them (30000 x 5120) 65 -> 85
   if (us > 0 && nz == 1 && hilo && epi == E_F32 && a.M <= 64 && (int64_t)a.N * a.K * 2 >= (int64_t)256 << 20) {
-    if (a.M <= 16) tile_go<E_F32, 16, 128, 1, 4, 4, true, true, 3>(p, nz, st);
-    else if (a.M <= 32) tile_go<E_F32, 32, 128, 2, 2, 3, true, true, 3>(p, nz, st);
-    else tile_go<E_F32, 64, 256, 2, 4, 3, true, true, 3>(p, nz, st);
-    return 1;
+    const bool few = a.M <= 32;
+    const int64_t cus = mn_num_cus(), tiles = mn_cdiv(a.N, few ? 128 : 256), places = few ? 2 * cus : cus;
+    if (few ? tiles <= cus || 10 * tiles >= 7 * places * mn_cdiv(tiles, places) : 100 * tiles >= 85 * places * mn_cdiv(tiles, places)) {
+      if (a.M <= 16) tile_go<E_F32, 16, 128, 1, 4, 4, true, true, 3>(p, nz, st);
+      else if (few) tile_go<E_F32, 32, 128, 2, 2, 3, true, true, 3>(p, nz, st);
+      else tile_go<E_F32, 64, 256, 2, 4, 3, true, true, 3>(p, nz, st);
+      return 1;
+    }
   }
   if (us > 0 && nz == 1 && mn_rows_gemm(&p, epi, us, st)) return 1;       // few tiles: forms whose waves split K (rows_gemm.hip)
 #define G256_GO(E)                                                                          \

@@ -309,8 +309,8 @@ constexpr Form forms[] = {{32, 1}, {16, 2}, {32, 2}, {32, 4}, {64, 2}, {64, 4}, 
 // (hi/lo 48 x 96, the one form whose waves' LDS reads take longer than its bytes, is 1025 rows by 1024 columns in one round: K = 1024 10.3 us, 2752 22.2, 4096 29.0; 64 x 64 tiles, 272 of them, 11.3, 24.2, 32.9)
 double own_time(const Form& f, bool hilo, int K) { return (f.bm * (hilo ? 2 : 1) + 16 * f.nj) * (double)K / (hilo && f.bm * f.nj > 256 ? 31e3 : 34e3); }
 // One row tile's weights nobody reads again, and where they take longer than all else they stream faster as non-temporal loads (16384 x 3072: 16 rows 20.0 -> 18.2 us, 36 rows 23.3 -> 22.1); smaller
-// ones, whose round trips count, do not: 8 rows 1024 x 4096 8.2 -> 9.9, 2304 x 768 3.9 -> 4.5.
-bool read_once(const Form& f, bool hilo, int M, int64_t wrows, int K) { return hilo && f.bm >= M && (double)wrows * K / 2.65e6 > own_time(f, hilo, K); }
+// ones, whose round trips count, do not: 8 rows 1024 x 4096 8.2 -> 9.9, 2304 x 768 3.9 -> 4.5, 26 of 15952 x 320 5.3 -> 6.0.
+bool read_once(const Form& f, bool hilo, int M, int64_t wrows, int K) { return hilo && f.bm >= M && wrows * K >= (int64_t)32 << 20 && (double)wrows * K / 2.65e6 > own_time(f, hilo, K); }
 double rows_time(const Form& f, bool hilo, int M, int64_t wrows, int K) {
   if (form_tiles(f, M, wrows) > mn_num_cus()) return 1e30;
   const double own = own_time(f, hilo, K), all = (double)wrows * K / (read_once(f, hilo, M, wrows, K) ? 3.1e6 : 2.65e6), hi = fmax(own, all), lo = fmin(own, all);
@@ -347,7 +347,7 @@ void go_hilo(int form, const RowsGemm& p, hipStream_t st) {
 
 bool shape_ok(const void* A, int64_t lda, const void* W, int64_t ldw, int64_t wrows, const void* bias, const void* C, int64_t ldc, int M, int N, int K) {
   return M >= 1 && N >= 4 && N % 4 == 0 && K >= 64 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldc % 4 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15) == 0 &&
-         ((uintptr_t)bias & 7) == 0 && (int64_t)M * lda * 2 < ((int64_t)1 << 32) && wrows * ldw * 2 < ((int64_t)1 << 32);
+         ((uintptr_t)bias & 7) == 0 && lda >= 0 && ldw >= 0 && ((int64_t)M * lda + K) * 2 < ((int64_t)1 << 32) && (wrows * ldw + K) * 2 < ((int64_t)1 << 32);      // (offsets of 32 bits)
 }
 
 }  // namespace
@@ -398,14 +398,14 @@ extern "C" int mn_resid_gemm_rows(const uint16_t* A, int64_t lda, const uint16_t
 // us, the tiles / these, cold weights, 40, 101, 256 and 600 rows: hi/lo 768 -> 768 7.5 / 3.8, 7.8 / 3.9, 7.9 / 4.7, 8.1 / 6.0; 2048 -> 768 15.3 / 5.9, 15.5 / 6.0, 15.7 / 7.1, 15.9 / 10.6;
 // 768 -> 2304 7.7 / 4.1, 7.9 / 5.8, 8.4 / 6.8, tiles; 4096 -> 1024 27.3 / 8.5, 27.9 / 8.8, 27.6 / 11.8, 28.4 / 21.8; 1024 -> 2 x 2752 gated 10.4 / 8.1, 10.5 / 9.4, tiles (14.1).  Plain rows, 70, 250, 450 and
 // 1000: 1024 -> 1024 6.9 / 3.8, 6.9 / 4.5, 7.1 / 5.6, tiles (7.4); 2048 -> 2048 10.5 / 6.1, 10.9 / 7.7, 11.2 / 10.5, 17.4 / 16.0; 8192 -> 2048 34.0 / 16.3, 36.7 / 25.9, 36.7 / 31.7, 57.9 / 51.4; 1024 -> 4096
-// 7.0 / 5.5, tiles (7.4).  The error is smaller throughout (eight sums of K / 8: 1.0e-7 for 1.9e-7 of 64 bits at K = 2048).
+// 7.0 / 5.5, tiles (7.4).  Gated products of fewer than 512 values stay (26 rows 320 -> 2 x 7976 5.3 / 5.7).  The error is smaller throughout (eight sums of K / 8: 1.0e-7 for 1.9e-7 of 64 bits at K = 2048).
 extern "C" int mn_rows_gemm(const mn_g256* a, int epi, double tile_us, void* stream) {
   const bool hilo = a->a_lo_off != 0, paired = epi == MN_G256_SWIGLU_SPLIT;
   const bool known = epi == MN_G256_F32 || epi == MN_G256_F32_RESID || (hilo ? epi == MN_G256_BF16_SPLIT || paired : epi == MN_G256_BF16);
   const int64_t wrows = paired ? a->w_pair_rows + a->N : a->N, rows = paired ? 2 * (int64_t)a->N : a->N;
-  if (!known || !(hilo || a->k_parts) || a->g_off || a->a_rows || a->f8 || (a->w_pair_rows != 0) != paired ||
+  if (!known || !(hilo || a->k_parts) || (paired && a->K < 512) || a->g_off || a->a_rows || a->f8 || (a->w_pair_rows != 0) != paired ||
       ((uintptr_t)a->C & (epi == MN_G256_F32 || epi == MN_G256_F32_RESID ? 15 : 7)) || a->c_lo_off % 4 || a->w_pair_rows % 4 ||
-      !shape_ok(a->A, a->lda, a->W, a->ldw, wrows, a->bias, nullptr, a->ldc, a->M, a->N, a->K) || ((int64_t)a->M * a->lda + a->a_lo_off) * 2 >= ((int64_t)1 << 32) || a->a_lo_off % 8)
+      !shape_ok(a->A, a->lda, a->W, a->ldw, wrows, a->bias, nullptr, a->ldc, a->M, a->N, a->K) || ((int64_t)a->M * a->lda + a->a_lo_off + a->K) * 2 >= ((int64_t)1 << 32) || a->a_lo_off < 0 || a->a_lo_off % 8)
     return 0;
   double us;
   const auto time = [&](const Form& f) { return (paired && f.nj == 1) ? 1e30 : rows_time(f, hilo, a->M, rows, a->K); };

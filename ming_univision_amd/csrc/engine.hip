@@ -16,6 +16,7 @@
 extern "C" size_t mn_attn_decode_workspace_bytes(int M, int n_q, int hd, int64_t t_max);
 extern "C" int mn_stream_mfma(const uint16_t* Y, const uint16_t* W, float* P, int M, int Ntot, int K, void* stream);
 extern "C" int mn_stream_mfma_slices(int M, int Ntot, int K);
+extern "C" int mn_stream_mfma_grouped_slices(int G, int max_rows, int Ntot, int K);
 extern "C" int mn_stream_kwalk_slices(int max_rows, int K);
 extern "C" int mn_stream_kwalk_grouped(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G,
                                        int max_rows, int Ntot, int K, void* stream);
@@ -64,6 +65,10 @@ static inline int stream_grouped(int wfmt, const uint16_t* Y, int y_rows, const 
                                           s_stride * mn_wq_scales_per_row(wfmt, K), P, p_rows, off, xrows, G, max_rows, Ntot, K, wfmt, stream)
               : mn_stream_kwalk_grouped(Y, y_rows, reinterpret_cast<const uint16_t*>(W), w_stride, P, p_rows, off, xrows, G, max_rows, Ntot,
                                         K, stream);
+}
+// slabs that stream_grouped writes at most (mn_stream_mfma_grouped_slices is the bound of the weight-only forms)
+static inline size_t stream_grouped_slabs(int wfmt, int G, int rows, int Ntot, int K) {
+  return (size_t)(wfmt ? mn_stream_mfma_grouped_slices(G, rows, Ntot, K) : mn_stream_kwalk_slices(rows, K));
 }
 
 namespace {
@@ -983,7 +988,7 @@ struct MoeWs {
   float *p1, *p2;
 };
 
-static size_t moe_carve(Carver& cv, int rows, int H, int I, int G, int n_slot, MoeWs* o) {
+static size_t moe_carve(Carver& cv, int wfmt, int rows, int H, int I, int G, int n_slot, MoeWs* o) {
   const size_t P = (size_t)rows * n_slot;
   const size_t before = cv.off;
   o->off = cv.take<int32_t>((size_t)G + 1);
@@ -991,8 +996,8 @@ static size_t moe_carve(Carver& cv, int rows, int H, int I, int G, int n_slot, M
   o->pair_pos = cv.take<int32_t>(P);
   o->y1 = cv.take<bf16_t>((size_t)2 * rows * H);
   o->y2 = cv.take<bf16_t>(2 * P * I);
-  o->p1 = cv.take<float>((size_t)mn_stream_kwalk_slices(rows, H) * P * 2 * I);
-  o->p2 = cv.take<float>((size_t)mn_stream_kwalk_slices(rows, I) * P * H);
+  o->p1 = cv.take<float>(stream_grouped_slabs(wfmt, G, rows, 2 * I, H) * P * 2 * I);
+  o->p2 = cv.take<float>(stream_grouped_slabs(wfmt, G, rows, H, I) * P * H);
   return cv.off - before;
 }
 
@@ -1074,7 +1079,7 @@ static size_t llm_carve(const mn_llm* m, int rows, int64_t t_max, void* ws, size
   o->attn_ws = cv.take<char>(o->attn_ws_bytes);
   o->sk_ws_bytes = sk_ws_need(rows, {{qkv_dim, m->hidden, 0}, {m->hidden, m->n_q * m->head_dim, 0}, {m->n_experts, m->hidden, 0}});
   o->sk_ws = cv.take<char>(o->sk_ws_bytes);
-  if (moe_mfma_ok(m, rows)) moe_carve(cv, rows, m->hidden, m->moe_inter, m->n_experts + m->n_shared_slots, n_slot, &o->moe);
+  if (moe_mfma_ok(m, rows)) moe_carve(cv, m->wfmt, rows, m->hidden, m->moe_inter, m->n_experts + m->n_shared_slots, n_slot, &o->moe);
   if (llm_chain_ok(m, rows)) {
     const int ad = m->n_q * m->head_dim;
     o->yh = cv.take<bf16_t>((size_t)2 * rows * m->hidden);
@@ -1144,15 +1149,19 @@ extern "C" int mn_rf_max_rows(const mn_rf_head* h) { return rf_wide_ok(h, 2048) 
 extern "C" int mn_semdec_max_rows(const mn_semdec* s) { return sem_wide_ok(s, 2048) ? 2048 : 64; }
 
 extern "C" size_t mn_llm_workspace_bytes(const mn_llm* m, int rows, int64_t t_max) {
-  size_t wide = 0;
+  size_t need = 0;
   if (llm_wide_ok(m, rows)) {
     LlmWideWs ww;
-    wide = llm_wide_carve(m, rows, t_max, nullptr, 0, &ww);
-    if (rows > 64) return wide;
+    need = llm_wide_carve(m, rows, t_max, nullptr, 0, &ww);
+    if (rows > 64) return need;
   }
-  LlmWs w{};                                 // <= 64 rows: a step with the image-gate override stays on the streaming route
-  const size_t narrow = llm_carve(m, rows, t_max, nullptr, 0, &w);
-  return narrow > wide ? narrow : wide;
+  // a few rows' products leave more slabs a row than many rows': a buffer for `rows` (up to 64) serves every smaller count
+  for (int r = rows <= 64 ? 1 : rows; r <= rows; ++r) {
+    LlmWs w{};
+    const size_t narrow = llm_carve(m, r, t_max, nullptr, 0, &w);
+    if (narrow > need) need = narrow;
+  }
+  return need;
 }
 
 extern "C" int mn_rows_advance(int32_t* a, int32_t* b, int32_t* c, int M, int delta, void* stream) {

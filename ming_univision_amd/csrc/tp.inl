@@ -300,16 +300,21 @@ static size_t llm_tp_carve(const mn_llm* m, const mn_llm_tp* tp, int rows, int64
     const size_t s3 = (size_t)stream_slices(m->wfmt, rows, H, SIc) * rows * H;
     if (s3 > psh) psh = s3;
     o->pps = cv.take<float>(pmax * rows);
-    o->p1 = cv.take<float>((size_t)mn_stream_kwalk_slices(rows, H) * Pn * 2 * I);
-    o->p2 = cv.take<float>((size_t)mn_stream_kwalk_slices(rows, I) * Pn * H);
+    o->p1 = cv.take<float>(stream_grouped_slabs(m->wfmt, m->n_experts, rows, 2 * I, H) * Pn * 2 * I);
+    o->p2 = cv.take<float>(stream_grouped_slabs(m->wfmt, m->n_experts, rows, H, I) * Pn * H);
   }
   o->psh = cv.take<float>(psh);
   return off + cv.off;
 }
 
 extern "C" size_t mn_llm_tp_workspace_bytes(const mn_llm* m, const mn_llm_tp* tp, int rows, int64_t t_max) {
-  LlmTpWs w;
-  return llm_tp_carve(m, tp, rows, t_max, nullptr, 0, &w);
+  size_t need = 0;
+  for (int r = rows <= 64 ? 1 : rows; r <= rows; ++r) {        // (every smaller count, as mn_llm_workspace_bytes)
+    LlmTpWs w;
+    const size_t n = llm_tp_carve(m, tp, r, t_max, nullptr, 0, &w);
+    if (n > need) need = n;
+  }
+  return need;
 }
 
 extern "C" int mn_llm_tp_segments(const mn_llm* m) { return 2 * m->n_layers + 1; }      // one-shot all-reduces (<= two_shot_rows rows)

@@ -204,6 +204,24 @@ def test_scratch_of_a_hybrid_prompt_grows_with_its_rows():
     assert size[2] - plain[1] < 16 * 65 * W * 4 + (4 << 20) and size[5] - plain[2] >= 8192 * W * 4 - 512 * W * 4
 
 
+def test_scratch_of_a_decoder_step_grows_with_its_rows():
+    """mn_llm_workspace_bytes and mn_llm_tp_workspace_bytes up to 64 rows: a caller's scratch for its most rows serves the steps of fewer, whose products leave more slabs a row."""
+    import ctypes
+    from ming_univision_amd import _lib
+    L = _lib.lib()
+    for H, heads, kv, E, top, shared, inter in ((2048, 16, 4, 64, 6, 2, 1408), (1024, 8, 2, 64, 6, 2, 1408), (256, 4, 2, 4, 4, 2, 64), (512, 8, 2, 12, 12, 1, 200), (4096, 32, 8, 64, 8, 1, 2048)):
+        for wfmt in (0, 1, 2, 3):
+            m = _lib.Llm(n_layers=2, hidden=H, n_q=heads, n_kv=kv, head_dim=128, n_experts=E, n_shared_slots=shared, top_k=top, moe_inter=inter, wfmt=wfmt)
+            for t_max in (64, 256, 1200, 4096):
+                size = [L.mn_llm_workspace_bytes(ctypes.byref(m), r, t_max) for r in range(1, 65)]
+                assert size == sorted(size), (H, wfmt, t_max)
+    m = _lib.Llm(n_layers=2, hidden=2048, n_q=16, n_kv=4, head_dim=128, n_experts=64, n_shared_slots=0, top_k=6, moe_inter=1408)
+    tp = _lib.LlmTp(shared_inter=2816)
+    for t_max in (256, 1200, 4096):
+        size = [L.mn_llm_tp_workspace_bytes(ctypes.byref(m), ctypes.byref(tp), r, t_max) for r in range(1, 65)]
+        assert size == sorted(size), t_max
+
+
 def test_config_shapes_and_sizes():
     cfg = C.MingUniVisionConfig.ming_univision_16b_a3b()
     n_llm = sum(int(torch.tensor(s).prod()) for s in C.llm_param_shapes(cfg.llm_config).values())

@@ -49,6 +49,9 @@ MN_DEV_API void mn_gemm_tile_tune(int form);
 MN_DEV_API void mn_attn_rows_tune(int form);
 /* Measurement only: K / V rows are rounded to bf16 when appended to the (fp32) cache — the values a bf16 KV cache would hold. */
 MN_DEV_API void mn_kv_round_bf16(int on);
+/* Internal products that tests hold against float64 by themselves. */
+MN_DEV_API int mn_stream_kwalk_grouped(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G,
+                                       int max_rows, int Ntot, int K, void* stream);
 
 #ifdef __cplusplus
 }

@@ -354,7 +354,11 @@ __global__ __launch_bounds__(KW * 64, 4) void stream_kwalk_kernel(const bf16_t* 
   // ---- the products' side: chunk c of tile ct ----
   int ct = begin / nch, c = begin - ct * nch, buf = 0;
   char* wt = ws + wave * 32 * ROWB;
-  f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  // A chain of sums for each half of a chunk, no longer than those of the grid form's two ranges.  Error against 64 bits, 24 rows, gate and up / down: grid 2.8 / 2.3e-7, one chain 3.5 / 2.7e-7, two
+  // 2.5 / 1.9e-7; the time is the same.
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) acc[s][0] = acc[s][1] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int jb = 0; jb < n; jb += D) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -370,8 +374,8 @@ __global__ __launch_bounds__(KW * 64, 4) void stream_kwalk_kernel(const bf16_t* 
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
             const bf16x8 w = *reinterpret_cast<const bf16x8*>(wt + cslot<CK>(t * 16 + fr, s * 4 + fq));
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, w, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, w, acc[t], 0, 0, 0);
+            acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, w, acc[s][t], 0, 0, 0);
+            acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, w, acc[s][t], 0, 0, 0);
           }
         }
         if (++c == nch || j + 1 == n) {                                 // this workgroup's part of the tile is done
@@ -385,11 +389,11 @@ __global__ __launch_bounds__(KW * 64, 4) void stream_kwalk_kernel(const bf16_t* 
               for (int r = 0; r < 4; ++r)
                 if (fq * 4 + r < b.rows) {
                   float* p_ = P + (int64_t)z * p_slab + (int64_t)(b.row0 + fq * 4 + r) * Ntot + nn;
-                  *p_ = acc[t][r];
+                  *p_ = acc[0][t][r] + acc[1][t][r];
                   for (int e = 1; e <= zeros; ++e) p_[e * p_slab] = 0.f;
                 }
             }
-            acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            acc[0][t] = acc[1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
           }
           c = 0;
           ++ct;

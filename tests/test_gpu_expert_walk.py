@@ -53,3 +53,37 @@ def test_rows_together_and_alone(rows, hidden, inter, experts, top, shared):
     assert int((~same).sum()) <= (0 if experts == top else 1 + rows // 32)
     err = (together - alone).norm(dim=1) / alone.norm(dim=1)
     assert float(err[same].max()) < 1e-4, err
+
+
+@pytest.mark.parametrize("rows,N,K", [(16, 2816, 2048), (24, 2816, 2048), (24, 2048, 1408), (64, 2048, 1408)])
+def test_error_of_whole_tiles(rows, N, K):
+    """Enough tiles that a workgroup's share holds whole ones: their two chains of K / 2 are as long as those of the grid form's two ranges, so the error against float64 is no larger than
+    its (same operands; half a percent for the draw)."""
+    import ctypes
+    import os
+    from ming_univision_amd import _lib
+    from ming_univision_amd._lib import ptr
+    dev = ctypes.CDLL(os.path.join(os.path.dirname(_lib.LIB_PATH), "libmingnative_dev.so"))
+    fn = dev.mn_stream_kwalk_grouped
+    fn.restype, fn.argtypes = _lib.SYMBOLS["mn_stream_mfma_grouped"]
+    G, slots = 64, 8
+    g = torch.Generator(device="cuda").manual_seed(rows + N)
+    picks = torch.stack([torch.randperm(G, device="cuda", generator=g)[:slots] for _ in range(rows)]).flatten()
+    order, count = torch.argsort(picks, stable=True), torch.bincount(picks, minlength=G)
+    src = (order // slots).int().contiguous()
+    off = torch.zeros(G + 1, dtype=torch.int32, device="cuda")
+    off[1:] = count.cumsum(0)
+    W = torch.empty(G, N, K, dtype=torch.bfloat16, device="cuda").normal_(0, K ** -0.5, generator=g)
+    x = torch.randn(rows, K, device="cuda", generator=g)
+    Y = torch.stack([x.bfloat16(), (x - x.bfloat16().float()).bfloat16()]).contiguous()
+    x64, pairs = (Y[0].double() + Y[1].double())[src.long()], rows * slots
+    want = torch.cat([x64[int(off[e]):int(off[e + 1])] @ W[e].double().t() for e in range(G)])
+    out = torch.empty(4, pairs, N, device="cuda")
+
+    def error(f):
+        out.fill_(float("nan"))
+        nz = f(ptr(Y), rows, ptr(W), N * K, ptr(out), pairs, ptr(off), ptr(src), G, rows, N, K, torch.cuda.current_stream().cuda_stream)
+        assert 1 <= nz <= 4
+        return float((out[:nz].sum(0).double() - want).norm() / want.norm())
+    walk, grid = error(fn), error(_lib.lib().mn_stream_mfma_grouped)
+    assert walk <= 1.005 * grid, (walk, grid)

@@ -18,8 +18,8 @@ extern "C" int mn_stream_mfma(const uint16_t* Y, const uint16_t* W, float* P, in
 extern "C" int mn_stream_mfma_slices(int M, int Ntot, int K);
 extern "C" int mn_stream_mfma_grouped_slices(int G, int max_rows, int Ntot, int K);
 extern "C" int mn_stream_kwalk_slices(int max_rows, int K);
-extern "C" int mn_stream_kwalk_grouped(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G,
-                                       int max_rows, int Ntot, int K, void* stream);
+extern "C" int mn_stream_experts(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G, int max_rows,
+                                 int Ntot, int K, void* stream);
 extern "C" int mn_rope_kv_from_partials(const float* qkv, int64_t ldqkv, int nz, int64_t slab, int M, int n_q, int n_kv, int hd,
                                         int rope, const float* cos_tab, const float* sin_tab, const int32_t* row_seq,
                                         const int32_t* row_slot, const int32_t* row_pos, int sec_t, int sec_h, float q_scale,
@@ -63,8 +63,8 @@ static inline int stream_grouped(int wfmt, const uint16_t* Y, int y_rows, const 
                                  void* stream) {
   return wfmt ? mn_stream_mfma_grouped_wq(Y, y_rows, reinterpret_cast<const uint8_t*>(W), w_stride, wscale,
                                           s_stride * mn_wq_scales_per_row(wfmt, K), P, p_rows, off, xrows, G, max_rows, Ntot, K, wfmt, stream)
-              : mn_stream_kwalk_grouped(Y, y_rows, reinterpret_cast<const uint16_t*>(W), w_stride, P, p_rows, off, xrows, G, max_rows, Ntot,
-                                        K, stream);
+              : mn_stream_experts(Y, y_rows, reinterpret_cast<const uint16_t*>(W), w_stride, P, p_rows, off, xrows, G, max_rows, Ntot, K,
+                                  stream);
 }
 // slabs that stream_grouped writes at most (mn_stream_mfma_grouped_slices is the bound of the weight-only forms)
 static inline size_t stream_grouped_slabs(int wfmt, int G, int rows, int Ntot, int K) {

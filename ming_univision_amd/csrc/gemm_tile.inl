@@ -28,7 +28,7 @@ __device__ __forceinline__ void wait_tiles(int rem) {
 }
 
 // GROUP 1, 2: the products of groups of rows with weights of their own (MoE experts), row tiles of BM from a device-built list.  2 and 3 (one dense product): the weights are read past
-// the caches, where all rows, or most groups, are one row tile: nobody reads them again, and lines that are let go at once stream faster (66 experts' 5632 x 2048 / 2048 x 1408 of 100
+// the caches, where all rows, or most groups, are one row tile: nobody reads them again, and lines that are let go at once stream faster (66 experts' 2816 x 2048 / 2048 x 1408 of 100
 // rows in tiles of 32 x 128, 6 picks a row and two for all: 146 -> 140 us / 74 -> 70, 70 rows 146 -> 135 / 73 -> 67, 5.6 TB/s; 240 rows, where a third of the groups are two tiles, 162 -> 165 /
 // 87 -> 89).
 template <int EPI, bool HILO, int BM, int BN, int WM, int WN, int S, bool TWO = false, int GROUP = 0>

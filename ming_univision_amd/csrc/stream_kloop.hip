@@ -16,6 +16,8 @@
 // fragment read from LDS feeds two MFMAs per half — with one tile per wave every 4 KiB weight chunk costs 32 KiB of x
 // fragment reads and the kernel is LDS-bound (RF w12 at 64 rows: 40 us with NT = 1, 28-29 us with NT = 2, ring depth 2;
 // a 4-deep ring spills).  At <= 32 rows it is on par with the K-slice kernel (23-25 vs 24 us), which stays the default there.
+#include <math.h>
+
 #include <type_traits>
 
 #include "common.h"
@@ -287,7 +289,7 @@ __global__ __launch_bounds__(KW * 64, (WQ == 1 && MT == 4 && NT == 2) ? 4 : 1) v
 
 // ---- the walk of bf16 groups ---------------------------------------------------------------------------------------------------
 // In the grid form above a workgroup is a column tile and a K-range of a group, two fit a CU, and a round of them that is not full costs a whole one: 66 experts of 2048 x 1408
-// in two ranges are 1056 workgroups on 512 places and stream at 4.9 TB/s, of 5632 x 2048 1452 and 5.8.  Here a resident set of workgroups, two a CU, takes the chunks of
+// in two ranges are 1056 workgroups on 512 places and stream at 4.9 TB/s, of 2816 x 2048 1452 and 5.8.  Here a resident set of workgroups, two a CU, takes the chunks of
 // all live groups' tiles (16 rows x 256 columns) one behind the other in equal shares, so that all end together whatever the number of live groups, which only the device knows.
 // A tile spans at most nz workgroups (a share is no less than a tile / (nz - 1)); each writes its part into a slab of its own, the one that ends a tile zeros in the slabs behind.  Weights and rows of the
 // next tile are asked for while the last one is multiplied: the loads in flight do not end at a tile's end.
@@ -543,11 +545,11 @@ extern "C" int mn_stream_kloop_grouped(const uint16_t* Y, int y_rows, const uint
   return nz;
 }
 
-// The grouped bf16 product of the decoder's steps, and the slabs it may write (the callers' buffers).  us, an expert layer's gate and up (5632 x 2048) / down (2048 x 1408) of 64 experts,
+// The walk as a product of its own, and the slabs that it writes.  us, an expert layer's gate and up (2816 x 2048) / down (2048 x 1408) of 64 experts,
 // 6 a row, and two that all rows share, grid in two ranges -> walk: 3 rows 46.7 -> 36.7 / 22.1 -> 21.5, 3 rows with the same experts 25.1 -> 19.2 / 17.3 -> 13.5, 4 51.1 -> 47.7 / 32.9 -> 26.1
 // (four slabs), 6 64.3 -> 58.4 / 36.2 -> 31.7, 8 77.1 -> 76.5 / 40.7 -> 38.9, 16 103 -> 100 / 55.6 -> 52.3, 20 126 -> 116 / 65.6 -> 59.7, 24 rows of 12 sets of experts 89.8 -> 83.0 / 51.0 -> 43.3
 // (three; with two a share is no less than a tile: 98.7 / 48.2).  Above 32 rows the blocks of 16 read the shared experts four times: 33 rows 119 -> 128 / 72.3 -> 65.8, 48 127 -> 133 /
-// 74.8 -> 71.3, 64 131 -> 141 / 76.9 -> 74.6 (two), so there only where the grid's last round would be mostly empty.
+// 74.8 -> 71.3, 64 131 -> 141 / 76.9 -> 74.6 (two).
 extern "C" int mn_stream_kwalk_slices(int max_rows, int K) {
   const int nch = (K + 63) / 64, want = max_rows <= 4 ? 4 : (max_rows <= 32 ? 3 : 2);
   return nch < want ? nch : want;
@@ -555,14 +557,36 @@ extern "C" int mn_stream_kwalk_slices(int max_rows, int K) {
 extern "C" int mn_stream_kwalk_grouped(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G,
                                        int max_rows, int Ntot, int K, void* stream) {
   const int nz = mn_stream_kwalk_slices(max_rows, K);
-  MN_CHECK_ARG(Y && W && P && off && G >= 1 && max_rows >= 1 && max_rows <= 64 && Ntot >= 1 && K >= 8 && (K % 8) == 0, "mn_stream_kwalk_grouped: bad args");
-  const int64_t places = 2 * (int64_t)mn_num_cus(), wgs = mn_cdiv(mn_cdiv(Ntot, 16), 2 * KW) * nz * G;
-  if (G > 256 || (max_rows > 32 && 5 * wgs >= 4 * mn_cdiv(wgs, places) * places))
-    return mn_stream_kloop_grouped(Y, y_rows, W, w_stride, P, p_rows, off, xrows, G, max_rows, 0, nz, Ntot, K, stream);
+  MN_CHECK_ARG(Y && W && P && off && G >= 1 && G <= 256 && max_rows >= 1 && max_rows <= 64 && Ntot >= 1 && K >= 8 && (K % 8) == 0, "mn_stream_kwalk_grouped: bad args");
   const KGroups g{off, xrows, w_stride, 0, max_rows, 0, 0};
-  hipLaunchKernelGGL(stream_kwalk_kernel, dim3((unsigned)places), dim3(KW * 64), 0, mn_stream(stream), Y, (int64_t)y_rows * K, W, P, (int64_t)p_rows * Ntot, Ntot, K, nz, G, g);
+  hipLaunchKernelGGL(stream_kwalk_kernel, dim3(2 * (unsigned)mn_num_cus()), dim3(KW * 64), 0, mn_stream(stream), Y, (int64_t)y_rows * K, W, P, (int64_t)p_rows * Ntot, Ntot, K, nz, G, g);
   MN_CHECK_LAUNCH("mn_stream_kwalk_grouped");
   return nz;
+}
+
+// Whether the walk is the faster one for `picks` groups a row, by an estimate of both, us: the grid's rounds of 512 workgroups, each half a tile's chunks at 0.93 or the live weights at
+// 6.0 TB/s behind 3.3, against the walk's longest share at 0.94 a chunk or its chunks of 256 columns at 7.6 TB/s behind 6.0 (the list of tiles, and its loads' second round trip; rates are those
+// of this estimate of the live groups).  Which groups are live only the device knows: as many as picks at random leave.  Few tiles make few shares, none less than a tile / (nz - 1), and small matrices do not pay for the list: us, grid / walk,
+// 8 experts of 384 x 512, 16 rows 5.4 / 8.7; 8 of 1408 x 1024 5 rows 9.6 / 13.0; 16 of 1024 x 2048 64 rows 25.6 / 44; 128 of 384 x 2048 64 rows 39.9 / 47.3; 128 of 1408 x 2048 32 rows 126 / 109.  Over 324
+// draws of experts, sizes and rows the faster one but for 1.5 % of the time, worst where rows share all their experts (6 rows in pairs, down 23.7 / 27.2).  Above 32 rows only where the
+// grid's last round would be mostly empty besides.
+static bool kwalk_pays(int G, double picks, int max_rows, int Ntot, int K, int nz) {
+  const double places = 2.0 * mn_num_cus(), live = G * (1.0 - pow(1.0 - fmin(1.0, picks / G), max_rows)), mb = 256 * 64 * 2 * 1e-6;
+  const int nch = (K + 63) / 64, tiles = (Ntot + 255) / 256, half = (nch + 1) / 2;
+  const int64_t wgs = (int64_t)tiles * 2 * G, all = (int64_t)places;
+  if (G > 256 || (max_rows > 32 && 5 * wgs >= 4 * mn_cdiv(wgs, all) * all)) return false;
+  double grid = 3.3;
+  for (double left = live * tiles * 2; left > 1e-9; left -= places) grid += fmax(0.93 * half, fmin(left, places) * half * mb * Ntot / (256.0 * tiles) / 6.0);
+  const double share = fmax(live * ceil(max_rows * picks / live / 16) * tiles * nch / places, nz > 1 ? (nch + nz - 2) / (nz - 1) : nch);
+  return 6.0 + fmax(0.94 * share, live * tiles * nch * mb / 7.6) < grid;
+}
+// The grouped bf16 product of the decoder's steps: the walk, or the grid form in the two ranges of mn_stream_mfma_grouped.
+extern "C" int mn_stream_experts(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G, int max_rows,
+                                 int Ntot, int K, void* stream) {
+  MN_CHECK_ARG(G >= 1 && max_rows >= 1 && K >= 8, "mn_stream_experts: bad args");
+  if (kwalk_pays(G, (double)p_rows / max_rows, max_rows, Ntot, K, mn_stream_kwalk_slices(max_rows, K)))
+    return mn_stream_kwalk_grouped(Y, y_rows, W, w_stride, P, p_rows, off, xrows, G, max_rows, Ntot, K, stream);
+  return mn_stream_kloop_grouped(Y, y_rows, W, w_stride, P, p_rows, off, xrows, G, max_rows, 0, K > 64 ? 2 : 1, Ntot, K, stream);
 }
 
 // Grouped form on 8-bit weights (group g: Wq + g * w_stride bytes, wscale + g * s_stride floats).

@@ -1,6 +1,6 @@
-"""Expert products of a decoder step that a resident set of workgroups shares in equal parts (3 rows and more; the down projection also above 32), against the same rows one by one,
-which take none of it: row counts where the number of slabs changes, groups of one row and of all, blocks of 16 rows and one row more, widths of whole and of part chunks and
-column tiles, fewer chunks than workgroups and many more.  bf16 hi / lo operands against fp32 ones, two layers: 2^-17 each of a handful of products, 1e-4 of a row's norm."""
+"""Expert products of a decoder step, in the grid form or (many tiles) shared in equal parts by a resident set of workgroups, against the same rows one by one, which take neither: row
+counts where the number of slabs changes, groups of one row and of all, blocks of 16 rows and one row more, layers on both sides of the rule.  bf16 hi / lo operands against fp32 ones,
+two layers: 2^-17 each of a handful of products, 1e-4 of a row's norm.  And both forms by themselves against float64."""
 import pytest
 import torch
 
@@ -55,19 +55,21 @@ def test_rows_together_and_alone(rows, hidden, inter, experts, top, shared):
     assert float(err[same].max()) < 1e-4, err
 
 
-@pytest.mark.parametrize("rows,N,K", [(16, 2816, 2048), (24, 2816, 2048), (24, 2048, 1408), (64, 2048, 1408)])
-def test_error_of_whole_tiles(rows, N, K):
-    """Enough tiles that a workgroup's share holds whole ones: their two chains of K / 2 are as long as those of the grid form's two ranges, so the error against float64 is no larger than
-    its (same operands; half a percent for the draw)."""
+def internal(name):
     import ctypes
     import os
     from ming_univision_amd import _lib
+    f = getattr(ctypes.CDLL(os.path.join(os.path.dirname(_lib.LIB_PATH), "libmingnative_dev.so")), name)
+    f.restype, f.argtypes = _lib.SYMBOLS["mn_stream_mfma_grouped"]
+    return f
+
+
+def products(rows, G, slots, N, K):
+    """A walk and a grid product of the same `slots` groups a row, as (slabs' sum, its float64 value, float64 sums of magnitudes)."""
+    from ming_univision_amd import _lib
     from ming_univision_amd._lib import ptr
-    dev = ctypes.CDLL(os.path.join(os.path.dirname(_lib.LIB_PATH), "libmingnative_dev.so"))
-    fn = dev.mn_stream_kwalk_grouped
-    fn.restype, fn.argtypes = _lib.SYMBOLS["mn_stream_mfma_grouped"]
-    G, slots = 64, 8
-    g = torch.Generator(device="cuda").manual_seed(rows + N)
+    walk = internal("mn_stream_kwalk_grouped")
+    g = torch.Generator(device="cuda").manual_seed(rows + N + K)
     picks = torch.stack([torch.randperm(G, device="cuda", generator=g)[:slots] for _ in range(rows)]).flatten()
     order, count = torch.argsort(picks, stable=True), torch.bincount(picks, minlength=G)
     src = (order // slots).int().contiguous()
@@ -77,13 +79,43 @@ def test_error_of_whole_tiles(rows, N, K):
     x = torch.randn(rows, K, device="cuda", generator=g)
     Y = torch.stack([x.bfloat16(), (x - x.bfloat16().float()).bfloat16()]).contiguous()
     x64, pairs = (Y[0].double() + Y[1].double())[src.long()], rows * slots
-    want = torch.cat([x64[int(off[e]):int(off[e + 1])] @ W[e].double().t() for e in range(G)])
-    out = torch.empty(4, pairs, N, device="cuda")
+    parts = [(x64[int(off[e]):int(off[e + 1])], W[e].double().t()) for e in range(G)]
+    want, size = torch.cat([a @ w for a, w in parts]), torch.cat([a.abs() @ w.abs() for a, w in parts])
 
-    def error(f):
-        out.fill_(float("nan"))
+    def run(f):
+        out = torch.full((4 * pairs + 1, N), float("nan"), device="cuda")
         nz = f(ptr(Y), rows, ptr(W), N * K, ptr(out), pairs, ptr(off), ptr(src), G, rows, N, K, torch.cuda.current_stream().cuda_stream)
-        assert 1 <= nz <= 4
-        return float((out[:nz].sum(0).double() - want).norm() / want.norm())
-    walk, grid = error(fn), error(_lib.lib().mn_stream_mfma_grouped)
-    assert walk <= 1.005 * grid, (walk, grid)
+        assert 1 <= nz <= 4 and bool(out[nz * pairs:].isnan().all())
+        return out[:nz * pairs].view(nz, pairs, N).sum(0).double()
+    return run(walk), run(_lib.lib().mn_stream_mfma_grouped), want, size
+
+
+@pytest.mark.parametrize("rows,N,K", [(16, 2816, 2048), (24, 2816, 2048), (24, 2048, 1408), (64, 2048, 1408)])
+def test_error_of_whole_tiles(rows, N, K):
+    """Enough tiles that a workgroup's share holds whole ones: their two chains of K / 2 are as long as those of the grid form's two ranges, so the error against float64 is that of the
+    grid but for the draw; rounding errors grow with the square root of a chain's length or faster, so a single chain of K would be between 1.1 (where the operands' products are most of it) and 1.4 times as far."""
+    walk, grid, want, _ = products(rows, 64, 8, N, K)
+    walk, grid = (float((y - want).norm() / want.norm()) for y in (walk, grid))
+    assert walk <= 1.05 * grid, (walk, grid)
+
+
+@pytest.mark.parametrize("rows,G,slots,N,K", [(1, 1, 1, 1, 8), (3, 1, 1, 257, 64), (4, 4, 3, 72, 72), (5, 12, 12, 255, 128), (16, 8, 2, 384, 512), (17, 3, 3, 512, 200), (32, 256, 4, 40, 320),
+                                              (33, 2, 2, 300, 1408), (64, 16, 1, 1024, 136), (64, 256, 16, 8, 64)])
+def test_products(rows, G, slots, N, K):
+    """Both forms at the edges: one group and 256, one row to 64 of a group, fewer chunks than workgroups, part chunks and part column tiles, one slab to four.  2 K products and their sums in fp32,
+    in some order: 2^-24 of the magnitudes each."""
+    walk, grid, want, size = products(rows, G, slots, N, K)
+    bound = (2 * K + 16) * 2.0 ** -24 * size
+    assert bool(((walk - want).abs() <= bound).all()) and bool(((grid - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("rows,G,slots,N,K,walks", [(16, 10, 4, 384, 512, 0), (5, 8, 4, 1408, 1024, 0), (5, 66, 6, 384, 256, 0), (3, 66, 8, 2816, 2048, 1), (24, 66, 8, 2048, 1408, 1)])
+def test_few_tiles_take_the_grid(rows, G, slots, N, K, walks):
+    """Two slabs are the grid's; the walk leaves three or four up to 32 rows.  Layers of few or small tiles took up to 1.7 times as long in the walk."""
+    from ming_univision_amd._lib import ptr
+    W, Y = torch.zeros(G, N, K, dtype=torch.bfloat16, device="cuda"), torch.zeros(2, rows, K, dtype=torch.bfloat16, device="cuda")
+    pairs = rows * slots
+    off = (torch.arange(G + 1, device="cuda") * pairs // G).to(torch.int32)
+    src, out = torch.arange(pairs, device="cuda", dtype=torch.int32) % rows, torch.empty(4, pairs, N, device="cuda")
+    nz = internal("mn_stream_experts")(ptr(Y), rows, ptr(W), N * K, ptr(out), pairs, ptr(off), ptr(src), G, rows, N, K, torch.cuda.current_stream().cuda_stream)
+    assert (nz > 2) == bool(walks)

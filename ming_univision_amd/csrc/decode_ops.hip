@@ -380,6 +380,9 @@ extern "C" int mn_rope_kv_append(const float* qkv, int64_t ldqkv, int M, int n_q
 // cover 4 consecutive q heads (= one GQA group when n_q/n_kv == 4, so K/V lines are shared in L1).
 // partial layout: [M][n_q][S][HD + 2]  (acc[HD], m, l)
 // -------------------------------------------------------------------------------------------
+// A row of up to 16 splits' keys is split that finely; a longer one into 16 or splits of four times the keys, 31 at most (with the counters they fit the scratch of 32 splits): us a layer of a
+// step of one row, 16 splits at most / these: 4000 keys 34.0 / 34.0, 16000 55.9 / 47.2, 31000 77.5 / 58.9.
+constexpr int JOIN_SHORT = 16, JOIN_LONG = 4, JOIN_MOST = 31, JOIN_ROWS = 128;
 // What mn_attn_decode_fused's launch takes instead of q: the RAW QKV projection; the rotary embedding of the row's q and new k, the q scale and the K / V append of the new token
 // happen in the attention launch.
 struct AttnFuse {
@@ -794,24 +797,87 @@ __global__ __launch_bounds__(1024) void attn_decode_one_kernel(
 // What bounds it is latency: the kernel's arguments, the row's numbers, K and V together, the partial results, the arrival, the join are one round trip each.
 //   * a lane group of 16 owns a key; it keeps its own running maximum, sum and G outputs, so that nothing crosses lanes inside the key loop but the score itself;
 //   * K and V of U keys a group are asked for at once, before the query is rotated;
-//   * a split is at least `keys` long: a short row is one split, which needs no join (the grid is sized for the cache, the row's length is known here);
+//   * a split is at least `keys` long: a short row is one split, which needs no join;
+//   * rows of one step differ in length, which only the device knows: with `fill` every workgroup reads all rows' lengths (one round trip, as its own row's alone would be), a row gets as
+//     many of `fill` splits a key head as its share of all keys is, at least one, and the workgroup's index says whose split it is; those behind the last one leave;
 //   * partials leave write-through (agent scope) and are drained before the arrival is counted; the last arrival (one counter a (row, KV head), zero between launches)
 //     reads them past its L1 in split order: the result does not depend on who is last.
 // -------------------------------------------------------------------------------------------
+__device__ __forceinline__ int join_splits(int len, int keys, int most) {
+  const int n = (len + keys - 1) >> __builtin_ctz(keys);
+  return len <= keys + keys / 2 ? 1 : min(most, n <= JOIN_SHORT ? n : max(JOIN_SHORT, (n + JOIN_LONG - 1) / JOIN_LONG));
+}
+// inclusive prefix sum over the lanes
+__device__ __forceinline__ int wave_prefix(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);      // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);      // row_bcast 15 into rows 1 and 3, 31 into rows 2 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+
 template <int HD, int G, int NW, int U, int WPE>
 __global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q, int n_kv, int64_t t_max, const int32_t* __restrict__ row_seq, const int32_t* __restrict__ row_len,
-                                                                   const uint8_t* __restrict__ key_mask, int64_t ld_mask, int S_max, int keys, float* __restrict__ partial,
+                                                                   const uint8_t* __restrict__ key_mask, int64_t ld_mask, int S_max, int keys, int fill, float* __restrict__ partial,
                                                                    uint32_t* __restrict__ arrived, float* __restrict__ out, bf16_t* __restrict__ split, const AttnFuse fz) {
-  constexpr int half = HD / 2, PER = HD / 16, V4 = PER / 4, GR = 4 * NW, N = G * PER, TH = NW * 64;
+  constexpr int half = HD / 2, PER = HD / 16, V4 = PER / 4, GR = 4 * NW, N = G * PER, TH = NW * 64, RL = JOIN_ROWS / 64;
   __shared__ __attribute__((aligned(16))) float qs[G * HD], knew[HD], vnew[HD];
   __shared__ __attribute__((aligned(16))) float part[NW][G * HD], mw[NW][G], lw[NW][G];
   __shared__ uint32_t last;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), sub = lane & 15, row4 = lane >> 4, grp = wave * 4 + row4;
-  const int m = blockIdx.x, kvh = blockIdx.y, s = blockIdx.z;
-  const int len = row_len[m], slot = fz.row_slot[m];
-  const int64_t seq = row_seq[m];
-  const int S = len <= keys + keys / 2 ? 1 : min(S_max, (len + keys - 1) / keys);
-  if (s >= S) return;                                    // uniform
+  const int kvh = blockIdx.y;
+  int m, s, S, len, slot, first;                         // first: the row's first slot among the partial results
+  int64_t seq;
+  if (fill == 0) {
+    m = blockIdx.x;
+    s = blockIdx.z;
+    len = row_len[m];
+    slot = fz.row_slot[m];
+    seq = row_seq[m];
+    S = join_splits(len, keys, S_max);
+    if (s >= S) return;                                  // uniform
+    first = m * S_max;
+  } else {
+    const int c = (fz.M + 63) >> 6, idx = blockIdx.z;    // rows lane * c .. + c - 1 are this lane's
+    int l[RL], at[RL], sq[RL], n[RL], own = 0, cnt = 0;
+#pragma unroll
+    for (int i = 0; i < RL; ++i) {
+      const int r = lane * c + i;
+      l[i] = at[i] = sq[i] = 0;
+      if (i < c && r < fz.M) { l[i] = row_len[r]; at[i] = fz.row_slot[r]; sq[i] = row_seq[r]; }
+      own += l[i];
+    }
+    const float share = (float)fill * 1.00001f * __builtin_amdgcn_rcpf(fmaxf(wave_sum((float)own), 1.f));      // (a whole number of splits stays one; they are `fill` together at most)
+#pragma unroll
+    for (int i = 0; i < RL; ++i) {
+      n[i] = 0;
+      if (i < c && lane * c + i < fz.M) n[i] = max(1, min(join_splits(l[i], keys, S_max), (int)((float)l[i] * share)));
+      cnt += n[i];
+    }
+    const int upto = wave_prefix(cnt);
+    if (idx >= __builtin_amdgcn_readlane(upto, 63)) return;      // uniform
+    const int src = __builtin_ctzll(__ballot(upto > idx));
+    first = __builtin_amdgcn_readlane(upto, src) - __builtin_amdgcn_readlane(cnt, src);
+    int i0 = 0;
+    S = __builtin_amdgcn_readlane(n[0], src);
+    len = __builtin_amdgcn_readlane(l[0], src);
+    slot = __builtin_amdgcn_readlane(at[0], src);
+    seq = __builtin_amdgcn_readlane(sq[0], src);
+#pragma unroll
+    for (int i = 1; i < RL; ++i)
+      if (i < c && idx >= first + S) {                   // uniform
+        first += S;
+        i0 = i;
+        S = __builtin_amdgcn_readlane(n[i], src);
+        len = __builtin_amdgcn_readlane(l[i], src);
+        slot = __builtin_amdgcn_readlane(at[i], src);
+        seq = __builtin_amdgcn_readlane(sq[i], src);
+      }
+    m = src * c + i0;
+    s = idx - first;
+  }
   const int chunk = (len + S - 1) / S, j0 = s * chunk, j1 = min(len, j0 + chunk);
   const float* Kb = fz.kv_cache_w + ((seq * 2 + 0) * n_kv + kvh) * t_max * HD + sub * PER;
   const float* Vb = fz.kv_cache_w + ((seq * 2 + 1) * n_kv + kvh) * t_max * HD + sub * PER;
@@ -949,7 +1015,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q,
   }
   __syncthreads();
   // ---- the waves' results meet in LDS; they are the row's (one split) or leave as the split's ----
-  float* base = partial + ((int64_t)m * n_q + kvh * G) * S_max * (HD + 2);
+  float* base = partial + ((int64_t)first * n_q + (int64_t)kvh * G * S) * (HD + 2);      // [query head][split]
   auto put = [&](int g, int d, float lt, float at) {
     float val;
     if (lt > 0.f) {
@@ -989,7 +1055,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q,
       put(g, d, lt, at);
       continue;
     }
-    float* o = base + ((int64_t)g * S_max + s) * (HD + 2);
+    float* o = base + ((int64_t)g * S + s) * (HD + 2);
     __hip_atomic_store(o + d, at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (d == 0) {
       __hip_atomic_store(o + HD, top, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1006,7 +1072,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q,
   if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (int t = tid; t < G * HD; t += TH) {               // (whole waves of one head; S <= 64: lane z holds split z's statistics)
     const int g = t / HD, d = t % HD;
-    const float* p = base + (int64_t)g * S_max * (HD + 2);
+    const float* p = base + (int64_t)g * S * (HD + 2);
     auto ld = [&](int z, int i) { return __hip_atomic_load(p + (int64_t)z * (HD + 2) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     float ms = -INFINITY, ls = 0.f, x[16], a = 0.f;
     if (lane < S) { ms = ld(lane, HD); ls = ld(lane, HD + 1); }
@@ -1127,20 +1193,38 @@ extern "C" int mn_attn_fused_ok(int M, int n_q, int n_kv, int hd) {
   const int ratio = n_kv > 0 && n_q % n_kv == 0 ? n_q / n_kv : 0;
   return M >= 1 && (hd == 64 || hd == 128) && (ratio == 1 || ratio == 2 || ratio == 4);
 }
-// a split of 64 KB of K and V: what a workgroup asks for at once
-static int attn_join_keys(int hd) { return 64 * 128 / hd; }
-static int attn_join_splits(int M, int n_kv, int hd, int64_t t_max) {
-  const int64_t most = mn_cdiv(t_max, attn_join_keys(hd)), fill = mn_num_cus() / ((int64_t)M * n_kv);
-  const int64_t s = most < fill ? most : fill;
-  return s < 1 ? 1 : (s > 16 ? 16 : (int)s);
+// Splits of a launch.  keys: 64 KB of K and V, what a workgroup asks for at once.  Where all rows can have all the splits their lengths allow, or a row has few of them, their number is that of
+// rows of one length: as many as make one round of the CUs.  Else, up to 128 rows, the lengths say (fill splits a key head), and with more rows 1024 keys are a split.  us a layer of a step with
+// small experts, a number of splits for all rows / this: 36 rows of 100 keys but one of 8000 223 / 56, 64 of 200 but one of 16000 550 / 73, 100 of 100 but one of 4000 166 / 64, 200 183 / 114; rows
+// of one length 3 x 1900 43.5 / 44.3, 36 x 1100 75.2 / 74.7, 64 x 1100 94.8 / 94.4, 100 x 1100 132 / 130.  The lengths cost 0.3 .. 0.7 (2 rows of 330 keys 30.5 / 31.3: not there), of 200 rows 3.7
+// (4 a lane: not there); empty workgroups of 1024 keys' splits 2 (200 rows of 100 keys, cache of 8192, 79.7 / 81.8).
+struct JoinPlan { int most, keys, fill, z; int64_t slots; };
+static JoinPlan attn_join_plan(int M, int n_kv, int hd, int64_t t_max) {
+  constexpr int LONG_KEYS = 1024, SHORT = 8;
+  JoinPlan p{1, 64 * 128 / hd, 0, 1, 0};
+  const int64_t fill = mn_num_cus() / n_kv;
+  if (M > JOIN_ROWS) p.keys = LONG_KEYS;
+  int64_t most = mn_cdiv(t_max, p.keys);
+  if (most > JOIN_MOST) most = JOIN_MOST;
+  if (M <= JOIN_ROWS && most > fill) most = fill;
+  p.fill = M <= JOIN_ROWS && M * most > fill && most > SHORT && t_max < 1 << 24 ? (int)fill : 0;      // (128 lengths' sum is of 32 bits)
+  if (M <= JOIN_ROWS && !p.fill && most > fill / M) most = fill / M;
+  if (most <= 1 || t_max <= p.keys + p.keys / 2) return JoinPlan{1, p.keys, 0, 1, 0};
+  p.most = p.z = (int)most;
+  p.slots = M * most;
+  if (p.fill) {
+    if (p.slots > M + fill) p.slots = M + fill;          // rows of one split, and the rest shares `fill`
+    p.z = (int)p.slots;
+  }
+  return p;
 }
-// The arrival counters of mn_attn_decode_fused, behind the partials in the scratch that mn_attn_decode_workspace_bytes sizes (its 32 splits of 32 keys are more than these): [M][n_kv],
+// The arrival counters of mn_attn_decode_fused, behind the partials in the scratch that mn_attn_decode_workspace_bytes sizes: [M][n_kv],
 // to be zeroed once before a step's first layer (*n words); NULL: one split a row, which needs none.
 extern "C" uint32_t* mn_attn_arrivals(int M, int n_q, int n_kv, int hd, int64_t t_max, void* workspace, size_t workspace_bytes, int* n) {
-  const int S = attn_join_splits(M, n_kv, hd, t_max);
-  const size_t part = (size_t)M * n_q * S * (hd + 2) * sizeof(float), need = part + (size_t)M * n_kv * sizeof(uint32_t);
+  const JoinPlan p = attn_join_plan(M, n_kv, hd, t_max);
+  const size_t part = (size_t)p.slots * n_q * (hd + 2) * sizeof(float), need = part + (size_t)M * n_kv * sizeof(uint32_t);
   *n = 0;
-  if (S == 1 || !workspace || need > workspace_bytes) return nullptr;
+  if (p.most == 1 || !workspace || need > workspace_bytes) return nullptr;
   *n = M * n_kv;
   return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(workspace) + part);
 }
@@ -1156,13 +1240,13 @@ extern "C" int mn_attn_decode_fused(const float* qkv, int64_t ldqkv, int nz, int
   AttnFuse fz;
   fz.qkv = qkv; fz.ldqkv = ldqkv; fz.nz = nz; fz.slab = slab; fz.rope = rope; fz.cos_tab = cos_tab; fz.sin_tab = sin_tab;
   fz.row_slot = row_slot; fz.row_pos = row_pos; fz.sec_t = sec_t; fz.sec_h = sec_h; fz.q_scale = q_scale; fz.M = M; fz.kv_cache_w = kv_cache;
-  const int S = arrived ? attn_join_splits(M, n_kv, hd, t_max) : 1, keys = attn_join_keys(hd);
+  const JoinPlan p = arrived ? attn_join_plan(M, n_kv, hd, t_max) : JoinPlan{1, 64 * 128 / hd, 0, 1, 0};
   const int64_t pairs = (int64_t)M * n_kv, cu = mn_num_cus();
   float* partial = reinterpret_cast<float*>(workspace);
-  const dim3 grid(M, n_kv, S);
+  const dim3 grid(p.fill ? 1 : M, n_kv, p.z);
   hipStream_t st = mn_stream(stream);
 #define MN_JOIN(HD_, G_, NW_, U_, W_) hipLaunchKernelGGL((attn_decode_join_kernel<HD_, G_, NW_, U_, W_>), grid, dim3(NW_ * 64), 0, st, n_q, n_kv, t_max, row_seq, row_len, key_mask, \
-                                                         ld_mask, S, keys, partial, arrived, out, split, fz)
+                                                         ld_mask, p.most, p.keys, p.fill, partial, arrived, out, split, fz)
   // from a workgroup a CU on: with one key a group in flight two of them fit a CU (1536 rows of 80 keys 195 -> 127 us, 64 rows 57 -> 55.5; 36 rows 37.4 -> 47); heads of 64, from four a
   // CU on: four waves each (64 rows of 40 keys 10.7 -> 9.6 us; 32 rows 9.9 -> 10.4)
 #define MN_JOIN_HD128(G_) do { if (pairs >= cu) MN_JOIN(128, G_, 8, 1, 4); else MN_JOIN(128, G_, 8, 2, 2); } while (0)

@@ -437,14 +437,15 @@ __global__ __launch_bounds__(1024) void rf_step_boundary_kernel(
   }
 }
 
-// semantic decoder input: de-normalise, Linear(in_dim -> D) + channel-repeat shortcut
-// (modeling_mingtok.py:168; vision_transformer.py:373-380)
-// (zero: n_zero words that the step's attention launches count arrivals in, here and in the two other kernels that start a step)
+// n_zero words that a step's attention launches count arrivals in: zeroed by the kernel that starts the step, or by itself
 __device__ __forceinline__ void zero_words(uint32_t* zero, int n_zero) {
   if (blockIdx.x == 0 && blockIdx.y == 0)
     for (int i = threadIdx.x; i < n_zero; i += blockDim.x) zero[i] = 0u;
 }
+__global__ void zero_words_kernel(uint32_t* __restrict__ zero, int n_zero) { zero_words(zero, n_zero); }
 
+// semantic decoder input: de-normalise, Linear(in_dim -> D) + channel-repeat shortcut
+// (modeling_mingtok.py:168; vision_transformer.py:373-380)
 __global__ void semdec_in_kernel(const float* __restrict__ latent, int in_dim, float scale, float mean,
                                  const bf16_t* __restrict__ w, const bf16_t* __restrict__ b, float* __restrict__ out,
                                  int D, uint32_t* __restrict__ zero, int n_zero) {

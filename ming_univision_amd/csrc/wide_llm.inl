@@ -130,6 +130,9 @@ static int llm_step_wide(const mn_llm* m, const float* x, int64_t ldx, int x_row
   WideGlue g;
   const bool f8 = llm_f8_mfma(m);
   const bool fuse_attn = (flags & MN_STEP_DISTINCT_SEQUENCES) && !span_tab && mn_attn_fused_ok(M, nq, nkv, hd);
+  int n_zero = 0;
+  uint32_t* arrived = fuse_attn ? mn_attn_arrivals(M, nq, nkv, hd, t_max, w.attn_ws, w.attn_ws_bytes, &n_zero) : nullptr;
+  if (arrived) hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(256), 0, st, arrived, n_zero);
   for (int l = 0; l <= m->n_layers; ++l) {
     // glue: (stack input | previous layer's expert combine + residual) -> RMSNorm(ln1 | final norm)
     const bool fin = l == m->n_layers;
@@ -149,9 +152,9 @@ static int llm_step_wide(const mn_llm* m, const float* x, int64_t ldx, int x_row
     a.c_zstride = (int64_t)M * qkv_dim;
     int nz = mn_gemm256_ex(&a, MN_G256_F32, w.ks_qkv, stream);
     if (nz < 0) return nz;
-    if (fuse_attn) {                                   // rows of distinct sequences: one launch, a split a row
+    if (fuse_attn) {                                   // rows of distinct sequences: one launch
       MN_TRY(mn_attn_decode_fused(w.pp, qkv_dim, nz, (int64_t)M * qkv_dim, M, nq, nkv, hd, 1, m->cos_tab, m->sin_tab, row_seq, row_slot, row_pos, m->mrope_sec_t,
-                                  m->mrope_sec_h, q_scale, kv_l, t_max, row_len, key_mask, ld_mask, nullptr, w.ya, nullptr, nullptr, stream));
+                                  m->mrope_sec_h, q_scale, kv_l, t_max, row_len, key_mask, ld_mask, nullptr, w.ya, w.attn_ws, arrived, stream));
     } else {
       MN_TRY(mn_rope_kv_from_partials(w.pp, qkv_dim, nz, (int64_t)M * qkv_dim, M, nq, nkv, hd, 1, m->cos_tab, m->sin_tab, row_seq,
                                       row_slot, row_pos, m->mrope_sec_t, m->mrope_sec_h, q_scale, w.q, kv_l, t_max, stream));

@@ -1,6 +1,7 @@
 """Decode attention that appends the new key itself and splits a row's keys over workgroups, the last of which joins them (decoder steps of rows of distinct sequences), against
 the launches that steps without that promise take: rows of one key, at the edges of a batch of keys and of the first split, up to the cache's end; row counts from one row to more than
-a workgroup a CU; one to four query heads a key head of 64 and of 128; holes in the mask and a row that attends nothing.  Both sum fp32 products of at most 1400 keys in
+a workgroup a CU; one to four query heads a key head of 64 and of 128; holes in the mask and a row that attends nothing; one long row among short ones (splits by the rows' lengths up to 128
+rows, of 1024 keys above).  Both sum fp32 products of at most 9000 keys in
 another order (1e-6 of the largest value), two layers and the products between them pass it on: 2e-5 of a row's norm."""
 import pytest
 import torch
@@ -50,6 +51,47 @@ def test_against_separate_launches(M, t_max, use_mask, n_q, n_kv, hd):
         assert torch.equal(got, again)
         assert float(((got - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-5
         assert float((kv1 - kv0).abs().max()) < 2e-5 * float(past.abs().max())
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd", [(4, 1, 128), (8, 2, 128), (4, 4, 64)])
+@pytest.mark.parametrize("M,t_max,long", [(2, 9000, 8999), (5, 9000, 9000), (36, 3000, 2900), (64, 1100, 1100), (65, 2500, 2500), (127, 1200, 1000), (128, 2049, 2049), (129, 2500, 2500), (200, 1537, 1537)])
+def test_one_long_row(M, t_max, long, n_q, n_kv, hd):
+    dec = decoder(n_q, n_kv, hd, t_max, M)
+    g = torch.Generator(device="cuda").manual_seed(M + t_max + hd)
+    past = torch.randn(dec.kv_cache.shape, generator=g, device="cuda")
+    x = torch.randn(M, 256, generator=g, device="cuda")
+    for turn in range(3):                                # the long row first, last and in between; the others from one key to 99, the second time all but one of a single key
+        slot = torch.randint(0, 99 if turn != 1 else 1, (M,), generator=g, device="cuda", dtype=torch.int32)
+        slot[(0, M - 1, M // 3)[turn]] = long - 1
+        seq = torch.randperm(M, generator=g, device="cuda").to(torch.int32)
+
+        def step(distinct):
+            dec.kv_cache.copy_(past)
+            return dec.step(x, seq, slot, slot, slot + 1, distinct_sequences=distinct).clone()
+        want, got, again = step(False), step(True), step(True)
+        assert torch.equal(got, again)
+        assert float(((got - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-5
+
+
+@pytest.mark.parametrize("M", [64, 100, 200])
+def test_a_long_row_is_shared(M):
+    """Sixteen thousand keys of one row among short ones, walked by one workgroup a key head, took nine times as long as the step without them; a step of that row alone says what they cost."""
+    def us(rows, longest):
+        dec = decoder(8, 2, 128, 16384, rows)
+        i32 = dict(dtype=torch.int32, device="cuda")
+        x, seq, slot = torch.randn(rows, 256, device="cuda"), torch.arange(rows, **i32), torch.full((rows,), 100, **i32)
+        slot[rows // 2] = longest
+        length, out, best = slot + 1, torch.empty(rows, 256, device="cuda"), 1e9
+        for _ in range(12):
+            a, b = torch.cuda.Event(True), torch.cuda.Event(True)
+            a.record()
+            for _ in range(8):
+                dec.step(x, seq, slot, slot, length, out=out, distinct_sequences=True)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+    assert us(M, 16000) < us(M, 100) + 2 * us(1, 16000)
 
 
 def test_replayed():

@@ -879,6 +879,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q,
     s = idx - first;
   }
   const int chunk = (len + S - 1) / S, j0 = s * chunk, j1 = min(len, j0 + chunk);
+  const int held = (int)min((int64_t)j1, t_max), behind = slot >= t_max && slot < j1 ? slot : -1;      // (a new key behind a full cache is attended, and kept nowhere)
   const float* Kb = fz.kv_cache_w + ((seq * 2 + 0) * n_kv + kvh) * t_max * HD + sub * PER;
   const float* Vb = fz.kv_cache_w + ((seq * 2 + 1) * n_kv + kvh) * t_max * HD + sub * PER;
   const uint8_t* mk = key_mask ? key_mask + (int64_t)m * ld_mask : nullptr;
@@ -887,9 +888,9 @@ __global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q,
   auto fetch = [&](int jb) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int j = jb + u * GR + grp, jc = min(j, j1 - 1);
-      keep[u] = j < j1;
-      if (keep[u] && mk) keep[u] = mk[j] != 0;
+      const int j = jb + u * GR + grp, jc = min(j, held - 1);
+      keep[u] = j < held || j == behind;
+      if (j < held && mk) keep[u] = mk[j] != 0;
 #pragma unroll
       for (int i = 0; i < V4; ++i) {
         k[u][i] = *reinterpret_cast<const f32x4*>(Kb + (int64_t)jc * HD + i * 4);
@@ -1027,7 +1028,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q,
       for (int j = 0; j < len; ++j) {
         float y = 0.f;
         if (j == slot) for (int z = 0; z < fz.nz; ++z) y += vp[(int64_t)z * fz.slab];      // (the arena's line of it may be another split's to write)
-        else y = Vd[(int64_t)j * HD];
+        else if (j < t_max) y = Vd[(int64_t)j * HD];
         sum += y;
       }
       val = len > 0 ? sum / (float)len : 0.f;

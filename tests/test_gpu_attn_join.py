@@ -73,6 +73,24 @@ def test_one_long_row(M, t_max, long, n_q, n_kv, hd):
         assert float(((got - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-5
 
 
+@pytest.mark.parametrize("M,t_max", [(1, 64), (3, 400), (24, 1100), (65, 96), (130, 1600)])
+def test_new_key_behind_a_full_cache(M, t_max):
+    """A slot of t_max is written nowhere and no line of the cache behind its last is read: the step attends the cache and the new key, as one whose cache has room for it does."""
+    dec, room = decoder(8, 2, 128, t_max, M), decoder(8, 2, 128, t_max + 1, M)
+    g = torch.Generator(device="cuda").manual_seed(M + t_max)
+    past = torch.randn(room.kv_cache.shape, generator=g, device="cuda")
+    x = torch.randn(M, 256, generator=g, device="cuda")
+    slot = torch.full((M,), t_max, device="cuda", dtype=torch.int32)
+    slot[:M // 2] = t_max // 2
+    seq, pos = torch.arange(M, device="cuda", dtype=torch.int32), slot.clamp(max=t_max - 1)
+    room.kv_cache.copy_(past)
+    want = room.step(x, seq, slot, pos, slot + 1, distinct_sequences=True)
+    dec.kv_cache.copy_(past[..., :t_max, :])
+    got = dec.step(x, seq, slot, pos, slot + 1, distinct_sequences=True)
+    assert float(((got - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-5
+    assert torch.equal(dec.kv_cache[:, M // 2:], past[:, M // 2:, ..., :t_max, :])
+
+
 @pytest.mark.parametrize("M", [64, 100, 200])
 def test_a_long_row_is_shared(M):
     """Sixteen thousand keys of one row among short ones, walked by one workgroup a key head, took nine times as long as the step without them; a step of that row alone says what they cost."""

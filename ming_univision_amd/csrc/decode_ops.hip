@@ -383,6 +383,7 @@ extern "C" int mn_rope_kv_append(const float* qkv, int64_t ldqkv, int M, int n_q
 // A row of up to 16 splits' keys is split that finely; a longer one into 16 or splits of four times the keys, 31 at most (with the counters they fit the scratch of 32 splits): us a layer of a
 // step of one row, 16 splits at most / these: 4000 keys 34.0 / 34.0, 16000 55.9 / 47.2, 31000 77.5 / 58.9.
 constexpr int JOIN_SHORT = 16, JOIN_LONG = 4, JOIN_MOST = 31, JOIN_ROWS = 128;
+static_assert(JOIN_MOST <= 64, "a lane a split");
 // What mn_attn_decode_fused's launch takes instead of q: the RAW QKV projection; the rotary embedding of the row's q and new k, the q scale and the K / V append of the new token
 // happen in the attention launch.
 struct AttnFuse {
@@ -1071,7 +1072,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q,
   __syncthreads();
   if (!last) return;
   if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  for (int t = tid; t < G * HD; t += TH) {               // (whole waves of one head; S <= 64: lane z holds split z's statistics)
+  for (int t = tid; t < G * HD; t += TH) {               // (whole waves of one head; lane z holds split z's statistics)
     const int g = t / HD, d = t % HD;
     const float* p = base + (int64_t)g * S * (HD + 2);
     auto ld = [&](int z, int i) { return __hip_atomic_load(p + (int64_t)z * (HD + 2) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
@@ -1086,7 +1087,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q,
 #pragma unroll
       for (int z = 0; z < 16; ++z) x[z] = z0 + z < S ? ld(z0 + z, d) : 0.f;
 #pragma unroll
-      for (int z = 0; z < 16; ++z) a = fmaf(lane_f(f, (z0 + z) & 63), x[z], a);
+      for (int z = 0; z < 16; ++z) a = fmaf(lane_f(f, z0 + z), x[z], a);
     }
     put(g, d, lt, a);
   }

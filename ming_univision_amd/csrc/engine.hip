@@ -36,9 +36,6 @@ extern "C" int mn_attn_decode_fused(const float* qkv, int64_t ldqkv, int nz, int
                                     const int32_t* row_pos, int sec_t, int sec_h, float q_scale, float* kv_cache, int64_t t_max,
                                     const int32_t* row_len, const uint8_t* key_mask, int64_t ld_mask, float* out, uint16_t* split,
                                     void* workspace, uint32_t* arrived, void* stream);
-extern "C" int mn_stream_mfma_grouped(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P,
-                                      int p_rows, const int32_t* off, const int32_t* xrows, int G, int max_rows,
-                                      int Ntot, int K, void* stream);
 extern "C" size_t mn_skinny_workspace_bytes_w8(int M, int N, int K, int epilogue);
 
 // ---- weight-format dispatch of the streaming launches (mingnative.h section 7): wfmt != 0 -> 8-bit bytes (e4m3 | int8) + fp32 row scales ----

@@ -631,8 +631,7 @@ static bool tile_launch(const G256& p, int form, int nz, bool hilo, hipStream_t 
 
 // The grouped products of few rows a group: row tiles of 32 or 64 of the list, rows and K-tiles as above.
 template <int EPI, int BM, int BN, int WM, int WN, int S, int GROUP>
-static void group_go(G256 p, hipStream_t st) {
-  p.group_m = 1;                                       // (bands of four row tiles: the same to 4 % slower)
+static void group_go(const G256& p, hipStream_t st) {
   const dim3 grid((unsigned)(p.max_mtiles * mn_cdiv(p.N, epi_paired(EPI) ? BN / 2 : BN)));
   hipLaunchKernelGGL((gemm_tile_kernel<EPI, true, BM, BN, WM, WN, S, false, GROUP>), grid, dim3(WM * WN * 64), 0, st, p);
 }

@@ -11,7 +11,7 @@
 //   * a workgroup asks for all it needs at once: its rows' LayerNorm input into registers, rows and weights by global_load_lds into up to 160 KiB of LDS, bias and residual;
 //   * tiles of 16 .. 64 rows by 16 .. 128 columns, the ones that bring a workgroup the fewest bytes while all of them are one round of the CUs;
 //   * LayerNorm is done again by every workgroup of a row tile (32 rows x 4 KB from its XCD's L2): that costs less than a launch of its own with its round trips, and
-//     no split-K slabs have to be summed by anyone: the eight waves split K inside the workgroup and meet in LDS once.
+//     no split-K slabs have to be summed by anyone: the eight waves split K inside the workgroup (in wide tiles four ways, and the columns two) and meet in LDS once.
 // us a launch with cold weights, these against a 64 x 64 tile launch and the launch that norms its rows or sums its slabs: 65 rows, 1024 -> 3072 7.5 / 7.7 + 4.6,
 // 1024 -> 1024 3.6 / 4.9 + 4.6, 2752 -> 1024 6.6 / 5.6 + 4.6, 1024 -> 2 x 2752 9.9 / 8.0 + 4.6; 256 rows, 1024 -> 4096 with GELU 12.2 / 10.5 + 5.2, 4096 -> 1024 10.8 / 8.8 + 5.2.
 // Of the 7.5: 0.7 until the first load (32-bit offsets, one multiply for the tile: 64-bit ones and a division took 1.1), 1.2 until all are issued (64 B a cycle), 1.4 for
@@ -305,7 +305,7 @@ double ln_time(const Form& f, int M, int64_t wrows, int K) {
 // Plain: 2.3 us, and 68 KB/us of its own or 5.3 TB/s of all weights (6.2 past the caches), whichever is longer, and somewhat more where they are near
 // each other; one round or nothing.  us, measured / this: 32 x 16 tiles of K = 1024 3.7 / 3.7, 32 x 32 of 1024 4.2 / 4.2, of 4096 9.7 / 10.0, of 8192 15.6 / 17.7, 64 x 32 of 1024 5.0 / 5.2, 64 x 64 of 4096
 // 16.6 / 17.7, 64 x 128 of 2048 15.9 / 13.9, of 8192 46.7 / 48.5; hi/lo, 16384 weight rows of 3072 (100 MB): 16 x 64 17.7 .. 18.2 / 19.4, 32 x 64 19.8 .. 20.9 / 20.3, 48 x 64 22.1 .. 23.8 / 21.7.
-constexpr Form forms[] = {{32, 1}, {16, 2}, {32, 2}, {32, 4}, {64, 2}, {64, 4}, {64, 8}}, hilo_forms[] = {{16, 2}, {32, 1}, {32, 2}, {32, 4}, {32, 6}, {32, 8}, {64, 2}, {64, 4}, {16, 4}, {48, 4}, {48, 6}};
+constexpr Form forms[] = {{32, 1}, {16, 2}, {32, 2}, {32, 4}, {64, 2}, {64, 4}, {64, 8}}, hilo_forms[] = {{16, 2}, {32, 1}, {32, 2}, {32, 4}, {32, 6}, {32, 8}, {64, 4}, {16, 4}, {48, 4}, {48, 6}};
 // (hi/lo 48 x 96, the one form whose waves' LDS reads take longer than its bytes, is 1025 rows by 1024 columns in one round: K = 1024 10.3 us, 2752 22.2, 4096 29.0; 64 x 64 tiles, 272 of them, 11.3, 24.2, 32.9)
 double own_time(const Form& f, bool hilo, int K) { return (f.bm * (hilo ? 2 : 1) + 16 * f.nj) * (double)K / (hilo && f.bm * f.nj > 256 ? 31e3 : 34e3); }
 // One row tile's weights nobody reads again, and where they take longer than all else they stream faster as non-temporal loads (16384 x 3072: 16 rows 20.0 -> 18.2 us, 36 rows 23.3 -> 22.1); smaller
@@ -337,10 +337,9 @@ void go_hilo(int form, const RowsGemm& p, hipStream_t st) {
     case 3: go<EPI, false, true, 32, 4, 4, 5>(p, st); break;
     case 4: go<EPI, false, true, 32, 6, 4, 4>(p, st); break;
     case 5: go<EPI, false, true, 32, 8, 4, 3>(p, st); break;
-    case 6: go<EPI, false, true, 64, 2, 4, 4>(p, st); break;
-    case 7: go<EPI, false, true, 64, 4, 4, 3>(p, st); break;
-    case 8: go<EPI, false, true, 16, 4, 8, 3>(p, st); break;
-    case 9: go<EPI, false, true, 48, 4, 4, 4>(p, st); break;
+    case 6: go<EPI, false, true, 64, 4, 4, 3>(p, st); break;
+    case 7: go<EPI, false, true, 16, 4, 8, 3>(p, st); break;
+    case 8: go<EPI, false, true, 48, 4, 4, 4>(p, st); break;
     default: go<EPI, false, true, 48, 6, 4, 3>(p, st); break;
   }
 }
@@ -394,11 +393,12 @@ extern "C" int mn_resid_gemm_rows(const uint16_t* A, int64_t lda, const uint16_t
   return MN_OK;
 }
 
-// One dense product of gemm256.hip, of tile_us on its tiles by its estimate: taken (1) where a form here is estimated a tenth faster, else 0 and nothing is launched.
+// One dense product of gemm256.hip, of tile_us on its tiles by its estimate: taken (1) where a form here is estimated a tenth faster (3 % where it reads weights past the caches, which the tiles'
+// estimate takes them not to), else 0 and nothing is launched.
 // us, the tiles / these, cold weights, 40, 101, 256 and 600 rows: hi/lo 768 -> 768 7.5 / 3.8, 7.8 / 3.9, 7.9 / 4.7, 8.1 / 6.0; 2048 -> 768 15.3 / 5.9, 15.5 / 6.0, 15.7 / 7.1, 15.9 / 10.6;
 // 768 -> 2304 7.7 / 4.1, 7.9 / 5.8, 8.4 / 6.8, tiles; 4096 -> 1024 27.3 / 8.5, 27.9 / 8.8, 27.6 / 11.8, 28.4 / 21.8; 1024 -> 2 x 2752 gated 10.4 / 8.1, 10.5 / 9.4, tiles (14.1).  Plain rows, 70, 250, 450 and
 // 1000: 1024 -> 1024 6.9 / 3.8, 6.9 / 4.5, 7.1 / 5.6, tiles (7.4); 2048 -> 2048 10.5 / 6.1, 10.9 / 7.7, 11.2 / 10.5, 17.4 / 16.0; 8192 -> 2048 34.0 / 16.3, 36.7 / 25.9, 36.7 / 31.7, 57.9 / 51.4; 1024 -> 4096
-// 7.0 / 5.5, tiles (7.4).  Gated products of fewer than 512 values stay (26 rows 320 -> 2 x 7976 5.3 / 5.7).  The error is smaller throughout (eight sums of K / 8: 1.0e-7 for 1.9e-7 of 64 bits at K = 2048).
+// 7.0 / 5.5, tiles (7.4).  Gated products of fewer than 512 values stay (26 rows 320 -> 2 x 7976 5.3 / 5.7).  The error is smaller throughout (eight sums of K / 8, or four of K / 4: 1.0e-7 for 1.9e-7 of 64 bits at K = 2048).
 extern "C" int mn_rows_gemm(const mn_g256* a, int epi, double tile_us, void* stream) {
   const bool hilo = a->a_lo_off != 0, paired = epi == MN_G256_SWIGLU_SPLIT;
   const bool known = epi == MN_G256_F32 || epi == MN_G256_F32_RESID || (hilo ? epi == MN_G256_BF16_SPLIT || paired : epi == MN_G256_BF16);
@@ -411,7 +411,7 @@ extern "C" int mn_rows_gemm(const mn_g256* a, int epi, double tile_us, void* str
   const auto time = [&](const Form& f) { return (paired && f.nj == 1) ? 1e30 : rows_time(f, hilo, a->M, rows, a->K); };
   const int form = hilo ? best_form(hilo_forms, time, &us) : best_form(forms, time, &us);
   const bool once = hilo && read_once(hilo_forms[form], true, a->M, rows, a->K);
-  if (us >= (once ? 0.97 : 0.9) * tile_us) return 0;      // (the tiles' estimate takes them to read as others do)
+  if (us >= (once ? 0.97 : 0.9) * tile_us) return 0;
   RowsGemm p{};
   p.once = once;
   p.A = a->A; p.lda = a->lda; p.a_lo = a->a_lo_off; p.W = a->W; p.ldw = a->ldw; p.bias = a->bias; p.pair = a->w_pair_rows; p.C = a->C; p.ldc = a->ldc; p.c_lo = a->c_lo_off;

@@ -778,7 +778,9 @@ MN_API int mn_gemm256_f8_slices(int K, int ksplit);
  *    sublayer results that are normalised before the residual add, and a polynomial-of-unit-norms feed-forward activation.
  *    Rows are fp32, weights bf16 [out, in]; every size and constant is a field or an argument.  The residual stream, norms,
  *    gates, softmax and the cached latents are fp32 in both arithmetic modes; `arith` chooses the matrix products:
- *    MN_SEQ_ARITH_BF16 = bf16 MFMA products with fp32 accumulation for steps of more than 8 rows (fp32 FMA below),
+ *    MN_SEQ_ARITH_BF16 = bf16 MFMA products with fp32 accumulation for steps of more than 8 rows (fp32 FMA below): how many rows a
+ *    call has chooses kernels and with them the order of fp32 sums, so a prompt's rows agree with those of the same prompt in another
+ *    call up to that order (and one unit of a bf16 rounding behind it), not to the bit,
  *    MN_SEQ_ARITH_F32 = fp32 FMA everywhere.
  * ------------------------------------------------------------------------------------------ */
 MN_API int mn_affine_ln_rows(const float* x, int64_t ldx, const uint16_t* w, const uint16_t* b, float eps, float* y, int64_t ldy,

@@ -299,7 +299,8 @@ class BailingMoeDecoder:
         x fp32 [M,H]; or [1,H] with rows=M to broadcast; or [M / x_row_div, H] with rows=M when the x_row_div CFG
         rows of an image share one embedding.  int32 device arrays per row; key_mask uint8 [M, >=len].
         distinct_sequences: every row is a different cache sequence and row_len == row_slot + 1 (a decode step, not a prefill
-        chunk) — RoPE and the K / V append then ride the attention launch (mn_llm_step_ex; same results).
+        chunk) — RoPE and the K / V append then ride the attention launch (mn_llm_step_ex; the same results up to the order
+        of fp32 sums).
         spans: a PREFILL chunk described as whole spans of cache sequences — a list of (seq, first row, length, past): rows
         [r0, r0 + len) are the slots [past, past + len) of sequence seq, in order, no key mask (mn_llm_step_spans: the wide route
         then runs tiled flash attention on hi/lo operands instead of row-by-row decode attention; same results).

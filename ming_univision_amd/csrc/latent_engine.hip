@@ -2,8 +2,8 @@
 // over the rows of a step as a chain of launches on the caller's stream.  Matrix products are routed per call:
 //   M <= 8 rows                      mn_skinny_gemm (weight streaming, fp32 FMA) — the decode route of the other decoder too
 //   MN_SEQ_ARITH_BF16, 9 .. 64 rows  mn_skinny_gemm's weight-streaming MFMA route on bf16 hi/lo rows (fp32-class products)
-//   MN_SEQ_ARITH_BF16, M > 64        mn_gemm_bf16 on the bf16 copy the producing kernel wrote (MFMA, fp32 accumulate)
-//   MN_SEQ_ARITH_F32, or a K that is no multiple of 8 / an unaligned weight: mn_gemm_f32_batched (fp32 FMA, more than 2 rows fp32 matrix cores)
+//   MN_SEQ_ARITH_BF16, M > 64        mn_gemm_bf16_parts on the bf16 copy the producing kernel wrote (MFMA, fp32 accumulate; the order of K follows the row count)
+//   MN_SEQ_ARITH_F32, or a K that is no multiple of 8 / an unaligned weight: mn_gemm_f32_batched (fp32 FMA; more than 2 rows, 8 where rows are not of whole 16 bytes: fp32 matrix cores)
 // The per-head absorb (q W_uk) and expand (latent W_uv^T) products are batched over heads in fp32 (mn_gemm_f32_batched) in both modes.
 #include "seq_linear.h"
 

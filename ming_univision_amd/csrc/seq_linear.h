@@ -1,8 +1,8 @@
 // seq_linear.h — product routing shared by the step functions of the sequence models (mingnative.h sections 9 and 10).
 //   M <= 8 rows                      mn_skinny_gemm (weight streaming, fp32 FMA)
 //   MN_SEQ_ARITH_BF16, 9 .. 64 rows  mn_skinny_gemm's weight-streaming MFMA route on bf16 hi/lo rows (fp32-class products)
-//   MN_SEQ_ARITH_BF16, M > 64        mn_gemm_bf16 on the bf16 copy the producing kernel wrote (MFMA, fp32 accumulate)
-//   MN_SEQ_ARITH_F32, or a K that is no multiple of 8 / an unaligned weight: mn_gemm_f32_batched (fp32 FMA, more than 2 rows fp32 matrix cores)
+//   MN_SEQ_ARITH_BF16, M > 64        mn_gemm_bf16_parts on the bf16 copy the producing kernel wrote (MFMA, fp32 accumulate; the order of K follows the row count)
+//   MN_SEQ_ARITH_F32, or a K that is no multiple of 8 / an unaligned weight: mn_gemm_f32_batched (fp32 FMA; more than 2 rows, 8 where rows are not of whole 16 bytes: fp32 matrix cores)
 #pragma once
 #include <string.h>
 

@@ -493,7 +493,8 @@ typedef struct mn_llm {
   int32_t arith;
 } mn_llm;
 
-/* up to 64 rows: serves the steps of every smaller row count too */
+/* up to 64 rows: serves the steps of every smaller row count too.  A step of up to 64 bf16 rows also runs in scratch that holds two slabs of each expert product and no more, which sizes for 65 rows and
+ * up may be. */
 MN_API size_t mn_llm_workspace_bytes(const mn_llm* m, int rows, int64_t t_max);
 MN_API int mn_llm_max_rows(const mn_llm* m);      /* 64, or 2048 (wide route: see mn_rf_max_rows) */
 /* x fp32 in (embeddings): row m is read from x + (m / x_row_div) * ldx (ldx == 0 broadcasts one row to all M

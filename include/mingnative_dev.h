@@ -54,7 +54,7 @@ MN_DEV_API int mn_stream_kwalk_grouped(const uint16_t* Y, int y_rows, const uint
                                        int max_rows, int Ntot, int K, void* stream);
 MN_DEV_API int mn_gemm_bf16_parts(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t ldw, const uint16_t* bias, void* C, int64_t ldc, int M, int N, int K, int epilogue, void* stream);
 MN_DEV_API int mn_stream_experts(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G, int max_rows,
-                                 int Ntot, int K, void* stream);
+                                 int Ntot, int K, int two_slabs, void* stream);
 
 #ifdef __cplusplus
 }

@@ -19,7 +19,7 @@ extern "C" int mn_stream_mfma_slices(int M, int Ntot, int K);
 extern "C" int mn_stream_mfma_grouped_slices(int G, int max_rows, int Ntot, int K);
 extern "C" int mn_stream_kwalk_slices(int max_rows, int K);
 extern "C" int mn_stream_experts(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G, int max_rows,
-                                 int Ntot, int K, void* stream);
+                                 int Ntot, int K, int two_slabs, void* stream);
 extern "C" int mn_rope_kv_from_partials(const float* qkv, int64_t ldqkv, int nz, int64_t slab, int M, int n_q, int n_kv, int hd,
                                         int rope, const float* cos_tab, const float* sin_tab, const int32_t* row_seq,
                                         const int32_t* row_slot, const int32_t* row_pos, int sec_t, int sec_h, float q_scale,
@@ -57,15 +57,15 @@ static inline int stream_dense(int wfmt, const uint16_t* Y, const void* W, const
 // grouped: w_stride counts weight ELEMENTS (= bytes for fp8), s_stride the row scales per group
 static inline int stream_grouped(int wfmt, const uint16_t* Y, int y_rows, const void* W, int64_t w_stride, const float* wscale, int64_t s_stride,
                                  float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G, int max_rows, int Ntot, int K,
-                                 void* stream) {
+                                 bool two_slabs, void* stream) {
   return wfmt ? mn_stream_mfma_grouped_wq(Y, y_rows, reinterpret_cast<const uint8_t*>(W), w_stride, wscale,
                                           s_stride * mn_wq_scales_per_row(wfmt, K), P, p_rows, off, xrows, G, max_rows, Ntot, K, wfmt, stream)
               : mn_stream_experts(Y, y_rows, reinterpret_cast<const uint16_t*>(W), w_stride, P, p_rows, off, xrows, G, max_rows, Ntot, K,
-                                  stream);
+                                  two_slabs, stream);
 }
-// slabs that stream_grouped writes at most (mn_stream_mfma_grouped_slices is the bound of the weight-only forms)
-static inline size_t stream_grouped_slabs(int wfmt, int G, int rows, int Ntot, int K) {
-  return (size_t)(wfmt ? mn_stream_mfma_grouped_slices(G, rows, Ntot, K) : mn_stream_kwalk_slices(rows, K));
+// slabs that stream_grouped writes at most (mn_stream_mfma_grouped_slices is the bound of the weight-only forms, and of bf16 with two_slabs)
+static inline size_t stream_grouped_slabs(int wfmt, int G, int rows, int Ntot, int K, bool two_slabs) {
+  return (size_t)(wfmt || two_slabs ? mn_stream_mfma_grouped_slices(G, rows, Ntot, K) : mn_stream_kwalk_slices(rows, K));
 }
 
 namespace {
@@ -986,7 +986,7 @@ struct MoeWs {
   float *p1, *p2;
 };
 
-static size_t moe_carve(Carver& cv, int wfmt, int rows, int H, int I, int G, int n_slot, MoeWs* o) {
+static size_t moe_carve(Carver& cv, int wfmt, int rows, int H, int I, int G, int n_slot, bool two_slabs, MoeWs* o) {
   const size_t P = (size_t)rows * n_slot;
   const size_t before = cv.off;
   o->off = cv.take<int32_t>((size_t)G + 1);
@@ -994,8 +994,8 @@ static size_t moe_carve(Carver& cv, int wfmt, int rows, int H, int I, int G, int
   o->pair_pos = cv.take<int32_t>(P);
   o->y1 = cv.take<bf16_t>((size_t)2 * rows * H);
   o->y2 = cv.take<bf16_t>(2 * P * I);
-  o->p1 = cv.take<float>(stream_grouped_slabs(wfmt, G, rows, 2 * I, H) * P * 2 * I);
-  o->p2 = cv.take<float>(stream_grouped_slabs(wfmt, G, rows, H, I) * P * H);
+  o->p1 = cv.take<float>(stream_grouped_slabs(wfmt, G, rows, 2 * I, H, two_slabs) * P * 2 * I);
+  o->p2 = cv.take<float>(stream_grouped_slabs(wfmt, G, rows, H, I, two_slabs) * P * H);
   return cv.off - before;
 }
 
@@ -1060,7 +1060,7 @@ struct LlmWs {
   size_t sk_ws_bytes;
 };
 
-static size_t llm_carve(const mn_llm* m, int rows, int64_t t_max, void* ws, size_t cap, LlmWs* o) {
+static size_t llm_carve(const mn_llm* m, int rows, int64_t t_max, void* ws, size_t cap, LlmWs* o, bool two_slabs = false) {
   Carver cv(ws, cap, ws == nullptr);
   const int n_slot = m->top_k + m->n_shared_slots;
   const int qkv_dim = (m->n_q + 2 * m->n_kv) * m->head_dim;
@@ -1077,7 +1077,7 @@ static size_t llm_carve(const mn_llm* m, int rows, int64_t t_max, void* ws, size
   o->attn_ws = cv.take<char>(o->attn_ws_bytes);
   o->sk_ws_bytes = sk_ws_need(rows, {{qkv_dim, m->hidden, 0}, {m->hidden, m->n_q * m->head_dim, 0}, {m->n_experts, m->hidden, 0}});
   o->sk_ws = cv.take<char>(o->sk_ws_bytes);
-  if (moe_mfma_ok(m, rows)) moe_carve(cv, m->wfmt, rows, m->hidden, m->moe_inter, m->n_experts + m->n_shared_slots, n_slot, &o->moe);
+  if (moe_mfma_ok(m, rows)) moe_carve(cv, m->wfmt, rows, m->hidden, m->moe_inter, m->n_experts + m->n_shared_slots, n_slot, two_slabs, &o->moe);
   if (llm_chain_ok(m, rows)) {
     const int ad = m->n_q * m->head_dim;
     o->yh = cv.take<bf16_t>((size_t)2 * rows * m->hidden);
@@ -1221,7 +1221,9 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
     return llm_step_wide(m, x, ldx, x_row_div, M, image_mask, row_seq, row_slot, row_pos, row_len, key_mask, ld_mask, kv_cache, n_seq, t_max,
                          hidden_out, workspace, workspace_bytes, flags, stream, span_tab, n_spans, span_max_len);
   LlmWs w{};
-  const size_t need = llm_carve(m, M, t_max, workspace, workspace_bytes, &w);
+  size_t need = llm_carve(m, M, t_max, workspace, workspace_bytes, &w);
+  const bool two_slabs = need > workspace_bytes;               // scratch sized for more than 64 rows may hold these steps' products in two slabs alone
+  if (two_slabs) need = llm_carve(m, M, t_max, workspace, workspace_bytes, &w, true);
   if (need > workspace_bytes) { mn_set_error("mn_llm_step: workspace %zu < %zu", workspace_bytes, need); return MN_ENOSPACE; }
   hipStream_t st = mn_stream(stream);
   const int H = m->hidden, hd = m->head_dim, nq = m->n_q, nkv = m->n_kv, I = m->moe_inter;
@@ -1298,12 +1300,12 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
       if (grouped) hipLaunchKernelGGL(moe_sort_pairs_kernel, dim3(1), dim3(1024), 0, st, w.ti, P, n_slot, G, w.moe.off, w.moe.xrows, w.moe.pair_pos);
       if (grouped) {
         nz = stream_grouped(m->wfmt, w.yh, M, m->w_gate_up[l], (int64_t)2 * I * H, m->wfmt ? m->w_gate_up_scale[l] : nullptr, 2 * I,
-                            w.moe.p1, P, w.moe.off, w.moe.xrows, G, M, 2 * I, H, stream);
+                            w.moe.p1, P, w.moe.off, w.moe.xrows, G, M, 2 * I, H, two_slabs, stream);
         if (nz < 0) return nz;
         hipLaunchKernelGGL(rf_glue_swiglu_split_kernel, dim3(mn_cdiv((int64_t)P * I, 1024)), dim3(256), 0, st, w.moe.p1, nz, P,
                            I, (const bf16_t*)nullptr, w.moe.y2);
         nz2 = stream_grouped(m->wfmt, w.moe.y2, P, m->w_down[l], (int64_t)H * I, m->wfmt ? m->w_down_scale[l] : nullptr, H, w.moe.p2, P,
-                             w.moe.off, nullptr, G, M, H, I, stream);
+                             w.moe.off, nullptr, G, M, H, I, two_slabs, stream);
         if (nz2 < 0) return nz2;
       } else {   // 2 rows: (row, expert) pairs on the fp32-FMA kernels, accumulated straight into h
         mn_skinny_args a = sk(w.xn, H, m->w_gate_up[l], H, nullptr, w.hmid, I, 1, I, H);
@@ -1373,12 +1375,12 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
       hipLaunchKernelGGL(moe_group_split_kernel, dim3(M + 1), dim3(256), 0, st, w.ti, M, n_slot, G, w.moe.off, w.moe.xrows,
                          w.moe.pair_pos, w.xn, H, w.moe.y1);
       int nz = stream_grouped(m->wfmt, w.moe.y1, M, m->w_gate_up[l], (int64_t)2 * I * H, m->wfmt ? m->w_gate_up_scale[l] : nullptr,
-                              2 * I, w.moe.p1, P, w.moe.off, w.moe.xrows, G, M, 2 * I, H, stream);
+                              2 * I, w.moe.p1, P, w.moe.off, w.moe.xrows, G, M, 2 * I, H, two_slabs, stream);
       if (nz < 0) return nz;
       hipLaunchKernelGGL(rf_glue_swiglu_split_kernel, dim3(mn_cdiv((int64_t)P * I, 1024)), dim3(256), 0, st, w.moe.p1, nz, P, I,
                          (const bf16_t*)nullptr, w.moe.y2);
       nz = stream_grouped(m->wfmt, w.moe.y2, P, m->w_down[l], (int64_t)H * I, m->wfmt ? m->w_down_scale[l] : nullptr, H, w.moe.p2, P,
-                          w.moe.off, nullptr, G, M, H, I, stream);
+                          w.moe.off, nullptr, G, M, H, I, two_slabs, stream);
       if (nz < 0) return nz;
       hipLaunchKernelGGL(moe_combine_resid_kernel, dim3(mn_cdiv((int64_t)M * H, 1024)), dim3(256), 0, st, w.moe.p2, nz,
                          (int64_t)P * H, M, H, n_slot, w.moe.pair_pos, w.tw, w.h);

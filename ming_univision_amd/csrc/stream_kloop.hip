@@ -580,11 +580,11 @@ static bool kwalk_pays(int G, double picks, int max_rows, int Ntot, int K, int n
   const double share = fmax(live * ceil(max_rows * picks / live / 16) * tiles * nch / places, nz > 1 ? (nch + nz - 2) / (nz - 1) : nch);
   return 6.0 + fmax(0.94 * share, live * tiles * nch * mb / 7.6) < grid;
 }
-// The grouped bf16 product of the decoder's steps: the walk, or the grid form in the two ranges of mn_stream_mfma_grouped.
+// The grouped bf16 product of the decoder's steps: the walk, or (also where P holds no more than its slabs: two_slabs) the grid form in the two ranges of mn_stream_mfma_grouped.
 extern "C" int mn_stream_experts(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G, int max_rows,
-                                 int Ntot, int K, void* stream) {
+                                 int Ntot, int K, int two_slabs, void* stream) {
   MN_CHECK_ARG(G >= 1 && max_rows >= 1 && K >= 8, "mn_stream_experts: bad args");
-  if (kwalk_pays(G, (double)p_rows / max_rows, max_rows, Ntot, K, mn_stream_kwalk_slices(max_rows, K)))
+  if (!two_slabs && kwalk_pays(G, (double)p_rows / max_rows, max_rows, Ntot, K, mn_stream_kwalk_slices(max_rows, K)))
     return mn_stream_kwalk_grouped(Y, y_rows, W, w_stride, P, p_rows, off, xrows, G, max_rows, Ntot, K, stream);
   return mn_stream_kloop_grouped(Y, y_rows, W, w_stride, P, p_rows, off, xrows, G, max_rows, 0, K > 64 ? 2 : 1, Ntot, K, stream);
 }

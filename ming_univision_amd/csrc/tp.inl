@@ -278,7 +278,7 @@ static bool llm_tp_ok(const mn_llm* m, const mn_llm_tp* tp, const mn_tp_comm* c,
          (tp->shared_inter == 0 || (tp->ws_gate_up && tp->ws_down));
 }
 
-static size_t llm_tp_carve(const mn_llm* m, const mn_llm_tp* tp, int rows, int64_t t_max, void* ws, size_t cap, LlmTpWs* o) {
+static size_t llm_tp_carve(const mn_llm* m, const mn_llm_tp* tp, int rows, int64_t t_max, void* ws, size_t cap, LlmTpWs* o, bool two_slabs = false) {
   // the wide route's carve on the SHARD's dimensions (local heads; n_experts = the global count: the router is replicated) ...
   size_t off = llm_wide_carve(m, rows, t_max, ws, cap, &o->w);
   Carver cv(ws ? (char*)ws + off : nullptr, cap > off ? cap - off : 0, ws == nullptr);
@@ -300,8 +300,8 @@ static size_t llm_tp_carve(const mn_llm* m, const mn_llm_tp* tp, int rows, int64
     const size_t s3 = (size_t)stream_slices(m->wfmt, rows, H, SIc) * rows * H;
     if (s3 > psh) psh = s3;
     o->pps = cv.take<float>(pmax * rows);
-    o->p1 = cv.take<float>(stream_grouped_slabs(m->wfmt, m->n_experts, rows, 2 * I, H) * Pn * 2 * I);
-    o->p2 = cv.take<float>(stream_grouped_slabs(m->wfmt, m->n_experts, rows, H, I) * Pn * H);
+    o->p1 = cv.take<float>(stream_grouped_slabs(m->wfmt, m->n_experts, rows, 2 * I, H, two_slabs) * Pn * 2 * I);
+    o->p2 = cv.take<float>(stream_grouped_slabs(m->wfmt, m->n_experts, rows, H, I, two_slabs) * Pn * H);
   }
   o->psh = cv.take<float>(psh);
   return off + cv.off;
@@ -335,7 +335,9 @@ extern "C" int mn_llm_step_tp(const mn_llm* m, const mn_llm_tp* tp, mn_tp_comm* 
   const int n_seg = 2 * ars * m->n_layers + 1;
   MN_CHECK_ARG(seg_begin >= 0 && seg_begin < seg_end && seg_end <= n_seg, "mn_llm_step_tp: segments [%d, %d) of %d", seg_begin, seg_end, n_seg);
   LlmTpWs tw;
-  const size_t need = llm_tp_carve(m, tp, M, t_max, workspace, workspace_bytes, &tw);
+  size_t need = llm_tp_carve(m, tp, M, t_max, workspace, workspace_bytes, &tw);
+  const bool two_slabs = need > workspace_bytes;       // (as mn_llm_step)
+  if (two_slabs) need = llm_tp_carve(m, tp, M, t_max, workspace, workspace_bytes, &tw, true);
   if (need > workspace_bytes) { mn_set_error("mn_llm_step_tp: workspace %zu < %zu", workspace_bytes, need); return MN_ENOSPACE; }
   LlmWideWs& w = tw.w;
   float* psh = tw.psh;
@@ -440,12 +442,12 @@ extern "C" int mn_llm_step_tp(const mn_llm* m, const mn_llm_tp* tp, mn_tp_comm* 
         // local experts on the grouped K-loop kernel: group g of the window = expert e0 + g, its rows are the sorted positions
         // [off[e0 + g], off[e0 + g + 1]) of the GLOBAL sort (gathered through perm); every distinct local expert is streamed once
         int nz1 = stream_grouped(m->wfmt, w.yh, M, m->w_gate_up[l], (int64_t)2 * I * H, m->wfmt ? m->w_gate_up_scale[l] : nullptr, 2 * I,
-                                 tw.p1, (int)P, w.off + e0, w.perm, e1 - e0, M, 2 * I, H, stream);
+                                 tw.p1, (int)P, w.off + e0, w.perm, e1 - e0, M, 2 * I, H, two_slabs, stream);
         if (nz1 < 0) return nz1;
         hipLaunchKernelGGL(rf_glue_swiglu_split_kernel, dim3(mn_cdiv(P * I, 1024)), dim3(256), 0, st, (const float*)tw.p1, nz1, (int)P, I,
                            (const bf16_t*)nullptr, w.y2, (const int32_t*)(w.off + e0), (const int32_t*)(w.off + e1));
         const int nz2 = stream_grouped(m->wfmt, w.y2, (int)P, m->w_down[l], (int64_t)H * I, m->wfmt ? m->w_down_scale[l] : nullptr, H,
-                                       tw.p2, (int)P, w.off + e0, nullptr, e1 - e0, M, H, I, stream);
+                                       tw.p2, (int)P, w.off + e0, nullptr, e1 - e0, M, H, I, two_slabs, stream);
         if (nz2 < 0) return nz2;
         p.cy = tw.p2; p.cy_nz = nz2; p.cy_slab = P * H;
         if (SI) {

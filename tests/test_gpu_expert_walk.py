@@ -117,5 +117,31 @@ def test_few_tiles_take_the_grid(rows, G, slots, N, K, walks):
     pairs = rows * slots
     off = (torch.arange(G + 1, device="cuda") * pairs // G).to(torch.int32)
     src, out = torch.arange(pairs, device="cuda", dtype=torch.int32) % rows, torch.empty(4, pairs, N, device="cuda")
-    nz = internal("mn_stream_experts")(ptr(Y), rows, ptr(W), N * K, ptr(out), pairs, ptr(off), ptr(src), G, rows, N, K, torch.cuda.current_stream().cuda_stream)
-    assert (nz > 2) == bool(walks)
+    f = internal("mn_stream_experts")
+    f.argtypes = f.argtypes[:-1] + [f.argtypes[-2], f.argtypes[-1]]
+    for two_slabs in (0, 1):                             # (and where the caller's scratch holds two: the grid whatever the tiles)
+        nz = f(ptr(Y), rows, ptr(W), N * K, ptr(out), pairs, ptr(off), ptr(src), G, rows, N, K, two_slabs, torch.cuda.current_stream().cuda_stream)
+        assert (nz > 2) == bool(walks and not two_slabs)
+
+
+@pytest.mark.parametrize("rows", [14, 15, 17])
+def test_scratch_of_more_rows(rows):
+    """Scratch sized for 65 rows holds a step of 14 .. 17 rows in two slabs a product, not in three: the step takes what there is.  Both orders of sums, fp32: 1e-4 of a row's norm as above."""
+    import ctypes
+    from ming_univision_amd._lib import lib
+    dec = decoder(1024, 1408, 64, 6, 2, rows)
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x, i32 = torch.randn(rows, 1024, generator=g, device="cuda"), dict(dtype=torch.int32, device="cuda")
+    seq, slot = torch.arange(rows, **i32), torch.full((rows,), 5, **i32)
+
+    def step():
+        dec.kv_cache.fill_(0.25)
+        return dec.step(x, seq, slot, slot, slot + 1, distinct_sequences=True).clone()
+    want = step()
+    (key, full), n = next(iter(dec._ws.items())), lib().mn_llm_workspace_bytes(ctypes.byref(dec.struct), 65, dec.t_max)
+    assert full.numel() > n
+    buf = torch.full((n + 4096,), 77, dtype=torch.uint8, device="cuda")
+    dec._ws[key] = buf[:n]
+    got = step()
+    assert bool((buf[n:] == 77).all())
+    assert float(((got - want).norm(dim=1) / want.norm(dim=1)).max()) < 1e-4

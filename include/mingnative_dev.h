@@ -55,6 +55,10 @@ MN_DEV_API int mn_stream_kwalk_grouped(const uint16_t* Y, int y_rows, const uint
 MN_DEV_API int mn_gemm_bf16_parts(const uint16_t* A, int64_t lda, const uint16_t* W, int64_t ldw, const uint16_t* bias, void* C, int64_t ldc, int M, int N, int K, int epilogue, void* stream);
 MN_DEV_API int mn_stream_experts(const uint16_t* Y, int y_rows, const uint16_t* W, int64_t w_stride, float* P, int p_rows, const int32_t* off, const int32_t* xrows, int G, int max_rows,
                                  int Ntot, int K, int two_slabs, void* stream);
+MN_DEV_API uint32_t* mn_attn_arrivals(int M, int n_q, int n_kv, int hd, int64_t t_max, void* workspace, size_t workspace_bytes, int* n);
+MN_DEV_API int mn_attn_decode_fused(const float* qkv, int64_t ldqkv, int nz, int64_t slab, int M, int n_q, int n_kv, int hd, int rope, const float* cos_tab, const float* sin_tab,
+                                    const int32_t* row_seq, const int32_t* row_slot, const int32_t* row_pos, int sec_t, int sec_h, float q_scale, float* kv_cache, int64_t t_max,
+                                    const int32_t* row_len, const uint8_t* key_mask, int64_t ld_mask, float* out, uint16_t* split, void* workspace, uint32_t* arrived, void* stream);
 
 #ifdef __cplusplus
 }

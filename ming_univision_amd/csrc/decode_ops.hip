@@ -1180,7 +1180,7 @@ extern "C" int mn_attn_decode_split(const float* q, int M, int n_q, int n_kv, in
 
 // Internal (engine.hip): RoPE + q scale + KV append + masked decode attention in ONE launch from the raw QKV projection (optionally as nz K-slice partial slabs): what
 // mn_rope_kv_append_3d / mn_rope_kv_from_partials followed by mn_attn_decode_split compute.  Rows of distinct sequences with row_len == row_slot + 1; n_q / n_kv in {1, 2, 4}.
-// Splits of a row: as many as make one round of the CUs with the other rows, 16 at most; arrived: mn_attn_arrivals' counters, zero (they are left zero), or NULL for one split a row.
+// arrived: mn_attn_arrivals' counters, zero (they are left zero), or NULL for one split a row.
 // us a launch over 24 layers' caches, the launches before (one workgroup a head up to 16 rows over 1024 keys; else the append, a launch of 32 splits and one that joins them; from
 // 40 (row, key head) pairs on a wave a key head) / this one.  16 heads of 128 over 4: 1 row of 80 keys 6.5 / 6.4, 330 13.1 / 7.7, 1100 13.0 / 9.7, 1900 16.9 / 9.9; 4 rows 7.1 / 7.5,
 // 13.3 / 8.9, 19.7 / 14.3, 27.0 / 15.7; 10 rows 7.7 / 7.6, 18.0 / 11.0, 25.7 / 16.4, 35.7 / 21.4; 36 rows 18.9 / 10.1, 22.8 / 18.0, 43.5 / 37.4, 64 / 57; 64 rows 19.6 / 11.3, 27.2 / 22.8,

@@ -2,7 +2,7 @@
 the launches that steps without that promise take: rows of one key, at the edges of a batch of keys and of the first split, up to the cache's end; row counts from one row to more than
 a workgroup a CU; one to four query heads a key head of 64 and of 128; holes in the mask and a row that attends nothing; one long row among short ones (splits by the rows' lengths up to 128
 rows, of 1024 keys above).  Both sum fp32 products of at most 9000 keys in
-another order (1e-6 of the largest value), two layers and the products between them pass it on: 2e-5 of a row's norm."""
+another order (1e-6 of the largest value), two layers and the products between them pass it on: 2e-5 of a row's norm.  And the launch by itself against float64."""
 import pytest
 import torch
 
@@ -89,6 +89,65 @@ def test_new_key_behind_a_full_cache(M, t_max):
     got = dec.step(x, seq, slot, pos, slot + 1, distinct_sequences=True)
     assert float(((got - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-5
     assert torch.equal(dec.kv_cache[:, M // 2:], past[:, M // 2:, ..., :t_max, :])
+
+
+def internal():
+    import ctypes
+    import os
+    from ming_univision_amd import _lib
+    dev = ctypes.CDLL(os.path.join(os.path.dirname(_lib.LIB_PATH), "libmingnative_dev.so"))
+    i, l, f, p = ctypes.c_int, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
+    dev.mn_attn_arrivals.restype, dev.mn_attn_arrivals.argtypes = p, [i, i, i, i, l, p, ctypes.c_size_t, p]
+    dev.mn_attn_decode_fused.restype, dev.mn_attn_decode_fused.argtypes = i, [p, l, i, l, i, i, i, i, i, p, p, p, p, p, i, i, f, p, l, p, p, l, p, p, p, p, p]
+    return dev
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd", [(8, 2, 128), (2, 1, 128), (4, 4, 64), (4, 1, 64)])
+@pytest.mark.parametrize("M,t_max,use_mask", [(1, 9000, False), (3, 400, True), (24, 1400, False), (65, 2500, True), (128, 1100, False), (150, 2500, False)])
+def test_against_float64(M, t_max, use_mask, n_q, n_kv, hd):
+    """The launch by itself, projections in three slabs, one long row among short ones.  Fp32: a score sums hd products whose magnitudes sum to about 0.64 sqrt(hd) in some twenty roundings (7e-6 at the
+    most, weights err twice that), values in chains of at most 9000 / 32: 3e-5 of a row's largest value."""
+    import ctypes
+    from ming_univision_amd._lib import lib, ptr
+    dev, half, nz, n = internal(), hd // 2, 3, ctypes.c_int()
+    g = torch.Generator(device="cuda").manual_seed(M + t_max + hd + n_q)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    kv, qkv, angle = rnd(M, 2, n_kv, t_max, hd), rnd(nz, M, n_q + 2 * n_kv, hd), 6.28 * torch.rand(t_max, half, generator=g, device="cuda")
+    cos, sin, seq = angle.cos(), angle.sin(), torch.randperm(M, generator=g, device="cuda").int()
+    slot = torch.randint(0, min(t_max, 300), (M,), generator=g, device="cuda").int()
+    slot[M // 2] = t_max - 1
+    length = slot + 1
+    mask = (torch.rand(M, t_max, generator=g, device="cuda") < 0.6).to(torch.uint8) if use_mask else None
+    if use_mask:
+        mask[0] = 0                                      # attends nothing: the mean of its values
+    cache, out, split, stream = kv.clone(), torch.empty(M, n_q, hd, device="cuda"), torch.empty(2, M, n_q, hd, dtype=torch.bfloat16, device="cuda"), torch.cuda.current_stream().cuda_stream
+    size = lib().mn_attn_decode_workspace_bytes(M, n_q, hd, t_max)
+    ws = torch.zeros(size // 4 + 64, dtype=torch.int32, device="cuda")
+    ws[size // 4:] = 77
+    arrived = dev.mn_attn_arrivals(M, n_q, n_kv, hd, t_max, ptr(ws), size, ctypes.byref(n))
+    assert dev.mn_attn_decode_fused(ptr(qkv), qkv[0, 0].numel(), nz, qkv[0].numel(), M, n_q, n_kv, hd, 1, ptr(cos), ptr(sin), ptr(seq), ptr(slot), ptr(slot), 0, 0, hd ** -0.5, ptr(cache), t_max,
+                                    ptr(length), ptr(mask), t_max if use_mask else 0, ptr(out), ptr(split), ptr(ws), arrived, stream) == 0
+    x = qkv.double().sum(0)
+    c, s = (t.double()[slot.long()][:, None] for t in (cos, sin))
+    turn = lambda a: torch.cat([a[..., :half] * c - a[..., half:] * s, a[..., half:] * c + a[..., :half] * s], -1)  # noqa: E731
+    q, k, v = turn(x[:, :n_q]) * hd ** -0.5, turn(x[:, n_q:n_q + n_kv]), x[:, n_q + n_kv:]
+    want = torch.empty(M, n_q, hd, dtype=torch.float64, device="cuda")
+    for m in range(M):
+        at = int(slot[m])
+        K, V = (kv[int(seq[m]), i, :, :at + 1].double() for i in (0, 1))
+        K[:, at], V[:, at] = k[m], v[m]
+        score = (K.repeat_interleave(n_q // n_kv, 0) @ q[m][:, :, None])[..., 0]
+        if use_mask:
+            score = score.masked_fill(mask[m, :at + 1] == 0, -torch.inf) if bool(mask[m, :at + 1].any()) else torch.zeros_like(score)
+        want[m] = (torch.softmax(score, -1)[:, None] @ V.repeat_interleave(n_q // n_kv, 0))[:, 0]
+        assert float((cache[int(seq[m]), 0, :, at].double() - k[m]).abs().max()) < 1e-5 and float((cache[int(seq[m]), 1, :, at].double() - v[m]).abs().max()) < 1e-5
+    err = (out.double() - want).abs().amax((1, 2)) / want.abs().amax((1, 2))
+    assert float(err.max()) < 3e-5, err
+    assert float((split.double().sum(0) - out.double()).abs().max()) < 2.0 ** -16 * float(out.abs().max())
+    assert bool((ws[size // 4:] == 77).all())
+    if arrived:
+        at = (arrived - ws.data_ptr()) // 4
+        assert bool((ws[at:at + n.value] == 0).all())
 
 
 @pytest.mark.parametrize("M", [64, 100, 200])

@@ -891,7 +891,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void attn_decode_join_kernel(int n_q,
     for (int u = 0; u < U; ++u) {
       const int j = jb + u * GR + grp, jc = min(j, held - 1);
       keep[u] = j < held || j == behind;
-      if (j < held && mk) keep[u] = mk[j] != 0;
+      if (mk && (j < held || (j == behind && j < ld_mask))) keep[u] = mk[j] != 0;      // (a mask of the cache's length alone says nothing of the key behind it)
 #pragma unroll
       for (int i = 0; i < V4; ++i) {
         k[u][i] = *reinterpret_cast<const f32x4*>(Kb + (int64_t)jc * HD + i * 4);

@@ -89,6 +89,16 @@ def test_new_key_behind_a_full_cache(M, t_max):
     got = dec.step(x, seq, slot, pos, slot + 1, distinct_sequences=True)
     assert float(((got - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-5
     assert torch.equal(dec.kv_cache[:, M // 2:], past[:, M // 2:, ..., :t_max, :])
+    for width in (t_max + 1, t_max):                     # a mask that covers the key behind the cache says of it too; one of the cache's length leaves it attended
+        masked, seen = (torch.ones(M, n, dtype=torch.uint8, device="cuda") for n in (width, t_max + 1))
+        masked[:, t_max // 3] = 0
+        masked[M // 2::2, t_max:] = 0
+        seen[:, :width] = masked
+        room.kv_cache.copy_(past)
+        want = room.step(x, seq, slot, pos, slot + 1, key_mask=seen, distinct_sequences=True)
+        dec.kv_cache.copy_(past[..., :t_max, :])
+        got = dec.step(x, seq, slot, pos, slot + 1, key_mask=masked, distinct_sequences=True)
+        assert float(((got - want).norm(dim=1) / want.norm(dim=1)).max()) < 2e-5
 
 
 def internal():

@@ -569,12 +569,13 @@ extern "C" int mn_stream_kwalk_grouped(const uint16_t* Y, int y_rows, const uint
 // of this estimate of the live groups).  Which groups are live only the device knows: as many as picks at random leave.  Few tiles make few shares, none less than a tile / (nz - 1), and small matrices do not pay for the list: us, grid / walk,
 // 8 experts of 384 x 512, 16 rows 5.4 / 8.7; 8 of 1408 x 1024 5 rows 9.6 / 13.0; 16 of 1024 x 2048 64 rows 25.6 / 44; 128 of 384 x 2048 64 rows 39.9 / 47.3; 128 of 1408 x 2048 32 rows 126 / 109.  Over 324
 // draws of experts, sizes and rows the faster one but for 1.5 % of the time, worst where rows share all their experts (6 rows in pairs, down 23.7 / 27.2).  Above 32 rows only where the
-// grid's last round would be mostly empty besides.
+// grid's last round would be mostly empty besides, and a share, a whole tile there, is left for no workgroup less: 48 experts of 1536 x 2048 are 288 tiles, which stream at 3.9 TB/s (33 rows 61.6 / 76.0, 64 rows
+// 65.0 / 78.5, with experts that most rows like 44.2 / 82.0); 17 of 4096 x 2048 64 rows 68.6 / 74.5.
 static bool kwalk_pays(int G, double picks, int max_rows, int Ntot, int K, int nz) {
   const double places = 2.0 * mn_num_cus(), live = G * (1.0 - pow(1.0 - fmin(1.0, picks / G), max_rows)), mb = 256 * 64 * 2 * 1e-6;
   const int nch = (K + 63) / 64, tiles = (Ntot + 255) / 256, half = (nch + 1) / 2;
   const int64_t wgs = (int64_t)tiles * 2 * G, all = (int64_t)places;
-  if (G > 256 || (max_rows > 32 && 5 * wgs >= 4 * mn_cdiv(wgs, all) * all)) return false;
+  if (G > 256 || (max_rows > 32 && (live * tiles < places || 5 * wgs >= 4 * mn_cdiv(wgs, all) * all))) return false;
   double grid = 3.3;
   for (double left = live * tiles * 2; left > 1e-9; left -= places) grid += fmax(0.93 * half, fmin(left, places) * half * mb * Ntot / (256.0 * tiles) / 6.0);
   const double share = fmax(live * ceil(max_rows * picks / live / 16) * tiles * nch / places, nz > 1 ? (nch + nz - 2) / (nz - 1) : nch);

@@ -124,6 +124,21 @@ def test_few_tiles_take_the_grid(rows, G, slots, N, K, walks):
         assert (nz > 2) == bool(walks and not two_slabs)
 
 
+@pytest.mark.parametrize("rows,G,slots,N,K,walks", [(33, 48, 8, 1536, 2048, 0), (64, 48, 8, 1536, 2048, 0), (64, 17, 3, 4096, 2048, 0), (64, 66, 8, 2048, 1408, 1)])
+def test_more_rows_take_the_grid(rows, G, slots, N, K, walks):
+    """Above 32 rows a workgroup of the walk has a whole tile at least: fewer tiles than workgroups took a quarter longer than the grid, with experts that most rows like nearly twice as long.
+    The walk zeros the second slab of a tile that one workgroup held; the grid has half of K there."""
+    from ming_univision_amd._lib import ptr
+    W, Y = torch.ones(G, N, K, dtype=torch.bfloat16, device="cuda"), torch.ones(2, rows, K, dtype=torch.bfloat16, device="cuda")
+    pairs = rows * slots
+    off = (torch.arange(G + 1, device="cuda") * pairs // G).to(torch.int32)
+    src, out = torch.arange(pairs, device="cuda", dtype=torch.int32) % rows, torch.empty(2, pairs, N, device="cuda")
+    f = internal("mn_stream_experts")
+    f.argtypes = f.argtypes[:-1] + [f.argtypes[-2], f.argtypes[-1]]
+    assert f(ptr(Y), rows, ptr(W), N * K, ptr(out), pairs, ptr(off), ptr(src), G, rows, N, K, 0, torch.cuda.current_stream().cuda_stream) == 2
+    assert bool((out.sum(0) == 2 * K).all()) and bool((out[1] == 0).any()) == bool(walks)
+
+
 @pytest.mark.parametrize("rows", [14, 15, 17])
 def test_scratch_of_more_rows(rows):
     """Scratch sized for 65 rows holds a step of 14 .. 17 rows in two slabs a product, not in three: the step takes what there is.  Both orders of sums, fp32: 1e-4 of a row's norm as above."""

@@ -91,7 +91,23 @@ __device__ __forceinline__ mn_u4_t fp8x8_to_bf16(uint32_t q0, uint32_t q1) {
 
 // ---- activations ----------------------------------------------------------------------------
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + __expf(-x)); }
-__device__ __forceinline__ float gelu_erf_f(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f)); }
+// Exact-erf GELU, x Phi(x) = max(x, 0) - |x| Phi(-|x|), with log2 Phi(-a) as a polynomial of degree 10: a weighted least-squares (Lawson) fit over 0 .. 6.5 of x Phi(x)'s absolute
+// error, 1.6e-10 before rounding, value at 0 exact; beyond it the polynomial falls on, so the tail goes to 0.  No subtraction of nearly equal numbers, unlike x (1 + erf) / 2 of a negative x:
+// relative 2-norm against 64 bits over normal x of deviation 1, 3 and 0.1: 2.8, 2.2 and 3.7e-8 (with a correctly rounded erf 3.7, 2.9 and 3.8e-8).  16 instructions, one of them exp2.
+__device__ __forceinline__ float gelu_erf_f(float x) {
+  const float a = fminf(fabsf(x), 16.0f);                  // (infinity times a tail of 0)
+  float q = fmaf(a, -5.39934142e-8f, 1.34703544e-6f);
+  q = fmaf(q, a, -1.48720201e-5f);
+  q = fmaf(q, a, 9.3071154e-5f);
+  q = fmaf(q, a, -3.20169347e-4f);
+  q = fmaf(q, a, 5.68195646e-5f);
+  q = fmaf(q, a, 6.90323347e-3f);
+  q = fmaf(q, a, -5.24251126e-2f);
+  q = fmaf(q, a, -4.59222823e-1f);
+  q = fmaf(q, a, -1.15110421f);
+  q = fmaf(q, a, -1.0f);
+  return fmaf(-a, __builtin_amdgcn_exp2f(q), fmaf(0.5f, fabsf(x), 0.5f * x));
+}
 // z (1 + tanh u) / 2 = z / (1 + exp(-2 u)): no cancellation on the negative side, where a norm behind it would magnify the error
 __device__ __forceinline__ float gelu_tanh_f(float z) { return z / (1.0f + expf(-1.5957691216057308f * (z + 0.044715f * z * z * z))); }
 // epilogues whose weights hold two row sets per output (the second set at row n + N)

@@ -123,32 +123,15 @@ __device__ __forceinline__ void g256_src_offsets(const G256& p, int wave, int la
     }
 }
 
-// Exact-erf GELU (nn.GELU(), mingtok mlp.py:34-40) for a bf16 result: erf by Abramowitz-Stegun 7.1.26 (|error| <= 1.5e-7, five
-// fma + rcp + exp2 where erff costs ~40 instructions; 128 values per lane of a 256 x 256 tile made erff 8 us of a 50 us tile).
-// The absolute error is 2^-14 of a bf16 ulp at |y| ~ 1; only the bf16 epilogue uses it.
-__device__ __forceinline__ float gelu_erf_bf16out(float x) {
-  const float z = fabsf(x) * 0.70710678118654752440f;
-  const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.0f));
-  float q = fmaf(1.061405429f, t, -1.453152027f);
-  q = fmaf(q, t, 1.421413741f);
-  q = fmaf(q, t, -0.284496736f);
-  q = fmaf(q, t, 0.254829592f);
-  const float e = q * t * __builtin_amdgcn_exp2f(-z * z * 1.4426950408889634f);      // 1 - erf(|x| / sqrt 2)
-  const float one_plus_erf = x >= 0.f ? 2.0f - e : e;
-  return 0.5f * x * one_plus_erf;
-}
-
 __host__ __device__ constexpr bool epi_split(int epi) { return epi == E_SWIGLU_SPLIT || epi == E_BF16_SPLIT; }
 __host__ __device__ constexpr bool epi_f32(int epi) { return epi == E_F32 || epi == E_F32_RESID || epi == E_F32_RESID_GATE || epi == E_F32_TAIL_RELU2; }
 
 __device__ __forceinline__ f32x4 bf16x4_f32(u32x2 b) { return f32x4{bf16lo_to_f32(b.x), bf16hi_to_f32(b.x), bf16lo_to_f32(b.y), bf16hi_to_f32(b.y)}; }
 
 // 4 consecutive output columns as bf16 (u: the paired "up" values; lo: the rest of a hi/lo pair).
-// EXACT_GELU: erff itself (the small-tile kernels, whose lanes hold 16 .. 32 values)
-template <int EPI, bool EXACT_GELU>
+template <int EPI>
 __device__ __forceinline__ void g256_pack(f32x4 v, f32x4 u, u32x2& hi, u32x2& lo) {
-  if (EPI == E_BF16_GELU && EXACT_GELU) v = f32x4{gelu_erf_f(v.x), gelu_erf_f(v.y), gelu_erf_f(v.z), gelu_erf_f(v.w)};
-  else if (EPI == E_BF16_GELU) v = f32x4{gelu_erf_bf16out(v.x), gelu_erf_bf16out(v.y), gelu_erf_bf16out(v.z), gelu_erf_bf16out(v.w)};
+  if (EPI == E_BF16_GELU) v = f32x4{gelu_erf_f(v.x), gelu_erf_f(v.y), gelu_erf_f(v.z), gelu_erf_f(v.w)};
   else if (EPI == E_GEGLU_BF16) v = f32x4{gelu_tanh_f(v.x) * u.x, gelu_tanh_f(v.y) * u.y, gelu_tanh_f(v.z) * u.z, gelu_tanh_f(v.w) * u.w};
   else if (epi_paired(EPI)) v = f32x4{silu_f(v.x) * u.x, silu_f(v.y) * u.y, silu_f(v.z) * u.z, silu_f(v.w) * u.w};
   if (EPI == E_BF16_RELU2) {                           // the squared relu of a feed-forward's hidden units
@@ -177,10 +160,11 @@ __device__ __forceinline__ u32x4 pair_lanes16(u32x2 a, u32x2 b) {
 // fragment before it has been stored, as the two might be the same memory, and its wait takes the store in too; so everything an epilogue reads is asked for
 // ahead of the stores: bias and scales of all columns at once, the residual a fragment row before it is added (two rows ahead measured the same, four spend
 // registers: 4112 x 1024 x 1024 21.1 and 22.1 us against 20.8).  With a bias, us, at its use -> ahead: residual 16384 x 1024 x 1024 48.3 -> 44.1, 16448 x 1024 x 4096
-// 181 -> 172, hi/lo 1025 x 768 x 768 9.5 -> 8.9; bf16 16384 x 3072 x 1024 110 -> 96, with GELU x 4096 162 -> 157.
+// 181 -> 172, hi/lo 1025 x 768 x 768 9.5 -> 8.9; bf16 16384 x 3072 x 1024 110 -> 96, with GELU x 4096 162 -> 157
+// (141 -> 138 with gelu_erf_f's polynomial, where a value took 23 issue slots of five fma, rcp and exp2, and 40 as erff in the small tiles).
 // bf16 results leave 16 bytes a lane where rows are of whole 16 bytes: two fragments' columns between lanes 16 apart (hi/lo rows of 1025 x 3072: 23.7 -> 21.7 us; 2048 x 3072 x 1024 21.8 -> 18.9); the 8-wave
 // kernel's gated units leave one fragment at a time (1409 x 4096 x 1024 of them 31.3 us, in pairs 32.4).
-template <int EPI, bool EXACT_GELU, bool F8, int MI, int NJ, class Row, class Col, class Val>
+template <int EPI, bool F8, int MI, int NJ, class Row, class Col, class Val>
 __device__ __forceinline__ void g256_out_b(const G256& p, char* Cz, const bool biased, int row0, int Mg, int grp, Row row, Col col, Val val) {
   constexpr bool paired = epi_paired(EPI), resid = EPI == E_F32_RESID || EPI == E_F32_RESID_GATE, gated = EPI == E_F32_RESID_GATE;
   constexpr bool at_once = paired && !epi_split(EPI) && MI == 8, pairs = !epi_f32(EPI) && NJ % 2 == 0 && !at_once;
@@ -249,7 +233,7 @@ __device__ __forceinline__ void g256_out_b(const G256& p, char* Cz, const bool b
       if (EPI == E_SWIGLU_BF16_SCALED) { v[j] *= rs[i]; u *= rs[i]; }
       if (gated) v[j] = res[i % AHEAD][j] + gt[i % AHEAD][j] * v[j];
       else if (resid) v[j] = res[i % AHEAD][j] + v[j];
-      if (!epi_f32(EPI)) g256_pack<EPI, EXACT_GELU>(v[j], u, hi[j], lo[j]);
+      if (!epi_f32(EPI)) g256_pack<EPI>(v[j], u, hi[j], lo[j]);
       if (at_once && m_ok && col(j) < p.N) *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(Cz) + m * p.ldc + col(j)) = hi[j];
     }
     if (resid && i + AHEAD < MI) ahead(i + AHEAD);
@@ -290,12 +274,12 @@ __device__ __forceinline__ void g256_out_b(const G256& p, char* Cz, const bool b
   }
 }
 
-template <int EPI, bool EXACT_GELU, bool F8, int MI, int NJ, class Row, class Col, class Val>
+template <int EPI, bool F8, int MI, int NJ, class Row, class Col, class Val>
 __device__ __forceinline__ void g256_out(const G256& p, char* Cz, int zslice, int row0, int Mg, int grp, Row row, Col col, Val val) {
   const bool biased = p.bias && zslice == 0;
   constexpr bool one = MI == 8 || epi_paired(EPI);     // one copy of the code (two spill accumulators of the 8-wave kernel)
-  if (one || !biased) g256_out_b<EPI, EXACT_GELU, F8, MI, NJ>(p, Cz, one && biased, row0, Mg, grp, row, col, val);
-  else g256_out_b<EPI, EXACT_GELU, F8, MI, NJ>(p, Cz, true, row0, Mg, grp, row, col, val);
+  if (one || !biased) g256_out_b<EPI, F8, MI, NJ>(p, Cz, one && biased, row0, Mg, grp, row, col, val);
+  else g256_out_b<EPI, F8, MI, NJ>(p, Cz, true, row0, Mg, grp, row, col, val);
 }
 
 // Epilogue of one output tile of the 8-wave kernel.
@@ -305,7 +289,7 @@ __device__ __forceinline__ void g256_epilogue(const G256& p, const f32x4 (&acc)[
   constexpr bool hilo = HILO, paired = epi_paired(EPI);
   char* Cz = reinterpret_cast<char*>(p.C);
   if (EPI == E_F32) Cz += (int64_t)zslice * p.c_zstride * 4;
-  g256_out<EPI, false, F8, hilo ? 4 : 8, paired ? 2 : 4>(
+  g256_out<EPI, F8, hilo ? 4 : 8, paired ? 2 : 4>(
       p, Cz, zslice, row0, Mg, grp, [&](int i) { return m0 + wr * (hilo ? 64 : 128) + i * 16 + fr; },
       [&](int j) { return n0 + wc * (paired ? 32 : 64) + j * 16 + fq * 4; },
       [&](int i, int j, f32x4& v, f32x4& u) {
@@ -534,7 +518,8 @@ extern "C" MN_DEV_API void mn_gemm256_tune_order(int group_m, int group_list) { 
 // twice pay for their epilogues from 6 (hi/lo 3) a CU on: 4100 x 6000 x 768 hi/lo 93 (256) against 122, 4096 x 4096 x 512 45 against 60.
 // Where the lines then lie, both sides measured: 65 x 3072 x 1024 bf16: 7.3 us (64 x 64) against 23.7 (256); 256 x 4096 x 1024: 8.2 against
 // 32.1; 1025 hi/lo rows x 1024 x 1024: 10.9 (64 x 64) against 22.3; x 3072: 20.0 (64 x 128) against 26.0; 2048 x 2048 x 8192: 79.6 (128 x 128) against 136.6;
-// 16384 x 1024 x 1024: 37.2 (256) against 54.2 (128 x 128); 1025 hi/lo rows x 2752 SwiGLU: 29.9 (256) against 37.8.
+// 16384 x 1024 x 1024: 37.2 (256) against 54.2 (128 x 128); 1025 hi/lo rows x 2752 SwiGLU: 29.9 (256) against 37.8.  With GELU the lines are the same (bf16 2048 x 4096 x 1024 24.2
+// (128 x 128) against 30.7 (256), x 256 12.2 against 22.6; 2600 rows 35.2 against 32.2).
 struct TileForm { int form, bm, bn; double fixed, alone, full, two, per; };
 static const TileForm tile_plain[] = {{1, 64, 64, 3.6, 0.23, 0.26, 0.42, 0.30}, {2, 64, 128, 3.9, 0.37, 0.40, 0.75, 0.48}, {3, 128, 128, 4.2, 0.50, 0.61, 0, 0},
                                       {4, 128, 128, 4.2, 0.55, 0.85, 1.16, 0.85}, {0, 256, 256, 11.0, 0.85, 1.30, 0, 0}};
@@ -568,13 +553,13 @@ static double tile_time(const TileForm& f, int M, int N, int k_tiles, int nz, bo
 }
 
 // the form of a dense M x N x K launch in nz K-slices of Kc, and the estimate of its time
-static int tile_form(int M, int N, int Kc, int nz, bool hilo, int epi, bool may256, double* us) {
+static int tile_form(int M, int N, int Kc, int nz, bool hilo, int epi, double* us) {
   const bool paired = epi_paired(epi);
   if (hilo && M <= 128) {
     int best = 0;
     double tb = 1e30;
     for (const FewForm& t : tile_few) {
-      if (M < t.min_m || M > t.max_m || (t.split && epi != E_SWIGLU_SPLIT) || (t.f.form == 0 && !may256)) continue;
+      if (M < t.min_m || M > t.max_m || (t.split && epi != E_SWIGLU_SPLIT)) continue;
       const double e = tile_time(t.f, M, N, Kc / BK, nz, true, paired);
       if (e < tb) { tb = e; best = t.f.form; }
     }
@@ -586,7 +571,6 @@ static int tile_form(int M, int N, int Kc, int nz, bool hilo, int epi, bool may2
   int best = 0;
   double tb = 1e30;
   for (int i = 0; i < n; ++i) {
-    if (t[i].form == 0 && !may256) continue;
     const double e = tile_time(t[i], M, N, Kc / BK, nz, hilo, paired);
     if (e < tb) { tb = e; best = t[i].form; }
   }
@@ -669,11 +653,8 @@ static int g256_launch(const G256& a, int epi, int ksplit, hipStream_t st) {
     else group_launch<E_SWIGLU_SPLIT>(p, st);
     return 1;
   }
-  // (the 256-tile kernel's GELU is the 1.5e-7 polynomial: it serves the problems of 128 tiles and more, where erff in the small tiles' epilogue costs more than they save:
-  // 4096 x 4096 x 256 26.9 us against 38.6, 8000 x 4000 x 192 45 against 69)
-  const bool may256 = epi != E_BF16_GELU || mn_cdiv(p.M, 256) * mn_cdiv(p.N, 256) >= 128;
   double us = 0;
-  const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : epi == E_BF16_GELU && may256 ? 0 : tile_form(p.M, p.N, p.Kc, nz, hilo, epi, may256, &us);
+  const int form = a.g_off || a.f8 ? 0 : g_g256_tile >= 0 ? g_g256_tile : tile_form(p.M, p.N, p.Kc, nz, hilo, epi, &us);
   // one row tile of a matrix that no cache holds (a vocabulary's logits): us at 126464 x 2048, the tiles below -> this: 5 rows 110 -> 86, 16 108 -> 91, 24 112 -> 98, 32 114 -> 101; 30000 x 5120 5 rows 56 -> 46,
   // 32 69 -> 53 (in the caches' reach the tiles below: 16384 x 3072 17 .. 20, this 23 .. 30).  Two workgroups a CU, and only where
   // their rounds are 0.7 full or all tiles have a CU of their own (98304 x 2048, 0.75 16 rows 87 -> 71; 80000, 0.61 65 -> 65; 66000, 0.50 59 -> 62).  Above 32 rows 64 x 256 tiles, one a CU, where their rounds are 0.85 full:
@@ -745,7 +726,7 @@ extern "C" int mn_gemm256_plan_ksplit(int M, int N, int K, int hilo) {
     const int Kc = ks == 1 ? K : (int)(mn_cdiv(mn_cdiv(K, ks), 2 * BK) * 2 * BK), nz = (int)mn_cdiv(K, Kc);
     if (nz != ks) continue;
     double t;
-    tile_form(M, N, Kc, nz, hilo != 0, E_F32, true, &t);
+    tile_form(M, N, Kc, nz, hilo != 0, E_F32, &t);
     t += nz * (double)M * N * 8.0 / 4.5e6;
     if (hilo && M <= 128) t += 0.25 * nz * fmin(1.0, N / 2048.0);         // (a few rows' slabs are read by a few workgroups)
     if (t < tb - 1e-9) { tb = t; best = ks; }

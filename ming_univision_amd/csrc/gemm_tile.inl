@@ -190,7 +190,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
     }
     return;
   }
-  g256_out<EPI, true, false, MI, paired ? (NJ + 1) / 2 : NJ>(
+  g256_out<EPI, false, MI, paired ? (NJ + 1) / 2 : NJ>(
       p, Cz, blockIdx.y, row0, Mg, grp, [&](int i) { return m0 + wm * (BM / WM) + i * 16 + fr; }, [&](int j) { return n0 + wn * (cols / WN) + j * 16 + fq * 4; },
       [&](int i, int j, f32x4& v, f32x4& u) {
         v = acc[i][j];

@@ -782,9 +782,7 @@ __global__ __launch_bounds__(1024) void latent_attn_kernel(const float* __restri
 // Latent attention on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands, fp32 accumulate — scores and weights stay
 // 32-bit).  A workgroup of 4 waves owns 16 query vectors (row, head) of one run of rows and walks its share of the sequence's latents
 // (LatentWalk, mfma_f32_tiles.h).
-// 32 rows of 16 heads over 2049 latents of 512 (134 MB, 28 us at the card's copy rate): 46 us (2.9 TB/s; a plain sum over
-// as much reaches 3.2); with the loads of the next tile waited for where they were issued, 16 keys a tile and four times the workgroups 60 us (8 rows: 60 us,
-// 18 here).
+// For few keys a workgroup and for latents of any size; long walks over latents of 128, 256, 384 or 512 are the form below's.
 struct PlainScore { __device__ __forceinline__ float operator()(float s) const { return s; } };
 template <int NB, int KF, bool VEC>
 __global__ __launch_bounds__(256, VEC && NB <= 8 ? 2 : 1) void latent_attn_mfma_kernel(const float* __restrict__ qabs, const float* __restrict__ arena,
@@ -831,6 +829,168 @@ __global__ __launch_bounds__(256, VEC && NB <= 8 ? 2 : 1) void latent_attn_mfma_
       part_ml[po * 2] = mrun;
       part_ml[po * 2 + 1] = lrun;
     }
+  }
+}
+
+// The same for latents of 16 NT values, up to 512: a wave takes whole tiles of 16 keys for itself, a running maximum and sum and the 16 NT x 16 sums of its own, and the four waves of a
+// workgroup meet once, at the end.  Nothing is exchanged between waves and no barrier stands in the walk.  The loads lie as the scores' A operand (lane: key l % 16, values 4 (l / 16) .. + 3
+// of every 16), so a tile goes from memory into registers and from there into the scores; the value products want it turned, which a tile of LDS that only this wave touches does.
+// A register that has been multiplied is asked for what follows half a tile further on: loads are in flight all the time.  What bounds it is memory in the walk (5.2 TB/s) and the ends, 5 us until
+// the first tile is there and 3 from the last one to the split's results.  us, the form above -> this, the splits' join with it: 32 rows of 16 heads over 2049 latents of 512 54.5 -> 44.4 (the walk alone
+// 41.7 -> 36.3; 134 MB, 23 us at the rate of a plain read), 64 rows over 1000 47.0 -> 40.7, 64 rows of 8 heads over 2048 of 256 39.1 -> 37.8; prompts of 2048, 1000, 300, 130 tokens, 16 heads over
+// latents of 512, 909 -> 760, 270 -> 240, 48.5 -> 43, 24.6 -> 22.7, 2048 tokens of 8 heads over 256 273 -> 222.
+// The sums are taken against a maximum that is raised only where a score is above it by more than 8 (weights up to e^8, which fp32 holds as well as 1): scaling sums that live in the
+// matrix cores' half of the registers would cost every tile a copy of them.  Error against 64 bits 1.4 .. 2.0e-7, the form above 1.7 .. 2.9e-7.
+__device__ __forceinline__ void wave_order() {         // what the lanes of a wave hand each other through LDS: the hardware keeps its order, this the compiler's
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+template <int NT>
+__global__ __launch_bounds__(256, NT <= 16 ? 2 : 1) void latent_attn_wave_kernel(const float* __restrict__ qabs, const float* __restrict__ arena, const int32_t* __restrict__ row_seq,
+                                                                                 const int32_t* __restrict__ row_len, const int32_t* __restrict__ blk_tab, int H, int t_max,
+                                                                                 float* __restrict__ lat, float* __restrict__ part_acc, float* __restrict__ part_ml, int KS, int M) {
+  constexpr int R = 16 * NT, LDK = R + 4, TILE = 16 * LDK, RG = NT % 16 == 0 ? 16 : 8;      // RG: loads of a lane in flight
+  static_assert(NT % RG == 0, "a ring slot keeps its place from tile to tile");
+  __shared__ __attribute__((aligned(16))) float lds[4 * TILE];
+  __shared__ float wm[4][16], wl[4][16];
+  __shared__ __attribute__((aligned(16))) float scale[NT > 16 ? 4 : 1][NT > 16 ? 1024 : 4];
+  const int row0 = blk_tab[2 * blockIdx.x], nrows = blk_tab[2 * blockIdx.x + 1];
+  const int nqv = nrows * H, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float* K = lds + wave * TILE;
+  // (one pass unless the grid was cut for runs of one row and this one is longer)
+  for (int qv0 = blockIdx.y * 16; qv0 < nqv; qv0 += 16 * gridDim.y) {
+    int lane = threadIdx.x & 63;
+    asm("" : "+v"(lane));                              // (what depends on it is not held over the passes: registers)
+    const int c = lane & 15, g4 = lane >> 4;
+    const int len = row_len[row0 + nrows - 1];
+    const bool on = qv0 + c < nqv;
+    const int qv = on ? qv0 + c : nqv - 1, mine = row_len[row0 + qv / H];
+    const int64_t o = (int64_t)(row0 + qv / H) * H + qv % H;
+    const float* kb = arena + (int64_t)row_seq[row0] * t_max * R + 4 * g4;
+    auto keys = [&](int tile) { return kb + (int64_t)min(16 * tile + c, len - 1) * R; };
+    // the run's own tiles in equal parts, a part's tiles to its waves in turn
+    const uint32_t n = (uint32_t)((len + 15) >> 4);
+    const int t1 = (int)((blockIdx.z + 1) * n / (uint32_t)KS);
+    int tile = (int)(blockIdx.z * n / (uint32_t)KS) + wave;
+    f32x4 k[RG], q[NT], acc[NT];
+    const float* p = keys(min(tile, (int)n - 1));
+    if (tile < t1) {
+#pragma unroll
+      for (int it = 0; it < RG; ++it) k[it] = *reinterpret_cast<const f32x4*>(p + 16 * it);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      const float* qr = qabs + o * R + 4 * g4;
+#pragma unroll
+      for (int it = 0; it < NT; ++it) q[it] = *reinterpret_cast<const f32x4*>(qr + 16 * it);
+    }
+#pragma unroll
+    for (int it = 0; it < NT; ++it) acc[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float mrun = -INFINITY, lrun = 0.f;
+    __builtin_amdgcn_s_waitcnt(0x0f70);                // (all of them, once: in the walk a wait for one register of the ring is then no wait for the others)
+    float* kw = K + c * LDK + 4 * g4;
+    const float* kr = K + 4 * g4 * LDK + c;
+    for (; tile < t1; tile += 4) {
+      const float* pn = keys(min(tile + 4, t1 - 1));      // (behind the last tile: something of this workgroup's, not used)
+      f32x4 s[8];                                      // eight chains of sums: no longer ones than those of four waves that split a key's values
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+      wave_order();                                    // the tile before has been read
+#pragma unroll
+      for (int it = 0; it < NT; ++it) {
+        *reinterpret_cast<f32x4*>(kw + 16 * it) = k[it % RG];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[it / (NT / 2) * 4 + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[it % RG][e], q[it][e], s[it / (NT / 2) * 4 + e], 0, 0, 0);
+        if (it + RG < NT) k[it % RG] = *reinterpret_cast<const f32x4*>(p + 16 * (it + RG));
+        else k[it % RG] = *reinterpret_cast<const f32x4*>(pn + 16 * (it + RG - NT));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      p = pn;
+      wave_order();
+      f32x4 w = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+      const int key0 = 16 * tile + 4 * g4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (key0 + i >= mine) w[i] = -INFINITY;
+      float mx = fmaxf(fmaxf(w[0], w[1]), fmaxf(w[2], w[3]));
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      if (__ballot(mx > mrun + 8.0f)) {
+        const float mnew = mx > mrun + 8.0f ? mx : mrun, corr = mrun == -INFINITY ? 0.f : fast_exp(mrun - mnew);
+        lrun *= corr;
+        const bool fresh = __ballot(mrun != -INFINITY) == 0;
+        mrun = mnew;
+        if (NT <= 16) {
+#pragma unroll
+          for (int x = 0; x < NT; ++x) acc[x] *= corr;
+        } else if (!fresh) {                           // the sums live in the matrix cores' half of the registers: scaled by way of LDS, or every tile would hold a copy of them
+          f32x4* z = reinterpret_cast<f32x4*>(scale[wave]) + lane;
+#pragma unroll
+          for (int x = 0; x < NT; x += 4) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) z[u * 64] = acc[x + u];
+            wave_order();
+#pragma unroll
+            for (int u = 0; u < 4; ++u) z[u * 64] *= corr;
+            wave_order();
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc[x + u] = z[u * 64];
+            wave_order();
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = w[i] == -INFINITY ? 0.f : fast_exp(w[i] - mrun);
+      lrun += (w[0] + w[1]) + (w[2] + w[3]);
+      float v[2][8];                                   // a group of eight products, the next one's values on their way
+      auto read = [&](int u) {
+#pragma unroll
+        for (int x = 0; x < 8; ++x) v[u & 1][x] = kr[(u / (NT / 8)) * LDK + 16 * (u % (NT / 8) * 8 + x)];
+      };
+      read(0);
+#pragma unroll
+      for (int u = 0; u < NT / 2; ++u) {
+        if (u + 1 < NT / 2) read(u + 1);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          f32x4& a = acc[u % (NT / 8) * 8 + x];
+          a = __builtin_amdgcn_mfma_f32_16x16x4f32(v[u & 1][x], w[u / (NT / 8)], a, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    lrun += __shfl_xor(lrun, 16);
+    lrun += __shfl_xor(lrun, 32);
+    // ---- the waves' results meet: wave w sums the column blocks w, w + 4, .. ----
+    if (g4 == 0) { wm[wave][c] = mrun; wl[wave][c] = lrun; }
+    wave_order();
+#pragma unroll
+    for (int x = 0; x < NT; ++x) *reinterpret_cast<f32x4*>(K + lane * 4 + x * 256) = acc[x];
+    __syncthreads();
+    float top = -INFINITY, l = 0.f, f[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) top = fmaxf(top, wm[u][c]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      f[u] = wm[u][c] == -INFINITY ? 0.f : fast_exp(wm[u][c] - top);
+      l = fmaf(f[u], wl[u][c], l);
+    }
+    const float inv = KS == 1 ? 1.0f / l : 1.0f;
+    float* dst = (KS == 1 ? lat + o * R : part_acc + ((int64_t)blockIdx.z * M * H + o) * R) + 16 * wave + 4 * g4;
+    const float* from = lds + wave * 256 + lane * 4;
+#pragma unroll
+    for (int y = 0; y < NT / 4; ++y) {
+      f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) a += f[u] * *reinterpret_cast<const f32x4*>(from + u * TILE + y * 1024);
+      if (on) *reinterpret_cast<f32x4*>(dst + 64 * y) = a * inv;
+    }
+    if (KS > 1 && on && wave == 0 && g4 == 0) {
+      const int64_t po = (int64_t)blockIdx.z * M * H + o;
+      part_ml[po * 2] = top;
+      part_ml[po * 2 + 1] = l;
+    }
+    __syncthreads();                                   // (another pass writes here)
   }
 }
 
@@ -1042,13 +1202,22 @@ static inline int latent_kt(int r, int variant) {
   return variant == MN_LATENT_ATTN_VALU ? (r <= 256 ? 64 : r <= 512 ? 32 : 16) : (r <= 512 ? 32 : 16);
 }
 
+static inline bool latent_wave(int r) { return r == 128 || r == 256 || r == 384 || r == 512; }
+// Whole tiles a wave: where a wave has two of them or more.  Below, the form whose waves share a tile is the faster one (us, shared / whole: 64 rows over 300 of 512 27.3 / 25.9 .. 28, 8 rows over 2049
+// 27.8 / 29.5, one 22.5 / 24.8, 64 over 64 11.6 / 14.1, 40 rows over 1111 of 256 22.4 / 27.9).
+static inline bool latent_by_wave(int r, int max_len, int ks) { return latent_wave(r) && max_len >= 128 * ks; }
+
 extern "C" int mn_latent_attn_splits(int n_blk, int max_len, int r) {
-  const int tiles = (int)mn_cdiv(max_len > 0 ? max_len : 1, 16);
-  int ks = (int)mn_cdiv(2 * (int64_t)mn_num_cus(), n_blk > 0 ? n_blk : 1);
+  const int tiles = (int)mn_cdiv(max_len > 0 ? max_len : 1, 16), blk = n_blk > 0 ? n_blk : 1;
   const int cap = (int)mn_cdiv(tiles, 4);              // a split works on at least 64 keys
+  int ks = (int)mn_cdiv(2 * (int64_t)mn_num_cus(), blk);      // two workgroups a CU
+  if (latent_wave(r)) {                                // one round of the form whose waves take whole tiles, where it is the one (latent_by_wave)
+    int kw = (r <= 256 ? 2 : 1) * mn_num_cus() / blk;
+    if (kw < 1) kw = 1;
+    if (latent_by_wave(r, max_len, kw)) ks = kw;
+  }
   if (ks > cap) ks = cap;
   if (ks > 64) ks = 64;
-  (void)r;
   return ks < 1 ? 1 : ks;
 }
 
@@ -1079,7 +1248,12 @@ extern "C" int mn_latent_attn_ex(const float* qabs, const float* arena, const in
 #define MN_LM(N_, F_, V_)                                                                                                           \
   hipLaunchKernelGGL((latent_attn_mfma_kernel<N_, F_, V_>), grid, dim3(256), 0, st, qabs, arena, row_seq, row_len, blk_tab, H, r, t_max, tps, lat, pacc, \
                      pml, ks, M)
-    if (r & 3) {                                         // (latents of any size but a multiple of 4 go value by value)
+    if (latent_by_wave(r, max_len, ks) && ((uintptr_t)qabs & 15) == 0 && ((uintptr_t)arena & 15) == 0 && ((uintptr_t)lat & 15) == 0 && ((uintptr_t)pacc & 15) == 0) {
+#define MN_LW(N_)                                                                                                                              \
+  hipLaunchKernelGGL((latent_attn_wave_kernel<N_>), grid, dim3(256), 0, st, qabs, arena, row_seq, row_len, blk_tab, H, t_max, lat, pacc, pml, ks, M)
+      if (r == 128) MN_LW(8); else if (r == 256) MN_LW(16); else if (r == 384) MN_LW(24); else MN_LW(32);
+#undef MN_LW
+    } else if (r & 3) {                                         // (latents of any size but a multiple of 4 go value by value)
       if (nbw <= 2) MN_LM(2, 2, false); else if (nbw <= 8) MN_LM(8, 2, false); else MN_LM(16, 1, false);
     } else {                                             // instantiated paddings: 64 .. 256, 384, 512, 768, 1024
       if (nbw == 1) MN_LM(1, 2, true); else if (nbw == 2) MN_LM(2, 2, true); else if (nbw == 3) MN_LM(3, 2, true); else if (nbw == 4) MN_LM(4, 2, true);

@@ -298,6 +298,7 @@ __global__ __launch_bounds__(256) void medium_epilogue_kernel(const mn_skinny_ar
 }
 
 #include "rows_kc.inl"
+#include "row_gemv.inl"
 
 int medium_ksplit(int Ntot, int K) {
   const int tiles = (Ntot + 127) / 128;
@@ -478,6 +479,10 @@ extern "C" int mn_skinny_gemm(const mn_skinny_args* args, void* stream) {
                "mn_skinny_gemm: weights must be 16-byte aligned");
   if (a.M >= 2 && ka.batch == 1 && ka.nseg == 1 && a.ldw == a.K && rows_kc(a, true, mn_stream(stream))) {
     MN_CHECK_LAUNCH("mn_skinny_gemm(rows)");
+    return MN_OK;
+  }
+  if (ka.batch == 1 && ka.nseg == 1 && row_gemv(a, mn_stream(stream))) {
+    MN_CHECK_LAUNCH("mn_skinny_gemm(row)");
     return MN_OK;
   }
   ka.nchunk = (a.K + 511) / 512;

@@ -1146,6 +1146,9 @@ extern "C" int mn_llm_max_rows(const mn_llm* m) { return llm_wide_ok(m, 2048) ? 
 extern "C" int mn_rf_max_rows(const mn_rf_head* h) { return rf_wide_ok(h, 2048) ? 2048 : 64; }
 extern "C" int mn_semdec_max_rows(const mn_semdec* s) { return sem_wide_ok(s, 2048) ? 2048 : 64; }
 
+// one row's routing as partial sums of the launch before it, behind that row's scratch; a step whose scratch ends before them routes without
+static size_t llm_gate_part_bytes(const mn_llm* m) { return moe_gate_parts_ok(m->hidden, m->n_experts) ? (size_t)(m->hidden / 8) * 65 * sizeof(float) : 0; }
+
 extern "C" size_t mn_llm_workspace_bytes(const mn_llm* m, int rows, int64_t t_max) {
   size_t need = 0;
   if (llm_wide_ok(m, rows)) {
@@ -1158,6 +1161,7 @@ extern "C" size_t mn_llm_workspace_bytes(const mn_llm* m, int rows, int64_t t_ma
     LlmWs w{};
     const size_t narrow = llm_carve(m, r, t_max, nullptr, 0, &w);
     if (narrow > need) need = narrow;
+    if (r == 1 && narrow + llm_gate_part_bytes(m) > need) need = narrow + llm_gate_part_bytes(m);
   }
   return need;
 }
@@ -1225,6 +1229,7 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
   const bool two_slabs = need > workspace_bytes;               // scratch sized for more than 64 rows may hold these steps' products in two slabs alone
   if (two_slabs) need = llm_carve(m, M, t_max, workspace, workspace_bytes, &w, true);
   if (need > workspace_bytes) { mn_set_error("mn_llm_step: workspace %zu < %zu", workspace_bytes, need); return MN_ENOSPACE; }
+  float* gate_part = M == 1 && llm_gate_part_bytes(m) && need + llm_gate_part_bytes(m) <= workspace_bytes ? reinterpret_cast<float*>((char*)workspace + need) : nullptr;
   hipStream_t st = mn_stream(stream);
   const int H = m->hidden, hd = m->head_dim, nq = m->n_q, nkv = m->n_kv, I = m->moe_inter;
   const int qkv_dim = (nq + 2 * nkv) * hd, n_slot = m->top_k + m->n_shared_slots;
@@ -1285,7 +1290,7 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
       if (gu_chain) {
         MN_TRY(moe_gate_up_routed(m->wfmt, w.h, H, m->ln2[l], m->rms_eps, m->gate[l], m->w_gate_up[l], (int64_t)2 * I * H,
                                   m->wfmt ? m->w_gate_up_scale[l] : nullptr, (int64_t)2 * I * mn_wq_scales_per_row(m->wfmt, H), M, H, I, E, m->top_k,
-                                  S, m->norm_topk_prob, w.hmid, (int64_t)n_slot * I, w.ti, w.tw, w.logits, w.pp, nz, (int64_t)M * H, stream));
+                                  S, m->norm_topk_prob, w.hmid, (int64_t)n_slot * I, w.ti, w.tw, w.logits, w.pp, nz, (int64_t)M * H, nullptr, stream));
         route_capture(l, w.ti, M, n_slot, st);
         MN_TRY(moe_down_rows(m->wfmt, w.hmid, (int64_t)n_slot * I, m->w_down[l], (int64_t)H * I, m->wfmt ? m->w_down_scale[l] : nullptr,
                              (int64_t)H * mn_wq_scales_per_row(m->wfmt, I), w.ti, w.tw, w.h, H, w.h, H, M, H, I, n_slot, stream, w.pp, nz,
@@ -1353,14 +1358,18 @@ static int llm_step_impl(const mn_llm* m, const float* x, int64_t ldx, int x_row
     }
     a = sk(w.attn, nq * hd, m->wdense[l], nq * hd, nullptr, w.h, H, M, H, nq * hd);
     a.epilogue = MN_EPI_RESID; a.res = w.h; a.ldres = H;
-    MN_TRY(mn_skinny_gemm(&a, stream));
+    const bool one_launch = g_moe_gate_up && M <= g_moe_gate_up_rows && !image_rows && g_moe_down &&
+                            moe_gate_up_ok(m->wfmt, H, I, m->n_experts, m->top_k, m->n_shared_slots) && moe_down_ok(m->wfmt, n_slot, H, I);
+    // ... leaving the next launch's routing as partial sums where there is scratch for them
+    const int parts = one_launch && gate_part ? mn_row_product_gated(a, m->gate[l], m->ln2[l], m->n_experts, gate_part, stream) : 0;
+    if (parts < 0) return parts;
+    if (!parts) MN_TRY(mn_skinny_gemm(&a, stream));
     // one row: RMSNorm + router + the selected experts' gate/up in ONE launch (moe_gate_up.hip), then the down projection (moe_down.hip) — every
     // weight format (int8 / NF4 decode per element like the grouped MFMA launch they replace here: text decode int8 434 -> 699, int4 426 -> 619 tokens/s)
-    if (g_moe_gate_up && M <= g_moe_gate_up_rows && !image_rows && g_moe_down &&
-        moe_gate_up_ok(m->wfmt, H, I, m->n_experts, m->top_k, m->n_shared_slots) && moe_down_ok(m->wfmt, n_slot, H, I)) {
+    if (one_launch) {
       MN_TRY(moe_gate_up_routed(m->wfmt, w.h, H, m->ln2[l], m->rms_eps, m->gate[l], m->w_gate_up[l], (int64_t)2 * I * H,
                                 m->wfmt ? m->w_gate_up_scale[l] : nullptr, (int64_t)2 * I * mn_wq_scales_per_row(m->wfmt, H), M, H, I, m->n_experts, m->top_k,
-                                m->n_shared_slots, m->norm_topk_prob, w.hmid, (int64_t)n_slot * I, w.ti, w.tw, w.logits, nullptr, 0, 0, stream));
+                                m->n_shared_slots, m->norm_topk_prob, w.hmid, (int64_t)n_slot * I, w.ti, w.tw, w.logits, nullptr, 0, 0, parts ? gate_part : nullptr, stream));
       route_capture(l, w.ti, M, n_slot, st);
       MN_TRY(moe_down_rows(m->wfmt, w.hmid, (int64_t)n_slot * I, m->w_down[l], (int64_t)H * I, m->wfmt ? m->w_down_scale[l] : nullptr, (int64_t)H * mn_wq_scales_per_row(m->wfmt, I), w.ti, w.tw, w.h, H, w.h, H, M, H, I, n_slot, stream));
       continue;

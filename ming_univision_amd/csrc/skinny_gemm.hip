@@ -442,6 +442,16 @@ static struct { int R, nt, bpc; } g_tune = {0, 0, 0};
 extern "C" MN_DEV_API void mn_skinny_tune(int R, int nt, int bpc) { g_tune.R = R; g_tune.nt = nt; g_tune.bpc = bpc; }
 #endif
 
+// One row's product with a residual whose outputs a router of up to 64 experts reads next: its share of the routing goes to part [N / 8][64] + [N / 8] (row_gemv.inl).  0: not a product of that form,
+// nothing was launched.
+int mn_row_product_gated(const mn_skinny_args& a, const bf16_t* gate_w, const bf16_t* gain, int experts, float* part, void* stream) {
+  if (!(a.M == 1 && a.N >= 1 && a.K >= 8 && (a.K % 8) == 0 && (a.ldw % 8) == 0 && a.x && a.w && a.out && a.prologue == MN_PRO_NONE && a.epilogue == MN_EPI_RESID && a.res && gate_w && gain && part &&
+        a.batch <= 1 && a.nseg <= 1 && (((uintptr_t)a.w) & 15) == 0)) return 0;
+  if (!row_gemv(a, mn_stream(stream), gate_w, gain, experts, part)) return 0;
+  MN_CHECK_LAUNCH("mn_row_product_gated");
+  return 1;
+}
+
 extern "C" int mn_skinny_gemm(const mn_skinny_args* args, void* stream) {
   MN_CHECK_ARG(args != nullptr, "mn_skinny_gemm: null args");
   KArgs ka;

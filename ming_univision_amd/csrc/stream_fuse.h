@@ -71,6 +71,9 @@ int moe_down_rows(int wfmt, const float* hmid, int64_t ld_hmid, const void* W, i
 // (the decoder chain at 2 rows): the row is h + the nz partial slabs P [nz][batch][H] of the attention output projection
 // (h is not updated: moe_down_rows adds the same slabs to its residual).
 bool moe_gate_up_ok(int wfmt, int H, int I, int E, int top_k, int n_shared);
+bool moe_gate_parts_ok(int H, int E);
+// the product before it, leaving the router's partial sums: > 0 launched, 0 not a product of that form (skinny_gemm.hip)
+int mn_row_product_gated(const mn_skinny_args& a, const bf16_t* gate_w, const bf16_t* gain, int experts, float* part, void* stream);
 int moe_gate_up_routed(int wfmt, const float* h, int64_t ldh, const bf16_t* norm_w, float eps, const bf16_t* gate_w, const void* W, int64_t w_stride,
                        const float* wscale, int64_t wscale_stride, int batch, int H, int I, int E, int top_k, int n_shared, int norm_topk_prob,
-                       float* hmid, int64_t ld_hmid, int32_t* ti, float* tw, float* logits, const float* P, int nz, int64_t slab, void* stream);
+                       float* hmid, int64_t ld_hmid, int32_t* ti, float* tw, float* logits, const float* P, int nz, int64_t slab, const float* part, void* stream);

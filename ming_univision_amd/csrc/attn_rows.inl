@@ -11,10 +11,18 @@
 // all of them see whole takes no mask arithmetic.  Key splits write the partial layout of the merge kernel, run by run.
 
 // A launch's workgroups: first the groups of every (head chunk, key split), then `alone` that take one run after the other.
-// Group x of the launch: long walks (late rows) first, the next 256 the other way round, so that the two workgroups a CU holds are a long and a short one.
-__device__ __forceinline__ int rows_group(int x, int groups) {
+// Workgroup x of the launch: long walks (late rows) first.  Where all are on the chip at once (two a CU), the second 256 go the other way round, so that a CU holds a long and a short one.
+// Where they follow each other the order is by length alone, the head chunks and splits of a group side by side: what is taken last is short, and no CU is left with a long walk at the
+// end.  us, every other 256 the other way round / by length (16 heads of 128 over four key heads): 8000 tokens 2968 / 2360 (111 TFLOP/s), 2600 446 / 315, 1500 in two splits
+// 164 / 137, 1000 in three 104 / 89, 16 sequences of 512 328 / 245, window 1024 of 3000 280 / 247; keys of 320 with the values inside, 5 prompts of 93 .. 470, 91 / 85.
+struct RowsItem { int group, gy, sp; };
+__device__ __forceinline__ RowsItem rows_item(int x, int groups, int gys, int items) {
+  if (items > 512) {
+    const int yzs = items / groups, yz = x % yzs;
+    return {groups - 1 - x / yzs, yz % gys, yz / gys};
+  }
   const int g = x % groups, first = x - g;                               // of this (head chunk, split): one direction for all of its groups
-  return ((first >> 8) & 1) ? g : groups - 1 - g;
+  return {((first >> 8) & 1) ? g : groups - 1 - g, x / groups % gys, x / groups / gys};
 }
 
 // the workgroup's runs: first row, rows, cache sequence, first position
@@ -98,6 +106,17 @@ __device__ __forceinline__ void emit4(const AttnTArgs& a, f32x4 v, int row, int6
     if (a.out) a.out[(int64_t)row * a.ldo + col0 + d + e] = v[e];
     if (a.out16) a.out16[(int64_t)row * a.ldo16 + col0 + d + e] = f32_to_bf16(v[e]);
   }
+}
+// values d .. d + 3 of vector qv's sums in a split's partial slab, 16 bytes at a time (value by value a launch of 5 prompts in three splits spent 18 of its 67 us on them and their merge)
+__device__ __forceinline__ void part4(const AttnTArgs& a, float* part, int qv, int d, f32x4 v) {
+  float* p = part + 2 * a.sq + (int64_t)qv * a.vdim + d;
+  if (d + 4 <= a.vdim) {
+    *reinterpret_cast<f32x4u*>(p) = v;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (d + e < a.vdim) p[e] = v[e];
 }
 __device__ __forceinline__ bool emit_vec(const AttnTArgs& a) {
   return (a.vdim & 3) == 0 && (!a.out || ((a.ldo & 3) == 0 && ((uintptr_t)a.out & 15) == 0)) &&
@@ -281,9 +300,7 @@ __device__ __forceinline__ void attn_run(const AttnTArgs& a, int b, int gy, int 
     if (d >= a.vdim) continue;
     const f32x4 r = acc[x] * inv;
     if (!part) { emit4(a, r, row, col0, d, vec); continue; }
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (d + e < a.vdim) part[2 * a.sq + (int64_t)c * a.vdim + d + e] = r[e];
+    part4(a, part, c, d, r);
   }
   if (part && wave == 0 && g4 == 0) { part[c] = mrun; part[a.sq + c] = lrun; }
   if (!VK && met) {
@@ -313,7 +330,7 @@ __global__ __launch_bounds__(256) void attn_runs_kernel(AttnTArgs a) {
 // K is read 16 bytes at a time (a lane's k slot = dims 16 it + 4 g .. + 3 over four steps, one accumulator per step: four short chains sum more
 // exactly than one long one), V likewise (row c of value fragment 4 vb + e = column 64 vb + 4 c + e); with row strides of 4 mod 64 floats
 // both reads touch every bank once.  One LDS-only barrier per tile.
-// 2048 tokens, 16 heads of 128 over 4 key/value heads (17.2 GF): 632 us in the form before, 211 us here (82 TFLOP/s).
+// 2048 tokens, 16 heads of 128 over 4 key/value heads (17.2 GF): 632 us in the form before, 198 us here (87 TFLOP/s).
 // VEC: dim and vdim are multiples of 4.
 template <int NBD, int NBV, bool VEC>
 __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_blk, int hv, int groups) {
@@ -332,10 +349,11 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_bl
                [&](int b, int gy, int sp) { attn_run<NBD, NBV, KF, VEC, false>(a, b, gy, sp, lds, met); });
     return;
   }
-  const int gy = (blockIdx.x / groups) % gys, sp = blockIdx.x / groups / gys;
+  const RowsItem it = rows_item(blockIdx.x, groups, gys, in_groups);
+  const int gy = it.gy, sp = it.sp;
   const int g = gy / chunks, h0 = g * rep + (gy % chunks) * a.hpc;
   const int Rc = min(a.hpc, g * rep + rep - h0);
-  const int b0 = rows_group(blockIdx.x, groups) * nbw, nb = min(nbw, n_blk - b0);
+  const int b0 = it.group * nbw, nb = min(nbw, n_blk - b0);
   rows_table(a, b0, nb, nbw, tid, tab);
   if (!rows_one_sequence(tab, nb)) return;
   // this lane's query: column c of the wave's 16
@@ -491,9 +509,7 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_bl
         if (d >= a.vdim) continue;
         const f32x4 r = f32x4{acc[4 * vb][i], acc[4 * vb + 1][i], acc[4 * vb + 2][i], acc[4 * vb + 3][i]} * inv;
         if (!part) { emit4(a, r, row, col0, d, vec); continue; }
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (d + e < a.vdim) part[2 * a.sq + (int64_t)qv * a.vdim + d + e] = r[e];
+        part4(a, part, qv, d, r);
       }
     if (part && g4 == 0) { part[qv] = mrun; part[a.sq + qv] = lrun; }
     if (met) {
@@ -532,9 +548,10 @@ __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, i
                [&](int b, int gy, int sp) { attn_run<NB, NB, 1, VEC, true>(a, b, gy, sp, K, met); });
     return;
   }
-  const int gy = (blockIdx.x / groups) % gys, sp = blockIdx.x / groups / gys, h0 = gy * a.hpc;
+  const RowsItem it = rows_item(blockIdx.x, groups, gys, in_groups);
+  const int gy = it.gy, sp = it.sp, h0 = gy * a.hpc;
   const int Rc = min(a.hpc, rep - h0);
-  const int b0 = rows_group(blockIdx.x, groups) * nbw, nb = min(nbw, n_blk - b0);
+  const int b0 = it.group * nbw, nb = min(nbw, n_blk - b0);
   rows_table(a, b0, nb, nbw, tid, tab);
   if (!rows_one_sequence(tab, nb)) return;
   const int hc = c % hv, dw = wave * 16 * NB;                           // this wave's dims: dw .. dw + 16 NB - 1
@@ -678,9 +695,7 @@ __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, i
       if (d >= a.vdim) continue;
       const f32x4 r = acc[f][x] * inv;
       if (!part) { emit4(a, r, row[f], col0, d, vec); continue; }
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (d + e < a.vdim) part[2 * a.sq + (int64_t)qv * a.vdim + d + e] = r[e];
+      part4(a, part, qv, d, r);
     }
     if (part && wave == 0 && g4 == 0) { part[qv] = mrun[f]; part[a.sq + qv] = lrun[f]; }
   }
@@ -719,9 +734,7 @@ __global__ __launch_bounds__(256) void attn_latent_decode_kernel(AttnTArgs a) {
     if (d >= a.vdim) continue;
     const f32x4 r = acc[x] * inv;
     if (!part) { emit4(a, r, b, col0, d, vec); continue; }
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (d + e < a.vdim) part[2 * a.sq + (int64_t)c * a.vdim + d + e] = r[e];
+    part4(a, part, c, d, r);
   }
   if (part && wave == 0 && g4 == 0) { part[c] = mrun; part[a.sq + c] = lrun; }
 }

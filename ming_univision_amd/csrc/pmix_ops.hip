@@ -808,6 +808,49 @@ __global__ __launch_bounds__(256) void window_attn_merge_kernel(AttnTArgs a) {
   }
 }
 
+// The same for a few splits of runs of rows: a thread takes four columns of one vector and works its splits' weights out by itself, everything asked for at once; no LDS and no barrier.
+// What bounds it is memory, but the kernel above spends its time on the weights (four vectors a wave, one after the other, in every slice of 64 columns): 353 runs of 8 heads x 256 in two splits, 34 MB,
+// 20.2 us there.  The whole attention, us, with value-by-value slabs and the merge above -> now: 16 heads of 128, 1500 tokens in 2 splits 138 -> 117, 1000 in 3 89 -> 65, 500 in 4 47 -> 31; 5 prompts,
+// 8 heads in 3 splits 67 -> 48; keys of 320 with the values inside, 5 prompts in 2 85 -> 67.  Up to 8 splits (their sums are in registers at once); more come of few rows, whose merge is short.
+// grid (n_blk, G * chunks, ceil(sq * ceil(vdim / 4) / 256))
+constexpr int MERGE_FEW = 8;
+template <int NS>
+__global__ __launch_bounds__(256) void window_attn_merge_few_kernel(AttnTArgs a) {
+  const int b = blockIdx.x, gy = blockIdx.y, quads = (a.vdim + 3) >> 2, e = blockIdx.z * 256 + threadIdx.x;
+  const int rep = a.H / a.G, chunks = (rep + a.hpc - 1) / a.hpc;
+  const int g = gy / chunks, h0 = g * rep + (gy % chunks) * a.hpc;
+  const int Rc = min(a.hpc, g * rep + rep - h0);
+  const int i = e / quads, d = 4 * (e - i * quads);
+  if (i >= min(a.blk_tab[2 * b + 1], a.rows_per_blk) * Rc) return;
+  const int64_t stride = (int64_t)a.sq * (2 + a.vdim);
+  const float* base = a.part + ((int64_t)b * gridDim.y + gy) * a.nsplit * stride;
+  const float* src = base + 2 * a.sq + (int64_t)i * a.vdim;
+  float m[NS], l[NS];
+  f32x4 v[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const int64_t o = min(s, a.nsplit - 1) * stride;
+    m[s] = base[o + i];
+    l[s] = base[o + a.sq + i];
+    if (d + 4 <= a.vdim) v[s] = *reinterpret_cast<const f32x4u*>(src + o + d);
+    else v[s] = load4<false>(src + o, d, a.vdim, true);
+  }
+  float top = -INFINITY, L = 0.f;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) top = fmaxf(top, m[s]);
+  f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const float w = m[s] == -INFINITY ? 0.f : expf(m[s] - top);
+    if (s >= a.nsplit) continue;
+    L = fmaf(l[s], w, L);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) t[x] = fmaf(v[s][x], w, t[x]);
+  }
+  const int h = h0 + i % Rc;
+  emit4(a, t * (softmax_inv(top, L, a.sink, h) * a.out_scale), a.blk_tab[2 * b] + i / Rc, (int64_t)h * a.vdim, d, emit_vec(a));
+}
+
 // ---------------------------------------------------------------------------------------------------------------------------
 // minGRU: grid (ceil(n / 256), M); the workgroup of a sequence's FIRST row in the step walks that sequence's rows
 __global__ __launch_bounds__(256) void mingru_kernel(const float* __restrict__ zx, int64_t ldzx, const float* __restrict__ g, int64_t ldg,
@@ -1158,11 +1201,13 @@ extern "C" int mn_window_attn_splits_heads(int n_blk, int H, int G, int one_row,
   const AttnShape sh = attn_shape(H, G, one_row);
   const int vec = one_row ? 16 : attn_run_vectors(dim, vdim, vk);
   const int64_t runs = vec == 16 ? 1 : attn_rows_runs(H / G) * vec / 64, tiles = mn_cdiv(max_keys, key_tile);
-  auto want = [&](int64_t wgs, int64_t most) { const int64_t ns = mn_cdiv(2 * (int64_t)mn_num_cus(), wgs); return ns < most ? (ns < 64 ? (int)ns : 64) : (most < 64 ? (int)most : 64); };
+  auto want = [&](int64_t wgs, int64_t most, int more = 0) { const int64_t two = 2 * (int64_t)mn_num_cus(), ns = mn_cdiv(two + more, wgs); return ns < most ? (ns < 64 ? (int)ns : 64) : (most < 64 ? (int)most : 64); };
   const int by_runs = want((int64_t)n_blk * G * sh.chunks, tiles);
   if (vec == 16) return by_runs;
   // (a group of 32 or 64 vectors has some 10 us of its own: a split of its walk below 128 keys costs more than it saves)
-  const int by_groups = want(mn_cdiv(n_blk, runs) * G * sh.chunks, mn_cdiv(max_keys, 128) < tiles ? mn_cdiv(max_keys, 128) : tiles);
+  const int64_t groups = mn_cdiv(n_blk, runs) * G * sh.chunks, most = mn_cdiv(max_keys, 128) < tiles ? mn_cdiv(max_keys, 128) : tiles;
+  // (values inside keys: more than two a CU, 8 heads of 2048 tokens, keys of 320, 1: 399, 2: 269; heads of 128 1: 200, 2: 200)
+  const int by_groups = want(groups, most, vk);
   return attn_runs_alone(n_blk, H, G, by_groups) ? by_runs : by_groups;
 }
 
@@ -1330,7 +1375,11 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
     }
     MN_CHECK_LAUNCH("mn_window_pool_attn_blocks(mfma)");
     if (nsplit > 1) {
-      hipLaunchKernelGGL((window_attn_merge_kernel<16>), dim3((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)mn_cdiv(vdim, MERGE_COLS)), dim3(256), 0, stm, a);
+      const dim3 few((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)mn_cdiv((int64_t)sh.sq * mn_cdiv(vdim, 4), 256));
+      if (!one_row && nsplit <= 2) hipLaunchKernelGGL((window_attn_merge_few_kernel<2>), few, dim3(256), 0, stm, a);
+      else if (!one_row && nsplit <= 4) hipLaunchKernelGGL((window_attn_merge_few_kernel<4>), few, dim3(256), 0, stm, a);
+      else if (!one_row && nsplit <= MERGE_FEW) hipLaunchKernelGGL((window_attn_merge_few_kernel<MERGE_FEW>), few, dim3(256), 0, stm, a);
+      else hipLaunchKernelGGL((window_attn_merge_kernel<16>), dim3((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)mn_cdiv(vdim, MERGE_COLS)), dim3(256), 0, stm, a);
       MN_CHECK_LAUNCH("mn_window_pool_attn_blocks(merge)");
     }
     return MN_OK;

@@ -311,6 +311,22 @@ __device__ __forceinline__ void f32_store(const GemmF32& a, int z, int m, int n,
   if (a.C16) a.C16[(int64_t)z * a.c16_bs + (int64_t)m * a.ldc16 + n] = f32_to_bf16(v);
 }
 
+// outputs n .. n + 3 of row m
+__device__ __forceinline__ void f32_store4(const GemmF32& a, int z, int m, int n, f32x4 v) {
+  float* c = a.C ? a.C + (int64_t)z * a.c_bs + (int64_t)m * a.ldc + n : nullptr;
+  if (n + 4 > a.N || !c || a.C16 || a.G) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f32_store(a, z, m, n + e, v[e]);
+    return;
+  }
+  v *= a.alpha;
+  if (a.bias) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += bf16_to_f32(a.bias[n + e]);
+  }
+  *reinterpret_cast<f32x4u*>(c) = v;                          // (rows may start at any float)
+}
+
 // More than 2 rows (8 where accesses go value by value) run on the fp32 matrix cores (v_mfma_f32_16x16x4f32: lane l holds row / column l & 15), fp32 rows and bf16 weights
 // widened on the way.  Both kernels give lane l the values 4 (l >> 4) .. + 3 of every 16 of K, so the four products of a 16-step take
 // one 16-byte read of each operand, in an order of K that both share.  Values past K enter as zeros.  V4: rows of A are 16-byte, rows
@@ -395,86 +411,137 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(GemmF32 a) {
   }
 }
 
-// Many tiles: 64 x 64 outputs a workgroup, 32 x 32 a wave, 32 values of K at a time in LDS (rows 36 floats apart: the 16-byte reads of 16
-// rows meet all 64 banks), double-buffered through registers; two accumulators per output tile halve the chain of roundings.  2048 rows x 4096 x 1024: 168 us = 102 TFLOP/s of
-// the 157 peak (FMA tiles: 292 us), error 2.0e-7 of the summed magnitudes (3.4e-7).
-template <bool V4>
-__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(GemmF32 a) {
-  constexpr int LD = 36;
-  __shared__ float As[2][64 * LD], Ws[2][64 * LD];
+// Many tiles: 64 x 64 outputs a workgroup, 32 x 32 a wave, on the bf16 matrix cores.  An fp32 value is the sum of three bf16 values, its upper, middle and lower 8 bits of mantissa cut off one
+// after the other, and a weight is one already: three products a pair, each exact in fp32, take a fifth of the fp32 cores' time for the one.  The rows are split once a workgroup, on their way to
+// LDS (8 instructions a value; what is left of an infinity is zero, of a NaN a NaN); 64 values of K at a time, rows 144 bytes apart (the 16-byte reads of 16 rows meet all 64 banks), two
+// stages of loads in flight in registers.  The upper products and the others have accumulators of their own.  An infinite weight would meet a part that is zero: a workgroup that saw one
+// takes its outputs over again, value by value.  NB: buffers of LDS: two (two workgroups a CU), or one and a second barrier (three a CU) where the tiles are more than two a CU: us, two / one: 900 rows of
+// 16 x 512 x 128 24.4 / 21.3, 2048 x 4096 x 1024 100 / 94, 8 x 2129 x 1676 x 302 241 / 216; 900 of 1024 x 1024 (240 tiles) 19.7 / 20.6.
+// us, fp32 matrix cores (values a lane stored one by one) -> here: 900 rows of 16 x 512 x 128 32 -> 21, of 16 x 128 x 512 28 -> 17, 1900 rows 53 -> 35 and 49 -> 31, 2048 x 4096 x 1024 168 -> 94 (183
+// TFLOP/s), 200 rows of 16 x 128 x 512 17.5 -> 11.2.  What bounds short K is a workgroup's round trips.  Error against 64 bits, rows of uneven magnitudes: 1.47e-7 -> 0.77e-7 at K = 128, 2.9e-7 -> 1.5e-7 at 512, 5.7e-7 ->
+// 2.9e-7 at 2048.  (Parts below 2^-126 may count as zero: rows of values below 1e-31 lose their last bits.)
+template <bool V4, int NB>
+__global__ __launch_bounds__(256, NB == 1 ? 3 : 2) void gemm_f32_tile_kernel(GemmF32 a) {
+  typedef short bf16x8 __attribute__((ext_vector_type(8)));
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  constexpr int LD = 72, PLANE = 64 * LD;
+  __shared__ __attribute__((aligned(16))) uint16_t lds[NB][4 * PLANE];      // [upper | middle | lower | weights][64][LD]
   const int z = blockIdx.z, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, q = lane >> 4;
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64, wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
   const float* A = a.A + (int64_t)z * a.a_bs;
   const bf16_t* W = a.W + (int64_t)z * a.w_bs;
-  f32x4 acc[2][2][2], fa[2];
-  ushort4 fw[2];
+  const int k4 = 4 * (tid & 15);
+  const float* ap[4];
+  const bf16_t* wp[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {                               // rows past the matrix repeat its last one; nothing of them is stored
+    const int row = (tid >> 4) + 16 * t;
+    ap[t] = A + (int64_t)min(m0 + row, a.M - 1) * a.lda;
+    wp[t] = W + (int64_t)min(n0 + row, a.N - 1) * a.ldw;
+  }
+  f32x4 fa[2][4];
+  ushort4 fw[2][4];
+  us2 top = {0, 0};                                           // the weights' largest magnitudes, as bits
+  auto fetch = [&](int k0, int h) {
+    const int k = k0 + k4;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      if (V4) {
+        const int kc = min(k, a.K - 4);
+        fa[h][t] = *reinterpret_cast<const f32x4*>(ap[t] + kc);
+        fw[h][t] = *reinterpret_cast<const ushort4*>(wp[t] + kc);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) fa[h][t][c] = ap[t][min(k + c, a.K - 1)];
+        fw[h][t] = ushort4{wp[t][min(k, a.K - 1)], wp[t][min(k + 1, a.K - 1)], wp[t][min(k + 2, a.K - 1)], wp[t][min(k + 3, a.K - 1)]};
+      }
+    }
+  };
+  auto put = [&](int b, int k0, int h) {
+    const int left = a.K - k0 - k4;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      uint32_t part[3][4], w01 = fw[h][t].x | (uint32_t)fw[h][t].y << 16, w23 = fw[h][t].z | (uint32_t)fw[h][t].w << 16;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float v = c < left ? fa[h][t][c] : 0.f;         // what is past K becomes zero here: a branch around the load is a wait
+        const float u = __uint_as_float(__float_as_uint(v) & 0xffff0000u), d = v == u ? 0.f : v - u;
+        const float m = __uint_as_float(__float_as_uint(d) & 0xffff0000u);
+        part[0][c] = __float_as_uint(v);
+        part[1][c] = __float_as_uint(d);
+        part[2][c] = __float_as_uint(d - m);
+      }
+      if (left < 4) {
+        w01 &= left > 1 ? 0xffffffffu : left > 0 ? 0xffffu : 0u;
+        w23 &= left > 3 ? 0xffffffffu : left > 2 ? 0xffffu : 0u;
+      }
+      const uint32_t b01 = w01 & 0x7fff7fffu, b23 = w23 & 0x7fff7fffu;
+      top = __builtin_elementwise_max(top, __builtin_elementwise_max(*reinterpret_cast<const us2*>(&b01), *reinterpret_cast<const us2*>(&b23)));
+      uint16_t* at = &lds[b % NB][((tid >> 4) + 16 * t) * LD + k4];
+#pragma unroll
+      for (int x = 0; x < 3; ++x)
+        *reinterpret_cast<uint2*>(at + x * PLANE) = uint2{__builtin_amdgcn_perm(part[x][1], part[x][0], 0x07060302u), __builtin_amdgcn_perm(part[x][3], part[x][2], 0x07060302u)};
+      *reinterpret_cast<uint2*>(at + 3 * PLANE) = uint2{w01, w23};
+    }
+  };
+  f32x4 acc[2][2][2];
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[u][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {                             // rows past the matrix repeat its last one; nothing of them is stored
-      const int e = tid + 256 * t, row = e >> 3, k = k0 + 4 * (e & 7);
-      const float* ap = A + (int64_t)min(m0 + row, a.M - 1) * a.lda;
-      const bf16_t* wp = W + (int64_t)min(n0 + row, a.N - 1) * a.ldw;
-      fa[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-      fw[t] = ushort4{0, 0, 0, 0};
-      if (V4) {
-        if (k < a.K) { fa[t] = *reinterpret_cast<const f32x4*>(ap + k); fw[t] = *reinterpret_cast<const ushort4*>(wp + k); }
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) fa[t][c] = ap[min(k + c, a.K - 1)];          // (what is past K becomes zero on the way to LDS: a branch here is a wait)
-        fw[t] = ushort4{wp[min(k, a.K - 1)], wp[min(k + 1, a.K - 1)], wp[min(k + 2, a.K - 1)], wp[min(k + 3, a.K - 1)]};
-      }
-    }
-  };
-  auto put = [&](int b, int k0) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int e = tid + 256 * t, at = (e >> 3) * LD + 4 * (e & 7);
-      if (!V4) {
-        const int left = a.K - k0 - 4 * (e & 7);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) fa[t][c] = c < left ? fa[t][c] : 0.f;
-        fw[t] = ushort4{left > 0 ? fw[t].x : (unsigned short)0, left > 1 ? fw[t].y : (unsigned short)0, left > 2 ? fw[t].z : (unsigned short)0, left > 3 ? fw[t].w : (unsigned short)0};
-      }
-      *reinterpret_cast<f32x4*>(&As[b][at]) = fa[t];
-      *reinterpret_cast<f32x4*>(&Ws[b][at]) = f32x4{bf16_to_f32(fw[t].x), bf16_to_f32(fw[t].y), bf16_to_f32(fw[t].z), bf16_to_f32(fw[t].w)};
-    }
-  };
-  fetch(0);
-  put(0, 0);
-  int b = 0;
-  for (int k0 = 0; k0 < a.K; k0 += 32, b ^= 1) {
-    const bool more = k0 + 32 < a.K;
-    if (more) fetch(k0 + 32);
-    __syncthreads();
+  auto step = [&](int k0, int b) {                            // buffer b holds K-step k0, registers b ^ 1 the one after it
+    if (k0 + 128 < a.K) fetch(k0 + 128, b);
+    lds_barrier();
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      f32x4 ra[2], rw[2];
+      bf16x8 fr[3][2], wr[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        ra[i] = *reinterpret_cast<const f32x4*>(&As[b][(wm + 16 * i + r) * LD + 16 * u + 4 * q]);
-        rw[i] = *reinterpret_cast<const f32x4*>(&Ws[b][(wn + 16 * i + r) * LD + 16 * u + 4 * q]);
+        wr[i] = *reinterpret_cast<const bf16x8*>(&lds[b % NB][3 * PLANE + (wn + 16 * i + r) * LD + 32 * u + 8 * q]);
+#pragma unroll
+        for (int x = 0; x < 3; ++x) fr[x][i] = *reinterpret_cast<const bf16x8*>(&lds[b % NB][x * PLANE + (wm + 16 * i + r) * LD + 32 * u + 8 * q]);
       }
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int x = 2; x >= 0; --x)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) acc[u][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[i][t], rw[j][t], acc[u][i][j], 0, 0, 0);
+          for (int j = 0; j < 2; ++j) acc[x == 0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[j], fr[x][i], acc[x == 0][i][j], 0, 0, 0);
     }
-    if (more) put(b ^ 1, k0 + 32);                                     // the buffer that every wave left before this step's barrier
+    if (k0 + 64 < a.K) {
+      if (NB == 1) lds_barrier();
+      put(b ^ 1, k0 + 64, b ^ 1);                             // NB 2: the buffer that every wave left before this step's barrier
+    }
+  };
+  fetch(0, 0);
+  if (64 < a.K) fetch(64, 1);
+  put(0, 0, 0);
+  for (int k0 = 0; k0 < a.K; k0 += 128) {
+    step(k0, 0);
+    if (k0 + 64 < a.K) step(k0 + 64, 1);
   }
+  const bool odd = __syncthreads_or(top.x >= 0x7f80 || top.y >= 0x7f80);
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) f32_store(a, z, m0 + wm + 16 * i + 4 * q + e, n0 + wn + 16 * j + r, acc[0][i][j][e] + acc[1][i][j][e]);
+    for (int j = 0; j < 2; ++j) {                             // a lane's four outputs are neighbours in a row
+      const int m = m0 + wm + 16 * i + r, n = n0 + wn + 16 * j + 4 * q;
+      f32x4 v = acc[0][i][j] + acc[1][i][j];
+      if (odd) {
+        const float* x = A + (int64_t)min(m, a.M - 1) * a.lda;
+#pragma unroll 1
+        for (int e = 0; e < 4; ++e) {
+          const bf16_t* w = W + (int64_t)min(n + e, a.N - 1) * a.ldw;
+          float t = 0.f;
+#pragma unroll 1
+          for (int k = 0; k < a.K; ++k) t = fmaf(x[k], bf16_to_f32(w[k]), t);
+          v = f32x4{e == 0 ? t : v[0], e == 1 ? t : v[1], e == 2 ? t : v[2], e == 3 ? t : v[3]};
+        }
+      }
+      if (m < a.M) f32_store4(a, z, m, n, v);
+    }
 }
 
 // Decode rows (every row alone in its sequence), one workgroup per row, the row in registers, up to three stages in one launch:
@@ -1188,8 +1255,11 @@ extern "C" int mn_gemm_f32_batched(const float* A, int64_t lda, int64_t a_bs, co
     else hipLaunchKernelGGL(gemm_f32_few_kernel<false>, grid, dim3(256), 0, st, a);
   } else {
     const dim3 grid((unsigned)mn_cdiv(N, 64), (unsigned)mn_cdiv(M, 64), (unsigned)batch);
-    if (v4) hipLaunchKernelGGL(gemm_f32_tile_kernel<true>, grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(gemm_f32_tile_kernel<false>, grid, dim3(256), 0, st, a);
+    const bool many = tiles > 2 * (int64_t)mn_num_cus();
+    if (v4 && many) hipLaunchKernelGGL((gemm_f32_tile_kernel<true, 1>), grid, dim3(256), 0, st, a);
+    else if (v4) hipLaunchKernelGGL((gemm_f32_tile_kernel<true, 2>), grid, dim3(256), 0, st, a);
+    else if (many) hipLaunchKernelGGL((gemm_f32_tile_kernel<false, 1>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((gemm_f32_tile_kernel<false, 2>), grid, dim3(256), 0, st, a);
   }
   MN_CHECK_LAUNCH("mn_gemm_f32_batched");
   return MN_OK;

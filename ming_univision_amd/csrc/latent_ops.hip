@@ -905,7 +905,8 @@ __global__ __launch_bounds__(256, VEC && NB <= 8 ? 2 : 1) void latent_attn_mfma_
 // A register that has been multiplied is asked for what follows half a tile further on: loads are in flight all the time.  What bounds it is memory in the walk (5.2 TB/s) and the ends, 5 us until
 // the first tile is there and 3 from the last one to the split's results.  us, the form above -> this, the splits' join with it: 32 rows of 16 heads over 2049 latents of 512 54.5 -> 44.4 (the walk alone
 // 41.7 -> 36.3; 134 MB, 23 us at the rate of a plain read), 64 rows over 1000 47.0 -> 40.7, 64 rows of 8 heads over 2048 of 256 39.1 -> 37.8; prompts of 2048, 1000, 300, 130 tokens, 16 heads over
-// latents of 512, 909 -> 760, 270 -> 240, 48.5 -> 43, 24.6 -> 22.7, 2048 tokens of 8 heads over 256 273 -> 222.
+// latents of 512, 909 -> 760, 270 -> 240, 48.5 -> 43, 24.6 -> 22.7, 2048 tokens of 8 heads over 256 273 -> 222.  With long walks taken first (prompts, us): 16 heads over 512 2048 tokens 715 -> 635, 900
+// 190 -> 155, 300 42.5 -> 32.7, five of 282 133 -> 117, 8 heads over 256 2048 tokens 206 -> 167.
 // The sums are taken against a maximum that is raised only where a score is above it by more than 8 (weights up to e^8, which fp32 holds as well as 1): scaling sums that live in the
 // matrix cores' half of the registers would cost every tile a copy of them.  Error against 64 bits 1.4 .. 2.0e-7, the form above 1.7 .. 2.9e-7.
 __device__ __forceinline__ void wave_order() {         // what the lanes of a wave hand each other through LDS: the hardware keeps its order, this the compiler's
@@ -921,11 +922,12 @@ __global__ __launch_bounds__(256, NT <= 16 ? 2 : 1) void latent_attn_wave_kernel
   __shared__ __attribute__((aligned(16))) float lds[4 * TILE];
   __shared__ float wm[4][16], wl[4][16];
   __shared__ __attribute__((aligned(16))) float scale[NT > 16 ? 4 : 1][NT > 16 ? 1024 : 4];
-  const int row0 = blk_tab[2 * blockIdx.x], nrows = blk_tab[2 * blockIdx.x + 1];
+  // long walks (a prompt's late rows) first, the query vectors of a run side by side: what is taken last is short
+  const int order = blockIdx.y * gridDim.x + blockIdx.x, run = gridDim.x - 1 - order / gridDim.y, row0 = blk_tab[2 * run], nrows = blk_tab[2 * run + 1];
   const int nqv = nrows * H, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   float* K = lds + wave * TILE;
   // (one pass unless the grid was cut for runs of one row and this one is longer)
-  for (int qv0 = blockIdx.y * 16; qv0 < nqv; qv0 += 16 * gridDim.y) {
+  for (int qv0 = order % gridDim.y * 16; qv0 < nqv; qv0 += 16 * gridDim.y) {
     int lane = threadIdx.x & 63;
     asm("" : "+v"(lane));                              // (what depends on it is not held over the passes: registers)
     const int c = lane & 15, g4 = lane >> 4;

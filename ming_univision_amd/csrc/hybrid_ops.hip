@@ -67,6 +67,41 @@ __global__ __launch_bounds__(256) void head_norm_temp_append_kernel(HeadNormArgs
   }
 }
 
+// The same for heads of quadruples up to 128 values: a head is half a wave's, 16 bytes a lane.  2048 rows of 24 heads of 128: 19.3 -> 14.4 us (50 MB): a wave's life is its round trips, and
+// it carries four times the bytes.
+__global__ __launch_bounds__(256) void head_norm_temp_append_vec_kernel(HeadNormArgs a) {
+  const int hv = blockIdx.x * 8 + (threadIdx.x >> 5), i = 4 * (threadIdx.x & 31), m = blockIdx.y;
+  const int nh = a.H + 2 * a.G;
+  if (hv >= nh) return;
+  const float* row = a.qkv + (int64_t)m * a.ldqkv;
+  const bool is_q = hv < a.H, is_v = hv >= a.H + a.G;
+  const int n = is_v ? a.vdim : a.dim;
+  const float* src = row + (is_v ? (int64_t)(a.H + a.G) * a.dim + (int64_t)(hv - a.H - a.G) * a.vdim : (int64_t)hv * a.dim);
+  f32x4 v = *reinterpret_cast<const f32x4*>(src + (i < n ? i : 0));
+  const int seq = a.row_seq[m], slot = a.row_slot[m];
+  const int64_t crow = (int64_t)seq * a.t_max + slot;
+  if (i >= n) v = f32x4{0.f, 0.f, 0.f, 0.f};
+  float ss = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) ss += __shfl_xor(ss, o);
+  float* dst = is_v ? a.v_arena + crow * ((int64_t)a.G * a.vdim) + (int64_t)(hv - a.H - a.G) * a.vdim
+               : is_q ? a.q_out + (int64_t)m * a.ldq + (int64_t)hv * a.dim
+                      : a.k_arena + crow * ((int64_t)a.G * a.dim) + (int64_t)(hv - a.H) * a.dim;
+  if (i >= n) return;
+  if (!is_v) {
+    const float r = 1.0f / sqrtf(ss / (float)a.dim + a.eps);
+    const bf16_t* w = is_q ? a.qw : a.kw;
+    float f = 1.0f;
+    if (is_q) {
+      f = a.q_scale;
+      if (a.temp_every > 0 && a.temp_coef != 0.f) f *= 1.0f + a.temp_coef * logf((float)((slot + 1) / a.temp_every) + 1.0f);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = v[e] * r * (w ? bf16_to_f32(w[i + e]) : 1.0f) * f;
+  }
+  *reinterpret_cast<f32x4*>(dst + i) = v;
+}
+
 // ---------------------------------------------------------------------------------------------------------------------------
 // Decayed linear-attention recurrence, one thread per (head, value column): S[:, c] = decay S[:, c] + k v[c], o[c] = S[:, c] . q, with
 // q, k, v = silu of the projected rows.  The workgroup of a sequence's FIRST row in the step walks that sequence's rows; q and k of
@@ -262,16 +297,17 @@ template <bool V4, typename F>
 __device__ __forceinline__ void stage_silu(float* __restrict__ dst, int ld, const float* __restrict__ src, int64_t lds_, int n, int d, int tid, F f) {
   if (V4) {
     const int lq = ld / 4, cnt = LCH * lq;
+    const float per = 1.0f / (float)lq;                // (x + 1/2) / lq is no nearer to a whole number than 1 / 2 lq: exact as floats up to 2^22 / lq rows
     for (int x0 = tid; x0 < cnt; x0 += 1024) {
       f32x4 t[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int x = x0 + 256 * u, j = x / lq, i = 4 * (x - j * lq);
+        const int x = x0 + 256 * u, j = (int)(((float)x + 0.5f) * per), i = 4 * (x - j * lq);
         t[u] = *reinterpret_cast<const f32x4*>(src + (int64_t)min(j, n - 1) * lds_ + (i < d ? i : 0));
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int x = x0 + 256 * u, j = x / lq, i = 4 * (x - j * lq);
+        const int x = x0 + 256 * u, j = (int)(((float)x + 0.5f) * per), i = 4 * (x - j * lq);
         if (x >= cnt) break;
         f32x4 r = f32x4{0.f, 0.f, 0.f, 0.f};
         if (j < n && i < d) {                          // (a chunk of a few rows: most waves have none)
@@ -291,8 +327,8 @@ __device__ __forceinline__ void stage_silu(float* __restrict__ dst, int ld, cons
 }
 
 // Pass 1 on the fp32 matrix cores: wave w owns the 16-row tiles w, w + 4, .. of the own sum, their k columns (all 32 rows) in registers, and walks
-// the 16-column tiles of v.  Bound by the staging and the 64 KB a (chunk, head) writes: 2048 rows x 16 heads of 128 + 128: 44 us with FMAs on
-// four-byte staged rows, 34 us here.
+// the 16-column tiles of v, which are the first operand: a lane's four sums are then neighbours in a row of the state and leave together (V4).  Bound by the staging and the 64 KB a (chunk, head)
+// writes: 2048 rows x 16 heads of 128 + 128: 44 us with FMAs on four-byte staged rows, 37 with sums stored one by one, 35.7 here.
 template <bool V4>
 __global__ __launch_bounds__(256) void light_scan_kv_mfma_kernel(LightScanArgs s, int ldk, int ldv) {
   extern __shared__ float lds[];             // k [32][ldk] (decayed), v [32][ldv]
@@ -318,15 +354,21 @@ __global__ __launch_bounds__(256) void light_scan_kv_mfma_kernel(LightScanArgs s
       const float* vb = vl + g4 * ldv + 16 * tc + c16;
 #pragma unroll
       for (int it = 0; it < LCH / 4; ++it) {
-        a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[it], vb[4 * it * ldv], a0, 0, 0, 0);
-        if (two) a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[it], vb[4 * it * ldv + 16], a1, 0, 0, 0);
+        a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(vb[4 * it * ldv], kf[it], a0, 0, 0, 0);
+        if (two) a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(vb[4 * it * ldv + 16], kf[it], a1, 0, 0, 0);
+      }
+      const int r = 16 * ti + c16, c = 16 * tc + 4 * g4;
+      if (r >= d) continue;
+      float* o = dst + (int64_t)r * e + c;
+      if (V4) {
+        if (c < e) *reinterpret_cast<f32x4*>(o) = a0;
+        if (c + 16 < e) *reinterpret_cast<f32x4*>(o + 16) = a1;
+        continue;
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = 16 * ti + 4 * g4 + i, c = 16 * tc + c16;
-        if (r >= d) continue;
-        if (c < e) dst[(int64_t)r * e + c] = a0[i];
-        if (two && c + 16 < e) dst[(int64_t)r * e + c + 16] = a1[i];
+        if (c + i < e) o[i] = a0[i];
+        if (c + i + 16 < e) o[i + 16] = a1[i];
       }
     }
   }
@@ -510,10 +552,10 @@ __global__ __launch_bounds__(256) void light_scan_out_kernel(LightScanArgs s) {
 // activated and zero padded; waves 0 .. 2 multiply the three 16 x 16 score tiles on or below the diagonal and park them, decayed and
 // masked, in LDS; then wave w owns the 16-column tiles w, w + 4, .. of the result, both row tiles at once: Q S0 with the carried state
 // read straight from the workspace (8 loads in flight), times lam^(i + 1) by rows, plus P V.  2048 rows, 16 heads of 128 + 128: 98 us
-// with four-byte staging and state reads, 52 us here (64 MB of states, 50 MB of rows).
+// with four-byte staging and state reads, 55 with two workgroups a CU and a division a staged quadruple, 50 us here (64 MB of states, 50 MB of rows).
 template <bool V4>
 __global__ __launch_bounds__(256) void light_scan_out_mfma_kernel(LightScanArgs s, int ldq, int ldv) {
-  extern __shared__ float lds[];             // q [32][ldq], k [32][ldq], v [32][ldv], P [32][36]
+  extern __shared__ float lds[];             // q [32][ldq], k [32][ldq] and, once they are multiplied, P [32][36], v [32][ldv]
   constexpr int LDP = 36;
   const LightArgs& a = s.b;
   const int ch = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, d = a.dim, e = a.vdim;
@@ -521,8 +563,8 @@ __global__ __launch_bounds__(256) void light_scan_out_mfma_kernel(LightScanArgs 
   const int wave = tid >> 6, lane = tid & 63, c16 = lane & 15, g4 = lane >> 4;
   float* ql = lds;
   float* kl = ql + LCH * ldq;
-  float* vl = kl + LCH * ldq;
-  float* P = vl + LCH * ldv;
+  float* vl = kl + LCH * max(ldq, LDP);
+  float* P = kl;                             // (a place of its own is 4.6 KB more: two workgroups a CU instead of three at heads of 128)
   const float lam = a.decay[h], ll = lam > 0.f ? logf(lam) : 0.f;
   const float* row0 = a.qkv + (int64_t)r0 * a.ldqkv;
   const auto one = [](int) { return 1.0f; };
@@ -531,9 +573,10 @@ __global__ __launch_bounds__(256) void light_scan_out_mfma_kernel(LightScanArgs 
   stage_silu<V4>(vl, ldv, row0 + (int64_t)2 * a.H * d + (int64_t)h * e, a.ldqkv, n, e, tid, one);
   __syncthreads();
   const int ksteps = (d + 3) / 4;            // ldq >= 4 ksteps, the padding is zero
-  if (wave < 3) {                            // score tiles (0, 0), (1, 0), (1, 1)
-    const int ti = wave == 0 ? 0 : 1, tj = wave == 2 ? 1 : 0;
-    f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f}, sc2 = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f}, sc2 = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int ti0 = wave == 0 ? 0 : 1, tj0 = wave == 2 ? 1 : 0;            // score tiles (0, 0), (1, 0), (1, 1)
+  if (wave < 3) {
+    const int ti = ti0, tj = tj0;
     const float* ap = ql + (16 * ti + c16) * ldq + g4;
     const float* bp = kl + (16 * tj + c16) * ldq + g4;
     int it = 0;
@@ -543,9 +586,12 @@ __global__ __launch_bounds__(256) void light_scan_out_mfma_kernel(LightScanArgs 
     }
     if (it < ksteps) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(ap[4 * it], bp[4 * it], sc, 0, 0, 0);
     sc += sc2;
+  }
+  __syncthreads();
+  if (wave < 3) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int row = 16 * ti + 4 * g4 + i, col = 16 * tj + c16;
+      const int row = 16 * ti0 + 4 * g4 + i, col = 16 * tj0 + c16;
       P[row * LDP + col] = col <= row ? sc[i] * powi32(lam, ll, row - col) : 0.f;
     }
   } else {                                   // the tile above the diagonal
@@ -673,6 +719,37 @@ __global__ __launch_bounds__(256) void rms_sigmoid_gate_kernel(const float* __re
   }
 }
 
+// The same for rows of quadruples up to 1024 Q values: row and gate are asked for once, 16 bytes at a time, and the row stays in registers.  2048 rows of 2048: 17.7 -> 12.8 us (42 MB).
+template <int Q>
+__global__ __launch_bounds__(256) void rms_sigmoid_gate_vec_kernel(const float* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ w, float eps, const float* __restrict__ g, int64_t ldg,
+                                                                   float* __restrict__ y, int64_t ldy, bf16_t* __restrict__ y16, int64_t ldy16, int n) {
+  __shared__ float red[4];
+  const int m = blockIdx.x, tid = threadIdx.x;
+  f32x4 v[Q], u[Q];
+  ushort4 k[Q];
+#pragma unroll
+  for (int j = 0; j < Q; ++j) {
+    const int i = 4 * (tid + 256 * j), ic = i < n ? i : 0;
+    v[j] = *reinterpret_cast<const f32x4*>(x + (int64_t)m * ldx + ic);
+    u[j] = *reinterpret_cast<const f32x4*>(g + (int64_t)m * ldg + ic);
+    k[j] = *reinterpret_cast<const ushort4*>(w + ic);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < Q; ++j)
+    if (4 * (tid + 256 * j) < n) ss += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
+  const float r = 1.0f / sqrtf(block_sum(ss, red) / (float)n + eps);
+#pragma unroll
+  for (int j = 0; j < Q; ++j) {
+    const int i = 4 * (tid + 256 * j);
+    if (i >= n) continue;
+    const f32x4 o = {v[j][0] * r * bf16_to_f32(k[j].x) * sigm32(u[j][0]), v[j][1] * r * bf16_to_f32(k[j].y) * sigm32(u[j][1]), v[j][2] * r * bf16_to_f32(k[j].z) * sigm32(u[j][2]),
+                     v[j][3] * r * bf16_to_f32(k[j].w) * sigm32(u[j][3])};
+    if (y) *reinterpret_cast<f32x4*>(y + (int64_t)m * ldy + i) = o;
+    if (y16) *reinterpret_cast<uint2*>(y16 + (int64_t)m * ldy16 + i) = uint2{cvt_pk_bf16(o[0], o[1]), cvt_pk_bf16(o[2], o[3])};
+  }
+}
+
 __global__ __launch_bounds__(256) void relu2_kernel(const float* __restrict__ x, int64_t ldx, float* __restrict__ y, int64_t ldy,
                                                     bf16_t* __restrict__ y16, int64_t ldy16, int n) {
   const int m = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
@@ -792,7 +869,9 @@ extern "C" int mn_head_norm_temp_append(const float* qkv, int64_t ldqkv, int M, 
                    vdim >= 1 && t_max >= 1, "mn_head_norm_temp_append: bad args (dim=%d: at most 512)", dim);
   HeadNormArgs a{qkv, ldqkv, H, G, dim, vdim, q_norm, k_norm, eps, q_scale, temp_coef, temp_every, row_seq, row_slot, q_out, ldq, k_arena, v_arena,
                  t_max};
-  hipLaunchKernelGGL(head_norm_temp_append_kernel, dim3((unsigned)mn_cdiv(H + 2 * G, 4), (unsigned)M), dim3(256), 0, mn_stream(stream), a);
+  const bool vec = dim <= 128 && vdim <= 128 && ((dim | vdim) % 4) == 0 && ((ldqkv | ldq) % 4) == 0 && (((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_arena | (uintptr_t)v_arena) & 15) == 0;
+  if (vec) hipLaunchKernelGGL(head_norm_temp_append_vec_kernel, dim3((unsigned)mn_cdiv(H + 2 * G, 8), (unsigned)M), dim3(256), 0, mn_stream(stream), a);
+  else hipLaunchKernelGGL(head_norm_temp_append_kernel, dim3((unsigned)mn_cdiv(H + 2 * G, 4), (unsigned)M), dim3(256), 0, mn_stream(stream), a);
   MN_CHECK_LAUNCH("mn_head_norm_temp_append");
   return MN_OK;
 }
@@ -839,7 +918,8 @@ namespace {
 // row strides of the matrix-core pass: q / k rows = 4 mod 32 floats, v rows = 16 mod 32 — the operand reads of a wave then fall two to a bank
 inline int scan_ldq(int dim) { const int p = (dim + 3) / 4 * 4; return p + ((p % 32) == 0 ? 4 : ((36 - p % 32) % 32)); }
 inline int scan_ldv(int vdim) { const int p = (vdim + 15) / 16 * 16; return p + ((p % 32) == 0 ? 16 : 0); }
-inline size_t scan_mfma_lds(int dim, int vdim) { return ((size_t)LCH * (2 * scan_ldq(dim) + scan_ldv(vdim)) + LCH * 36) * sizeof(float); }
+inline size_t scan_mfma_lds(int dim, int vdim) { return ((size_t)LCH * (2 * scan_ldq(dim) + scan_ldv(vdim)) + LCH * 36) * sizeof(float); }      // (what decides whether the pass is taken)
+inline size_t scan_out_lds(int dim, int vdim) { return (size_t)LCH * (scan_ldq(dim) + (scan_ldq(dim) > 36 ? scan_ldq(dim) : 36) + scan_ldv(vdim)) * sizeof(float); }
 }  // namespace
 
 extern "C" int mn_lightning_rows_scan(const float* qkv, int64_t ldqkv, int M, int H, int dim, int vdim, const float* decay, float* state,
@@ -888,9 +968,9 @@ extern "C" int mn_lightning_rows_scan_ex(const float* qkv, int64_t ldqkv, int M,
   if (variant == MN_LIGHTNING_SCAN_MFMA) {
     MN_CHECK_ARG(scan_mfma_lds(dim, vdim) <= 64 * 1024, "mn_lightning_rows_scan: heads of %d + %d values do not fit the matrix-core pass", dim, vdim);
     // (the vector form deals out 64 columns at a time to four waves a SIMD, where the other has six: 1024 chunks of one row, 2 heads of 16 x 16: 19.5 against 12.5 us)
-    if (r4 && vdim > 32) hipLaunchKernelGGL((light_scan_out_mfma_kernel<true>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), scan_mfma_lds(dim, vdim), st, s,
+    if (r4 && vdim > 32) hipLaunchKernelGGL((light_scan_out_mfma_kernel<true>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), scan_out_lds(dim, vdim), st, s,
                                             scan_ldq(dim), scan_ldv(vdim));
-    else hipLaunchKernelGGL((light_scan_out_mfma_kernel<false>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), scan_mfma_lds(dim, vdim), st, s,
+    else hipLaunchKernelGGL((light_scan_out_mfma_kernel<false>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), scan_out_lds(dim, vdim), st, s,
                             scan_ldq(dim), scan_ldv(vdim));
   } else if (v4) hipLaunchKernelGGL((light_scan_out_kernel<4>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), lds3, st, s);
   else hipLaunchKernelGGL((light_scan_out_kernel<1>), dim3((unsigned)n_chunks, (unsigned)H), dim3(256), lds3, st, s);
@@ -901,7 +981,15 @@ extern "C" int mn_lightning_rows_scan_ex(const float* qkv, int64_t ldqkv, int M,
 extern "C" int mn_rms_sigmoid_gate_rows(const float* x, int64_t ldx, const uint16_t* w, float eps, const float* g, int64_t ldg, float* y,
                                         int64_t ldy, uint16_t* y16, int64_t ldy16, int M, int n, void* stream) {
   MN_CHECK_ARG(x && w && g && (y || y16) && M >= 1 && n >= 1, "mn_rms_sigmoid_gate_rows: bad args");
-  hipLaunchKernelGGL(rms_sigmoid_gate_kernel, dim3((unsigned)M), dim3(256), 0, mn_stream(stream), x, ldx, w, eps, g, ldg, y, ldy, y16, ldy16, n);
+  hipStream_t st = mn_stream(stream);
+  const bool vec = n <= 4096 && (n % 4) == 0 && ((ldx | ldg) % 4) == 0 && (((uintptr_t)x | (uintptr_t)g | (uintptr_t)y) & 15) == 0 && (((uintptr_t)w | (uintptr_t)y16) & 7) == 0 &&
+                   (!y || ldy % 4 == 0) && (!y16 || ldy16 % 4 == 0);
+#define MN_RSG(Q_) hipLaunchKernelGGL((rms_sigmoid_gate_vec_kernel<Q_>), dim3((unsigned)M), dim3(256), 0, st, x, ldx, w, eps, g, ldg, y, ldy, y16, ldy16, n)
+  if (!vec) hipLaunchKernelGGL(rms_sigmoid_gate_kernel, dim3((unsigned)M), dim3(256), 0, st, x, ldx, w, eps, g, ldg, y, ldy, y16, ldy16, n);
+  else if (n <= 1024) MN_RSG(1);
+  else if (n <= 2048) MN_RSG(2);
+  else MN_RSG(4);
+#undef MN_RSG
   MN_CHECK_LAUNCH("mn_rms_sigmoid_gate_rows");
   return MN_OK;
 }

@@ -400,7 +400,13 @@ __device__ __forceinline__ float dpp_add_to(float own, float other) {
   return own + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(other), CTRL, 0xf, 0xf, true));
 }
 
-// The same walk for heads of at most 256 state rows, without a branch in the step: grid (H * ceil(vdim / CPB), S):
+// of every two neighbouring rows of 16 lanes: in the first one a's sum over both, in the second b's
+__device__ __forceinline__ float rows_sum(float a, float b) {
+  const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+}
+
+// The same walk for heads of at most 256 state rows, without a branch in the step: workgroups x < H * ceil(vdim / CPB), y < S:
 // workgroup y takes the step's sequences y, y + S, .., from a table of their first rows that it makes once (TABLE: at most 2048 rows).  LPC lanes share a value column
 // (CPB = 256 / LPC columns a workgroup); a lane holds the state rows 4 (s + LPC jj) + t, t < 4, jj < NS / 4, so that q and k come from
 // LDS in 16-byte reads; LDS rows are padded with zeros to DP = NS * LPC values, under which the padded state rows stay zero.
@@ -410,17 +416,14 @@ __device__ __forceinline__ float dpp_add_to(float own, float other) {
 // 128 + 128: 74 us (98 with loads of 4 bytes and sums row by row, 83 with the wide loads alone); one sequence of 2048 rows 288 (397); 300 rows, 2 heads of 256 + 128 78
 // (110); 256 sequences of two rows 152 (181).  Operands read two rows ahead took 87 for 83, four rows solved at once (their products with each other made beforehand) 105.
 template <int NS, int LPC, int DBT, bool TABLE, bool VEC>
-__global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
+__device__ __forceinline__ void delta_walk(const DeltaArgs& a, int bx, int by, int ny, float* __restrict__ lds, const uint16_t* __restrict__ first, uint64_t (&mask)[32], int count) {
   constexpr int CPB = 256 / LPC, DP = NS * LPC, NQ = DBT * 2 * DP / 256, NV = (DBT * CPB + 255) / 256;
-  extern __shared__ float lds[];             // [DBT][2 DP] q, k; [DBT][CPB] v; [DBT] beta, decay; [DBT][CPB] outputs
-  const int ncb = (a.vdim + CPB - 1) / CPB, h = blockIdx.x / ncb, cb = blockIdx.x - h * ncb;
+  // lds: [DBT][2 DP] q, k; [DBT][CPB] v; [DBT] beta, decay; [DBT][CPB] outputs
+  const int ncb = (a.vdim + CPB - 1) / CPB, h = bx / ncb, cb = bx - h * ncb;
   const int tid = threadIdx.x, s = tid % LPC, cl = tid / LPC, c = cb * CPB + cl;
   const int d = a.dim, kvh = h / (a.H / a.G);
   const bool on = c < a.vdim;
-  __shared__ uint64_t mask[32];
-  __shared__ uint16_t first[2049];
-  const int count = TABLE ? sequence_starts(a.row_back, a.M, mask, first) : a.M;
-  for (int seq = blockIdx.y; seq < count; seq += gridDim.y) {
+  for (int seq = by; seq < count; seq += ny) {
     int m0, n;
     if constexpr (TABLE) {
       m0 = __builtin_amdgcn_readfirstlane(first[seq]);
@@ -521,7 +524,8 @@ __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
 #pragma unroll
           for (int i = 0; i < NS; i += 2) { pk = fmaf(S[i], kk[b][i], pk); pk2 = fmaf(S[i + 1], kk[b][i + 1], pk2); }
           pk += pk2;
-          if (LPC == 16) pk = row16_sum(pk); else pk = sum8(pk);
+          if (LPC == 8) pk = sum8(pk); else pk = row16_sum(pk);
+          if (LPC == 32) pk = rows_sum(pk, pk);
           const float u = beta[b] * (v[b] - g[b] * pk);
 #pragma unroll
           for (int i = 0; i < NS; ++i) S[i] = fmaf(g[b], S[i], kk[b][i] * u);
@@ -529,12 +533,15 @@ __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
           for (int i = 0; i < NS; i += 2) { pq = fmaf(S[i], qq[b][i], pq); pq2 = fmaf(S[i + 1], qq[b][i + 1], pq2); }
           o[j] = pq + pq2;
         }
-        // four rows' outputs at once: lanes that hold the sums of one row each after two exchanges (with the lane mirrored in 16, then in 8; of 8 lanes: in 8, then in 4)
-        const bool hi1 = LPC == 16 ? (s & 8) != 0 : (s & 4) != 0, hi2 = LPC == 16 ? (s & 4) != 0 : (s & 2) != 0;
-        constexpr int M1 = LPC == 16 ? 0x140 : 0x141, M2 = LPC == 16 ? 0x141 : 0x1B;
-        const float x = dpp_add_to<M1>(hi1 ? o[1] : o[0], hi1 ? o[0] : o[1]), y = dpp_add_to<M1>(hi1 ? o[3] : o[2], hi1 ? o[2] : o[3]);
+        // four rows' outputs at once: lanes that hold the sums of one row each after two exchanges (of 32 lanes: between the rows of 16, then with the lane mirrored in 16; of 16: in 16, then in 8;
+        // of 8: in 8, then in 4)
+        const bool hi1 = (s & LPC / 2) != 0, hi2 = (s & LPC / 4) != 0;
+        constexpr int M1 = LPC == 16 ? 0x140 : 0x141, M2 = LPC == 32 ? 0x140 : LPC == 16 ? 0x141 : 0x1B;
+        const float x = LPC == 32 ? rows_sum(o[0], o[1]) : dpp_add_to<M1>(hi1 ? o[1] : o[0], hi1 ? o[0] : o[1]);
+        const float y = LPC == 32 ? rows_sum(o[2], o[3]) : dpp_add_to<M1>(hi1 ? o[3] : o[2], hi1 ? o[2] : o[3]);
         float z = dpp_add_to<M2>(hi2 ? y : x, hi2 ? x : y);
-        if (LPC == 16) z = dpp_add<0x4E>(z);
+        if (LPC == 32) z = dpp_add<0x141>(z);
+        if (LPC >= 16) z = dpp_add<0x4E>(z);
         z = dpp_add<0xB1>(z);
         os[(r0 + (hi1 ? 1 : 0) + (hi2 ? 2 : 0)) * CPB + cl] = z;
       }
@@ -552,6 +559,45 @@ __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
         if (i < d) sp[(int64_t)i * a.vdim] = S[j];
       }
     }
+  }
+}
+
+template <int NS, int LPC, int DBT, bool TABLE, bool VEC>
+__global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
+  extern __shared__ float lds[];
+  __shared__ uint64_t mask[32];
+  __shared__ uint16_t first[2049];
+  const int count = TABLE ? sequence_starts(a.row_back, a.M, mask, first) : a.M;
+  delta_walk<NS, LPC, DBT, TABLE, VEC>(a, blockIdx.x, blockIdx.y, gridDim.y, lds, first, mask, count);
+}
+
+// Heads of 65 .. 128 state rows with a table: 32 lanes a column, 8 columns a workgroup, where the longest sequence's chain of steps is the time, and 16 lanes a column where all sequences
+// together fill the chip: a step of 32 lanes is 33 instructions, one of 16 50 for twice the columns.  us, 16 lanes alone -> here, heads of 128 x 128: 1900 rows of 8 heads 272 -> 217, of 16 277 -> 230, 300
+// of 2 47 -> 38, 470 .. 93 rows of 5 sequences, 8 heads 78 -> 67; of 16 heads 87 and 85, two of 500 81 and 79 (32 lanes: 90 and 82), 16 of 64 37 (32 lanes 41).  The rule is an estimate of both: a
+// step of a chain takes 110 / 138 ns, a step of a workgroup on a CU that is full of them 64 / 118 for half the workgroups; 15 % in favour of 16 lanes, whose rows are staged for twice the columns.
+// Looking for the longest costs sequences of two rows 1 % (256 of them, 8 heads 112.8 -> 114).
+// Grid (2 H ceil(vdim / 16), S): of 16 lanes, the second half of x takes every other sequence.
+template <bool VEC>
+__global__ __launch_bounds__(256) void delta_rows_lanes_kernel(DeltaArgs a) {
+  extern __shared__ float lds[];
+  __shared__ uint64_t mask[32];
+  __shared__ uint16_t first[2049];
+  __shared__ int longest;
+  if (threadIdx.x == 0) longest = 0;
+  const int count = sequence_starts(a.row_back, a.M, mask, first);
+  int n = 0;
+  for (int i = threadIdx.x; i < count; i += 256) n = max(n, (int)first[i + 1] - (int)first[i]);
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) n = max(n, __shfl_xor(n, o));
+  if (n && (threadIdx.x & 63) == 0) atomicMax(&longest, n);
+  __syncthreads();
+  const int x16 = a.H * ((a.vdim + 15) / 16), x32 = a.H * ((a.vdim + 7) / 8);
+  const float chain = (float)longest, all = (float)a.M * x32 / 256.0f;
+  if (1.15f * fmaxf(110.0f * chain, 64.0f * all) < fmaxf(138.0f * chain, 59.0f * all)) {
+    if ((int)blockIdx.x < x32) delta_walk<4, 32, 32, true, VEC>(a, blockIdx.x, blockIdx.y, gridDim.y, lds, first, mask, count);
+  } else {
+    const int late = (int)blockIdx.x >= x16;
+    delta_walk<8, 16, 32, true, VEC>(a, blockIdx.x - late * x16, 2 * blockIdx.y + late, 2 * gridDim.y, lds, first, mask, count);
   }
 }
 
@@ -746,7 +792,15 @@ extern "C" int mn_gated_delta_rows(const float* qkv, int64_t ld, const float* bd
     if (M <= 2048) { if (vec) MN_DFT(NS_, LPC_, DB_, true, true); else MN_DFT(NS_, LPC_, DB_, true, false); }            \
     else { if (vec) MN_DFT(NS_, LPC_, DB_, false, true); else MN_DFT(NS_, LPC_, DB_, false, false); }                    \
   } while (0)
-    if (dim <= 32) MN_DF(4, 8, 32); else if (dim <= 64) MN_DF(4, 16, 32); else if (dim <= 128) MN_DF(8, 16, 32); else MN_DF(16, 16, 16);
+    if (dim <= 32) MN_DF(4, 8, 32); else if (dim <= 64) MN_DF(4, 16, 32); else if (dim > 128) MN_DF(16, 16, 16);
+    else if (M > 2048) MN_DF(8, 16, 32);
+    else {
+      const int64_t gx = 2 * (int64_t)H * mn_cdiv(vdim, 16);
+      const dim3 lanes((unsigned)gx, slots(gx));
+      const size_t bytes = ((size_t)32 * 256 + 2 * 32 * 16 + 2 * 32) * sizeof(float);
+      if (dim == 128 && (ld % 4) == 0 && ((uintptr_t)qkv & 15) == 0) hipLaunchKernelGGL(delta_rows_lanes_kernel<true>, lanes, dim3(256), bytes, st, a);
+      else hipLaunchKernelGGL(delta_rows_lanes_kernel<false>, lanes, dim3(256), bytes, st, a);
+    }
 #undef MN_DF
 #undef MN_DFT
   } else {

@@ -764,6 +764,125 @@ __global__ __launch_bounds__(256) void window_attn_tiled_kernel(AttnTArgs a) {
 
 #include "attn_rows.inl"
 
+// Decode rows (a row a run) of up to four heads a key head, heads of 68 .. 128 values in quadruples: a wave takes groups of 16 keys for itself, keys and values 16 bytes a lane, and asks for the next
+// group's as soon as this one's are in use; nothing crosses waves until the end.  Scores: four lanes a key; the softmax: lane (key, head); values: half a wave a key, four columns a lane.  The tiled
+// form above asks for a tile's values, 4 bytes a lane, behind two barriers and the scores.  24 rows of 16 heads of 128 over four key heads and 1000 keys (98 MB): 37.2 -> 26.5 us with the join, 64 rows of 2048 keys 169 -> 103 (5.2 TB/s), one
+// row of 1000 16.3 -> 11.0; error against 64 bits 2.5e-7 -> 1.7e-7.
+__global__ __launch_bounds__(256) void window_attn_decode_kernel(AttnTArgs a) {
+  __shared__ __attribute__((aligned(16))) float qs[4 * 128], red[4][4][128], pk[4][16][4], fix[4][4], wm[4][4], wl[4][4];
+  const int tid = threadIdx.x, b = blockIdx.x, gy = blockIdx.y, sp = blockIdx.z, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int rep = a.H / a.G, chunks = (rep + a.hpc - 1) / a.hpc;
+  const int g = gy / chunks, h0 = g * rep + (gy % chunks) * a.hpc, Rc = min(a.hpc, g * rep + rep - h0);
+  const int seq = a.row_seq[b], pos = a.row_slot[b];
+  const int nb = win_nb(pos, a.window, a.pool), tF = first_key(a, pos), nk = nb + (pos - tF + 1);      // (a row sees all of these)
+  const int ntile = (nk + AKT - 1) / AKT, tps = (ntile + a.nsplit - 1) / a.nsplit, k0 = sp * tps * AKT, k1 = min(nk, k0 + tps * AKT);
+  const int Gd = a.G * a.dim, Gv = a.G * a.vdim;
+  const float* kb = a.k + ((int64_t)seq * a.t_max + tF) * a.ldk + (int64_t)g * a.dim;
+  const float* vb = a.v + ((int64_t)seq * a.t_max + tF) * a.ldv + (int64_t)g * a.vdim;
+  const float* pkb = a.pk ? a.pk + (int64_t)seq * a.n_pool_max * Gd + (int64_t)g * a.dim : nullptr;
+  const float* pvb = a.pv ? a.pv + (int64_t)seq * a.n_pool_max * Gv + (int64_t)g * a.vdim : nullptr;
+  const int key = lane >> 2, part = lane & 3, half = lane >> 5, col = 4 * (lane & 31), cc = col < a.vdim ? col : 0;
+  f32x4 kv[8], vv[8];
+  auto keys = [&](int j0) {
+    const int j = min(j0 + key, k1 - 1);
+    const float* p = j < nb ? pkb + (int64_t)j * Gd : kb + (int64_t)(j - nb) * a.ldk;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) kv[u] = *reinterpret_cast<const f32x4*>(p + (4 * (part + 4 * u) < a.dim ? 4 * (part + 4 * u) : 0));      // (past the head: times a zero of the query)
+  };
+  auto values = [&](int j0) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int j = min(j0 + 2 * u + half, k1 - 1);
+      vv[u] = *reinterpret_cast<const f32x4*>((j < nb ? pvb + (int64_t)j * Gv : vb + (int64_t)(j - nb) * a.ldv) + cc);
+    }
+  };
+  const int first = k0 + 16 * wave;
+  if (first < k1) { keys(first); values(first); }
+  for (int e = tid; e < 4 * 128; e += 256) {
+    const int i = e >> 7, d = e & 127;
+    qs[e] = i < Rc && d < a.dim ? a.q[(int64_t)b * a.ldq + (int64_t)(h0 + i) * a.dim + d] : 0.f;
+  }
+  __syncthreads();
+  f32x4 acc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float mrun = -INFINITY, lrun = 0.f;                  // of head `part`; lrun: this lane's keys
+  const auto order = [] { asm volatile("" ::: "memory"); __builtin_amdgcn_wave_barrier(); };      // (a wave's LDS accesses keep their order: this is the compiler's)
+  for (int j0 = first; j0 < k1; j0 += 64) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const f32x4 q = *reinterpret_cast<const f32x4*>(qs + i * 128 + 4 * (part + 4 * u));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[e] = fmaf(q[e], 4 * (part + 4 * u) < a.dim ? kv[u][e] : 0.f, t[e]);
+      }
+      float v = (t[0] + t[1]) + (t[2] + t[3]);
+      v += __shfl_xor(v, 1);
+      v += __shfl_xor(v, 2);
+      s = part == i ? v : s;
+    }
+    if (j0 + 64 < k1) keys(j0 + 64);
+    s = j0 + key < k1 ? soft_cap(s, a.cap) : -INFINITY;
+    float mx = s;
+#pragma unroll
+    for (int o = 4; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    const float mnew = fmaxf(mrun, mx), corr = mrun == -INFINITY ? 0.f : expf(mrun - mnew);
+    const float p = mnew == -INFINITY || j0 + key >= k1 ? 0.f : expf(s - mnew);
+    lrun = fmaf(lrun, corr, p);
+    order();
+    pk[wave][key][part] = p;
+    if (lane < 4) fix[wave][lane] = corr;
+    order();
+    if (__ballot(mnew != mrun)) {
+      const f32x4 c = *reinterpret_cast<const f32x4*>(fix[wave]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] *= c[i];
+    }
+    mrun = mnew;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const f32x4 w = *reinterpret_cast<const f32x4*>(pk[wave][2 * u + half]), v = j0 + 2 * u + half < k1 ? vv[u] : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] = fmaf(w[i], v[e], acc[i][e]);
+    }
+    if (j0 + 64 < k1) values(j0 + 64);
+  }
+#pragma unroll
+  for (int o = 4; o < 64; o <<= 1) lrun += __shfl_xor(lrun, o);
+  if (lane < 4) { wm[wave][lane] = mrun; wl[wave][lane] = lrun; }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[i][e] += __shfl_xor(acc[i][e], 32);
+    if (half == 0) *reinterpret_cast<f32x4*>(&red[wave][i][col]) = acc[i];
+  }
+  __syncthreads();
+  const int i = tid >> 5;
+  if (i >= Rc || col >= a.vdim) return;
+  float top = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) top = fmaxf(top, wm[w][i]);
+  f32x4 r = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float f = wm[w][i] == -INFINITY ? 0.f : expf(wm[w][i] - top);
+    l = fmaf(wl[w][i], f, l);
+    r += *reinterpret_cast<const f32x4*>(&red[w][i][col]) * f;
+  }
+  if (a.nsplit > 1) {
+    float* part_out = a.part + (((int64_t)b * gridDim.y + gy) * a.nsplit + sp) * ((int64_t)a.sq * (2 + a.vdim));
+    if (col == 0) { part_out[i] = top; part_out[a.sq + i] = l; }
+    part4(a, part_out, i, col, r);
+    return;
+  }
+  emit4(a, r * (softmax_inv(top, l, a.sink, h0 + i) * a.out_scale), b, (int64_t)(h0 + i) * a.vdim, col, emit_vec(a));
+}
+
 // grid (n_blk, G * chunks, ceil(vdim / MERGE_COLS)): the splits' statistics and sums of every vector become its result; a workgroup
 // takes a slice of the value columns (one workgroup a run left the merge of a single decode row on one CU)
 constexpr int MERGE_COLS = 64;
@@ -821,7 +940,7 @@ __global__ __launch_bounds__(256) void window_attn_merge_few_kernel(AttnTArgs a)
   const int g = gy / chunks, h0 = g * rep + (gy % chunks) * a.hpc;
   const int Rc = min(a.hpc, g * rep + rep - h0);
   const int i = e / quads, d = 4 * (e - i * quads);
-  if (i >= min(a.blk_tab[2 * b + 1], a.rows_per_blk) * Rc) return;
+  if (i >= (a.blk_tab ? min(a.blk_tab[2 * b + 1], a.rows_per_blk) : 1) * Rc) return;
   const int64_t stride = (int64_t)a.sq * (2 + a.vdim);
   const float* base = a.part + ((int64_t)b * gridDim.y + gy) * a.nsplit * stride;
   const float* src = base + 2 * a.sq + (int64_t)i * a.vdim;
@@ -848,7 +967,16 @@ __global__ __launch_bounds__(256) void window_attn_merge_few_kernel(AttnTArgs a)
     for (int x = 0; x < 4; ++x) t[x] = fmaf(v[s][x], w, t[x]);
   }
   const int h = h0 + i % Rc;
-  emit4(a, t * (softmax_inv(top, L, a.sink, h) * a.out_scale), a.blk_tab[2 * b] + i / Rc, (int64_t)h * a.vdim, d, emit_vec(a));
+  emit4(a, t * (softmax_inv(top, L, a.sink, h) * a.out_scale), (a.blk_tab ? a.blk_tab[2 * b] : b) + i / Rc, (int64_t)h * a.vdim, d, emit_vec(a));
+}
+
+static void attn_merge(const AttnTArgs& a, int n_blk, int gys, int aq, hipStream_t st) {
+  const dim3 few((unsigned)n_blk, (unsigned)gys, (unsigned)mn_cdiv((int64_t)a.sq * mn_cdiv(a.vdim, 4), 256)), cols((unsigned)n_blk, (unsigned)gys, (unsigned)mn_cdiv(a.vdim, MERGE_COLS));
+  if (a.nsplit <= 2) hipLaunchKernelGGL((window_attn_merge_few_kernel<2>), few, dim3(256), 0, st, a);
+  else if (a.nsplit <= 4) hipLaunchKernelGGL((window_attn_merge_few_kernel<4>), few, dim3(256), 0, st, a);
+  else if (a.nsplit <= MERGE_FEW) hipLaunchKernelGGL((window_attn_merge_few_kernel<MERGE_FEW>), few, dim3(256), 0, st, a);
+  else if (aq == 4) hipLaunchKernelGGL((window_attn_merge_kernel<4>), cols, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((window_attn_merge_kernel<16>), cols, dim3(256), 0, st, a);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -1375,11 +1503,7 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
     }
     MN_CHECK_LAUNCH("mn_window_pool_attn_blocks(mfma)");
     if (nsplit > 1) {
-      const dim3 few((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)mn_cdiv((int64_t)sh.sq * mn_cdiv(vdim, 4), 256));
-      if (!one_row && nsplit <= 2) hipLaunchKernelGGL((window_attn_merge_few_kernel<2>), few, dim3(256), 0, stm, a);
-      else if (!one_row && nsplit <= 4) hipLaunchKernelGGL((window_attn_merge_few_kernel<4>), few, dim3(256), 0, stm, a);
-      else if (!one_row && nsplit <= MERGE_FEW) hipLaunchKernelGGL((window_attn_merge_few_kernel<MERGE_FEW>), few, dim3(256), 0, stm, a);
-      else hipLaunchKernelGGL((window_attn_merge_kernel<16>), dim3((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)mn_cdiv(vdim, MERGE_COLS)), dim3(256), 0, stm, a);
+      attn_merge(a, n_blk, G * sh.chunks, sh.aq, stm);
       MN_CHECK_LAUNCH("mn_window_pool_attn_blocks(merge)");
     }
     return MN_OK;
@@ -1389,7 +1513,10 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
   const bool vec = (dim % 4) == 0 && (ldq % 4) == 0 && (ldk % 4) == 0 && (((uintptr_t)q | (uintptr_t)k_arena | (uintptr_t)pk) & 15) == 0;
   const dim3 grid((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)nsplit);
   hipStream_t st = mn_stream(stream);
-  if (sh.aq == 4) {
+  const bool quads = vec && vdim % 4 == 0 && ldv % 4 == 0 && (((uintptr_t)v_arena | (uintptr_t)pv) & 15) == 0;
+  if (one_row && sh.aq == 4 && quads && dim > 64 && dim <= 128 && vdim > 64 && vdim <= 128) {
+    hipLaunchKernelGGL(window_attn_decode_kernel, grid, dim3(256), 0, st, a);
+  } else if (sh.aq == 4) {
     if (vec) hipLaunchKernelGGL((window_attn_tiled_kernel<4, true>), grid, dim3(256), lds, st, a);
     else hipLaunchKernelGGL((window_attn_tiled_kernel<4, false>), grid, dim3(256), lds, st, a);
   } else {
@@ -1398,9 +1525,7 @@ extern "C" int mn_window_pool_attn_blocks_gate(const float* q, int64_t ldq, cons
   }
   MN_CHECK_LAUNCH("mn_window_pool_attn_blocks");
   if (nsplit > 1) {
-    const dim3 mg((unsigned)n_blk, (unsigned)(G * sh.chunks), (unsigned)mn_cdiv(vdim, MERGE_COLS));
-    if (sh.aq == 4) hipLaunchKernelGGL((window_attn_merge_kernel<4>), mg, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((window_attn_merge_kernel<16>), mg, dim3(256), 0, st, a);
+    attn_merge(a, n_blk, G * sh.chunks, sh.aq, st);
     MN_CHECK_LAUNCH("mn_window_pool_attn_blocks(merge)");
   }
   return MN_OK;

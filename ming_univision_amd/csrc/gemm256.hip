@@ -578,9 +578,31 @@ static int tile_form(int M, int N, int Kc, int nz, bool hilo, int epi, double* u
   return best;
 }
 
+// Column tiles that the small tiles' order takes together: an XCD's eighth of the tiles, row by row of a band, is about a square of them, where column by column it is all rows by a few columns.
+// For plain rows and weights that are both more than most of an XCD's L2 (4 MB): workgroups that are not in step then find less of either.  us, column by column / in bands, weights from HBM: 900 x
+// 2048 x 8192 61 / 50, x 2048 19.0 / 16.7, 1409 x 1024 x 4096 27.5 / 26.6, 2048 x 1024 x 4096 32.7 / 31.3, 2048 x 4096 x 1024 24.7 / 23.2, 4112 x 1024 x 2752 46.4 / 41.7, 3000 x 512 x 8192 67 / 45; with rows or weights
+// below that 600 x 2048 x 2048 13.4 / 14.4, 1300 x 3072 x 1024 16.6 / 17.3, 4112 x 1024 x 1024 19.6 / 20.2; with weights over three times the rows, which more XCDs then read, 512 x 4096 x 4096 32.3 / 33.6,
+// 600 x 2048 x 8192 43.4 / 45.0; hi/lo rows 1025 x 3072 x 1024 21.1 / 21.8, 1058 x 2048 x 2048 32.1 / 31.4.
+static int order_band(int tiles_m, int tiles_n, int bm, int bn, int64_t a_bytes, int64_t w_bytes) {
+  if (a_bytes <= (int64_t)3 << 20 || w_bytes <= (int64_t)3 << 20 || w_bytes > 3 * a_bytes) return 1;
+  const double q = tiles_m * (double)tiles_n / 8;
+  int best = 1;
+  double tb = 1e30;
+  for (int nb = 1; nb <= tiles_n; ++nb) {
+    const int band = (int)mn_cdiv(tiles_n, nb);
+    const double t = fmin(tiles_m, q / band + 1) * bm + fmin(tiles_n, fmax(band, q / tiles_m + 1)) * bn;
+    if (t <= tb) { tb = t; best = band; }
+  }
+  return best;
+}
+
 template <int EPI, int BM, int BN, int WM, int WN, int S, bool HILO, bool TWO = false, int GROUP = 0>
-static void tile_go(const G256& p, int nz, hipStream_t st) {
-  const dim3 grid((unsigned)(mn_cdiv(p.M, BM) * mn_cdiv(p.N, epi_paired(EPI) ? BN / 2 : BN)), nz);
+static void tile_go(const G256& a, int nz, hipStream_t st) {
+  constexpr int cols = epi_paired(EPI) ? BN / 2 : BN;
+  const int tm = (int)mn_cdiv(a.M, BM), tn = (int)mn_cdiv(a.N, cols);
+  G256 p = a;
+  p.group_m = HILO ? 1 : order_band(tm, tn, BM, BN, (int64_t)p.M * p.K * 2, (int64_t)p.N * (BN / cols) * p.K * 2);
+  const dim3 grid((unsigned)((int64_t)tm * tn), nz);
   hipLaunchKernelGGL((gemm_tile_kernel<EPI, HILO, BM, BN, WM, WN, S, TWO, GROUP>), grid, dim3(WM * WN * 64), 0, st, p);
 }
 

@@ -66,8 +66,14 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
     row0 = p.g_off[grp];
     Mg = p.g_cnt[grp];
   } else {
-    m0 = (bid % tiles_m) * BM;
-    n0 = (bid / tiles_m) * cols;
+    int tm = bid % tiles_m, tn = bid / tiles_m;
+    if (p.group_m > 1) {                               // bands of column tiles, row by row (order_band)
+      const int per = tiles_m * p.group_m, b = bid / per, in = bid - b * per, w = min(p.group_m, tiles_n - b * p.group_m);
+      tm = in / w;
+      tn = b * p.group_m + in - tm * w;
+    }
+    m0 = tm * BM;
+    n0 = tn * cols;
   }
   const int kbeg = blockIdx.y * p.Kc, kend = min(p.K, kbeg + p.Kc);
   const int nk = (kend - kbeg) / BK;

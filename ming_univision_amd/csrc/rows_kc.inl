@@ -194,7 +194,9 @@ __global__ __launch_bounds__(512) void rows_kc_kernel(const mn_skinny_args a, in
 // operands read straight from memory, 16 rows apart lane by lane, come at a quarter of that (38 GB/s a CU: 7 of 12 us for 32 rows of 2048).  Each wave has a ring of
 // its own, so nothing but the sum at the end is a barrier.  What is left is the split (130 vector instructions for 32 values of 32 rows, 4 us of the
 // 2048).  Rows of 16-byte aligned values; 2048 x 2048 at 32 rows 14.5 -> 11.1 us.  NX eights of rows are fetched, as many as there are: with sixteen of them always, 5 rows of
-// 32000 x 1024 took 23.4 us beside other work, with eight 16.5.
+// 32000 x 1024 took 23.4 us beside other work, with eight 16.5.  Grid (tiles, rows / 8 NX): 17 .. 32 rows go 16 and the rest where a CU is free for either: half of the rows a CU takes in, and half of
+// the split; the weights come a second time from L2 (us, 32 rows at once / in halves: 2048 x 2048 11.1 / 7.8, 2048 x 768 5.6 / 4.2, 1024 x 1024 6.5 / 4.6; 17
+// rows of 2048 x 2048 10.5 / 7.4; against three launches 2048 x 4096 17.2 / 12.1).
 template <int NX, int NT, int PRO>
 __global__ __launch_bounds__(512) void rows_kc_lds_kernel(const mn_skinny_args a, int paired) {
   constexpr int MT = (NX + 1) / 2;                     // NX: eights of rows that are fetched
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(512) void rows_kc_lds_kernel(const mn_skinny_args a
   __shared__ __attribute__((aligned(1024))) char lds[BYTES];
   float (*red)[R][64] = reinterpret_cast<float (*)[R][64]>(lds);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
-  const int K = a.K, M = a.M, N = a.N, G = paired ? NT / 2 : NT;             // G: tiles of units per workgroup
+  const int mb = blockIdx.y * (8 * NX), K = a.K, M = a.M - mb, N = a.N, G = paired ? NT / 2 : NT;      // mb: this workgroup's first row; G: tiles of units per workgroup
   const int n0 = blockIdx.x * 16 * G;
   // what this lane fetches: row 8 i + lane / 8 of the rows (16 bytes: slot lane % 8, in the order that leaves no bank twice), row lane / 4 of every weight tile
   typedef const __attribute__((address_space(1))) void gptr;
@@ -215,7 +217,7 @@ __global__ __launch_bounds__(512) void rows_kc_lds_kernel(const mn_skinny_args a
   for (int i = 0; i < NX; ++i) {
     const int row = 8 * i + xr;
     xk[i] = 4 * ((lane & 7) ^ ((row >> 1) & 7));
-    xp[i] = a.x + (int64_t)min(row, M - 1) * a.ldx;
+    xp[i] = a.x + (int64_t)(mb + min(row, M - 1)) * a.ldx;
   }
   const int wk = 8 * ((lane & 3) ^ ((wr >> 2) & 3));
   const bf16_t* wp[NT];
@@ -333,7 +335,7 @@ __global__ __launch_bounds__(512) void rows_kc_lds_kernel(const mn_skinny_args a
     for (int t = 0; t < NT; ++t) {
       const int n = n0 + 16 * t + r;
       if (t >= G || n >= N) continue;
-      medium_finish(a, ml, n, y[t], NT > 1 ? y[NT > 1 && paired ? t + NT / 2 : 0] : 0.f);
+      medium_finish(a, mb + ml, n, y[t], NT > 1 ? y[NT > 1 && paired ? t + NT / 2 : 0] : 0.f);
     }
   }
 }

@@ -335,7 +335,7 @@ extern "C" size_t mn_skinny_workspace_bytes_w8(int M, int N, int K, int epilogue
 }
 
 // One launch (rows_kc.inl) for up to 32 rows of bf16 weights, where it is estimated faster than the three launches (`fma` false) or the fp32 FMA kernel of
-// 2 .. 8 rows: 2.5 us + (0.85 + 0.042 M) for every 512 values of K (x 1.7 with two tiles a workgroup, x 1.4 behind an RMSNorm) and round over the CUs, or 0.22 a
+// 2 .. 8 rows: 2.5 us + (0.85 + 0.042 M, or 1.1 where 17 .. 32 rows go in halves) for every 512 values of K (x 1.7 with two tiles a workgroup, x 1.4 behind an RMSNorm) and round over the CUs, or 0.22 a
 // megabyte of weights, against
 // 8.8 + 0.08 M + 0.2 a megabyte of weights, or 3.2 + 0.19 a megabyte + 0.3 per 1024 of K and as much again a row (8 rows at once; 5 .. 7 as 4 + the rest).  The lines
 // this draws, both sides measured: 32 rows of 2048 x 2048 11.9 / 13.7, of 1024 x 4096 20.1 / 14.8, of 8192 x 2048 (two tiles) 18.8 / 22.4, of 3072 x 3072 17.7 /
@@ -358,21 +358,23 @@ static bool rows_kc(const mn_skinny_args& a, bool fma, hipStream_t st, bool ask 
   const int nt = paired || tiles > mn_num_cus() ? 2 : 1;
   const int64_t g = paired ? tiles : mn_cdiv(a.N, 16 * nt);
   const double mb = (paired ? 2.0 : 1.0) * a.N * a.K * 2e-6, kk = a.K / 1024.0;
-  const double here = 2.5 + fmax(0.22 * mb, mn_cdiv(a.K, 512) * (0.85 + 0.042 * a.M) * (nt == 2 ? 1.7 : 1.0) * (a.prologue == MN_PRO_RMSNORM ? 1.4 : 1.0) * mn_cdiv(g, mn_num_cus()));
-  const double row = 0.4 + 0.25 * kk + 0.02 * mb, once = 3.2 + 0.19 * mb + 0.3 * kk;
-  const double there = !fma ? 8.8 + 0.08 * a.M + 0.2 * mb : (a.M > 4 && a.M < 8 ? 2 * once + (a.M - 2) * row : once + (a.M - 1) * row) / 1.15;
-  if (fma && (a.M == 2 || (a.M == 3 && nt == 2 && !paired && a.K <= 1024))) return false;
-  if (g > (fma ? 4 : 1) * mn_num_cus() || here >= there) return false;
-  if (ask) return true;
   // through LDS from 5 rows on, where the rows' loads are the launch (us straight from memory / through LDS: 2048 x 2048 at 4 rows 6.9 / 7.0, 8 rows 7.3 / 7.0, 16
   // rows 8.8 / 7.6, 32 rows 14.5 / 11.1; 1024 x 1024 at 5 rows 4.6 / 4.3, 24 rows 7.5 / 6.4; 32000 x 1024 at 5 rows 19.1 / 19.1), from 7 with two tiles a workgroup
   // and more than 1024 values, whose weights are more (8192 x 2048 at 2 rows 10.7 / 11.9, 6 rows 11.3 / 11.9, 8 rows 12.0 / 11.9, 32 rows 19.6 / 16.3); a norm's gain
   // or a second row would be a load that waits for the pieces in flight behind it
   const bool lds = a.M > (nt == 2 && a.K > 1024 ? 6 : 4) && (a.prologue == MN_PRO_NONE || a.prologue == MN_PRO_SILU) && ((uintptr_t)a.x & 15) == 0 && (a.ldx % 4) == 0;
+  const bool halves = lds && a.M > 16 && 2 * g <= mn_num_cus();      // 16 rows a workgroup
+  const double here = 2.5 + fmax(0.22 * mb, mn_cdiv(a.K, 512) * (halves ? 1.1 : 0.85 + 0.042 * a.M) * (nt == 2 ? 1.7 : 1.0) * (a.prologue == MN_PRO_RMSNORM ? 1.4 : 1.0) * mn_cdiv(g, mn_num_cus()));
+  const double row = 0.4 + 0.25 * kk + 0.02 * mb, once = 3.2 + 0.19 * mb + 0.3 * kk;
+  const double there = !fma ? 8.8 + 0.08 * a.M + 0.2 * mb : (a.M > 4 && a.M < 8 ? 2 * once + (a.M - 2) * row : once + (a.M - 1) * row) / 1.15;
+  if (fma && (a.M == 2 || (a.M == 3 && nt == 2 && !paired && a.K <= 1024))) return false;
+  if (g > (fma ? 4 : 1) * mn_num_cus() || here >= there) return false;
+  if (ask) return true;
 #define MN_KC(MT_, NT_, P_) hipLaunchKernelGGL((rows_kc_kernel<MT_, NT_, P_>), dim3((unsigned)g), dim3(512), 0, st, a, paired ? 1 : 0)
 #define MN_KCL(MT_, NT_, P_)                                                                                                                          \
   do {                                                                                                                                               \
-    if (a.M <= 16 * (MT_) - 8) hipLaunchKernelGGL((rows_kc_lds_kernel<2 * (MT_) - 1, NT_, P_>), dim3((unsigned)g), dim3(512), 0, st, a, paired ? 1 : 0); \
+    if (halves) hipLaunchKernelGGL((rows_kc_lds_kernel<2, NT_, P_>), dim3((unsigned)g, 2), dim3(512), 0, st, a, paired ? 1 : 0);                       \
+    else if (a.M <= 16 * (MT_) - 8) hipLaunchKernelGGL((rows_kc_lds_kernel<2 * (MT_) - 1, NT_, P_>), dim3((unsigned)g), dim3(512), 0, st, a, paired ? 1 : 0); \
     else hipLaunchKernelGGL((rows_kc_lds_kernel<2 * (MT_), NT_, P_>), dim3((unsigned)g), dim3(512), 0, st, a, paired ? 1 : 0);                          \
   } while (0)
 #define MN_KC_P(MT_, NT_)                                              \

@@ -327,10 +327,9 @@ __device__ __forceinline__ void f32_store4(const GemmF32& a, int z, int m, int n
   *reinterpret_cast<f32x4u*>(c) = v;                          // (rows may start at any float)
 }
 
-// More than 2 rows (8 where accesses go value by value) run on the fp32 matrix cores (v_mfma_f32_16x16x4f32: lane l holds row / column l & 15), fp32 rows and bf16 weights
-// widened on the way.  Both kernels give lane l the values 4 (l >> 4) .. + 3 of every 16 of K, so the four products of a 16-step take
-// one 16-byte read of each operand, in an order of K that both share.  Values past K enter as zeros.  V4: rows of A are 16-byte, rows
-// of W 8-byte aligned; else value by value.
+// More than 2 rows (8 where accesses go value by value) run on the matrix cores, fp32 rows and bf16 weights: few tiles on the fp32 ones (v_mfma_f32_16x16x4f32: lane l holds row / column l & 15,
+// weights widened on the way; lane l takes the values 4 (l >> 4) .. + 3 of every 16 of K, so the four products of a 16-step take one 16-byte read of each operand), many on the bf16 ones.
+// Values past K enter as zeros.  V4: rows of A are 16-byte, rows of W 8-byte aligned; else value by value.
 
 // Few tiles: 32 x 16 outputs a workgroup, whose four waves split K; operands straight from memory, the next 32 values in flight during
 // the products.  Latency bounds it (32 rows x 16 heads of 512 x 128: 5 us here, 45 us as one wave a column and 8 rows).  A block of 32
@@ -1249,8 +1248,8 @@ extern "C" int mn_gemm_f32_batched(const float* A, int64_t lda, int64_t a_bs, co
   MN_CHECK_ARG(mn_cdiv(M, 64) <= 65535, "mn_gemm_f32_batched: too many rows");
   const int64_t tiles = mn_cdiv(M, 64) * mn_cdiv(N, 64) * batch;
   // up to 64 rows always take the kernel that keeps its roundings (they are decode rows: error against 64 bits 0.2 .. 0.6e-7 of the summed
-  // magnitudes, the tiles' 2e-7).  More rows: 128 tiles are the break-even (256 rows x 16 x 128 x 512: 17 us either way; 128 rows x 16 x 512 x 128, 256
-  // tiles: 10.6 and 7.3 us; 2048 rows x 4096 x 1024: 354 and 168 us, 292 us on FMA tiles before)
+  // magnitudes).  More rows, from 128 tiles on (us, few / tiles: 200 rows of 16 x 128 x 512, 128 tiles, 17.5 / 11.2; 128 rows, 64 tiles, 10.3 / as many K-steps as those 11.2;
+  // 2048 rows x 4096 x 1024 354 / 94)
   if (M <= 64 || 2 * tiles < mn_num_cus()) {
     const dim3 grid((unsigned)mn_cdiv(N, 16), (unsigned)mn_cdiv(M, 32), (unsigned)batch);
     if (v4) hipLaunchKernelGGL(gemm_f32_few_kernel<true>, grid, dim3(256), 0, st, a);

@@ -43,7 +43,7 @@ Plan make_plan(const mn_seq_model* m, int M, int max_len) {
     if (d.hr > p.hr) p.hr = d.hr;
     if (d.q_rank > p.q_rank) p.q_rank = d.q_rank;
     if (d.ff > p.ff) p.ff = d.ff;
-    // the workspace covers the finest cut of the rows (one run per row) and the most key splits that cut can ask for
+    // the workspace covers the coarsest cut of the rows, which asks for the most key splits, at this length and every shorter one
     const int ks = mn_latent_attn_splits((int)mn_cdiv(M, RB), max_len, l.kv_rank);
     const size_t w = mn_latent_attn_workspace_bytes(M, l.heads, l.kv_rank, ks);
     if (w > p.attn_ws) p.attn_ws = w;

@@ -1273,23 +1273,26 @@ static inline int latent_kt(int r, int variant) {
   return variant == MN_LATENT_ATTN_VALU ? (r <= 256 ? 64 : r <= 512 ? 32 : 16) : (r <= 512 ? 32 : 16);
 }
 
-static inline bool latent_wave(int r) { return r == 128 || r == 256 || r == 384 || r == 512; }
-// Whole tiles a wave: where a wave has two of them or more.  Below, the form whose waves share a tile is the faster one (us, shared / whole: 64 rows over 300 of 512 27.3 / 25.9 .. 28, 8 rows over 2049
-// 27.8 / 29.5, one 22.5 / 24.8, 64 over 64 11.6 / 14.1, 40 rows over 1111 of 256 22.4 / 27.9).
-static inline bool latent_by_wave(int r, int max_len, int ks) { return latent_wave(r) && max_len >= 128 * ks; }
-
+// Two workgroups a CU, at least 64 keys a split.  Never fewer for longer sequences or for fewer runs: scratch sized by it for the longest serves every shorter step.
 extern "C" int mn_latent_attn_splits(int n_blk, int max_len, int r) {
-  const int tiles = (int)mn_cdiv(max_len > 0 ? max_len : 1, 16), blk = n_blk > 0 ? n_blk : 1;
-  const int cap = (int)mn_cdiv(tiles, 4);              // a split works on at least 64 keys
-  int ks = (int)mn_cdiv(2 * (int64_t)mn_num_cus(), blk);      // two workgroups a CU
-  if (latent_wave(r)) {                                // one round of the form whose waves take whole tiles, where it is the one (latent_by_wave)
-    int kw = (r <= 256 ? 2 : 1) * mn_num_cus() / blk;
-    if (kw < 1) kw = 1;
-    if (latent_by_wave(r, max_len, kw)) ks = kw;
-  }
+  const int tiles = (int)mn_cdiv(max_len > 0 ? max_len : 1, 16);
+  int ks = (int)mn_cdiv(2 * (int64_t)mn_num_cus(), n_blk > 0 ? n_blk : 1);
+  const int cap = (int)mn_cdiv(tiles, 4);
   if (ks > cap) ks = cap;
   if (ks > 64) ks = 64;
+  (void)r;
   return ks < 1 ? 1 : ks;
+}
+
+// Whole tiles a wave (0: not that form): where a wave has two of them or more in one round of its workgroups, which is then all the splits there are, of the `ks` that the caller has scratch for;
+// wgs: workgroups a split.  With fewer tiles the form whose waves share one is the faster one (us, shared / whole: 64 rows over 300 of 512 27.3 / 25.9 .. 28, 8 rows over 2049
+// 27.8 / 29.5, one 22.5 / 24.8, 64 over 64 11.6 / 14.1, 40 rows over 1111 of 256 22.4 / 27.9).
+static inline int latent_wave_splits(int r, int max_len, int64_t wgs, int ks) {
+  if (r != 128 && r != 256 && r != 384 && r != 512) return 0;
+  int64_t kw = (r <= 256 ? 2 : 1) * mn_num_cus() / wgs;
+  if (kw < 1) kw = 1;
+  if (kw > ks) kw = ks;
+  return max_len >= 128 * kw ? (int)kw : 0;
 }
 
 extern "C" size_t mn_latent_attn_workspace_bytes(int M, int H, int r, int ks) {
@@ -1306,20 +1309,24 @@ extern "C" int mn_latent_attn_ex(const float* qabs, const float* arena, const in
   MN_CHECK_ARG(ws_bytes >= mn_latent_attn_workspace_bytes(M, H, r, ks) && (ks == 1 || ws), "mn_latent_attn: workspace too small");
   MN_CHECK_ARG(variant == MN_LATENT_ATTN_MFMA || variant == MN_LATENT_ATTN_VALU, "mn_latent_attn: unknown variant %d", variant);
   const int KT = latent_kt(r, variant), RB = mn_latent_attn_block_rows();
-  const int tiles = (int)mn_cdiv(max_len, KT), tps = (int)mn_cdiv(tiles, ks);
+  const int gy = (int)mn_cdiv((n_blk == M ? 1 : RB) * (int64_t)H, 16);
   float* pacc = reinterpret_cast<float*>(ws);
+  const bool aligned = (((uintptr_t)qabs | (uintptr_t)arena | (uintptr_t)lat | (uintptr_t)pacc) & 15) == 0;
+  const int kw = variant == MN_LATENT_ATTN_MFMA && aligned ? latent_wave_splits(r, max_len, (int64_t)n_blk * gy, ks) : 0;
+  if (kw) ks = kw;
+  const int tiles = (int)mn_cdiv(max_len, KT), tps = (int)mn_cdiv(tiles, ks);
   float* pml = pacc ? pacc + (size_t)ks * M * H * r : nullptr;
   hipStream_t st = mn_stream(stream);
   if (variant == MN_LATENT_ATTN_MFMA) {
     const int nbw = (int)mn_cdiv(r, 64);
     // as many runs as rows: one row each, or longer ones beside empty ones, whose workgroups go round again (workgroups for the rows a run does not have
     // still wait for their LDS: 3 of 4 in a decode step)
-    const dim3 grid((unsigned)n_blk, (unsigned)mn_cdiv((n_blk == M ? 1 : RB) * H, 16), (unsigned)ks);
+    const dim3 grid((unsigned)n_blk, (unsigned)gy, (unsigned)ks);
     MN_CHECK_ARG(mn_cdiv(RB * H, 16) <= 65535 && ks <= 64, "mn_latent_attn: too many heads or key splits");
 #define MN_LM(N_, F_, V_)                                                                                                           \
   hipLaunchKernelGGL((latent_attn_mfma_kernel<N_, F_, V_>), grid, dim3(256), 0, st, qabs, arena, row_seq, row_len, blk_tab, H, r, t_max, tps, lat, pacc, \
                      pml, ks, M)
-    if (latent_by_wave(r, max_len, ks) && ((uintptr_t)qabs & 15) == 0 && ((uintptr_t)arena & 15) == 0 && ((uintptr_t)lat & 15) == 0 && ((uintptr_t)pacc & 15) == 0) {
+    if (kw) {
 #define MN_LW(N_)                                                                                                                              \
   hipLaunchKernelGGL((latent_attn_wave_kernel<N_>), grid, dim3(256), 0, st, qabs, arena, row_seq, row_len, blk_tab, H, t_max, lat, pacc, pml, ks, M)
       if (r == 128) MN_LW(8); else if (r == 256) MN_LW(16); else if (r == 384) MN_LW(24); else MN_LW(32);

@@ -412,18 +412,21 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(GemmF32 a) {
 
 // Many tiles: 64 x 64 outputs a workgroup, 32 x 32 a wave, on the bf16 matrix cores.  An fp32 value is the sum of three bf16 values, its upper, middle and lower 8 bits of mantissa cut off one
 // after the other, and a weight is one already: three products a pair, each exact in fp32, take a fifth of the fp32 cores' time for the one.  The rows are split once a workgroup, on their way to
-// LDS (8 instructions a value; what is left of an infinity is zero, of a NaN a NaN); 64 values of K at a time, rows 144 bytes apart (the 16-byte reads of 16 rows meet all 64 banks), two
-// stages of loads in flight in registers.  The upper products and the others have accumulators of their own.  An infinite weight would meet a part that is zero: a workgroup that saw one
-// takes its outputs over again, value by value.  NB: buffers of LDS: two (two workgroups a CU), or one and a second barrier (three a CU) where the tiles are more than two a CU: us, two / one: 900 rows of
+// LDS (7 instructions a value); 64 values of K at a time, rows 144 bytes apart (the 16-byte reads of 16 rows meet all 64 banks), two stages of loads in flight in registers.  The upper products
+// and the others have accumulators of their own.  The middle and lower parts enter times 2^24, exact down to the smallest value (as they are, rows below 2^-110 lost their last bits: 2.5e-7 at
+// 2^-112, 7e-5 at 2^-120).  Values from 2^112 on overflow there and of an infinite one nothing but NaN is left: an output whose lower parts have no finite sum, while the upper ones do not say
+// NaN, is taken over again value by value, and so are all of a workgroup that saw an infinite weight, which would meet a part that is zero.
+// NB: buffers of LDS: two (two workgroups a CU), or one and a second barrier (three a CU) where the tiles are more than two a CU: us, two / one: 900 rows of
 // 16 x 512 x 128 24.4 / 21.3, 2048 x 4096 x 1024 100 / 94, 8 x 2129 x 1676 x 302 241 / 216; 900 of 1024 x 1024 (240 tiles) 19.7 / 20.6.
-// us, fp32 matrix cores (values a lane stored one by one) -> here: 900 rows of 16 x 512 x 128 32 -> 21, of 16 x 128 x 512 28 -> 17, 1900 rows 53 -> 35 and 49 -> 31, 2048 x 4096 x 1024 168 -> 94 (183
+// us, fp32 matrix cores (values a lane stored one by one) -> here: 900 rows of 16 x 512 x 128 32 -> 21.5, of 16 x 128 x 512 28 -> 17, 1900 rows 53 -> 35 and 49 -> 30, 2048 x 4096 x 1024 168 -> 87 (197
 // TFLOP/s), 200 rows of 16 x 128 x 512 17.5 -> 11.2.  What bounds short K is a workgroup's round trips.  Error against 64 bits, rows of uneven magnitudes: 1.47e-7 -> 0.77e-7 at K = 128, 2.9e-7 -> 1.5e-7 at 512, 5.7e-7 ->
-// 2.9e-7 at 2048.  (Parts below 2^-126 may count as zero: rows of values below 1e-31 lose their last bits.)
+// 2.9e-7 at 2048.
 template <bool V4, int NB>
 __global__ __launch_bounds__(256, NB == 1 ? 3 : 2) void gemm_f32_tile_kernel(GemmF32 a) {
   typedef short bf16x8 __attribute__((ext_vector_type(8)));
   typedef unsigned short us2 __attribute__((ext_vector_type(2)));
   constexpr int LD = 72, PLANE = 64 * LD;
+  constexpr float LOW = 0x1p24f;
   __shared__ __attribute__((aligned(16))) uint16_t lds[NB][4 * PLANE];      // [upper | middle | lower | weights][64][LD]
   const int z = blockIdx.z, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, q = lane >> 4;
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64, wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
@@ -464,7 +467,7 @@ __global__ __launch_bounds__(256, NB == 1 ? 3 : 2) void gemm_f32_tile_kernel(Gem
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const float v = c < left ? fa[h][t][c] : 0.f;         // what is past K becomes zero here: a branch around the load is a wait
-        const float u = __uint_as_float(__float_as_uint(v) & 0xffff0000u), d = v == u ? 0.f : v - u;
+        const float u = __uint_as_float(__float_as_uint(v) & 0xffff0000u), d = (v - u) * LOW;
         const float m = __uint_as_float(__float_as_uint(d) & 0xffff0000u);
         part[0][c] = __float_as_uint(v);
         part[1][c] = __float_as_uint(d);
@@ -527,16 +530,24 @@ __global__ __launch_bounds__(256, NB == 1 ? 3 : 2) void gemm_f32_tile_kernel(Gem
 #pragma unroll
     for (int j = 0; j < 2; ++j) {                             // a lane's four outputs are neighbours in a row
       const int m = m0 + wm + 16 * i + r, n = n0 + wn + 16 * j + 4 * q;
-      f32x4 v = acc[0][i][j] + acc[1][i][j];
-      if (odd) {
+      const f32x4 up = acc[1][i][j], low = acc[0][i][j];
+      f32x4 v = up + low * (1.0f / LOW);
+      const f32x4 lost = low * 0.f;                           // zero, or NaN
+      if (odd || (lost[0] + lost[1]) + (lost[2] + lost[3]) != 0.f) {
         const float* x = A + (int64_t)min(m, a.M - 1) * a.lda;
 #pragma unroll 1
         for (int e = 0; e < 4; ++e) {
+          const float ue = e == 0 ? up[0] : e == 1 ? up[1] : e == 2 ? up[2] : up[3], le = e == 0 ? lost[0] : e == 1 ? lost[1] : e == 2 ? lost[2] : lost[3];
+          if (!odd && (le == 0.f || ue != ue)) continue;
           const bf16_t* w = W + (int64_t)min(n + e, a.N - 1) * a.ldw;
-          float t = 0.f;
+          float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-          for (int k = 0; k < a.K; ++k) t = fmaf(x[k], bf16_to_f32(w[k]), t);
-          v = f32x4{e == 0 ? t : v[0], e == 1 ? t : v[1], e == 2 ? t : v[2], e == 3 ? t : v[3]};
+          for (int k = 0; k < a.K; k += 8)
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+              if (k + c < a.K) t[c] = fmaf(x[k + c], bf16_to_f32(w[k + c]), t[c]);
+          const float r = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+          v = f32x4{e == 0 ? r : v[0], e == 1 ? r : v[1], e == 2 ? r : v[2], e == 3 ? r : v[3]};
         }
       }
       if (m < a.M) f32_store4(a, z, m, n, v);
@@ -1249,7 +1260,7 @@ extern "C" int mn_gemm_f32_batched(const float* A, int64_t lda, int64_t a_bs, co
   const int64_t tiles = mn_cdiv(M, 64) * mn_cdiv(N, 64) * batch;
   // up to 64 rows always take the kernel that keeps its roundings (they are decode rows: error against 64 bits 0.2 .. 0.6e-7 of the summed
   // magnitudes).  More rows, from 128 tiles on (us, few / tiles: 200 rows of 16 x 128 x 512, 128 tiles, 17.5 / 11.2; 128 rows, 64 tiles, 10.3 / as many K-steps as those 11.2;
-  // 2048 rows x 4096 x 1024 354 / 94)
+  // 2048 rows x 4096 x 1024 354 / 87)
   if (M <= 64 || 2 * tiles < mn_num_cus()) {
     const dim3 grid((unsigned)mn_cdiv(N, 16), (unsigned)mn_cdiv(M, 32), (unsigned)batch);
     if (v4) hipLaunchKernelGGL(gemm_f32_few_kernel<true>, grid, dim3(256), 0, st, a);

@@ -40,14 +40,21 @@ __device__ __forceinline__ int sequence_start(const int32_t* __restrict__ row_ba
   return -1;
 }
 
-// The step's sequences at once, where its rows are at most 2048: first[j] = sequence j's first row, first[count] = M; the count comes back (256 threads)
-__device__ __forceinline__ int sequence_starts(const int32_t* __restrict__ row_back, int M, uint64_t (&mask)[32], uint16_t (&first)[2049]) {
+// The step's sequences at once, where its rows are at most 2048: first[j] = sequence j's first row, first[count] = M; the count comes back (256 threads).  far (or null): does a wave see a
+// sequence of `rows` rows?
+__device__ __forceinline__ int sequence_starts(const int32_t* __restrict__ row_back, int M, uint64_t (&mask)[32], uint16_t (&first)[2049], int rows = 0, int* far = nullptr) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  bool there = false;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    const int m = 256 * k + tid;
-    const uint64_t b = __ballot(m < M && row_back[m < M ? m : 0] == 0);
+    const int m = 256 * k + tid, back = m < M ? row_back[m] : -1;
+    const uint64_t b = __ballot(back == 0);
+    there |= back + 1 >= rows;
     if (lane == 0) mask[4 * k + wave] = b;
+  }
+  if (far) {
+    const bool any = __ballot(there) != 0;
+    if (lane == 0) far[wave] = any;
   }
   __syncthreads();
   const int own = lane < 32 ? __popcll(mask[lane & 31]) : 0;

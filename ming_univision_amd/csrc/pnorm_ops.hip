@@ -574,31 +574,29 @@ __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
 // Heads of 65 .. 128 state rows with a table: 32 lanes a column, 8 columns a workgroup, where the longest sequence's chain of steps is the time, and 16 lanes a column where all sequences
 // together fill the chip: a step of 32 lanes is 33 instructions, one of 16 50 for twice the columns.  us, 16 lanes alone -> here, heads of 128 x 128: 1900 rows of 8 heads 272 -> 217, of 16 277 -> 230, 300
 // of 2 47 -> 38, 470 .. 93 rows of 5 sequences, 8 heads 78 -> 67; of 16 heads 87 and 85, two of 500 81 and 79 (32 lanes: 90 and 82), 16 of 64 37 (32 lanes 41).  The rule is an estimate of both: a
-// step of a chain takes 110 / 138 ns, a step of a workgroup on a CU that is full of them 64 / 118 for half the workgroups; 15 % in favour of 16 lanes, whose rows are staged for twice the columns.
-// Looking for the longest costs sequences of two rows 1 % (256 of them, 8 heads 112.8 -> 114).
+// step of a chain takes 110 / 138 ns, a step of a workgroup on a CU that is full of them 64 / 118 for half the workgroups; 15 % in favour of 16 lanes, whose rows are staged for twice the columns
+// (delta_long_rows).  A sequence's sums are in another order with 32 lanes than with 16: its last bits depend on the sequences beside it.
 // Grid (2 H ceil(vdim / 16), S): of 16 lanes, the second half of x takes every other sequence.
 template <bool VEC>
-__global__ __launch_bounds__(256) void delta_rows_lanes_kernel(DeltaArgs a) {
+__global__ __launch_bounds__(256) void delta_rows_lanes_kernel(DeltaArgs a, int long_rows) {
   extern __shared__ float lds[];
   __shared__ uint64_t mask[32];
   __shared__ uint16_t first[2049];
-  __shared__ int longest;
-  if (threadIdx.x == 0) longest = 0;
-  const int count = sequence_starts(a.row_back, a.M, mask, first);
-  int n = 0;
-  for (int i = threadIdx.x; i < count; i += 256) n = max(n, (int)first[i + 1] - (int)first[i]);
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) n = max(n, __shfl_xor(n, o));
-  if (n && (threadIdx.x & 63) == 0) atomicMax(&longest, n);
-  __syncthreads();
+  __shared__ int far[4];
+  const int count = sequence_starts(a.row_back, a.M, mask, first, long_rows, far);
   const int x16 = a.H * ((a.vdim + 15) / 16), x32 = a.H * ((a.vdim + 7) / 8);
-  const float chain = (float)longest, all = (float)a.M * x32 / 256.0f;
-  if (1.15f * fmaxf(110.0f * chain, 64.0f * all) < fmaxf(138.0f * chain, 59.0f * all)) {
+  if (__builtin_amdgcn_readfirstlane(far[0] | far[1] | far[2] | far[3])) {
     if ((int)blockIdx.x < x32) delta_walk<4, 32, 32, true, VEC>(a, blockIdx.x, blockIdx.y, gridDim.y, lds, first, mask, count);
   } else {
     const int late = (int)blockIdx.x >= x16;
     delta_walk<8, 16, 32, true, VEC>(a, blockIdx.x - late * x16, 2 * blockIdx.y + late, 2 * gridDim.y, lds, first, mask, count);
   }
+}
+
+// rows of a sequence from which a step of M rows takes 32 lanes a column: 1.15 max(110 rows, 64 all) < max(138 rows, 59 all), all = the steps of its workgroups a CU
+static int delta_long_rows(int M, int H, int vdim) {
+  const double all = (double)M * H * (double)mn_cdiv(vdim, 8) / mn_num_cus(), rows = 1.15 * 64 / 138 * all;
+  return rows < 4096 ? (int)rows + 1 : 4096;             // (M is at most 2048)
 }
 
 // Decode rows (every row alone in its sequence): grid (M, H, ceil(vdim / 32)); a workgroup owns 32 value columns of one head's
@@ -798,8 +796,9 @@ extern "C" int mn_gated_delta_rows(const float* qkv, int64_t ld, const float* bd
       const int64_t gx = 2 * (int64_t)H * mn_cdiv(vdim, 16);
       const dim3 lanes((unsigned)gx, slots(gx));
       const size_t bytes = ((size_t)32 * 256 + 2 * 32 * 16 + 2 * 32) * sizeof(float);
-      if (dim == 128 && (ld % 4) == 0 && ((uintptr_t)qkv & 15) == 0) hipLaunchKernelGGL(delta_rows_lanes_kernel<true>, lanes, dim3(256), bytes, st, a);
-      else hipLaunchKernelGGL(delta_rows_lanes_kernel<false>, lanes, dim3(256), bytes, st, a);
+      const int long_rows = delta_long_rows(M, H, vdim);
+      if (dim == 128 && (ld % 4) == 0 && ((uintptr_t)qkv & 15) == 0) hipLaunchKernelGGL(delta_rows_lanes_kernel<true>, lanes, dim3(256), bytes, st, a, long_rows);
+      else hipLaunchKernelGGL(delta_rows_lanes_kernel<false>, lanes, dim3(256), bytes, st, a, long_rows);
     }
 #undef MN_DF
 #undef MN_DFT

@@ -11,18 +11,34 @@
 // all of them see whole takes no mask arithmetic.  Key splits write the partial layout of the merge kernel, run by run.
 
 // A launch's workgroups: first the groups of every (head chunk, key split), then `alone` that take one run after the other.
-// Workgroup x of the launch: long walks (late rows) first.  Where all are on the chip at once (two a CU), the second 256 go the other way round, so that a CU holds a long and a short one.
-// Where they follow each other the order is by length alone, the head chunks and splits of a group side by side: what is taken last is short, and no CU is left with a long walk at the
-// end.  us, every other 256 the other way round / by length (16 heads of 128 over four key heads): 8000 tokens 2968 / 2360 (111 TFLOP/s), 2600 446 / 315, 1500 in two splits
-// 164 / 137, 1000 in three 104 / 89, 16 sequences of 512 328 / 245, window 1024 of 3000 280 / 247; keys of 320 with the values inside, 5 prompts of 93 .. 470, 91 / 85.
+// Workgroup x of the launch.  Where all are on the chip at once (two a CU), group by group of a (head chunk, split), every other CU-full the other way round, so that a CU holds a long walk and a
+// short one.  Where they follow each other: the table's last groups (a sequence's long walks) first, the head chunks and splits of a group side by side, so that what is taken last is short; of the
+// workgroups that start together the second half the other way round.
+// Sequences whose workgroups are a multiple of 16 would meet on the CUs with their long walks (the launch's count is then one, which spares the others the look at the table, 1 us): where all are as
+// long as the last one and a whole number of groups, as 64 runs of the table say, groups go by length, a group of every sequence after the other.
+// us, every CU-full the other way round / the table's order backwards / as here: heads of 128, 16 over four, 8000 tokens 2984 / 2360 / 2340 (112 TFLOP/s), 4096 950 / 683 / 630, 2600 453 / 316 / 294,
+// 1030 in two splits 115 / 81 / 70, window 1024 of 3000 280 / 246 / 249, 16 sequences of 512 326 / 246 / 195, 8 of 512 118 / 148 / 104, 16 of 256 72 / 92 / 69; over 16 of 64, 8 of 512 71 / 84 / 66; keys of
+// 320 with the values inside, 5 prompts of 93 .. 470 in two splits 91 / 68 / 70, 10 of 384 146 / 153 / 103, 16 heads, 16 of 128 58 / 74 / 54.  Over 230 batches of equal prompts of 24 .. 1000 tokens 1 / 0.98 /
+// 0.91 of the time on average, unequal ones 0.94.  What is left slower than the first form: many sequences of some 64 rows whose workgroups are no multiple of 16 (93 of 64, 8 heads of 128, 33 / 38 / 37).
+constexpr int ROWS_CUS = 256;          // (the card's; as another argument it costs every kernel here scalar registers, which they spill: 16 heads of 64, 85 sequences of 48, 190 -> 205 us)
 struct RowsItem { int group, gy, sp; };
-__device__ __forceinline__ RowsItem rows_item(int x, int groups, int gys, int items) {
-  if (items > 512) {
-    const int yzs = items / groups, yz = x % yzs;
-    return {groups - 1 - x / yzs, yz % gys, yz / gys};
+__device__ __forceinline__ RowsItem rows_item(const AttnTArgs& a, int x, int groups, int nbw, int n_blk, int gys, int items) {
+  if (items <= 2 * ROWS_CUS) {
+    const int g = x % groups, first = x - g;                             // of this (head chunk, split): one direction for all of its groups
+    return {((first / ROWS_CUS) & 1) ? g : groups - 1 - g, x / groups % gys, x / groups / gys};
   }
-  const int g = x % groups, first = x - g;                               // of this (head chunk, split): one direction for all of its groups
-  return {((first >> 8) & 1) ? g : groups - 1 - g, x / groups % gys, x / groups / gys};
+  if (x >= ROWS_CUS && x < 2 * ROWS_CUS) x = 3 * ROWS_CUS - 1 - x;
+  const int yzs = items / groups, yz = x % yzs, r = x / yzs;
+  int g = groups - 1 - r;
+  if ((items & 15) == 0) {
+    const int q = (groups + 63) >> 6, b = min(min((((int)threadIdx.x & 63) + 1) * q, groups) * nbw, n_blk) - 1;
+    const int first = a.row_slot[a.blk_tab[0]], at = a.row_slot[a.blk_tab[2 * b]] - first, len = __builtin_amdgcn_readlane(at, 63) / a.rows_per_blk + 1;      // len: runs of the last sequence
+    if (len * a.rows_per_blk >= 64 && len < n_blk && len % nbw == 0 && __ballot(at != a.rows_per_blk * (b % len)) == 0) {
+      const int seqs = n_blk / len, per = len / nbw;                     // (the last run is where it lies in all of them: n_blk = seqs len)
+      g = r % seqs * per + per - 1 - r / seqs;
+    }
+  }
+  return {g, yz % gys, yz / gys};
 }
 
 // the workgroup's runs: first row, rows, cache sequence, first position
@@ -349,7 +365,7 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(AttnTArgs a, int n_bl
                [&](int b, int gy, int sp) { attn_run<NBD, NBV, KF, VEC, false>(a, b, gy, sp, lds, met); });
     return;
   }
-  const RowsItem it = rows_item(blockIdx.x, groups, gys, in_groups);
+  const RowsItem it = rows_item(a, blockIdx.x, groups, nbw, n_blk, gys, in_groups);
   const int gy = it.gy, sp = it.sp;
   const int g = gy / chunks, h0 = g * rep + (gy % chunks) * a.hpc;
   const int Rc = min(a.hpc, g * rep + rep - h0);
@@ -548,7 +564,7 @@ __global__ __launch_bounds__(256, 2) void attn_latent_rows_kernel(AttnTArgs a, i
                [&](int b, int gy, int sp) { attn_run<NB, NB, 1, VEC, true>(a, b, gy, sp, K, met); });
     return;
   }
-  const RowsItem it = rows_item(blockIdx.x, groups, gys, in_groups);
+  const RowsItem it = rows_item(a, blockIdx.x, groups, nbw, n_blk, gys, in_groups);
   const int gy = it.gy, sp = it.sp, h0 = gy * a.hpc;
   const int Rc = min(a.hpc, rep - h0);
   const int b0 = it.group * nbw, nb = min(nbw, n_blk - b0);

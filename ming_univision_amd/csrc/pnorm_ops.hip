@@ -573,9 +573,11 @@ __global__ __launch_bounds__(256) void delta_rows_fast_kernel(DeltaArgs a) {
 
 // Heads of 65 .. 128 state rows with a table: 32 lanes a column, 8 columns a workgroup, where the longest sequence's chain of steps is the time, and 16 lanes a column where all sequences
 // together fill the chip: a step of 32 lanes is 33 instructions, one of 16 50 for twice the columns.  us, 16 lanes alone -> here, heads of 128 x 128: 1900 rows of 8 heads 272 -> 217, of 16 277 -> 230, 300
-// of 2 47 -> 38, 470 .. 93 rows of 5 sequences, 8 heads 78 -> 67; of 16 heads 87 and 85, two of 500 81 and 79 (32 lanes: 90 and 82), 16 of 64 37 (32 lanes 41).  The rule is an estimate of both: a
-// step of a chain takes 110 / 138 ns, a step of a workgroup on a CU that is full of them 64 / 118 for half the workgroups; 15 % in favour of 16 lanes, whose rows are staged for twice the columns
-// (delta_long_rows).  A sequence's sums are in another order with 32 lanes than with 16: its last bits depend on the sequences beside it.
+// of 2 47 -> 38, 470 .. 93 rows of 5 sequences, 8 heads 78 -> 67; of 16 heads 87 and 85, two of 500 81 and 79 (32 lanes: 90 and 82), 16 of 64 37 (32 lanes 41).  The rule
+// (delta_long_rows): one sequence's rows against the step's rows times the workgroups a CU that one sequence makes.  0.62 where rows are staged 16 bytes at a time, 0.8 elsewhere, as staging is then as
+// much as the steps and 32 lanes do it twice as often, and 48 rows for such a workgroup a CU.  us, 16 lanes / 32, where 0.53 for all was too low: heads of 128 x 128, 4 of 7 sequences of 142 rows (0.57) 27.7 /
+// 29.1, 16 of 4 of 2 .. 28 11.0 / 13.1; 100 x 128, 4 of 27 of 2 .. 372 75.7 / 90.2.  With more sequences than S a workgroup takes several, twice as many of them with 32 lanes: not where
+// that makes its rows a ninth more (2 heads of 19 sequences of 4 .. 391 rows 66.5 / 79.4).  A sequence's sums are in another order with 32 lanes than with 16: its last bits depend on the sequences beside it.
 // Grid (2 H ceil(vdim / 16), S): of 16 lanes, the second half of x takes every other sequence.
 template <bool VEC>
 __global__ __launch_bounds__(256) void delta_rows_lanes_kernel(DeltaArgs a, int long_rows) {
@@ -584,8 +586,26 @@ __global__ __launch_bounds__(256) void delta_rows_lanes_kernel(DeltaArgs a, int 
   __shared__ uint16_t first[2049];
   __shared__ int far[4];
   const int count = sequence_starts(a.row_back, a.M, mask, first, long_rows, far);
-  const int x16 = a.H * ((a.vdim + 15) / 16), x32 = a.H * ((a.vdim + 7) / 8);
-  if (__builtin_amdgcn_readfirstlane(far[0] | far[1] | far[2] | far[3])) {
+  const int x16 = a.H * ((a.vdim + 15) / 16), x32 = a.H * ((a.vdim + 7) / 8), S = gridDim.y;
+  bool wide = __builtin_amdgcn_readfirstlane(far[0] | far[1] | far[2] | far[3]);
+  if (wide && count > S) {                              // (every wave for itself)
+    int most = 0;                                       // rows that one workgroup takes, of 32 lanes in the lower half
+    for (int y = threadIdx.x & 63; y < 2 * S; y += 64) {
+      int n = 0, n32 = 0;
+      for (int q = y; q < count; q += 2 * S) n += first[q + 1] - first[q];
+      if (y < S)
+        for (int q = y; q < count; q += S) n32 += first[q + 1] - first[q];
+      most = max(most >> 16, n) << 16 | max(most & 0xffff, n32);
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_xor(most, o);
+      most = max(most >> 16, t >> 16) << 16 | max(most & 0xffff, t & 0xffff);
+    }
+    most = __builtin_amdgcn_readfirstlane(most);
+    wide = 9 * (most & 0xffff) <= 10 * (most >> 16);
+  }
+  if (wide) {
     if ((int)blockIdx.x < x32) delta_walk<4, 32, 32, true, VEC>(a, blockIdx.x, blockIdx.y, gridDim.y, lds, first, mask, count);
   } else {
     const int late = (int)blockIdx.x >= x16;
@@ -593,9 +613,9 @@ __global__ __launch_bounds__(256) void delta_rows_lanes_kernel(DeltaArgs a, int 
   }
 }
 
-// rows of a sequence from which a step of M rows takes 32 lanes a column: 1.15 max(110 rows, 64 all) < max(138 rows, 59 all), all = the steps of its workgroups a CU
-static int delta_long_rows(int M, int H, int vdim) {
-  const double all = (double)M * H * (double)mn_cdiv(vdim, 8) / mn_num_cus(), rows = 1.15 * 64 / 138 * all;
+// rows of a sequence from which a step of M rows takes 32 lanes a column; vec: rows are staged 16 bytes at a time
+static int delta_long_rows(int M, int H, int vdim, bool vec) {
+  const double wgs = (double)H * (double)mn_cdiv(vdim, 8) / mn_num_cus(), rows = wgs * fmax((vec ? 0.62 : 0.8) * M, 48);
   return rows < 4096 ? (int)rows + 1 : 4096;             // (M is at most 2048)
 }
 
@@ -796,8 +816,9 @@ extern "C" int mn_gated_delta_rows(const float* qkv, int64_t ld, const float* bd
       const int64_t gx = 2 * (int64_t)H * mn_cdiv(vdim, 16);
       const dim3 lanes((unsigned)gx, slots(gx));
       const size_t bytes = ((size_t)32 * 256 + 2 * 32 * 16 + 2 * 32) * sizeof(float);
-      const int long_rows = delta_long_rows(M, H, vdim);
-      if (dim == 128 && (ld % 4) == 0 && ((uintptr_t)qkv & 15) == 0) hipLaunchKernelGGL(delta_rows_lanes_kernel<true>, lanes, dim3(256), bytes, st, a, long_rows);
+      const bool vec = dim == 128 && (ld % 4) == 0 && ((uintptr_t)qkv & 15) == 0;
+      const int long_rows = delta_long_rows(M, H, vdim, vec);
+      if (vec) hipLaunchKernelGGL(delta_rows_lanes_kernel<true>, lanes, dim3(256), bytes, st, a, long_rows);
       else hipLaunchKernelGGL(delta_rows_lanes_kernel<false>, lanes, dim3(256), bytes, st, a, long_rows);
     }
 #undef MN_DF

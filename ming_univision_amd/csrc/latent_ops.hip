@@ -1297,12 +1297,17 @@ extern "C" int mn_latent_attn_splits(int n_blk, int max_len, int r) {
 
 // Whole tiles a wave (0: not that form): where a wave has two of them or more in one round of its workgroups, which is then all the splits there are, of the `ks` that the caller has scratch for;
 // wgs: workgroups a split.  With fewer tiles the form whose waves share one is the faster one (us, shared / whole: 64 rows over 300 of 512 27.3 / 25.9 .. 28, 8 rows over 2049
-// 27.8 / 29.5, one 22.5 / 24.8, 64 over 64 11.6 / 14.1, 40 rows over 1111 of 256 22.4 / 27.9).
-static inline int latent_wave_splits(int r, int max_len, int64_t wgs, int ks) {
+// 27.8 / 29.5, one 22.5 / 24.8, 64 over 64 11.6 / 14.1, 40 rows over 1111 of 256 22.4 / 27.9).  A prompt's rows see half of max_len on average: with more workgroups than one round (above 256 values: three) the
+// short walks are the time, and from 160 (320) keys on whole tiles are worth it (16 heads, of 512: 4 prompts of 128 24.0 / 28.6, 5 of 200 68 / 75, 15 of 200 160 / 203, 6 of 300 143 / 153, 4 of 512 272 / 226, one of
+// 300 48 / 33; 32 heads, 10 of 200 204 / 264; of 256, 16 heads: 16 of 128 55 / 59, 5 of 11 .. 140 23.8 / 18.4, 8 of 256 86 / 77).
+static inline int latent_wave_splits(int r, int max_len, int64_t wgs, int ks, bool runs) {
   if (r != 128 && r != 256 && r != 384 && r != 512) return 0;
-  int64_t kw = (r <= 256 ? 2 : 1) * mn_num_cus() / wgs;
+  const int cus = mn_num_cus();
+  int64_t kw = (r <= 256 ? 2 : 1) * cus / wgs;
   if (kw < 1) kw = 1;
   if (kw > ks) kw = ks;
+  if (runs && max_len < 160 && (r <= 256 ? wgs >= 2 * cus : wgs > cus)) return 0;
+  if (runs && max_len < 320 && r > 256 && wgs > 3 * cus) return 0;
   return max_len >= 128 * kw ? (int)kw : 0;
 }
 
@@ -1323,7 +1328,7 @@ extern "C" int mn_latent_attn_ex(const float* qabs, const float* arena, const in
   const int gy = (int)mn_cdiv((n_blk == M ? 1 : RB) * (int64_t)H, 16);
   float* pacc = reinterpret_cast<float*>(ws);
   const bool aligned = (((uintptr_t)qabs | (uintptr_t)arena | (uintptr_t)lat | (uintptr_t)pacc) & 15) == 0;
-  const int kw = variant == MN_LATENT_ATTN_MFMA && aligned ? latent_wave_splits(r, max_len, (int64_t)n_blk * gy, ks) : 0;
+  const int kw = variant == MN_LATENT_ATTN_MFMA && aligned ? latent_wave_splits(r, max_len, (int64_t)n_blk * gy, ks, n_blk < M) : 0;
   if (kw) ks = kw;
   const int tiles = (int)mn_cdiv(max_len, KT), tps = (int)mn_cdiv(tiles, ks);
   float* pml = pacc ? pacc + (size_t)ks * M * H * r : nullptr;

@@ -49,3 +49,24 @@ def test_fewer_splits_than_the_scratch_holds():
         k = arena[seq[m], :lens[m]].double()
         want = torch.softmax(q[m].double() @ k.T, -1) @ k
         assert float((out[m] - want).norm() / want.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("r,n,length", [(512, 5, 160), (512, 4, 320), (384, 9, 96), (256, 5, 128), (256, 4, 160)])
+def test_prompts_on_both_sides_of_the_line(r, n, length):
+    """Prompts of n sequences, 16 heads: more workgroups than rounds of them are worth whole tiles a wave, and on the other side of that line."""
+    from ming_univision_amd._lib import check, current_stream, lib, ptr
+    g = torch.Generator().manual_seed(r + n)
+    M, H = n * length, 16
+    q, arena = (torch.randn(M, H, r, generator=g) * 2 * r ** -0.5).cuda(), torch.randn(n, length, r, generator=g).cuda()
+    seq, lens = torch.arange(M, dtype=torch.int32, device="cuda") // length, torch.arange(M, dtype=torch.int32, device="cuda") % length + 1
+    blk = torch.stack([torch.arange(0, M, 4, dtype=torch.int32), torch.full((M // 4,), 4, dtype=torch.int32)], 1).cuda()
+    ks = lib().mn_latent_attn_splits(M // 4 * 4, length, r)
+    ws, out = torch.empty(max(16, lib().mn_latent_attn_workspace_bytes(M, H, r, ks)), dtype=torch.uint8, device="cuda"), torch.empty(M, H, r, device="cuda")
+    check(lib().mn_latent_attn(ptr(q), ptr(arena), ptr(seq), ptr(lens), ptr(blk), M // 4, M, H, r, length, length, ks, ptr(out), ptr(ws), ws.numel(), current_stream()), "latent")
+    for i in range(n):
+        rows = slice(i * length, (i + 1) * length)
+        k = arena[i].double()
+        see = torch.arange(length, device="cuda")[None] <= torch.arange(length, device="cuda")[:, None]
+        s = (q[rows].double() @ k.T).masked_fill(~see[:, None], -float("inf"))
+        want = torch.softmax(s, -1) @ k
+        assert float((out[rows] - want).norm() / want.norm()) < 1e-6

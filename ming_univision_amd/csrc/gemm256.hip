@@ -579,12 +579,15 @@ static int tile_form(int M, int N, int Kc, int nz, bool hilo, int epi, double* u
 }
 
 // Column tiles that the small tiles' order takes together: an XCD's eighth of the tiles, row by row of a band, is about a square of them, where column by column it is all rows by a few columns.
-// For plain rows and weights that are both more than most of an XCD's L2 (4 MB): workgroups that are not in step then find less of either.  us, column by column / in bands, weights from HBM: 900 x
-// 2048 x 8192 61 / 50, x 2048 19.0 / 16.7, 1409 x 1024 x 4096 27.5 / 26.6, 2048 x 1024 x 4096 32.7 / 31.3, 2048 x 4096 x 1024 24.7 / 23.2, 4112 x 1024 x 2752 46.4 / 41.7, 3000 x 512 x 8192 67 / 45; with rows or weights
-// below that 600 x 2048 x 2048 13.4 / 14.4, 1300 x 3072 x 1024 16.6 / 17.3, 4112 x 1024 x 1024 19.6 / 20.2; with weights over three times the rows, which more XCDs then read, 512 x 4096 x 4096 32.3 / 33.6,
+// For plain rows and weights that are both more than most of an XCD's L2 (4 MB): workgroups that are not in step then find less of either.  Where rows are one and a half times the weights (us, column by
+// column / in bands, weights from HBM: 2364 x 512 x 8192 61 / 42, 2620 x 512 x 4096 32.8 / 24.3, 4112 x 1024 x 2752 46.4 / 41.7), or 64 x 64 tiles fill two a CU by 0.7 and more (900 x 2048 x 8192 61 / 50, x 2048
+// 19.0 / 16.7, 907 x 1024 units x 4096 31.3 / 26.4, 1409 x 1024 x 4096 27.5 / 26.6).  Elsewhere as often the other way (1064 x 1024 x 3264 18.0 / 21.2, 884 x 768 units x 3072 17.0 / 19.8, 1034 x 2048 x 1920 20.0 /
+// 22.3; 1071 x 2752 x 2752 37.3 / 30.2); with rows or weights below 3 MB 600 x 2048 x 2048 13.4 / 14.4, 4112 x 1024 x 1024 19.6 / 20.2; with weights over three times the rows, which more XCDs then read,
 // 600 x 2048 x 8192 43.4 / 45.0; hi/lo rows 1025 x 3072 x 1024 21.1 / 21.8, 1058 x 2048 x 2048 32.1 / 31.4.
 static int order_band(int tiles_m, int tiles_n, int bm, int bn, int64_t a_bytes, int64_t w_bytes) {
   if (a_bytes <= (int64_t)3 << 20 || w_bytes <= (int64_t)3 << 20 || w_bytes > 3 * a_bytes) return 1;
+  const int64_t tiles = (int64_t)tiles_m * tiles_n, two = 2 * (int64_t)mn_num_cus();
+  if (2 * a_bytes < 3 * w_bytes && !(bm == 64 && bn == 64 && 10 * tiles > 7 * two && tiles <= two)) return 1;
   const double q = tiles_m * (double)tiles_n / 8;
   int best = 1;
   double tb = 1e30;
@@ -600,9 +603,15 @@ template <int EPI, int BM, int BN, int WM, int WN, int S, bool HILO, bool TWO = 
 static void tile_go(const G256& a, int nz, hipStream_t st) {
   constexpr int cols = epi_paired(EPI) ? BN / 2 : BN;
   const int tm = (int)mn_cdiv(a.M, BM), tn = (int)mn_cdiv(a.N, cols);
-  G256 p = a;
-  p.group_m = HILO ? 1 : order_band(tm, tn, BM, BN, (int64_t)p.M * p.K * 2, (int64_t)p.N * (BN / cols) * p.K * 2);
   const dim3 grid((unsigned)((int64_t)tm * tn), nz);
+  G256 p = a;
+  if constexpr (!HILO && GROUP == 0) {
+    p.group_m = order_band(tm, tn, BM, BN, (int64_t)p.M * p.K * 2, (int64_t)p.N * (BN / cols) * p.K * 2);
+    if (p.group_m > 1) {
+      hipLaunchKernelGGL((gemm_tile_kernel<EPI, HILO, BM, BN, WM, WN, S, TWO, 4>), grid, dim3(WM * WN * 64), 0, st, p);
+      return;
+    }
+  }
   hipLaunchKernelGGL((gemm_tile_kernel<EPI, HILO, BM, BN, WM, WN, S, TWO, GROUP>), grid, dim3(WM * WN * 64), 0, st, p);
 }
 

@@ -30,7 +30,7 @@ __device__ __forceinline__ void wait_tiles(int rem) {
 // GROUP 1, 2: the products of groups of rows with weights of their own (MoE experts), row tiles of BM from a device-built list.  2 and 3 (one dense product): the weights are read past
 // the caches, where all rows, or most groups, are one row tile: nobody reads them again, and lines that are let go at once stream faster (66 experts' 2816 x 2048 / 2048 x 1408 of 100
 // rows in tiles of 32 x 128, 6 picks a row and two for all: 146 -> 140 us / 74 -> 70, 70 rows 146 -> 135 / 73 -> 67, 5.6 TB/s; 240 rows, where a third of the groups are two tiles, 162 -> 165 /
-// 87 -> 89).
+// 87 -> 89).  4: one dense product, tiles in bands (order_band; a kernel of its own, as the divisions behind a branch cost every small product 0.2 us of 4 .. 8).
 template <int EPI, bool HILO, int BM, int BN, int WM, int WN, int S, bool TWO = false, int GROUP = 0>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
   constexpr int NW = WM * WN, AR = HILO ? 2 * BM : BM, QA = AR / 8 / NW, QW = BN / 8 / NW, STAGE = (AR + BN) * 128;
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
     Mg = p.g_cnt[grp];
   } else {
     int tm = bid % tiles_m, tn = bid / tiles_m;
-    if (p.group_m > 1) {                               // bands of column tiles, row by row (order_band)
+    if constexpr (GROUP == 4) {                        // bands of column tiles, row by row
       const int per = tiles_m * p.group_m, b = bid / per, in = bid - b * per, w = min(p.group_m, tiles_n - b * p.group_m);
       tm = in / w;
       tn = b * p.group_m + in - tm * w;
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(const G256 p) {
     char* dst = &lds[buf * STAGE];
 #pragma unroll
     for (int q = 0; q < QW; ++q)
-      __builtin_amdgcn_global_load_lds((glb_void*)(Wb + (srcW[q] + koff)), (lds_void*)(dst + AR * 128 + (wave * QW + q) * 1024), 16, 0, GROUP >= 2 ? 2 : 0);
+      __builtin_amdgcn_global_load_lds((glb_void*)(Wb + (srcW[q] + koff)), (lds_void*)(dst + AR * 128 + (wave * QW + q) * 1024), 16, 0, GROUP == 2 || GROUP == 3 ? 2 : 0);
 #pragma unroll
     for (int q = 0; q < QA; ++q)
       __builtin_amdgcn_global_load_lds((glb_void*)(Ab + (srcA[q] + koff)), (lds_void*)(dst + (wave * QA + q) * 1024), 16, 0, 0);

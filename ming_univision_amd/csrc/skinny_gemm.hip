@@ -335,11 +335,11 @@ extern "C" size_t mn_skinny_workspace_bytes_w8(int M, int N, int K, int epilogue
 }
 
 // One launch (rows_kc.inl) for up to 32 rows of bf16 weights, where it is estimated faster than the three launches (`fma` false) or the fp32 FMA kernel of
-// 2 .. 8 rows: 2.5 us + (0.85 + 0.042 M, or 1.1 where 17 .. 32 rows go in halves) for every 512 values of K (x 1.7 with two tiles a workgroup, x 1.4 behind an RMSNorm) and round over the CUs, or 0.22 a
+// 2 .. 8 rows: 2.5 us + (0.85 + 0.042 M, or 1.1, behind a silu 1.8, where 17 .. 32 rows go in halves) for every 512 values of K (x 1.7 with two tiles a workgroup, x 1.4 behind an RMSNorm) and round over the CUs, or 0.22 a
 // megabyte of weights, against
 // 8.8 + 0.08 M + 0.2 a megabyte of weights, or 3.2 + 0.19 a megabyte + 0.3 per 1024 of K and as much again a row (8 rows at once; 5 .. 7 as 4 + the rest).  The lines
 // this draws, both sides measured: 32 rows of 2048 x 2048 11.9 / 13.7, of 1024 x 4096 20.1 / 14.8, of 8192 x 2048 (two tiles) 18.8 / 22.4, of 3072 x 3072 17.7 /
-// 17.2, of 3072 x 2048 behind an RMSNorm 17.4 / 16.2; 16 rows of 32 x 3072 9.5 / 8.7; against FMA 2 rows of 2048 x 2048 6.2 / 5.4, of 4096 x 1024 4.6 / 5.3; 4 rows of
+// 17.2, of 3072 x 2048 behind an RMSNorm 17.4 / 16.2; in halves behind a silu, which every workgroup takes, 24 rows of 394 x 4096 17.0 / 13.4, 31 of 37 x 2944 13.1 / 11.1; 16 rows of 32 x 3072 9.5 / 8.7; against FMA 2 rows of 2048 x 2048 6.2 / 5.4, of 4096 x 1024 4.6 / 5.3; 4 rows of
 // 2048 x 2048 6.3 / 7.1; 5 rows of it 6.2 / 11.8; 8 rows of 8192 x 2048 11.8 / 22.5; 2 rows of 32000 x 2048 32.0 / 28.2, 3 rows 33.6 / 36.0.  Two rows stay on FMA,
 // and three of plain products of more than 4096 columns and up to 1024 values: the launch itself is shorter here (7424 x 1024 6.4 / 8.4), but the ones behind it are
 // longer by as much and more (decode steps of 2 rows, four layers of width 1024: 208 / 189, 302 / 280, 191 / 184 us, of 3 rows of such products 211 / 198; of width
@@ -364,7 +364,7 @@ static bool rows_kc(const mn_skinny_args& a, bool fma, hipStream_t st, bool ask 
   // or a second row would be a load that waits for the pieces in flight behind it
   const bool lds = a.M > (nt == 2 && a.K > 1024 ? 6 : 4) && (a.prologue == MN_PRO_NONE || a.prologue == MN_PRO_SILU) && ((uintptr_t)a.x & 15) == 0 && (a.ldx % 4) == 0;
   const bool halves = lds && a.M > 16 && 2 * g <= mn_num_cus();      // 16 rows a workgroup
-  const double here = 2.5 + fmax(0.22 * mb, mn_cdiv(a.K, 512) * (halves ? 1.1 : 0.85 + 0.042 * a.M) * (nt == 2 ? 1.7 : 1.0) * (a.prologue == MN_PRO_RMSNORM ? 1.4 : 1.0) * mn_cdiv(g, mn_num_cus()));
+  const double here = 2.5 + fmax(0.22 * mb, mn_cdiv(a.K, 512) * (halves ? (a.prologue == MN_PRO_SILU ? 1.8 : 1.1) : 0.85 + 0.042 * a.M) * (nt == 2 ? 1.7 : 1.0) * (a.prologue == MN_PRO_RMSNORM ? 1.4 : 1.0) * mn_cdiv(g, mn_num_cus()));
   const double row = 0.4 + 0.25 * kk + 0.02 * mb, once = 3.2 + 0.19 * mb + 0.3 * kk;
   const double there = !fma ? 8.8 + 0.08 * a.M + 0.2 * mb : (a.M > 4 && a.M < 8 ? 2 * once + (a.M - 2) * row : once + (a.M - 1) * row) / 1.15;
   if (fma && (a.M == 2 || (a.M == 3 && nt == 2 && !paired && a.K <= 1024))) return false;

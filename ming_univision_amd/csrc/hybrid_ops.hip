@@ -68,36 +68,40 @@ __global__ __launch_bounds__(256) void head_norm_temp_append_kernel(HeadNormArgs
 }
 
 // The same for heads of quadruples up to 128 values: a head is half a wave's, 16 bytes a lane.  2048 rows of 24 heads of 128: 19.3 -> 14.4 us (50 MB): a wave's life is its round trips, and
-// it carries four times the bytes.
+// it carries four times the bytes.  All loads are on their way before the sum, which takes no LDS (with the weights behind it a few rows of heads of 32 took 3.5 us for 3.2).
 __global__ __launch_bounds__(256) void head_norm_temp_append_vec_kernel(HeadNormArgs a) {
   const int hv = blockIdx.x * 8 + (threadIdx.x >> 5), i = 4 * (threadIdx.x & 31), m = blockIdx.y;
   const int nh = a.H + 2 * a.G;
   if (hv >= nh) return;
   const float* row = a.qkv + (int64_t)m * a.ldqkv;
   const bool is_q = hv < a.H, is_v = hv >= a.H + a.G;
-  const int n = is_v ? a.vdim : a.dim;
+  const int n = is_v ? a.vdim : a.dim, ic = i < n ? i : 0;
   const float* src = row + (is_v ? (int64_t)(a.H + a.G) * a.dim + (int64_t)(hv - a.H - a.G) * a.vdim : (int64_t)hv * a.dim);
-  f32x4 v = *reinterpret_cast<const f32x4*>(src + (i < n ? i : 0));
+  f32x4 v = *reinterpret_cast<const f32x4*>(src + ic), w = {1.f, 1.f, 1.f, 1.f};
   const int seq = a.row_seq[m], slot = a.row_slot[m];
-  const int64_t crow = (int64_t)seq * a.t_max + slot;
-  if (i >= n) v = f32x4{0.f, 0.f, 0.f, 0.f};
-  float ss = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+  const bf16_t* wp = is_q ? a.qw : a.kw;
+  if (wp && !is_v) {
 #pragma unroll
-  for (int o = 1; o < 32; o <<= 1) ss += __shfl_xor(ss, o);
+    for (int e = 0; e < 4; ++e) w[e] = bf16_to_f32(wp[ic + e]);
+  }
+  const int64_t crow = (int64_t)seq * a.t_max + slot;
+  float f = 1.0f;
+  if (is_q) {
+    f = a.q_scale;
+    if (a.temp_every > 0 && a.temp_coef != 0.f) f *= 1.0f + a.temp_coef * logf((float)((slot + 1) / a.temp_every) + 1.0f);
+  }
+  if (i >= n) v = f32x4{0.f, 0.f, 0.f, 0.f};
+  float ss = row16_sum((v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]));
+  const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);      // the other 16 lanes of the head
+  ss = __uint_as_float(both[0]) + __uint_as_float(both[1]);
   float* dst = is_v ? a.v_arena + crow * ((int64_t)a.G * a.vdim) + (int64_t)(hv - a.H - a.G) * a.vdim
                : is_q ? a.q_out + (int64_t)m * a.ldq + (int64_t)hv * a.dim
                       : a.k_arena + crow * ((int64_t)a.G * a.dim) + (int64_t)(hv - a.H) * a.dim;
   if (i >= n) return;
   if (!is_v) {
     const float r = 1.0f / sqrtf(ss / (float)a.dim + a.eps);
-    const bf16_t* w = is_q ? a.qw : a.kw;
-    float f = 1.0f;
-    if (is_q) {
-      f = a.q_scale;
-      if (a.temp_every > 0 && a.temp_coef != 0.f) f *= 1.0f + a.temp_coef * logf((float)((slot + 1) / a.temp_every) + 1.0f);
-    }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = v[e] * r * (w ? bf16_to_f32(w[i + e]) : 1.0f) * f;
+    for (int e = 0; e < 4; ++e) v[e] = v[e] * r * w[e] * f;
   }
   *reinterpret_cast<f32x4*>(dst + i) = v;
 }

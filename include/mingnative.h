@@ -814,7 +814,8 @@ MN_API int mn_gated_norm_filter_rows(float* x, int64_t ldx, const float* g, int6
                                      float* h, int64_t ldh, int M, int n, void* stream);
 MN_API int mn_softcap_rows(float* z, int64_t ld, int M, int n, float cap, void* stream);
 /* C[z] = alpha * A[z] W[z]^T (+ bias) (* sigmoid(G[z])) for z < batch, operands of batch entry z at base + z * (their _bs stride):
- * fp32 products and sums (FMA; more than 2 rows: the fp32 matrix cores, 8 where rows are not of whole 16 bytes), any M / N / K.  C (fp32) and C16 (bf16 copy) are both optional outputs. */
+ * fp32 products and sums (FMA; more than 2 rows: the fp32 matrix cores, 8 where rows are not of whole 16 bytes; many tiles: the bf16 matrix
+ * cores, rows as three exact bf16 parts), any M / N / K.  C (fp32) and C16 (bf16 copy) are both optional outputs. */
 MN_API int mn_gemm_f32_batched(const float* A, int64_t lda, int64_t a_bs, const uint16_t* W, int64_t ldw, int64_t w_bs,
                                const uint16_t* bias, float* C, int64_t ldc, int64_t c_bs, uint16_t* C16, int64_t ldc16, int64_t c16_bs,
                                const float* G, int64_t ldg, int64_t g_bs, int M, int N, int K, int batch, float alpha, void* stream);

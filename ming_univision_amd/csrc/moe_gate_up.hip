@@ -11,10 +11,10 @@
 //  - PARTS (one row, H of 1536 and 2048): the product before this launch has left the gate's dot products as partial sums (row_gemv.inl), 64 KB a workgroup instead of 256 KB of gate rows and
 //    their 4096 wave instructions: routed 2.0 us after the start instead of 5.3, 22.4 -> 17.7 us a launch of 92 MB.  The sums are of the unscaled row; the norm's scale multiplies them.
 //  - a shared expert's wave asks for its weights as soon as the barrier is passed.
-//  - few units in flight: a unit is multiplied while the next arrives.  All 6 requested at once, 48 loads a wave, took 6 us to issue and left 2.6 us of multiplying behind the last: 17.7 -> 16.9
+//  - few units in flight: a unit is multiplied while the next arrives.  All 6 requested at once, 48 loads a wave, took 6 us to issue and left 2.6 us of multiplying behind the last: 17.7 -> 16.9, 17.9 in a traced step
 //    (1 unit 16.9, 2 16.9 - 17.5, 3 16.9, 4 17.1; e4m3 with 1, 2, 3, 6 of its half as long ones 38.3, 38.1, 38.6, 39.6 us a layer, int8 44.1, 42.2, 43.2, 45.0, NF4 49.2, 48.2, 48.6, 49.8).
-// The logits' per-lane arithmetic and the tie rule (lowest expert id among equal probabilities) are moe_router_row_kernel's
-// (decode_ops.hip); the row's square sum is reduced per wave here, per workgroup there — 1-ulp differences of the logits.
+// The tie rule (lowest expert id among equal probabilities) is moe_router_row_kernel's (decode_ops.hip), and without PARTS the logits' per-lane arithmetic, but for the row's square sum, reduced
+// per wave here, per workgroup there: 1-ulp differences of the logits.  With PARTS a logit is a sum of H / 8 sums of eight products.
 #include <type_traits>
 
 #include "common.h"

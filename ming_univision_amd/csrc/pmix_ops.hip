@@ -1334,7 +1334,9 @@ extern "C" int mn_window_attn_splits_heads(int n_blk, int H, int G, int one_row,
   if (vec == 16) return by_runs;
   // (a group of 32 or 64 vectors has some 10 us of its own: a split of its walk below 128 keys costs more than it saves)
   const int64_t groups = mn_cdiv(n_blk, runs) * G * sh.chunks, most = mn_cdiv(max_keys, 128) < tiles ? mn_cdiv(max_keys, 128) : tiles;
-  // (values inside keys: more than two a CU, 8 heads of 2048 tokens, keys of 320, 1: 399, 2: 269; heads of 128 1: 200, 2: 200)
+  // (values inside keys, groups that fill two a CU evenly: one split more, us, without / with it, keys of 320: 8 heads, one prompt of 2048 399 / 268, 2 of 1024 208 / 143, 4 of 512 108 / 88, 8 of 256 71 / 62,
+  // one of 1024 114 / 83, 2 of 512 69 / 56, 4 of 256 45.5 / 42.7; 16 heads, 1024 207 / 142, 4 of 256 70 / 61.5, 512 68 / 55.  Heads of 128, 2048 tokens 190 / 197.  Above 512 groups one split stays: one prompt
+  // of 2052 .. 2800 363 .. 513 / 273 .. 468, but 5 of 409 93 / 100, 5 of 500 124 / 127)
   const int by_groups = want(groups, most, vk);
   return attn_runs_alone(n_blk, H, G, by_groups) ? by_runs : by_groups;
 }
